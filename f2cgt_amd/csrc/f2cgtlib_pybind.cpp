@@ -17,6 +17,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "../../include/f2cgt.h"
 
@@ -153,7 +154,9 @@ torch::Tensor sq_compress(torch::Tensor src, torch::Tensor codebooks, int64_t ta
 }
 
 // Extension: the storage tensor in one pass (= sq_compress -> cast -> packbits of the callers).
-torch::Tensor sq_encode(torch::Tensor src, torch::Tensor codebooks, int64_t target_bits, int64_t column_slice) {
+// `out`: where to put it (a contiguous [rows, words] block of a larger table), instead of a new tensor.
+torch::Tensor sq_encode(torch::Tensor src, torch::Tensor codebooks, int64_t target_bits, int64_t column_slice,
+                        c10::optional<torch::Tensor> into) {
   src = dev_contig(src, "src");
   TORCH_CHECK(src.dim() == 2 && src.scalar_type() == torch::kFloat32, "src must be float32 [rows, feat_dim]");
   TORCH_CHECK(target_bits == 1 || target_bits == 2 || target_bits == 4 || target_bits == 8 || target_bits == 16,
@@ -161,12 +164,46 @@ torch::Tensor sq_encode(torch::Tensor src, torch::Tensor codebooks, int64_t targ
   codebooks = sq_codebooks_checked(codebooks);
   c10::DeviceGuard guard(src.device());
   const int64_t d = src.size(1);
-  auto out = target_bits < 8
-                 ? torch::empty({src.size(0), (d * target_bits + 7) / 8}, src.options().dtype(torch::kInt8))
-                 : torch::empty({src.size(0), d}, src.options().dtype(target_bits == 8 ? torch::kInt8 : torch::kInt16));
+  const int64_t words = target_bits < 8 ? (d * target_bits + 7) / 8 : d;
+  const auto dtype = target_bits <= 8 ? torch::kInt8 : torch::kInt16;
+  torch::Tensor out;
+  if (into.has_value()) {
+    out = *into;
+    TORCH_CHECK(out.device() == src.device() && out.scalar_type() == dtype && out.dim() == 2 && out.is_contiguous() &&
+                    out.size(0) == src.size(0) && out.size(1) == words,
+                "out must be a contiguous ", dtype, " GPU tensor [", src.size(0), ", ", words, "]");
+  } else {
+    out = torch::empty({src.size(0), words}, src.options().dtype(dtype));
+  }
   check_rc(f2cgt_sq_encode(src.data_ptr<float>(), out.data_ptr(), codebooks.data_ptr<float>(), src.size(0), d,
                            codebooks.size(0), (int)target_bits, column_slice, current_stream()),
            "sq_encode");
+  return out;
+}
+
+// Extension: order statistics, sum and NaN flag of |x| per column slice of the rows `rows` (None: all of them), for the
+// codebooks of sq_encode.  ranks: four ranks in a full slice, four in the last one.  -> float64 [n_slices, 6] on the GPU.
+torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
+                              const std::vector<int64_t>& ranks) {
+  TORCH_CHECK(x.defined() && x.device().is_cuda(), "x must be a GPU tensor");
+  TORCH_CHECK(x.dim() == 2 && x.scalar_type() == torch::kFloat32, "x must be float32 [rows, feat_dim]");
+  if (x.stride(1) != 1) x = x.contiguous();
+  TORCH_CHECK(ranks.size() == 8, "ranks must hold eight values");
+  TORCH_CHECK(column_slice > 0, "column_slice must be positive");
+  torch::Tensor r;
+  if (rows.has_value()) {
+    r = dev_contig(*rows, "rows");
+    TORCH_CHECK(r.dim() == 1 && r.scalar_type() == torch::kInt64, "rows must be int64 [m]");
+  }
+  c10::DeviceGuard guard(x.device());
+  const int64_t m = r.defined() ? r.numel() : x.size(0), cols = x.size(1);
+  auto opts = torch::TensorOptions().device(x.device());
+  auto out = torch::empty({(cols + column_slice - 1) / column_slice, 6}, opts.dtype(torch::kFloat64));
+  auto ws = torch::empty({f2cgt_abs_order_stats_workspace_bytes(m, cols, column_slice)}, opts.dtype(torch::kUInt8));
+  check_rc(f2cgt_abs_order_stats(x.data_ptr<float>(), x.stride(0), r.defined() ? r.data_ptr<int64_t>() : nullptr, m,
+                                 x.size(0), cols, column_slice, ranks.data(), ws.data_ptr(), ws.numel(),
+                                 out.data_ptr<double>(), current_stream()),
+           "abs_order_stats");
   return out;
 }
 
@@ -748,7 +785,8 @@ PYBIND11_MODULE(F2CGTLib, m) {
            py::arg("column_slice"), py::arg("feat_dim"), py::arg("weight"), py::arg("bias") = py::none(),
            py::arg("block_rows") = 0, py::arg("overlap") = false)
       .def("sq_encode", &sq_encode, py::arg("src"), py::arg("codebooks"), py::arg("target_bits"),
-           py::arg("column_slice"))
+           py::arg("column_slice"), py::arg("out") = py::none())
+      .def("abs_order_stats", &abs_order_stats, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"))
       .def("kmeans_predict", &kmeans_predict, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode", &vq_encode, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("fetch_rows", &fetch_rows, py::arg("table"), py::arg("index"), py::arg("hot") = py::none(),

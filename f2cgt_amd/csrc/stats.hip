@@ -1,0 +1,377 @@
+// Order statistics and mean of |x| over column slices of a (sampled) feature table: what the scalar quantiser's codebook
+// is made of (examples/process_compress.py:45-68: two percentiles and the mean of the absolute values of a slice).
+//
+// The statistics are exact: the requested ranks are found by a radix selection on the bit pattern of |x| (for
+// non-negative floats the order of the values is the order of the bit patterns), three digits of 12, 10 and 9 bits, each
+// one pass over the sample.  A pass counts the next digit of the values that share the digits found so far with a
+// wanted rank; the counts stay in LDS and are written once per workgroup, a small kernel adds the workgroups' counts, and
+// the next pass finds the digit from the sums in its prologue.  Nothing is sorted, nothing is copied (the rows are read
+// through the sample's row list each time; a sample that fits the 256 MB last-level cache comes from there in the second
+// and third pass), and no counter is shared between workgroups: the hot bins of a normal distribution lie in a dozen
+// cache lines, on which device-wide atomics of 256 workgroups would queue up.
+//
+// What bounds it: the three reads of the sample (17 us each at 120 000 x 100 values, 2.9 TB/s through the row list; the
+// sums between them 3-4 us each).  The seven launches take 66 us where the host took 195 ms on a copy of the sample
+// (np.percentile, two selections); the whole sq_compress call, with one read-back and one upload of the codebook,
+// 132 us against 195-228 ms.
+#include "common.hpp"
+
+namespace f2cgt {
+namespace {
+
+constexpr int kStatThreads = 1024;
+constexpr int kBins = 4096;          // counters of a pass: 4096, 4 x 1024 or 4 x 512
+constexpr int kReplicas = 4;         // copies of the first pass's counters in LDS, by lane: its hot bins are few
+constexpr int kMaxBlocks = 256;      // workgroups per pass over all slices (one per CU)
+
+struct StatState {                   // per slice, written by the first workgroup of a pass for the passes after it
+  uint32_t prefix[4];                // digits found so far of the value at each wanted rank
+  uint32_t pad[4];
+  uint64_t rank[4];                  // its rank among the values that share them
+};
+
+struct StatArgs {
+  const float* x;
+  const int64_t* rows;               // row list of the sample; null: rows [0, m)
+  int64_t m, num_rows, ld;
+  int cols, slice, n_slices;
+  int blocks;                        // workgroups per slice
+  uint64_t ranks[8];                 // wanted ranks of a full slice, and of the last one
+  uint32_t* partial;                 // [n_slices][blocks][kBins]
+  uint32_t* hist;                    // [n_slices][kBins]
+  StatState* state;                  // [2][n_slices]: after the first and the second digit
+  double* sums;                      // [n_slices][blocks]
+  uint32_t* nans;                    // [n_slices][blocks]
+  double* out;                       // [n_slices][6]
+};
+
+// Finds, in `groups` runs of kBins / groups counters, the counter that holds rank[t] (run t, or the only run), for all
+// four ranks, by the whole workgroup: digit[t] is the counter's place in its run and rank[t] becomes the rank inside it.
+template <int GROUPS, int USED>
+__device__ __forceinline__ void find_digits(const uint32_t* __restrict__ hist, const uint64_t (&rank)[4],
+                                            uint64_t* s_scan, uint32_t* s_digit, uint64_t* s_rest) {
+  constexpr int PER = USED / (kStatThreads / GROUPS);   // counters per thread
+  static_assert(PER >= 1, "a thread owns at least one counter");
+  const int t = threadIdx.x;
+  const int group = t / (kStatThreads / GROUPS), at = t % (kStatThreads / GROUPS);
+  uint32_t c[PER];
+  uint64_t own = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    c[i] = hist[group * USED + at * PER + i];
+    own += c[i];
+  }
+  uint64_t run = own;                                   // inclusive sum over the wave
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint64_t other = __shfl_up(run, off);
+    run += (t & (kWave - 1)) >= off ? other : 0;
+  }
+  if ((t & (kWave - 1)) == kWave - 1) s_scan[t / kWave] = run;
+  if (t < 4) { s_digit[t] = 0; s_rest[t] = 0; }
+  __syncthreads();
+  constexpr int WPG = kStatThreads / kWave / GROUPS;    // waves per run
+  uint64_t before = run - own;
+  for (int w = group * WPG; w < t / kWave; ++w) before += s_scan[w];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if (GROUPS > 1 && k != group) continue;
+    const uint64_t want = rank[k];
+    if (want < before || want >= before + own) continue;
+    uint64_t lo = before;
+    int found = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (want >= lo && want < lo + c[i]) { found = i; s_rest[k] = want - lo; }
+      lo += c[i];
+    }
+    s_digit[k] = (uint32_t)(at * PER + found);
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ void wanted_ranks(const StatArgs& a, int slice, uint64_t (&rank)[4]) {
+  const int base = slice == a.n_slices - 1 ? 4 : 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) rank[k] = a.ranks[base + k];
+}
+
+// The digits known after pass PASS - 1 (prefix of every wanted rank, rank inside it), by every workgroup from the summed
+// counters of that pass.
+template <int PASS>
+__device__ __forceinline__ void known_digits(const StatArgs& a, int slice, uint64_t* s_scan, uint32_t* s_digit,
+                                             uint64_t* s_rest, uint32_t (&prefix)[4], uint64_t (&rank)[4]) {
+  const uint32_t* hist = a.hist + (int64_t)slice * kBins;
+  if (PASS == 1) {
+    wanted_ranks(a, slice, rank);
+    find_digits<1, 4096>(hist, rank, s_scan, s_digit, s_rest);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) prefix[k] = s_digit[k];
+  } else {
+    const StatState& st = a.state[(PASS - 2) * a.n_slices + slice];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) rank[k] = st.rank[k];
+    find_digits<4, PASS == 2 ? 1024 : 512>(hist, rank, s_scan, s_digit, s_rest);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) prefix[k] = (st.prefix[k] << (PASS == 2 ? 10 : 9)) | s_digit[k];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) rank[k] = s_rest[k];
+}
+
+// One pass over the sample.  A thread keeps its place in the row (a V-wide column group) and walks rows; four rows are in
+// flight at a time.
+template <int PASS, int V>
+__global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
+  __shared__ __align__(16) uint32_t s_hist[PASS == 0 ? kBins * kReplicas : kBins];
+  __shared__ uint64_t s_scan[kStatThreads / kWave];
+  __shared__ uint32_t s_digit[4];
+  __shared__ uint64_t s_rest[4];
+  __shared__ double s_sum[kStatThreads / kWave];
+  __shared__ uint32_t s_nan;
+  const int t = threadIdx.x, slice = blockIdx.y;
+  constexpr int LDS_BINS = PASS == 0 ? kBins * kReplicas : kBins;
+  for (int i = t; i < LDS_BINS / 4; i += kStatThreads) reinterpret_cast<uint4*>(s_hist)[i] = make_uint4(0u, 0u, 0u, 0u);
+  if (t == 0) s_nan = 0u;
+  uint32_t prefix[4] = {0u, 0u, 0u, 0u};
+  if constexpr (PASS > 0) {
+    uint64_t rank[4];
+    known_digits<PASS>(a, slice, s_scan, s_digit, s_rest, prefix, rank);
+    if (blockIdx.x == 0 && t == 0) {
+      StatState& st = a.state[(PASS - 1) * a.n_slices + slice];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) { st.prefix[k] = prefix[k]; st.rank[k] = rank[k]; }
+    }
+  }
+  __syncthreads();
+
+  const int col0 = slice * a.slice;
+  const int width = a.cols - col0 < a.slice ? a.cols - col0 : a.slice;
+  const int groups = width / V;
+  const int cg = groups < kStatThreads ? groups : kStatThreads;
+  const int rpp = kStatThreads / cg;                    // rows per pass of the workgroup
+  const int r0 = t / cg, c0 = t - r0 * cg;
+  const int64_t step = (int64_t)a.blocks * rpp;
+  double sum = 0.0;
+  bool nan = false;
+  auto take = [&](float v) {
+    const uint32_t mag = __float_as_uint(v) & 0x7fffffffu;
+    if constexpr (PASS == 0) {
+      sum += (double)__uint_as_float(mag);
+      nan = nan || mag > 0x7f800000u;
+      atomicAdd(&s_hist[(mag >> 19) * kReplicas + (t & (kReplicas - 1))], 1u);
+    } else if constexpr (PASS == 1) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if ((mag >> 19) == prefix[k]) atomicAdd(&s_hist[k * 1024 + ((mag >> 9) & 1023u)], 1u);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if ((mag >> 9) == prefix[k]) atomicAdd(&s_hist[k * 512 + (mag & 511u)], 1u);
+    }
+  };
+  if (r0 < rpp) {
+    constexpr int U = 4;
+    for (int64_t r = (int64_t)blockIdx.x * rpp + r0; r < a.m; r += step * U) {
+      int64_t id[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t ru = r + u * step < a.m ? r + u * step : r;
+        id[u] = ru;
+        if (a.rows != nullptr) {
+          const int64_t want = a.rows[ru];
+          id[u] = clamp_idx(want < 0 ? want + a.num_rows : want, a.num_rows);
+        }
+      }
+      for (int c = c0; c < groups; c += cg) {
+        float v[U][V];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float* p = a.x + id[u] * a.ld + col0 + c * V;
+          if constexpr (V == 4) {
+            const float4 q = *reinterpret_cast<const float4*>(p);
+            v[u][0] = q.x; v[u][1] = q.y; v[u][2] = q.z; v[u][3] = q.w;
+          } else if constexpr (V == 2) {
+            const float2 q = *reinterpret_cast<const float2*>(p);
+            v[u][0] = q.x; v[u][1] = q.y;
+          } else {
+            v[u][0] = *p;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (u > 0 && r + u * step >= a.m) break;
+#pragma unroll
+          for (int i = 0; i < V; ++i) take(v[u][i]);
+        }
+      }
+    }
+  }
+  if constexpr (PASS == 0) {
+    if (nan) atomicOr(&s_nan, 1u);
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    if ((t & (kWave - 1)) == 0) s_sum[t / kWave] = sum;
+  }
+  __syncthreads();
+  uint32_t* dst = a.partial + ((int64_t)slice * a.blocks + blockIdx.x) * kBins;
+  for (int i = t; i < (PASS == 2 ? 2048 : kBins); i += kStatThreads) {
+    if constexpr (PASS == 0) {
+      uint32_t c = 0;
+#pragma unroll
+      for (int k = 0; k < kReplicas; ++k) c += s_hist[i * kReplicas + k];
+      dst[i] = c;
+    } else {
+      dst[i] = s_hist[i];
+    }
+  }
+  if (PASS == 0 && t == 0) {
+    double total = 0.0;
+    for (int w = 0; w < kStatThreads / kWave; ++w) total += s_sum[w];
+    a.sums[(int64_t)slice * a.blocks + blockIdx.x] = total;
+    a.nans[(int64_t)slice * a.blocks + blockIdx.x] = s_nan;
+  }
+}
+
+// hist[bin] = sum of the workgroups' counts: a wave reads 64 neighbouring bins of every sixteenth workgroup, all its
+// reads in flight at once (with four waves to 64 bins, four rounds of reads each, the kernel took 9 us instead of 4).
+__global__ __launch_bounds__(kStatThreads) void stat_reduce_kernel(StatArgs a) {
+  constexpr int WAVES = kStatThreads / kWave;
+  __shared__ uint32_t s_part[WAVES][kWave];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int bin = blockIdx.x * kWave + lane, slice = blockIdx.y;
+  const uint32_t* src = a.partial + (int64_t)slice * a.blocks * kBins + bin;
+  uint32_t c = 0;
+#pragma unroll 16
+  for (int b = wave; b < a.blocks; b += WAVES) c += src[(int64_t)b * kBins];
+  s_part[wave][lane] = c;
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int w = 1; w < WAVES; ++w) c += s_part[w][lane];
+  a.hist[(int64_t)slice * kBins + bin] = c;
+}
+
+// Last digit, and the outputs of a slice: the values at the four ranks, the sum, whether a NaN was seen.
+__global__ __launch_bounds__(kStatThreads) void stat_finish_kernel(StatArgs a) {
+  __shared__ uint64_t s_scan[kStatThreads / kWave];
+  __shared__ uint32_t s_digit[4];
+  __shared__ uint64_t s_rest[4];
+  const int slice = blockIdx.x, t = threadIdx.x;
+  uint32_t prefix[4];
+  uint64_t rank[4];
+  known_digits<3>(a, slice, s_scan, s_digit, s_rest, prefix, rank);
+  if (t < 4) a.out[slice * 6 + t] = (double)__uint_as_float(t == 0 ? prefix[0] : t == 1 ? prefix[1] : t == 2 ? prefix[2] : prefix[3]);
+  if (t >= kWave && t < 2 * kWave) {                    // the second wave
+    double total = 0.0;
+    uint32_t nan = 0;
+    for (int b = t - kWave; b < a.blocks; b += kWave) {
+      total += a.sums[(int64_t)slice * a.blocks + b];
+      nan |= a.nans[(int64_t)slice * a.blocks + b];
+    }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+      total += __shfl_xor(total, off);
+      nan |= __shfl_xor(nan, off);
+    }
+    if (t == kWave) {
+      a.out[slice * 6 + 4] = total;
+      a.out[slice * 6 + 5] = nan ? 1.0 : 0.0;
+    }
+  }
+}
+
+// Workgroups per slice: one per CU over all slices, each with at least 32 values per thread.
+int stat_blocks(int64_t m, int64_t cols, int64_t slice, int64_t n_slices) {
+  const int64_t width = cols < slice ? cols : slice;
+  int64_t b = ceil_div(m * width, (int64_t)kStatThreads * 32);
+  const int64_t cap = n_slices >= kMaxBlocks / 4 ? 4 : kMaxBlocks / n_slices;
+  b = b > cap ? cap : b;
+  return (int)(b < 1 ? 1 : b);
+}
+
+int64_t round256(int64_t v) { return (v + 255) / 256 * 256; }
+
+struct StatLayout { int64_t hist, state, sums, nans, total; };
+StatLayout stat_layout(int64_t blocks, int64_t n_slices) {
+  StatLayout l;
+  l.hist = round256(n_slices * blocks * kBins * 4);
+  l.state = l.hist + round256(n_slices * kBins * 4);
+  l.sums = l.state + round256(2 * n_slices * (int64_t)sizeof(StatState));
+  l.nans = l.sums + round256(n_slices * blocks * 8);
+  l.total = l.nans + round256(n_slices * blocks * 4);
+  return l;
+}
+
+template <int V>
+void stat_launch(const StatArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)a.blocks, (unsigned)a.n_slices), rgrid(kBins / kWave, (unsigned)a.n_slices);
+  const dim3 rgrid_last(2048 / kWave, (unsigned)a.n_slices);
+  stat_pass_kernel<0, V><<<grid, kStatThreads, 0, st>>>(a);
+  stat_reduce_kernel<<<rgrid, kStatThreads, 0, st>>>(a);
+  stat_pass_kernel<1, V><<<grid, kStatThreads, 0, st>>>(a);
+  stat_reduce_kernel<<<rgrid, kStatThreads, 0, st>>>(a);
+  stat_pass_kernel<2, V><<<grid, kStatThreads, 0, st>>>(a);
+  stat_reduce_kernel<<<rgrid_last, kStatThreads, 0, st>>>(a);
+  stat_finish_kernel<<<(unsigned)a.n_slices, kStatThreads, 0, st>>>(a);
+}
+
+int stat_check(const char* what, int64_t m, int64_t cols, int64_t slice) {
+  F2CGT_REQUIRE(m > 0 && cols > 0 && slice > 0, F2CGT_E_INVALID, "%s: sizes must be positive", what);
+  F2CGT_REQUIRE(cols < (1ll << 24) && ceil_div(cols, slice) <= 65535, F2CGT_E_UNSUPPORTED, "%s: too many columns or slices", what);
+  return 0;
+}
+
+}  // namespace
+}  // namespace f2cgt
+
+using namespace f2cgt;
+
+extern "C" int64_t f2cgt_abs_order_stats_workspace_bytes(int64_t m, int64_t cols, int64_t column_slice) {
+  if (m <= 0 || cols <= 0 || column_slice <= 0) return 0;
+  const int64_t n_slices = ceil_div(cols, column_slice);
+  return stat_layout(stat_blocks(m, cols, column_slice, n_slices), n_slices).total;
+}
+
+extern "C" int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows,
+                                     int64_t cols, int64_t column_slice, const int64_t* ranks, void* workspace,
+                                     int64_t workspace_bytes, double* out, void* stream) {
+  const char* what = "abs_order_stats";
+  if (int rc = stat_check(what, m, cols, column_slice)) return rc;
+  F2CGT_REQUIRE(ld >= cols && num_rows > 0 && (rows != nullptr || m <= num_rows), F2CGT_E_INVALID,
+                "%s: the sample does not fit the table", what);
+  F2CGT_REQUIRE(x && ranks && workspace && out && aligned(workspace, 256), F2CGT_E_INVALID,
+                "%s: null buffer or misaligned workspace", what);
+  F2CGT_REQUIRE(workspace_bytes >= f2cgt_abs_order_stats_workspace_bytes(m, cols, column_slice), F2CGT_E_INVALID,
+                "%s: workspace too small", what);
+  const int64_t n_slices = ceil_div(cols, column_slice);
+  const int64_t full = (cols < column_slice ? cols : column_slice) * m, last = (cols - (n_slices - 1) * column_slice) * m;
+  F2CGT_REQUIRE(full < (1ll << 32), F2CGT_E_UNSUPPORTED, "%s: a slice of the sample has more than 2^32 values", what);
+  for (int k = 0; k < 8; ++k) {
+    F2CGT_REQUIRE(ranks[k] >= 0 && ranks[k] < (k < 4 ? full : last), F2CGT_E_INVALID, "%s: rank %lld out of range", what,
+                  (long long)ranks[k]);
+  }
+  StatArgs a{};
+  a.x = x; a.rows = rows; a.m = m; a.num_rows = num_rows; a.ld = ld;
+  a.cols = (int)cols; a.slice = (int)(column_slice < cols ? column_slice : cols); a.n_slices = (int)n_slices;
+  a.blocks = stat_blocks(m, cols, column_slice, n_slices);
+  for (int k = 0; k < 8; ++k) a.ranks[k] = (uint64_t)ranks[k];
+  const StatLayout l = stat_layout(a.blocks, n_slices);
+  char* ws = static_cast<char*>(workspace);
+  a.partial = reinterpret_cast<uint32_t*>(ws);
+  a.hist = reinterpret_cast<uint32_t*>(ws + l.hist);
+  a.state = reinterpret_cast<StatState*>(ws + l.state);
+  a.sums = reinterpret_cast<double*>(ws + l.sums);
+  a.nans = reinterpret_cast<uint32_t*>(ws + l.nans);
+  a.out = out;
+  // widest access that every slice of every row is a multiple of
+  const int64_t last_width = cols - (n_slices - 1) * column_slice;
+  auto fits = [&](int v) {
+    return ld % v == 0 && (n_slices == 1 || column_slice % v == 0) && last_width % v == 0 && aligned(x, 4 * v);
+  };
+  hipStream_t st = as_stream(stream);
+  if (fits(4)) stat_launch<4>(a, st);
+  else if (fits(2)) stat_launch<2>(a, st);
+  else stat_launch<1>(a, st);
+  return launch_status(what);
+}

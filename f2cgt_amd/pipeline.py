@@ -47,20 +47,69 @@ def sampling(sample_size, num_items, hotness=None, generator=None):
     return torch.from_numpy(np.random.choice(num_items, size, replace=False, p=p))
 
 
+_PERCENTILES = (0.5, 99.5)
+
+
+def _percentile_place(n, percent):
+    """Where numpy's linear percentile of n float32 values lies: (rank below, rank above, weight of the latter).  numpy
+    evaluates the place in the sample's own precision, so (n - 1) * percent / 100 is a float32 here too: beyond 2^24
+    values it falls on a whole rank near the exact one."""
+    place = np.float32(n - 1) * (np.float32(percent) / np.float32(100))
+    if place >= np.float32(n - 1):
+        return n - 1, n - 1, np.float32(0)
+    below = np.floor(place)
+    return int(below), int(below) + 1, np.float32(place - below)
+
+
+def _between(below, above, weight):
+    """The value `weight` of the way from below to above, in float32, from the nearer of the two."""
+    with np.errstate(invalid="ignore"):
+        gap = above - below
+        return below + gap * weight if weight < np.float32(0.5) else above - gap * (np.float32(1) - weight)
+
+
+def _sq_codebook(lo, hi, level):
+    """(fmin, fmax, emin, emax, mean) from the two percentiles and the mean of |x|."""
+    floor = 1e-5
+    fmin, fmax = torch.tensor(max(lo, floor)), torch.tensor(max(hi, 2 * floor))
+    level = level + 0.1 if level < 0.1 else level
+    return fmin, fmax, torch.log2(fmin), torch.log2(fmax) + floor, level
+
+
+def _device_statistics(values, rows, column_slice):
+    """Per column slice of float32 GPU rows: (0.5th and 99.5th percentile, mean) of |x|, from exact order statistics
+    found on the device; the percentile's interpolation is numpy's, in float32."""
+    m = values.shape[0] if rows is None else rows.numel()
+    cols = values.shape[1]
+    count = (cols + column_slice - 1) // column_slice
+    sizes = [m * min(column_slice, cols), m * (cols - (count - 1) * column_slice)]
+    places = [[_percentile_place(n, q) for q in _PERCENTILES] for n in sizes]
+    ranks = [r for per_size in places for place in per_size for r in place[:2]]
+    stats = _capi().abs_order_stats(values, rows, column_slice, ranks).cpu().numpy()
+    out = []
+    for i in range(count):
+        last = int(i == count - 1)
+        if stats[i, 5]:
+            lo = hi = np.float32("nan")
+        else:
+            lo, hi = (_between(np.float32(stats[i, 2 * q]), np.float32(stats[i, 2 * q + 1]), places[last][q][2]) for q in (0, 1))
+        out.append((lo, hi, torch.tensor(np.float32(stats[i, 4] / sizes[last]))))
+    return out
+
+
 def sq_metadata(sample):
     """(fmin, fmax, emin, emax, mean) of one column slice from a sample of its rows:
-    float64 percentiles of |x| floored at 1e-5 / 2e-5, log2 in float64, mean lifted by 0.1 when
-    below 0.1 (examples/process_compress.py:45-68)."""
-    floor = 1e-5
+    percentiles of |x| floored at 1e-5 / 2e-5, their log2, mean lifted by 0.1 when
+    below 0.1 (examples/process_compress.py:45-68).  A sample on the GPU is reduced there."""
+    if sample.is_cuda and sample.numel():
+        values = sample.float()
+        return _sq_codebook(*_device_statistics(values.reshape(values.shape[0], -1), None, values[0].numel())[0])
     magnitude = sample.float().abs().cpu()
     # one percentile and one log2 at a time, as the reference does: numpy returns the sample's own
     # precision for a scalar quantile (float64 for a list of them), and torch's scalar and vector
     # log2 do not agree to the last bit
-    lo, hi = np.percentile(magnitude.numpy(), 0.5), np.percentile(magnitude.numpy(), 99.5)
-    fmin, fmax = torch.tensor(max(lo, floor)), torch.tensor(max(hi, 2 * floor))
-    level = magnitude.mean()
-    level = level + 0.1 if level < 0.1 else level
-    return fmin, fmax, torch.log2(fmin), torch.log2(fmax) + floor, level
+    lo, hi = (np.percentile(magnitude.numpy(), q) for q in _PERCENTILES)
+    return _sq_codebook(lo, hi, magnitude.mean())
 
 
 def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=None, batch_rows=1_000_000):
@@ -71,14 +120,12 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
     num_items, feat_dim = features.shape
     if sample_index is None:
         sample_index = sampling(250_000, num_items, hotness)
-    num_codebooks = (feat_dim + column_slice - 1) // column_slice
-    codebooks = torch.zeros((num_codebooks, 5), dtype=torch.float32)
-    for i in range(num_codebooks):
-        lo, hi = i * column_slice, min((i + 1) * column_slice, feat_dim)
-        vals = sq_metadata(features[sample_index.to(features.device), lo:hi])
-        for j, v in enumerate(vals):
-            codebooks[i, j] = v
-    codebooks = codebooks.cuda()
+    sample_index = sample_index.to(features.device)
+    if features.is_cuda and features.dtype == torch.float32 and sample_index.dtype == torch.int64 and sample_index.numel():
+        stats = _device_statistics(features, sample_index, column_slice)     # the sample's rows are read in place
+    else:
+        stats = _device_statistics(features[sample_index].float().cuda(), None, column_slice)
+    codebooks = torch.tensor([[float(v) for v in _sq_codebook(*values)] for values in stats], dtype=torch.float32).cuda()
     if target_bits <= 8:
         dtype, tdim = torch.int8, int(math.ceil(feat_dim / 8 * target_bits))
     elif target_bits <= 16:
@@ -90,7 +137,7 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
         end = min(start + batch_rows, num_items)
         data = features[start:end].cuda().to(torch.float32)
         # one pass; the reference calls sq_compress, casts and packs (process_compress.py:128-139)
-        out[start:end].copy_(capi.sq_encode(data, codebooks, target_bits, column_slice))
+        capi.sq_encode(data, codebooks, target_bits, column_slice, out[start:end])
     return out, codebooks
 
 

@@ -1,0 +1,74 @@
+"""Order statistics of |x| per column slice (f2cgt_abs_order_stats) against a sorted copy, and the SQ codebooks made from
+them against numpy's percentiles."""
+import numpy as np
+import pytest
+import torch
+
+import f2cgt_amd
+import f2cgt_oracle as oc
+
+pytestmark = pytest.mark.gpu
+
+
+def _values(kind, rng, n, d):
+    if kind == "normal":
+        return rng.standard_normal((n, d)).astype(np.float32) * np.float32(3)
+    if kind == "equal":
+        return np.full((n, d), -0.75, dtype=np.float32)
+    if kind == "bits":         # every exponent, denormal numbers and infinities among them
+        bits = rng.integers(0, 0x7f800001, size=(n, d), dtype=np.uint32) | (rng.integers(0, 2, size=(n, d), dtype=np.uint32) << 31)
+        return bits.view(np.float32)
+    return np.where(rng.random((n, d)) < 0.6, 0.0, rng.standard_normal((n, d))).astype(np.float32)   # mostly zeros
+
+
+# one value; a row wider than a workgroup; slices of 8 with a ragged last one; odd widths (scalar loads), pairs, quads;
+# more slices than workgroups per slice; enough rows for every workgroup and an odd remainder
+@pytest.mark.parametrize("kind", ["normal", "equal", "bits", "sparse"])
+@pytest.mark.parametrize("n,d,slice_", [(1, 1, 1), (3, 1500, 1500), (4097, 20, 8), (5000, 7, 7), (2049, 30, 30),
+                                        (700, 602, 8), (40001, 100, 104), (1023, 4100, 4100)])
+def test_ranks_sum_and_flag(kind, n, d, slice_):
+    rng = np.random.default_rng(n + d)
+    table = _values(kind, rng, n + 50, d)
+    rows = rng.integers(-n, n + 50, size=n)
+    sample = np.abs(table[rows])
+    count = (d + slice_ - 1) // slice_
+    widths = [min(slice_, d), d - (count - 1) * slice_]
+    ranks = []
+    for w in widths:
+        total = n * w
+        ranks += [0, total // 200, total * 199 // 200, total - 1]
+    got = f2cgt_amd.load().abs_order_stats(torch.from_numpy(table).cuda(), torch.from_numpy(rows).cuda(), slice_, ranks)
+    got = got.cpu().numpy()
+    assert got.shape == (count, 6)
+    for i in range(count):
+        part = np.sort(sample[:, i * slice_:(i + 1) * slice_].ravel())
+        want = part[ranks[4:] if i == count - 1 else ranks[:4]]
+        assert np.array_equal(got[i, :4].astype(np.float32), want)
+        assert got[i, 5] == 0.0
+        # fp64 sums of non-negative values in any order: (number of terms) roundings of the total at most
+        assert np.allclose(got[i, 4], part.sum(dtype=np.float64), rtol=part.size * 2.0 ** -52)
+
+
+def test_a_nan_is_reported():
+    x = torch.rand((3000, 24), device="cuda")
+    x[2111, 17] = float("nan")
+    got = f2cgt_amd.load().abs_order_stats(x, None, 8, [0, 1, 2, 3] * 2).cpu()
+    assert got[:, 5].tolist() == [0.0, 0.0, 1.0]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("n,d,slice_", [(2000, 100, 104), (1501, 37, 16)])
+def test_codebooks_on_the_device_are_numpys(dtype, n, d, slice_):
+    from f2cgt_amd import pipeline
+    rng = np.random.default_rng(d)
+    x = torch.from_numpy(rng.standard_normal((n, d)).astype(np.float32)).to(dtype)
+    pick = torch.from_numpy(rng.permutation(n)[:n * 3 // 4])
+    for where in ("cuda", "cpu"):
+        _, books = pipeline.sq_compress(x.to(where), 4, slice_, sample_index=pick)
+        for i in range(books.shape[0]):
+            want = oc.sq_codebook(x[pick].float().numpy()[:, i * slice_:(i + 1) * slice_])
+            got = books[i].cpu().numpy()
+            assert np.array_equal(got[:4], want[:4]) and np.isclose(got[4], want[4], rtol=1e-6)
+    one = np.array([float(v) for v in pipeline.sq_metadata(x[pick].cuda())], dtype=np.float32)
+    want = oc.sq_codebook(x[pick].float().numpy())
+    assert np.array_equal(one[:4], want[:4]) and np.isclose(one[4], want[4], rtol=1e-6)
