@@ -1000,11 +1000,14 @@ struct RowsArgs {
   int64_t R, E, N;
   int src_dim, feat_dim;
   int rows_per_block, edge_cap;
+  int id_cap;            // source ids kept in LDS; edge_cap of them with their code rows
   int eff_bytes, pitch;  // useful bytes of a code row; staged bytes per edge (multiple of 8)
   int lanes, lane_shift;
   int f4_per_row, fin_group, fin_slots;
   uint32_t fin_magic;
   int nt_out;            // output larger than the last-level cache: non-temporal stores
+  int items_per_row;     // FLAT: column groups of a row, and ceil(2^32 / that)
+  uint32_t item_magic;
 };
 
 
@@ -1013,12 +1016,27 @@ __device__ __forceinline__ float mean_of(float sum, float d, float r) {
   return __fmaf_rn(__fmaf_rn(-q, d, sum), r, q);
 }
 
+// Adds the eight 1-bit values of a code byte to s: +plus where the bit is set, -plus where it is not, the two values a
+// 1-bit log-domain codebook has.  The bits become the signs of halves (-1 or 1, two per instruction) and the sums
+// fma(+-1, -plus, s), which rounds as the addition does: two instructions per value and no table read.
+__device__ __forceinline__ void add_signs8(float (&s)[8], uint32_t byte, float minus_plus) {
+  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+  const uint32_t w = byte | (byte << 12);        // bit i at i, bit i + 4 at i + 16
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t pair = ((w << (15 - i)) & 0x80008000u) | 0x3c003c00u;
+    const half2v h = __builtin_bit_cast(half2v, pair);
+    s[i] = __builtin_fmaf((float)h[0], minus_plus, s[i]);
+    s[i + 4] = __builtin_fmaf((float)h[1], minus_plus, s[i + 4]);
+  }
+}
+
 // HALF: 0, or 1 / 2 for output rows at any multiple of 8 bytes, possibly with a last group of two columns (rows of
 // 4 k + 2 columns), written with cached / streamed stores (see acc_fin_params).  4- and 8-bit rows always take 1 or 2:
 // with the store form fixed at compile time the row loop came out 3-5 % faster at 100-256 columns and 17-19 % at 600
 // (3e6 edges, 10 per row, 4 bit: 97.8 -> 93.7 us at 128 columns, 592 -> 489 us at 600); 1- and 2-bit rows measured
 // level to 2 % slower and keep the run-time test.
-template <int BITS, bool AFFINE, typename Idx, int TB, int HALF = 0>
+template <int BITS, bool AFFINE, typename Idx, int TB, int HALF = 0, bool FLAT = false>
 __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __restrict__ indptr,
                                                              const Idx* __restrict__ indices,
                                                              float* __restrict__ out) {
@@ -1033,7 +1051,7 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
   int* s_cnt = s_ptr + a.rows_per_block + 4;                                     // [16] rows per degree class
   int* s_order = s_cnt + 16;                                                     // [RB] rows, heaviest first
   uint32_t* s_ids = reinterpret_cast<uint32_t*>(s_order + a.rows_per_block);     // [edge_cap]
-  unsigned char* s_codes = reinterpret_cast<unsigned char*>(s_ids + a.edge_cap); // [edge_cap][pitch]
+  unsigned char* s_codes = reinterpret_cast<unsigned char*>(s_ids + a.id_cap);   // [edge_cap][pitch]
 
   const int t = threadIdx.x;
   const int64_t row0 = (int64_t)blockIdx.x * a.rows_per_block;
@@ -1064,6 +1082,7 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
   __syncthreads();
   const int ne = s_ptr[nrows];
   const bool staged = ne <= a.edge_cap;
+  const bool have_ids = ne <= a.id_cap;
 
   // Rows are visited heaviest first (counting sort on min(degree, 15)), so the lanes of a wave,
   // which each walk one row's edges, loop about equally long instead of all waiting for the
@@ -1079,7 +1098,7 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
       my_rank[k] = atomicAdd(&s_cnt[my_class[k]], 1);
     }
   }
-  if (staged)
+  if (have_ids)
     for (int i = t; i < ne; i += TB) s_ids[i] = (uint32_t)clamp_idx(indices[e0 + i], a.N);
   __syncthreads();
 #pragma unroll
@@ -1120,6 +1139,86 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
     }
   }
   __syncthreads();
+
+  if constexpr (FLAT) {
+    // decode + sum: (row, column group) items dealt to the lanes one after the other.  Bound by instruction issue: two
+    // to three per value with 1-bit codes, an LDS read and three with the others; 60001 rows of 602 columns at 10
+    // edges per row write 2.0 TB/s with 1-bit codes (staged rows with a column group per lane: 0.77 TB/s).
+    constexpr int G = BITS == 1 ? 8 : 4;                 // columns of an item
+    constexpr int GB = G * BITS / 8;                     // its code bytes
+    const int items = nrows * a.items_per_row;
+    const float minus_plus = -s_lut[1];
+    for (int item = t; item < items; item += TB) {
+      const int ri = (int)__umulhi((uint32_t)item, a.item_magic);
+      const int c = item - ri * a.items_per_row;
+      const int r = s_order[ri];
+      const int b = s_ptr[r], e = s_ptr[r + 1];
+      const int left = a.feat_dim - c * G;               // columns to the row's end, at least two
+      float s[G];
+#pragma unroll
+      for (int i = 0; i < G; ++i) s[i] = 0.f;
+      auto read = [&](int k) -> uint32_t {
+        if (staged) {
+          const unsigned char* q = s_codes + k * a.pitch + c * GB;
+          if constexpr (GB == 4) return *reinterpret_cast<const uint32_t*>(q);
+          else if constexpr (GB == 2) return *reinterpret_cast<const uint16_t*>(q);
+          else return *q;
+        }
+        const uint32_t id = have_ids ? s_ids[k] : (uint32_t)clamp_idx(indices[e0 + k], a.N);
+        const uint8_t* q = a.codes + ((uint64_t)id * (uint32_t)a.src_dim + (uint32_t)(c * GB));
+        if constexpr (GB == 1) return *q;
+        uint32_t w = 0;                                  // a last group of two columns has half the bytes
+        if (HALF != 0 && left < G) __builtin_memcpy(&w, q, GB / 2);
+        else __builtin_memcpy(&w, q, GB);
+        return w;
+      };
+      auto add = [&](uint32_t w) {
+        if constexpr (BITS == 1) {
+          add_signs8(s, w, minus_plus);
+        } else {
+#pragma unroll
+          for (int i = 0; i < G; ++i) s[i] += s_lut[(w >> (BITS * i)) & MASK];
+        }
+      };
+      int k = b;
+      for (; k + 4 <= e; k += 4) {
+        const uint32_t w0 = read(k), w1 = read(k + 1), w2 = read(k + 2), w3 = read(k + 3);
+        add(w0); add(w1); add(w2); add(w3);
+      }
+      if (k + 2 <= e) {
+        const uint32_t w0 = read(k), w1 = read(k + 1);
+        add(w0); add(w1);
+        k += 2;
+      }
+      if (k < e) add(read(k));
+      const int deg = e - b;
+      if (deg > 1) {
+        const float d = (float)deg;
+        float rc = __builtin_amdgcn_rcpf(d);
+        rc = __fmaf_rn(__fmaf_rn(-d, rc, 1.f), rc, rc);
+#pragma unroll
+        for (int i = 0; i < G; ++i) s[i] = mean_of(s[i], d, rc);
+      }
+      float* dst = out + ((row0 + r) * (int64_t)a.feat_dim + c * G);
+#pragma unroll
+      for (int i = 0; i < G; i += 4) {
+        if (i >= left) break;
+        if constexpr (HALF != 0) {
+          if (left - i < 4) {
+            if constexpr (HALF == 2) store_nt2(dst + i, s[i], s[i + 1]);
+            else *reinterpret_cast<float2*>(dst + i) = make_float2(s[i], s[i + 1]);
+          } else {
+            if constexpr (HALF == 2) store_nt4_align8(dst + i, s[i], s[i + 1], s[i + 2], s[i + 3]);
+            else store4_align8(dst + i, s[i], s[i + 1], s[i + 2], s[i + 3]);
+          }
+        } else {
+          if (a.nt_out) store_nt4(dst + i, s[i], s[i + 1], s[i + 2], s[i + 3]);
+          else *reinterpret_cast<float4*>(dst + i) = make_float4(s[i], s[i + 1], s[i + 2], s[i + 3]);
+        }
+      }
+    }
+    return;
+  }
 
   // decode + sum: a lane keeps one float4 column group and walks the rows
   const int g = (int)(((uint32_t)t * a.fin_magic) >> 16);
@@ -1226,14 +1325,9 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
   }
 }
 
-template <int BITS, bool AFFINE>
-int launch_sq_rows(RowsArgs a, const void* indptr, const void* indices, int idx_dtype, float* out, hipStream_t st,
+template <int BITS, bool AFFINE, int TB, bool FLAT>
+int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, int idx_dtype, float* out, hipStream_t st,
                    const char* what) {
-  // 4- and 8-bit rows: 256 threads walk the same staged rows (twice the lanes in the decode + sum
-  // phase, which sets this kernel's time: 35.7 -> 31.9 us and 43.9 -> 34.8 us on the 2.5e5-row
-  // power-law block; 512 threads: 36.6 and 41.6); 1- and 2-bit rows are faster with 128 (27.7 against
-  // 30.8 us), 64 lose everywhere
-  constexpr int TB = BITS >= 4 ? 256 : 128;
   a.eff_bytes = (int)ceil_div(a.feat_dim, 8 / BITS);
   a.pitch = (a.eff_bytes + 7) & ~7;
   a.lanes = a.pitch / 8;
@@ -1244,6 +1338,8 @@ int launch_sq_rows(RowsArgs a, const void* indptr, const void* indices, int idx_
   a.fin_group = a.f4_per_row < TB ? a.f4_per_row : TB;
   a.fin_slots = TB / a.fin_group;
   a.fin_magic = (uint32_t)((65536 + a.fin_group - 1) / a.fin_group);
+  a.items_per_row = (int)ceil_div(a.feat_dim, BITS == 1 ? 8 : 4);
+  a.item_magic = (uint32_t)(((1ull << 32) + a.items_per_row - 1) / a.items_per_row);   // items < 64 * 1024: exact
   a.nt_out = stream_output(a.R * (int64_t)a.feat_dim * 4, (int64_t)a.feat_dim * 4,
                            a.R > 0 ? (double)a.E / (double)a.R : 0.0) ? 1 : 0;
   const size_t lut_bytes = AFFINE ? 0 : (size_t)(((a.num_codebooks << BITS) + 3) & ~3) * 4;
@@ -1264,8 +1360,24 @@ int launch_sq_rows(RowsArgs a, const void* indptr, const void* indices, int idx_
   }
   a.edge_cap = (cap < 8 ? 8 : cap) & ~1;  // even: keeps the staging 8-byte aligned
   int rb = ((int)(0.6 * a.edge_cap / dg) + 4) / 8 * 8;
+  // Direct reads: the source ids alone are kept in LDS and the lanes read the code rows where they are.  An item's
+  // read is 4 bytes (8-bit codes) or covers eight columns (1-bit codes), neighbouring lanes read neighbouring bytes,
+  // and without the staged rows twice the workgroups fit a CU, so this wins for 1- and 8-bit rows at any width, for
+  // rows of more than 128 bytes, and wherever eight rows do not fit the staging (staged / direct, us: 1 bit, 602
+  // columns, 10 edges per row 91 / 73; 8 bit, 128 columns 79 / 67; 2 bit, 602 columns 85 / 75, at 25 edges per row
+  // 247 / 131; 4 bit, 602 columns 152 / 88).  Short 2- and 4-bit rows are better staged (2 bit, 256 columns, 25
+  // edges per row 87 / 96; 4 bit, 100 columns, power-law degrees 34 / 39).
+  const bool direct = FLAT && (BITS == 1 || BITS == 8 || a.pitch > 128 || (int)(8.0 * dg * 1.1) + 8 > a.edge_cap);
+  if (direct) {
+    // about two rounds of items per thread for 1-bit codes, four for the others; at most 480 edges in a block of more
+    // than eight rows, so that long rows spread over the chip
+    a.edge_cap = 0;
+    rb = ((BITS == 1 ? 600 : 1024) / a.items_per_row + 4) / 8 * 8;
+    const int few = (int)(480.0 / dg) / 8 * 8;
+    rb = rb > few ? few : rb;
+  }
   rb = rb < 8 ? 8 : (rb > 64 ? 64 : rb);
-  rb = shrink_rows_per_block(rb, a.R, 16, 8, 1024);
+  rb = shrink_rows_per_block(rb, a.R, direct ? 8 : 16, 8, 1024);
 #ifdef F2CGT_EXPERIMENTS
   if (const char* v = getenv("F2CGT_ROWS_RB")) {
     const int want = atoi(v);
@@ -1281,20 +1393,21 @@ int launch_sq_rows(RowsArgs a, const void* indptr, const void* indices, int idx_
   {
     int need = ((int)(rb * dg / 0.6) + 15) & ~15;
     need = need < 64 ? 64 : need;
-    if (need < a.edge_cap) a.edge_cap = need;
+    if (direct) a.id_cap = need < 2048 ? need : 2048;
+    else a.id_cap = a.edge_cap = need < a.edge_cap ? need : a.edge_cap;
   }
-  const size_t lds = lut_bytes + (size_t)(rb + 4) * 4 + 64 + (size_t)rb * 4 + (size_t)a.edge_cap * 4 +
+  const size_t lds = lut_bytes + (size_t)(rb + 4) * 4 + 64 + (size_t)rb * 4 + (size_t)a.id_cap * 4 +
                      (size_t)a.edge_cap * a.pitch + 16;
   const int64_t grid = ceil_div(a.R, rb);
   if (grid > 0x7fffffffll) return fail(F2CGT_E_UNSUPPORTED, "%s: too many row blocks", what);
   if (plan_only()) {
     plan_record("sq_rows_kernel", grid, TB, (int64_t)lds, a.rows_per_block, a.fin_slots, TB >> a.lane_shift,
-                a.edge_cap);
+                a.id_cap);
     return 0;
   }
   const int half = (a.feat_dim % 4 == 0 && BITS < 4) ? 0 : (a.nt_out ? 2 : 1);
 #define F2CGT_ROWS_GO(I, H)                                                      \
-  sq_rows_kernel<BITS, AFFINE, I, TB, H><<<(unsigned)grid, TB, lds, st>>>(       \
+  sq_rows_kernel<BITS, AFFINE, I, TB, H, FLAT><<<(unsigned)grid, TB, lds, st>>>(       \
       a, static_cast<const I*>(indptr), static_cast<const I*>(indices), out)
 #define F2CGT_ROWS_IDX(I)                                                        \
   do {                                                                           \
@@ -1309,6 +1422,25 @@ int launch_sq_rows(RowsArgs a, const void* indptr, const void* indices, int idx_
 #undef F2CGT_ROWS_IDX
 #undef F2CGT_ROWS_GO
   return launch_status(what);
+}
+
+template <int BITS, bool AFFINE>
+int launch_sq_rows(RowsArgs a, const void* indptr, const void* indices, int idx_dtype, float* out, hipStream_t st,
+                   const char* what) {
+  // One codebook for all columns (what the encoder writes for scalar codes): no state belongs to a column, and the
+  // (row, column group) items go to 256 threads one after the other, so that no lane is idle where a row's groups do
+  // not divide the workgroup (602 columns: 151 groups on 256 threads).  60001 rows of 602 columns, 10 edges per row:
+  // 1 bit 187 -> 73 us, 2 bit 185 -> 77, 4 bit 185 -> 88, 8 bit 243 -> 119; 200000 rows of 128 columns: 1 bit
+  // 55 -> 38 us, 2 bit 57 -> 52, 4 bit 64 -> 59, 8 bit 88 -> 67.
+  if constexpr (!AFFINE) {
+    if (a.num_codebooks == 1)
+      return launch_sq_rows_sized<BITS, AFFINE, 256, true>(a, indptr, indices, idx_dtype, out, st, what);
+  }
+  // Several codebooks, or column parameters: a lane keeps its columns.  4- and 8-bit rows: 256 threads (twice the
+  // lanes in the decode + sum phase, which sets this kernel's time: 35.7 -> 31.9 us and 43.9 -> 34.8 us on the
+  // 2.5e5-row power-law block; 512 threads: 36.6 and 41.6); 1- and 2-bit rows are faster with 128 (27.7 against
+  // 30.8 us), 64 lose everywhere.
+  return launch_sq_rows_sized<BITS, AFFINE, BITS >= 4 ? 256 : 128, false>(a, indptr, indices, idx_dtype, out, st, what);
 }
 
 

@@ -112,6 +112,38 @@ def test_fused_sq_rows_of_an_even_number_of_columns_that_is_no_multiple_of_four(
             assert err <= RTOL * 3.0, (fanout, mode, float(err))
 
 
+@pytest.mark.parametrize("idx", [np.int64, np.int32])
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+def test_fused_log_sq_of_one_codebook_equals_that_codebook_given_per_slice(bits, idx):
+    """One codebook for all columns deals (row, column group) items to the lanes, several codebooks keep a column group
+    per lane: the same codebook repeated for every slice gives the same values in the same order, so the results are
+    equal bit for bit.  Rows without edges and rows past the ids a block keeps, one edge up to several hundred, staged
+    and direct code rows, plain and streamed stores, a negative, zero, infinite and NaN level."""
+    rng = np.random.default_rng(41 * bits + (idx == np.int32))
+    n, per = 3000, 8 // bits
+    for feat_dim in (64, 66, 100, 128, 260, 300, 602, 1030, 2040):
+        src_dim = (feat_dim + per - 1) // per
+        codes = rng.integers(0, 256, size=(n, src_dim), dtype=np.uint8)
+        stored = dev(codes.view(np.int8))
+        for rows, fanout, ragged in ((1, 5, False), (70, 1, True), (400, 12, True), (333, 40, True), (40, 700, True)):
+            indptr, indices = fixed_fanout(rng, rows, n, fanout, ragged)
+            indices[::5] = n - 1
+            ip, ix = dev(indptr.astype(idx)), dev(indices.astype(idx))
+            for level in (0.4, -0.4, 0.0, np.inf, np.nan) if rows == 70 else (0.4,):
+                cb = np.array([[0.01, 3.0, -6.643856, 1.5849625, level]], dtype=np.float32)
+                one = dev(cb)
+                slices = dev(np.repeat(cb, (feat_dim + 7) // 8, axis=0))
+                for mode in (capi.STORE_CACHED, capi.STORE_STREAM):
+                    was = capi.set_store_mode(mode)
+                    try:
+                        got = capi.sq_decompress_spmm_csr(stored, one, ip, ix, bits, (feat_dim + 7) // 8 * 8, feat_dim)
+                        want = capi.sq_decompress_spmm_csr(stored, slices, ip, ix, bits, 8, feat_dim)
+                        torch.cuda.synchronize()
+                    finally:
+                        capi.set_store_mode(was)
+                    assert np.array_equal(got.cpu().numpy(), want.cpu().numpy(), equal_nan=True), (feat_dim, rows, level, mode)
+
+
 @pytest.mark.parametrize("rows", [16383, 16384, 32767, 32768, 65535, 65536, 114687, 114688])
 def test_fused_sq_on_both_sides_of_the_rows_per_block_steps(rows):
     # launches below ~2000 workgroups shrink their row blocks in steps of 8 rows: the integer-accumulating
