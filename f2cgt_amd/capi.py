@@ -42,6 +42,8 @@ SIGNATURES = {
     "f2cgt_abs_order_stats": ([P, L, P, L, L, L, L, P, P, L, P, P], c_int),
     "f2cgt_pairwise_distance": ([P, P, P, L, L, L, I, P], c_int),
     "f2cgt_kmeans_predict": ([P, P, P, P, L, L, L, I, P], c_int),
+    "f2cgt_vq_encode_slices_covers": ([L, L], c_int),
+    "f2cgt_vq_encode_slices": ([P, L, L, P, P, L, L, L, L, L, I, P], c_int),
     "f2cgt_kmeans_update_workspace_bytes": ([L, L], c_int64),
     "f2cgt_kmeans_update": ([P, P, P, P, P, P, I, ctypes.c_float, P, L, L, L, L, P], c_int),
     "f2cgt_kmeans_update_static": ([P, P, P, P, P, P, I, ctypes.c_float, L, L, L, P], c_int),

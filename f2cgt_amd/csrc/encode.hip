@@ -37,6 +37,7 @@ namespace f2cgt {
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4_dword __attribute__((ext_vector_type(4), aligned(4)));   // loaded from any float's address
 
 // Absolute part of the near-tie bound: the matrix core flushes products (and, for the split form,
 // piece products 2^-8 and 2^-16 of the full one) that fall below the smallest normal fp32 number,
@@ -44,31 +45,34 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 constexpr float kTinyGap = 1e-33f;
 
 // ---- exact assignment of one row by a whole wave (fp64) ------------------------------
+// kx <= k: how many values the row has; it counts as zero in the dimensions after them.
 __device__ int exact_argmin_row(const float* __restrict__ xrow, const float* __restrict__ centers,
-                                int n, int k, int metric, int lane) {
+                                int n, int k, int kx, int metric, int lane) {
   double bestv = DBL_MAX;
   int besti = INT_MAX;
   double xn = 0.0;
   if (metric == F2CGT_METRIC_COSINE)
-    for (int t = 0; t < k; ++t) xn += (double)xrow[t] * (double)xrow[t];
+    for (int t = 0; t < kx; ++t) xn += (double)xrow[t] * (double)xrow[t];
   for (int c = lane; c < n; c += kWave) {
     const float* cr = centers + (int64_t)c * k;
     double d;
     if (metric == F2CGT_METRIC_COSINE) {
       double dot = 0.0, cn = 0.0;
-      for (int t = 0; t < k; ++t) {
+      for (int t = 0; t < kx; ++t) {
         dot += (double)xrow[t] * (double)cr[t];
         cn += (double)cr[t] * (double)cr[t];
       }
+      for (int t = kx; t < k; ++t) cn += (double)cr[t] * (double)cr[t];
       double den = sqrt(xn) * sqrt(cn);
       den = den > 1e-8 ? den : 1e-8;
       d = 1.0 - dot / den;
     } else {
       d = 0.0;
-      for (int t = 0; t < k; ++t) {
+      for (int t = 0; t < kx; ++t) {
         const double df = (double)xrow[t] - (double)cr[t];
         d += df * df;
       }
+      for (int t = kx; t < k; ++t) d += (double)cr[t] * (double)cr[t];
     }
     if (d < bestv) { bestv = d; besti = c; }
   }
@@ -133,7 +137,7 @@ __global__ __launch_bounds__(256) void predict_exact_kernel(const float* __restr
   const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t stride = (int64_t)gridDim.x * 4;
   for (int64_t row = wave; row < m; row += stride) {
-    const int best = exact_argmin_row(x + row * k, centers, n, k, metric, lane);
+    const int best = exact_argmin_row(x + row * k, centers, n, k, k, metric, lane);
     if (lane == 0) {
       if (lab64) lab64[row] = best;
       if (lab8) lab8[row] = (uint8_t)best;
@@ -296,7 +300,7 @@ __global__ __launch_bounds__(256) void predict_mfma_kernel(const float* __restri
       const int src = __ffsll((unsigned long long)todo) - 1;
       todo &= todo - 1;
       const int64_t rrow = tile * 32 + (src & 31);
-      const int exact = cosine ? exact_argmin_row(x + rrow * k, centers, n, k, metric, lane)
+      const int exact = cosine ? exact_argmin_row(x + rrow * k, centers, n, k, k, metric, lane)
                                : exact_argmin_row_l2_lds(x + rrow * k, cT, n, n_pad, KH, khalf, k, lane);
       if (lane == src) besti = exact;
     }
@@ -339,13 +343,13 @@ __device__ __forceinline__ void split3(float v, __bf16& p0, __bf16& p1, __bf16& 
 // row decides between them (fp64, from the arrays in HBM); with three or more that close the
 // function returns -1 - (its choice) and the caller evaluates every centre.
 template <int S>
-__device__ int exact_argmin_row_l2_pieces(const float* __restrict__ xrow, float* xs, const bf16x8* ap, int n, int n_ct,
-                                          int k, int lane, const float* mu, float cmax,
+__device__ __forceinline__ int exact_argmin_row_l2_pieces(const float* __restrict__ xrow, float* xs, const bf16x8* ap, int n, int n_ct,
+                                          int k, int kx, int lane, const float* mu, float cmax,
                                           const float* __restrict__ centers) {
   // the row goes through a wave-private LDS slot (16 S floats, zero padded) and the loops over the
   // 8-dimension chunks stay rolled: this rare path must not raise the kernel's register count
   const int piece_stride = n_ct * S * 64;                // operands per piece
-  if (lane < 16 * S) xs[lane] = lane < k ? xrow[lane] - mu[lane] : 0.f;
+  if (lane < 16 * S) xs[lane] = lane < k ? (lane < kx ? xrow[lane] : 0.f) - mu[lane] : 0.f;
   __builtin_amdgcn_wave_barrier();                       // LDS operations of one wave execute in order
   // fp32 centre values of chunk ch (dimensions [8 ch, 8 ch + 8)) of centre c: one operand per piece
   auto centre8 = [&](int c, int ch, float (&cv)[8]) {
@@ -507,7 +511,7 @@ __device__ int exact_argmin_row_l2_pieces(const float* __restrict__ xrow, float*
   // exactly two centres can be the nearest one of the original row: decide between them there
   double da = 0.0, db = 0.0;
   for (int t = lane; t < k; t += kWave) {
-    const double xv = (double)xrow[t];
+    const double xv = t < kx ? (double)xrow[t] : 0.0;
     const double ea = xv - (double)centers[(int64_t)besti * k + t], eb = xv - (double)centers[(int64_t)nexti * k + t];
     da += ea * ea;
     db += eb * eb;
@@ -529,10 +533,10 @@ __device__ int exact_argmin_row_l2_pieces(const float* __restrict__ xrow, float*
 // distance; those go through the fp32 dot product with all three pieces, and what that leaves is
 // evaluated exactly, in fp64 from the centres in HBM, by the formula of exact_argmin_row.  Needs every centre to have a direction (|c|^2 > 1e-12).
 template <int S>
-__device__ int exact_argmin_row_cosine_pieces(const float* __restrict__ xrow, float* xs, const bf16x8* ap,
+__device__ __forceinline__ int exact_argmin_row_cosine_pieces(const float* __restrict__ xrow, float* xs, const bf16x8* ap,
                                               const float* __restrict__ centers, int n, int n_ct, int k,
-                                              int lane, float cdev) {
-  if (lane < 16 * S) xs[lane] = lane < k ? xrow[lane] : 0.f;
+                                              int kx, int lane, float cdev) {
+  if (lane < 16 * S) xs[lane] = lane < kx ? xrow[lane] : 0.f;
   __builtin_amdgcn_wave_barrier();
   float xnorm2 = lane < 16 * S ? xs[lane] * xs[lane] : 0.f;
 #pragma unroll
@@ -581,7 +585,7 @@ __device__ int exact_argmin_row_cosine_pieces(const float* __restrict__ xrow, fl
   for (int off = 32; off >= 1; off >>= 1) s32max = fmaxf(s32max, __shfl_xor(s32max, off));
   const float floor32 = s32max - 1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) * sqrtf(xnorm2) * 1.001f - 1e-30f;
   double xn = 0.0;
-  for (int t = 0; t < k; ++t) xn += (double)xrow[t] * (double)xrow[t];
+  for (int t = 0; t < kx; ++t) xn += (double)xrow[t] * (double)xrow[t];
   double bestv = DBL_MAX;
   int besti = INT_MAX;
   for (int c = lane; c < n; c += kWave) {
@@ -589,10 +593,11 @@ __device__ int exact_argmin_row_cosine_pieces(const float* __restrict__ xrow, fl
     if (!(dot32(c) >= floor32)) continue;
     const float* cr = centers + (int64_t)c * k;
     double dot = 0.0, cn = 0.0;
-    for (int t = 0; t < k; ++t) {
+    for (int t = 0; t < kx; ++t) {
       dot += (double)xrow[t] * (double)cr[t];
       cn += (double)cr[t] * (double)cr[t];
     }
+    for (int t = kx; t < k; ++t) cn += (double)cr[t] * (double)cr[t];
     double den = sqrt(xn) * sqrt(cn);
     den = den > 1e-8 ? den : 1e-8;
     const double d = 1.0 - dot / den;
@@ -610,20 +615,48 @@ __device__ int exact_argmin_row_cosine_pieces(const float* __restrict__ xrow, fl
   return besti == INT_MAX ? 0 : besti;
 }
 
+// One launch labels several column slices of a table, each against its own centres (slices == 1: rows of ldx
+// floats, labels label_stride apart).  The grid is a multiple of 8 * slices workgroups then.
+struct SliceArgs {
+  int slices;
+  int feat_dim;            // columns of the table; the last slice may have fewer than k
+  int64_t ldx, label_stride;
+};
+
 // PW = false: labels of the nearest centre (KMeans.predict).  PW = true: the distance matrix itself
 // (pairwise_distance), dist[row * ldd + centre], from the same scores.  The squared L2 distance
 // does not change when one vector is subtracted from both arguments, and fl(v - mu) carries a
 // relative error of 2^-24 of the difference itself, so for L2 both modes first subtract the mean of
 // the centres from every x and centre: data far from the origin would otherwise lose most of the
 // expanded form's bits to cancellation (and send most rows to the exact re-evaluation).
-template <int S, int NB, bool PW>
-__global__ __launch_bounds__(256) void predict_split_kernel(const float* __restrict__ x,
+// SL: the slice form, with rows of any pitch and start (a kernel of its own: the row addressing costs the plain
+// form 2 to 3 %).
+template <int S, int NB, bool PW, bool SL>
+__global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kernel(const float* __restrict__ x,
                                                             const float* __restrict__ centers,
                                                             int64_t* __restrict__ lab64,
                                                             uint8_t* __restrict__ lab8, int64_t m,
                                                             int n, int k, int metric, int n_pad,
-                                                            float* __restrict__ dist, int64_t ldd) {
+                                                            float* __restrict__ dist, int64_t ldd,
+                                                            SliceArgs sl) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
+  int64_t share = blockIdx.x, shares = gridDim.x;
+  int slice = 0;
+  if (SL && sl.slices > 1) {
+    // Workgroups go round-robin to the 8 XCDs: with 8 shares side by side, the slices of a share run on one
+    // XCD, whose L2 then serves the lines of x that two slices have in common and joins their code bytes.
+    const int turn = blockIdx.x / (8 * sl.slices), at = blockIdx.x % (8 * sl.slices);
+    slice = at >> 3;
+    share = turn * 8 + (at & 7);
+    shares = gridDim.x / sl.slices;
+    x += slice * k;
+    centers += (int64_t)slice * n * k;
+    lab8 += slice;
+  }
+  int kx = SL ? sl.feat_dim - slice * k : k;                     // dimensions the rows have (zeros after them)
+  kx = kx < k ? kx : k;
+  const int64_t ldx = SL ? sl.ldx : k;
+  const int64_t ldl = SL ? sl.label_stride : 1;
   const int n_ct = n_pad >> 5;                                   // 32-centre tiles
   bf16x8* ap = reinterpret_cast<bf16x8*>(smem_raw);              // [3][n_ct][S][64]
   float* bias = reinterpret_cast<float*>(smem_raw + (size_t)3 * n_ct * S * 64 * 16);   // [n_pad]
@@ -883,10 +916,11 @@ __global__ __launch_bounds__(256) void predict_split_kernel(const float* __restr
   const float unit = 5.9604645e-8f * (float)(2 * (68 * S + k + 16));
   const float xscale = cosine ? -1.f : -2.f;
   const bool vec4 = (k % 8 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0);
+  const bool wide = kx >= 8;      // a row holds the eight values that an idle lane reads from row 0
   // A workgroup owns a contiguous share of the row groups and its four waves draw from it through
   // a counter in LDS: a wave held up by exact re-evaluations simply takes fewer groups.
-  const int64_t per_wg = (n_groups + gridDim.x - 1) / gridDim.x;
-  const int64_t wg_lo = (int64_t)blockIdx.x * per_wg;
+  const int64_t per_wg = (n_groups + shares - 1) / shares;
+  const int64_t wg_lo = share * per_wg;
   const int64_t wg_hi = wg_lo + per_wg < n_groups ? wg_lo + per_wg : n_groups;
   for (;;) {
     int draw = 0;
@@ -904,16 +938,32 @@ __global__ __launch_bounds__(256) void predict_split_kernel(const float* __restr
       for (int st = 0; st < S; ++st) {
         const int kk0 = 16 * st + 8 * g;
         float q[8];
-        if (vec4) {
+        if (!SL && vec4) {
           const bool in = valid && kk0 < k;                   // loads always issued, from row 0 when idle
           const float4* xp4 = reinterpret_cast<const float4*>(x + (in ? row * k + kk0 : 0));
           const float4 u = xp4[0], w = xp4[1];
           q[0] = u.x; q[1] = u.y; q[2] = u.z; q[3] = u.w; q[4] = w.x; q[5] = w.y; q[6] = w.z; q[7] = w.w;
 #pragma unroll
           for (int e = 0; e < 8; ++e) q[e] = in ? q[e] : 0.f;
-        } else {
+        } else if (!SL) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) q[e] = (valid && kk0 + e < k) ? x[row * k + kk0 + e] : 0.f;
+        }
+        if (SL && wide) {
+          // whole chunks: 16-byte loads, which rows of any width and start take (4-byte alignment)
+          const bool in = valid && kk0 + 8 <= kx;             // loads always issued, from row 0 when idle
+          const floatx4_dword* xp4 = reinterpret_cast<const floatx4_dword*>(x + (in ? row * ldx + kk0 : 0));
+          const floatx4_dword u = xp4[0], w = xp4[1];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { q[e] = in ? u[e] : 0.f; q[4 + e] = in ? w[e] : 0.f; }
+        }
+        if (SL && (!wide || (kx & 7))) {                              // the chunk that a row ends in
+          const bool part = valid && kk0 < kx && kk0 + 8 > kx;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            if (!wide) q[e] = 0.f;
+            if (part && kk0 + e < kx) q[e] = x[row * ldx + kk0 + e];
+          }
         }
         if (use_mu) {
 #pragma unroll
@@ -1115,14 +1165,14 @@ __global__ __launch_bounds__(256) void predict_split_kernel(const float* __restr
       while (td) {
         const int src = __ffsll((unsigned long long)td) - 1;
         td &= td - 1;
-        const int64_t rrow = grp * kGroupRows + 32 * b + (src & 31);
+        const float* xr = x + (grp * kGroupRows + 32 * b + (src & 31)) * ldx;
         int exact;
         if (!cosine) {
-          exact = exact_argmin_row_l2_pieces<S>(x + rrow * k, xs, ap, n, n_ct, k, lane, mu, cmax, centers);
-          if (exact < 0) exact = exact_argmin_row(x + rrow * k, centers, n, k, metric, lane);   // the original row decides
+          exact = exact_argmin_row_l2_pieces<S>(xr, xs, ap, n, n_ct, k, kx, lane, mu, cmax, centers);
+          if (exact < 0) exact = exact_argmin_row(xr, centers, n, k, kx, metric, lane);   // the original row decides
         }
-        else if (plain_cosine) exact = exact_argmin_row(x + rrow * k, centers, n, k, metric, lane);
-        else exact = exact_argmin_row_cosine_pieces<S>(x + rrow * k, xs, ap, centers, n, n_ct, k, lane, cdev);
+        else if (plain_cosine) exact = exact_argmin_row(xr, centers, n, k, kx, metric, lane);
+        else exact = exact_argmin_row_cosine_pieces<S>(xr, xs, ap, centers, n, n_ct, k, kx, lane, cdev);
 #pragma unroll
         for (int q = 0; q < NB; ++q) besti[q] = (b == q && lane == src) ? exact : besti[q];
       }
@@ -1131,8 +1181,8 @@ __global__ __launch_bounds__(256) void predict_split_kernel(const float* __restr
     for (int b = 0; b < NB; ++b) {
       const int64_t row = grp * kGroupRows + 32 * b + j;
       if (row < m && g == 0) {
-        if (lab64) lab64[row] = besti[b];
-        if (lab8) lab8[row] = (uint8_t)besti[b];
+        if (lab64) lab64[row * ldl] = besti[b];
+        if (lab8) lab8[row * ldl] = (uint8_t)besti[b];
       }
     }
   }
@@ -1371,7 +1421,7 @@ __global__ __launch_bounds__(256) void predict_tiled_kernel(const float* __restr
     const int again = s_count;
     for (int f = wave; f < again; f += 4) {
       const int64_t i = i0 + s_again[f];
-      const int lab = exact_argmin_row(x + i * k, centers, n, k, metric, lane);
+      const int lab = exact_argmin_row(x + i * k, centers, n, k, k, metric, lane);
       if (lane == 0) {
         if (lab64) lab64[i] = lab;
         if (lab8) lab8[i] = (uint8_t)lab;
@@ -1411,10 +1461,11 @@ int launch_mfma(const float* x, const float* centers, int64_t* l64, uint8_t* l8,
   return launch_status("kmeans_predict");
 }
 
-template <int S, int NB, bool PW = false>
+template <int S, int NB, bool PW = false, bool SL = false>
 int launch_split(const float* x, const float* centers, int64_t* l64, uint8_t* l8, int64_t m, int n, int k,
-                 int metric, int n_pad, size_t lds, hipStream_t st, float* dist = nullptr, int64_t ldd = 0) {
-  auto kern = predict_split_kernel<S, NB, PW>;
+                 int metric, int n_pad, size_t lds, hipStream_t st, float* dist = nullptr, int64_t ldd = 0,
+                 const SliceArgs* slices = nullptr) {
+  auto kern = predict_split_kernel<S, NB, PW, SL>;
   if (lds > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1433,8 +1484,41 @@ int launch_split(const float* x, const float* centers, int64_t* l64, uint8_t* l8
   }
   const int64_t need = ceil_div(ceil_div(m, 32 * NB), 4);
   const int64_t cap = (int64_t)num_cus() * cached_per_cu;
-  kern<<<(int)(need < cap ? need : cap), 256, lds, st>>>(x, centers, l64, l8, m, n, k, metric, n_pad, dist, ldd);
+  int64_t grid = need < cap ? need : cap;
+  SliceArgs sl{1, k, k, 1};
+  if constexpr (SL) {
+    sl = *slices;
+    if (sl.slices > 1) {
+      // the resident grid shared out over the slices, eight shares at least (one per XCD)
+      int64_t per = cap / sl.slices / 8 * 8;
+      const int64_t most = ceil_div(need, 8) * 8;
+      per = per < 8 ? 8 : per;
+      grid = (per < most ? per : most) * sl.slices;
+    }
+  }
+  kern<<<(int)grid, 256, lds, st>>>(x, centers, l64, l8, m, n, k, metric, n_pad, dist, ldd, sl);
   return launch_status(PW ? "pairwise_distance" : "kmeans_predict");
+}
+
+// split-bf16 path: up to 64 dimensions, operand pieces and biases within 96 KB of LDS
+size_t split_lds(int64_t n, int64_t k) {
+  const int64_t steps = ceil_div(k, 16), n_pad32 = ceil_div(n, 32) * 32;
+  return (size_t)(3 * (n_pad32 / 32) * steps * 64 * 16 + 2 * n_pad32 * 4 + 16 + 5 * 16 * steps * 4);
+}
+
+bool split_fits(int64_t n, int64_t k) { return k <= 64 && n <= 65536 && split_lds(n, k) <= 96 * 1024; }
+
+template <bool SL>
+int predict_split(const float* x, const float* centers, int64_t* l64, uint8_t* l8, int64_t m, int n, int k, int metric,
+                  hipStream_t st, const SliceArgs* sl = nullptr) {
+  const int n_pad = (int)ceil_div(n, 32) * 32;
+  const size_t lds = split_lds(n, k);
+  switch (ceil_div(k, 16)) {
+    case 1: return launch_split<1, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
+    case 2: return launch_split<2, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
+    case 3: return launch_split<3, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
+    default: return launch_split<4, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
+  }
 }
 
 }  // namespace
@@ -1498,20 +1582,7 @@ extern "C" int f2cgt_kmeans_predict(const float* x, const float* centers, int64_
   F2CGT_REQUIRE(x && centers && (labels_i64 || labels_u8), F2CGT_E_INVALID,
                 "kmeans_predict: null buffer");
   hipStream_t st = as_stream(stream);
-  {  // split-bf16 path: up to 64 dimensions, operand pieces and biases within 96 KB of LDS
-    const int steps = (int)ceil_div(k, 16);
-    const int n_pad32 = (int)ceil_div(n, 32) * 32;
-    const size_t lds = (size_t)3 * (n_pad32 / 32) * steps * 64 * 16 + (size_t)2 * n_pad32 * 4 + 16 +
-                       (size_t)5 * 16 * steps * 4;
-    if (steps <= 4 && lds <= 96 * 1024) {
-      switch (steps) {
-        case 1: return launch_split<1, 2>(x, centers, labels_i64, labels_u8, m, (int)n, (int)k, metric, n_pad32, lds, st);
-        case 2: return launch_split<2, 2>(x, centers, labels_i64, labels_u8, m, (int)n, (int)k, metric, n_pad32, lds, st);
-        case 3: return launch_split<3, 2>(x, centers, labels_i64, labels_u8, m, (int)n, (int)k, metric, n_pad32, lds, st);
-        default: return launch_split<4, 2>(x, centers, labels_i64, labels_u8, m, (int)n, (int)k, metric, n_pad32, lds, st);
-      }
-    }
-  }
+  if (split_fits(n, k)) return predict_split<false>(x, centers, labels_i64, labels_u8, m, (int)n, (int)k, metric, st);
   const int khalf = (int)((k + 1) / 2);
   int kh = pow2_ceil(khalf);
   if (kh < 4) kh = 4;
@@ -1537,4 +1608,27 @@ extern "C" int f2cgt_kmeans_predict(const float* x, const float* centers, int64_
   predict_exact_kernel<<<(int)(need < cap ? need : cap), 256, 0, st>>>(x, centers, labels_i64, labels_u8, m,
                                                                       (int)n, (int)k, metric);
   return launch_status("kmeans_predict");
+}
+
+extern "C" int f2cgt_vq_encode_slices_covers(int64_t n, int64_t k) {
+  return n > 0 && n <= 256 && k > 0 && split_fits(n, k) ? 1 : 0;
+}
+
+extern "C" int f2cgt_vq_encode_slices(const float* x, int64_t ldx, int64_t feat_dim, const float* codebooks, uint8_t* codes,
+                                      int64_t code_stride, int64_t m, int64_t slices, int64_t n, int64_t k, int metric,
+                                      void* stream) {
+  const char* what = "vq_encode_slices";
+  F2CGT_REQUIRE(m >= 0 && slices > 0 && n > 0 && k > 0 && feat_dim > 0, F2CGT_E_INVALID, "%s: sizes must be positive", what);
+  F2CGT_REQUIRE(f2cgt_vq_encode_slices_covers(n, k), F2CGT_E_UNSUPPORTED,
+                "%s: %lld centres of %lld columns are left to kmeans_predict, one slice at a time", what, (long long)n,
+                (long long)k);
+  F2CGT_REQUIRE(slices <= 65536 && feat_dim < (1 << 22), F2CGT_E_UNSUPPORTED, "%s: table too wide", what);
+  F2CGT_REQUIRE((slices - 1) * k < feat_dim, F2CGT_E_INVALID, "%s: a slice without columns", what);
+  F2CGT_REQUIRE(ldx >= feat_dim && code_stride >= slices, F2CGT_E_INVALID, "%s: rows overlap", what);
+  F2CGT_REQUIRE(metric == F2CGT_METRIC_L2 || metric == F2CGT_METRIC_COSINE, F2CGT_E_INVALID, "%s: unknown metric %d", what,
+                metric);
+  if (m == 0) return 0;
+  F2CGT_REQUIRE(x && codebooks && codes, F2CGT_E_INVALID, "%s: null buffer", what);
+  const SliceArgs sl{(int)slices, (int)feat_dim, ldx, code_stride};
+  return predict_split<true>(x, codebooks, nullptr, codes, m, (int)n, (int)k, metric, as_stream(stream), &sl);
 }

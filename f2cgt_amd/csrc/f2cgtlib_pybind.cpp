@@ -736,6 +736,28 @@ torch::Tensor vq_encode(torch::Tensor x, torch::Tensor centers, std::string metr
   return kmeans_predict_impl(x, centers, metric, true);
 }
 
+// Codes of all column slices of a table in one launch, into `out` (uint8 [m, slices]).  -> false, with nothing
+// written, for the calls that it does not take (the caller then goes slice by slice through KMeans.predict).
+bool vq_encode_slices(torch::Tensor x, torch::Tensor codebooks, torch::Tensor out, std::string metric) {
+  const bool plain = x.is_cuda() && x.device() == codebooks.device() && x.device() == out.device() && x.dim() == 2 &&
+                     codebooks.dim() == 3 && out.dim() == 2 && x.scalar_type() == torch::kFloat32 &&
+                     codebooks.scalar_type() == torch::kFloat32 && out.scalar_type() == torch::kUInt8;
+  if (!plain || x.size(1) < 1 || x.stride(1) != 1 || x.stride(0) < x.size(1) || out.size(0) != x.size(0) ||
+      out.size(1) != codebooks.size(0) || out.stride(1) != 1 || out.stride(0) < out.size(1))
+    return false;
+  const int64_t slices = codebooks.size(0), n = codebooks.size(1), k = codebooks.size(2);
+  if (!f2cgt_vq_encode_slices_covers(n, k) || slices < 1 || slices > 65536 || x.size(1) >= (1 << 22) ||
+      (slices - 1) * k >= x.size(1))
+    return false;
+  codebooks = codebooks.contiguous();
+  c10::DeviceGuard guard(x.device());
+  check_rc(f2cgt_vq_encode_slices(x.data_ptr<float>(), x.stride(0), x.size(1), codebooks.data_ptr<float>(),
+                                  out.data_ptr<uint8_t>(), out.stride(0), x.size(0), slices, n, k, metric_tag(metric),
+                                  current_stream()),
+           "vq_encode_slices");
+  return true;
+}
+
 }  // namespace
 
 // Output store policy of the SQ aggregation operators: "auto" (by output size), "stream"
@@ -789,6 +811,7 @@ PYBIND11_MODULE(F2CGTLib, m) {
       .def("abs_order_stats", &abs_order_stats, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"))
       .def("kmeans_predict", &kmeans_predict, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode", &vq_encode, py::arg("x"), py::arg("centers"), py::arg("metric"))
+      .def("vq_encode_slices", &vq_encode_slices, py::arg("x"), py::arg("codebooks"), py::arg("out"), py::arg("metric"))
       .def("fetch_rows", &fetch_rows, py::arg("table"), py::arg("index"), py::arg("hot") = py::none(),
            py::arg("slot_map") = py::none())
       .def("kmeans_update", &kmeans_update, py::arg("data"), py::arg("labels"), py::arg("centers"),

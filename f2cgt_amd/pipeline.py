@@ -254,9 +254,15 @@ def vq_compress(features, n_clusters, column_slice, hotness=None, codebooks=None
     else:
         raise NotImplementedError("more than 32767 centres do not fit the int16 code type")
     out = torch.empty((num_items, num_slice), dtype=dtype, device="cuda")
-    predictors = [capi.KMeans(codebooks[i].contiguous(), "cosine") for i in range(num_slice)]
+    predictors = None
     for start in range(0, num_items, batch_rows):
         end = min(start + batch_rows, num_items)
+        # float32 rows on the device and up to 256 centres: all slices in one launch, the rows read in place
+        if (tuple(codebooks.shape[2:]) == (column_slice,) and
+                capi.vq_encode_slices(features[start:end], codebooks, out[start:end], "cosine")):
+            continue
+        if predictors is None:
+            predictors = [capi.KMeans(codebooks[i].contiguous(), "cosine") for i in range(num_slice)]
         for i in range(num_slice):
             lo, hi = i * column_slice, min((i + 1) * column_slice, feat_dim)
             if hi <= lo:

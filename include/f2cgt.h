@@ -254,6 +254,15 @@ int f2cgt_kmeans_predict(const float* x, const float* centers, int64_t* labels_i
                          uint8_t* labels_u8, int64_t m, int64_t n, int64_t k, int metric,
                          void* stream);
 
+/* Codes of a whole feature table in one launch: column slice s (columns [s k, s k + k) of the rows; the last slice may
+ * have fewer, which count as zeros) against its own centres, as f2cgt_kmeans_predict labels it
+ * (examples/process_compress.py:234-292, one slice at a time).  x: row r starts ldx floats after row r - 1, ldx >=
+ * feat_dim; codebooks fp32 [slices, n, k]; codes uint8, row r at r * code_stride, code_stride >= slices.
+ * f2cgt_vq_encode_slices_covers: 1 where the shape is taken (n <= 256, k <= 64, centres within 96 KB of LDS), else 0. */
+int f2cgt_vq_encode_slices_covers(int64_t n, int64_t k);
+int f2cgt_vq_encode_slices(const float* x, int64_t ldx, int64_t feat_dim, const float* codebooks, uint8_t* codes,
+                           int64_t code_stride, int64_t m, int64_t slices, int64_t n, int64_t k, int metric, void* stream);
+
 /* One Lloyd iteration's centre update, after f2cgt_kmeans_predict has produced the labels.
  * Replaces the update half of the reference's two training loops: compute_new_centers and the
  * centre-shift test of examples/my_kmeans.py:87-113,128-147 (plain mean whatever the metric, a centre

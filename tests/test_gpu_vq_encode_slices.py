@@ -1,0 +1,65 @@
+"""Codes of a whole table in one launch (f2cgt_vq_encode_slices) against the oracle's labels of every column slice."""
+import numpy as np
+import pytest
+import torch
+
+import f2cgt_oracle as oc
+import f2cgt_amd
+from f2cgt_amd import pipeline
+
+pytestmark = pytest.mark.gpu
+
+
+def padded(table, s, k):
+    part = table[:, s * k:(s + 1) * k]
+    return np.ascontiguousarray(np.pad(part, ((0, 0), (0, k - part.shape[1]))))
+
+
+# m: below, at and beyond a wave's 64 rows, and more shares than rows; dim: a last slice of 1 to k columns, fewer than eight
+# columns in all, one slice; start / pitch: rows that begin at any float and leave a gap; n: one padded tile, all of it used
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("m,dim,k,n,start,pitch", [
+    (1, 3, 8, 5, 0, 3), (63, 16, 16, 32, 0, 16), (64, 100, 16, 256, 0, 100), (65, 33, 32, 33, 1, 37), (3000, 137, 32, 256, 3, 141),
+    (700, 96, 8, 200, 2, 99), (129, 40, 24, 256, 1, 41), (2500, 90, 48, 256, 0, 90), (500, 130, 64, 64, 1, 131), (70, 600, 8, 16, 0, 600),
+    (200, 17, 32, 7, 5, 23)])
+def test_vq_encode_slices(metric, m, dim, k, n, start, pitch):
+    print("case vq_encode_slices", metric, m, dim, k, n, start, pitch, flush=True)
+    rng = np.random.default_rng(m + dim + k)
+    slices = (dim + k - 1) // k
+    table = rng.standard_normal((m, dim)).astype(np.float32)
+    books = rng.standard_normal((slices, n, k)).astype(np.float32)           # nonzero also beyond the table's last column
+    flat = torch.zeros(m * pitch + start, device="cuda")
+    x = flat[start:].view(m, pitch)[:, :dim]
+    x.copy_(torch.from_numpy(table))
+    out = torch.full((m + 2, slices + 3), 77, dtype=torch.uint8, device="cuda")
+    assert f2cgt_amd.load().vq_encode_slices(x, torch.from_numpy(books).cuda(), out[1:m + 1, 1:slices + 1], metric)
+    got = out.cpu().numpy()
+    for s in range(slices):
+        want, near = oc.kmeans_predict(padded(table, s, k), books[s], metric)
+        assert np.array_equal(got[1:m + 1, 1 + s][~near], want[~near]) and near.mean() < 0.02
+    got[1:m + 1, 1:slices + 1] = 77
+    assert (got == 77).all()                                                 # nothing else is written
+
+
+def test_vq_encode_slices_leaves_other_calls():
+    lib = f2cgt_amd.load()
+    x, books = torch.randn((10, 20), device="cuda"), torch.randn((2, 16, 10), device="cuda")
+    out = torch.empty((10, 2), dtype=torch.uint8, device="cuda")
+    assert lib.vq_encode_slices(x, books, out, "cosine")
+    assert not lib.vq_encode_slices(x.double(), books, out, "cosine")
+    assert not lib.vq_encode_slices(x.t().contiguous().t(), books, out, "cosine")
+    assert not lib.vq_encode_slices(x, torch.randn((2, 300, 10), device="cuda"), out, "cosine")
+    assert not lib.vq_encode_slices(x, torch.randn((2, 16, 20), device="cuda"), out, "cosine")      # a slice without columns
+    assert not lib.vq_encode_slices(x[:1].expand(10, 20), books, out, "cosine")
+
+
+@pytest.mark.parametrize("dim,k,n", [(100, 16, 256), (45, 8, 40), (70, 70, 16)])
+def test_vq_compress_equals_its_slices(dim, k, n):
+    """One launch, the same rows from the host (slice by slice), and rows that are not contiguous: the same codes."""
+    rng = np.random.default_rng(dim)
+    x = torch.from_numpy(rng.standard_normal((1000, dim)).astype(np.float32))
+    books = torch.from_numpy(rng.standard_normal(((dim + k - 1) // k, n, k)).astype(np.float32)).cuda()
+    by_slice, _ = pipeline.vq_compress(x, n, k, codebooks=books)
+    for features in (x.cuda(), x.cuda().t().contiguous().t()):
+        codes, _ = pipeline.vq_compress(features, n, k, codebooks=books, batch_rows=600)
+        assert torch.equal(codes, by_slice)
