@@ -325,6 +325,52 @@ __global__ __launch_bounds__(256) void predict_mfma_kernel(const float* __restri
 // rounding bound of this evaluation are re-evaluated exactly in fp64.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
+// Three-way minimum of scores with the NaN behaviour of the instruction (the builtin minimum would first quieten
+// each operand with an instruction of its own).  A NaN ends in the row's exact evaluation wherever it comes out.
+__device__ __forceinline__ float min3_raw(float a, float b, float c) {
+  float d;
+  asm("v_min3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+  return d;
+}
+__device__ __forceinline__ float min_raw(float a, float b) {
+  float d;
+  asm("v_min_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+  return d;
+}
+__device__ __forceinline__ float max_raw(float a, float b) {
+  float d;
+  asm("v_max_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+  return d;
+}
+
+// Running (best, second) over the 16 scores of a tile.  A score carries its slot in its four lowest bits (one
+// v_and_or, a change below 2^-19 of it that the near-tie bound includes), so that the index needs no compare and
+// select of its own and the rest is a tree of three-way minima and medians: 39 instructions for 16 scores where
+// compare, two selects and a median took 64.
+__device__ __forceinline__ void argmin_update_packed(const floatx16& acc, int ct, float& best, float& second, int& bct) {
+  float p[16];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) p[v] = __int_as_float((__float_as_int(acc[v]) & ~15) | v);
+  float lo[6], mid[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    lo[i] = min3_raw(p[3 * i], p[3 * i + 1], p[3 * i + 2]);
+    mid[i] = __builtin_amdgcn_fmed3f(p[3 * i], p[3 * i + 1], p[3 * i + 2]);
+  }
+  lo[5] = p[15];
+  const float lo_a = min3_raw(lo[0], lo[1], lo[2]), mid_a = __builtin_amdgcn_fmed3f(lo[0], lo[1], lo[2]);
+  const float lo_b = min3_raw(lo[3], lo[4], lo[5]), mid_b = __builtin_amdgcn_fmed3f(lo[3], lo[4], lo[5]);
+  const float before = best;
+  const float behind_a = max_raw(best, lo_a);
+  best = min_raw(best, lo_a);
+  const float behind_b = max_raw(best, lo_b);
+  best = min_raw(best, lo_b);
+  const float s0 = min3_raw(mid[0], mid[1], mid[2]), s1 = min3_raw(mid[3], mid[4], mid_a);
+  second = min3_raw(second, s0, s1);
+  second = min3_raw(second, mid_b, min_raw(behind_a, behind_b));
+  bct = best < before ? ct : bct;
+}
+
 __device__ __forceinline__ void split3(float v, __bf16& p0, __bf16& p1, __bf16& p2) {
   p0 = (__bf16)v;
   float r = v - (float)p0;      // exact: the rounding error of a narrower format
@@ -640,6 +686,10 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
                                                             float* __restrict__ dist, int64_t ldd,
                                                             SliceArgs sl) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
+  // Scores that carry their slot: up to 16 dimensions, where the update is as long as the products (1e6 x 16 against
+  // 256 centres, cosine: 78 -> 68 us; L2: 78 -> 74).  From there on the tree's registers cost what its
+  // instructions save (32 dimensions: 118 us either way; 64: 138 -> 179).
+  constexpr bool kPacked = !PW && S == 1;
   int64_t share = blockIdx.x, shares = gridDim.x;
   int slice = 0;
   if (SL && sl.slices > 1) {
@@ -789,7 +839,8 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
     float sc = 1.f;
     if (cosine) sc = (float)(1.0 / sqrt(cn64 > 1e-60 ? cn64 : 1e-60));
     inv[jj] = sc;
-    bias[jj] = jj >= n ? INFINITY : (cosine ? 0.f : cn);
+    // padding: finite where the lowest bits of a score are its slot
+    bias[jj] = jj >= n ? (kPacked ? FLT_MAX : INFINITY) : (cosine ? 0.f : cn);
     if (jj < n && !cosine) atomicMax(cmax_bits, __float_as_int(cn));
     if (jj < n && cosine && !(cn > 1e-12f)) atomicOr(cmax_bits + 1, 1);   // a centre without a direction
     if (PW && jj < n && cosine) atomicMin(cmax_bits + 3, __float_as_int(cn));
@@ -987,11 +1038,14 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
     for (int b = 0; b < NB; ++b) { best[b] = INFINITY; second[b] = INFINITY; bv[b] = 0; bct[b] = 0; }
     for (int ct = 0; ct < n_ct; ++ct) {
       floatx16 bz;
-      const float* bp = bias + ct * 32 + 4 * g;
+      const bool biased = !kPacked || !cosine || ct * 32 + 32 > n;   // cosine: only a tile with padding has any
+      if (biased) {
+        const float* bp = bias + ct * 32 + 4 * g;
 #pragma unroll
-      for (int v4 = 0; v4 < 4; ++v4) {
-        const float4 t4 = *reinterpret_cast<const float4*>(bp + 8 * v4);
-        bz[4 * v4] = t4.x; bz[4 * v4 + 1] = t4.y; bz[4 * v4 + 2] = t4.z; bz[4 * v4 + 3] = t4.w;
+        for (int v4 = 0; v4 < 4; ++v4) {
+          const float4 t4 = *reinterpret_cast<const float4*>(bp + 8 * v4);
+          bz[4 * v4] = t4.x; bz[4 * v4 + 1] = t4.y; bz[4 * v4 + 2] = t4.z; bz[4 * v4 + 3] = t4.w;
+        }
       }
       bf16x8 a[3][S];
 #pragma unroll
@@ -1124,9 +1178,12 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
       } else {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
+          if (biased) {
 #pragma unroll
-          for (int v = 0; v < 16; ++v) acc[b][v] += bz[v];
-          argmin_update(acc[b], ct * 32, best[b], second[b], bv[b], bct[b]);
+            for (int v = 0; v < 16; ++v) acc[b][v] += bz[v];
+          }
+          if constexpr (kPacked) argmin_update_packed(acc[b], ct * 32, best[b], second[b], bct[b]);
+          else argmin_update(acc[b], ct * 32, best[b], second[b], bv[b], bct[b]);
         }
       }
     }
@@ -1136,7 +1193,8 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const bool valid = grp * kGroupRows + 32 * b + j < m;
-      int bi = bct[b] + 8 * (bv[b] >> 2) + 4 * g + (bv[b] & 3);
+      const int slot = kPacked ? __float_as_int(best[b]) & 15 : bv[b];
+      int bi = bct[b] + 8 * (slot >> 2) + 4 * g + (slot & 3);
       float bs = best[b], sd = second[b];
       {  // merge the two halves of the wave (same x row, disjoint centres)
         const float ob = __shfl_xor(bs, 32);
@@ -1153,8 +1211,14 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
       // cosine: the evaluation's share shrinks with the operands, the rounding of c / |c| (norm in
       // fp64, one rounding for 1 / |c|, one for the product, one for - m: 3 units, doubled) does not
       const float scale = cosine ? sqrtf(xn[b]) * (cdev + 3.5762787e-7f / unit) : xn[b] + cmax;
+      float bound = unit * scale + kTinyGap;
+      bool ask = false;
+      if (kPacked) {      // the slots: 2^-19 of each of the two; padding leads only where every real score has overflowed
+        bound += 1.92e-6f * (fabsf(bs) + fabsf(sd));
+        ask = bi >= n;
+      }
       besti[b] = bi;
-      todo[b] = __ballot(valid && g == 0 && !((sd - bs) > unit * scale + kTinyGap));
+      todo[b] = __ballot(valid && g == 0 && (ask || !((sd - bs) > bound)));
     }
     // exact re-evaluation of the flagged rows: one copy of the code, whichever tile the row is in
 #pragma nounroll

@@ -5,7 +5,7 @@ import torch
 
 import f2cgt_oracle as oc
 import f2cgt_amd
-from f2cgt_amd import pipeline
+from f2cgt_amd import capi, pipeline
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +63,19 @@ def test_vq_compress_equals_its_slices(dim, k, n):
     for features in (x.cuda(), x.cuda().t().contiguous().t()):
         codes, _ = pipeline.vq_compress(features, n, k, codebooks=books, batch_rows=600)
         assert torch.equal(codes, by_slice)
+
+
+@pytest.mark.parametrize("metric", ["l2", "cosine"])
+@pytest.mark.parametrize("n,k", [(2, 4), (34, 8), (100, 13), (256, 16), (254, 16), (256, 17)])
+def test_kmeans_predict_close_pairs(metric, n, k):
+    """Centres in pairs 2^-10 to 2^-15 of their size apart: up to 16 dimensions the lowest four bits of a score are its slot,
+    which changes scores by as much as what tells the two of a pair apart, and some of the slots are padding."""
+    rng = np.random.default_rng(n + k)
+    x = rng.standard_normal((4000, k)).astype(np.float32)
+    c = rng.standard_normal((n, k)).astype(np.float32)
+    c[1::2] = c[0::2] * (1 + rng.choice([-1, 1], (n // 2, k)) * 2.0 ** -rng.integers(10, 16, (n // 2, 1))).astype(np.float32)
+    want, near = oc.kmeans_predict(x, c, metric)
+    got = capi.kmeans_predict(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), metric).cpu().numpy()
+    # a cosine gap is about 2^-j / sqrt(k) wide, the oracle's near-ties are those below 1e-6: 7 % of the rows of one pair in
+    # 4 dimensions, 1 to 3 % where the rows spread over many pairs
+    assert near.mean() < 0.1 and np.array_equal(got[~near], want[~near])
