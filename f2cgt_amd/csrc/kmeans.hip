@@ -7,9 +7,12 @@
 // empty clusters keep the previous centre) and :100-111 (centre shift and stopping rule);
 // raft's kmeans::fit (src/kmeans.cu:61-75) stops on the squared form of the same shift.
 //
-// The partial sums are scratch memory beyond inputs and outputs (n * k floats and n counters):
-// f2cgt_kmeans_update takes them from a workspace the caller passes, f2cgt_kmeans_update_static
-// from a device array of this file (for callers that cannot allocate).
+// The partial sums are scratch memory beyond inputs and outputs.  f2cgt_kmeans_update takes them from a
+// workspace the caller passes: up to 256 workgroups each leave their own n * k sums and n counters there, which
+// one workgroup per centre adds up, moves the centre and counts itself in; the last one to arrive decides about
+// the stop.  f2cgt_kmeans_update_static uses a device array of this file (for callers that cannot allocate),
+// which has room for one set of sums: all workgroups add into it in memory, as they do from a workspace when
+// n * k does not fit LDS.
 #include "common.hpp"
 
 namespace f2cgt {
@@ -17,6 +20,9 @@ namespace {
 
 constexpr int kKmThreads = 256;
 constexpr int kKmLdsFloats = 12 * 1024;   // per-workgroup partial sums kept in LDS up to this many entries
+constexpr int kKmParts = 256;             // sets of partial sums in a workspace: one workgroup per CU
+constexpr int kKmPartThreads = 1024;
+constexpr int kKmBatch = 8;               // values per thread in flight
 
 // Scratch of the allocation-free entry point: 65536 sums and 4096 counters, 272 KB that every device
 // the library runs on holds until the process ends.  The name is a host-side stand-in, not a device
@@ -130,13 +136,135 @@ __global__ __launch_bounds__(kKmThreads) void km_finalize_kernel(KmArgs a) {
 
 // Decides, on the device, whether the centres just written are final (so that a training loop
 // needs no host read-back per iteration: every later step sees the flag and does nothing).
-__global__ void km_decide_kernel(KmArgs a) {
+__device__ void km_decide(const KmArgs& a, float sum, float sq) {
   if (a.stop == nullptr || *a.stop != 0 || a.rule == 0) return;
-  const float s = a.rule == 1 ? a.shift[1] : a.shift[0] * a.shift[0];
+  const float s = a.rule == 1 ? sq : sum * sum;
   // a shift that is not a number never passes `s < tol`: flag it (2) so that the loop ends and the
   // caller can tell (examples/my_kmeans.py:108-109 gives up on such a fit)
   if (s != s) *a.stop = 2;
   else if (s < a.tol) *a.stop = 1;
+}
+
+__global__ void km_decide_kernel(KmArgs a) { km_decide(a, a.shift[0], a.shift[1]); }
+
+// Partial sums of a workgroup's rows, left in the workspace: set blockIdx.x of n * k sums and n counters.
+// The kernel is a latency chain (label, value, LDS add), not bandwidth: 1024 threads with eight values each in
+// flight take a workgroup's share of a 150 000 x 16 step (256 centres) in two rounds, and plain stores of the sums
+// replace the 138 device-wide adds per sum that the workgroups used to queue for.  Clear and accumulate 40 us
+// before, 18 now; finalize and decide 13.7, km_merge_kernel 11.5.
+__global__ __launch_bounds__(kKmPartThreads) void km_partial_kernel(KmArgs a, uint32_t* arrived) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (km_stopped(a)) return;
+  float* s_sum = reinterpret_cast<float*>(smem);
+  const int entries = a.n * a.k, words = entries + a.n;
+  uint32_t* s_cnt = reinterpret_cast<uint32_t*>(s_sum + entries);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *arrived = 0u;
+  for (int i = threadIdx.x; i < words; i += kKmPartThreads) reinterpret_cast<uint32_t*>(smem)[i] = 0u;
+  __syncthreads();
+  const int64_t row0 = (int64_t)blockIdx.x * a.rows_per_block;
+  const int64_t left = a.m - row0;
+  const int nrows = (int)(left < a.rows_per_block ? (left > 0 ? left : 0) : a.rows_per_block);
+  const float* x = a.x + row0 * a.k;
+  const int step_r = kKmPartThreads / a.k, step_c = kKmPartThreads - step_r * a.k;
+  int r = threadIdx.x / a.k, col = threadIdx.x - r * a.k;
+  while (r < nrows) {
+    float v[kKmBatch];
+    int at[kKmBatch], cnt_at[kKmBatch];
+#pragma unroll
+    for (int u = 0; u < kKmBatch; ++u) {
+      const bool in = r < nrows;
+      const int rr = in ? r : 0;                       // row 0 of the share: there is one, the loop has begun
+      const int c = km_label(a, row0 + rr);
+      v[u] = x[(int64_t)rr * a.k + col];
+      at[u] = in ? c * a.k + col : -1;
+      cnt_at[u] = in && col == 0 ? c : -1;
+      r += step_r;
+      col += step_c;
+      if (col >= a.k) { col -= a.k; ++r; }
+    }
+#pragma unroll
+    for (int u = 0; u < kKmBatch; ++u) {
+      if (at[u] >= 0) add_f32<true>(s_sum + at[u], v[u]);
+      if (cnt_at[u] >= 0) atomicAdd(s_cnt + cnt_at[u], 1u);
+    }
+  }
+  __syncthreads();
+  uint32_t* part = reinterpret_cast<uint32_t*>(a.sums) + (int64_t)blockIdx.x * words;
+  for (int i = threadIdx.x; i < words; i += kKmPartThreads) part[i] = reinterpret_cast<const uint32_t*>(smem)[i];
+}
+
+// One workgroup per centre: adds up its sums over the `parts` sets, writes the new centre and its squared shift;
+// the workgroup that arrives last adds the shifts in order and applies the stop rule.
+__global__ __launch_bounds__(kKmThreads) void km_merge_kernel(KmArgs a, int parts, float* moves, uint32_t* arrived) {
+  if (km_stopped(a)) return;
+  __shared__ float s_part[kKmThreads];
+  __shared__ float s_d2[kKmThreads / kWave];
+  __shared__ uint32_t s_cnt[kKmThreads / kWave];
+  __shared__ int s_last;
+  const int c = blockIdx.x, t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
+  const int64_t words = (int64_t)a.n * a.k + a.n;
+  uint32_t cnt = 0;
+  for (int p = t; p < parts; p += kKmThreads) cnt += reinterpret_cast<const uint32_t*>(a.sums)[p * words + (int64_t)a.n * a.k + c];
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off);
+  if (lane == 0) s_cnt[wv] = cnt;
+  __syncthreads();
+  cnt = 0;
+#pragma unroll
+  for (int w = 0; w < kKmThreads / kWave; ++w) cnt += s_cnt[w];
+  const float members = (float)cnt;
+  const int cols = a.k < kKmThreads ? a.k : kKmThreads, side = kKmThreads / cols;   // sets read side by side
+  const int col = t % cols, p0 = t / cols;
+  float d2 = 0.f;
+  for (int j0 = 0; j0 < a.k; j0 += cols) {
+    float s = 0.f;
+    if (p0 < side && j0 + col < a.k) {
+      const float* from = a.sums + (int64_t)c * a.k + j0 + col;
+#pragma unroll 8
+      for (int p = p0; p < parts; p += side) s += from[p * words];
+    }
+    s_part[t] = s;
+    __syncthreads();
+    if (t < cols && j0 + t < a.k && cnt > 0u) {
+      float sum = 0.f;
+      for (int q = 0; q < side; ++q) sum += s_part[q * cols + t];
+      float* centre = a.centers + (int64_t)c * a.k + j0 + t;
+      const float now = sum / members;
+      const float d = now - *centre;
+      d2 += d * d;
+      *centre = now;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) d2 += __shfl_xor(d2, off);
+  if (lane == 0) s_d2[wv] = d2;
+  __syncthreads();
+  if (t == 0) {
+    d2 = 0.f;
+    for (int w = 0; w < kKmThreads / kWave; ++w) d2 += s_d2[w];
+    // device-wide: the workgroup that reads the shifts may run behind another L2
+    __hip_atomic_store(moves + c, d2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)a.n - 1u;
+  }
+  __syncthreads();
+  if (!s_last || t >= kWave) return;
+  float sum = 0.f, sq = 0.f;
+  for (int i = lane; i < a.n; i += kWave) {
+    const float m2 = __hip_atomic_load(moves + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sum += sqrtf(m2);
+    sq += m2;
+  }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    sum += __shfl_xor(sum, off);
+    sq += __shfl_xor(sq, off);
+  }
+  if (lane == 0) {
+    a.shift[0] = sum;
+    a.shift[1] = sq;
+    km_decide(a, sum, sq);
+  }
 }
 
 int km_check(const char* what, const float* x, const int64_t* l64, const uint8_t* l8, float* centers, float* shift,
@@ -149,6 +277,26 @@ int km_check(const char* what, const float* x, const int64_t* l64, const uint8_t
   F2CGT_REQUIRE(centers != nullptr && shift != nullptr && (m == 0 || x != nullptr), F2CGT_E_INVALID,
                 "%s: null buffer", what);
   return 0;
+}
+
+bool km_by_parts(int64_t n, int64_t k) { return n * k + n <= kKmLdsFloats; }
+
+// The workspace of km_run_parts: kKmParts sets of sums and counters, the centres' shifts, the arrival counter.
+int64_t km_parts_words(int64_t n, int64_t k) { return kKmParts * (n * k + n) + n + 1; }
+
+int km_run_parts(const char* what, KmArgs a, hipStream_t st) {
+  const int64_t words = (int64_t)a.n * a.k + a.n;
+  // a set of sums for every 64 rows at least: fewer cost more to add up than to find
+  int64_t rpb = ceil_div(a.m, (int64_t)kKmParts);
+  rpb = rpb < 64 ? 64 : rpb;
+  if (rpb > 0x7fffffff / 2) return fail(F2CGT_E_UNSUPPORTED, "%s: too many rows", what);
+  a.rows_per_block = (int)rpb;
+  const int parts = (int)(a.m > 0 ? ceil_div(a.m, rpb) : 1);
+  float* moves = a.sums + kKmParts * words;
+  uint32_t* arrived = reinterpret_cast<uint32_t*>(moves + a.n);
+  km_partial_kernel<<<parts, kKmPartThreads, (size_t)words * 4, st>>>(a, arrived);
+  km_merge_kernel<<<(unsigned)a.n, kKmThreads, 0, st>>>(a, parts, moves, arrived);
+  return launch_status(what);
 }
 
 int km_run(const char* what, KmArgs a, hipStream_t st) {
@@ -182,7 +330,8 @@ using namespace f2cgt;
 
 extern "C" int64_t f2cgt_kmeans_update_workspace_bytes(int64_t n, int64_t k) {
   if (n <= 0 || k <= 0) return 0;
-  return ((n * k + n) * 4 + 255) / 256 * 256;
+  const int64_t words = km_by_parts(n, k) ? km_parts_words(n, k) : n * k + n;
+  return (words * 4 + 255) / 256 * 256;
 }
 
 extern "C" int f2cgt_kmeans_update(const float* x, const int64_t* labels_i64, const uint8_t* labels_u8,
@@ -200,6 +349,7 @@ extern "C" int f2cgt_kmeans_update(const float* x, const int64_t* labels_i64, co
   a.sums = static_cast<float*>(workspace);
   a.counts = reinterpret_cast<uint32_t*>(a.sums + n * k);
   a.m = m; a.n = (int)n; a.k = (int)k; a.rule = stop_rule; a.tol = tol;
+  if (km_by_parts(n, k)) return km_run_parts(what, a, as_stream(stream));
   return km_run(what, a, as_stream(stream));
 }
 

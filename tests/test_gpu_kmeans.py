@@ -48,6 +48,24 @@ def test_update_step_vs_oracle(m, n, k, u8):
     assert np.isclose(sh[0], s_abs, rtol=1e-4) and np.isclose(sh[1], s_sq, rtol=1e-4)
 
 
+# sets of partial sums: one, an uneven last one, none full; columns below, at and beyond the 256 that the merge takes in one
+# pass and the 1024 threads that the accumulation steps by
+@pytest.mark.parametrize("m,n,k", [(1, 4, 8), (63, 3, 1), (65, 7, 255), (300, 5, 256), (129, 9, 257), (200, 4, 1024), (131, 3, 1500),
+                                   (16385, 100, 12), (40000, 256, 47)])
+def test_update_step_by_partial_sums(m, n, k):
+    print("case kmeans_update m=%d n=%d k=%d" % (m, n, k), flush=True)
+    rng = np.random.default_rng(m + n + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    centers = rng.standard_normal((n, k)).astype(np.float32)
+    labels = rng.integers(0, max(1, n - 1), size=m)
+    want, s_abs, s_sq = oc.kmeans_update(x, labels, centers)
+    c = dev(centers)
+    shift = capi.kmeans_update(dev(x), dev(labels.astype(np.int64)), c).cpu().numpy()
+    assert np.allclose(c.cpu().numpy(), want, rtol=RTOL, atol=RTOL)
+    assert np.allclose(shift, [s_abs, s_sq], rtol=1e-4, atol=1e-6)
+
+
+
 def test_update_step_stop_flag_and_rules():
     rng = np.random.default_rng(5)
     x = rng.standard_normal((4000, 8)).astype(np.float32)
