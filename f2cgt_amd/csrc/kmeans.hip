@@ -281,6 +281,8 @@ int km_check(const char* what, const float* x, const int64_t* l64, const uint8_t
 
 bool km_by_parts(int64_t n, int64_t k) { return n * k + n <= kKmLdsFloats; }
 
+int64_t km_bytes(int64_t words) { return (words * 4 + 255) / 256 * 256; }
+
 // The workspace of km_run_parts: kKmParts sets of sums and counters, the centres' shifts, the arrival counter.
 int64_t km_parts_words(int64_t n, int64_t k) { return kKmParts * (n * k + n) + n + 1; }
 
@@ -330,8 +332,7 @@ using namespace f2cgt;
 
 extern "C" int64_t f2cgt_kmeans_update_workspace_bytes(int64_t n, int64_t k) {
   if (n <= 0 || k <= 0) return 0;
-  const int64_t words = km_by_parts(n, k) ? km_parts_words(n, k) : n * k + n;
-  return (words * 4 + 255) / 256 * 256;
+  return km_bytes(km_by_parts(n, k) ? km_parts_words(n, k) : n * k + n);
 }
 
 extern "C" int f2cgt_kmeans_update(const float* x, const int64_t* labels_i64, const uint8_t* labels_u8,
@@ -340,16 +341,16 @@ extern "C" int f2cgt_kmeans_update(const float* x, const int64_t* labels_i64, co
                                    void* stream) {
   const char* what = "kmeans_update";
   if (int rc = km_check(what, x, labels_i64, labels_u8, centers, shift, m, n, k, stop_rule)) return rc;
-  F2CGT_REQUIRE(workspace != nullptr && workspace_bytes >= f2cgt_kmeans_update_workspace_bytes(n, k) &&
-                    aligned(workspace, 16),
+  // room for one set of sums is enough: all workgroups then add into it
+  F2CGT_REQUIRE(workspace != nullptr && workspace_bytes >= km_bytes(n * k + n) && aligned(workspace, 16),
                 F2CGT_E_INVALID, "%s: workspace of %lld bytes (16-byte aligned) needed", what,
-                (long long)f2cgt_kmeans_update_workspace_bytes(n, k));
+                (long long)km_bytes(n * k + n));
   KmArgs a{};
   a.x = x; a.labels_i64 = labels_i64; a.labels_u8 = labels_u8; a.centers = centers; a.shift = shift; a.stop = stop;
   a.sums = static_cast<float*>(workspace);
   a.counts = reinterpret_cast<uint32_t*>(a.sums + n * k);
   a.m = m; a.n = (int)n; a.k = (int)k; a.rule = stop_rule; a.tol = tol;
-  if (km_by_parts(n, k)) return km_run_parts(what, a, as_stream(stream));
+  if (km_by_parts(n, k) && workspace_bytes >= f2cgt_kmeans_update_workspace_bytes(n, k)) return km_run_parts(what, a, as_stream(stream));
   return km_run(what, a, as_stream(stream));
 }
 

@@ -273,7 +273,8 @@ int f2cgt_vq_encode_slices(const float* x, int64_t ldx, int64_t feat_dim, const 
  * sets it when stop_rule says the centres are final (1: sum_c |dc|^2 < tol, raft's rule; 2:
  * (sum_c |dc|)^2 < tol, the rule of examples/my_kmeans.py:105; 0: never) -- a training loop can then
  * run without reading anything back per iteration.  workspace: device scratch for the partial sums,
- * at least f2cgt_kmeans_update_workspace_bytes(n, k) bytes, 16-byte aligned, contents irrelevant.
+ * f2cgt_kmeans_update_workspace_bytes(n, k) bytes, 16-byte aligned, contents irrelevant (4 (n k + n) bytes, rounded up
+ * to 256, are enough for the slower form that adds into one set of sums).
  * The sums are fp32 atomic adds: their last bits depend on the order the hardware takes them in. */
 int64_t f2cgt_kmeans_update_workspace_bytes(int64_t n, int64_t k);
 int f2cgt_kmeans_update(const float* x, const int64_t* labels_i64, const uint8_t* labels_u8, float* centers,

@@ -66,6 +66,22 @@ def test_update_step_by_partial_sums(m, n, k):
 
 
 
+def test_update_step_with_room_for_one_set_of_sums():
+    rng = np.random.default_rng(11)
+    m, n, k = 5000, 64, 16
+    words = n * k + n
+    assert capi.lib().f2cgt_kmeans_update_workspace_bytes(n, k) > words * 4
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    labels = rng.integers(0, n, m)
+    start = rng.normal(size=(n, k)).astype(np.float32)
+    small = torch.empty(((words * 4 + 255) // 256 * 256,), dtype=torch.uint8, device="cuda")
+    got = dev(start)
+    capi.kmeans_update(dev(x), dev(labels.astype(np.int64)), got, workspace=small)
+    want = np.stack([x[labels == c].astype(np.float64).mean(axis=0) for c in range(n)])
+    # about 80 rows a centre, |x| < 6: 80 roundings of sums below 500 and the division
+    assert np.abs(got.cpu().numpy() - want).max() < 80 * 500 * 2.0 ** -24 / 40
+
+
 def test_update_step_stop_flag_and_rules():
     rng = np.random.default_rng(5)
     x = rng.standard_normal((4000, 8)).astype(np.float32)
