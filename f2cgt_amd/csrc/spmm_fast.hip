@@ -1056,11 +1056,14 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
   const int t = threadIdx.x;
   const int64_t row0 = (int64_t)blockIdx.x * a.rows_per_block;
   const int nrows = (int)((a.R - row0) < a.rows_per_block ? (a.R - row0) : a.rows_per_block);
-  int64_t e0 = (int64_t)indptr[row0];
+  int64_t e0 = (int64_t)indptr[row0], e1 = (int64_t)indptr[row0 + nrows];
   e0 = e0 < 0 ? 0 : (e0 > a.E ? a.E : e0);
+  e1 = e1 < e0 ? e0 : (e1 > a.E ? a.E : e1);
   for (int i = t; i <= nrows; i += TB) {
+    // offsets that decrease inside the block: no row reaches past the block's last edge, so that every position a
+    // row walks below has its id (and its code row) in LDS where the block keeps them
     int64_t v = (int64_t)indptr[row0 + i];
-    v = v < e0 ? e0 : (v > a.E ? a.E : v);
+    v = v < e0 ? e0 : (v > e1 ? e1 : v);
     s_ptr[i] = (int)(v - e0 > 0x7fffffff ? 0x7fffffff : v - e0);
   }
   if (t < 16) s_cnt[t] = 0;

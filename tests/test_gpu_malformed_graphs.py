@@ -1,0 +1,49 @@
+"""Row offsets that decrease: sums of the rows concerned are wrong, nothing is read outside the operands, and blocks of rows
+with ordinary offsets keep their results."""
+import numpy as np
+import pytest
+import torch
+
+import f2cgt_oracle as oc
+from f2cgt_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def graph(rng, rows, fanout, n):
+    """Rows of `fanout` edges; in the middle third two offsets of every eight are replaced by one far ahead and one
+    behind.  -> indptr, indices, the rows at least 64 (the largest block) away from a replaced offset."""
+    indptr = np.arange(rows + 1, dtype=np.int64) * fanout
+    lo, hi = rows // 3 // 64 * 64, 2 * rows // 3 // 64 * 64
+    for r in range(lo, hi, 8):
+        indptr[r + 2] = min(indptr[r + 2] + 40 * fanout, rows * fanout)
+        indptr[r + 5] = max(indptr[r + 5] - 40 * fanout, 0)
+    sound = np.ones(rows, dtype=bool)
+    sound[max(0, lo - 64):hi + 64] = False
+    return indptr, rng.integers(0, n, size=rows * fanout), sound
+
+
+@pytest.mark.parametrize("idx", [np.int64, np.int32])
+@pytest.mark.parametrize("bits", [1, 2, 4, 8])
+@pytest.mark.parametrize("books", [1, 3])
+def test_log_sq_with_decreasing_offsets(bits, books, idx):
+    rng = np.random.default_rng(bits + 10 * books)
+    n = 3000
+    cb = np.repeat(np.array([[0.01, 3.0, -6.643856, 1.5849625, 0.4]], dtype=np.float32), books, axis=0)
+    for feat_dim in (64, 66, 300, 602):
+        column_slice = (-(-feat_dim // books) + 7) // 8 * 8
+        codes = rng.integers(0, 256, size=(n, (feat_dim * bits + 7) // 8), dtype=np.uint8)
+        stored = codes.view(np.int8) if bits == 8 else codes
+        for rows, fanout in ((900, 1), (900, 10), (600, 40), (400, 300)):
+            print("case log sq bits=%d books=%d dim=%d rows=%d fanout=%d" % (bits, books, feat_dim, rows, fanout), flush=True)
+            indptr, indices, sound = graph(rng, rows, fanout, n)
+            got = capi.sq_decompress_spmm_csr(dev(stored), dev(cb), dev(indptr.astype(idx)), dev(indices.astype(idx)), bits,
+                                              column_slice, feat_dim)
+            torch.cuda.synchronize()
+            plain = np.arange(rows + 1, dtype=np.int64) * fanout
+            want = oc.sq_decompress_spmm_csr(stored, cb, plain, indices, bits, column_slice, feat_dim)
+            assert sound.any() and np.allclose(got.cpu().numpy()[sound], want[sound], rtol=1e-5, atol=3e-5)
