@@ -634,7 +634,9 @@ __global__ __launch_bounds__(TB) void sq_affine_acc_kernel(AccArgs a, const Idx*
       v2 = v2 < e0 ? e0 : (v2 > a.E ? a.E : v2);
       const int deg = (int)(v2 - e0 > 0x7fffffff ? 0x7fffffff : v2 - e0) - p;
       s_rdeg[i] = deg > 0 ? __builtin_amdgcn_rcpf((float)deg) : 0.f;
-      level |= (deg > CAP_N ? 1u : 0u) | (deg > CAP_W ? 2u : 0u);
+      // a decreasing offset (a negative length) compares as too long: such a block takes the direct form, which keeps
+      // no edges by position
+      level |= ((uint32_t)deg > (uint32_t)CAP_N ? 1u : 0u) | ((uint32_t)deg > (uint32_t)CAP_W ? 2u : 0u);
     }
   }
   {
@@ -737,7 +739,7 @@ __global__ __launch_bounds__(TB) void sq_affine_acc_pkernel(AccArgs a, const Idx
         v2 = v2 < e0 ? e0 : (v2 > a.E ? a.E : v2);
         const int deg = (int)(v2 - e0 > 0x7fffffff ? 0x7fffffff : v2 - e0) - p;
         s_rdeg[t] = deg > 0 ? __builtin_amdgcn_rcpf((float)deg) : 0.f;
-        level = (deg > CAP_N ? 1u : 0u) | (deg > CAP_W ? 2u : 0u);
+        level = ((uint32_t)deg > (uint32_t)CAP_N ? 1u : 0u) | ((uint32_t)deg > (uint32_t)CAP_W ? 2u : 0u);
       }
     }
     {
