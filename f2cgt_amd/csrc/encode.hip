@@ -326,7 +326,8 @@ __global__ __launch_bounds__(256) void predict_mfma_kernel(const float* __restri
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 // Three-way minimum of scores with the NaN behaviour of the instruction (the builtin minimum would first quieten
-// each operand with an instruction of its own).  A NaN ends in the row's exact evaluation wherever it comes out.
+// each operand with an instruction of its own).  A quiet NaN operand is left out, and the median of a triple with one
+// is its minimum, so that a triple's best is then its second as well and the row ends in the exact evaluation.
 __device__ __forceinline__ float min3_raw(float a, float b, float c) {
   float d;
   asm("v_min3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
@@ -346,7 +347,9 @@ __device__ __forceinline__ float max_raw(float a, float b) {
 // Running (best, second) over the 16 scores of a tile.  A score carries its slot in its four lowest bits (one
 // v_and_or, a change below 2^-19 of it that the near-tie bound includes), so that the index needs no compare and
 // select of its own and the rest is a tree of three-way minima and medians: 39 instructions for 16 scores where
-// compare, two selects and a median took 64.
+// compare, two selects and a median took 64.  Scores have to be finite or quiet NaNs: an infinity with a slot in its low
+// bits is a signalling NaN, which takes the other operands of a minimum with it.  The caller evaluates rows whose scores
+// could overflow exactly.
 __device__ __forceinline__ void argmin_update_packed(const floatx16& acc, int ct, float& best, float& second, int& bct) {
   float p[16];
 #pragma unroll
@@ -967,6 +970,9 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
   const float unit = 5.9604645e-8f * (float)(2 * (68 * S + k + 16));
   const float xscale = cosine ? -1.f : -2.f;
   const bool vec4 = (k % 8 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0);
+  // Packed scores have to be finite.  An L2 score |c|^2 - 2 x . c is at most 2 (|x|^2 + |c|^2), which may exceed the
+  // largest float (3.4e38) while the bound above is finite; cosine has |x . c^| <= |x|, below 2e19 wherever |x|^2 is finite.
+  const float finite_below = cosine ? INFINITY : 1.6e38f;
   const bool wide = kx >= 8;      // a row holds the eight values that an idle lane reads from row 0
   // A workgroup owns a contiguous share of the row groups and its four waves draw from it through
   // a counter in LDS: a wave held up by exact re-evaluations simply takes fewer groups.
@@ -1213,9 +1219,10 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
       const float scale = cosine ? sqrtf(xn[b]) * (cdev + 3.5762787e-7f / unit) : xn[b] + cmax;
       float bound = unit * scale + kTinyGap;
       bool ask = false;
-      if (kPacked) {      // the slots: 2^-19 of each of the two; padding leads only where every real score has overflowed
+      if (kPacked) {      // the slots: 2^-19 of each of the two
         bound += 1.92e-6f * (fabsf(bs) + fabsf(sd));
-        ask = bi >= n;
+        // padding leads where no real score is a number
+        ask = bi >= n || !(scale < finite_below);
       }
       besti[b] = bi;
       todo[b] = __ballot(valid && g == 0 && (ask || !((sd - bs) > bound)));

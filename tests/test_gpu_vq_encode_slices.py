@@ -79,3 +79,17 @@ def test_kmeans_predict_close_pairs(metric, n, k):
     # a cosine gap is about 2^-j / sqrt(k) wide, the oracle's near-ties are those below 1e-6: 7 % of the rows of one pair in
     # 4 dimensions, 1 to 3 % where the rows spread over many pairs
     assert near.mean() < 0.1 and np.array_equal(got[~near], want[~near])
+
+
+@pytest.mark.parametrize("n", [33, 256])
+@pytest.mark.parametrize("k", [2, 4, 8, 16, 17])
+def test_l2_scores_beyond_the_largest_float(n, k):
+    """|x|^2 = 1e38 and |c|^2 = 2e38: |c|^2 - 2 x . c is infinite in fp32 for centres on the far side, |x|^2 + |c|^2 is not."""
+    rng = np.random.default_rng(n + k)
+    x, c = rng.standard_normal((3000, k)), rng.standard_normal((n, k))
+    x = (x / np.linalg.norm(x, axis=1, keepdims=True) * 1e19).astype(np.float32)
+    c = (c / np.linalg.norm(c, axis=1, keepdims=True) * 2 ** 0.5 * 1e19).astype(np.float32)
+    want, near = oc.kmeans_predict(x, c, "l2")
+    assert ((c[None].astype(np.float64) ** 2).sum(2) - 2 * x.astype(np.float64) @ c.T.astype(np.float64)).max() > 3.41e38
+    got = capi.kmeans_predict(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), "l2").cpu().numpy()
+    assert near.mean() < 0.01 and np.array_equal(got[~near], want[~near])
