@@ -181,8 +181,8 @@ torch::Tensor sq_encode(torch::Tensor src, torch::Tensor codebooks, int64_t targ
   return out;
 }
 
-// Extension: order statistics, sum and NaN flag of |x| per column slice of the rows `rows` (None: all of them), for the
-// codebooks of sq_encode.  ranks: four ranks in a full slice, four in the last one.  -> float64 [n_slices, 6] on the GPU.
+// Extension: order statistics, sum and flags (1: a NaN, 2: a row id outside the table) of |x| per column slice of the rows
+// `rows` (None: all of them), for the codebooks of sq_encode.  ranks: four ranks in a full slice, four in the last one.  -> float64 [n_slices, 6] on the GPU.
 torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
                               const std::vector<int64_t>& ranks) {
   TORCH_CHECK(x.defined() && x.device().is_cuda(), "x must be a GPU tensor");

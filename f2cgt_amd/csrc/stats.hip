@@ -24,6 +24,8 @@ constexpr int kBins = 4096;          // counters of a pass: 4096, 4 x 1024 or 4 
 constexpr int kReplicas = 4;         // copies of the first pass's counters in LDS, by lane: its hot bins are few
 constexpr int kMaxBlocks = 256;      // workgroups per pass over all slices (one per CU)
 
+constexpr uint32_t kSawNan = 1u, kSawBadRow = 2u;   // a NaN among the values; a row id outside the table
+
 struct StatState {                   // per slice, written by the first workgroup of a pass for the passes after it
   uint32_t prefix[4];                // digits found so far of the value at each wanted rank
   uint32_t pad[4];
@@ -41,7 +43,7 @@ struct StatArgs {
   uint32_t* hist;                    // [n_slices][kBins]
   StatState* state;                  // [2][n_slices]: after the first and the second digit
   double* sums;                      // [n_slices][blocks]
-  uint32_t* nans;                    // [n_slices][blocks]
+  uint32_t* flags;                   // [n_slices][blocks]: kSawNan, kSawBadRow
   double* out;                       // [n_slices][6]
 };
 
@@ -128,11 +130,11 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   __shared__ uint32_t s_digit[4];
   __shared__ uint64_t s_rest[4];
   __shared__ double s_sum[kStatThreads / kWave];
-  __shared__ uint32_t s_nan;
+  __shared__ uint32_t s_flags;
   const int t = threadIdx.x, slice = blockIdx.y;
   constexpr int LDS_BINS = PASS == 0 ? kBins * kReplicas : kBins;
   for (int i = t; i < LDS_BINS / 4; i += kStatThreads) reinterpret_cast<uint4*>(s_hist)[i] = make_uint4(0u, 0u, 0u, 0u);
-  if (t == 0) s_nan = 0u;
+  if (t == 0) s_flags = 0u;
   uint32_t prefix[4] = {0u, 0u, 0u, 0u};
   if constexpr (PASS > 0) {
     uint64_t rank[4];
@@ -153,12 +155,12 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   const int r0 = t / cg, c0 = t - r0 * cg;
   const int64_t step = (int64_t)a.blocks * rpp;
   double sum = 0.0;
-  bool nan = false;
+  uint32_t flags = 0u;
   auto take = [&](float v) {
     const uint32_t mag = __float_as_uint(v) & 0x7fffffffu;
     if constexpr (PASS == 0) {
       sum += (double)__uint_as_float(mag);
-      nan = nan || mag > 0x7f800000u;
+      flags |= mag > 0x7f800000u ? kSawNan : 0u;
       atomicAdd(&s_hist[(mag >> 19) * kReplicas + (t & (kReplicas - 1))], 1u);
     } else if constexpr (PASS == 1) {
 #pragma unroll
@@ -179,8 +181,10 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
         const int64_t ru = r + u * step < a.m ? r + u * step : r;
         id[u] = ru;
         if (a.rows != nullptr) {
-          const int64_t want = a.rows[ru];
-          id[u] = clamp_idx(want < 0 ? want + a.num_rows : want, a.num_rows);
+          int64_t want = a.rows[ru];
+          want = want < 0 ? want + a.num_rows : want;
+          id[u] = clamp_idx(want, a.num_rows);
+          if (PASS == 0) flags |= id[u] != want ? kSawBadRow : 0u;
         }
       }
       for (int c = c0; c < groups; c += cg) {
@@ -208,7 +212,7 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
     }
   }
   if constexpr (PASS == 0) {
-    if (nan) atomicOr(&s_nan, 1u);
+    if (flags) atomicOr(&s_flags, flags);
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
     if ((t & (kWave - 1)) == 0) s_sum[t / kWave] = sum;
@@ -229,7 +233,7 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
     double total = 0.0;
     for (int w = 0; w < kStatThreads / kWave; ++w) total += s_sum[w];
     a.sums[(int64_t)slice * a.blocks + blockIdx.x] = total;
-    a.nans[(int64_t)slice * a.blocks + blockIdx.x] = s_nan;
+    a.flags[(int64_t)slice * a.blocks + blockIdx.x] = s_flags;
   }
 }
 
@@ -252,7 +256,7 @@ __global__ __launch_bounds__(kStatThreads) void stat_reduce_kernel(StatArgs a) {
   a.hist[(int64_t)slice * kBins + bin] = c;
 }
 
-// Last digit, and the outputs of a slice: the values at the four ranks, the sum, whether a NaN was seen.
+// Last digit, and the outputs of a slice: the values at the four ranks, the sum, the flags.
 __global__ __launch_bounds__(kStatThreads) void stat_finish_kernel(StatArgs a) {
   __shared__ uint64_t s_scan[kStatThreads / kWave];
   __shared__ uint32_t s_digit[4];
@@ -264,19 +268,19 @@ __global__ __launch_bounds__(kStatThreads) void stat_finish_kernel(StatArgs a) {
   if (t < 4) a.out[slice * 6 + t] = (double)__uint_as_float(t == 0 ? prefix[0] : t == 1 ? prefix[1] : t == 2 ? prefix[2] : prefix[3]);
   if (t >= kWave && t < 2 * kWave) {                    // the second wave
     double total = 0.0;
-    uint32_t nan = 0;
+    uint32_t flags = 0;
     for (int b = t - kWave; b < a.blocks; b += kWave) {
       total += a.sums[(int64_t)slice * a.blocks + b];
-      nan |= a.nans[(int64_t)slice * a.blocks + b];
+      flags |= a.flags[(int64_t)slice * a.blocks + b];
     }
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) {
       total += __shfl_xor(total, off);
-      nan |= __shfl_xor(nan, off);
+      flags |= __shfl_xor(flags, off);
     }
     if (t == kWave) {
       a.out[slice * 6 + 4] = total;
-      a.out[slice * 6 + 5] = nan ? 1.0 : 0.0;
+      a.out[slice * 6 + 5] = (double)flags;
     }
   }
 }
@@ -292,14 +296,14 @@ int stat_blocks(int64_t m, int64_t cols, int64_t slice, int64_t n_slices) {
 
 int64_t round256(int64_t v) { return (v + 255) / 256 * 256; }
 
-struct StatLayout { int64_t hist, state, sums, nans, total; };
+struct StatLayout { int64_t hist, state, sums, flags, total; };
 StatLayout stat_layout(int64_t blocks, int64_t n_slices) {
   StatLayout l;
   l.hist = round256(n_slices * blocks * kBins * 4);
   l.state = l.hist + round256(n_slices * kBins * 4);
   l.sums = l.state + round256(2 * n_slices * (int64_t)sizeof(StatState));
-  l.nans = l.sums + round256(n_slices * blocks * 8);
-  l.total = l.nans + round256(n_slices * blocks * 4);
+  l.flags = l.sums + round256(n_slices * blocks * 8);
+  l.total = l.flags + round256(n_slices * blocks * 4);
   return l;
 }
 
@@ -362,7 +366,7 @@ extern "C" int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* 
   a.hist = reinterpret_cast<uint32_t*>(ws + l.hist);
   a.state = reinterpret_cast<StatState*>(ws + l.state);
   a.sums = reinterpret_cast<double*>(ws + l.sums);
-  a.nans = reinterpret_cast<uint32_t*>(ws + l.nans);
+  a.flags = reinterpret_cast<uint32_t*>(ws + l.flags);
   a.out = out;
   // widest access that every slice of every row is a multiple of
   const int64_t last_width = cols - (n_slices - 1) * column_slice;

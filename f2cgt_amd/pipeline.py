@@ -86,10 +86,13 @@ def _device_statistics(values, rows, column_slice):
     places = [[_percentile_place(n, q) for q in _PERCENTILES] for n in sizes]
     ranks = [r for per_size in places for place in per_size for r in place[:2]]
     stats = _capi().abs_order_stats(values, rows, column_slice, ranks).cpu().numpy()
+    flags = stats[:, 5].astype(np.int64)
+    if (flags & 2).any():
+        raise IndexError("a sample id lies outside the table's %d rows" % values.shape[0])
     out = []
     for i in range(count):
         last = int(i == count - 1)
-        if stats[i, 5]:
+        if flags[i] & 1:
             lo = hi = np.float32("nan")
         else:
             lo, hi = (_between(np.float32(stats[i, 2 * q]), np.float32(stats[i, 2 * q + 1]), places[last][q][2]) for q in (0, 1))

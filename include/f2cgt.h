@@ -228,10 +228,10 @@ int f2cgt_fetch_rows(const void* table, const void* hot, const int32_t* slot_map
 
 /* The statistics behind an SQ codebook (examples/process_compress.py:45-68), of the absolute values of every column
  * slice of a sample: x fp32 [num_rows, cols] with row stride ld; rows int64 [m] (device) lists the sample's rows (negative
- * ones count from the end; clamped to the table), NULL takes rows [0, m).  ranks (host, 8 values): four ranks (0 = smallest) among the
- * m * column_slice values of a full slice, then four among those of the last slice.
- * out fp64 [ceil(cols / column_slice), 6] (device): the exact |x| at the four ranks, the sum of |x| (fp64), and 1 when a
- * NaN was among the values (0 otherwise).  workspace: device scratch, 256-byte aligned, contents irrelevant. */
+ * ones count from the end; others outside the table are clamped to it and reported), NULL takes rows [0, m).  ranks (host,
+ * 8 values): four ranks (0 = smallest) among the m * column_slice values of a full slice, then four among those of the
+ * last slice.  out fp64 [ceil(cols / column_slice), 6] (device): the exact |x| at the four ranks, the sum of |x| (fp64),
+ * and the sum of 1 when a NaN was among the values and 2 when rows held an id outside the table.  workspace: device scratch, 256-byte aligned, contents irrelevant. */
 int64_t f2cgt_abs_order_stats_workspace_bytes(int64_t m, int64_t cols, int64_t column_slice);
 int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols,
                           int64_t column_slice, const int64_t* ranks, void* workspace, int64_t workspace_bytes,

@@ -72,3 +72,17 @@ def test_codebooks_on_the_device_are_numpys(dtype, n, d, slice_):
     one = np.array([float(v) for v in pipeline.sq_metadata(x[pick].cuda())], dtype=np.float32)
     want = oc.sq_codebook(x[pick].float().numpy())
     assert np.array_equal(one[:4], want[:4]) and np.isclose(one[4], want[4], rtol=1e-6)
+
+
+@pytest.mark.parametrize("where", ["cuda", "cpu"])
+@pytest.mark.parametrize("bad", [300, -301, 2 ** 40])
+def test_sample_ids_outside_the_table_are_refused(where, bad):
+    from f2cgt_amd import pipeline
+    x = torch.rand((300, 24))
+    pick = torch.arange(-300, 300)
+    if where == "cuda":      # on the host the same list is refused by the gather
+        got = f2cgt_amd.load().abs_order_stats(x.cuda(), pick.cuda(), 8, [0, 1, 2, 3] * 2).cpu()
+        assert got[:, 5].tolist() == [0.0, 0.0, 0.0]
+    pick[77] = bad
+    with pytest.raises(IndexError):
+        pipeline.sq_compress(x.to(where), 4, 8, sample_index=pick)
