@@ -187,7 +187,9 @@ torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows
                               const std::vector<int64_t>& ranks) {
   TORCH_CHECK(x.defined() && x.device().is_cuda(), "x must be a GPU tensor");
   TORCH_CHECK(x.dim() == 2 && x.scalar_type() == torch::kFloat32, "x must be float32 [rows, feat_dim]");
-  if (x.stride(1) != 1) x = x.contiguous();
+  // columns apart, or rows that overlap (an expanded row): a copy.  The stride of a single row may be anything.
+  if (x.stride(1) != 1 || x.stride(0) < x.size(1)) x = x.contiguous();
+  const int64_t ld = x.size(0) > 1 ? x.stride(0) : x.size(1);
   TORCH_CHECK(ranks.size() == 8, "ranks must hold eight values");
   TORCH_CHECK(column_slice > 0, "column_slice must be positive");
   torch::Tensor r;
@@ -200,7 +202,7 @@ torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows
   auto opts = torch::TensorOptions().device(x.device());
   auto out = torch::empty({(cols + column_slice - 1) / column_slice, 6}, opts.dtype(torch::kFloat64));
   auto ws = torch::empty({f2cgt_abs_order_stats_workspace_bytes(m, cols, column_slice)}, opts.dtype(torch::kUInt8));
-  check_rc(f2cgt_abs_order_stats(x.data_ptr<float>(), x.stride(0), r.defined() ? r.data_ptr<int64_t>() : nullptr, m,
+  check_rc(f2cgt_abs_order_stats(x.data_ptr<float>(), ld, r.defined() ? r.data_ptr<int64_t>() : nullptr, m,
                                  x.size(0), cols, column_slice, ranks.data(), ws.data_ptr(), ws.numel(),
                                  out.data_ptr<double>(), current_stream()),
            "abs_order_stats");

@@ -86,3 +86,17 @@ def test_sample_ids_outside_the_table_are_refused(where, bad):
     pick[77] = bad
     with pytest.raises(IndexError):
         pipeline.sq_compress(x.to(where), 4, 8, sample_index=pick)
+
+
+def test_rows_that_overlap():
+    """A row expanded to a table (row stride 0) and a one-row table seen through a transpose (row stride 1)."""
+    from f2cgt_amd import pipeline
+    row = torch.randn((1, 40), generator=torch.Generator().manual_seed(3))
+    pick = torch.arange(0, 300, 3)
+    for table, rows in ((row.cuda().expand(300, 40), pick), (torch.randn((40, 1)).cuda().t(), torch.zeros(5, dtype=torch.int64))):
+        assert table.stride(0) < table.shape[1]
+        whole = torch.empty(table.shape, device="cuda").copy_(table)
+        codes, books = pipeline.sq_compress(table, 4, 16, sample_index=rows)
+        want_codes, want_books = pipeline.sq_compress(whole, 4, 16, sample_index=rows)
+        assert torch.equal(books, want_books) and torch.equal(codes, want_codes)
+        assert [float(v) for v in pipeline.sq_metadata(table)] == [float(v) for v in pipeline.sq_metadata(whole)]
