@@ -124,7 +124,8 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
     if sample_index is None:
         sample_index = sampling(250_000, num_items, hotness)
     sample_index = sample_index.to(features.device)
-    if features.is_cuda and features.dtype == torch.float32 and sample_index.dtype == torch.int64 and sample_index.numel():
+    if (features.is_cuda and features.dtype == torch.float32 and features.stride(1) == 1 and features.stride(0) >= feat_dim and
+            sample_index.dtype == torch.int64 and sample_index.numel()):
         stats = _device_statistics(features, sample_index, column_slice)     # the sample's rows are read in place
     else:
         stats = _device_statistics(features[sample_index].float().cuda(), None, column_slice)

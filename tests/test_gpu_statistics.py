@@ -100,3 +100,18 @@ def test_rows_that_overlap():
         want_codes, want_books = pipeline.sq_compress(whole, 4, 16, sample_index=rows)
         assert torch.equal(books, want_books) and torch.equal(codes, want_codes)
         assert [float(v) for v in pipeline.sq_metadata(table)] == [float(v) for v in pipeline.sq_metadata(whole)]
+
+
+@pytest.mark.parametrize("kind", ["columns apart", "one row expanded"])
+def test_a_table_that_is_no_plain_one_is_not_copied_whole(kind):
+    from f2cgt_amd import pipeline
+    table = torch.randn((40, 100000), device="cuda").t() if kind == "columns apart" else torch.randn((1, 40), device="cuda").expand(100000, 40)
+    pick = torch.arange(0, 100000, 100)
+    _, want = pipeline.sq_compress(table[pick.cuda()], 4, 16, sample_index=torch.arange(1000))
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    codes, books = pipeline.sq_compress(table, 4, 16, sample_index=pick, batch_rows=1000)
+    assert torch.equal(books, want)
+    # the codes, the sample and scratch of a few MB; the table is 16 MB
+    assert torch.cuda.max_memory_allocated() - before - codes.numel() < 12 << 20
