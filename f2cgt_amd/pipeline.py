@@ -100,19 +100,38 @@ def _device_statistics(values, rows, column_slice):
     return out
 
 
+def _device_takes(rows, cols, column_slice):
+    """What the device statistics count in: 32 bits of values per slice, 24 of columns, 16 of slices."""
+    return (0 < rows * min(cols, column_slice) < 1 << 32 and cols < 1 << 24 and
+            (cols + column_slice - 1) // column_slice < 1 << 16)
+
+
 def sq_metadata(sample):
     """(fmin, fmax, emin, emax, mean) of one column slice from a sample of its rows:
     percentiles of |x| floored at 1e-5 / 2e-5, their log2, mean lifted by 0.1 when
     below 0.1 (examples/process_compress.py:45-68).  A sample on the GPU is reduced there."""
     if sample.is_cuda and sample.numel():
         values = sample.float()
-        return _sq_codebook(*_device_statistics(values.reshape(values.shape[0], -1), None, values[0].numel())[0])
+        values = values.reshape(-1, values.shape[-1] if values.dim() > 1 else 1)
+        if _device_takes(*values.shape, values.shape[1]):
+            return _sq_codebook(*_device_statistics(values, None, values.shape[1])[0])
     magnitude = sample.float().abs().cpu()
     # one percentile and one log2 at a time, as the reference does: numpy returns the sample's own
     # precision for a scalar quantile (float64 for a list of them), and torch's scalar and vector
     # log2 do not agree to the last bit
     lo, hi = (np.percentile(magnitude.numpy(), q) for q in _PERCENTILES)
     return _sq_codebook(lo, hi, magnitude.mean())
+
+
+def _sampled_sq_codebook(features, sample_index, lo, hi):
+    """Codebook of columns [lo, hi) from a gathered sample: on the GPU, or on the host where it does not fit there."""
+    sample = features[sample_index, lo:hi]
+    if not sample.is_cuda:
+        try:
+            return sq_metadata(sample.cuda())
+        except torch.OutOfMemoryError:
+            pass
+    return sq_metadata(sample)
 
 
 def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=None, batch_rows=1_000_000):
@@ -125,11 +144,14 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
         sample_index = sampling(250_000, num_items, hotness)
     sample_index = sample_index.to(features.device)
     if (features.is_cuda and features.dtype == torch.float32 and features.stride(1) == 1 and features.stride(0) >= feat_dim and
-            sample_index.dtype == torch.int64 and sample_index.numel()):
-        stats = _device_statistics(features, sample_index, column_slice)     # the sample's rows are read in place
+            sample_index.dtype == torch.int64 and sample_index.dim() == 1 and
+            _device_takes(sample_index.numel(), feat_dim, column_slice)):
+        # the sample's rows are read in place
+        per_slice = [_sq_codebook(*values) for values in _device_statistics(features, sample_index, column_slice)]
     else:
-        stats = _device_statistics(features[sample_index].float().cuda(), None, column_slice)
-    codebooks = torch.tensor([[float(v) for v in _sq_codebook(*values)] for values in stats], dtype=torch.float32).cuda()
+        per_slice = [_sampled_sq_codebook(features, sample_index, lo, min(lo + column_slice, feat_dim))
+                     for lo in range(0, feat_dim, column_slice)]
+    codebooks = torch.tensor([[float(v) for v in values] for values in per_slice], dtype=torch.float32).reshape(-1, 5).cuda()
     if target_bits <= 8:
         dtype, tdim = torch.int8, int(math.ceil(feat_dim / 8 * target_bits))
     elif target_bits <= 16:

@@ -115,3 +115,42 @@ def test_a_table_that_is_no_plain_one_is_not_copied_whole(kind):
     assert torch.equal(books, want)
     # the codes, the sample and scratch of a few MB; the table is 16 MB
     assert torch.cuda.max_memory_allocated() - before - codes.numel() < 12 << 20
+
+
+@pytest.mark.parametrize("where", ["cuda", "cpu"])
+def test_samples_of_any_shape(where, monkeypatch):
+    """A list of lists of ids, a single id, a mask; a host sample that the GPU has no room for; more values than the
+    device counts (the limit lowered): the codebooks of the flat list, and numpy's, as from a host table."""
+    from f2cgt_amd import pipeline
+    rng = np.random.default_rng(9)
+    x = torch.from_numpy(rng.standard_normal((400, 30)).astype(np.float32))
+    pick = torch.from_numpy(rng.permutation(400)[:240])
+    table = x.to(where)
+
+    def books(index):
+        return pipeline.sq_compress(table, 4, 8, sample_index=index)[1].cpu().numpy()
+
+    want = np.stack([oc.sq_codebook(x[pick].numpy()[:, lo:lo + 8]) for lo in range(0, 30, 8)])
+    mask = torch.zeros(400, dtype=torch.bool)
+    mask[pick] = True
+    for index in (pick, pick.view(12, 20), pick.int(), mask):
+        got = books(index)
+        assert np.array_equal(got[:, :4], want[:, :4]) and np.allclose(got[:, 4], want[:, 4], rtol=1e-6)
+    one = np.stack([oc.sq_codebook(x[7].numpy()[None, lo:lo + 8]) for lo in range(0, 30, 8)])
+    assert np.array_equal(books(torch.tensor(7))[:, :4], one[:, :4])
+    whole = [float(v) for v in pipeline.sq_metadata(table)]
+    assert [float(v) for v in pipeline.sq_metadata(table.view(20, 20, 30))] == whole
+    assert float(pipeline.sq_metadata(table[3, 3])[0]) == max(abs(float(x[3, 3])), 1e-5)
+
+    monkeypatch.setattr(pipeline, "_device_takes", lambda *sizes: False)
+    monkeypatch.setattr(pipeline, "_device_statistics", None)
+    assert np.array_equal(books(pick)[:, :4], want[:, :4])
+    monkeypatch.undo()
+
+    def full(*args, **kwargs):
+        raise torch.OutOfMemoryError("no room")
+    if where == "cpu":
+        with monkeypatch.context() as m:
+            to_gpu = torch.Tensor.cuda
+            m.setattr(torch.Tensor, "cuda", lambda t, *a, **k: full() if t.shape == (240, 8) else to_gpu(t, *a, **k))
+            assert np.array_equal(books(pick)[:, :4], want[:, :4])

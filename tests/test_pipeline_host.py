@@ -39,3 +39,16 @@ def test_layer_rejects_other_aggregators():
     import pytest
     with pytest.raises(ValueError):
         pipeline.MySAGEConv(8, 4, "pool", None)
+
+
+def test_what_the_device_statistics_take():
+    """The sizes that sq_compress keeps from the device statistics are those that the library refuses (its checks come
+    before anything is read: the buffers are stand-ins)."""
+    import ctypes
+    from f2cgt_amd import capi
+    a, ranks = ctypes.c_void_p(1 << 20), (ctypes.c_int64 * 8)()
+    assert pipeline._device_takes(1, 1, 1) and pipeline._device_takes(2 ** 32 - 1, 1, 1)
+    assert pipeline._device_takes(5, 2 ** 24 - 1, 300) and pipeline._device_takes(3, 65535, 1)
+    for m, cols, width in ((2 ** 32, 1, 1), (2 ** 25, 500, 128), (3, 2 ** 24, 2 ** 24), (3, 65536, 1), (0, 8, 8), (8, 0, 8)):
+        assert not pipeline._device_takes(m, cols, width)
+        assert capi.lib().f2cgt_abs_order_stats(a, max(cols, 1), a, m, max(m, 1), cols, width, ranks, a, 1 << 62, a, None)
