@@ -110,7 +110,8 @@ def sq_metadata(sample):
     """(fmin, fmax, emin, emax, mean) of one column slice from a sample of its rows:
     percentiles of |x| floored at 1e-5 / 2e-5, their log2, mean lifted by 0.1 when
     below 0.1 (examples/process_compress.py:45-68).  A sample on the GPU is reduced there."""
-    if sample.is_cuda and sample.numel():
+    # (a sample that is part of a graph keeps the host's refusal)
+    if sample.is_cuda and sample.numel() and not sample.requires_grad:
         values = sample.float()
         values = values.reshape(-1, values.shape[-1] if values.dim() > 1 else 1)
         if _device_takes(*values.shape, values.shape[1]):
@@ -144,7 +145,7 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
         sample_index = sampling(250_000, num_items, hotness)
     sample_index = sample_index.to(features.device)
     if (features.is_cuda and features.dtype == torch.float32 and features.stride(1) == 1 and features.stride(0) >= feat_dim and
-            sample_index.dtype == torch.int64 and sample_index.dim() == 1 and
+            sample_index.dtype == torch.int64 and sample_index.dim() == 1 and not features.requires_grad and
             _device_takes(sample_index.numel(), feat_dim, column_slice)):
         # the sample's rows are read in place
         per_slice = [_sq_codebook(*values) for values in _device_statistics(features, sample_index, column_slice)]

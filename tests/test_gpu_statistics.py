@@ -154,3 +154,15 @@ def test_samples_of_any_shape(where, monkeypatch):
             to_gpu = torch.Tensor.cuda
             m.setattr(torch.Tensor, "cuda", lambda t, *a, **k: full() if t.shape == (240, 8) else to_gpu(t, *a, **k))
             assert np.array_equal(books(pick)[:, :4], want[:, :4])
+
+
+def test_features_that_require_a_gradient_are_refused():
+    from f2cgt_amd import pipeline
+    table = torch.randn((300, 24), device="cuda", requires_grad=True)
+    pick = torch.arange(0, 300, 2)
+    for call in (lambda: pipeline.sq_compress(table, 4, 8, sample_index=pick), lambda: pipeline.sq_metadata(table)):
+        with pytest.raises(RuntimeError, match="requires grad"):
+            call()
+    with torch.no_grad():
+        assert torch.equal(pipeline.sq_compress(table, 4, 8, sample_index=pick)[1],
+                           pipeline.sq_compress(table.detach(), 4, 8, sample_index=pick)[1])
