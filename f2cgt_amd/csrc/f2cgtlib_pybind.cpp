@@ -195,7 +195,8 @@ torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows
   torch::Tensor r;
   if (rows.has_value()) {
     r = dev_contig(*rows, "rows");
-    TORCH_CHECK(r.dim() == 1 && r.scalar_type() == torch::kInt64, "rows must be int64 [m]");
+    TORCH_CHECK(r.dim() == 1 && r.scalar_type() == torch::kInt64 && r.device() == x.device(),
+                "rows must be int64 [m] on the device of x");
   }
   c10::DeviceGuard guard(x.device());
   const int64_t m = r.defined() ? r.numel() : x.size(0), cols = x.size(1);

@@ -166,3 +166,9 @@ def test_features_that_require_a_gradient_are_refused():
     with torch.no_grad():
         assert torch.equal(pipeline.sq_compress(table, 4, 8, sample_index=pick)[1],
                            pipeline.sq_compress(table.detach(), 4, 8, sample_index=pick)[1])
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs two GPUs")
+def test_row_ids_on_another_device_are_refused():
+    with pytest.raises(RuntimeError, match="on the device of x"):
+        f2cgt_amd.load().abs_order_stats(torch.rand((30, 8), device="cuda:0"), torch.arange(5, device="cuda:1"), 8, [0, 1, 2, 3] * 2)
