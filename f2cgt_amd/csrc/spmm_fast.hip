@@ -1008,7 +1008,7 @@ struct RowsArgs {
   int f4_per_row, fin_group, fin_slots;
   uint32_t fin_magic;
   int nt_out;            // output larger than the last-level cache: non-temporal stores
-  int items_per_row;     // FLAT: column groups of a row, and ceil(2^32 / that)
+  int items_per_row;     // ITEM: column groups of a row, and ceil(2^32 / that)
   uint32_t item_magic;
 };
 
@@ -1018,18 +1018,19 @@ __device__ __forceinline__ float mean_of(float sum, float d, float r) {
   return __fmaf_rn(__fmaf_rn(-q, d, sum), r, q);
 }
 
-// Adds the eight 1-bit values of a code byte to s: +plus where the bit is set, -plus where it is not, the two values a
+// Adds the first G 1-bit values of a code byte to s: +plus where the bit is set, -plus where it is not, the two values a
 // 1-bit log-domain codebook has.  The bits become the signs of halves (-1 or 1, two per instruction) and the sums
 // fma(+-1, -plus, s), which rounds as the addition does: two instructions per value and no table read.
-__device__ __forceinline__ void add_signs8(float (&s)[8], uint32_t byte, float minus_plus) {
+template <int G>
+__device__ __forceinline__ void add_signs(float (&s)[G], uint32_t byte, float minus_plus) {
   typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-  const uint32_t w = byte | (byte << 12);        // bit i at i, bit i + 4 at i + 16
+  const uint32_t w = byte | (byte << (16 - G / 2));   // bit i at i, bit i + G / 2 at i + 16
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < G / 2; ++i) {
     const uint32_t pair = ((w << (15 - i)) & 0x80008000u) | 0x3c003c00u;
     const half2v h = __builtin_bit_cast(half2v, pair);
     s[i] = __builtin_fmaf((float)h[0], minus_plus, s[i]);
-    s[i + 4] = __builtin_fmaf((float)h[1], minus_plus, s[i + 4]);
+    s[i + G / 2] = __builtin_fmaf((float)h[1], minus_plus, s[i + G / 2]);
   }
 }
 
@@ -1038,7 +1039,8 @@ __device__ __forceinline__ void add_signs8(float (&s)[8], uint32_t byte, float m
 // with the store form fixed at compile time the row loop came out 3-5 % faster at 100-256 columns and 17-19 % at 600
 // (3e6 edges, 10 per row, 4 bit: 97.8 -> 93.7 us at 128 columns, 592 -> 489 us at 600); 1- and 2-bit rows measured
 // level to 2 % slower and keep the run-time test.
-template <int BITS, bool AFFINE, typename Idx, int TB, int HALF = 0, bool FLAT = false>
+// ITEM: 0 (a lane keeps a column group), or the columns of the items that are dealt to the lanes: 4, or 8 (1 bit).
+template <int BITS, bool AFFINE, typename Idx, int TB, int HALF = 0, int ITEM = 0>
 __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __restrict__ indptr,
                                                              const Idx* __restrict__ indices,
                                                              float* __restrict__ out) {
@@ -1145,12 +1147,13 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
   }
   __syncthreads();
 
-  if constexpr (FLAT) {
-    // decode + sum: (row, column group) items dealt to the lanes one after the other.  Bound by instruction issue: two
-    // to three per value with 1-bit codes, an LDS read and three with the others; 60001 rows of 602 columns at 10
-    // edges per row write 2.0 TB/s with 1-bit codes (staged rows with a column group per lane: 0.77 TB/s).
-    constexpr int G = BITS == 1 ? 8 : 4;                 // columns of an item
-    constexpr int GB = G * BITS / 8;                     // its code bytes
+  if constexpr (ITEM != 0) {
+    // decode + sum: (row, column group) items dealt to the lanes one after the other.  60001 rows of 602 columns at 10
+    // edges per row write 2.5 TB/s with 1-bit codes (staged rows with a column group per lane: 0.77 TB/s).  The two or
+    // three instructions per value (an LDS read and three with the other codes) are 23 us of the 57.8 there and the
+    // output 30; the rest is the trips of a row's dependent loads (offset, id, code).
+    constexpr int G = ITEM;                              // columns of an item
+    constexpr int GB = G * BITS < 8 ? 1 : G * BITS / 8;  // code bytes that hold them
     const int items = nrows * a.items_per_row;
     const float minus_plus = -s_lut[1];
     for (int item = t; item < items; item += TB) {
@@ -1167,18 +1170,20 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
       // issued together (with a branch per load they were waited for one by one: 1000 rows of 300 edges, 128
       // columns, 4 bit 129 -> 64 us; 30000 rows of power-law degrees, 100 columns, 4 bit 105 -> 59, 8 bit 112 -> 59).
       const bool half = GB > 1 && HALF != 0 && left < G;
-      const uint32_t at = (uint32_t)(c * GB - (half ? GB / 2 : 0));
+      const int first = c * (G * BITS) / 8;              // first code byte; four 1-bit codes start at bit 0 or 4 of it
+      const uint32_t bit = G * BITS < 8 ? (uint32_t)(c * (G * BITS)) & 7u : 0u;
+      const uint32_t at = (uint32_t)(first - (half ? GB / 2 : 0));
       const uint32_t sh = half ? 4 * GB : 0;
       auto code_at = [&](uint32_t id) -> uint32_t {
         const uint8_t* q = a.codes + ((uint64_t)id * (uint32_t)a.src_dim + at);
-        if constexpr (GB == 1) return *q;
+        if constexpr (GB == 1) return (uint32_t)*q >> bit;
         uint32_t w = 0;
         __builtin_memcpy(&w, q, GB);
         return w >> sh;
       };
       auto add = [&](uint32_t w) {
         if constexpr (BITS == 1) {
-          add_signs8(s, w, minus_plus);
+          add_signs<G>(s, w, minus_plus);
         } else {
 #pragma unroll
           for (int i = 0; i < G; ++i) s[i] += s_lut[(w >> (BITS * i)) & MASK];
@@ -1199,10 +1204,10 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
       };
       if (staged) {
         walk([&](int k) -> uint32_t {
-          const unsigned char* q = s_codes + k * a.pitch + c * GB;
+          const unsigned char* q = s_codes + k * a.pitch + first;
           if constexpr (GB == 4) return *reinterpret_cast<const uint32_t*>(q);
           else if constexpr (GB == 2) return *reinterpret_cast<const uint16_t*>(q);
-          else return *q;
+          else return (uint32_t)*q >> bit;
         });
       } else if (have_ids) {
         walk([&](int k) -> uint32_t { return code_at(s_ids[k]); });
@@ -1343,7 +1348,7 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
   }
 }
 
-template <int BITS, bool AFFINE, int TB, bool FLAT>
+template <int BITS, bool AFFINE, int TB, bool DEAL>
 int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, int idx_dtype, float* out, hipStream_t st,
                    const char* what) {
   a.eff_bytes = (int)ceil_div(a.feat_dim, 8 / BITS);
@@ -1356,12 +1361,18 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
   a.fin_group = a.f4_per_row < TB ? a.f4_per_row : TB;
   a.fin_slots = TB / a.fin_group;
   a.fin_magic = (uint32_t)((65536 + a.fin_group - 1) / a.fin_group);
-  a.items_per_row = (int)ceil_div(a.feat_dim, BITS == 1 ? 8 : 4);
-  a.item_magic = (uint32_t)(((1ull << 32) + a.items_per_row - 1) / a.items_per_row);   // items < 64 * 1024: exact
   a.nt_out = stream_output(a.R * (int64_t)a.feat_dim * 4, (int64_t)a.feat_dim * 4,
                            a.R > 0 ? (double)a.E / (double)a.R : 0.0) ? 1 : 0;
   const size_t lut_bytes = AFFINE ? 0 : (size_t)(((a.num_codebooks << BITS) + 3) & ~3) * 4;
   const double avg_deg = a.R > 0 ? (double)a.E / (double)a.R : 1.0;
+  // 1-bit items of eight columns read a code byte once, but a lane's two 16-byte stores have every store instruction
+  // write 16 of every 32 bytes, which streamed stores take to memory as partial lines: streamed outputs take items of
+  // four columns, whose stores are contiguous (240000 rows of 256 columns: 115 us with eight, 46 with four at one edge
+  // per row, 81 and 71 at eight; 60001 x 602 at 10 edges per row: 65.6 and 57.8).  Cached outputs take eight columns from
+  // two edges per row on (60000 rows of 128 columns, half an edge per row: 11 against 10 us).
+  const bool wide = DEAL && BITS == 1 && !a.nt_out && avg_deg >= 2.0;
+  a.items_per_row = (int)ceil_div(a.feat_dim, wide ? 8 : 4);
+  a.item_magic = (uint32_t)(((1ull << 32) + a.items_per_row - 1) / a.items_per_row);   // items < 64 * 1024: exact
   const double dg = avg_deg > 0.5 ? avg_deg : 0.5;
   int cap = (int)((20 * 1024) / (a.pitch + 4));
   cap = cap > 2 * TB ? 2 * TB : cap;
@@ -1385,12 +1396,12 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
   // columns, 10 edges per row 91 / 73; 8 bit, 128 columns 79 / 67; 2 bit, 602 columns 85 / 75, at 25 edges per row
   // 247 / 131; 4 bit, 602 columns 152 / 88).  Short 2- and 4-bit rows are better staged (2 bit, 256 columns, 25
   // edges per row 87 / 96; 4 bit, 100 columns, power-law degrees 34 / 39).
-  const bool direct = FLAT && (BITS == 1 || BITS == 8 || a.pitch > 128 || (int)(8.0 * dg * 1.1) + 8 > a.edge_cap);
+  const bool direct = DEAL && (BITS == 1 || BITS == 8 || a.pitch > 128 || (int)(8.0 * dg * 1.1) + 8 > a.edge_cap);
   if (direct) {
-    // about two rounds of items per thread for 1-bit codes, four for the others; at most 480 edges in a block of more
+    // about two rounds of items per thread for eight columns, four for four; at most 480 edges in a block of more
     // than eight rows, so that long rows spread over the chip
     a.edge_cap = 0;
-    rb = ((BITS == 1 ? 600 : 1024) / a.items_per_row + 4) / 8 * 8;
+    rb = ((wide ? 600 : 1024) / a.items_per_row + 4) / 8 * 8;
     const int few = (int)(480.0 / dg) / 8 * 8;
     rb = rb > few ? few : rb;
   }
@@ -1423,17 +1434,21 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
                 a.id_cap);
     return 0;
   }
-  const int half = (a.feat_dim % 4 == 0 && BITS < 4) ? 0 : (a.nt_out ? 2 : 1);
-#define F2CGT_ROWS_GO(I, H)                                                      \
-  sq_rows_kernel<BITS, AFFINE, I, TB, H, FLAT><<<(unsigned)grid, TB, lds, st>>>(       \
+  constexpr bool STORE_FIXED = BITS >= 4 || (DEAL && BITS == 1);   // the store kind is always fixed when the kernel is chosen
+  const int half = (a.feat_dim % 4 == 0 && !STORE_FIXED) ? 0 : (a.nt_out ? 2 : 1);
+#define F2CGT_ROWS_GO(I, H, N)                                                   \
+  sq_rows_kernel<BITS, AFFINE, I, TB, H, N><<<(unsigned)grid, TB, lds, st>>>(    \
       a, static_cast<const I*>(indptr), static_cast<const I*>(indices), out)
 #define F2CGT_ROWS_IDX(I)                                                        \
   do {                                                                           \
-    if constexpr (BITS < 4) {                                                    \
-      if (half == 0) F2CGT_ROWS_GO(I, 0);                                        \
+    if constexpr (!STORE_FIXED) {                                                \
+      if (half == 0) F2CGT_ROWS_GO(I, 0, DEAL ? 4 : 0);                          \
     }                                                                            \
-    if (half == 1) F2CGT_ROWS_GO(I, 1);                                          \
-    else if (half == 2) F2CGT_ROWS_GO(I, 2);                                     \
+    if constexpr (DEAL && BITS == 1) {                                           \
+      if (wide) { F2CGT_ROWS_GO(I, 1, 8); break; }                               \
+    }                                                                            \
+    if (half == 1) F2CGT_ROWS_GO(I, 1, DEAL ? 4 : 0);                            \
+    else if (half == 2) F2CGT_ROWS_GO(I, 2, DEAL ? 4 : 0);                       \
   } while (0)
   if (idx_dtype == F2CGT_DT_I32) F2CGT_ROWS_IDX(int32_t);
   else F2CGT_ROWS_IDX(int64_t);
