@@ -1368,9 +1368,9 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
   // 1-bit items of eight columns read a code byte once, but a lane's two 16-byte stores have every store instruction
   // write 16 of every 32 bytes, which streamed stores take to memory as partial lines: streamed outputs take items of
   // four columns, whose stores are contiguous (240000 rows of 256 columns: 115 us with eight, 46 with four at one edge
-  // per row, 81 and 71 at eight; 60001 x 602 at 10 edges per row: 65.6 and 57.8).  Cached outputs take eight columns from
-  // two edges per row on (60000 rows of 128 columns, half an edge per row: 11 against 10 us).
-  const bool wide = DEAL && BITS == 1 && !a.nt_out && avg_deg >= 2.0;
+  // per row, 81 and 71 at eight; 60001 x 602 at 10 edges per row: 65.6 and 57.8).  Cached outputs take eight columns
+  // (1000 rows of 300 columns, one edge per row: 4.0 against 4.4 us; 60000 rows of 128 columns, level).
+  const bool wide = DEAL && BITS == 1 && !a.nt_out;
   a.items_per_row = (int)ceil_div(a.feat_dim, wide ? 8 : 4);
   a.item_magic = (uint32_t)(((1ull << 32) + a.items_per_row - 1) / a.items_per_row);   // items < 64 * 1024: exact
   const double dg = avg_deg > 0.5 ? avg_deg : 0.5;
@@ -1444,10 +1444,7 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
     if constexpr (!STORE_FIXED) {                                                \
       if (half == 0) F2CGT_ROWS_GO(I, 0, DEAL ? 4 : 0);                          \
     }                                                                            \
-    if constexpr (DEAL && BITS == 1) {                                           \
-      if (wide) { F2CGT_ROWS_GO(I, 1, 8); break; }                               \
-    }                                                                            \
-    if (half == 1) F2CGT_ROWS_GO(I, 1, DEAL ? 4 : 0);                            \
+    if (half == 1) F2CGT_ROWS_GO(I, 1, DEAL ? (BITS == 1 ? 8 : 4) : 0);          \
     else if (half == 2) F2CGT_ROWS_GO(I, 2, DEAL ? 4 : 0);                       \
   } while (0)
   if (idx_dtype == F2CGT_DT_I32) F2CGT_ROWS_IDX(int32_t);
@@ -1465,8 +1462,23 @@ int launch_sq_rows(RowsArgs a, const void* indptr, const void* indices, int idx_
   // not divide the workgroup (602 columns: 151 groups on 256 threads).  60001 rows of 602 columns, 10 edges per row:
   // 1 bit 187 -> 73 us, 2 bit 185 -> 77, 4 bit 185 -> 88, 8 bit 243 -> 119; 200000 rows of 128 columns: 1 bit
   // 55 -> 38 us, 2 bit 57 -> 52, 4 bit 64 -> 59, 8 bit 88 -> 67.
+  // Large launches of at most 256 columns with an edge or two per row have too little to deal: the few edges of a block
+  // do not pay for its setup, and the column form takes twice the rows per block.  1 and 2 bit: up to two edges per row,
+  // cached outputs, 100000 rows, 24 MB (one edge per row, column form / items, us: 200000 rows of 128 columns 1 bit 22 / 28,
+  // 2 bit 26 / 26; 240000 rows of 32 columns 2 bit 13 / 15; but 60000 rows of 128 columns 1 bit 12 / 10, 120000 rows of
+  // 300 columns 35 / 31, 480000 rows of 256 columns, streamed, 100 / 91).  8 bit: one edge per row, 50000 rows, 48 MB (200000
+  // rows of 128 columns 24 / 29, 480000, streamed, 50 / 56; 60000 rows of 200 columns 16 / 18; but of 100 11 / 10).
+  // 4 bit: level or ahead with items.
   if constexpr (!AFFINE) {
-    if (a.num_codebooks == 1)
+    const double per_row = a.R > 0 ? (double)a.E / (double)a.R : 1.0;
+    const int64_t values = a.R * (int64_t)a.feat_dim;
+    bool too_little = false;
+    if (BITS == 8) too_little = per_row <= 1.25 && a.R >= 50000 && values >= 12000000;
+    if (BITS <= 2)
+      too_little = per_row <= 2.0 && a.R >= 100000 && values >= 6000000 &&
+                   !stream_output(values * 4, (int64_t)a.feat_dim * 4, per_row);
+    too_little = too_little && a.feat_dim <= 256;
+    if (a.num_codebooks == 1 && !too_little)
       return launch_sq_rows_sized<BITS, AFFINE, 256, true>(a, indptr, indices, idx_dtype, out, st, what);
   }
   // Several codebooks, or column parameters: a lane keeps its columns.  4- and 8-bit rows: 256 threads (twice the

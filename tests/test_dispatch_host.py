@@ -194,3 +194,20 @@ def test_fused_vq_store_form_by_shape():
     assert lanes(1_000_000, 3, 200, 25, 8) == 1 and lanes(300_000, 10, 200, 25, 8) == 2
     assert lanes(1_000_000, 3, 192, 24, 8) == 2 and form(1_000_000, 3, 192, 24, 8, 1_000_000) == (1, 0)
     assert lanes(1_000_000, 3, 224, 7, 32) == 2 and lanes(1_000_000, 3, 600, 19, 32) == 1
+
+
+def test_dealt_items_and_column_form_of_one_codebook():
+    """1-bit rows: items take 256 threads per workgroup, the column form 128."""
+    def block(rows, dim, fanout, n_cb=1, bits=1):
+        rc, plan = plan_log_sq(bits, dim, rows, fanout, n_cb)
+        assert rc == 0 and check_geometry(plan) == "sq_rows_kernel"
+        return plan.block
+    assert block(200000, 128, 10) == 256 and block(200000, 128, 10, n_cb=2) == 128
+    # few edges per row: the column form in large cached launches of narrow rows only
+    for bits in (1, 2):
+        assert block(200000, 128, 1, bits=bits) == 128 and block(200000, 128, 2, bits=bits) == 128
+        assert block(200000, 128, 3, bits=bits) == 256           # more edges per row
+        assert block(99999, 128, 1, bits=bits) == 256            # fewer rows
+        assert block(120000, 300, 1, bits=bits) == 256           # wider rows
+        assert block(480000, 128, 1, bits=bits) == 256           # streamed output (246 MB)
+    assert block(100000, 32, 1, bits=2) == 256                   # fewer values
