@@ -11,8 +11,8 @@
 // workspace the caller passes: up to 256 workgroups each leave their own n * k sums and n counters there, which
 // one workgroup per centre adds up, moves the centre and counts itself in; the last one to arrive decides about
 // the stop.  f2cgt_kmeans_update_static uses a device array of this file (for callers that cannot allocate),
-// which has room for one set of sums: all workgroups add into it in memory, as they do from a workspace when
-// n * k does not fit LDS.
+// which has room for one set of sums: all workgroups add into it in memory, as they do from a workspace where a
+// set per workgroup does not pay (km_by_parts).
 #include "common.hpp"
 
 namespace f2cgt {
@@ -213,28 +213,23 @@ __global__ __launch_bounds__(kKmThreads) void km_merge_kernel(KmArgs a, int part
 #pragma unroll
   for (int w = 0; w < kKmThreads / kWave; ++w) cnt += s_cnt[w];
   const float members = (float)cnt;
-  const int cols = a.k < kKmThreads ? a.k : kKmThreads, side = kKmThreads / cols;   // sets read side by side
-  const int col = t % cols, p0 = t / cols;
-  float d2 = 0.f;
-  for (int j0 = 0; j0 < a.k; j0 += cols) {
-    float s = 0.f;
-    if (p0 < side && j0 + col < a.k) {
-      const float* from = a.sums + (int64_t)c * a.k + j0 + col;
+  const int side = kKmThreads / a.k;                    // sets read side by side (k <= kKmThreads)
+  const int col = t % a.k, p0 = t / a.k;
+  float d2 = 0.f, s = 0.f;
+  if (p0 < side) {
+    const float* from = a.sums + (int64_t)c * a.k + col;
 #pragma unroll 8
-      for (int p = p0; p < parts; p += side) s += from[p * words];
-    }
-    s_part[t] = s;
-    __syncthreads();
-    if (t < cols && j0 + t < a.k && cnt > 0u) {
-      float sum = 0.f;
-      for (int q = 0; q < side; ++q) sum += s_part[q * cols + t];
-      float* centre = a.centers + (int64_t)c * a.k + j0 + t;
-      const float now = sum / members;
-      const float d = now - *centre;
-      d2 += d * d;
-      *centre = now;
-    }
-    __syncthreads();
+    for (int p = p0; p < parts; p += side) s += from[p * words];
+  }
+  s_part[t] = s;
+  __syncthreads();
+  if (t < a.k && cnt > 0u) {
+    float sum = 0.f;
+    for (int q = 0; q < side; ++q) sum += s_part[q * a.k + t];
+    float* centre = a.centers + (int64_t)c * a.k + t;
+    const float now = sum / members;
+    d2 = (now - *centre) * (now - *centre);
+    *centre = now;
   }
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) d2 += __shfl_xor(d2, off);
@@ -279,7 +274,19 @@ int km_check(const char* what, const float* x, const int64_t* l64, const uint8_t
   return 0;
 }
 
-bool km_by_parts(int64_t n, int64_t k) { return n * k + n <= kKmLdsFloats; }
+// Shapes with a set of sums per workgroup: what fits LDS, with the columns of a centre in one pass of km_merge_kernel
+// (wider ones leave its few workgroups a long chain of sets: 2 centres of 1000 columns, 2000 rows, 29 us with one set, 96
+// by parts) and not so many centres that their arrivals at one counter take longer than the sums (2000 x 4, 8000 rows: 53
+// and 70 us; 6000 x 1: 23 and 189; 500 x 4: 22.5 and 21.4).
+bool km_parts_shape(int64_t n, int64_t k) { return n * k + n <= kKmLdsFloats && n <= 512 && k <= kKmThreads; }
+
+// And the rows that pay for the sets: hundreds of centres need a few rows each (500 x 4: 500 rows 11.3 us with one set,
+// 17.4 by parts; 2000 rows 19.4 and 19.6), a few wide ones more parts than 64 rows make (2 x 128: 2000 rows 14.0 and
+// 18.1, 8000 rows 32 and 22; 8 x 128: 8000 rows 19.4 and 22.3; 16 x 128: 2000 rows 20.5 and 18.9).  Narrower ones are level
+// on the device, with two launches for four.
+bool km_by_parts(int64_t m, int64_t n, int64_t k) {
+  return km_parts_shape(n, k) && (n < 256 || m >= 4 * n) && (k <= 64 || n >= 12 || m >= 2500 * n);
+}
 
 int64_t km_bytes(int64_t words) { return (words * 4 + 255) / 256 * 256; }
 
@@ -332,7 +339,7 @@ using namespace f2cgt;
 
 extern "C" int64_t f2cgt_kmeans_update_workspace_bytes(int64_t n, int64_t k) {
   if (n <= 0 || k <= 0) return 0;
-  return km_bytes(km_by_parts(n, k) ? km_parts_words(n, k) : n * k + n);
+  return km_bytes(km_parts_shape(n, k) ? km_parts_words(n, k) : n * k + n);
 }
 
 extern "C" int f2cgt_kmeans_update(const float* x, const int64_t* labels_i64, const uint8_t* labels_u8,
@@ -350,7 +357,7 @@ extern "C" int f2cgt_kmeans_update(const float* x, const int64_t* labels_i64, co
   a.sums = static_cast<float*>(workspace);
   a.counts = reinterpret_cast<uint32_t*>(a.sums + n * k);
   a.m = m; a.n = (int)n; a.k = (int)k; a.rule = stop_rule; a.tol = tol;
-  if (km_by_parts(n, k) && workspace_bytes >= f2cgt_kmeans_update_workspace_bytes(n, k)) return km_run_parts(what, a, as_stream(stream));
+  if (km_by_parts(m, n, k) && workspace_bytes >= f2cgt_kmeans_update_workspace_bytes(n, k)) return km_run_parts(what, a, as_stream(stream));
   return km_run(what, a, as_stream(stream));
 }
 

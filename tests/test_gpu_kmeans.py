@@ -51,7 +51,10 @@ def test_update_step_vs_oracle(m, n, k, u8):
 # sets of partial sums: one, an uneven last one, none full; columns below, at and beyond the 256 that the merge takes in one
 # pass and the 1024 threads that the accumulation steps by
 @pytest.mark.parametrize("m,n,k", [(1, 4, 8), (63, 3, 1), (65, 7, 255), (300, 5, 256), (129, 9, 257), (200, 4, 1024), (131, 3, 1500),
-                                   (16385, 100, 12), (40000, 256, 47)])
+                                   (16385, 100, 12), (40000, 256, 47),
+                                   # both sides of the rows, centres and columns that take a set per workgroup
+                                   (4999, 2, 256), (5000, 2, 256), (500, 11, 64), (500, 11, 65), (500, 12, 65), (1023, 256, 8),
+                                   (1024, 256, 8), (2047, 512, 4), (2048, 512, 4), (2048, 513, 4)])
 def test_update_step_by_partial_sums(m, n, k):
     print("case kmeans_update m=%d n=%d k=%d" % (m, n, k), flush=True)
     rng = np.random.default_rng(m + n + k)
