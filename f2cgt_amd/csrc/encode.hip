@@ -680,7 +680,8 @@ struct SliceArgs {
 // expanded form's bits to cancellation (and send most rows to the exact re-evaluation).
 // SL: the slice form, with rows of any pitch and start (a kernel of its own: the row addressing costs the plain
 // form 2 to 3 %).
-template <int S, int NB, bool PW, bool SL>
+// PACKED: scores that carry their slot (argmin_update_packed).
+template <int S, int NB, bool PW, bool SL, bool PACKED>
 __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kernel(const float* __restrict__ x,
                                                             const float* __restrict__ centers,
                                                             int64_t* __restrict__ lab64,
@@ -689,10 +690,6 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
                                                             float* __restrict__ dist, int64_t ldd,
                                                             SliceArgs sl) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  // Scores that carry their slot: up to 16 dimensions, where the update is as long as the products (1e6 x 16 against
-  // 256 centres, cosine: 78 -> 68 us; L2: 78 -> 74).  From there on the tree's registers cost what its
-  // instructions save (32 dimensions: 118 us either way; 64: 138 -> 179).
-  constexpr bool kPacked = !PW && S == 1;
   int64_t share = blockIdx.x, shares = gridDim.x;
   int slice = 0;
   if (SL && sl.slices > 1) {
@@ -843,7 +840,7 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
     if (cosine) sc = (float)(1.0 / sqrt(cn64 > 1e-60 ? cn64 : 1e-60));
     inv[jj] = sc;
     // padding: finite where the lowest bits of a score are its slot
-    bias[jj] = jj >= n ? (kPacked ? FLT_MAX : INFINITY) : (cosine ? 0.f : cn);
+    bias[jj] = jj >= n ? (PACKED ? FLT_MAX : INFINITY) : (cosine ? 0.f : cn);
     if (jj < n && !cosine) atomicMax(cmax_bits, __float_as_int(cn));
     if (jj < n && cosine && !(cn > 1e-12f)) atomicOr(cmax_bits + 1, 1);   // a centre without a direction
     if (PW && jj < n && cosine) atomicMin(cmax_bits + 3, __float_as_int(cn));
@@ -1044,7 +1041,7 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
     for (int b = 0; b < NB; ++b) { best[b] = INFINITY; second[b] = INFINITY; bv[b] = 0; bct[b] = 0; }
     for (int ct = 0; ct < n_ct; ++ct) {
       floatx16 bz;
-      const bool biased = !kPacked || !cosine || ct * 32 + 32 > n;   // cosine: only a tile with padding has any
+      const bool biased = !PACKED || !cosine || ct * 32 + 32 > n;   // cosine: only a tile with padding has any
       if (biased) {
         const float* bp = bias + ct * 32 + 4 * g;
 #pragma unroll
@@ -1188,7 +1185,7 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[b][v] += bz[v];
           }
-          if constexpr (kPacked) argmin_update_packed(acc[b], ct * 32, best[b], second[b], bct[b]);
+          if constexpr (PACKED) argmin_update_packed(acc[b], ct * 32, best[b], second[b], bct[b]);
           else argmin_update(acc[b], ct * 32, best[b], second[b], bv[b], bct[b]);
         }
       }
@@ -1199,7 +1196,7 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const bool valid = grp * kGroupRows + 32 * b + j < m;
-      const int slot = kPacked ? __float_as_int(best[b]) & 15 : bv[b];
+      const int slot = PACKED ? __float_as_int(best[b]) & 15 : bv[b];
       int bi = bct[b] + 8 * (slot >> 2) + 4 * g + (slot & 3);
       float bs = best[b], sd = second[b];
       {  // merge the two halves of the wave (same x row, disjoint centres)
@@ -1219,7 +1216,7 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
       const float scale = cosine ? sqrtf(xn[b]) * (cdev + 3.5762787e-7f / unit) : xn[b] + cmax;
       float bound = unit * scale + kTinyGap;
       bool ask = false;
-      if (kPacked) {      // the slots: 2^-19 of each of the two
+      if (PACKED) {      // the slots: 2^-19 of each of the two
         bound += 1.92e-6f * (fabsf(bs) + fabsf(sd));
         // padding leads where no real score is a number
         ask = bi >= n || !(scale < finite_below);
@@ -1532,11 +1529,11 @@ int launch_mfma(const float* x, const float* centers, int64_t* l64, uint8_t* l8,
   return launch_status("kmeans_predict");
 }
 
-template <int S, int NB, bool PW = false, bool SL = false>
+template <int S, int NB, bool PW = false, bool SL = false, bool PACKED = false>
 int launch_split(const float* x, const float* centers, int64_t* l64, uint8_t* l8, int64_t m, int n, int k,
                  int metric, int n_pad, size_t lds, hipStream_t st, float* dist = nullptr, int64_t ldd = 0,
                  const SliceArgs* slices = nullptr) {
-  auto kern = predict_split_kernel<S, NB, PW, SL>;
+  auto kern = predict_split_kernel<S, NB, PW, SL, PACKED>;
   if (lds > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1584,8 +1581,14 @@ int predict_split(const float* x, const float* centers, int64_t* l64, uint8_t* l
                   hipStream_t st, const SliceArgs* sl = nullptr) {
   const int n_pad = (int)ceil_div(n, 32) * 32;
   const size_t lds = split_lds(n, k);
+  // Packed scores: from 4 to 16 dimensions, where the update is as long as the products (1e6 x 16 against 256 centres,
+  // cosine: 78 -> 68 us; L2: 78 -> 74).  In fewer dimensions so many centres are close to a row that the wider near-tie
+  // bound sends more rows to the exact evaluation than the update saves (1e6 x 2, 256 centres, cosine: 461 -> 543 us);
+  // in more, the tree's registers cost what its instructions save (32 dimensions: 118 us either way; 64: 138 -> 179).
   switch (ceil_div(k, 16)) {
-    case 1: return launch_split<1, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
+    case 1:
+      if (k < 4) return launch_split<1, 2, false, SL, false>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
+      return launch_split<1, 2, false, SL, true>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
     case 2: return launch_split<2, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
     case 3: return launch_split<3, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
     default: return launch_split<4, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);

@@ -66,9 +66,9 @@ def test_vq_compress_equals_its_slices(dim, k, n):
 
 
 @pytest.mark.parametrize("metric", ["l2", "cosine"])
-@pytest.mark.parametrize("n,k", [(2, 4), (34, 8), (100, 13), (256, 16), (254, 16), (256, 17)])
+@pytest.mark.parametrize("n,k", [(2, 3), (2, 4), (34, 8), (100, 13), (256, 16), (254, 16), (256, 17)])
 def test_kmeans_predict_close_pairs(metric, n, k):
-    """Centres in pairs 2^-10 to 2^-15 of their size apart: up to 16 dimensions the lowest four bits of a score are its slot,
+    """Centres in pairs 2^-10 to 2^-15 of their size apart: from 4 to 16 dimensions the lowest four bits of a score are its slot,
     which changes scores by as much as what tells the two of a pair apart, and some of the slots are padding."""
     rng = np.random.default_rng(n + k)
     x = rng.standard_normal((4000, k)).astype(np.float32)
