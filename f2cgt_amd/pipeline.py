@@ -124,15 +124,27 @@ def sq_metadata(sample):
     return _sq_codebook(lo, hi, magnitude.mean())
 
 
-def _sampled_sq_codebook(features, sample_index, lo, hi):
-    """Codebook of columns [lo, hi) from a gathered sample: on the GPU, or on the host where it does not fit there."""
-    sample = features[sample_index, lo:hi]
-    if not sample.is_cuda:
+def _sampled_sq_codebooks(features, sample_index, column_slice):
+    """The codebooks from a gathered sample: all slices at once up to 2^28 values (1 GB), else one slice at a time,
+    which goes to the host's percentiles where it does not fit the GPU."""
+    feat_dim = features.shape[1]
+    if sample_index.dim() == 1 and sample_index.numel() * feat_dim <= 1 << 28 and not features.requires_grad:
         try:
-            return sq_metadata(sample.cuda())
+            sample = features[sample_index].cuda().float()
+            if _device_takes(*sample.shape, column_slice):
+                return [_sq_codebook(*values) for values in _device_statistics(sample, None, column_slice)]
         except torch.OutOfMemoryError:
             pass
-    return sq_metadata(sample)
+    per_slice = []
+    for lo in range(0, feat_dim, column_slice):
+        sample = features[sample_index, lo:lo + column_slice]
+        try:
+            per_slice.append(sq_metadata(sample.cuda()))
+        except torch.OutOfMemoryError:
+            if sample.is_cuda:
+                raise
+            per_slice.append(sq_metadata(sample))
+    return per_slice
 
 
 def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=None, batch_rows=1_000_000):
@@ -150,8 +162,7 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
         # the sample's rows are read in place
         per_slice = [_sq_codebook(*values) for values in _device_statistics(features, sample_index, column_slice)]
     else:
-        per_slice = [_sampled_sq_codebook(features, sample_index, lo, min(lo + column_slice, feat_dim))
-                     for lo in range(0, feat_dim, column_slice)]
+        per_slice = _sampled_sq_codebooks(features, sample_index, column_slice)
     codebooks = torch.tensor([[float(v) for v in values] for values in per_slice], dtype=torch.float32).reshape(-1, 5).cuda()
     if target_bits <= 8:
         dtype, tdim = torch.int8, int(math.ceil(feat_dim / 8 * target_bits))
