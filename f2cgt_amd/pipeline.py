@@ -86,13 +86,12 @@ def _device_statistics(values, rows, column_slice):
     places = [[_percentile_place(n, q) for q in _PERCENTILES] for n in sizes]
     ranks = [r for per_size in places for place in per_size for r in place[:2]]
     stats = _capi().abs_order_stats(values, rows, column_slice, ranks).cpu().numpy()
-    flags = stats[:, 5].astype(np.int64)
-    if (flags & 2).any():
-        raise IndexError("a sample id lies outside the table's %d rows" % values.shape[0])
     out = []
     for i in range(count):
         last = int(i == count - 1)
-        if flags[i] & 1:
+        if stats[i, 5] >= 2:
+            raise IndexError("a sample id lies outside the table's %d rows" % values.shape[0])
+        if stats[i, 5]:
             lo = hi = np.float32("nan")
         else:
             lo, hi = (_between(np.float32(stats[i, 2 * q]), np.float32(stats[i, 2 * q + 1]), places[last][q][2]) for q in (0, 1))
@@ -163,7 +162,8 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
         per_slice = [_sq_codebook(*values) for values in _device_statistics(features, sample_index, column_slice)]
     else:
         per_slice = _sampled_sq_codebooks(features, sample_index, column_slice)
-    codebooks = torch.tensor([[float(v) for v in values] for values in per_slice], dtype=torch.float32).reshape(-1, 5).cuda()
+    per_slice = [[float(v) for v in values] for values in per_slice]
+    codebooks = (torch.tensor(per_slice, dtype=torch.float32) if per_slice else torch.zeros((0, 5))).cuda()
     if target_bits <= 8:
         dtype, tdim = torch.int8, int(math.ceil(feat_dim / 8 * target_bits))
     elif target_bits <= 16:
