@@ -172,3 +172,26 @@ def test_features_that_require_a_gradient_are_refused():
 def test_row_ids_on_another_device_are_refused():
     with pytest.raises(RuntimeError, match="on the device of x"):
         f2cgt_amd.load().abs_order_stats(torch.rand((30, 8), device="cuda:0"), torch.arange(5, device="cuda:1"), 8, [0, 1, 2, 3] * 2)
+
+
+# tables whose rows have a pitch and start at any float, as a column range of a wider table has them: quads, pairs and single
+# floats per load, whole slices and a ragged last one; with a row list, and all rows without one
+@pytest.mark.parametrize("listed", [True, False])
+@pytest.mark.parametrize("n,d,slice_,start,pitch", [(3001, 32, 16, 4, 40), (3001, 32, 16, 2, 42), (3001, 32, 16, 1, 40), (2000, 30, 8, 6, 36),
+                                                    (2000, 31, 31, 3, 37), (40001, 100, 104, 4, 104), (70, 602, 602, 1, 605), (1, 24, 8, 5, 40)])
+def test_rows_with_a_pitch(listed, n, d, slice_, start, pitch):
+    rng = np.random.default_rng(n + start)
+    wide = rng.standard_normal((n, pitch)).astype(np.float32)
+    wide[:, :start] = wide[:, start + d:] = 1e30                     # what lies between the rows must not be counted
+    table = torch.from_numpy(wide).cuda()[:, start:start + d]
+    rows = rng.integers(-n, n, size=n // 2 + 1) if listed else np.arange(n)
+    m, count = rows.size, (d + slice_ - 1) // slice_
+    ranks = []
+    for w in (min(slice_, d), d - (count - 1) * slice_):
+        ranks += [0, m * w // 3, m * w * 2 // 3, m * w - 1]
+    got = f2cgt_amd.load().abs_order_stats(table, torch.from_numpy(rows).cuda() if listed else None, slice_, ranks).cpu().numpy()
+    sample = np.abs(wide[:, start:start + d][rows])
+    for i in range(count):
+        part = np.sort(sample[:, i * slice_:(i + 1) * slice_].ravel())
+        assert np.array_equal(got[i, :4].astype(np.float32), part[ranks[4:] if i == count - 1 else ranks[:4]]) and got[i, 5] == 0.0
+        assert np.allclose(got[i, 4], part.sum(dtype=np.float64), rtol=part.size * 2.0 ** -52)

@@ -93,3 +93,35 @@ def test_l2_scores_beyond_the_largest_float(n, k):
     assert ((c[None].astype(np.float64) ** 2).sum(2) - 2 * x.astype(np.float64) @ c.T.astype(np.float64)).max() > 3.41e38
     got = capi.kmeans_predict(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), "l2").cpu().numpy()
     assert near.mean() < 0.01 and np.array_equal(got[~near], want[~near])
+
+
+@pytest.mark.parametrize("metric", ["l2", "cosine"])
+@pytest.mark.parametrize("k", [4, 8, 16])
+@pytest.mark.parametrize("what", ["one centre", "zero rows", "all zero", "nan centres", "only nan centres", "infinite centre"])
+def test_scores_that_are_zero_or_no_numbers(what, k, metric):
+    """The same rows and centres with zeros up to 17 dimensions take plain scores: the same labels.  A zero score with a slot
+    in its low bits is a denormal number; a centre that is no number is never nearest."""
+    rng = np.random.default_rng(k)
+    n = 1 if what == "one centre" else 70
+    x, c = rng.standard_normal((1000, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    if what == "zero rows":
+        x[::3], c[5] = 0, 0
+    elif what == "all zero":
+        x[:], c[:] = 0, 0
+    elif what == "nan centres":
+        c[::7, 1] = np.nan
+    elif what == "only nan centres":
+        c[:] = np.nan
+    elif what == "infinite centre":
+        c[9, 0] = np.inf
+
+    def labels(k_pad):
+        pad = [torch.from_numpy(np.pad(a, ((0, 0), (0, k_pad - k)))).cuda() for a in (x, c)]
+        return capi.kmeans_predict(*pad, metric).cpu().numpy()
+
+    got = labels(k)
+    assert got.min() >= 0 and got.max() < n and np.array_equal(got, labels(17))
+    if metric == "cosine" and what == "nan centres":
+        assert not np.isin(got, np.arange(0, n, 7)).any()
+    if what in ("one centre", "all zero", "only nan centres"):
+        assert not got.any()
