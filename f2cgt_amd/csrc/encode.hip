@@ -679,7 +679,9 @@ struct SliceArgs {
 // the centres from every x and centre: data far from the origin would otherwise lose most of the
 // expanded form's bits to cancellation (and send most rows to the exact re-evaluation).
 // SL: the slice form, with rows of any pitch and start (a kernel of its own: the row addressing costs the plain
-// form 2 to 3 %).
+// form 2 to 3 %).  Up to 32 dimensions it is held to three waves per SIMD: at 17 to 32 that keeps three registers in
+// scratch, and two waves without any are slower (300000 x 128, codes of 24 columns, 256 centres: 179 against 189 us; of
+// 32 columns, 64 centres: 62 against 71).
 // PACKED: scores that carry their slot (argmin_update_packed).
 template <int S, int NB, bool PW, bool SL, bool PACKED>
 __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kernel(const float* __restrict__ x,

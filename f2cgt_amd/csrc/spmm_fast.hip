@@ -1148,10 +1148,10 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
   __syncthreads();
 
   if constexpr (ITEM != 0) {
-    // decode + sum: (row, column group) items dealt to the lanes one after the other.  60001 rows of 602 columns at 10
-    // edges per row write 2.5 TB/s with 1-bit codes (staged rows with a column group per lane: 0.77 TB/s).  The two or
-    // three instructions per value (an LDS read and three with the other codes) are 23 us of the 57.8 there and the
-    // output 30; the rest is the trips of a row's dependent loads (offset, id, code).
+    // decode + sum: (row, column group) items dealt to the lanes one after the other.  Bound by instruction issue: 60001
+    // rows of 602 columns, 10 edges per row, 1 bit, execute 30.9 million vector instructions (5.5 per wave of values, ids
+    // and addresses included), 50 us of the 58 at four clocks each; the vector ALUs are active in 99 % of the CUs' busy
+    // clocks.  The output goes out at 2.5 TB/s (staged rows with a column group per lane: 0.9 TB/s).
     constexpr int G = ITEM;                              // columns of an item
     constexpr int GB = G * BITS < 8 ? 1 : G * BITS / 8;  // code bytes that hold them
     const int items = nrows * a.items_per_row;
@@ -1389,13 +1389,13 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
   }
   a.edge_cap = (cap < 8 ? 8 : cap) & ~1;  // even: keeps the staging 8-byte aligned
   int rb = ((int)(0.6 * a.edge_cap / dg) + 4) / 8 * 8;
-  // Direct reads: the source ids alone are kept in LDS and the lanes read the code rows where they are.  An item's
-  // read is 4 bytes (8-bit codes) or covers eight columns (1-bit codes), neighbouring lanes read neighbouring bytes,
-  // and without the staged rows twice the workgroups fit a CU, so this wins for 1- and 8-bit rows at any width, for
-  // rows of more than 128 bytes, and wherever eight rows do not fit the staging (staged / direct, us: 1 bit, 602
-  // columns, 10 edges per row 91 / 73; 8 bit, 128 columns 79 / 67; 2 bit, 602 columns 85 / 75, at 25 edges per row
-  // 247 / 131; 4 bit, 602 columns 152 / 88).  Short 2- and 4-bit rows are better staged (2 bit, 256 columns, 25
-  // edges per row 87 / 96; 4 bit, 100 columns, power-law degrees 34 / 39).
+  // Direct reads: the source ids alone are kept in LDS and the lanes read the code rows where they are.  Neighbouring
+  // lanes read neighbouring bytes, and without the staged rows twice the workgroups fit a CU: 1- and 8-bit rows at any
+  // width, rows of more than 128 bytes, and wherever eight rows do not fit the staging (staged / direct, us, 10 edges per
+  // row: 1 bit, 100000 x 256 37 / 33, 60001 x 602 48 / 51; 8 bit, 200000 x 128 84 / 60; 2 bit, 60001 x 602 57 / 59, at
+  // 25 edges per row 145 / 106; 4 bit 89 / 66).  Shorter 2- and 4-bit rows stay staged: ahead with power-law degrees
+  // (250000 x 100, 2 bit 31 / 36, 4 bit 35 / 38), level to a tenth behind at 10 edges per row (250000 x 128, 2 bit 64 / 61,
+  // 4 bit 71 / 68; 100000 x 256, 4 bit 53 / 47).
   const bool direct = DEAL && (BITS == 1 || BITS == 8 || a.pitch > 128 || (int)(8.0 * dg * 1.1) + 8 > a.edge_cap);
   if (direct) {
     // about two rounds of items per thread for eight columns, four for four; at most 480 edges in a block of more
@@ -1460,8 +1460,8 @@ int launch_sq_rows(RowsArgs a, const void* indptr, const void* indices, int idx_
   // One codebook for all columns (what the encoder writes for scalar codes): no state belongs to a column, and the
   // (row, column group) items go to 256 threads one after the other, so that no lane is idle where a row's groups do
   // not divide the workgroup (602 columns: 151 groups on 256 threads).  60001 rows of 602 columns, 10 edges per row:
-  // 1 bit 187 -> 73 us, 2 bit 185 -> 77, 4 bit 185 -> 88, 8 bit 243 -> 119; 200000 rows of 128 columns: 1 bit
-  // 55 -> 38 us, 2 bit 57 -> 52, 4 bit 64 -> 59, 8 bit 88 -> 67.
+  // 1 bit 159 -> 54 us, 2 bit 131 -> 59, 4 bit 181 -> 66, 8 bit 186 -> 87; 200000 rows of 128 columns: 1 bit
+  // 54 -> 41 us, 2 bit 58 -> 53, 4 bit 65 -> 58, 8 bit 86 -> 60.
   // Large launches of at most 256 columns with an edge or two per row have too little to deal: the few edges of a block
   // do not pay for its setup, and the column form takes twice the rows per block.  1 and 2 bit: up to two edges per row,
   // cached outputs, 100000 rows, 24 MB (one edge per row, column form / items, us: 200000 rows of 128 columns 1 bit 22 / 28,

@@ -274,8 +274,10 @@ int f2cgt_vq_encode_slices(const float* x, int64_t ldx, int64_t feat_dim, const 
  * (sum_c |dc|)^2 < tol, the rule of examples/my_kmeans.py:105; 0: never) -- a training loop can then
  * run without reading anything back per iteration.  workspace: device scratch for the partial sums,
  * f2cgt_kmeans_update_workspace_bytes(n, k) bytes, 16-byte aligned, contents irrelevant (4 (n k + n) bytes, rounded up
- * to 256, are enough for the slower form that adds into one set of sums).
- * The sums are fp32 atomic adds: their last bits depend on the order the hardware takes them in. */
+ * to 256, are enough for the form that adds into one set of sums, which is slower for most shapes that ask for more).
+ * The sums are fp32.  With one set of them all rows are added atomically, in device memory; with a set per workgroup the
+ * rows of a workgroup are, in LDS, and the sets are then added in a fixed order.  Either way the last bits depend on the
+ * order the hardware takes the atomic adds in. */
 int64_t f2cgt_kmeans_update_workspace_bytes(int64_t n, int64_t k);
 int f2cgt_kmeans_update(const float* x, const int64_t* labels_i64, const uint8_t* labels_u8, float* centers,
                         float* shift, int32_t* stop, int stop_rule, float tol, void* workspace,
