@@ -1839,7 +1839,8 @@ __global__ __launch_bounds__(TB) F2CGT_SGPR_AS_SHIPPED void hybrid_acc_kernel(Hy
           add_edge((v & kVqFlag) ? -(int64_t)(v & 0x3fffffffu) - 1 : (int64_t)(v & 0x3fffffffu));
         }
       } else {
-        for (int k = b; k < e; ++k) {
+        const int end = in_lds && e > ne ? ne : e;       // a decreasing offset: no further than the edges s_row holds
+        for (int k = b; k < end; ++k) {
           int64_t m;
           if (in_lds) {
             const uint32_t v = s_row[k];

@@ -66,3 +66,26 @@ def test_affine_sq_with_decreasing_offsets(bits, idx):
             plain = np.arange(rows + 1, dtype=np.int64) * fanout
             want = oc.sq_affine_decompress_spmm_csr(codes, params, plain, indices, bits, feat_dim)
             assert np.allclose(got.cpu().numpy()[sound], want[sound], rtol=1e-5, atol=1e-5 * np.abs(want).max())
+
+
+@pytest.mark.parametrize("idx", [np.int64, np.int32])
+def test_hybrid_with_decreasing_offsets(idx):
+    rng = np.random.default_rng(4)
+    n, n_sq, w = 3000, 1200, 16
+    row_map = np.empty(n, dtype=np.int32)
+    row_map[:n_sq] = rng.permutation(n_sq)
+    row_map[n_sq:] = -rng.permutation(n - n_sq) - 1
+    for feat_dim in (48, 128):
+        sq_codes = rng.integers(0, 256, size=(n_sq, feat_dim), dtype=np.uint8)
+        params = np.stack([rng.standard_normal(feat_dim) - 3, 0.01 + 0.02 * rng.random(feat_dim)]).astype(np.float32)
+        vq_codes = rng.integers(0, 256, size=(n - n_sq, feat_dim // w), dtype=np.uint8)
+        vcb = rng.standard_normal((feat_dim // w, 256, w)).astype(np.float32)
+        for rows, fanout in ((900, 1), (900, 10), (600, 40), (700, 300)):
+            print("case hybrid dim=%d rows=%d fanout=%d" % (feat_dim, rows, fanout), flush=True)
+            indptr, indices, sound = graph(rng, rows, fanout, n)
+            got = capi.hybrid_decompress_spmm_csr(dev(row_map), dev(sq_codes), dev(params), dev(vq_codes), dev(vcb),
+                                                  dev(indptr.astype(idx)), dev(indices.astype(idx)), feat_dim)
+            torch.cuda.synchronize()
+            plain = np.arange(rows + 1, dtype=np.int64) * fanout
+            want = oc.hybrid_decompress_spmm_csr(row_map, sq_codes, params, vq_codes, vcb, plain, indices, feat_dim)
+            assert np.allclose(got.cpu().numpy()[sound], want[sound], rtol=1e-5, atol=8e-5)
