@@ -144,6 +144,29 @@ def test_fused_log_sq_of_one_codebook_equals_that_codebook_given_per_slice(bits,
                     assert np.array_equal(got.cpu().numpy(), want.cpu().numpy(), equal_nan=True), (feat_dim, rows, level, mode)
 
 
+# one codebook with an edge or two per row: the column form on one side of the lines, dealt items on the other
+@pytest.mark.parametrize("bits,rows,dim,fanout", [(1, 99999, 64, 1), (1, 100000, 64, 1), (1, 100000, 66, 2), (1, 100000, 64, 3),
+                                                  (2, 187499, 32, 1), (2, 187500, 32, 1), (2, 100000, 258, 1), (2, 100000, 102, 2),
+                                                  (8, 93749, 128, 1), (8, 93750, 128, 1), (8, 60000, 200, 2), (4, 100000, 66, 1)])
+def test_fused_log_sq_with_few_edges_per_row_equals_unfused(bits, rows, dim, fanout):
+    rng = np.random.default_rng(rows + bits)
+    n = 5000
+    codes = dev(rng.integers(0, 256, size=(n, (dim * bits + 7) // 8), dtype=np.uint8).view(np.int8))
+    cb = dev(np.array([[0.01, 3.0, -6.643856, 1.5849625, 0.4]], dtype=np.float32))
+    indptr = dev(np.arange(rows + 1, dtype=np.int64) * fanout)
+    indices = dev(rng.integers(0, n, size=rows * fanout))
+    width = (dim + 7) // 8 * 8
+    want = capi.spmm_csr(capi.sq_decompress(codes, cb, bits, width, dim), indptr, indices)
+    for mode in (capi.STORE_CACHED, capi.STORE_STREAM):
+        was = capi.set_store_mode(mode)
+        try:
+            got = capi.sq_decompress_spmm_csr(codes, cb, indptr, indices, bits, width, dim)
+            torch.cuda.synchronize()
+        finally:
+            capi.set_store_mode(was)
+        assert torch.equal(got, want), mode
+
+
 @pytest.mark.parametrize("rows", [16383, 16384, 32767, 32768, 65535, 65536, 114687, 114688])
 def test_fused_sq_on_both_sides_of_the_rows_per_block_steps(rows):
     # launches below ~2000 workgroups shrink their row blocks in steps of 8 rows: the integer-accumulating
