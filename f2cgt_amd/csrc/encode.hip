@@ -1,7 +1,7 @@
-// VQ encode: pairwise distance and nearest-centre assignment.
+// VQ encode: pairwise distance, and the nearest-centre assignment of the shapes that assign.hip leaves.
 //
 // pairwise_distance materialises the [m,n] matrix.  With 9 to 64 dimensions the scores come from
-// the matrix cores, as in predict_split_kernel below (its PW mode): |x|^2 + |y|^2 - 2 x.y with x.y
+// the matrix cores (pairwise_split_kernel): |x|^2 + |y|^2 - 2 x.y with x.y
 // from three bf16 pieces per value, after the mean of y has been subtracted from both (L2).  That
 // form loses what x and y have in common, so an entry below an eighth of |x|^2 + |y|^2 is
 // evaluated again as sum((x-y)^2) by its lane (cosine: rows and columns whose |x||y| can reach the
@@ -10,83 +10,25 @@
 // lines, and the matrix write bounds the kernel.  Other dimensions take pairwise_kernel: the
 // unexpanded form with fused multiply-adds on the vector ALUs.
 //
-// kmeans_predict never writes the matrix.  For L2 it works, like pairwise_distance, on x - mu and
-// c - mu (mu = mean of the centres): a common offset of the data then costs nothing, and the rows
-// whose best two centres are closer than the rounding of that subtraction are decided from the
-// original arrays.  For cosine the normalised centres lose their mean direction m when |m| > 1/2
-// (argmin -x . c^ = argmin -x . (c^ - m)): the scores then resolve the differences between the
-// centres' directions, which is all that data far from the origin leaves.  A wave owns rows of x and walks the centres a tile
-// at a time on the matrix core: A = centre tile, B = x tile, so every lane holds 16 centre
-// scores of ONE x row per tile and the running arg-min stays in registers.  Scores use the
-// expanded form (|c|^2 - 2 x.c, the row constant |x|^2 dropped); rows whose two best scores are
-// closer than the rounding bound of that evaluation are re-evaluated exactly in fp64 by the
-// whole wave, so the label is the true first minimum.  Two evaluations of x.c:
-//   * predict_split_kernel (up to 64 dimensions, operands within 96 KB of LDS): every fp32
-//     value as three bf16 pieces, six v_mfma_f32_32x32x16_bf16 per 16 dimensions;
-//   * predict_mfma_kernel: fp32 MFMA (v_mfma_f32_32x32x2_f32).  Vector instructions do not run in
-//     the shadow of fp32 matrix instructions of the same SIMD (measured: a 128-instruction update
-//     per 34 MFMAs costs its full issue time with one to three waves per SIMD), so there the
-//     update is kept to four instructions per score and everything else is folded into the
-//     MFMA operands.
-#include "common.hpp"
-
-#include <cfloat>
-#include <climits>
+// kmeans_predict never writes the matrix.  Up to 64 dimensions with the centres' operands in LDS it is assign_kernel
+// (assign.hip).  Beyond that: predict_mfma_kernel, fp32 MFMA (v_mfma_f32_32x32x2_f32), where a wave owns rows of x and
+// walks the centres a tile at a time; vector instructions do not run in the shadow of fp32 matrix instructions of the
+// same SIMD (measured: a 128-instruction update per 34 MFMAs costs its full issue time with one to three waves per
+// SIMD), so there the update is kept to four instructions per score and everything else is folded into the MFMA
+// operands; predict_tiled_kernel on the vector ALUs; and a wave per row in float64 for a handful of rows.  Scores use the
+// expanded form (|c|^2 - 2 x.c, the row constant |x|^2 dropped); rows whose two best scores are closer than the rounding
+// bound of that evaluation are re-evaluated exactly in fp64 by the whole wave, so the label is the true first minimum.
+#include "assign.hpp"
+#include "assign_exact.hpp"
 
 namespace f2cgt {
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4_dword __attribute__((ext_vector_type(4), aligned(4)));   // loaded from any float's address
 
-// Absolute part of the near-tie bound: the matrix core flushes products (and, for the split form,
-// piece products 2^-8 and 2^-16 of the full one) that fall below the smallest normal fp32 number,
-// which the relative bound does not see.  A few hundred such terms stay below this.
+// Absolute part of the near-tie bound: the matrix core flushes products that fall below the smallest normal fp32
+// number, which the relative bound does not see.  A few hundred such terms stay below this.
 constexpr float kTinyGap = 1e-33f;
-
-// ---- exact assignment of one row by a whole wave (fp64) ------------------------------
-// kx <= k: how many values the row has; it counts as zero in the dimensions after them.
-__device__ int exact_argmin_row(const float* __restrict__ xrow, const float* __restrict__ centers,
-                                int n, int k, int kx, int metric, int lane) {
-  double bestv = DBL_MAX;
-  int besti = INT_MAX;
-  double xn = 0.0;
-  if (metric == F2CGT_METRIC_COSINE)
-    for (int t = 0; t < kx; ++t) xn += (double)xrow[t] * (double)xrow[t];
-  for (int c = lane; c < n; c += kWave) {
-    const float* cr = centers + (int64_t)c * k;
-    double d;
-    if (metric == F2CGT_METRIC_COSINE) {
-      double dot = 0.0, cn = 0.0;
-      for (int t = 0; t < kx; ++t) {
-        dot += (double)xrow[t] * (double)cr[t];
-        cn += (double)cr[t] * (double)cr[t];
-      }
-      for (int t = kx; t < k; ++t) cn += (double)cr[t] * (double)cr[t];
-      double den = sqrt(xn) * sqrt(cn);
-      den = den > 1e-8 ? den : 1e-8;
-      d = 1.0 - dot / den;
-    } else {
-      d = 0.0;
-      for (int t = 0; t < kx; ++t) {
-        const double df = (double)xrow[t] - (double)cr[t];
-        d += df * df;
-      }
-      for (int t = kx; t < k; ++t) d += (double)cr[t] * (double)cr[t];
-    }
-    if (d < bestv) { bestv = d; besti = c; }
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const double ov = __shfl_xor(bestv, off);
-    const int oi = __shfl_xor(besti, off);
-    if (ov < bestv || (ov == bestv && oi < besti)) { bestv = ov; besti = oi; }
-  }
-  // a row without a single comparable distance (NaN or infinite entries) goes to centre 0, where the
-  // callers' trainer sends it (examples/my_kmeans.py:92-94 turns such distances into 1 before the
-  // arg-min); the label must be a valid index whatever the data
-  return besti == INT_MAX ? 0 : besti;
-}
 
 // LDS layout of the MFMA A operands: [pair of 32-centre tiles][step][half][centre % 32][tile of pair].
 // Step 0 is the bias step, step 1 + t holds dimension half * khalf + t.  A lane reads both tiles
@@ -115,16 +57,7 @@ __device__ int exact_argmin_row_l2_lds(const float* __restrict__ xrow, const flo
     }
     if (d < bestv) { bestv = d; besti = c; }
   }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const double ov = __shfl_xor(bestv, off);
-    const int oi = __shfl_xor(besti, off);
-    if (ov < bestv || (ov == bestv && oi < besti)) { bestv = ov; besti = oi; }
-  }
-  // a row without a single comparable distance (NaN or infinite entries) goes to centre 0, where the
-  // callers' trainer sends it (examples/my_kmeans.py:92-94 turns such distances into 1 before the
-  // arg-min); the label must be a valid index whatever the data
-  return besti == INT_MAX ? 0 : besti;
+  return first_minimum(bestv, besti);
 }
 
 // ---- general fallback: one wave per row, exact -------------------------------------------
@@ -311,68 +244,17 @@ __global__ __launch_bounds__(256) void predict_mfma_kernel(const float* __restri
   }
 }
 
-// ---- split-bf16 MFMA path ------------------------------------------------------------------
-// The same scores at the bf16 matrix rate.  An fp32 value is the exact sum of three bf16 pieces
+// ---- pairwise distance from split bf16 ------------------------------------------------------
+// An fp32 value is the exact sum of three bf16 pieces
 // (round to nearest, then the residual, then its residual: 3 x 8 significand bits plus the signs
-// cover 24), a product of two pieces is exact in fp32, and of the nine piece products of x * c the
+// cover 24), a product of two pieces is exact in fp32, and of the nine piece products of x * y the
 // three of relative size <= 2^-24 are dropped, so six v_mfma_f32_32x32x16_bf16 per 16 dimensions
-// give x . c to fp32 accuracy at a sixth of the bf16 rate, 2.7 times the fp32 MFMA rate, and, unlike
-// fp32 MFMA, with the vector ALUs free for the arg-min update while the matrix core runs.  The
-// centre pieces sit in LDS in operand order ([piece][tile][step][lane] x 16 B, one ds_read_b128 per
-// operand), a wave keeps the pieces of NB x 32 rows of x in registers so that every operand read
-// feeds NB instructions, and the bias |c|^2 enters as the C operand of a tile's first instruction.
-// Labels are decided as in the fp32 kernel: rows whose two best scores are closer than the
-// rounding bound of this evaluation are re-evaluated exactly in fp64.
+// give x . y to fp32 accuracy at a sixth of the bf16 rate, 2.7 times the fp32 MFMA rate, and, unlike
+// fp32 MFMA, with the vector ALUs free while the matrix core runs.  The
+// pieces of y (`centers` here) sit in LDS in operand order ([piece][tile][step][lane] x 16 B, one ds_read_b128 per
+// operand), and a wave keeps the pieces of NB x 32 rows of x in registers so that every operand read
+// feeds NB instructions.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-// Three-way minimum of scores with the NaN behaviour of the instruction (the builtin minimum would first quieten
-// each operand with an instruction of its own).  A quiet NaN operand is left out, and the median of a triple with one
-// is its minimum, so that a triple's best is then its second as well and the row ends in the exact evaluation.
-__device__ __forceinline__ float min3_raw(float a, float b, float c) {
-  float d;
-  asm("v_min3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
-  return d;
-}
-__device__ __forceinline__ float min_raw(float a, float b) {
-  float d;
-  asm("v_min_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
-  return d;
-}
-__device__ __forceinline__ float max_raw(float a, float b) {
-  float d;
-  asm("v_max_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
-  return d;
-}
-
-// Running (best, second) over the 16 scores of a tile.  A score carries its slot in its four lowest bits (one
-// v_and_or, a change below 2^-19 of it that the near-tie bound includes), so that the index needs no compare and
-// select of its own and the rest is a tree of three-way minima and medians: 39 instructions for 16 scores where
-// compare, two selects and a median took 64.  Scores have to be finite or quiet NaNs: an infinity with a slot in its low
-// bits is a signalling NaN, which takes the other operands of a minimum with it.  The caller evaluates rows whose scores
-// could overflow exactly.
-__device__ __forceinline__ void argmin_update_packed(const floatx16& acc, int ct, float& best, float& second, int& bct) {
-  float p[16];
-#pragma unroll
-  for (int v = 0; v < 16; ++v) p[v] = __int_as_float((__float_as_int(acc[v]) & ~15) | v);
-  float lo[6], mid[5];
-#pragma unroll
-  for (int i = 0; i < 5; ++i) {
-    lo[i] = min3_raw(p[3 * i], p[3 * i + 1], p[3 * i + 2]);
-    mid[i] = __builtin_amdgcn_fmed3f(p[3 * i], p[3 * i + 1], p[3 * i + 2]);
-  }
-  lo[5] = p[15];
-  const float lo_a = min3_raw(lo[0], lo[1], lo[2]), mid_a = __builtin_amdgcn_fmed3f(lo[0], lo[1], lo[2]);
-  const float lo_b = min3_raw(lo[3], lo[4], lo[5]), mid_b = __builtin_amdgcn_fmed3f(lo[3], lo[4], lo[5]);
-  const float before = best;
-  const float behind_a = max_raw(best, lo_a);
-  best = min_raw(best, lo_a);
-  const float behind_b = max_raw(best, lo_b);
-  best = min_raw(best, lo_b);
-  const float s0 = min3_raw(mid[0], mid[1], mid[2]), s1 = min3_raw(mid[3], mid[4], mid_a);
-  second = min3_raw(second, s0, s1);
-  second = min3_raw(second, mid_b, min_raw(behind_a, behind_b));
-  bct = best < before ? ct : bct;
-}
 
 __device__ __forceinline__ void split3(float v, __bf16& p0, __bf16& p1, __bf16& p2) {
   p0 = (__bf16)v;
@@ -382,342 +264,24 @@ __device__ __forceinline__ void split3(float v, __bf16& p0, __bf16& p1, __bf16& 
   p2 = (__bf16)r;
 }
 
-// Exact L2 assignment of one row by a whole wave from the centre pieces in LDS (their sum is the
-// fp32 centre, exactly); same result as exact_argmin_row on the array in HBM.  The unexpanded fp32
-// distance has relative error <= (k + 3) 2^-24 (all terms positive), so it decides which centres
-// can be the minimum at all; only those, usually two, are evaluated in fp64.
-// The pieces hold the centres minus mu and the row is compared as fl(x - mu): the decision is exact
-// for those rounded vectors, whose distances differ from the original ones by at most
-// 2^-22 (|x - mu|^2 + |c - mu|^2) each.  When the best two are closer than twice that, the original
-// row decides between them (fp64, from the arrays in HBM); with three or more that close the
-// function returns -1 - (its choice) and the caller evaluates every centre.
-template <int S>
-__device__ __forceinline__ int exact_argmin_row_l2_pieces(const float* __restrict__ xrow, float* xs, const bf16x8* ap, int n, int n_ct,
-                                          int k, int kx, int lane, const float* mu, float cmax,
-                                          const float* __restrict__ centers) {
-  // the row goes through a wave-private LDS slot (16 S floats, zero padded) and the loops over the
-  // 8-dimension chunks stay rolled: this rare path must not raise the kernel's register count
-  const int piece_stride = n_ct * S * 64;                // operands per piece
-  if (lane < 16 * S) xs[lane] = lane < k ? (lane < kx ? xrow[lane] : 0.f) - mu[lane] : 0.f;
-  __builtin_amdgcn_wave_barrier();                       // LDS operations of one wave execute in order
-  // fp32 centre values of chunk ch (dimensions [8 ch, 8 ch + 8)) of centre c: one operand per piece
-  auto centre8 = [&](int c, int ch, float (&cv)[8]) {
-    const bf16x8* q = ap + (c >> 5) * S * 64 + (ch >> 1) * 64 + (ch & 1) * 32 + (c & 31);
-    const bf16x8 p0 = q[0], p1 = q[piece_stride], p2 = q[2 * piece_stride];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) cv[e] = ((float)p0[e] + (float)p1[e]) + (float)p2[e];
-  };
-  // first pass: distance from the leading pieces only (relative error of a centre value 2^-8),
-  // one operand per chunk
-  auto dist_lead = [&](int c) -> float {
-    float d = 0.f;
-#pragma nounroll
-    for (int ch = 0; ch < 2 * S; ++ch) {
-      const bf16x8 p0 = ap[(c >> 5) * S * 64 + (ch >> 1) * 64 + (ch & 1) * 32 + (c & 31)];
-      const float4 xa = *reinterpret_cast<const float4*>(xs + 8 * ch);
-      const float4 xb = *reinterpret_cast<const float4*>(xs + 8 * ch + 4);
-      const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float df = xv[e] - (float)p0[e];
-        d = __fmaf_rn(df, df, d);
-      }
-    }
-    return d;
-  };
-  auto dist32 = [&](int c) -> float {
-    float d = 0.f;
-#pragma nounroll
-    for (int ch = 0; ch < 2 * S; ++ch) {
-      float cv[8];
-      centre8(c, ch, cv);
-      const float4 xa = *reinterpret_cast<const float4*>(xs + 8 * ch);
-      const float4 xb = *reinterpret_cast<const float4*>(xs + 8 * ch + 4);
-      const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float df = xv[e] - cv[e];                  // dimensions >= k hold zeros on both sides
-        d = __fmaf_rn(df, df, d);
-      }
-    }
-    return d;
-  };
-  // With c' the leading pieces (8 significant bits, round to nearest), |c - c'| <= 2^-8 |c| per
-  // component, so | sqrt(d) - sqrt(d') | <= 2^-8 |c| <= 2^-8 (|x| + sqrt(d)): the centre c0 with the
-  // smallest d' has sqrt(d0) <= (sqrt(dmin') + 2^-8 |x|) / (1 - 2^-8), the true minimum is no
-  // farther, and so its own sqrt(d') <= (sqrt(dmin') + 2^-7 |x|) * (1 + 2^-6) (slack for the fp32
-  // sums included).
-  constexpr int kKeep = 4;            // first-pass distances kept in registers (all of them up to 256 centres)
-  float dkeep[kKeep] = {0.f, 0.f, 0.f, 0.f};
-  float dmin = INFINITY;
-  // the lane's first four centres two at a time: two independent chains per chunk
-#pragma unroll
-  for (int i0 = 0; i0 < kKeep; i0 += 2) {
-    int slot[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      int c = lane + (i0 + i) * kWave;
-      c = c < n ? c : 0;
-      slot[i] = (c >> 5) * S * 64 + (c & 31);
-    }
-#pragma nounroll
-    for (int ch = 0; ch < 2 * S; ++ch) {
-      const int at = (ch >> 1) * 64 + (ch & 1) * 32;
-      const bf16x8 pa = ap[slot[0] + at], pb = ap[slot[1] + at];
-      const float4 xa = *reinterpret_cast<const float4*>(xs + 8 * ch);
-      const float4 xb = *reinterpret_cast<const float4*>(xs + 8 * ch + 4);
-      const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float da = xv[e] - (float)pa[e], db = xv[e] - (float)pb[e];
-        dkeep[i0] = __fmaf_rn(da, da, dkeep[i0]);
-        dkeep[i0 + 1] = __fmaf_rn(db, db, dkeep[i0 + 1]);
-      }
-    }
-    asm volatile("" ::: "memory");
-  }
-#pragma unroll
-  for (int i = 0; i < kKeep; ++i) {
-    if (lane + i * kWave >= n) dkeep[i] = INFINITY;
-    dmin = fminf(dmin, dkeep[i]);
-  }
-  for (int c = lane + kKeep * kWave; c < n; c += kWave) dmin = fminf(dmin, dist_lead(c));
-  float xnorm2 = lane < 16 * S ? xs[lane] * xs[lane] : 0.f;
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    dmin = fminf(dmin, __shfl_xor(dmin, off));
-    xnorm2 += __shfl_xor(xnorm2, off);
-  }
-  // centres whose exact distance is within `margin` of the smallest must reach the fp64 stage, so
-  // that everything left out is known to be farther than that (2^-21 = 4.77e-7; the constants
-  // leave room for the fp32 evaluation of the norms)
-  const float marginf = 5.2e-7f * (xnorm2 + cmax);
-  const float reach = (sqrtf(dmin) + 0.0078125f * sqrtf(xnorm2) + sqrtf(marginf)) * 1.015625f;
-  const float lead_limit = reach * reach * 1.0001f + 1e-37f;
-  // second pass: full fp32 distance of the survivors, then the exact fp64 one of those that can
-  // still be the minimum (relative error of the fp32 sum <= (k + 3) 2^-24, all terms positive)
-  float d32min = INFINITY;
-#pragma unroll
-  for (int i = 0; i < kKeep; ++i) {      // the kept distances become the fp32 ones
-    const int c = lane + i * kWave;
-    dkeep[i] = (c < n && dkeep[i] <= lead_limit) ? dist32(c) : INFINITY;
-    d32min = fminf(d32min, dkeep[i]);
-    asm volatile("" ::: "memory");
-  }
-  for (int c = lane + kKeep * kWave; c < n; c += kWave)
-    if (dist_lead(c) <= lead_limit) d32min = fminf(d32min, dist32(c));
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) d32min = fminf(d32min, __shfl_xor(d32min, off));
-  const float limit = d32min * (1.f + 1.1920929e-7f * (float)(k + 4)) + 1e-37f + marginf;
-  double bestv = DBL_MAX, nextv = DBL_MAX, thirdv = DBL_MAX;   // the three smallest exact distances
-  int besti = INT_MAX, nexti = INT_MAX;
-  for (int c = lane, i = 0; c < n; c += kWave, ++i) {
-    float d32 = dkeep[0];
-#pragma unroll
-    for (int q = 1; q < kKeep; ++q) d32 = i == q ? dkeep[q] : d32;
-    if (i >= kKeep) d32 = dist_lead(c) <= lead_limit ? dist32(c) : INFINITY;
-    if (!(d32 <= limit)) continue;
-    double dd = 0.0;
-#pragma nounroll
-    for (int ch = 0; ch < 2 * S; ++ch) {
-      float cv[8];
-      centre8(c, ch, cv);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const double df = (double)xs[8 * ch + e] - (double)cv[e];
-        dd += df * df;
-      }
-    }
-    if (dd < bestv) { thirdv = nextv; nextv = bestv; nexti = besti; bestv = dd; besti = c; }
-    else if (dd < nextv) { thirdv = nextv; nextv = dd; nexti = c; }
-    else if (dd < thirdv) thirdv = dd;
-  }
-  // merge of two sorted triples (a lane's centres ascend, and ties go to the smaller index)
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const double ob = __shfl_xor(bestv, off), on = __shfl_xor(nextv, off), ot = __shfl_xor(thirdv, off);
-    const int oi = __shfl_xor(besti, off), oj = __shfl_xor(nexti, off);
-    double m1, m2, m3;
-    int i1, i2;
-    if (ob < bestv || (ob == bestv && oi < besti)) {       // the other triple leads
-      m1 = ob; i1 = oi;
-      if (on < bestv || (on == bestv && oj < besti)) { m2 = on; i2 = oj; m3 = ot < bestv ? ot : bestv; }
-      else { m2 = bestv; i2 = besti; m3 = on < nextv ? on : nextv; }
-    } else {
-      m1 = bestv; i1 = besti;
-      if (ob < nextv || (ob == nextv && oi < nexti)) { m2 = ob; i2 = oi; m3 = on < nextv ? on : nextv; }
-      else { m2 = nextv; i2 = nexti; m3 = ob < thirdv ? ob : thirdv; }
-    }
-    bestv = m1; besti = i1; nextv = m2; nexti = i2; thirdv = m3;
-  }
-  const double margin = 4.9e-7 * ((double)xnorm2 + (double)cmax);
-  // no candidate at all (a row with NaN or infinite entries: nothing compares below the limit), or one:
-  // the stages below index the centres with besti and nexti and must not see INT_MAX
-  if (besti == INT_MAX) return 0;
-  if (nexti == INT_MAX) return besti;
-  if (nextv - bestv > margin) return besti;
-  if (thirdv - bestv <= margin) return -1 - besti;       // three or more: the caller takes every centre
-  // exactly two centres can be the nearest one of the original row: decide between them there
-  double da = 0.0, db = 0.0;
-  for (int t = lane; t < k; t += kWave) {
-    const double xv = t < kx ? (double)xrow[t] : 0.0;
-    const double ea = xv - (double)centers[(int64_t)besti * k + t], eb = xv - (double)centers[(int64_t)nexti * k + t];
-    da += ea * ea;
-    db += eb * eb;
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    da += __shfl_xor(da, off);
-    db += __shfl_xor(db, off);
-  }
-  const int lo = besti < nexti ? besti : nexti, hi = besti < nexti ? nexti : besti;
-  const double dlo = besti < nexti ? da : db, dhi = besti < nexti ? db : da;
-  return dhi < dlo ? hi : lo;
-}
-
-// Exact cosine assignment of one row by a whole wave.  The LDS pieces hold d = c / |c| - m (m: the
-// mean direction or zero, the same for every centre, so x . m does not matter), |d| <= cdev; with
-// d' their leading pieces, |x . d - x . d'| <= 2^-8 |x| cdev (1 + 2^-20), so only
-// centres whose leading-piece dot product is within 2^-6 |x| cdev of the largest can have the smallest
-// distance; those go through the fp32 dot product with all three pieces, and what that leaves is
-// evaluated exactly, in fp64 from the centres in HBM, by the formula of exact_argmin_row.  Needs every centre to have a direction (|c|^2 > 1e-12).
-template <int S>
-__device__ __forceinline__ int exact_argmin_row_cosine_pieces(const float* __restrict__ xrow, float* xs, const bf16x8* ap,
-                                              const float* __restrict__ centers, int n, int n_ct, int k,
-                                              int kx, int lane, float cdev) {
-  if (lane < 16 * S) xs[lane] = lane < kx ? xrow[lane] : 0.f;
-  __builtin_amdgcn_wave_barrier();
-  float xnorm2 = lane < 16 * S ? xs[lane] * xs[lane] : 0.f;
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) xnorm2 += __shfl_xor(xnorm2, off);
-  auto dot_lead = [&](int c) -> float {
-    float d = 0.f;
-#pragma nounroll
-    for (int ch = 0; ch < 2 * S; ++ch) {
-      const bf16x8 p0 = ap[(c >> 5) * S * 64 + (ch >> 1) * 64 + (ch & 1) * 32 + (c & 31)];
-      const float4 xa = *reinterpret_cast<const float4*>(xs + 8 * ch);
-      const float4 xb = *reinterpret_cast<const float4*>(xs + 8 * ch + 4);
-      const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) d = __fmaf_rn(xv[e], (float)p0[e], d);
-    }
-    return d;
-  };
-  float smax = -INFINITY;
-  for (int c = lane; c < n; c += kWave) smax = fmaxf(smax, dot_lead(c));
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) smax = fmaxf(smax, __shfl_xor(smax, off));
-  const float floor_s = smax - 0.015625f * cdev * sqrtf(xnorm2) - 1e-30f;
-  // second filter: the fp32 dot product with the whole operand (the sum of its pieces) is within
-  // ((k + 2) cdev + 3) 2^-24 |x| of x . (c / |c| - m) (the sum; the roundings of 1 / |c|, of the
-  // product and of the subtraction), so the nearest centre is within twice that of the largest one.  Data far from the origin passes
-  // the first filter with every centre; this one leaves the few that the fp64 stage has to read.
-  auto dot32 = [&](int c) -> float {
-    float d = 0.f;
-    const int piece_stride = n_ct * S * 64;
-#pragma nounroll
-    for (int ch = 0; ch < 2 * S; ++ch) {
-      const bf16x8* q = ap + (c >> 5) * S * 64 + (ch >> 1) * 64 + (ch & 1) * 32 + (c & 31);
-      const bf16x8 p0 = q[0], p1 = q[piece_stride], p2 = q[2 * piece_stride];
-      const float4 xa = *reinterpret_cast<const float4*>(xs + 8 * ch);
-      const float4 xb = *reinterpret_cast<const float4*>(xs + 8 * ch + 4);
-      const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) d = __fmaf_rn(xv[e], ((float)p0[e] + (float)p1[e]) + (float)p2[e], d);
-    }
-    return d;
-  };
-  float s32max = -INFINITY;
-  for (int c = lane; c < n; c += kWave)
-    if (dot_lead(c) >= floor_s) s32max = fmaxf(s32max, dot32(c));
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) s32max = fmaxf(s32max, __shfl_xor(s32max, off));
-  const float floor32 = s32max - 1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) * sqrtf(xnorm2) * 1.001f - 1e-30f;
-  double xn = 0.0;
-  for (int t = 0; t < kx; ++t) xn += (double)xrow[t] * (double)xrow[t];
-  double bestv = DBL_MAX;
-  int besti = INT_MAX;
-  for (int c = lane; c < n; c += kWave) {
-    if (!(dot_lead(c) >= floor_s)) continue;
-    if (!(dot32(c) >= floor32)) continue;
-    const float* cr = centers + (int64_t)c * k;
-    double dot = 0.0, cn = 0.0;
-    for (int t = 0; t < kx; ++t) {
-      dot += (double)xrow[t] * (double)cr[t];
-      cn += (double)cr[t] * (double)cr[t];
-    }
-    for (int t = kx; t < k; ++t) cn += (double)cr[t] * (double)cr[t];
-    double den = sqrt(xn) * sqrt(cn);
-    den = den > 1e-8 ? den : 1e-8;
-    const double d = 1.0 - dot / den;
-    if (d < bestv) { bestv = d; besti = c; }
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const double ov = __shfl_xor(bestv, off);
-    const int oi = __shfl_xor(besti, off);
-    if (ov < bestv || (ov == bestv && oi < besti)) { bestv = ov; besti = oi; }
-  }
-  // a row without a single comparable distance (NaN or infinite entries) goes to centre 0, where the
-  // callers' trainer sends it (examples/my_kmeans.py:92-94 turns such distances into 1 before the
-  // arg-min); the label must be a valid index whatever the data
-  return besti == INT_MAX ? 0 : besti;
-}
-
-// One launch labels several column slices of a table, each against its own centres (slices == 1: rows of ldx
-// floats, labels label_stride apart).  The grid is a multiple of 8 * slices workgroups then.
-struct SliceArgs {
-  int slices;
-  int feat_dim;            // columns of the table; the last slice may have fewer than k
-  int64_t ldx, label_stride;
-};
-
-// PW = false: labels of the nearest centre (KMeans.predict).  PW = true: the distance matrix itself
-// (pairwise_distance), dist[row * ldd + centre], from the same scores.  The squared L2 distance
+// The squared L2 distance
 // does not change when one vector is subtracted from both arguments, and fl(v - mu) carries a
-// relative error of 2^-24 of the difference itself, so for L2 both modes first subtract the mean of
+// relative error of 2^-24 of the difference itself, so for L2 the kernel first subtracts the mean of
 // the centres from every x and centre: data far from the origin would otherwise lose most of the
-// expanded form's bits to cancellation (and send most rows to the exact re-evaluation).
-// SL: the slice form, with rows of any pitch and start (a kernel of its own: the row addressing costs the plain
-// form 2 to 3 %).  Up to 32 dimensions it is held to three waves per SIMD: at 17 to 32 that keeps three registers in
-// scratch, and two waves without any are slower (300000 x 128, codes of 24 columns, 256 centres: 179 against 189 us; of
-// 32 columns, 64 centres: 62 against 71).
-// PACKED: scores that carry their slot (argmin_update_packed).
-template <int S, int NB, bool PW, bool SL, bool PACKED>
-__global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kernel(const float* __restrict__ x,
-                                                            const float* __restrict__ centers,
-                                                            int64_t* __restrict__ lab64,
-                                                            uint8_t* __restrict__ lab8, int64_t m,
-                                                            int n, int k, int metric, int n_pad,
-                                                            float* __restrict__ dist, int64_t ldd,
-                                                            SliceArgs sl) {
+// expanded form's bits to cancellation.
+template <int S, int NB>
+__global__ __launch_bounds__(256, 1) void pairwise_split_kernel(const float* __restrict__ x, const float* __restrict__ centers,
+                                                                int64_t m, int n, int k, int metric, int n_pad,
+                                                                float* __restrict__ dist, int64_t ldd) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  int64_t share = blockIdx.x, shares = gridDim.x;
-  int slice = 0;
-  if (SL && sl.slices > 1) {
-    // Workgroups go round-robin to the 8 XCDs: with 8 shares side by side, the slices of a share run on one
-    // XCD, whose L2 then serves the lines of x that two slices have in common and joins their code bytes.
-    const int turn = blockIdx.x / (8 * sl.slices), at = blockIdx.x % (8 * sl.slices);
-    slice = at >> 3;
-    share = turn * 8 + (at & 7);
-    shares = gridDim.x / sl.slices;
-    x += slice * k;
-    centers += (int64_t)slice * n * k;
-    lab8 += slice;
-  }
-  int kx = SL ? sl.feat_dim - slice * k : k;                     // dimensions the rows have (zeros after them)
-  kx = kx < k ? kx : k;
-  const int64_t ldx = SL ? sl.ldx : k;
-  const int64_t ldl = SL ? sl.label_stride : 1;
   const int n_ct = n_pad >> 5;                                   // 32-centre tiles
   bf16x8* ap = reinterpret_cast<bf16x8*>(smem_raw);              // [3][n_ct][S][64]
   float* bias = reinterpret_cast<float*>(smem_raw + (size_t)3 * n_ct * S * 64 * 16);   // [n_pad]
   float* inv = bias + n_pad;                                     // [n_pad] 1 / |c| (cosine) or 1
   int* cmax_bits = reinterpret_cast<int*>(inv + n_pad);
-  float* xs = reinterpret_cast<float*>(cmax_bits + 4) + (threadIdx.x >> 6) * 16 * S;   // one row of x per wave
-  float* mu = reinterpret_cast<float*>(cmax_bits + 4) + 4 * 16 * S;                    // [16 S]
+  float* mu = reinterpret_cast<float*>(cmax_bits + 4);                                 // [16 S]
   constexpr int kTrPitch = 36;
-  float* tr = mu + 16 * S + (threadIdx.x >> 6) * 32 * kTrPitch;                        // PW only
+  float* tr = mu + 16 * S + (threadIdx.x >> 6) * 32 * kTrPitch;
   const bool cosine = metric == F2CGT_METRIC_COSINE;
   if (threadIdx.x == 0) { cmax_bits[0] = 0; cmax_bits[1] = 0; cmax_bits[2] = 0; cmax_bits[3] = 0x7f800000; }
   // Staging works on items (centre, chunk of 8 dimensions) = one half-operand, four items per
@@ -842,70 +406,11 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
     if (cosine) sc = (float)(1.0 / sqrt(cn64 > 1e-60 ? cn64 : 1e-60));
     inv[jj] = sc;
     // padding: finite where the lowest bits of a score are its slot
-    bias[jj] = jj >= n ? (PACKED ? FLT_MAX : INFINITY) : (cosine ? 0.f : cn);
-    if (jj < n && !cosine) atomicMax(cmax_bits, __float_as_int(cn));
+    bias[jj] = jj >= n ? INFINITY : (cosine ? 0.f : cn);
     if (jj < n && cosine && !(cn > 1e-12f)) atomicOr(cmax_bits + 1, 1);   // a centre without a direction
-    if (PW && jj < n && cosine) atomicMin(cmax_bits + 3, __float_as_int(cn));
+    if (jj < n && cosine) atomicMin(cmax_bits + 3, __float_as_int(cn));
   }
   __syncthreads();
-  // Cosine assignment: argmin_c -x . c^ = argmin_c -x . (c^ - m) for any m, and with m the mean of
-  // the normalised centres c^ the operands of the matrix core shrink to the spread of the centres'
-  // directions: what data far from the origin leaves of the evaluation's resolution goes to the
-  // differences between centres.  Used when |m| > 1/2; mu[] then holds m (zeros otherwise).
-  if (!PW && cosine) {
-    float* psum = reinterpret_cast<float*>(smem_raw);            // [4][64]
-    const int t = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const bool degenerate = cmax_bits[1] != 0;
-    if (cvec) {
-      // as for the L2 mean: a float4 column of every 16th row per lane, sixteen loads in flight
-      const int col = t & 15, part = threadIdx.x >> 4;
-      float4 a4 = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (!degenerate && 4 * col < k) {
-        const float* base = centers + 4 * col;
-        int c = part;
-        for (; c + 16 * 15 < n; c += 16 * 16) {
-          float4 v[16];
-#pragma unroll
-          for (int u = 0; u < 16; ++u) v[u] = *reinterpret_cast<const float4*>(base + (int64_t)(c + 16 * u) * k);
-#pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            const float sc = inv[c + 16 * u];
-            a4.x = __fmaf_rn(v[u].x, sc, a4.x); a4.y = __fmaf_rn(v[u].y, sc, a4.y);
-            a4.z = __fmaf_rn(v[u].z, sc, a4.z); a4.w = __fmaf_rn(v[u].w, sc, a4.w);
-          }
-        }
-        for (; c < n; c += 16) {
-          const float4 v = *reinterpret_cast<const float4*>(base + (int64_t)c * k);
-          const float sc = inv[c];
-          a4.x = __fmaf_rn(v.x, sc, a4.x); a4.y = __fmaf_rn(v.y, sc, a4.y);
-          a4.z = __fmaf_rn(v.z, sc, a4.z); a4.w = __fmaf_rn(v.w, sc, a4.w);
-        }
-      }
-#pragma unroll
-      for (int off = 16; off <= 32; off <<= 1) {
-        a4.x += __shfl_xor(a4.x, off); a4.y += __shfl_xor(a4.y, off);
-        a4.z += __shfl_xor(a4.z, off); a4.w += __shfl_xor(a4.w, off);
-      }
-      if (t < 16) *reinterpret_cast<float4*>(psum + wv * 64 + 4 * t) = a4;
-    } else {
-      float sum = 0.f;
-      if (!degenerate && t < k)
-        for (int c = wv; c < n; c += 4) sum = __fmaf_rn(centers[(int64_t)c * k + t], inv[c], sum);
-      psum[wv * 64 + t] = sum;
-    }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-      const float mt = ((psum[t] + psum[64 + t]) + (psum[128 + t] + psum[192 + t])) / (float)n;
-      float m2 = mt * mt;
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) m2 += __shfl_xor(m2, off);
-      const bool use = !degenerate && m2 > 0.25f;
-      if (t < 16 * S) mu[t] = use ? mt : 0.f;
-      if (t == 0) cmax_bits[3] = use ? 1 : 0;
-    }
-    __syncthreads();
-  }
-  float dev2max = 0.f;
   for (int i0 = threadIdx.x; i0 < n_items; i0 += blockDim.x * 4) {
     float v[4][8];
 #pragma unroll
@@ -920,17 +425,12 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
       const int c = it / kChunks, ch = it % kChunks;
       const float sc = inv[c];
       bf16x8 p0, p1, p2;
-      float dev2 = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        float val = v[u][e] * sc;
-        if (cosine) val = (c < n && 8 * ch + e < k) ? val - mu[8 * ch + e] : 0.f;
-        dev2 = __fmaf_rn(val, val, dev2);
         __bf16 a0, a1, a2;
-        split3(val, a0, a1, a2);
+        split3(v[u][e] * sc, a0, a1, a2);
         p0[e] = a0; p1[e] = a1; p2[e] = a2;
       }
-      dev2max = fmaxf(dev2max, dev2);                            // largest 8-dimension share of |c^ - m|^2
       // chunk ch of centre c is lane (c % 32) + 32 (ch % 2) of step ch / 2 of tile c / 32
       const int at = ((c >> 5) * S + (ch >> 1)) * 64 + (ch & 1) * 32 + (c & 31);
       ap[at] = p0;
@@ -938,45 +438,22 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
       ap[2 * n_ct * S * 64 + at] = p2;
     }
   }
-  if (cosine) {                                                  // one LDS atomic per wave
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) dev2max = fmaxf(dev2max, __shfl_xor(dev2max, off));
-    if ((threadIdx.x & 63) == 0) atomicMax(cmax_bits, __float_as_int(dev2max));
-  }
   __syncthreads();
-  const float cmax = __int_as_float(cmax_bits[0]);
   const bool use_mu = centred && __builtin_amdgcn_readfirstlane(cmax_bits[3]) != 0;
-  const bool plain_cosine = cmax_bits[1] != 0;   // degenerate centres: no candidate filter for cosine
-  // cosine: upper bound of |c^ - m| over the centres (1 without the mean; never above 2)
-  float cdev = 1.f;
-  if (!PW && cosine && !plain_cosine && cmax_bits[3] == 1) {
-    cdev = sqrtf((float)kChunks * cmax) * 1.0001f;
-    cdev = cdev < 2.f ? cdev : 2.f;
-  }
-  cdev = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(cdev)));
-  const float cmin_norm = sqrtf(__int_as_float(cmax_bits[3]));   // PW, cosine: smallest |c|
+  const bool plain_cosine = cmax_bits[1] != 0;   // a centre without a direction
+  const float cmin_norm = sqrtf(__int_as_float(cmax_bits[3]));   // cosine: smallest |c|
 
   const int lane = threadIdx.x & 63;
   const int j = lane & 31;
   const int g = lane >> 5;
   constexpr int kGroupRows = 32 * NB;
   const int64_t n_groups = (m + kGroupRows - 1) / kGroupRows;
-  // Error bound of one score in units of 2^-24 (|x|^2 + max |c|^2), which is >= 2 |x||c| = P and
-  // >= |c|^2: each of the S leading instructions cuts its 17 addends at 2^-22 of the largest
-  // (<= P): 68 S; the small pairs (2^-8 P and below) together stay below 4; the bias sum k + 1;
-  // its addition 2; the dropped pairs (2^-24 P each way) 2; the rounding of x - mu and c - mu 4
-  // (L2: 2^-22 (|x|^2 + |c|^2)); 3 spare.  Doubled for the two scores of a gap.
-  const float unit = 5.9604645e-8f * (float)(2 * (68 * S + k + 16));
   const float xscale = cosine ? -1.f : -2.f;
   const bool vec4 = (k % 8 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0);
-  // Packed scores have to be finite.  An L2 score |c|^2 - 2 x . c is at most 2 (|x|^2 + |c|^2), which may exceed the
-  // largest float (3.4e38) while the bound above is finite; cosine has |x . c^| <= |x|, below 2e19 wherever |x|^2 is finite.
-  const float finite_below = cosine ? INFINITY : 1.6e38f;
-  const bool wide = kx >= 8;      // a row holds the eight values that an idle lane reads from row 0
   // A workgroup owns a contiguous share of the row groups and its four waves draw from it through
   // a counter in LDS: a wave held up by exact re-evaluations simply takes fewer groups.
-  const int64_t per_wg = (n_groups + shares - 1) / shares;
-  const int64_t wg_lo = share * per_wg;
+  const int64_t per_wg = (n_groups + gridDim.x - 1) / gridDim.x;
+  const int64_t wg_lo = (int64_t)blockIdx.x * per_wg;
   const int64_t wg_hi = wg_lo + per_wg < n_groups ? wg_lo + per_wg : n_groups;
   for (;;) {
     int draw = 0;
@@ -994,32 +471,16 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
       for (int st = 0; st < S; ++st) {
         const int kk0 = 16 * st + 8 * g;
         float q[8];
-        if (!SL && vec4) {
+        if (vec4) {
           const bool in = valid && kk0 < k;                   // loads always issued, from row 0 when idle
           const float4* xp4 = reinterpret_cast<const float4*>(x + (in ? row * k + kk0 : 0));
           const float4 u = xp4[0], w = xp4[1];
           q[0] = u.x; q[1] = u.y; q[2] = u.z; q[3] = u.w; q[4] = w.x; q[5] = w.y; q[6] = w.z; q[7] = w.w;
 #pragma unroll
           for (int e = 0; e < 8; ++e) q[e] = in ? q[e] : 0.f;
-        } else if (!SL) {
+        } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e) q[e] = (valid && kk0 + e < k) ? x[row * k + kk0 + e] : 0.f;
-        }
-        if (SL && wide) {
-          // whole chunks: 16-byte loads, which rows of any width and start take (4-byte alignment)
-          const bool in = valid && kk0 + 8 <= kx;             // loads always issued, from row 0 when idle
-          const floatx4_dword* xp4 = reinterpret_cast<const floatx4_dword*>(x + (in ? row * ldx + kk0 : 0));
-          const floatx4_dword u = xp4[0], w = xp4[1];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) { q[e] = in ? u[e] : 0.f; q[4 + e] = in ? w[e] : 0.f; }
-        }
-        if (SL && (!wide || (kx & 7))) {                              // the chunk that a row ends in
-          const bool part = valid && kk0 < kx && kk0 + 8 > kx;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            if (!wide) q[e] = 0.f;
-            if (part && kk0 + e < kx) q[e] = x[row * ldx + kk0 + e];
-          }
         }
         if (use_mu) {
 #pragma unroll
@@ -1037,20 +498,13 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
       xn[b] = sum;
     }
 
-    float best[NB], second[NB];
-    int bv[NB], bct[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) { best[b] = INFINITY; second[b] = INFINITY; bv[b] = 0; bct[b] = 0; }
     for (int ct = 0; ct < n_ct; ++ct) {
       floatx16 bz;
-      const bool biased = !PACKED || !cosine || ct * 32 + 32 > n;   // cosine: only a tile with padding has any
-      if (biased) {
-        const float* bp = bias + ct * 32 + 4 * g;
+      const float* bp = bias + ct * 32 + 4 * g;
 #pragma unroll
-        for (int v4 = 0; v4 < 4; ++v4) {
-          const float4 t4 = *reinterpret_cast<const float4*>(bp + 8 * v4);
-          bz[4 * v4] = t4.x; bz[4 * v4 + 1] = t4.y; bz[4 * v4 + 2] = t4.z; bz[4 * v4 + 3] = t4.w;
-        }
+      for (int v4 = 0; v4 < 4; ++v4) {
+        const float4 t4 = *reinterpret_cast<const float4*>(bp + 8 * v4);
+        bz[4 * v4] = t4.x; bz[4 * v4 + 1] = t4.y; bz[4 * v4 + 2] = t4.z; bz[4 * v4 + 3] = t4.w;
       }
       bf16x8 a[3][S];
 #pragma unroll
@@ -1080,7 +534,7 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
           for (int b = 0; b < NB; ++b)
             acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pc[term]][st], xp[b][st][px[term]], acc[b], 0, 0, 0);
         }
-      if constexpr (PW) {
+      {
         // Distances of this 32-centre tile.  L2: |x|^2 + |c|^2 - 2 x.c (of the centred vectors) loses
         // what the two have in common, so an entry below an eighth of |x|^2 + |c|^2 (three bits gone)
         // is evaluated again as sum((x - c)^2); cosine needs that only near the clamp of |x||c|.
@@ -1180,79 +634,6 @@ __global__ __launch_bounds__(256, SL && S <= 2 ? 3 : 1) void predict_split_kerne
             }
           }
         }
-      } else {
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          if (biased) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[b][v] += bz[v];
-          }
-          if constexpr (PACKED) argmin_update_packed(acc[b], ct * 32, best[b], second[b], bct[b]);
-          else argmin_update(acc[b], ct * 32, best[b], second[b], bv[b], bct[b]);
-        }
-      }
-    }
-    if constexpr (PW) continue;
-    int besti[NB];
-    uint64_t todo[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const bool valid = grp * kGroupRows + 32 * b + j < m;
-      const int slot = PACKED ? __float_as_int(best[b]) & 15 : bv[b];
-      int bi = bct[b] + 8 * (slot >> 2) + 4 * g + (slot & 3);
-      float bs = best[b], sd = second[b];
-      {  // merge the two halves of the wave (same x row, disjoint centres)
-        const float ob = __shfl_xor(bs, 32);
-        const float os = __shfl_xor(sd, 32);
-        const int oi = __shfl_xor(bi, 32);
-        if (ob < bs || (ob == bs && oi < bi)) {
-          sd = fminf(bs, os);
-          bs = ob;
-          bi = oi;
-        } else {
-          sd = fminf(sd, ob);
-        }
-      }
-      // cosine: the evaluation's share shrinks with the operands, the rounding of c / |c| (norm in
-      // fp64, one rounding for 1 / |c|, one for the product, one for - m: 3 units, doubled) does not
-      const float scale = cosine ? sqrtf(xn[b]) * (cdev + 3.5762787e-7f / unit) : xn[b] + cmax;
-      float bound = unit * scale + kTinyGap;
-      bool ask = false;
-      if (PACKED) {      // the slots: 2^-19 of each of the two
-        bound += 1.92e-6f * (fabsf(bs) + fabsf(sd));
-        // padding leads where no real score is a number
-        ask = bi >= n || !(scale < finite_below);
-      }
-      besti[b] = bi;
-      todo[b] = __ballot(valid && g == 0 && (ask || !((sd - bs) > bound)));
-    }
-    // exact re-evaluation of the flagged rows: one copy of the code, whichever tile the row is in
-#pragma nounroll
-    for (int b = 0; b < NB; ++b) {
-      uint64_t td = todo[0];
-#pragma unroll
-      for (int q = 1; q < NB; ++q) td = b == q ? todo[q] : td;
-      while (td) {
-        const int src = __ffsll((unsigned long long)td) - 1;
-        td &= td - 1;
-        const float* xr = x + (grp * kGroupRows + 32 * b + (src & 31)) * ldx;
-        int exact;
-        if (!cosine) {
-          exact = exact_argmin_row_l2_pieces<S>(xr, xs, ap, n, n_ct, k, kx, lane, mu, cmax, centers);
-          if (exact < 0) exact = exact_argmin_row(xr, centers, n, k, kx, metric, lane);   // the original row decides
-        }
-        else if (plain_cosine) exact = exact_argmin_row(xr, centers, n, k, kx, metric, lane);
-        else exact = exact_argmin_row_cosine_pieces<S>(xr, xs, ap, centers, n, n_ct, k, kx, lane, cdev);
-#pragma unroll
-        for (int q = 0; q < NB; ++q) besti[q] = (b == q && lane == src) ? exact : besti[q];
-      }
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int64_t row = grp * kGroupRows + 32 * b + j;
-      if (row < m && g == 0) {
-        if (lab64) lab64[row * ldl] = besti[b];
-        if (lab8) lab8[row * ldl] = (uint8_t)besti[b];
       }
     }
   }
@@ -1531,15 +912,14 @@ int launch_mfma(const float* x, const float* centers, int64_t* l64, uint8_t* l8,
   return launch_status("kmeans_predict");
 }
 
-template <int S, int NB, bool PW = false, bool SL = false, bool PACKED = false>
-int launch_split(const float* x, const float* centers, int64_t* l64, uint8_t* l8, int64_t m, int n, int k,
-                 int metric, int n_pad, size_t lds, hipStream_t st, float* dist = nullptr, int64_t ldd = 0,
-                 const SliceArgs* slices = nullptr) {
-  auto kern = predict_split_kernel<S, NB, PW, SL, PACKED>;
+template <int S, int NB>
+int launch_pairwise_split(const float* x, const float* centers, int64_t m, int n, int k, int metric, int n_pad, size_t lds,
+                          hipStream_t st, float* dist, int64_t ldd) {
+  auto kern = pairwise_split_kernel<S, NB>;
   if (lds > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return fail((int)e, "kmeans_predict: cannot reserve %zu B of LDS", lds);
+    if (e != hipSuccess) return fail((int)e, "pairwise_distance: cannot reserve %zu B of LDS", lds);
   }
   // resident grid, as for the fp32 kernel
   static thread_local size_t cached_lds = 0;
@@ -1554,47 +934,8 @@ int launch_split(const float* x, const float* centers, int64_t* l64, uint8_t* l8
   }
   const int64_t need = ceil_div(ceil_div(m, 32 * NB), 4);
   const int64_t cap = (int64_t)num_cus() * cached_per_cu;
-  int64_t grid = need < cap ? need : cap;
-  SliceArgs sl{1, k, k, 1};
-  if constexpr (SL) {
-    sl = *slices;
-    if (sl.slices > 1) {
-      // the resident grid shared out over the slices, eight shares at least (one per XCD)
-      int64_t per = cap / sl.slices / 8 * 8;
-      const int64_t most = ceil_div(need, 8) * 8;
-      per = per < 8 ? 8 : per;
-      grid = (per < most ? per : most) * sl.slices;
-    }
-  }
-  kern<<<(int)grid, 256, lds, st>>>(x, centers, l64, l8, m, n, k, metric, n_pad, dist, ldd, sl);
-  return launch_status(PW ? "pairwise_distance" : "kmeans_predict");
-}
-
-// split-bf16 path: up to 64 dimensions, operand pieces and biases within 96 KB of LDS
-size_t split_lds(int64_t n, int64_t k) {
-  const int64_t steps = ceil_div(k, 16), n_pad32 = ceil_div(n, 32) * 32;
-  return (size_t)(3 * (n_pad32 / 32) * steps * 64 * 16 + 2 * n_pad32 * 4 + 16 + 5 * 16 * steps * 4);
-}
-
-bool split_fits(int64_t n, int64_t k) { return k <= 64 && n <= 65536 && split_lds(n, k) <= 96 * 1024; }
-
-template <bool SL>
-int predict_split(const float* x, const float* centers, int64_t* l64, uint8_t* l8, int64_t m, int n, int k, int metric,
-                  hipStream_t st, const SliceArgs* sl = nullptr) {
-  const int n_pad = (int)ceil_div(n, 32) * 32;
-  const size_t lds = split_lds(n, k);
-  // Packed scores: from 4 to 16 dimensions, where the update is as long as the products (1e6 x 16 against 256 centres,
-  // cosine: 78 -> 68 us; L2: 78 -> 74).  In fewer dimensions so many centres are close to a row that the wider near-tie
-  // bound sends more rows to the exact evaluation than the update saves (1e6 x 2, 256 centres, cosine: 461 -> 543 us);
-  // in more, the tree's registers cost what its instructions save (32 dimensions: 118 us either way; 64: 138 -> 179).
-  switch (ceil_div(k, 16)) {
-    case 1:
-      if (k < 4) return launch_split<1, 2, false, SL, false>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
-      return launch_split<1, 2, false, SL, true>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
-    case 2: return launch_split<2, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
-    case 3: return launch_split<3, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
-    default: return launch_split<4, 2, false, SL>(x, centers, l64, l8, m, n, k, metric, n_pad, lds, st, nullptr, 0, sl);
-  }
+  kern<<<(int)(need < cap ? need : cap), 256, lds, st>>>(x, centers, m, n, k, metric, n_pad, dist, ldd);
+  return launch_status("pairwise_distance");
 }
 
 }  // namespace
@@ -1627,10 +968,10 @@ extern "C" int f2cgt_pairwise_distance(const float* x, const float* y, float* di
         hipStream_t st = as_stream(stream);
         int rc;
         switch (steps) {
-          case 1: rc = launch_split<1, 2, true>(x, yc, nullptr, nullptr, m, nn, (int)k, metric, n_pad32, lds, st, dc, n); break;
-          case 2: rc = launch_split<2, 2, true>(x, yc, nullptr, nullptr, m, nn, (int)k, metric, n_pad32, lds, st, dc, n); break;
-          case 3: rc = launch_split<3, 2, true>(x, yc, nullptr, nullptr, m, nn, (int)k, metric, n_pad32, lds, st, dc, n); break;
-          default: rc = launch_split<4, 2, true>(x, yc, nullptr, nullptr, m, nn, (int)k, metric, n_pad32, lds, st, dc, n); break;
+          case 1: rc = launch_pairwise_split<1, 2>(x, yc, m, nn, (int)k, metric, n_pad32, lds, st, dc, n); break;
+          case 2: rc = launch_pairwise_split<2, 2>(x, yc, m, nn, (int)k, metric, n_pad32, lds, st, dc, n); break;
+          case 3: rc = launch_pairwise_split<3, 2>(x, yc, m, nn, (int)k, metric, n_pad32, lds, st, dc, n); break;
+          default: rc = launch_pairwise_split<4, 2>(x, yc, m, nn, (int)k, metric, n_pad32, lds, st, dc, n); break;
         }
         if (rc != 0) return rc;
       }
@@ -1658,7 +999,7 @@ extern "C" int f2cgt_kmeans_predict(const float* x, const float* centers, int64_
   F2CGT_REQUIRE(x && centers && (labels_i64 || labels_u8), F2CGT_E_INVALID,
                 "kmeans_predict: null buffer");
   hipStream_t st = as_stream(stream);
-  if (split_fits(n, k)) return predict_split<false>(x, centers, labels_i64, labels_u8, m, (int)n, (int)k, metric, st);
+  if (assign_fits(n, k)) return assign_rows(x, centers, labels_i64, labels_u8, m, (int)n, (int)k, metric, st);
   const int khalf = (int)((k + 1) / 2);
   int kh = pow2_ceil(khalf);
   if (kh < 4) kh = 4;
@@ -1684,27 +1025,4 @@ extern "C" int f2cgt_kmeans_predict(const float* x, const float* centers, int64_
   predict_exact_kernel<<<(int)(need < cap ? need : cap), 256, 0, st>>>(x, centers, labels_i64, labels_u8, m,
                                                                       (int)n, (int)k, metric);
   return launch_status("kmeans_predict");
-}
-
-extern "C" int f2cgt_vq_encode_slices_covers(int64_t n, int64_t k) {
-  return n > 0 && n <= 256 && k > 0 && split_fits(n, k) ? 1 : 0;
-}
-
-extern "C" int f2cgt_vq_encode_slices(const float* x, int64_t ldx, int64_t feat_dim, const float* codebooks, uint8_t* codes,
-                                      int64_t code_stride, int64_t m, int64_t slices, int64_t n, int64_t k, int metric,
-                                      void* stream) {
-  const char* what = "vq_encode_slices";
-  F2CGT_REQUIRE(m >= 0 && slices > 0 && n > 0 && k > 0 && feat_dim > 0, F2CGT_E_INVALID, "%s: sizes must be positive", what);
-  F2CGT_REQUIRE(f2cgt_vq_encode_slices_covers(n, k), F2CGT_E_UNSUPPORTED,
-                "%s: %lld centres of %lld columns are left to kmeans_predict, one slice at a time", what, (long long)n,
-                (long long)k);
-  F2CGT_REQUIRE(slices <= 65536 && feat_dim < (1 << 22), F2CGT_E_UNSUPPORTED, "%s: table too wide", what);
-  F2CGT_REQUIRE((slices - 1) * k < feat_dim, F2CGT_E_INVALID, "%s: a slice without columns", what);
-  F2CGT_REQUIRE(ldx >= feat_dim && code_stride >= slices, F2CGT_E_INVALID, "%s: rows overlap", what);
-  F2CGT_REQUIRE(metric == F2CGT_METRIC_L2 || metric == F2CGT_METRIC_COSINE, F2CGT_E_INVALID, "%s: unknown metric %d", what,
-                metric);
-  if (m == 0) return 0;
-  F2CGT_REQUIRE(x && codebooks && codes, F2CGT_E_INVALID, "%s: null buffer", what);
-  const SliceArgs sl{(int)slices, (int)feat_dim, ldx, code_stride};
-  return predict_split<true>(x, codebooks, nullptr, codes, m, (int)n, (int)k, metric, as_stream(stream), &sl);
 }

@@ -23,7 +23,7 @@ with 300 steps for c4 and c5 (30 and 100 warm-up launches); T = B except for c2,
                     TCP_TA_TCP_STATE_READ_sum ... -- B
     fetch_copy / write_copy   the FETCH_SIZE / WRITE_SIZE runs of `python3 bench.py --calibrate-copy`
     trace_all   rocprofv3 --kernel-trace --stats ... -- python3 bench.py --all --steps 200 --warmup 20 --cpu-seconds 0
-    mfma_all    rocprofv3 --pmc SQ_INSTS_VALU_MFMA_MOPS_BF16 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES
+    mfma_all    rocprofv3 --pmc SQ_INSTS_VALU_MFMA_MOPS_F16 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES
                     SQ_INSTS_MFMA SQ_INSTS_VALU GRBM_GUI_ACTIVE ... -- (the --all command)
 
 Missing directories are skipped.  Counter values are means per dispatch of the named kernel.
@@ -217,22 +217,22 @@ def main(argv):
             fh.write("\n")
     A = "python3 bench.py --all --steps 200 --warmup 20 --cpu-seconds 0"
     tall = os.path.join(O, "trace_all")
-    k = kstats(tall, "predict_split_kernel<2, 2, false>")
+    k = kstats(tall, "assign_kernel<2, 4, true>")
     if k:
-        with open(os.path.join(P, "predict_split_kernel_c5_encode.md"), "w") as fh:
-            fh.write("# predict_split_kernel<2, 2, false> on the C5 encode step (1e6 x 32 fp32 vs 256 centres, squared L2 + arg-min)\n\n")
+        with open(os.path.join(P, "assign_kernel_c5_encode.md"), "w") as fh:
+            fh.write("# assign_kernel<2, 4, true> on the C5 encode step (1e6 x 32 fp32 vs 256 centres, squared L2 + arg-min)\n\n")
             fh.write("Commands (separate runs):\n\n")
             fh.write("    rocprofv3 --kernel-trace --stats --output-format csv -d out/trace_all -o t -- %s\n" % A)
-            fh.write("    rocprofv3 --pmc SQ_INSTS_VALU_MFMA_MOPS_BF16 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_INSTS_MFMA "
+            fh.write("    rocprofv3 --pmc SQ_INSTS_VALU_MFMA_MOPS_F16 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_INSTS_MFMA "
                      "SQ_INSTS_VALU GRBM_GUI_ACTIVE --output-format csv -d out/mfma_all -o t -- %s\n\n" % A)
             fh.write("| kernel | calls | avg us | min us | max us |\n|---|---|---|---|---|\n")
             fh.write("| `%s` | %d | %.2f | %.2f | %.2f |\n\n" % (k[0][:60], k[1], k[2], k[3], k[4]))
             fl = 2.0 * 1e6 * 256 * 32
-            fh.write("2*m*n*k = %.4g flop per launch -> %.1f TFLOP/s algorithmic; the kernel executes six bf16 MFMAs per fp32 "
-                     "product block (three bf16 pieces per value), i.e. %.0f TFLOP/s of bf16 MFMA = %.3f of the 2500 TFLOP/s "
-                     "bf16 peak.\n\n" % (fl, fl / (k[2] * 1e-6) / 1e12, 6 * fl / (k[2] * 1e-6) / 1e12,
-                                         6 * fl / (k[2] * 1e-6) / 1e12 / 2500))
-            vals = counters(os.path.join(O, "mfma_all"), "predict_split_kernel<2, 2, false>")
+            fh.write("2*m*n*k = %.4g flop per launch -> %.1f TFLOP/s algorithmic; the kernel executes three fp16 MFMAs per fp32 "
+                     "product block (two fp16 pieces per value), i.e. %.0f TFLOP/s of fp16 MFMA = %.3f of the 2500 TFLOP/s "
+                     "peak.\n\n" % (fl, fl / (k[2] * 1e-6) / 1e12, 3 * fl / (k[2] * 1e-6) / 1e12,
+                                         3 * fl / (k[2] * 1e-6) / 1e12 / 2500))
+            vals = counters(os.path.join(O, "mfma_all"), "assign_kernel<2, 4, true>")
             if vals:
                 fh.write("| counter (mean per dispatch) | value |\n|---|---|\n")
                 for cn in sorted(vals):
@@ -241,10 +241,10 @@ def main(argv):
                     util = vals["SQ_VALU_MFMA_BUSY_CYCLES"][0] / N_SIMD / (vals["GRBM_GUI_ACTIVE"][0] / N_XCD)
                     fh.write("\nMFMA utilisation = SQ_VALU_MFMA_BUSY_CYCLES / %d SIMDs / (GRBM_GUI_ACTIVE / %d XCDs) = %.3f\n"
                              % (N_SIMD, N_XCD, util))
-        k = kstats(tall, "predict_split_kernel<2, 2, true>")
+        k = kstats(tall, "pairwise_split_kernel<2, 2>")
         if k:
-            with open(os.path.join(P, "predict_split_kernel_pairwise_c5_encode_shape.md"), "w") as fh:
-                fh.write("# predict_split_kernel<2, 2, true> (pairwise_distance) at the C5 encode shape: 1e6 x 32 against 256 rows, L2 and cosine\n\n")
+            with open(os.path.join(P, "pairwise_split_kernel_c5_encode_shape.md"), "w") as fh:
+                fh.write("# pairwise_split_kernel<2, 2> (pairwise_distance) at the C5 encode shape: 1e6 x 32 against 256 rows, L2 and cosine\n\n")
                 fh.write("    rocprofv3 --kernel-trace --stats --output-format csv -d out/trace_all -o t -- %s\n\n" % A)
                 fh.write("| kernel | calls | avg us | min us | max us |\n|---|---|---|---|---|\n")
                 fh.write("| `%s` | %d | %.2f | %.2f | %.2f |\n\n" % (k[0][:60], k[1], k[2], k[3], k[4]))

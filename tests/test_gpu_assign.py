@@ -1,0 +1,86 @@
+"""Nearest-centre labels on the matrix cores (assign_kernel) against float64 distances of the original values: the labels
+are the true first minimum, so they have to be equal wherever the two smallest float64 distances differ by more than
+float64 rounding."""
+import numpy as np
+import pytest
+import torch
+
+from f2cgt_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def labels64(x, c, metric):
+    x, c = x.astype(np.float64), c.astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        if metric == "cosine":
+            den = np.linalg.norm(x, axis=1)[:, None] * np.linalg.norm(c, axis=1)[None]
+            d = 1.0 - (x @ c.T) / np.maximum(den, 1e-8)
+        else:
+            d = ((x[:, None] - c[None]) ** 2).sum(-1)
+    d = np.where(np.isfinite(d), d, np.inf)
+    two = np.partition(d, 1, axis=1)[:, :2] if c.shape[0] > 1 else np.stack([d[:, 0], d[:, 0] + 1], 1)
+    two = np.minimum(two, np.finfo(np.float64).max)
+    near = two[:, 1] - two[:, 0] <= 1e-12 * (1.0 + np.abs(two[:, 0]))        # float64 sums in another order
+    return d.argmin(1), near
+
+
+def check(x, c, metric):
+    want, near = labels64(x, c, metric)
+    got = capi.kmeans_predict(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), metric).cpu().numpy()
+    assert np.array_equal(got[~near], want[~near])
+    assert ((got >= 0) & (got < c.shape[0])).all()
+    return near
+
+
+# n: one tile, one centre, full and ragged last tiles, chunks of an odd number of tiles, several chunks;
+# k: operand steps from 1 to 4 and both sides of each, rows that end in every mix of fours, twos and ones;
+# m: a group of 32 rows, one less, one more, more groups than a workgroup has waves
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 1), (31, 2, 3), (32, 31, 4), (33, 32, 7), (400, 33, 8), (500, 64, 9), (1000, 65, 15), (2000, 96, 16), (700, 97, 17),
+    (300, 128, 22), (300, 129, 31), (3000, 160, 32), (500, 161, 33), (500, 256, 47), (500, 200, 48), (500, 65, 49), (500, 63, 61),
+    (9000, 256, 64), (700, 1000, 16), (300, 1, 40), (600, 30, 5)])
+def test_labels_are_the_first_minimum(metric, m, n, k):
+    print("case assign", metric, m, n, k, flush=True)
+    rng = np.random.default_rng(m * 7 + n * 3 + k)
+    check(rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32), metric)
+
+
+# rows and centres of very different lengths, down to where products vanish and up to where squares overflow, and data
+# far from the origin: the scales of the pieces, the mean and the exact evaluation
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("spread,centre_scale,shift", [(8, 1.0, 0.0), (0, 1e-12, 0.0), (0, 1e15, 0.0), (3, 1.0, 50.0), (18, 1e18, 0.0)])
+@pytest.mark.parametrize("k", [16, 30])
+def test_labels_over_scales(metric, spread, centre_scale, shift, k):
+    print("case assign scales", metric, spread, centre_scale, shift, k, flush=True)
+    rng = np.random.default_rng(k + spread)
+    x = rng.standard_normal((600, k)) * 10.0 ** rng.uniform(-spread, spread, (600, 1)) + shift
+    c = (rng.standard_normal((140, k)) + shift) * centre_scale
+    x, c = x.astype(np.float32), c.astype(np.float32)
+    if metric == "cosine":        # the clamp of |x||c| at 1e-8 makes float64 ties of its own
+        x = x[np.linalg.norm(x.astype(np.float64), axis=1) * np.linalg.norm(c.astype(np.float64), axis=1).min() > 1e-7]
+    if len(x):
+        check(x, c, metric)
+
+
+# a centre that is no number is never the nearest, wherever its tile and slot, and takes no other one of its class along
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("n,bad", [(256, (0, 37, 255)), (40, (33,)), (20, (3,))])
+def test_centres_that_are_no_numbers(metric, value, n, bad):
+    print("case assign bad centres", metric, value, n, flush=True)
+    rng = np.random.default_rng(n)
+    x, c = rng.standard_normal((500, 16)).astype(np.float32), rng.standard_normal((n, 16)).astype(np.float32)
+    for b in bad:
+        c[b, b % 16] = value
+    check(x, c, metric)
+
+
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+def test_rows_that_are_no_numbers(metric):
+    rng = np.random.default_rng(3)
+    x, c = rng.standard_normal((200, 24)).astype(np.float32), rng.standard_normal((100, 24)).astype(np.float32)
+    x[5, 3], x[64, 0], x[199, 23] = np.nan, np.inf, -np.inf
+    near = check(x, c, metric)
+    assert near.sum() <= 3 + 1
