@@ -44,6 +44,11 @@ SIGNATURES = {
     "f2cgt_kmeans_predict": ([P, P, P, P, L, L, L, I, P], c_int),
     "f2cgt_vq_encode_slices_covers": ([L, L], c_int),
     "f2cgt_vq_encode_slices": ([P, L, L, P, P, L, L, L, L, L, I, P], c_int),
+    "f2cgt_slice_rows": ([P, L, P, L, L, L, L, P, P, P, P], c_int),
+    "f2cgt_keep_rows": ([P, P, ctypes.c_float, ctypes.c_float, L, L, P, P], c_int),
+    "f2cgt_kmeans_slices_covers": ([L, L, L], c_int),
+    "f2cgt_kmeans_slices_workspace_bytes": ([L, L, L, L], c_int64),
+    "f2cgt_kmeans_slices_step": ([P, P, P, P, I, ctypes.c_float, P, L, L, L, L, L, I, P], c_int),
     "f2cgt_kmeans_update_workspace_bytes": ([L, L], c_int64),
     "f2cgt_kmeans_update": ([P, P, P, P, P, P, I, ctypes.c_float, P, L, L, L, L, P], c_int),
     "f2cgt_kmeans_update_static": ([P, P, P, P, P, P, I, ctypes.c_float, L, L, L, P], c_int),

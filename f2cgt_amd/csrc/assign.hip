@@ -1,5 +1,6 @@
-// Nearest-centre labels on the matrix cores: kmeans_predict up to 64 dimensions, and the codes of all column slices
-// of a table in one launch (vq_encode_slices).
+// Nearest-centre labels on the matrix cores: kmeans_predict up to 64 dimensions, the codes of all column slices
+// of a table in one launch (vq_encode_slices), and the training step of all slices of a sample (kmeans_slices_step,
+// which adds the rows up by label instead of writing the labels).
 //
 // The distances are never written.  For L2 the kernel works on x - mu and c - mu (mu = mean of the centres) where that
 // matters: a common offset of the data then costs nothing.  For cosine the normalised centres lose their mean direction
@@ -59,7 +60,13 @@ struct AssignArgs {
   // label_stride apart); the grid is a multiple of 8 * slices workgroups then
   int slices;
   int feat_dim;            // columns of the table; the last slice may have fewer than k
-  int64_t ldx, label_stride;
+  int64_t ldx, label_stride, slice_step;   // slice_step: from a row of a slice to the same row of the next, in floats
+  // training step: the rows' sums and counts by label instead of the labels
+  const int32_t* stop;     // [slices]: nonzero = the slice's centres are final
+  const uint32_t* keep;    // [slices][keep_words]: bit r % 32 of word r / 32 = row r takes part; null: all do
+  int64_t keep_words;
+  float* sums;             // [slices][shares][n * k + n]
+  uint32_t* arrived;       // [slices]: cleared for the merging kernel
 };
 
 // Minima and maxima that keep a NaN (v_minimum3, v_maximum3): no instruction to quieten the operands first, and a row with
@@ -248,8 +255,9 @@ __device__ __forceinline__ int exact_row(const AssignArgs& a, const float* __res
   return first_minimum(bestv, besti);
 }
 
-// S: steps of 16 dimensions.  T: tiles of a chunk (a class has T centres).  PACKED: update_packed.
-template <int S, int T, bool PACKED>
+// S: steps of 16 dimensions.  T: tiles of a chunk (a class has T centres).  PACKED: update_packed.  SUMS: the training
+// step, which adds the rows up by label in LDS (n * (16 S + 1) doubles) and leaves a set of sums per workgroup.
+template <int S, int T, bool PACKED, bool SUMS>
 __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kernel(AssignArgs a) {
   constexpr int kThreads = assign_threads(S), kWaves = kThreads / kWave;
   constexpr int U = T == 1 ? 1 : 2;                              // tiles a step
@@ -264,26 +272,38 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
   if (a.slices > 1) {
     // Workgroups go round-robin to the 8 XCDs: with 8 shares side by side, the slices of a share run on one
     // XCD, whose L2 then serves the lines of x that two slices have in common and joins their code bytes.
-    const int turn = blockIdx.x / (8 * a.slices), at = blockIdx.x % (8 * a.slices);
-    slice = at >> 3;
-    share = turn * 8 + (at & 7);
     shares = gridDim.x / a.slices;
-    x += slice * k;
+    if (shares & 7) {
+      slice = blockIdx.x % a.slices;
+      share = blockIdx.x / a.slices;
+    } else {
+      const int turn = blockIdx.x / (8 * a.slices), at = blockIdx.x % (8 * a.slices);
+      slice = at >> 3;
+      share = turn * 8 + (at & 7);
+    }
+    x += slice * a.slice_step;
     centers += (int64_t)slice * n * k;
     lab8 += slice;
   }
+  if (SUMS && a.stop[slice] != 0) return;
   int kx = a.feat_dim - slice * k;                               // dimensions the rows have (zeros after them)
   kx = kx < k ? kx : k;
   const int64_t ldx = a.ldx, ldl = a.label_stride;
   const int n_ct = (n + 31) >> 5;                                // 32-centre tiles
   const int piece = (n_pad >> 5) * S * 64;                             // operands per piece
   half8* ap = reinterpret_cast<half8*>(smem_raw);                // [2][n_pad / 32][S][64]
-  float* bias = reinterpret_cast<float*>(smem_raw + (size_t)2 * piece * 16);   // [n_pad]
+  double* norm2 = reinterpret_cast<double*>(smem_raw + (size_t)2 * piece * 16);   // [n_pad] |c|^2
+  float* bias = reinterpret_cast<float*>(norm2 + n_pad);         // [n_pad]
   float* inv = bias + n_pad;                                     // [n_pad] 1 / |c| (cosine) or 1; 0: no number
   int* flags = reinterpret_cast<int*>(inv + n_pad);              // max |c|^2, degenerate centre, draws, mean in use
   float* mu = reinterpret_cast<float*>(flags + 4);               // [16 S]
   float* psum = mu + 16 * S;                                     // [2][kThreads]
   float* xs = psum + 2 * kThreads + (threadIdx.x >> 6) * 32 * S;   // one row of x per wave, centred and as it is
+  constexpr int kPitch = 16 * S + 1;                             // (odd: the centres' sums start in different banks)
+  // SUMS: [n][kPitch] sums, then [n] counts.  In fp64: the LDS adds a float in 178 clocks per wave and CU, a double in 19
+  // (measured, addresses as here; 32-bit integers 6): a step of six slices of 150 000 x 16 rows took 110 us, now 54.
+  double* sums = reinterpret_cast<double*>(psum + 2 * kThreads + kWaves * 32 * S);
+  uint32_t* counts = reinterpret_cast<uint32_t*>(sums + n * kPitch);
   const bool cosine = a.metric == F2CGT_METRIC_COSINE;
   const int lane = threadIdx.x & 63;
   const int j = lane & 31;
@@ -294,7 +314,7 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
   const int64_t per_wg = (n_groups + shares - 1) / shares;
   const int64_t wg_lo = share * per_wg;
   const int64_t wg_hi = wg_lo + per_wg < n_groups ? wg_lo + per_wg : n_groups;
-  if (wg_lo >= wg_hi) return;                                    // the whole workgroup
+  if (!SUMS && wg_lo >= wg_hi) return;                           // the whole workgroup
 
   // Staging.  The centres are read once, into the places where their pieces go: item (centre c, chunk ch of 8 dimensions)
   // is operand lane (c % 32) + 32 (ch % 2) of step ch / 2 of tile c / 32, and its first four values lie where its leading
@@ -375,7 +395,13 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     }
   };
   int64_t grp = wg_lo + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  load_rows(grp < wg_hi ? grp : wg_lo);
+  load_rows(grp < wg_hi ? grp : wg_lo < n_groups ? wg_lo : 0);
+  if constexpr (SUMS) {
+    for (int i = threadIdx.x; i < n * kPitch; i += kThreads) sums[i] = 0.0;
+    for (int i = threadIdx.x; i < n; i += kThreads) counts[i] = 0u;
+    if (share == 0 && threadIdx.x == 0) a.arrived[slice] = 0u;
+  }
+  for (int c = threadIdx.x; c < n_pad; c += kThreads) norm2[c] = 0.0;
   if (threadIdx.x < 4) flags[threadIdx.x] = threadIdx.x == 2 ? kWaves : 0;
   // Column sums of raw * weight (and of the squares), a thread per column and row class; then the mean by the first wave.
   auto column_mean = [&](bool weighted) {
@@ -395,12 +421,19 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     __syncthreads();
     if (threadIdx.x < 64) {                                      // the first wave, all of it
       float mt = 0.f, st = 0.f;
-      if (lane < kWidth)
-#pragma unroll 4
-        for (int q = 0; q < kParts; ++q) {
-          mt += psum[q * kWidth + lane];
-          st += psum[kThreads + q * kWidth + lane];
+      constexpr int kSide = 64 / kWidth;                         // lanes to a column
+      if (lane < kSide * kWidth)
+#pragma unroll
+        for (int q = 0; q < (kParts + kSide - 1) / kSide; ++q) {
+          const int from = (q * kSide + lane / kWidth) * kWidth + lane % kWidth;
+          if (from < kParts * kWidth) {
+            mt += psum[from];
+            st += psum[kThreads + from];
+          }
         }
+      if constexpr (kSide >= 2) { mt += __shfl_xor(mt, 32); st += __shfl_xor(st, 32); }
+      if constexpr (kSide == 4) { mt += __shfl_xor(mt, 16); st += __shfl_xor(st, 16); }
+      if (lane >= kWidth) mt = st = 0.f;
       mt /= (float)n;
       st /= (float)n;
       float m2 = mt * mt, var = st - mt * mt;                    // dimensions from k on hold zeros
@@ -421,21 +454,24 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
   // matters, |mu|^2 above twice the summed variance of the centres (otherwise mu is zero and the
   // subtraction of the hot loop is skipped).
   if (!cosine) column_mean(false);
-  // Norms, a thread per centre.
+  // Norms, in fp64 (1 / |c| must be good to a rounding or two): a thread per chunk, then a thread per centre.
+#pragma nounroll
+  for (int at = threadIdx.x; at < piece; at += kThreads) {
+    const int c = at / (64 * S) * 32 + (at & 31), d0 = (at / 64 % S) * 16 + (at & 32) / 4;
+    const float4 p = lo4[at], w = hi4[at];
+    float v[8] = {p.x, p.y, p.z, p.w, w.x, w.y, w.z, w.w};
+    double sq = 0.0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if (!cosine) v[e] -= mu[d0 + e];
+      sq += (double)v[e] * (double)v[e];
+    }
+    unsafeAtomicAdd(norm2 + c, sq);
+  }
+  __syncthreads();
   float top = 0.f;
   for (int c = threadIdx.x; c < n_pad; c += kThreads) {
-    double cn64 = 0.0;                       // fp64: 1 / |c| must be good to a rounding or two
-#pragma unroll 2
-    for (int t = 0; t < kWidth; t += 4) {
-      const int at = ((c >> 5) * S + (t >> 4)) * 64 + ((t >> 3) & 1) * 32 + (c & 31);
-      const float4 r4 = (t & 4) ? hi4[at] : lo4[at];
-      float v[4] = {r4.x, r4.y, r4.z, r4.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (!cosine) v[e] -= mu[t + e];
-        cn64 += (double)v[e] * (double)v[e];
-      }
-    }
+    const double cn64 = norm2[c];
     const float cn = (float)cn64;
     float sc = 1.f;
     if (cosine) sc = (float)(1.0 / sqrt(cn64 > 1e-60 ? cn64 : 1e-60));
@@ -492,7 +528,7 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     ap[at] = p0;
     ap[piece + at] = p1;
   }
-  if (cosine) {                                                  // one LDS atomic per wave
+  if (cosine && flags[3] == 1) {                                 // one LDS atomic per wave
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) dev2max = fmaxf(dev2max, __shfl_xor(dev2max, off));
     if (lane == 0) atomicMax(flags, __float_as_int(dev2max));
@@ -534,6 +570,13 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     int drawn = 0;
     if (lane == 0) drawn = atomicAdd(flags + 2, 1);
     half8 xp[S][2];
+    float own[SUMS ? S : 1][8];
+    if constexpr (SUMS) {
+#pragma unroll
+      for (int st = 0; st < S; ++st)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) own[st][e] = q[st][e];
+    }
     if (ragged) {
 #pragma unroll
       for (int st = 0; st < S; ++st)
@@ -569,7 +612,7 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
       }
     // The next rows travel while these are scored, behind the last ones' labels: the wait for the rows is one for every
     // access before them too, and a store that has just been issued takes as long as the rows.
-    if (labelled >= 0) store_labels();
+    if (!SUMS && labelled >= 0) store_labels();
     const int64_t next = wg_lo + __builtin_amdgcn_readfirstlane(drawn);
     load_rows(next < wg_hi ? next : grp);
     asm volatile("" ::: "memory");
@@ -694,16 +737,65 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
                                              : exact_row<S>(a, xr, centers, xs, ap, inv, kx, lane, mu, pow2(-c_shift), cmax, cdev);
       besti = lane == src ? exact : besti;
     }
+    if constexpr (SUMS) {
+      const int to = (int)halves((uint32_t)besti).lo;            // the exact evaluation's label is in the lower half
+      const bool in = grp * 32 + j < m && (a.keep == nullptr || (a.keep[slice * a.keep_words + grp] >> j & 1u));
+      if (in) {
+#pragma unroll
+        for (int st = 0; st < S; ++st)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int d = 16 * st + 8 * g + e;
+            if (d < kx) unsafeAtomicAdd(sums + to * kPitch + d, (double)own[st][e]);
+          }
+        if (g == 0) atomicAdd(counts + to, 1u);
+      }
+    }
     label = besti;
     labelled = grp;
     grp = next;
   }
-  if (labelled >= 0) store_labels();
+  if constexpr (SUMS) {
+    __syncthreads();
+    const int words = n * k + n;
+    float* part = a.sums + ((int64_t)slice * shares + share) * words;
+    for (int i = threadIdx.x; i < n * k; i += kThreads) part[i] = (float)sums[i / k * kPitch + i % k];
+    for (int i = threadIdx.x; i < n; i += kThreads) reinterpret_cast<uint32_t*>(part)[n * k + i] = counts[i];
+  } else {
+    if (labelled >= 0) store_labels();
+  }
 }
 
-template <int S, int T, bool PACKED>
+// Two pieces, norms, biases, 1 / |c|, flags, the mean, column sums and a row per wave.
+// Tiles of a chunk: longer ones halve the updates and double the centres of the class that is evaluated again, whose cost
+// goes with the dimensions; up to 64 centres there are only one or two tiles.
+int assign_chunk(int64_t n, int64_t k) { return n <= 32 ? 1 : n <= 64 || k > 32 ? 2 : 4; }
+int64_t assign_pad(int64_t n, int64_t k) { return ceil_div(n, 32 * assign_chunk(n, k)) * 32 * assign_chunk(n, k); }
+size_t assign_lds(int64_t n, int64_t k) {
+  const int64_t steps = ceil_div(k, 16), n_pad = assign_pad(n, k);
+  const int64_t pieces = 2 * (n_pad / 32) * steps * 64 * 16, threads = assign_threads((int)steps);
+  return (size_t)(pieces + 4 * n_pad * 4 + 16 + (1 + 2 * threads / kWave) * 16 * steps * 4 + 2 * threads * 4);
+}
+
+// Workgroups per slice: what takes the `resident` ones the fewest turns, with the staging of a workgroup about as long as
+// two groups of rows of each of its waves.  A multiple of eight, which keeps the slices of a row on one XCD, is taken while
+// it costs no more than a tenth (18 slices of 8 columns, 92 000 rows: 86 us with eight workgroups each, 144 in all, 61
+// with fourteen).
+int64_t assign_shares(int64_t m, int64_t slices, int64_t resident, int waves) {
+  const int64_t groups = ceil_div(m, 32), most = groups < 4 * resident ? groups : 4 * resident;
+  int64_t best = 1, best8 = 0, least = 0, least8 = 0;
+  for (int64_t s = 1; s <= most && (s == 1 || s * slices <= 4 * resident); ++s) {
+    const int64_t cost = ceil_div(s * slices, resident) * (2 + ceil_div(groups, s * waves));
+    if (s == 1 || cost < least) { least = cost; best = s; }
+    if (s % 8 == 0 && (best8 == 0 || cost < least8)) { least8 = cost; best8 = s; }
+  }
+  return best8 != 0 && 10 * least8 <= 11 * least ? best8 : best;
+}
+size_t assign_sums_lds(int64_t n, int64_t k) { return assign_lds(n, k) + (size_t)(n * (16 * ceil_div(k, 16) + 1) * 8 + n * 4); }
+
+template <int S, int T, bool PACKED, bool SUMS>
 int launch_assign(AssignArgs a, size_t lds, hipStream_t st) {
-  auto kern = assign_kernel<S, T, PACKED>;
+  auto kern = assign_kernel<S, T, PACKED, SUMS>;
   constexpr int threads = assign_threads(S);
   if (lds > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -725,47 +817,41 @@ int launch_assign(AssignArgs a, size_t lds, hipStream_t st) {
   const int64_t need = ceil_div(a.m, 32);             // a group per workgroup at least
   const int64_t cap = (int64_t)num_cus() * cached_per_cu;
   int64_t grid = need < cap ? need : cap;
-  if (a.slices > 1) {
-    // the resident grid shared out over the slices, eight shares at least (one per XCD)
-    int64_t per = cap / a.slices / 8 * 8;
-    const int64_t most = ceil_div(need, 8) * 8;
-    per = per < 8 ? 8 : per;
-    grid = (per < most ? per : most) * a.slices;
-  }
+  if (SUMS || a.slices > 1) grid = assign_shares(a.m, a.slices, SUMS ? num_cus() : cap, threads / kWave) * a.slices;
   kern<<<(int)grid, threads, lds, st>>>(a);
   return launch_status("kmeans_predict");
 }
 
-// Two pieces, biases, 1 / |c|, flags, the mean, column sums and a row per wave.
-// Tiles of a chunk: longer ones halve the updates and double the centres of the class that is evaluated again, whose cost
-// goes with the dimensions; up to 32 centres there is only one tile.
-int assign_chunk(int64_t n, int64_t k) { return n <= 32 ? 1 : k <= 32 ? 4 : 2; }
-int64_t assign_pad(int64_t n, int64_t k) { return ceil_div(n, 32 * assign_chunk(n, k)) * 32 * assign_chunk(n, k); }
-size_t assign_lds(int64_t n, int64_t k) {
-  const int64_t steps = ceil_div(k, 16), n_pad = assign_pad(n, k);
-  const int64_t pieces = 2 * (n_pad / 32) * steps * 64 * 16, threads = assign_threads((int)steps);
-  return (size_t)(pieces + 2 * n_pad * 4 + 16 + (1 + 2 * threads / kWave) * 16 * steps * 4 + 2 * threads * 4);
-}
-
 template <int S, int T>
 int assign_pick(const AssignArgs& a, size_t lds, hipStream_t st) {
+  if (a.sums != nullptr) return launch_assign<S, T, true, true>(a, lds, st);
   if constexpr (S == 1) {
     // In fewer than four dimensions so many centres are close to a row that the slots' share of the near-tie bound
     // sends more rows to the exact evaluation than the packed update saves.
-    if (a.k < 4) return a.n <= 32 ? launch_assign<1, 1, false>(a, lds, st) : launch_assign<1, T, false>(a, lds, st);
+    if (a.k < 4) return launch_assign<1, T, false, false>(a, lds, st);
   }
-  if (a.n <= 32) return launch_assign<S, 1, true>(a, lds, st);
-  return launch_assign<S, T, true>(a, lds, st);
+  return launch_assign<S, T, true, false>(a, lds, st);
+}
+
+template <int S>
+int assign_chunks(const AssignArgs& a, size_t lds, hipStream_t st) {
+  switch (assign_chunk(a.n, a.k)) {
+    case 1: return assign_pick<S, 1>(a, lds, st);
+    case 2: return assign_pick<S, 2>(a, lds, st);
+    default:
+      if constexpr (S <= 2) return assign_pick<S, 4>(a, lds, st);
+      else return fail(F2CGT_E_UNSUPPORTED, "kmeans_predict: no chunks of four tiles at this width");
+  }
 }
 
 int assign_dispatch(AssignArgs a, hipStream_t st) {
   a.n_pad = (int)assign_pad(a.n, a.k);
-  const size_t lds = assign_lds(a.n, a.k);
+  const size_t lds = a.sums != nullptr ? assign_sums_lds(a.n, a.k) : assign_lds(a.n, a.k);
   switch (ceil_div(a.k, 16)) {
-    case 1: return assign_pick<1, 4>(a, lds, st);
-    case 2: return assign_pick<2, 4>(a, lds, st);
-    case 3: return assign_pick<3, 2>(a, lds, st);
-    default: return assign_pick<4, 2>(a, lds, st);
+    case 1: return assign_chunks<1>(a, lds, st);
+    case 2: return assign_chunks<2>(a, lds, st);
+    case 3: return assign_chunks<3>(a, lds, st);
+    default: return assign_chunks<4>(a, lds, st);
   }
 }
 
@@ -778,6 +864,25 @@ int assign_rows(const float* x, const float* centers, int64_t* lab64, uint8_t* l
   AssignArgs a{};
   a.x = x; a.centers = centers; a.lab64 = lab64; a.lab8 = lab8; a.m = m; a.n = n; a.k = k; a.metric = metric;
   a.slices = 1; a.feat_dim = k; a.ldx = k; a.label_stride = 1;
+  return assign_dispatch(a, st);
+}
+
+// The sums take LDS beside the operands, in a workgroup that has a CU to itself; as many slices as CUs.
+bool assign_sums_fits(int64_t slices, int64_t n, int64_t k) {
+  return slices >= 1 && slices <= 256 && assign_fits(n, k) && assign_sums_lds(n, k) <= 160 * 1024;
+}
+
+int64_t assign_sums_shares(int64_t m, int64_t slices, int64_t k) {
+  return assign_shares(m, slices, num_cus(), assign_threads((int)ceil_div(k, (int64_t)16)) / kWave);
+}
+
+int assign_sums(const float* x, int64_t slice_step, const uint32_t* keep, int64_t keep_words, const float* centers,
+                const int32_t* stop, float* sums, uint32_t* arrived, int64_t m, int slices, int n, int k, int metric,
+                hipStream_t st) {
+  AssignArgs a{};
+  a.x = x; a.centers = centers; a.m = m; a.n = n; a.k = k; a.metric = metric;
+  a.slices = slices; a.feat_dim = slices * k; a.ldx = k; a.slice_step = slice_step;
+  a.stop = stop; a.keep = keep; a.keep_words = keep_words; a.sums = sums; a.arrived = arrived;
   return assign_dispatch(a, st);
 }
 
@@ -807,5 +912,6 @@ extern "C" int f2cgt_vq_encode_slices(const float* x, int64_t ldx, int64_t feat_
   AssignArgs a{};
   a.x = x; a.centers = codebooks; a.lab8 = codes; a.m = m; a.n = (int)n; a.k = (int)k; a.metric = metric;
   a.slices = (int)slices; a.feat_dim = (int)feat_dim; a.ldx = ldx; a.label_stride = code_stride;
+  a.slice_step = k;
   return assign_dispatch(a, as_stream(stream));
 }

@@ -363,6 +363,94 @@ torch::Tensor kmeans_update(torch::Tensor x, torch::Tensor labels, torch::Tensor
   return shift;
 }
 
+// The rows of a sample, column slice by column slice: (rows fp32 [slices, m, k], their lengths fp32 [m, slices], flag
+// int32 [1] on the device: an id lies outside the table).
+std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> slice_rows(torch::Tensor x, c10::optional<torch::Tensor> rows,
+                                                                   int64_t column_slice) {
+  TORCH_CHECK(x.defined() && x.is_cuda() && x.dim() == 2 && x.scalar_type() == torch::kFloat32,
+              "x must be a float32 GPU tensor [rows, feat_dim]");
+  TORCH_CHECK(x.size(0) > 0 && x.size(1) > 0 && column_slice > 0, "x and column_slice must not be empty");
+  if (x.stride(1) != 1 || x.stride(0) < x.size(1)) x = x.contiguous();
+  const int64_t ld = x.size(0) > 1 ? x.stride(0) : x.size(1);
+  torch::Tensor r;
+  if (rows.has_value()) {
+    r = dev_contig(*rows, "rows");
+    TORCH_CHECK(r.dim() == 1 && r.scalar_type() == torch::kInt64 && r.device() == x.device(),
+                "rows must be int64 [m] on the device of x");
+  }
+  c10::DeviceGuard guard(x.device());
+  const int64_t m = r.defined() ? r.numel() : x.size(0), cols = x.size(1), slices = (cols + column_slice - 1) / column_slice;
+  auto out = empty_f32({slices, m, column_slice}, x);
+  auto norms = empty_f32({m, slices}, x);
+  auto bad = torch::zeros({1}, torch::TensorOptions().dtype(torch::kInt32).device(x.device()));
+  check_rc(f2cgt_slice_rows(x.data_ptr<float>(), ld, r.defined() ? r.data_ptr<int64_t>() : nullptr, m, x.size(0), cols,
+                            column_slice, out.data_ptr<float>(), norms.data_ptr<float>(), bad.data_ptr<int32_t>(),
+                            current_stream()),
+           "slice_rows");
+  return {out, norms, bad};
+}
+
+// Bits (int32 [slices, ceil(m / 32)]) of the rows that are as long as a quantile of their slice's lengths, from the order
+// statistics of `norms` on both sides of it.
+torch::Tensor keep_rows(torch::Tensor norms, torch::Tensor stats, double weight, double weight_last) {
+  norms = dev_contig(norms, "norms");
+  stats = dev_contig(stats, "stats");
+  TORCH_CHECK(norms.dim() == 2 && norms.scalar_type() == torch::kFloat32, "norms must be float32 [m, slices]");
+  TORCH_CHECK(stats.dim() == 2 && stats.size(0) == norms.size(1) && stats.size(1) == 6 &&
+                  stats.scalar_type() == torch::kFloat64 && stats.device() == norms.device(),
+              "stats must be float64 [slices, 6] on the device of norms");
+  c10::DeviceGuard guard(norms.device());
+  auto keep = torch::empty({norms.size(1), (norms.size(0) + 31) / 32},
+                           torch::TensorOptions().dtype(torch::kInt32).device(norms.device()));
+  check_rc(f2cgt_keep_rows(norms.data_ptr<float>(), stats.data_ptr<double>(), (float)weight, (float)weight_last, norms.size(0),
+                           norms.size(1), reinterpret_cast<uint32_t*>(keep.data_ptr<int32_t>()), current_stream()),
+           "keep_rows");
+  return keep;
+}
+
+bool kmeans_slices_covers(int64_t slices, int64_t n, int64_t k) { return f2cgt_kmeans_slices_covers(slices, n, k) != 0; }
+
+// Lloyd iterations of all slices on x [slices, m, k] from `centers` [slices, n, k] (updated in place), until every slice
+// has met `rule` or for max_iter steps; tol grows by `growth` each step.  The flags are read every check_every steps and
+// at the end.  -> int32 [slices] on the host: 0 not met, 1 met, 2 the shift became NaN.
+torch::Tensor kmeans_slices_fit(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, std::string metric,
+                                int64_t rule, double tol, double growth, int64_t max_iter, int64_t check_every) {
+  x = dev_contig(x, "x");
+  TORCH_CHECK(x.dim() == 3 && x.scalar_type() == torch::kFloat32, "x must be float32 [slices, m, k]");
+  TORCH_CHECK(centers.is_cuda() && centers.is_contiguous() && centers.scalar_type() == torch::kFloat32 && centers.dim() == 3 &&
+                  centers.size(0) == x.size(0) && centers.size(2) == x.size(2) && centers.device() == x.device(),
+              "centers must be a contiguous float32 tensor [slices, n, k] on the device of x (it is updated in place)");
+  const int64_t slices = x.size(0), m = x.size(1), k = x.size(2), n = centers.size(1);
+  const uint32_t* bits = nullptr;
+  if (keep.has_value()) {
+    TORCH_CHECK(keep->device() == x.device() && keep->is_contiguous() && keep->scalar_type() == torch::kInt32 &&
+                    keep->dim() == 2 && keep->size(0) == slices && keep->size(1) == (m + 31) / 32,
+                "keep must be a contiguous int32 tensor [slices, ceil(m / 32)] on the device of x");
+    bits = reinterpret_cast<const uint32_t*>(keep->data_ptr<int32_t>());
+  }
+  TORCH_CHECK(check_every > 0, "check_every must be positive");
+  const int tag = metric_tag(metric);
+  c10::DeviceGuard guard(x.device());
+  auto stop = torch::zeros({slices}, torch::TensorOptions().dtype(torch::kInt32).device(x.device()));
+  auto ws = torch::empty({f2cgt_kmeans_slices_workspace_bytes(m, slices, n, k)},
+                         torch::TensorOptions().dtype(torch::kUInt8).device(x.device()));
+  py::gil_scoped_release unlocked;
+  for (int64_t it = 0; it < max_iter; ++it) {
+    check_rc(f2cgt_kmeans_slices_step(x.data_ptr<float>(), bits, centers.data_ptr<float>(), stop.data_ptr<int32_t>(), (int)rule,
+                                      (float)tol, ws.data_ptr(), ws.numel(), m, slices, n, k, tag, current_stream()),
+             "kmeans_slices_fit");
+    tol *= growth;
+    if (it % check_every == check_every - 1 && it + 1 < max_iter) {
+      auto seen = stop.cpu();
+      const int32_t* f = seen.data_ptr<int32_t>();
+      bool all = true;
+      for (int64_t s = 0; s < slices; ++s) all = all && f[s] != 0;
+      if (all) return seen;
+    }
+  }
+  return stop.cpu();
+}
+
 // Counterpart of the reference's raft-backed KMeans (src/kmeans.h:13-31, src/kmeans.cu).
 // predict() is the fused MFMA distance + arg-min kernel.  fit() is Lloyd's algorithm on the device:
 // assignment (f2cgt_kmeans_predict) and centre update (f2cgt_kmeans_update) per iteration, stopped by
@@ -819,6 +907,11 @@ PYBIND11_MODULE(F2CGTLib, m) {
            py::arg("slot_map") = py::none())
       .def("kmeans_update", &kmeans_update, py::arg("data"), py::arg("labels"), py::arg("centers"),
            py::arg("stop") = py::none(), py::arg("rule") = 0, py::arg("tol") = 0.0)
+      .def("slice_rows", &slice_rows, py::arg("x"), py::arg("rows"), py::arg("column_slice"))
+      .def("keep_rows", &keep_rows, py::arg("norms"), py::arg("stats"), py::arg("weight"), py::arg("weight_last"))
+      .def("kmeans_slices_covers", &kmeans_slices_covers, py::arg("slices"), py::arg("n"), py::arg("k"))
+      .def("kmeans_slices_fit", &kmeans_slices_fit, py::arg("x"), py::arg("keep"), py::arg("centers"), py::arg("metric"),
+           py::arg("rule"), py::arg("tol"), py::arg("growth"), py::arg("max_iter"), py::arg("check_every"))
       .def("set_store_mode", &set_store_mode, py::arg("mode"));
   py::class_<KMeans>(m, "KMeans")
       .def(py::init<int64_t, int64_t, std::string, int, double, int, double, int, int, bool>(),

@@ -179,6 +179,20 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
     return out, codebooks
 
 
+def _circle_centers(n, width, generator=None, slices=1):
+    """[slices * n, width] random unit-circle pairs on the host, the draws of one slice after those of the one before."""
+    half = width // 2
+    if width % 2 == 0:
+        angles = torch.rand((slices * n, half), generator=generator) * (2 * math.pi)
+        return torch.cat([torch.cos(angles), torch.sin(angles)], dim=1).float()
+    parts = []
+    for _ in range(slices):
+        radii = torch.rand((n, 1), generator=generator)
+        angles = torch.rand((n, half + 1), generator=generator) * (2 * math.pi)
+        parts.append(radii * torch.cat([torch.cos(angles[:, :half]), torch.sin(angles)], dim=1))
+    return torch.cat(parts).float()
+
+
 class KMeansTrainer:
     """Codebook trainer of the offline compressor (examples/my_kmeans.py:73-113, 150-184), on the
     device from start to finish: assignment by `kmeans_predict`, centre update and stopping rule by
@@ -205,15 +219,7 @@ class KMeansTrainer:
     def _initial_centers(self, data):
         n, width = self.num_clusters, data.shape[1]
         if self.metric == "cosine":
-            half = width // 2
-            if width % 2 == 0:
-                angles = torch.rand((n, half), generator=self.generator) * (2 * math.pi)
-                start = torch.cat([torch.cos(angles), torch.sin(angles)], dim=1)
-            else:
-                radii = torch.rand((n, 1), generator=self.generator)
-                angles = torch.rand((n, half + 1), generator=self.generator) * (2 * math.pi)
-                start = radii * torch.cat([torch.cos(angles[:, :half]), torch.sin(angles)], dim=1)
-            return start.float().cuda()
+            return _circle_centers(n, width, self.generator).cuda()
         alive = torch.nonzero(torch.count_nonzero(data, dim=1)).flatten()
         if alive.numel() < n:
             raise ValueError("fewer non-zero rows than clusters")
@@ -251,6 +257,57 @@ class KMeansTrainer:
         return _capi().kmeans_predict(data.float().cuda().contiguous(), self.centers, metric)
 
 
+def _rim_quantile(width):
+    return min(1.0, 0.00625 * (width / 8))
+
+
+def _rim_place(m, width):
+    """Where torch's linear quantile of m float32 values lies: (rank below, rank above, weight of the latter), in the
+    values' own precision."""
+    place = np.float32(_rim_quantile(width)) * np.float32(m - 1)
+    below = np.floor(place)
+    return int(below), int(np.ceil(place)), float(np.float32(place - below))
+
+
+def _train_all_slices(features, n_clusters, column_slice, sample_index, max_iter):
+    """The codebooks of vq_metadata with every step made for all slices at once, or None where that is not covered: more
+    slices, centres or columns than a step takes, samples that are no plain list of row ids, empty or beyond 2^24 rows
+    (torch's quantile) or 2^28 values."""
+    capi = _capi()
+    feat_dim = features.shape[1]
+    slices = (feat_dim + column_slice - 1) // column_slice
+    m = sample_index.numel()
+    if not (sample_index.dtype == torch.int64 and sample_index.dim() == 1 and 0 < m <= 1 << 24 and m * feat_dim <= 1 << 28 and
+            capi.kmeans_slices_covers(slices, n_clusters, column_slice) and features.shape[0] > 0):
+        return None
+    if features.is_cuda and features.dtype == torch.float32 and features.stride(1) == 1 and features.stride(0) >= feat_dim:
+        table, rows = features, sample_index.to(features.device)
+    else:
+        table, rows = features[sample_index.to(features.device)].to(torch.float32).cuda(), None
+    data, lengths, bad_row = capi.slice_rows(table, rows, column_slice)
+    last = feat_dim - (slices - 1) * column_slice
+    places = [_rim_place(m, width) for width in (min(column_slice, feat_dim), last)]
+    stats = capi.abs_order_stats(lengths, None, 1, [r for p in places for r in (p[0], p[1], p[0], p[1])])
+    keep = capi.keep_rows(lengths, stats, places[0][2], places[1][2])
+    # the draws of the trainers, slice after slice
+    whole = slices - 1 if last < column_slice else slices
+    start = torch.zeros((slices, n_clusters, column_slice))
+    if whole:
+        start[:whole] = _circle_centers(n_clusters, column_slice, slices=whole).view(whole, n_clusters, column_slice)
+    if whole < slices:
+        start[whole, :, :last] = _circle_centers(n_clusters, last)
+    centers = start.cuda()
+    flags = capi.kmeans_slices_fit(data, keep, centers, "cosine", 2, 5e-2, 1.2, max_iter, 8)
+    if rows is not None and int(bad_row.item()):
+        raise IndexError("a sample id lies outside the table's %d rows" % features.shape[0])
+    if bool((flags == 2).any()):
+        import warnings
+        warnings.warn("vq_metadata: the centre shift became NaN; no centres were produced")
+        raise TypeError("a column slice has no centres")
+    norms = torch.linalg.vector_norm(centers, ord=2, dim=2, keepdim=True)
+    return (centers / norms) * norms.mean(dim=1, keepdim=True)
+
+
 def vq_metadata(features, n_clusters, column_slice, hotness=None, sample_index=None, max_iter=1000):
     """Codebooks fp32 [ceil(D / column_slice), n_clusters, column_slice]: per slice, rows of a
     sample inside the rim quantile are dropped, k-means (cosine, tol 5e-2) runs on the rest and the
@@ -260,12 +317,17 @@ def vq_metadata(features, n_clusters, column_slice, hotness=None, sample_index=N
     if sample_index is None:
         sample_index = sampling(150_000, num_items, hotness)
     num_slice = (feat_dim + column_slice - 1) // column_slice
-    codebooks = torch.zeros((num_slice, n_clusters, column_slice), device="cuda", dtype=torch.float32)
-    for i in range(num_slice):
+    codebooks = _train_all_slices(features, n_clusters, column_slice, sample_index, max_iter)
+    if codebooks is None:
+        codebooks = torch.zeros((num_slice, n_clusters, column_slice), device="cuda", dtype=torch.float32)
+        per_slice = range(num_slice)
+    else:
+        per_slice = ()
+    for i in per_slice:
         lo, hi = i * column_slice, min((i + 1) * column_slice, feat_dim)
         data = features[sample_index.to(features.device), lo:hi].to(torch.float32).cuda()
         distance = data.norm(dim=1, p=2)
-        rim = torch.quantile(distance, min(1.0, 0.00625 * (data.shape[1] / 8)))
+        rim = torch.quantile(distance, _rim_quantile(data.shape[1]))
         data = data[torch.ge(distance, rim)].contiguous()
         km = KMeansTrainer(n_clusters, metric="cosine", tol=5e-2, max_iter=max_iter)
         km.fit(data)

@@ -296,6 +296,34 @@ int f2cgt_kmeans_update_static(const float* x, const int64_t* labels_i64, const 
                                float* centers, float* shift, int32_t* stop, int stop_rule, float tol,
                                int64_t m, int64_t n, int64_t k, void* stream);
 
+/* Codebook training of all column slices of a sample at once (examples/process_compress.py:147-182, one slice at a time).
+ *
+ * f2cgt_slice_rows: the sample, slice by slice.  x: row r starts ld floats after row r - 1; rows int64 [m] (NULL: rows
+ * [0, m)), negative ids count from the end; slice s has the columns [s k, s k + k), zeros after the last one (k <= 64).
+ * out fp32 [slices, m, k]; norms fp32 [m, slices]; bad_row (device int32): set where an id lies outside the table (the row
+ * read is then another one of it).
+ *
+ * f2cgt_keep_rows: which rows take part, the ones at least as long as a quantile of their slice's lengths.  stats fp64
+ * [slices, 6] as f2cgt_abs_order_stats leaves them for norms: the lengths below and above the quantile and, last, flags
+ * (a slice with NaN keeps no row); weight, weight_last: where between the two it lies (of a slice, and of the last one).
+ * keep uint32 [slices, ceil(m / 32)]: bit r % 32 of word r / 32.
+ *
+ * f2cgt_kmeans_slices_step: one Lloyd iteration of every slice whose stop flag is zero, as f2cgt_kmeans_predict and
+ * f2cgt_kmeans_update would make it from the rows kept: x fp32 [slices, m, k], keep as above or NULL (all), centers fp32
+ * [slices, n, k] updated in place, stop int32 [slices] (device) with stop_rule and tol as in f2cgt_kmeans_update.  A label
+ * is the true first minimum; the sums are fp32, a workgroup's rows added in LDS, the sets in a fixed order.
+ * workspace: f2cgt_kmeans_slices_workspace_bytes, 16-byte aligned.  f2cgt_kmeans_slices_covers: 1 where the shape is
+ * taken (operands and sums of a slice in LDS, up to 256 slices, 512 centres, 64 columns), else 0. */
+int f2cgt_slice_rows(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols, int64_t k,
+                     float* out, float* norms, int32_t* bad_row, void* stream);
+int f2cgt_keep_rows(const float* norms, const double* stats, float weight, float weight_last, int64_t m, int64_t slices,
+                    uint32_t* keep, void* stream);
+int f2cgt_kmeans_slices_covers(int64_t slices, int64_t n, int64_t k);
+int64_t f2cgt_kmeans_slices_workspace_bytes(int64_t m, int64_t slices, int64_t n, int64_t k);
+int f2cgt_kmeans_slices_step(const float* x, const uint32_t* keep, float* centers, int32_t* stop, int stop_rule, float tol,
+                             void* workspace, int64_t workspace_bytes, int64_t m, int64_t slices, int64_t n, int64_t k,
+                             int metric, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
