@@ -183,14 +183,15 @@ torch::Tensor sq_encode(torch::Tensor src, torch::Tensor codebooks, int64_t targ
 
 // Extension: order statistics, sum and flags (1: a NaN, 2: a row id outside the table) of |x| per column slice of the rows
 // `rows` (None: all of them), for the codebooks of sq_encode.  ranks: four ranks in a full slice, four in the last one.  -> float64 [n_slices, 6] on the GPU.
-torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
-                              const std::vector<int64_t>& ranks) {
+std::tuple<torch::Tensor, torch::Tensor> order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
+                                                     const std::vector<int64_t>& ranks, const std::vector<float>* weights) {
   TORCH_CHECK(x.defined() && x.device().is_cuda(), "x must be a GPU tensor");
   TORCH_CHECK(x.dim() == 2 && x.scalar_type() == torch::kFloat32, "x must be float32 [rows, feat_dim]");
   // columns apart, or rows that overlap (an expanded row): a copy.  The stride of a single row may be anything.
   if (x.stride(1) != 1 || x.stride(0) < x.size(1)) x = x.contiguous();
   const int64_t ld = x.size(0) > 1 ? x.stride(0) : x.size(1);
   TORCH_CHECK(ranks.size() == 8, "ranks must hold eight values");
+  TORCH_CHECK(weights == nullptr || weights->size() == 4, "weights must hold four values");
   TORCH_CHECK(column_slice > 0, "column_slice must be positive");
   torch::Tensor r;
   if (rows.has_value()) {
@@ -200,14 +201,35 @@ torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows
   }
   c10::DeviceGuard guard(x.device());
   const int64_t m = r.defined() ? r.numel() : x.size(0), cols = x.size(1);
+  const int64_t slices = (cols + column_slice - 1) / column_slice;
   auto opts = torch::TensorOptions().device(x.device());
-  auto out = torch::empty({(cols + column_slice - 1) / column_slice, 6}, opts.dtype(torch::kFloat64));
+  auto out = torch::empty({slices, 6}, opts.dtype(torch::kFloat64));
   auto ws = torch::empty({f2cgt_abs_order_stats_workspace_bytes(m, cols, column_slice)}, opts.dtype(torch::kUInt8));
-  check_rc(f2cgt_abs_order_stats(x.data_ptr<float>(), ld, r.defined() ? r.data_ptr<int64_t>() : nullptr, m,
-                                 x.size(0), cols, column_slice, ranks.data(), ws.data_ptr(), ws.numel(),
-                                 out.data_ptr<double>(), current_stream()),
-           "abs_order_stats");
-  return out;
+  const int64_t* list = r.defined() ? r.data_ptr<int64_t>() : nullptr;
+  torch::Tensor books;
+  if (weights != nullptr) {
+    books = torch::empty({slices, 5}, opts.dtype(torch::kFloat32));
+    check_rc(f2cgt_sq_codebooks(x.data_ptr<float>(), ld, list, m, x.size(0), cols, column_slice, ranks.data(), weights->data(),
+                                ws.data_ptr(), ws.numel(), out.data_ptr<double>(), books.data_ptr<float>(), current_stream()),
+             "sq_codebooks");
+  } else {
+    check_rc(f2cgt_abs_order_stats(x.data_ptr<float>(), ld, list, m, x.size(0), cols, column_slice, ranks.data(),
+                                   ws.data_ptr(), ws.numel(), out.data_ptr<double>(), current_stream()),
+             "abs_order_stats");
+  }
+  return {out, books};
+}
+
+torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
+                              const std::vector<int64_t>& ranks) {
+  return std::get<0>(order_stats(x, rows, column_slice, ranks, nullptr));
+}
+
+// -> (codebooks fp32 [slices, 5], the statistics they were made from fp64 [slices, 6]), both on the device.
+std::tuple<torch::Tensor, torch::Tensor> sq_codebooks(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
+                                                      const std::vector<int64_t>& ranks, const std::vector<float>& weights) {
+  auto both = order_stats(x, rows, column_slice, ranks, &weights);
+  return {std::get<1>(both), std::get<0>(both)};
 }
 
 torch::Tensor sq_decompress(torch::Tensor compress_data, torch::Tensor codebooks, int64_t target_bits,
@@ -900,6 +922,8 @@ PYBIND11_MODULE(F2CGTLib, m) {
       .def("sq_encode", &sq_encode, py::arg("src"), py::arg("codebooks"), py::arg("target_bits"),
            py::arg("column_slice"), py::arg("out") = py::none())
       .def("abs_order_stats", &abs_order_stats, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"))
+      .def("sq_codebooks", &sq_codebooks, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"),
+           py::arg("weights"))
       .def("kmeans_predict", &kmeans_predict, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode", &vq_encode, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode_slices", &vq_encode_slices, py::arg("x"), py::arg("codebooks"), py::arg("out"), py::arg("metric"))

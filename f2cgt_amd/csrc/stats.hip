@@ -12,8 +12,9 @@
 //
 // What bounds it: the three reads of the sample (17 us each at 120 000 x 100 values, 2.9 TB/s through the row list; the
 // sums between them 3-4 us each).  The seven launches take 66 us where the host took 195 ms on a copy of the sample
-// (np.percentile, two selections); the whole sq_compress call, with one read-back and one upload of the codebook,
-// 132 us against 195-228 ms.
+// (np.percentile, two selections).  The codebook is made by the last of them, so that the encoder can follow at once: the
+// whole sq_compress call took 130 us with a read-back, the host's arithmetic and an upload in between (195-228 ms with the
+// host's percentiles), now 105, of which the encoder is 15 and the read-back of the flags at the end about 20.
 #include "common.hpp"
 
 namespace f2cgt {
@@ -45,6 +46,8 @@ struct StatArgs {
   double* sums;                      // [n_slices][blocks]
   uint32_t* flags;                   // [n_slices][blocks]: kSawNan, kSawBadRow
   double* out;                       // [n_slices][6]
+  float* books;                      // [n_slices][5], or null
+  float weights[4];                  // lower and upper percentile of a slice, and of the last one: where between its ranks
 };
 
 // Finds, in `groups` runs of kBins / groups counters, the counter that holds rank[t] (run t, or the only run), for all
@@ -256,6 +259,31 @@ __global__ __launch_bounds__(kStatThreads) void stat_reduce_kernel(StatArgs a) {
   a.hist[(int64_t)slice * kBins + bin] = c;
 }
 
+// The quantiser's codebook of a slice (fmin, fmax, emin, emax, mean) from its statistics: percentiles interpolated in
+// float32 from the nearer rank, floored at 1e-5 and 2e-5, their log2 correctly rounded, and the mean, lifted by 0.1 where
+// it is below 0.1 (examples/process_compress.py:45-68).  A NaN stays one.
+__device__ void sq_codebook(const StatArgs& a, int slice, const float (&at)[4], double total, uint32_t flags) {
+  const bool last = slice == a.n_slices - 1;
+  auto between = [](float below, float above, float w) {
+    const float gap = above - below;
+    return w < 0.5f ? below + gap * w : above - gap * (1.f - w);
+  };
+  float lo = between(at[0], at[1], a.weights[last ? 2 : 0]), hi = between(at[2], at[3], a.weights[last ? 3 : 1]);
+  if (flags & kSawNan) lo = hi = __uint_as_float(0x7fc00000u);
+  const float floor = 1e-5f;
+  lo = floor > lo ? floor : lo;
+  hi = 2e-5f > hi ? 2e-5f : hi;
+  const int64_t width = last ? a.cols - (int64_t)slice * a.slice : a.slice;
+  float level = (float)(total / (double)(a.m * width));
+  level = level < 0.1f ? level + 0.1f : level;
+  float* book = a.books + slice * 5;
+  book[0] = lo;
+  book[1] = hi;
+  book[2] = log2_cr(lo);
+  book[3] = log2_cr(hi) + floor;
+  book[4] = level;
+}
+
 // Last digit, and the outputs of a slice: the values at the four ranks, the sum, the flags.
 __global__ __launch_bounds__(kStatThreads) void stat_finish_kernel(StatArgs a) {
   __shared__ uint64_t s_scan[kStatThreads / kWave];
@@ -281,6 +309,11 @@ __global__ __launch_bounds__(kStatThreads) void stat_finish_kernel(StatArgs a) {
     if (t == kWave) {
       a.out[slice * 6 + 4] = total;
       a.out[slice * 6 + 5] = (double)flags;
+      if (a.books != nullptr) {
+        const float at[4] = {__uint_as_float(prefix[0]), __uint_as_float(prefix[1]), __uint_as_float(prefix[2]),
+                             __uint_as_float(prefix[3])};
+        sq_codebook(a, slice, at, total, flags);
+      }
     }
   }
 }
@@ -337,10 +370,10 @@ extern "C" int64_t f2cgt_abs_order_stats_workspace_bytes(int64_t m, int64_t cols
   return stat_layout(stat_blocks(m, cols, column_slice, n_slices), n_slices).total;
 }
 
-extern "C" int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows,
-                                     int64_t cols, int64_t column_slice, const int64_t* ranks, void* workspace,
-                                     int64_t workspace_bytes, double* out, void* stream) {
-  const char* what = "abs_order_stats";
+namespace {
+int order_stats(const char* what, const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols,
+                int64_t column_slice, const int64_t* ranks, const float* weights, void* workspace, int64_t workspace_bytes,
+                double* out, float* books, void* stream) {
   if (int rc = stat_check(what, m, cols, column_slice)) return rc;
   F2CGT_REQUIRE(ld >= cols && num_rows > 0 && (rows != nullptr || m <= num_rows), F2CGT_E_INVALID,
                 "%s: the sample does not fit the table", what);
@@ -368,6 +401,9 @@ extern "C" int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* 
   a.sums = reinterpret_cast<double*>(ws + l.sums);
   a.flags = reinterpret_cast<uint32_t*>(ws + l.flags);
   a.out = out;
+  a.books = books;
+  if (books != nullptr)
+    for (int k = 0; k < 4; ++k) a.weights[k] = weights[k];
   // widest access that every slice of every row is a multiple of
   const int64_t last_width = cols - (n_slices - 1) * column_slice;
   auto fits = [&](int v) {
@@ -378,4 +414,20 @@ extern "C" int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* 
   else if (fits(2)) stat_launch<2>(a, st);
   else stat_launch<1>(a, st);
   return launch_status(what);
+}
+}  // namespace
+
+extern "C" int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows,
+                                     int64_t cols, int64_t column_slice, const int64_t* ranks, void* workspace,
+                                     int64_t workspace_bytes, double* out, void* stream) {
+  return order_stats("abs_order_stats", x, ld, rows, m, num_rows, cols, column_slice, ranks, nullptr, workspace,
+                     workspace_bytes, out, nullptr, stream);
+}
+
+extern "C" int f2cgt_sq_codebooks(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols,
+                                  int64_t column_slice, const int64_t* ranks, const float* weights, void* workspace,
+                                  int64_t workspace_bytes, double* stats, float* codebooks, void* stream) {
+  F2CGT_REQUIRE(weights && codebooks, F2CGT_E_INVALID, "sq_codebooks: null buffer");
+  return order_stats("sq_codebooks", x, ld, rows, m, num_rows, cols, column_slice, ranks, weights, workspace,
+                     workspace_bytes, stats, codebooks, stream);
 }

@@ -76,14 +76,20 @@ def _sq_codebook(lo, hi, level):
     return fmin, fmax, torch.log2(fmin), torch.log2(fmax) + floor, level
 
 
+def _percentile_places(m, cols, column_slice):
+    """Sizes of a full slice and of the last one, and for both the place of either percentile."""
+    count = (cols + column_slice - 1) // column_slice
+    sizes = [m * min(column_slice, cols), m * (cols - (count - 1) * column_slice)]
+    return sizes, [[_percentile_place(n, q) for q in _PERCENTILES] for n in sizes]
+
+
 def _device_statistics(values, rows, column_slice):
     """Per column slice of float32 GPU rows: (0.5th and 99.5th percentile, mean) of |x|, from exact order statistics
     found on the device; the percentile's interpolation is numpy's, in float32."""
     m = values.shape[0] if rows is None else rows.numel()
     cols = values.shape[1]
     count = (cols + column_slice - 1) // column_slice
-    sizes = [m * min(column_slice, cols), m * (cols - (count - 1) * column_slice)]
-    places = [[_percentile_place(n, q) for q in _PERCENTILES] for n in sizes]
+    sizes, places = _percentile_places(m, cols, column_slice)
     ranks = [r for per_size in places for place in per_size for r in place[:2]]
     stats = _capi().abs_order_stats(values, rows, column_slice, ranks).cpu().numpy()
     out = []
@@ -155,15 +161,18 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
     if sample_index is None:
         sample_index = sampling(250_000, num_items, hotness)
     sample_index = sample_index.to(features.device)
+    stats = None
     if (features.is_cuda and features.dtype == torch.float32 and features.stride(1) == 1 and features.stride(0) >= feat_dim and
             sample_index.dtype == torch.int64 and sample_index.dim() == 1 and not features.requires_grad and
             _device_takes(sample_index.numel(), feat_dim, column_slice)):
-        # the sample's rows are read in place
-        per_slice = [_sq_codebook(*values) for values in _device_statistics(features, sample_index, column_slice)]
+        # the sample's rows are read in place, the codebooks made where they are used; a bad id is found at the end
+        places = _percentile_places(sample_index.numel(), feat_dim, column_slice)[1]
+        codebooks, stats = capi.sq_codebooks(features, sample_index, column_slice,
+                                             [r for per_size in places for place in per_size for r in place[:2]],
+                                             [place[2] for per_size in places for place in per_size])
     else:
-        per_slice = _sampled_sq_codebooks(features, sample_index, column_slice)
-    per_slice = [[float(v) for v in values] for values in per_slice]
-    codebooks = (torch.tensor(per_slice, dtype=torch.float32) if per_slice else torch.zeros((0, 5))).cuda()
+        per_slice = [[float(v) for v in values] for values in _sampled_sq_codebooks(features, sample_index, column_slice)]
+        codebooks = (torch.tensor(per_slice, dtype=torch.float32) if per_slice else torch.zeros((0, 5))).cuda()
     if target_bits <= 8:
         dtype, tdim = torch.int8, int(math.ceil(feat_dim / 8 * target_bits))
     elif target_bits <= 16:
@@ -176,6 +185,8 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
         data = features[start:end].cuda().to(torch.float32)
         # one pass; the reference calls sq_compress, casts and packs (process_compress.py:128-139)
         capi.sq_encode(data, codebooks, target_bits, column_slice, out[start:end])
+    if stats is not None and stats.cpu().numpy()[:, 5].max() >= 2:
+        raise IndexError("a sample id lies outside the table's %d rows" % num_items)
     return out, codebooks
 
 

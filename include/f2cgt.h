@@ -237,6 +237,13 @@ int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* rows, int64
                           int64_t column_slice, const int64_t* ranks, void* workspace, int64_t workspace_bytes,
                           double* out, void* stream);
 
+/* The same with the SQ codebooks themselves (fp32 [slices, 5] on the device: fmin, fmax, emin, emax, mean): ranks below and
+ * above the lower percentile, then those of the upper one; weights (host, 4 values): how far each percentile lies from its
+ * rank below to the one above, in a full slice and in the last one.  The log2 are correctly rounded. */
+int f2cgt_sq_codebooks(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols,
+                       int64_t column_slice, const int64_t* ranks, const float* weights, void* workspace,
+                       int64_t workspace_bytes, double* stats, float* codebooks, void* stream);
+
 /* ---- VQ encode ---------------------------------------------------------------- */
 
 /* Replaces pairwise_distance(), src/kmeans.cu:102-118 (raft L2Unexpanded /

@@ -195,3 +195,27 @@ def test_rows_with_a_pitch(listed, n, d, slice_, start, pitch):
         part = np.sort(sample[:, i * slice_:(i + 1) * slice_].ravel())
         assert np.array_equal(got[i, :4].astype(np.float32), part[ranks[4:] if i == count - 1 else ranks[:4]]) and got[i, 5] == 0.0
         assert np.allclose(got[i, 4], part.sum(dtype=np.float64), rtol=part.size * 2.0 ** -52)
+
+
+@pytest.mark.parametrize("scale", [1e-7, 1e-3, 1.0, 1e6])
+@pytest.mark.parametrize("n,d,slice_", [(1, 1, 8), (3, 5, 2), (2000, 33, 16), (300, 64, 64)])
+def test_codebooks_made_on_the_device(n, d, slice_, scale):
+    """Percentiles, floors and the lifted mean as from the statistics on the host; log2 correctly rounded."""
+    from f2cgt_amd import pipeline
+    x = (torch.randn((n, d), generator=torch.Generator().manual_seed(n + d)) * scale).cuda()
+    places = pipeline._percentile_places(n, d, slice_)[1]
+    books, stats = f2cgt_amd.load().sq_codebooks(x, None, slice_, [r for s in places for p in s for r in p[:2]],
+                                                 [p[2] for s in places for p in s])
+    want = [[float(v) for v in pipeline._sq_codebook(*values)] for values in pipeline._device_statistics(x, None, slice_)]
+    got, want = books.cpu().numpy(), np.array(want, dtype=np.float32)
+    assert np.array_equal(got[:, [0, 1, 4]], want[:, [0, 1, 4]]) and not stats.cpu()[:, 5].any()
+    assert np.array_equal(got[:, 2], np.log2(got[:, 0].astype(np.float64)).astype(np.float32))
+    assert np.array_equal(got[:, 3], np.log2(got[:, 1].astype(np.float64)).astype(np.float32) + np.float32(1e-5))
+
+
+def test_codebook_of_a_nan():
+    x = torch.rand((500, 16), device="cuda")
+    x[3, 9] = float("nan")
+    from f2cgt_amd import pipeline
+    books = pipeline.sq_compress(x, 4, 8, sample_index=torch.arange(500))[1].cpu()
+    assert not torch.isnan(books[0]).any() and torch.isnan(books[1]).all()
