@@ -38,6 +38,8 @@ SIGNATURES = {
     "f2cgt_hybrid_decompress_spmm_csr":
         ([P, P, P, L, P, P, P, P, I, P, L, L, L, L, L, L, L, L, L, P], c_int),
     "f2cgt_fetch_rows": ([P, P, P, P, I, P, L, L, L, L, P], c_int),
+    "f2cgt_vq_decompress_rows": ([P, P, I, P, P, L, L, L, L, L, L, P], c_int),
+    "f2cgt_sq_decompress_rows": ([P, I, P, I, P, L, P, P, P, L, L, L, L, L, I, L, P], c_int),
     "f2cgt_abs_order_stats_workspace_bytes": ([L, L, L], c_int64),
     "f2cgt_abs_order_stats": ([P, L, P, L, L, L, L, P, P, L, P, P], c_int),
     "f2cgt_sq_codebooks": ([P, L, P, L, L, L, L, P, P, P, L, P, P, P], c_int),

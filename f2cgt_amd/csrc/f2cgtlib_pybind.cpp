@@ -845,6 +845,86 @@ torch::Tensor fetch_rows(torch::Tensor table, torch::Tensor index, c10::optional
   return out;
 }
 
+// Rows `index` of a code table in device memory, decoded without a copy of their codes; where a shape is not covered,
+// fetched and decoded.
+torch::Tensor vq_decompress_rows(torch::Tensor table, torch::Tensor index, torch::Tensor codebooks, int64_t feat_dim) {
+  const bool plain = table.defined() && index.defined() && codebooks.defined() && table.is_cuda() && index.device() == table.device() &&
+                     codebooks.device() == table.device() && table.dim() == 2 && table.is_contiguous() && index.dim() == 1 &&
+                     codebooks.dim() == 3 && table.scalar_type() == torch::kUInt8 && codebooks.scalar_type() == torch::kFloat32 &&
+                     (index.scalar_type() == torch::kInt64 || index.scalar_type() == torch::kInt32) &&
+                     table.size(0) > 0 && table.size(1) == codebooks.size(0) && feat_dim >= 0;
+  if (plain) {
+    index = index.contiguous();
+    codebooks = codebooks.contiguous();
+    c10::DeviceGuard guard(table.device());
+    auto out = empty_f32({index.numel(), feat_dim}, table);
+    const int rc = f2cgt_vq_decompress_rows(table.data_ptr<uint8_t>(), index.data_ptr(),
+                                            index.scalar_type() == torch::kInt64 ? F2CGT_DT_I64 : F2CGT_DT_I32,
+                                            codebooks.data_ptr<float>(), out.data_ptr<float>(), index.numel(), table.size(0),
+                                            feat_dim, codebooks.size(0), codebooks.size(1), codebooks.size(2), current_stream());
+    if (rc >= 0) {
+      check_rc(rc, "vq_decompress_rows");
+      return out;
+    }
+  }
+  return vq_decompress(fetch_rows(table, index, c10::nullopt, c10::nullopt), codebooks, feat_dim);
+}
+
+// The same for scalar codes.  With a slot map the rows are slot_map[index]; check: ids without a row raise KeyError, ids
+// outside the map IndexError, behind a wait for the current stream.
+torch::Tensor sq_decompress_rows(torch::Tensor table, torch::Tensor index, torch::Tensor codebooks, int64_t target_bits,
+                                 int64_t column_slice, int64_t feat_dim, c10::optional<torch::Tensor> slot_map, bool check) {
+  const bool plain = table.defined() && index.defined() && table.is_cuda() && index.device() == table.device() && table.dim() == 2 &&
+                     table.is_contiguous() && index.dim() == 1 && table.size(0) > 0 &&
+                     (table.scalar_type() == torch::kInt8 || table.scalar_type() == torch::kUInt8) &&
+                     (index.scalar_type() == torch::kInt64 || index.scalar_type() == torch::kInt32) && feat_dim >= 0;
+  const bool mapped = slot_map.has_value();
+  if (mapped)
+    TORCH_CHECK(slot_map->device() == table.device() && slot_map->dim() == 1 && slot_map->is_contiguous() &&
+                    slot_map->scalar_type() == torch::kInt32 && slot_map->numel() > 0,
+                "slot_map must be a contiguous int32 tensor on the device of table");
+  if (plain) {
+    index = index.contiguous();
+    auto books = sq_codebooks_checked(codebooks);
+    c10::DeviceGuard guard(table.device());
+    auto out = empty_f32({index.numel(), feat_dim}, table);
+    torch::Tensor bad;
+    int32_t* flag = nullptr;
+    if (mapped && check) {
+      // one word of pinned memory, which the kernel writes only for a bad id
+      bad = torch::empty({1}, torch::TensorOptions().dtype(torch::kInt32).pinned_memory(true));
+      flag = bad.data_ptr<int32_t>();
+      *flag = 0;
+    }
+    const int rc = f2cgt_sq_decompress_rows(
+        table.data_ptr(), dtype_tag(table, "table"), index.data_ptr(),
+        index.scalar_type() == torch::kInt64 ? F2CGT_DT_I64 : F2CGT_DT_I32, mapped ? slot_map->data_ptr<int32_t>() : nullptr,
+        mapped ? slot_map->numel() : 0, flag, books.data_ptr<float>(), out.data_ptr<float>(), index.numel(), table.size(0),
+        table.size(1), feat_dim, books.size(0), (int)target_bits, column_slice, current_stream());
+    if (rc >= 0) {
+      check_rc(rc, "sq_decompress_rows");
+      if (flag != nullptr) {
+        {
+          py::gil_scoped_release unlocked;
+          c10::hip::getCurrentHIPStream().synchronize();
+        }
+        const int32_t seen = *const_cast<volatile int32_t*>(flag);
+        if (seen == 1) throw py::key_error("a requested id is not a seed row");
+        if (seen != 0) throw py::index_error("an id lies outside the slot map");
+      }
+      return out;
+    }
+  }
+  if (mapped) {
+    auto slots = slot_map->index({index.to(torch::kInt64)}).to(torch::kInt64);
+    if (check && slots.lt(0).any().item<bool>()) throw py::key_error("a requested id is not a seed row");
+    index = slots;
+  } else if (index.scalar_type() != torch::kInt64 && index.scalar_type() != torch::kInt32) {
+    index = index.to(torch::kInt64);
+  }
+  return sq_decompress(fetch_rows(table, index, c10::nullopt, c10::nullopt), codebooks, target_bits, column_slice, feat_dim);
+}
+
 torch::Tensor vq_encode(torch::Tensor x, torch::Tensor centers, std::string metric) {
   return kmeans_predict_impl(x, centers, metric, true);
 }
@@ -927,6 +1007,11 @@ PYBIND11_MODULE(F2CGTLib, m) {
       .def("kmeans_predict", &kmeans_predict, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode", &vq_encode, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode_slices", &vq_encode_slices, py::arg("x"), py::arg("codebooks"), py::arg("out"), py::arg("metric"))
+      .def("vq_decompress_rows", &vq_decompress_rows, py::arg("table"), py::arg("index"), py::arg("codebooks"),
+           py::arg("feat_dim"))
+      .def("sq_decompress_rows", &sq_decompress_rows, py::arg("table"), py::arg("index"), py::arg("codebooks"),
+           py::arg("target_bits"), py::arg("column_slice"), py::arg("feat_dim"), py::arg("slot_map") = py::none(),
+           py::arg("check") = false)
       .def("fetch_rows", &fetch_rows, py::arg("table"), py::arg("index"), py::arg("hot") = py::none(),
            py::arg("slot_map") = py::none())
       .def("kmeans_update", &kmeans_update, py::arg("data"), py::arg("labels"), py::arg("centers"),

@@ -5,6 +5,8 @@
 // (4 B per element against bits/8 B on the packed side).
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace f2cgt {
 namespace {
 
@@ -224,9 +226,32 @@ struct F4Args {
   uint32_t f4_per_row;
   uint32_t magic;         // ceil(2^32 / f4_per_row)
   int feat_dim;           // sq_decode_pairs_kernel: columns of a row
+  // ROWS: output row r is decoded from row index[r] of a table of num_rows, or, with a slot map, from row
+  // slot[index[r]]; *bad (host memory) becomes 1 where the map has no row for an id, 2 where an id is not on the map
+  const void* index;
+  const int32_t* slot;
+  int64_t num_rows, num_slots;
+  int32_t* bad;
 };
 
-template <int BITS, bool AFFINE>
+// Table row of output row r (ROWS: int32_t or int64_t ids, void without).  The lookup, the check of its ids, the fetch and
+// the decode are one kernel that way: seven launches and a copied row less for the seed rows of a minibatch.
+template <typename ROWS>
+__device__ __forceinline__ int64_t table_row(const F4Args& a, int64_t r) {
+  if constexpr (std::is_void<ROWS>::value) {
+    return r;
+  } else {
+    int64_t id = (int64_t)static_cast<const ROWS*>(a.index)[r];
+    if (a.slot == nullptr) return clamp_idx(id, a.num_rows);
+    id = id < 0 ? id + a.num_slots : id;
+    const bool on = id >= 0 && id < a.num_slots;
+    const int32_t s = a.slot[on ? id : 0];
+    if (a.bad != nullptr && (!on || s < 0)) *a.bad = on ? 1 : 2;
+    return clamp_idx(on ? s : 0, a.num_rows);
+  }
+}
+
+template <int BITS, bool AFFINE, typename ROWS = void>
 __global__ __launch_bounds__(kBlock) void sq_decode_f4_kernel(F4Args a) {
   constexpr int NCODE = 1 << BITS;
   constexpr uint32_t MASK = NCODE - 1;
@@ -264,7 +289,7 @@ __global__ __launch_bounds__(kBlock) void sq_decode_f4_kernel(F4Args a) {
     const uint32_t rl = __umulhi(li, a.magic);
     const uint32_t c4 = li - rl * a.f4_per_row;
     const bool on = base + threadIdx.x + k * kBlock < a.total_f4;
-    const uint8_t* src = a.codes + (on ? (rb + rl) * a.src_dim : 0);
+    const uint8_t* src = a.codes + (on ? table_row<ROWS>(a, rb + rl) * a.src_dim : 0);
     c4s[k] = c4;
     if (BITS == 8) {
       uint32_t w; __builtin_memcpy(&w, src + (on ? 4 * c4 : 0), 4); word[k] = w;
@@ -307,7 +332,7 @@ __global__ __launch_bounds__(kBlock) void sq_decode_f4_kernel(F4Args a) {
 // a nibble, two bits), the per-column tables from LDS, and one aligned 16-byte store, so that the stores of a
 // workgroup are as dense as for rows of whole float4 groups (4e5 rows of 602 columns, 4 bit: 253 us with a group of
 // four columns per lane and stores that start 8 bytes off, 176 us at 600 columns).
-template <int BITS, bool AFFINE>
+template <int BITS, bool AFFINE, typename ROWS = void>
 __global__ __launch_bounds__(kBlock) void sq_decode_pairs_kernel(F4Args a) {
   constexpr int NCODE = 1 << BITS;
   constexpr uint32_t MASK = NCODE - 1;
@@ -342,7 +367,7 @@ __global__ __launch_bounds__(kBlock) void sq_decode_pairs_kernel(F4Args a) {
     const uint32_t li = l0 + (uint32_t)(p - 2 * base);
     const uint32_t rl = __umulhi(li, a.magic);
     const uint32_t cp = li - rl * ppr;
-    const uint8_t* src = a.codes + (rb + rl) * a.src_dim;
+    const uint8_t* src = a.codes + table_row<ROWS>(a, rb + rl) * a.src_dim;
     uint32_t c0, c1;
     if (BITS == 8) {
       uint16_t w; __builtin_memcpy(&w, src + 2 * cp, 2);
@@ -389,13 +414,14 @@ __global__ __launch_bounds__(kBlock) void sq_decode_pairs_kernel(F4Args a) {
 template <int BITS, bool AFFINE>
 int decode_f4_launch(const uint8_t* codes, float* out, const float* table, int64_t param_stride,
                      int64_t column_slice, int n_cb, int64_t rows, int64_t src_dim, int64_t feat_dim,
-                     hipStream_t st, const char* what) {
+                     hipStream_t st, const char* what, const F4Args* ids = nullptr, int idx_dtype = 0) {
   // (one float4 per row would need the reciprocal 2^32, which does not fit the 32-bit multiplier)
   if (feat_dim % 2 != 0 || feat_dim < 8 || feat_dim > 8192 || !aligned(out, 16)) return -1;
   const size_t lds = AFFINE ? (size_t)feat_dim * 8
                             : ((((size_t)n_cb << BITS) + 3) / 4 * 4 + (size_t)feat_dim) * 4;
   if (lds > (size_t)kMaxLutBytes) return -1;
   F4Args a{};
+  if (ids != nullptr) a = *ids;
   a.codes = codes; a.out = out; a.table = table;
   a.param_stride = param_stride; a.column_slice = column_slice; a.n_cb = AFFINE ? 0 : n_cb;
   a.src_dim = src_dim;
@@ -409,6 +435,15 @@ int decode_f4_launch(const uint8_t* codes, float* out, const float* table, int64
   const int64_t lanes = pairs ? a.total_f4 / 2 + 1 : a.total_f4;
   const int64_t grid = ceil_div(lanes, kF4Items * kBlock);
   if (grid > 0x7fffffffll) return -1;
+  if constexpr (!AFFINE) {
+    if (ids != nullptr) {
+      void (*kern)(F4Args);
+      if (idx_dtype == F2CGT_DT_I64) kern = pairs ? sq_decode_pairs_kernel<BITS, false, int64_t> : sq_decode_f4_kernel<BITS, false, int64_t>;
+      else kern = pairs ? sq_decode_pairs_kernel<BITS, false, int32_t> : sq_decode_f4_kernel<BITS, false, int32_t>;
+      kern<<<(unsigned)grid, kBlock, lds, st>>>(a);
+      return launch_status(what);
+    }
+  }
   if (pairs) sq_decode_pairs_kernel<BITS, AFFINE><<<(unsigned)grid, kBlock, lds, st>>>(a);
   else sq_decode_f4_kernel<BITS, AFFINE><<<(unsigned)grid, kBlock, lds, st>>>(a);
   return launch_status(what);
@@ -771,4 +806,40 @@ extern "C" int f2cgt_sq_affine_decompress(const uint8_t* codes, float* out, cons
   switch (target_bits) { F2CGT_CASE(1) F2CGT_CASE(2) F2CGT_CASE(4) F2CGT_CASE(8) }
 #undef F2CGT_CASE
   return launch_status("sq_affine_decompress");
+}
+
+extern "C" int f2cgt_sq_decompress_rows(const void* table, int code_dtype, const void* index, int idx_dtype,
+                                        const int32_t* slot_map, int64_t num_slots, int32_t* bad, const float* codebooks,
+                                        float* out, int64_t num_index, int64_t num_rows, int64_t src_dim, int64_t feat_dim,
+                                        int64_t num_codebooks, int target_bits, int64_t column_slice, void* stream) {
+  const char* what = "sq_decompress_rows";
+  F2CGT_REQUIRE(num_index >= 0 && num_rows >= 0 && src_dim >= 0 && feat_dim >= 0 && num_slots >= 0, F2CGT_E_INVALID,
+                "%s: negative size", what);
+  F2CGT_REQUIRE(column_slice > 0 && num_codebooks > 0 && num_codebooks < (1 << 20) && num_codebooks * column_slice >= feat_dim,
+                F2CGT_E_INVALID, "%s: the codebooks do not cover feat_dim", what);
+  F2CGT_REQUIRE(target_bits == 1 || target_bits == 2 || target_bits == 4 || target_bits == 8, F2CGT_E_UNSUPPORTED,
+                "%s: target_bits must be 1, 2, 4 or 8 (got %d)", what, target_bits);
+  F2CGT_REQUIRE(code_dtype == F2CGT_DT_I8 || (code_dtype == F2CGT_DT_U8 && target_bits != 8), F2CGT_E_UNSUPPORTED,
+                "%s: codes must be int8, or uint8 below 8 bits", what);
+  F2CGT_REQUIRE(src_dim * (8 / target_bits) >= feat_dim, F2CGT_E_INVALID, "%s: rows too short for feat_dim", what);
+  F2CGT_REQUIRE(idx_dtype == F2CGT_DT_I32 || idx_dtype == F2CGT_DT_I64, F2CGT_E_UNSUPPORTED, "%s: index must be int32 or int64", what);
+  if (num_index * feat_dim == 0) return 0;
+  F2CGT_REQUIRE(num_rows > 0 && (slot_map == nullptr || num_slots > 0), F2CGT_E_INVALID, "%s: rows requested from an empty table", what);
+  F2CGT_REQUIRE(table && index && out && codebooks, F2CGT_E_INVALID, "%s: null buffer", what);
+  F4Args ids{};
+  ids.index = index; ids.slot = slot_map; ids.num_rows = num_rows; ids.num_slots = num_slots; ids.bad = bad;
+  const uint8_t* codes = static_cast<const uint8_t*>(table);
+  const int n_cb = (int)num_codebooks;
+  hipStream_t st = as_stream(stream);
+  int rc = -1;
+  if ((int64_t)n_cb * (1 << target_bits) * 4 <= kMaxLutBytes) {
+    switch (target_bits) {
+      case 1: rc = decode_f4_launch<1, false>(codes, out, codebooks, 0, column_slice, n_cb, num_index, src_dim, feat_dim, st, what, &ids, idx_dtype); break;
+      case 2: rc = decode_f4_launch<2, false>(codes, out, codebooks, 0, column_slice, n_cb, num_index, src_dim, feat_dim, st, what, &ids, idx_dtype); break;
+      case 4: rc = decode_f4_launch<4, false>(codes, out, codebooks, 0, column_slice, n_cb, num_index, src_dim, feat_dim, st, what, &ids, idx_dtype); break;
+      default: rc = decode_f4_launch<8, false>(codes, out, codebooks, 0, column_slice, n_cb, num_index, src_dim, feat_dim, st, what, &ids, idx_dtype); break;
+    }
+  }
+  F2CGT_REQUIRE(rc >= 0, F2CGT_E_UNSUPPORTED, "%s: this shape is left to fetch_rows and sq_decompress", what);
+  return rc;
 }

@@ -5,6 +5,8 @@
 // read through L1/L2.
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace f2cgt {
 namespace {
 
@@ -66,13 +68,19 @@ struct VqTileArgs {
   int64_t rows;
   int feat_dim, n_cb, K, w;
   int n_tiles, n_stripes;
+  const void* index;     // ROWS: row index[r] of a table of num_rows code rows instead of row r (ids are held to the table)
+  int64_t num_rows;
 };
 
+// ROWS (int32_t or int64_t ids, void without): the ids are read two steps ahead, the code bytes they name one, so that the
+// rows need not be copied first.  200 000 rows of 8 codes, 128 columns, of a 2.4e6-row table: fetched and decoded 8.8 +
+// 22.1 us, 26.3 here.
 // HALF: rows of 4 k + 2 columns.  Output rows start at multiples of 8 bytes only, which a 16-byte store takes at any
 // dword; the row's last column group holds two columns and stores them alone (the tile is staged up to the next
 // multiple of four: the codebooks hold those columns, n_cb * w being a multiple of four that is at least feat_dim).
-template <bool HALF>
+template <bool HALF, typename ROWS>
 __global__ __launch_bounds__(kTileThreads) void vq_decompress_tile_kernel(VqTileArgs a) {
+  constexpr bool kRows = !std::is_void<ROWS>::value;
   extern __shared__ __align__(16) float s_cb[];
   const int tile = blockIdx.x % a.n_tiles;
   const int stripe = blockIdx.x / a.n_tiles;
@@ -99,17 +107,32 @@ __global__ __launch_bounds__(kTileThreads) void vq_decompress_tile_kernel(VqTile
   const int64_t steps = a.rows / kTileRows;   // full steps
   const uint32_t kmax = (uint32_t)a.K - 1u;
 
+  auto row_of = [&](int64_t r) -> int64_t {
+    if constexpr (kRows) return clamp_idx(static_cast<const ROWS*>(a.index)[r], a.num_rows);
+    else return r;
+  };
   uint32_t code[8];
+  int64_t ahead[kRows ? 8 : 1];          // rows of the next step
   int64_t s = stripe;
   if (s < steps) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) code[u] = cp[(s * kTileRows + rs + 32 * u) * a.n_cb];
+    for (int u = 0; u < 8; ++u) code[u] = cp[row_of(s * kTileRows + rs + 32 * u) * a.n_cb];
+    if constexpr (kRows) {
+      const int64_t sn = s + a.n_stripes < steps ? s + a.n_stripes : s;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) ahead[u] = row_of(sn * kTileRows + rs + 32 * u);
+    }
   }
   for (; s < steps; s += a.n_stripes) {
     const int64_t sn = s + a.n_stripes < steps ? s + a.n_stripes : s;  // last step reloads itself
     uint32_t next[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) next[u] = cp[(sn * kTileRows + rs + 32 * u) * a.n_cb];
+    for (int u = 0; u < 8; ++u) next[u] = cp[(kRows ? ahead[kRows ? u : 0] : sn * kTileRows + rs + 32 * u) * a.n_cb];
+    if constexpr (kRows) {
+      const int64_t sm = sn + a.n_stripes < steps ? sn + a.n_stripes : sn;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) ahead[u] = row_of(sm * kTileRows + rs + 32 * u);
+    }
     float4 x[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -125,7 +148,7 @@ __global__ __launch_bounds__(kTileThreads) void vq_decompress_tile_kernel(VqTile
   // the rows after the last full step, one stripe
   if (stripe == (int)(steps % a.n_stripes)) {
     for (int64_t r = steps * kTileRows + rs; r < a.rows; r += 32) {
-      uint32_t c = cp[r * a.n_cb];
+      uint32_t c = cp[row_of(r) * a.n_cb];
       c = c < kmax ? c : kmax;
       const float4 x = *reinterpret_cast<const float4*>(cbp + c * 128);
       store(op + r * (int64_t)a.feat_dim, x);
@@ -135,22 +158,24 @@ __global__ __launch_bounds__(kTileThreads) void vq_decompress_tile_kernel(VqTile
 
 // Returns -1 when the shape is not covered.
 int launch_tile(const uint8_t* codes, const float* codebooks, float* out, int64_t rows, int64_t feat_dim,
-                int n_cb, int K, int w, hipStream_t st) {
+                int n_cb, int K, int w, hipStream_t st, const void* index = nullptr, int idx_dtype = 0,
+                int64_t num_rows = 0) {
   if (K > 256 || w < 4 || 128 % w != 0 || feat_dim % 2 != 0 || feat_dim < 64) return -1;
   if (!aligned(out, 16) || rows < 4 * kTileRows) return -1;
-  VqTileArgs a{codes, codebooks, out, rows, (int)feat_dim, n_cb, K, w, 0, 0};
+  VqTileArgs a{codes, codebooks, out, rows, (int)feat_dim, n_cb, K, w, 0, 0, index, num_rows};
   a.n_tiles = (int)ceil_div(feat_dim, 128);
   const int cus = num_cus();
   if (a.n_tiles > cus) return -1;
   a.n_stripes = cus / a.n_tiles;
   const size_t lds = (size_t)K * 128 * 4;
   const bool half = feat_dim % 4 != 0;
-  hipError_t e = hipFuncSetAttribute(half ? reinterpret_cast<const void*>(vq_decompress_tile_kernel<true>)
-                                          : reinterpret_cast<const void*>(vq_decompress_tile_kernel<false>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  void (*kern)(VqTileArgs);
+  if (index == nullptr) kern = half ? vq_decompress_tile_kernel<true, void> : vq_decompress_tile_kernel<false, void>;
+  else if (idx_dtype == F2CGT_DT_I64) kern = half ? vq_decompress_tile_kernel<true, int64_t> : vq_decompress_tile_kernel<false, int64_t>;
+  else kern = half ? vq_decompress_tile_kernel<true, int32_t> : vq_decompress_tile_kernel<false, int32_t>;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return fail((int)e, "vq_decompress: cannot reserve %zu B of LDS", lds);
-  if (half) vq_decompress_tile_kernel<true><<<(unsigned)(a.n_stripes * a.n_tiles), kTileThreads, lds, st>>>(a);
-  else vq_decompress_tile_kernel<false><<<(unsigned)(a.n_stripes * a.n_tiles), kTileThreads, lds, st>>>(a);
+  kern<<<(unsigned)(a.n_stripes * a.n_tiles), kTileThreads, lds, st>>>(a);
   return launch_status("vq_decompress");
 }
 
@@ -228,4 +253,22 @@ extern "C" int f2cgt_vq_decompress(const void* codes, int code_dtype, const void
     default:
       return fail(F2CGT_E_UNSUPPORTED, "vq_decompress: codes must be uint8, int8 or int16");
   }
+}
+
+extern "C" int f2cgt_vq_decompress_rows(const uint8_t* table, const void* index, int idx_dtype, const float* codebooks, float* out,
+                                        int64_t num_index, int64_t num_rows, int64_t feat_dim, int64_t num_codebooks, int64_t K,
+                                        int64_t width, void* stream) {
+  const char* what = "vq_decompress_rows";
+  F2CGT_REQUIRE(num_index >= 0 && num_rows >= 0 && feat_dim >= 0, F2CGT_E_INVALID, "%s: negative size", what);
+  F2CGT_REQUIRE(num_codebooks > 0 && K > 0 && width > 0 && feat_dim <= num_codebooks * width &&
+                    num_codebooks * K * width < (1ll << 31) && feat_dim < (1ll << 31),
+                F2CGT_E_INVALID, "%s: codebooks must be [n>0, K>0, w>0] and cover feat_dim", what);
+  F2CGT_REQUIRE(idx_dtype == F2CGT_DT_I32 || idx_dtype == F2CGT_DT_I64, F2CGT_E_UNSUPPORTED, "%s: index must be int32 or int64", what);
+  if (num_index * feat_dim == 0) return 0;
+  F2CGT_REQUIRE(num_rows > 0, F2CGT_E_INVALID, "%s: rows requested from an empty table", what);
+  F2CGT_REQUIRE(table && index && out && codebooks, F2CGT_E_INVALID, "%s: null buffer", what);
+  const int rc = launch_tile(table, codebooks, out, num_index, feat_dim, (int)num_codebooks, (int)K, (int)width,
+                             as_stream(stream), index, idx_dtype, num_rows);
+  F2CGT_REQUIRE(rc >= 0, F2CGT_E_UNSUPPORTED, "%s: this shape is left to fetch_rows and vq_decompress", what);
+  return rc;
 }

@@ -561,6 +561,19 @@ class CompressionManager:
         return capi.sq_decompress(data, self.codebooks[level], self.configs[level][1], self.configs[level][0],
                                   self.feat_dim)
 
+    def _decode_rows(self, level, cache, keys):
+        """Decoded rows `keys` of a code table: read by the decoder itself where the whole table is in device memory,
+        fetched and decoded otherwise."""
+        if not cache.data.is_cuda or cache.has_cache:
+            return self._decompress(level, cache[keys])
+        capi = _capi()
+        if keys.dtype not in (torch.int32, torch.int64):
+            keys = keys.long()
+        if self.methods[level] == "vq":
+            return capi.vq_decompress_rows(cache.data, keys, self.codebooks[level], self.feat_dim)
+        return capi.sq_decompress_rows(cache.data, keys, self.codebooks[level], self.configs[level][1],
+                                       self.configs[level][0], self.feat_dim)
+
     def get_seeds_data(self, seeds_key):
         """Decoded first-level rows of `seeds_key`, produced on `seeds_task_stream`; the result may be
         used on another stream only after `seeds_task_event` (reorganize_seeds_data waits for it)."""
@@ -571,6 +584,14 @@ class CompressionManager:
         with torch.cuda.stream(side):
             # the caller may drop seeds_key as soon as this returns: tie its memory to the side stream
             seeds_key.record_stream(side)
+            seeds = self.seeds_data
+            if self.methods[0] == "sq" and seeds.data.is_cuda and not seeds.has_cache and seeds_key.dtype in (torch.int32, torch.int64):
+                # lookup, check, fetch and decode in one kernel
+                seeds_feature = _capi().sq_decompress_rows(seeds.data, seeds_key, self.codebooks[0], self.configs[0][1],
+                                                           self.configs[0][0], self.feat_dim, self.seed_slot,
+                                                           self.check_seed_keys)
+                self.seeds_task_event.record(side)
+                return seeds_feature
             slots = self.seed_slot[seeds_key.long()].long()
             if self.check_seed_keys and bool((slots < 0).any()):
                 raise KeyError("a requested id is not a seed row")
@@ -579,10 +600,9 @@ class CompressionManager:
         return seeds_feature
 
     def get_all_data(self, keys):
-        data = self.data[keys]
         if self.is_fusion:
-            return data
-        return self._decompress(1 if self.is_two_level else 0, data)
+            return self.data[keys]
+        return self._decode_rows(1 if self.is_two_level else 0, self.data, keys)
 
     def aggregate_global(self, indptr, indices, input_nodes):
         """Mean aggregation of a sampled block straight from the device-resident code table:

@@ -224,6 +224,23 @@ int f2cgt_fetch_rows(const void* table, const void* hot, const int32_t* slot_map
                      const void* index, int idx_dtype, void* out, int64_t num_index,
                      int64_t row_bytes, int64_t num_rows, int64_t num_hot_rows, void* stream);
 
+/* Decode through a row list: out[i] = the decoded row index[i] of a table in device memory, as f2cgt_fetch_rows followed
+ * by f2cgt_vq_decompress / f2cgt_sq_decompress, without the copy of the code rows.  F2CGT_E_UNSUPPORTED, with nothing
+ * launched, for the shapes left to those (the caller falls back).
+ * f2cgt_vq_decompress_rows: uint8 codes [num_rows, num_codebooks], fp32 codebooks; widths that divide 128 (4 and more),
+ * K <= 256, even feat_dim >= 64, at least 1024 rows, out 16-byte aligned.
+ * f2cgt_sq_decompress_rows: 1, 2, 4 or 8-bit codes, even feat_dim from 8 to 8192, out 16-byte aligned, the decode table
+ * in LDS.  slot_map (int32 [num_slots], may be NULL): row slot_map[index[i]] instead; an id below zero counts from the end
+ * of the map.  bad (int32, device-accessible host memory, may be NULL; zero on entry): 1 when the map has no row
+ * (a negative entry) for an id, 2 when an id lies outside it; such rows are decoded from some row of the table. */
+int f2cgt_vq_decompress_rows(const uint8_t* table, const void* index, int idx_dtype, const float* codebooks, float* out,
+                             int64_t num_index, int64_t num_rows, int64_t feat_dim, int64_t num_codebooks, int64_t K,
+                             int64_t width, void* stream);
+int f2cgt_sq_decompress_rows(const void* table, int code_dtype, const void* index, int idx_dtype, const int32_t* slot_map,
+                             int64_t num_slots, int32_t* bad, const float* codebooks, float* out, int64_t num_index,
+                             int64_t num_rows, int64_t src_dim, int64_t feat_dim, int64_t num_codebooks, int target_bits,
+                             int64_t column_slice, void* stream);
+
 /* ---- codebook statistics ------------------------------------------------------- */
 
 /* The statistics behind an SQ codebook (examples/process_compress.py:45-68), of the absolute values of every column
