@@ -10,11 +10,15 @@
 // and third pass), and no counter is shared between workgroups: the hot bins of a normal distribution lie in a dozen
 // cache lines, on which device-wide atomics of 256 workgroups would queue up.
 //
-// What bounds it: the three reads of the sample (17 us each at 120 000 x 100 values, 2.9 TB/s through the row list; the
-// sums between them 3-4 us each).  The seven launches take 66 us where the host took 195 ms on a copy of the sample
-// (np.percentile, two selections).  The codebook is made by the last of them, so that the encoder can follow at once: the
-// whole sq_compress call took 130 us with a read-back, the host's arithmetic and an upload in between (195-228 ms with the
-// host's percentiles), now 105, of which the encoder is 15 and the read-back of the flags at the end about 20.
+// What bounds it: two reads of the sample (17 us each at 120 000 x 100 values, 2.9 TB/s through the row list; the first is
+// as long on its LDS counters as on its loads), the sums between the passes (4 us each) and the third pass, which reads
+// what the second kept and takes 5 us (17 with the sample read again).  The seven launches take 56 us, with eight rows and
+// the next eight ids in flight per thread, where four rows without the ids of the next took 66 and the host took 195 ms
+// on a copy of the sample (np.percentile, two selections).  The codebook is made by the last of them, so that the encoder
+// can follow at once: the whole sq_compress call takes 90 us (130 with the codebook made on the host, 102 with three
+// reads), of which the encoder is 15 and the read-back of the flags at the end about 20.  100 000 x 602 values 598 -> 445;
+// tables on which a workgroup has to read its rows again are no slower than before (all values equal 438 -> 412, 80 %
+// zeros 253 -> 219).
 #include "common.hpp"
 
 namespace f2cgt {
@@ -24,6 +28,9 @@ constexpr int kStatThreads = 1024;
 constexpr int kBins = 4096;          // counters of a pass: 4096, 4 x 1024 or 4 x 512
 constexpr int kReplicas = 4;         // copies of the first pass's counters in LDS, by lane: its hot bins are few
 constexpr int kMaxBlocks = 256;      // workgroups per pass over all slices (one per CU)
+constexpr int kStatWaves = kStatThreads / kWave;
+constexpr int kKept = 512;           // values a wave of the second pass can hand to the third
+constexpr int kKeepBlocks = 1024;    // more workgroups than that in all hand over none (32 KB of workspace each)
 
 constexpr uint32_t kSawNan = 1u, kSawBadRow = 2u;   // a NaN among the values; a row id outside the table
 
@@ -45,6 +52,9 @@ struct StatArgs {
   StatState* state;                  // [2][n_slices]: after the first and the second digit
   double* sums;                      // [n_slices][blocks]
   uint32_t* flags;                   // [n_slices][blocks]: kSawNan, kSawBadRow
+  int keep;                          // kKept, or 0 where there is no room for them
+  uint32_t* kept;                    // [n_slices][blocks][kStatWaves][keep]: values that share the first digit of a wanted rank
+  uint32_t* n_kept;                  // [n_slices][blocks][kStatWaves]: how many; more than `keep`: not all of them are there
   double* out;                       // [n_slices][6]
   float* books;                      // [n_slices][5], or null
   float weights[4];                  // lower and upper percentile of a slice, and of the last one: where between its ranks
@@ -124,8 +134,12 @@ __device__ __forceinline__ void known_digits(const StatArgs& a, int slice, uint6
   for (int k = 0; k < 4; ++k) rank[k] = s_rest[k];
 }
 
-// One pass over the sample.  A thread keeps its place in the row (a V-wide column group) and walks rows; four rows are in
-// flight at a time.
+// One pass over the sample.  A thread keeps its place in the row (a V-wide column group) and walks rows; eight rows are in
+// flight at a time, and the ids of the eight after them.
+//
+// The second pass meets all the values that the third will count, those that share the first digit of a wanted rank: one in
+// a few hundred of a feature table.  Its waves keep them, and the third pass reads these instead of the sample.  A
+// workgroup with a wave that met more than `keep` of them (a table of few different values) reads its rows again.
 template <int PASS, int V>
 __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   __shared__ __align__(16) uint32_t s_hist[PASS == 0 ? kBins * kReplicas : kBins];
@@ -134,14 +148,19 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   __shared__ uint64_t s_rest[4];
   __shared__ double s_sum[kStatThreads / kWave];
   __shared__ uint32_t s_flags;
-  const int t = threadIdx.x, slice = blockIdx.y;
+  __shared__ uint32_t s_kept[PASS == 1 ? kStatWaves * kKept : 1];
+  __shared__ uint32_t s_n_kept[kStatWaves];
+  const int t = threadIdx.x, slice = blockIdx.y, wave = t / kWave;
   constexpr int LDS_BINS = PASS == 0 ? kBins * kReplicas : kBins;
   for (int i = t; i < LDS_BINS / 4; i += kStatThreads) reinterpret_cast<uint4*>(s_hist)[i] = make_uint4(0u, 0u, 0u, 0u);
   if (t == 0) s_flags = 0u;
+  if (t < kStatWaves) s_n_kept[t] = 0u;
   uint32_t prefix[4] = {0u, 0u, 0u, 0u};
   if constexpr (PASS > 0) {
     uint64_t rank[4];
     known_digits<PASS>(a, slice, s_scan, s_digit, s_rest, prefix, rank);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) prefix[k] = __builtin_amdgcn_readfirstlane(prefix[k]);
     if (blockIdx.x == 0 && t == 0) {
       StatState& st = a.state[(PASS - 1) * a.n_slices + slice];
 #pragma unroll
@@ -166,43 +185,75 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
       flags |= mag > 0x7f800000u ? kSawNan : 0u;
       atomicAdd(&s_hist[(mag >> 19) * kReplicas + (t & (kReplicas - 1))], 1u);
     } else if constexpr (PASS == 1) {
+      const uint32_t digit = mag >> 19;
+      if ((digit == prefix[0]) | (digit == prefix[1]) | (digit == prefix[2]) | (digit == prefix[3])) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if ((mag >> 19) == prefix[k]) atomicAdd(&s_hist[k * 1024 + ((mag >> 9) & 1023u)], 1u);
+        for (int k = 0; k < 4; ++k)
+          if (digit == prefix[k]) atomicAdd(&s_hist[k * 1024 + ((mag >> 9) & 1023u)], 1u);
+        // a place for every lane that is here, by one addition for the wave
+        const uint64_t all = __ballot(true);
+        const uint32_t before = __popcll(all & ((1ull << (t & (kWave - 1))) - 1));
+        uint32_t at = before == 0 ? atomicAdd(&s_n_kept[wave], (uint32_t)__popcll(all)) : 0u;
+        at = __builtin_amdgcn_readfirstlane(at) + before;
+        if (at < (uint32_t)a.keep) s_kept[wave * kKept + at] = mag;
+      }
     } else {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
         if ((mag >> 9) == prefix[k]) atomicAdd(&s_hist[k * 512 + (mag & 511u)], 1u);
     }
   };
-  if (r0 < rpp) {
-    constexpr int U = 4;
-    for (int64_t r = (int64_t)blockIdx.x * rpp + r0; r < a.m; r += step * U) {
-      int64_t id[U];
+  const int64_t place = (int64_t)slice * a.blocks + blockIdx.x;
+  bool read_rows = true;
+  if constexpr (PASS == 2) {
+    uint32_t most = 0;
+#pragma unroll
+    for (int w = 0; w < kStatWaves; ++w) {
+      const uint32_t n = a.n_kept[place * kStatWaves + w];
+      most = n > most ? n : most;
+    }
+    if (most <= (uint32_t)a.keep) {
+      read_rows = false;
+      const uint32_t n = a.n_kept[place * kStatWaves + wave];
+      const uint32_t* kept = a.kept + (place * kStatWaves + wave) * a.keep;
+      for (uint32_t i = t & (kWave - 1); i < n; i += kWave) take(__uint_as_float(kept[i]));
+    }
+  }
+  if (read_rows && r0 < rpp) {
+    constexpr int U = 8;
+    int64_t id[U];
+    // the rows r, r + step, ...: a place beyond the sample takes row r again, which the sample has
+    auto row_ids = [&](int64_t r, int64_t (&id)[U]) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int64_t ru = r + u * step < a.m ? r + u * step : r;
-        id[u] = ru;
-        if (a.rows != nullptr) {
-          int64_t want = a.rows[ru];
-          want = want < 0 ? want + a.num_rows : want;
-          id[u] = clamp_idx(want, a.num_rows);
-          if (PASS == 0) flags |= id[u] != want ? kSawBadRow : 0u;
-        }
+        id[u] = a.rows != nullptr ? a.rows[ru] : ru;
       }
+    };
+    const int64_t first = (int64_t)blockIdx.x * rpp + r0;
+    if (first < a.m) row_ids(first, id);
+    for (int64_t r = first; r < a.m; r += step * U) {
+      const float* p[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t want = id[u] < 0 ? id[u] + a.num_rows : id[u];
+        const int64_t at = clamp_idx(want, a.num_rows);
+        if (PASS == 0) flags |= at != want ? kSawBadRow : 0u;
+        p[u] = a.x + at * a.ld + col0;
+      }
+      if (r + step * U < a.m) row_ids(r + step * U, id);
       for (int c = c0; c < groups; c += cg) {
         float v[U][V];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const float* p = a.x + id[u] * a.ld + col0 + c * V;
           if constexpr (V == 4) {
-            const float4 q = *reinterpret_cast<const float4*>(p);
+            const float4 q = *reinterpret_cast<const float4*>(p[u] + c * V);
             v[u][0] = q.x; v[u][1] = q.y; v[u][2] = q.z; v[u][3] = q.w;
           } else if constexpr (V == 2) {
-            const float2 q = *reinterpret_cast<const float2*>(p);
+            const float2 q = *reinterpret_cast<const float2*>(p[u] + c * V);
             v[u][0] = q.x; v[u][1] = q.y;
           } else {
-            v[u][0] = *p;
+            v[u][0] = p[u][c];
           }
         }
 #pragma unroll
@@ -221,7 +272,13 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
     if ((t & (kWave - 1)) == 0) s_sum[t / kWave] = sum;
   }
   __syncthreads();
-  uint32_t* dst = a.partial + ((int64_t)slice * a.blocks + blockIdx.x) * kBins;
+  if constexpr (PASS == 1) {
+    const uint32_t n = s_n_kept[wave];
+    if ((t & (kWave - 1)) == 0) a.n_kept[place * kStatWaves + wave] = n;
+    uint32_t* kept = a.kept + (place * kStatWaves + wave) * a.keep;
+    for (uint32_t i = t & (kWave - 1); i < (n < (uint32_t)a.keep ? n : (uint32_t)a.keep); i += kWave) kept[i] = s_kept[wave * kKept + i];
+  }
+  uint32_t* dst = a.partial + place * kBins;
   for (int i = t; i < (PASS == 2 ? 2048 : kBins); i += kStatThreads) {
     if constexpr (PASS == 0) {
       uint32_t c = 0;
@@ -235,8 +292,8 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   if (PASS == 0 && t == 0) {
     double total = 0.0;
     for (int w = 0; w < kStatThreads / kWave; ++w) total += s_sum[w];
-    a.sums[(int64_t)slice * a.blocks + blockIdx.x] = total;
-    a.flags[(int64_t)slice * a.blocks + blockIdx.x] = s_flags;
+    a.sums[place] = total;
+    a.flags[place] = s_flags;
   }
 }
 
@@ -329,14 +386,18 @@ int stat_blocks(int64_t m, int64_t cols, int64_t slice, int64_t n_slices) {
 
 int64_t round256(int64_t v) { return (v + 255) / 256 * 256; }
 
-struct StatLayout { int64_t hist, state, sums, flags, total; };
+int stat_keep(int64_t blocks, int64_t n_slices) { return n_slices * blocks <= kKeepBlocks ? kKept : 0; }
+
+struct StatLayout { int64_t hist, state, sums, flags, kept, n_kept, total; };
 StatLayout stat_layout(int64_t blocks, int64_t n_slices) {
   StatLayout l;
   l.hist = round256(n_slices * blocks * kBins * 4);
   l.state = l.hist + round256(n_slices * kBins * 4);
   l.sums = l.state + round256(2 * n_slices * (int64_t)sizeof(StatState));
   l.flags = l.sums + round256(n_slices * blocks * 8);
-  l.total = l.flags + round256(n_slices * blocks * 4);
+  l.kept = l.flags + round256(n_slices * blocks * 4);
+  l.n_kept = l.kept + round256(n_slices * blocks * kStatWaves * stat_keep(blocks, n_slices) * 4);
+  l.total = l.n_kept + round256(n_slices * blocks * kStatWaves * 4);
   return l;
 }
 
@@ -400,6 +461,9 @@ int order_stats(const char* what, const float* x, int64_t ld, const int64_t* row
   a.state = reinterpret_cast<StatState*>(ws + l.state);
   a.sums = reinterpret_cast<double*>(ws + l.sums);
   a.flags = reinterpret_cast<uint32_t*>(ws + l.flags);
+  a.keep = stat_keep(a.blocks, n_slices);
+  a.kept = reinterpret_cast<uint32_t*>(ws + l.kept);
+  a.n_kept = reinterpret_cast<uint32_t*>(ws + l.n_kept);
   a.out = out;
   a.books = books;
   if (books != nullptr)

@@ -25,7 +25,10 @@ def _values(kind, rng, n, d):
 # more slices than workgroups per slice; enough rows for every workgroup and an odd remainder
 @pytest.mark.parametrize("kind", ["normal", "equal", "bits", "sparse"])
 @pytest.mark.parametrize("n,d,slice_", [(1, 1, 1), (3, 1500, 1500), (4097, 20, 8), (5000, 7, 7), (2049, 30, 30),
-                                        (700, 602, 8), (40001, 100, 104), (1023, 4100, 4100)])
+                                        (700, 602, 8), (40001, 100, 104), (1023, 4100, 4100),
+                                        # what a wave hands from the second pass to the third: one value less than fits,
+                                        # exactly that many, one more; more workgroups than hand anything on
+                                        (8191, 1, 1), (8192, 1, 1), (8193, 1, 1), (300, 2100, 2), (300, 2100, 8)])
 def test_ranks_sum_and_flag(kind, n, d, slice_):
     rng = np.random.default_rng(n + d)
     table = _values(kind, rng, n + 50, d)
