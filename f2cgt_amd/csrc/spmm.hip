@@ -115,6 +115,56 @@ __global__ __launch_bounds__(kMaxBlock) void agg_kernel(Dec dec, const Idx* __re
   }
 }
 
+// Uncompressed rows in groups of eight lanes and more.  A row costs three dependent round trips, row bounds, ids, source
+// rows, and nothing but them: what bounds it is how many source bytes are in flight.  The lanes of a group fetch the ids of
+// up to G edges with one load and hand them round by lane shuffles, and eight source rows are in flight at a time (the
+// skeleton above fetches four ids, waits, fetches four source rows, waits).  Columns beyond a group's width go to further
+// workgroups (blockIdx.x), not to further walks over the rows.  Sums in edge order, as above.  30 000 rows of up to 15
+// edges over 200 000 x 128 decoded rows that the cache still holds (115 MB read, 15 MB written): 27.3 -> 22.5 us, 5.8 TB/s.
+constexpr int kPlainUnroll = 8;
+
+template <class Dec, typename Idx>
+__global__ __launch_bounds__(256) void agg_plain_kernel(Dec dec, const Idx* __restrict__ indptr,
+                                                        const Idx* __restrict__ indices,
+                                                        typename Dec::Out* __restrict__ out, int64_t R, int64_t E,
+                                                        int64_t N, int feat_dim, int G, bool vec_ok) {
+  constexpr int NOUT = Dec::NOUT;
+  using Acc = typename Dec::Acc;
+  const int lane = threadIdx.x & (G - 1);
+  const int gpb = 256 / G;
+  const int64_t col = ((int64_t)blockIdx.x * G + lane) * NOUT;
+  const bool mine = col < feat_dim;                  // a lane beyond the columns only carries ids
+  const int col0 = mine ? (int)col : 0;
+  const typename Dec::Ctx ctx = dec.column_setup(col0);
+  const int nvalid = (feat_dim - col0) < NOUT ? (feat_dim - col0) : NOUT;
+  for (int64_t r = (int64_t)blockIdx.y * gpb + threadIdx.x / G; r < R; r += (int64_t)gridDim.y * gpb) {
+    int64_t b, e;
+    row_range(indptr, r, E, b, e);
+    const Acc deg = (Acc)(float)((e - b) == 0 ? 1 : (e - b));
+    Acc acc[NOUT];
+#pragma unroll
+    for (int i = 0; i < NOUT; ++i) acc[i] = (Acc)0;
+    for (int64_t k = b; k < e; k += G) {
+      const int n = (e - k) < G ? (int)(e - k) : G;
+      const int64_t own = lane < n ? clamp_idx(indices[k + lane], N) : 0;
+      for (int u0 = 0; u0 < n; u0 += kPlainUnroll) {  // G is a multiple of kPlainUnroll: every shuffle stays in the group
+        typename Dec::Raw raw[kPlainUnroll];
+#pragma unroll
+        for (int u = 0; u < kPlainUnroll; ++u) {
+          const int64_t s = __shfl(own, u0 + u, G);
+          if (mine && u0 + u < n) raw[u] = dec.load(ctx, s);
+        }
+#pragma unroll
+        for (int u = 0; u < kPlainUnroll; ++u)
+          if (mine && u0 + u < n) dec.accum(ctx, raw[u], acc);
+      }
+    }
+    if (mine)
+      store_mean<NOUT, Acc, typename Dec::Out, dec_align8<Dec>::value>(out + r * (int64_t)feat_dim + col0, acc, deg, nvalid,
+                                                                       vec_ok);
+  }
+}
+
 // ---- decoders ---------------------------------------------------------------------
 
 // Uncompressed fp32 features of 4 k + 2 columns (602): rows start at multiples of 8 bytes only.  A lane still owns
@@ -532,6 +582,32 @@ int run(Dec dec, const void* indptr, const void* indices, int idx_dtype, typenam
   return launch_status(what);
 }
 
+// Plain features: a group is as wide as a row needs (a row of 4 k columns takes D / 4 lanes).  Rows of four lanes and
+// fewer stay with the skeleton: eight rows in flight need ids for eight edges from one load of the group.  So do rows
+// beyond what the grid counts in.
+constexpr int64_t kPlainBlocks = 1 << 15;   // row blocks of the grid; more rows go round
+template <class Dec>
+int run_plain(Dec dec, const void* indptr, const void* indices, int idx_dtype, typename Dec::Out* out, int64_t R, int64_t E,
+              int64_t N, int feat_dim, bool vec_ok, hipStream_t st, const char* what) {
+  const Geometry g = plan(R, feat_dim, 1, Dec::NOUT, 0);
+  const int64_t passes = ceil_div(feat_dim, (int64_t)g.G * Dec::NOUT);
+  if (g.G < kPlainUnroll || passes > 65535)
+    return run(dec, indptr, indices, idx_dtype, out, R, E, N, feat_dim, g, 0, vec_ok, st, what);
+  const int64_t blocks = ceil_div(R, 256 / g.G);
+  const dim3 grid((unsigned)passes, (unsigned)(blocks < kPlainBlocks ? blocks : kPlainBlocks));
+  if (plan_only()) {
+    plan_record("agg_plain_kernel", (int64_t)grid.x * grid.y, 256, 0, 0, 256 / g.G);
+    return 0;
+  }
+  if (idx_dtype == F2CGT_DT_I32)
+    agg_plain_kernel<Dec, int32_t><<<grid, 256, 0, st>>>(dec, static_cast<const int32_t*>(indptr),
+                                                         static_cast<const int32_t*>(indices), out, R, E, N, feat_dim, g.G, vec_ok);
+  else
+    agg_plain_kernel<Dec, int64_t><<<grid, 256, 0, st>>>(dec, static_cast<const int64_t*>(indptr),
+                                                         static_cast<const int64_t*>(indices), out, R, E, N, feat_dim, g.G, vec_ok);
+  return launch_status(what);
+}
+
 int check_graph(const char* what, const void* indptr, const void* indices, int idx_dtype,
                 const void* out, int64_t R, int64_t E, int64_t N, int64_t feat_dim) {
   F2CGT_REQUIRE(R >= 0 && E >= 0 && N >= 0 && feat_dim >= 0, F2CGT_E_INVALID, "%s: negative size", what);
@@ -666,13 +742,13 @@ extern "C" int f2cgt_spmm_csr(const void* feat, int feat_dtype, void* out, const
       const bool v4 = D % 4 == 0 && aligned(feat, 16) && aligned(out, 16);
       if (v4) {
         PlainDec<float, 4> d{static_cast<const float*>(feat), feat_dim};
-        return run(d, indptr, indices, idx_dtype, static_cast<float*>(out), num_rows, num_edges,
-                   num_src_rows, D, plan(num_rows, D, 1, 4, 0), 0, true, st, what);
+        return run_plain(d, indptr, indices, idx_dtype, static_cast<float*>(out), num_rows, num_edges,
+                         num_src_rows, D, true, st, what);
       }
       if (D % 2 == 0 && D >= 6 && aligned(feat, 8) && aligned(out, 8)) {   // rows of 4 k + 2 columns
         PlainPairsDec d{static_cast<const float*>(feat), feat_dim};
-        return run(d, indptr, indices, idx_dtype, static_cast<float*>(out), num_rows, num_edges,
-                   num_src_rows, D, plan(num_rows, D, 1, 4, 0), 0, true, st, what);
+        return run_plain(d, indptr, indices, idx_dtype, static_cast<float*>(out), num_rows, num_edges,
+                         num_src_rows, D, true, st, what);
       }
       if (D % 2 == 0 && aligned(feat, 8) && aligned(out, 8)) {   // two columns
         PlainDec<float, 2> d{static_cast<const float*>(feat), feat_dim};
@@ -680,18 +756,18 @@ extern "C" int f2cgt_spmm_csr(const void* feat, int feat_dtype, void* out, const
                    num_src_rows, D, plan(num_rows, D, 1, 2, 0), 0, true, st, what);
       }
       PlainDec<float, 1> d{static_cast<const float*>(feat), feat_dim};
-      return run(d, indptr, indices, idx_dtype, static_cast<float*>(out), num_rows, num_edges,
-                 num_src_rows, D, plan(num_rows, D, 1, 1, 0), 0, false, st, what);
+      return run_plain(d, indptr, indices, idx_dtype, static_cast<float*>(out), num_rows, num_edges,
+                       num_src_rows, D, false, st, what);
     }
     case F2CGT_DT_F16: {
       PlainDec<__half, 1> d{static_cast<const __half*>(feat), feat_dim};
-      return run(d, indptr, indices, idx_dtype, static_cast<__half*>(out), num_rows, num_edges,
-                 num_src_rows, D, plan(num_rows, D, 1, 1, 0), 0, false, st, what);
+      return run_plain(d, indptr, indices, idx_dtype, static_cast<__half*>(out), num_rows, num_edges,
+                       num_src_rows, D, false, st, what);
     }
     case F2CGT_DT_F64: {
       PlainDec<double, 1> d{static_cast<const double*>(feat), feat_dim};
-      return run(d, indptr, indices, idx_dtype, static_cast<double*>(out), num_rows, num_edges,
-                 num_src_rows, D, plan(num_rows, D, 1, 1, 0), 0, false, st, what);
+      return run_plain(d, indptr, indices, idx_dtype, static_cast<double*>(out), num_rows, num_edges,
+                       num_src_rows, D, false, st, what);
     }
     default:
       return fail(F2CGT_E_UNSUPPORTED, "%s: feat must be float32, float16 or float64", what);
