@@ -1339,8 +1339,17 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
   // shape: 845 -> 405 us); from about 8 edges per row the detour through LDS costs more than it saves
   a.dense_store = avg_deg <= 8.0;
   // Above that (up to 16 edges per row, four-row mini-blocks) the form is chosen by what binds the launch:
-  //  * the code table beyond the caches (over 192 MB) or rows of more than four column tiles: the gather binds, the
-  //    results are stored as they are (24 x 32 from a 5.8 GB table: 423 us; 446 through LDS, 454 with the exchange);
+  //  * a code table beyond the 256 MB last-level cache, rows of one to four whole column lines (feat_dim a multiple of 32,
+  //    at most 512) and an output of 32 MB and more: through LDS.  A minibatch finds neither its ids nor its output's lines
+  //    in the caches, and then a store instruction that writes half lines waits longest (four graphs in turn, skewed /
+  //    uniform ids, plain -> LDS: 16 x 8 at 15 edges per row from 480 MB 130 -> 117 / 205 -> 193 us, at 12 21.1 -> 20.0 /
+  //    40.0 -> 38.0; 16 x 16 at 10 64 -> 52 / 103 -> 92; 32 x 16 at 10 from 640 MB 43.6 -> 31.6 / 58.0 -> 54.5, at 15 253 ->
+  //    223 / 312 -> 289; an output of 24 MB 14.0 -> 13.8).  One graph again and again 63 -> 52 (16 x 16), 43 -> 35 (32 x 16),
+  //    85 -> 93 (16 x 8 at 15, skewed; uniform 204 -> 191).  304 columns 45 -> 50: rows that end inside a line stay as they are;
+  //  * a code table of 192 to 256 MB, or rows of more than four column tiles: the results are stored as they are (24 x 32
+  //    at 12 edges per row from 240 MB, graphs in turn: 193 us, 208 through LDS; from 120 MB 178 against 195).  From 5.8 GB
+  //    at 10 per row one graph again and again takes 420 us, 442 through LDS, and graphs in turn 681 against 585:
+  //    F2CGT_STORE_STREAM is for the latter;
   //  * an output of 200 MB and more from a table of 64 to 192 MB, which shares the last-level cache with it: through
   //    LDS as for sparse rows, the form whose store instructions write whole lines.  Warm it is level with the exchange
   //    (7.5e6 edges at 15 per row from a 160 MB table, 16 x 8: 79.1 against 79.4 us; plain 80.7), with graphs and
@@ -1353,15 +1362,17 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
   //    at 10 per row, plain -> exchange: 16 x 16 121 -> 87 us, 32 x 16 166 -> 90, 8 x 32 126 -> 90, 64 x 8 150 -> 93,
   //    16 x 8 49 -> 42; the plain form's time at these shapes varies by a factor of two between builds and boxes,
   //    the exchange's does not).  64-column tiles (half the lanes of a row idle) measured 6-13 % slower with it.
-  // F2CGT_STORE_STREAM (the caller's outputs are written once and read later) takes the LDS form throughout: with
-  // buffers in rotation the 5.8 GB case runs in 588 us against 681.
+  // F2CGT_STORE_STREAM (the caller's outputs are written once and read later) takes the LDS form throughout.
   const bool rpm4 = avg_deg <= 16.0 * ((a.R > 0 && a.E % a.R == 0) ? 1.0 : 0.9);
+  const int64_t out_bytes = a.R * (int64_t)a.feat_dim * 4;
+  const bool big_table = a.N * (int64_t)a.n_cb > (256ll << 20);
   if (!a.dense_store && a.feat_dim % 8 == 0 && rpm4) {
     const bool cached_table = a.N * (int64_t)a.n_cb <= (192ll << 20);
-    if (store_mode() == F2CGT_STORE_STREAM) {
+    if (store_mode() == F2CGT_STORE_STREAM ||
+        (big_table && a.feat_dim >= 128 && a.feat_dim % 32 == 0 && a.n_tiles <= 4 && out_bytes >= (32ll << 20))) {
       a.dense_store = 1;
     } else if (cached_table && a.feat_dim >= 128 && a.n_tiles <= 4) {
-      const bool big_out = a.R * (int64_t)a.feat_dim * 4 >= (200ll << 20);
+      const bool big_out = out_bytes >= (200ll << 20);
       if (big_out && a.N * (int64_t)a.n_cb >= (64ll << 20)) a.dense_store = 1;
       else if (big_out || avg_deg <= 11.0) a.dense_store = 4;
     }
@@ -1435,7 +1446,19 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
     // 25 x 8 326 / 165 -> 299 / 146 us, 21 x 8 299 / 150 -> 257 / 123, 15 x 8 186 / 102 -> 152 / 76, 19 x 32 at 600
     // columns 603 / 313 -> 551 / 279; rows of whole lines the other way round: 24 x 8 172 / 101 against 191 / 100,
     // 7 x 32 180 / 96 against 192 / 103).
-    if (avg_deg <= 8.0 && a.feat_dim % 32 != 0) {
+    // Above that, rows that are no whole 64-byte pieces (feat_dim an odd multiple of 8): the same, where the eight-column
+    // form has no exchange (more than four column tiles, or a table beyond the last-level cache) from 100 MB of output on,
+    // else from the size of the last-level cache on; up to 12 edges per row, and up to 16 from a table beyond that cache.
+    // Graphs in turn, skewed / uniform ids, eight-column form -> this: 19 x 32 at 600 columns, 9 edges per row, 457 MB
+    // 223 -> 144 / 180 -> 145 us, 12 per row, 114 MB 52 -> 44 / 51 -> 45, 16 per row from 362 MB of codes 60 -> 58 / 91 -> 85;
+    // 712 columns 127 -> 96 / 126 -> 100; 25 x 8 at 200, 305 MB, 9 per row 127 -> 112 / 173 -> 151, 12 per row 119 -> 117 /
+    // 206 -> 192; 152 columns 183 -> 163 / 199 -> 182.  At 13 and more from a small table it is ahead with uniform ids only
+    // (200 columns 214 -> 172, skewed 123 -> 132), below those sizes level; one tile loses (104 columns 82 -> 96), and so do
+    // rows of whole 64-byte pieces (304 columns 97 -> 108, 144 columns 137 -> 149).
+    const bool split_rows = a.feat_dim % 16 == 8 && a.n_tiles > 1 && rpm4 && store_mode() != F2CGT_STORE_STREAM &&
+                            out_bytes >= (a.n_tiles > 4 || big_table ? 100000000ll : 256ll << 20) &&
+                            (avg_deg <= 12.0 || big_table);
+    if ((avg_deg <= 8.0 && a.feat_dim % 32 != 0) || split_rows) {
       a.dense_store = 0;
       a.own_lg = 0;
       return launch_wave<BT, 1, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);

@@ -196,6 +196,31 @@ def test_fused_vq_store_form_by_shape():
     assert lanes(1_000_000, 3, 224, 7, 32) == 2 and lanes(1_000_000, 3, 600, 19, 32) == 1
 
 
+def test_fused_vq_forms_for_tables_beyond_the_last_level_cache_and_rows_of_split_pieces():
+    def plan(rows, fanout, d, n_cb, w, n_src):
+        rc, p = capi.dry_run("f2cgt_vq_decompress_spmm_csr", A16, capi.DT_U8, A16, A16, A16, capi.DT_I64, A16, rows,
+                             rows * fanout, n_src, d, n_cb, 256, w, None)
+        assert rc == 0 and p.kernel.decode() == "vq_wave_kernel"
+        return p.aux[0], p.aux[2]          # float4 per lane and edge, store form
+    # a table of more than 256 MB: through LDS from 32 MB of output on, up to four column tiles of whole lines
+    assert plan(65_536, 15, 128, 16, 8, 16_777_217) == (2, 1)
+    assert plan(65_535, 15, 128, 16, 8, 16_777_217) == (2, 0)
+    assert plan(65_536, 15, 128, 16, 8, 16_777_216) == (2, 0)
+    assert plan(65_536, 15, 512, 32, 16, 10_000_000) == (2, 1)
+    assert plan(65_536, 15, 544, 34, 16, 10_000_000) == (2, 0)
+    assert plan(65_536, 15, 304, 19, 16, 20_000_000) == (2, 0)
+    assert plan(65_536, 17, 128, 16, 8, 16_777_217) == (2, 0)
+    # odd multiples of eight columns: one float4 per lane
+    assert plan(41_667, 12, 600, 19, 32, 1_000_000) == (1, 0)
+    assert plan(41_666, 12, 600, 19, 32, 1_000_000) == (2, 0)
+    assert plan(41_667, 13, 600, 19, 32, 1_000_000) == (2, 0)
+    assert plan(41_667, 16, 600, 19, 32, 15_000_000) == (1, 0)
+    assert plan(335_545, 12, 200, 25, 8, 1_000_000)[0] == 1 and plan(335_544, 12, 200, 25, 8, 1_000_000)[0] == 2
+    assert plan(125_000, 12, 200, 25, 8, 12_000_000)[0] == 1
+    assert plan(700_000, 9, 104, 13, 8, 1_000_000)[0] == 2          # one column tile
+    assert plan(400_000, 12, 208, 26, 8, 1_000_000)[0] == 2         # whole 64-byte pieces
+
+
 def test_dealt_items_and_column_form_of_one_codebook():
     """1-bit rows: items take 256 threads per workgroup, the column form 128."""
     def block(rows, dim, fanout, n_cb=1, bits=1):
