@@ -232,6 +232,7 @@ struct F4Args {
   const int32_t* slot;
   int64_t num_rows, num_slots;
   int32_t* bad;
+  int64_t rows;           // ROWS: output rows
 };
 
 // Table row of output row r (ROWS: int32_t or int64_t ids, void without).  The lookup, the check of its ids, the fetch and
@@ -251,11 +252,32 @@ __device__ __forceinline__ int64_t table_row(const F4Args& a, int64_t r) {
   }
 }
 
+// ROWS: the table rows of a workgroup's span, looked up once into LDS while its decode table is made.  With the lookup at
+// every item, a 16-byte piece of two column pairs waited for two ids and two code bytes (161 000 rows of 154 columns, 4 bit:
+// 39.5 us, 30.1 here, with the rows fetched first 11.8 + 19.9; 304 000 of 256 columns, 8 bit: 89.6, 73.7, 38.1 + 56.8; the
+// 1024 seed rows of a minibatch, 128 columns through the id map: 9.3, 5.9).
+constexpr int kSpanRows = kF4Items * kBlock / 2 + 2;     // a row has two items and more
+template <typename ROWS>
+__device__ __forceinline__ void stage_span_rows(const F4Args& a, int64_t first, uint32_t count, int64_t* s_rows) {
+  const int64_t left = a.rows - first;
+  const int n = (int)((int64_t)count < left ? (int64_t)count : left);
+  for (int i = threadIdx.x; i < n; i += kBlock) s_rows[i] = table_row<ROWS>(a, first + i);
+}
+
 template <int BITS, bool AFFINE, typename ROWS = void>
 __global__ __launch_bounds__(kBlock) void sq_decode_f4_kernel(F4Args a) {
+  constexpr bool kRows = !std::is_void<ROWS>::value;
+  __shared__ int64_t s_rows[kRows ? kSpanRows : 1];
   constexpr int NCODE = 1 << BITS;
   constexpr uint32_t MASK = NCODE - 1;
   extern __shared__ __align__(16) float s_tab[];
+  const int64_t base = (int64_t)blockIdx.x * (kF4Items * kBlock);
+  // first row of the span: floor(base / f4_per_row), from the fp64 quotient and a fix-up
+  int64_t rb = (int64_t)((double)base / (double)a.f4_per_row);
+  if (rb * a.f4_per_row > base) --rb;
+  if ((rb + 1) * (int64_t)a.f4_per_row <= base) ++rb;
+  const uint32_t cb0 = (uint32_t)(base - rb * a.f4_per_row);
+  if constexpr (kRows) stage_span_rows<ROWS>(a, rb, (cb0 + kF4Items * kBlock - 1) / a.f4_per_row + 1, s_rows);
   // affine: [f4][mn x4, scale x4]; log domain: LUT [n_cb][NCODE], then the codebook of each column
   const int feat_dim = (int)a.f4_per_row * 4;
   int* s_cbi = reinterpret_cast<int*>(s_tab + ((a.n_cb * NCODE + 3) & ~3));
@@ -275,13 +297,6 @@ __global__ __launch_bounds__(kBlock) void sq_decode_f4_kernel(F4Args a) {
   }
   __syncthreads();
 
-  const int64_t base = (int64_t)blockIdx.x * (kF4Items * kBlock);
-  // first row of the span: floor(base / f4_per_row), from the fp64 quotient and a fix-up
-  int64_t rb = (int64_t)((double)base / (double)a.f4_per_row);
-  if (rb * a.f4_per_row > base) --rb;
-  if ((rb + 1) * (int64_t)a.f4_per_row <= base) ++rb;
-  const uint32_t cb0 = (uint32_t)(base - rb * a.f4_per_row);
-
   uint32_t word[kF4Items], c4s[kF4Items];
 #pragma unroll
   for (int k = 0; k < kF4Items; ++k) {
@@ -289,7 +304,9 @@ __global__ __launch_bounds__(kBlock) void sq_decode_f4_kernel(F4Args a) {
     const uint32_t rl = __umulhi(li, a.magic);
     const uint32_t c4 = li - rl * a.f4_per_row;
     const bool on = base + threadIdx.x + k * kBlock < a.total_f4;
-    const uint8_t* src = a.codes + (on ? table_row<ROWS>(a, rb + rl) * a.src_dim : 0);
+    int64_t row = rb + rl;
+    if constexpr (kRows) row = on ? s_rows[rl] : 0;
+    const uint8_t* src = a.codes + (on ? row * a.src_dim : 0);
     c4s[k] = c4;
     if (BITS == 8) {
       uint32_t w; __builtin_memcpy(&w, src + (on ? 4 * c4 : 0), 4); word[k] = w;
@@ -336,6 +353,18 @@ template <int BITS, bool AFFINE, typename ROWS = void>
 __global__ __launch_bounds__(kBlock) void sq_decode_pairs_kernel(F4Args a) {
   constexpr int NCODE = 1 << BITS;
   constexpr uint32_t MASK = NCODE - 1;
+  constexpr bool kRows = !std::is_void<ROWS>::value;
+  __shared__ int64_t s_rows[kRows ? kSpanRows : 1];
+  const uint32_t ppr = a.f4_per_row;             // pairs per row (feat_dim / 2)
+  const int64_t total_pairs = a.total_f4;        // rows * pairs per row
+  const int64_t base = (int64_t)blockIdx.x * (kF4Items * kBlock);
+  // first row of the workgroup's span of pairs: floor(2 base / ppr), from the fp64 quotient and a fix-up; the pairs
+  // of the span are then counted from that row's first, small enough for the 32-bit multiply-high to be exact
+  int64_t rb = (int64_t)((double)(2 * base) / (double)ppr);
+  if (rb * ppr > 2 * base) --rb;
+  if ((rb + 1) * (int64_t)ppr <= 2 * base) ++rb;
+  const uint32_t l0 = (uint32_t)(2 * base - rb * ppr);
+  if constexpr (kRows) stage_span_rows<ROWS>(a, rb, (l0 + 2 * kF4Items * kBlock - 1) / ppr + 1, s_rows);
   extern __shared__ __align__(16) float s_tab[];
   // affine: [column][min, scale]; log domain: LUT [n_cb][NCODE], then the LUT base of each column
   int* s_cbi = reinterpret_cast<int*>(s_tab + ((a.n_cb * NCODE + 3) & ~3));
@@ -354,20 +383,13 @@ __global__ __launch_bounds__(kBlock) void sq_decode_pairs_kernel(F4Args a) {
     }
   }
   __syncthreads();
-  const uint32_t ppr = a.f4_per_row;             // pairs per row (feat_dim / 2)
-  const int64_t total_pairs = a.total_f4;        // rows * pairs per row
-  const int64_t base = (int64_t)blockIdx.x * (kF4Items * kBlock);
-  // first row of the workgroup's span of pairs: floor(2 base / ppr), from the fp64 quotient and a fix-up; the pairs
-  // of the span are then counted from that row's first, small enough for the 32-bit multiply-high to be exact
-  int64_t rb = (int64_t)((double)(2 * base) / (double)ppr);
-  if (rb * ppr > 2 * base) --rb;
-  if ((rb + 1) * (int64_t)ppr <= 2 * base) ++rb;
-  const uint32_t l0 = (uint32_t)(2 * base - rb * ppr);
   auto pair = [&](int64_t p, float& v0, float& v1) {
     const uint32_t li = l0 + (uint32_t)(p - 2 * base);
     const uint32_t rl = __umulhi(li, a.magic);
     const uint32_t cp = li - rl * ppr;
-    const uint8_t* src = a.codes + table_row<ROWS>(a, rb + rl) * a.src_dim;
+    int64_t row = rb + rl;
+    if constexpr (kRows) row = s_rows[rl];
+    const uint8_t* src = a.codes + row * a.src_dim;
     uint32_t c0, c1;
     if (BITS == 8) {
       uint16_t w; __builtin_memcpy(&w, src + 2 * cp, 2);
@@ -431,6 +453,7 @@ int decode_f4_launch(const uint8_t* codes, float* out, const float* table, int64
   const bool pairs = feat_dim % 4 != 0;
   a.f4_per_row = (uint32_t)(pairs ? feat_dim / 2 : feat_dim / 4);
   a.total_f4 = rows * a.f4_per_row;
+  a.rows = rows;
   a.magic = (uint32_t)((0x100000000ull + a.f4_per_row - 1) / a.f4_per_row);
   const int64_t lanes = pairs ? a.total_f4 / 2 + 1 : a.total_f4;
   const int64_t grid = ceil_div(lanes, kF4Items * kBlock);
