@@ -146,6 +146,9 @@ __device__ __forceinline__ void split2(float v, _Float16& hi, _Float16& lo) {
 //   rounding of the centring by 2^-22 (|x'|^2 + |c'|^2): 4 * 2^-22 (9.6e-7) for each of two distances.
 //   Cosine: -x . d with |d| <= cdev; fp32 sum, roundings of the normalisation and of m ((k + 2) cdev + 3) 2^-24 |x|, the
 //   pieces 2^-22 |x| cdev, for each of two scores.
+//   Where fp32 has no number for a distance (a centre beyond the range of the pieces, which |c|^2 beyond the largest float
+//   admits; sums that overflow) it leaves nothing out: such a distance passes, and where it makes the limit no number, or
+//   a row's dot products may overflow (|x| >= 1e38), every centre does.
 template <int S>
 __device__ __forceinline__ int exact_row(const AssignArgs& a, const float* __restrict__ xrow,
                                          const float* __restrict__ centers, float* xs, const half8* ap, const float* inv,
@@ -211,8 +214,9 @@ __device__ __forceinline__ int exact_row(const AssignArgs& a, const float* __res
     xnorm2 += __shfl_xor(xnorm2, off);
     xn += __shfl_xor(xn, off);
   }
-  const float limit = cosine ? nearest + (1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) + 4.9e-7f * cdev) * sqrtf(xnorm2) * 1.001f + 1e-30f
-                             : nearest * (1.f + 1.1920929e-7f * (float)(k + 4)) + 1e-37f + 2.1e-6f * (xnorm2 + cmax);
+  float limit = cosine ? nearest + (1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) + 4.9e-7f * cdev) * sqrtf(xnorm2) * 1.001f + 1e-30f
+                       : nearest * (1.f + 1.1920929e-7f * (float)(k + 4)) + 1e-37f + 2.1e-6f * (xnorm2 + cmax);
+  if (cosine && !(xn < 1e76)) limit = INFINITY;
   double bestv = DBL_MAX;
   int besti = INT_MAX;
   for (int c0 = lane; c0 < n; c0 += kKeep * kWave) {
@@ -223,7 +227,7 @@ __device__ __forceinline__ int exact_row(const AssignArgs& a, const float* __res
       float di = c0 == lane ? keep[0] : d[0];
 #pragma unroll
       for (int q = 1; q < kKeep; ++q) di = i == q ? (c0 == lane ? keep[q] : d[q]) : di;
-      if (!(di <= limit) || c >= n) continue;
+      if (di > limit || c >= n) continue;                // (passes what is no number)
       // float64 on the original values, eight of the centre's in flight
       const float* cr = centers + (int64_t)c * k;
       double dot = 0.0, cn = 0.0;

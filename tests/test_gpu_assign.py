@@ -84,3 +84,32 @@ def test_rows_that_are_no_numbers(metric):
     x[5, 3], x[64, 0], x[199, 23] = np.nan, np.inf, -np.inf
     near = check(x, c, metric)
     assert near.sum() <= 3 + 1
+
+
+# squares beyond the largest float, of some centres or of all, with rows beside the large centres and far from them: neither
+# the scores nor the fp32 distances hold a number, and float64 on the original values decides
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("scale", [1e20, 1.5e20, 1e21, 1e25, 1e30, 1e36])
+@pytest.mark.parametrize("large", ["one", "half", "all"])
+@pytest.mark.parametrize("k", [1, 16, 30, 64])
+def test_values_whose_squares_overflow(metric, scale, large, k):
+    print("case assign overflow", metric, scale, large, k, flush=True)
+    rng = np.random.default_rng(k)
+    n = 300 if k == 16 else 140
+    c = rng.standard_normal((n, k))
+    pick = {"one": [n - 3], "half": list(range(0, n, 2)), "all": list(range(n))}[large]
+    c[pick] *= scale
+    x = rng.standard_normal((500, k))
+    x[::2] *= scale
+    x[:n] = np.where(np.arange(n)[:, None] % 3 == 0, c * 1.0001, x[:n])
+    check(x.astype(np.float32), c.astype(np.float32), metric)
+
+
+# cosine: rows whose fp32 dot products overflow, in every order of signs
+@pytest.mark.parametrize("size", [1e38, 3.3e38])
+@pytest.mark.parametrize("k", [4, 16, 50])
+def test_rows_whose_products_overflow(size, k):
+    print("case assign overflow rows", size, k, flush=True)
+    rng = np.random.default_rng(k)
+    x = (np.sign(rng.standard_normal((300, k))) * size * rng.uniform(0.5, 1.0, (300, k))).astype(np.float32)
+    check(x, rng.standard_normal((70, k)).astype(np.float32), "cosine")

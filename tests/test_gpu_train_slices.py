@@ -97,6 +97,26 @@ def test_one_step(metric, slices, m, n, k, masked):
         assert np.abs(got[s] - want).max() <= 6e-8 * 5.0 * max(2, m / n * 8)
 
 
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("scale", [1e21, 1e30])
+@pytest.mark.parametrize("k", [16, 30])
+def test_one_step_with_centres_whose_squares_overflow(metric, scale, k):
+    print("case kmeans_slices overflow", metric, scale, k, flush=True)
+    rng = np.random.default_rng(k)
+    x, c = rng.standard_normal((2, 700, k)), rng.standard_normal((2, 40, k))
+    x[:, ::2] *= scale
+    c[:, ::3] *= scale
+    x, c = x.astype(np.float32), c.astype(np.float32)
+    centers = torch.from_numpy(c).cuda()
+    f2cgt_amd.load().kmeans_slices_fit(torch.from_numpy(x).cuda(), None, centers, metric, 0, 0.0, 1.0, 1, 8)
+    got = centers.cpu().numpy().astype(np.float64)
+    for s in range(2):
+        want = step64(x[s], np.ones(700, bool), c[s], metric)
+        # a mean of fp64 sums rounded once per set and a few times behind them: below 2^-20 of the largest member
+        assert (np.abs(got[s] - want) <= 1e-6 * np.abs(x[s]).max()).all()
+        assert (np.abs(got[s] - want) <= 1e-6 * np.maximum(np.abs(want).max(1, keepdims=True), 8.0)).all()
+
+
 def test_slices_stop_one_by_one():
     """A slice that has met the rule keeps its centres while the others go on; NaN in one flags only that one."""
     rng = np.random.default_rng(5)
