@@ -214,7 +214,8 @@ __device__ __forceinline__ int exact_row(const AssignArgs& a, const float* __res
     xnorm2 += __shfl_xor(xnorm2, off);
     xn += __shfl_xor(xn, off);
   }
-  float limit = cosine ? nearest + (1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) + 4.9e-7f * cdev) * sqrtf(xnorm2) * 1.001f + 1e-30f
+  // (cosine: |x| from the fp64 sum, its square may vanish in fp32)
+  float limit = cosine ? nearest + (1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) + 4.9e-7f * cdev) * (float)sqrt(xn) * 1.001f + 1e-30f
                        : nearest * (1.f + 1.1920929e-7f * (float)(k + 4)) + 1e-37f + 2.1e-6f * (xnorm2 + cmax);
   if (cosine && !(xn < 1e76)) limit = INFINITY;
   double bestv = DBL_MAX;
@@ -729,8 +730,9 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     // fp64, one rounding for 1 / |c|, one for the product, one for - m: 3 units, doubled) does not
     const float scale = cosine ? sqrtf(xn) * (cdev + 3.5762787e-7f / unit) : xn + cmax;
     const float bound = unit * scale + kTinyGap + slack;
-    // padding leads where no real score is a number
-    const bool ask = besti >= n || !(scale < finite_below) || !((runner - bs) > bound);
+    // Padding leads where no real score is a number.  A row whose square is below the smallest normal float has pieces of
+    // too few bits and no norm to bound that by; L2 has the centres' norm, or products below kTinyGap.
+    const bool ask = besti >= n || !(scale < finite_below) || !((runner - bs) > bound) || (cosine && xn < FLT_MIN);
     uint64_t todo = __ballot(grp * 32 + j < m && g == 0 && ask);
     // exact evaluation of the flagged rows
     while (todo) {

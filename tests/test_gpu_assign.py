@@ -113,3 +113,16 @@ def test_rows_whose_products_overflow(size, k):
     rng = np.random.default_rng(k)
     x = (np.sign(rng.standard_normal((300, k))) * size * rng.uniform(0.5, 1.0, (300, k))).astype(np.float32)
     check(x, rng.standard_normal((70, k)).astype(np.float32), "cosine")
+
+
+# cosine: rows so short that their squares vanish in fp32, against centres so long that |x||c| stays above the clamp at 1e-8
+@pytest.mark.parametrize("short", [18.5, 19.5, 21, 23, 26, 30, 36])
+@pytest.mark.parametrize("k", [3, 16, 30, 64])
+def test_rows_whose_squares_vanish(short, k):
+    print("case assign short rows", short, k, flush=True)
+    rng = np.random.default_rng(k)
+    x = rng.standard_normal((600, k)) * 10.0 ** -short
+    x[::50] = 0
+    c = rng.standard_normal((140, k)) * 1e31
+    near = check(x.astype(np.float32), c.astype(np.float32), "cosine")
+    assert near.sum() < 40
