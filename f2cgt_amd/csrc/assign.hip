@@ -574,6 +574,8 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
   while (grp < wg_hi) {
     int drawn = 0;
     if (lane == 0) drawn = atomicAdd(flags + 2, 1);
+    uint32_t kept = ~0u;                    // the group's rows that take part
+    if (SUMS && a.keep != nullptr) kept = a.keep[slice * a.keep_words + grp];
     half8 xp[S][2];
     float own[SUMS ? S : 1][8];
     if constexpr (SUMS) {
@@ -733,8 +735,9 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     // Padding leads where no real score is a number.  A row whose square is below the smallest normal float has pieces of
     // too few bits and no norm to bound that by; L2 has the centres' norm, or products below kTinyGap.
     const bool ask = besti >= n || !(scale < finite_below) || !((runner - bs) > bound) || (cosine && xn < FLT_MIN);
-    uint64_t todo = __ballot(grp * 32 + j < m && g == 0 && ask);
-    // exact evaluation of the flagged rows
+    // exact evaluation of the flagged rows (of a training step, of those that take part: the rows left out are the shortest
+    // ones, and a row of zeros ties with every centre)
+    uint64_t todo = __ballot(grp * 32 + j < m && g == 0 && ask) & kept;
     while (todo) {
       const int src = __ffsll((unsigned long long)todo) - 1;
       todo &= todo - 1;
@@ -745,7 +748,7 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     }
     if constexpr (SUMS) {
       const int to = (int)halves((uint32_t)besti).lo;            // the exact evaluation's label is in the lower half
-      const bool in = grp * 32 + j < m && (a.keep == nullptr || (a.keep[slice * a.keep_words + grp] >> j & 1u));
+      const bool in = grp * 32 + j < m && (kept >> j & 1u);
       if (in) {
 #pragma unroll
         for (int st = 0; st < S; ++st)

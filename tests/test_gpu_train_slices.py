@@ -117,6 +117,27 @@ def test_one_step_with_centres_whose_squares_overflow(metric, scale, k):
         assert (np.abs(got[s] - want) <= 1e-6 * np.maximum(np.abs(want).max(1, keepdims=True), 8.0)).all()
 
 
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("value", [0.0, 1e-25, float("nan"), float("inf")])
+def test_rows_left_out_do_not_count(metric, value):
+    """Rows outside the mask that tie with every centre, or are no numbers: as if they were not there."""
+    rng = np.random.default_rng(9)
+    x, c = rng.standard_normal((3, 1000, 12)).astype(np.float32), rng.standard_normal((3, 50, 12)).astype(np.float32)
+    keep = rng.random((3, 1000)) < 0.6
+    x[~keep] = value
+    padded = np.zeros((3, 1024), bool)
+    padded[:, :1000] = keep
+    bits = torch.from_numpy(np.packbits(padded, axis=1, bitorder="little").view(np.int32).copy()).cuda()
+    centers = torch.from_numpy(c).cuda()
+    f2cgt_amd.load().kmeans_slices_fit(torch.from_numpy(x).cuda(), bits, centers, metric, 0, 0.0, 1.0, 1, 8)
+    got = centers.cpu().numpy().astype(np.float64)
+    for s in range(3):
+        mine = x[s][keep[s]]
+        want = step64(mine, np.ones(len(mine), bool), c[s], metric)
+        # fp64 sums, rounded once per set of rows: a few 2^-24 of the largest value
+        assert np.abs(got[s] - want).max() <= 2.0 ** -21 * np.abs(mine).max()
+
+
 def test_slices_stop_one_by_one():
     """A slice that has met the rule keeps its centres while the others go on; NaN in one flags only that one."""
     rng = np.random.default_rng(5)
