@@ -170,6 +170,7 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
         codebooks, stats = capi.sq_codebooks(features, sample_index, column_slice,
                                              [r for per_size in places for place in per_size for r in place[:2]],
                                              [place[2] for per_size in places for place in per_size])
+        codebooks = codebooks.cuda()      # (the codes are made on the current device, wherever the table lies)
     else:
         per_slice = [[float(v) for v in values] for values in _sampled_sq_codebooks(features, sample_index, column_slice)]
         codebooks = (torch.tensor(per_slice, dtype=torch.float32) if per_slice else torch.zeros((0, 5))).cuda()

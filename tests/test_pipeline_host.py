@@ -1,6 +1,10 @@
 """Host-side pieces of f2cgt_amd/pipeline.py that need no GPU."""
+import types
+
 import numpy as np
+import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
 import f2cgt_oracle as oc
 from f2cgt_amd import pipeline
@@ -52,3 +56,33 @@ def test_what_the_device_statistics_take():
     for m, cols, width in ((2 ** 32, 1, 1), (2 ** 25, 500, 128), (3, 2 ** 24, 2 ** 24), (3, 65536, 1), (0, 8, 8), (8, 0, 8)):
         assert not pipeline._device_takes(m, cols, width)
         assert capi.lib().f2cgt_abs_order_stats(a, max(cols, 1), a, m, max(m, 1), cols, width, ranks, a, 1 << 62, a, None)
+
+
+class _Devices:
+    """Stands for the operator library: checks that the tensors of a call lie on one device, computes nothing."""
+
+    def __init__(self):
+        self.calls = []
+
+    def sq_codebooks(self, x, rows, column_slice, ranks, weights):
+        self.calls.append("sq_codebooks")
+        assert rows.device == x.device
+        slices = -(-x.shape[1] // column_slice)
+        stats = types.SimpleNamespace(cpu=lambda: types.SimpleNamespace(numpy=lambda: np.zeros((slices, 6))))
+        return torch.empty((slices, 5), device=x.device), stats
+
+    def sq_encode(self, data, codebooks, bits, column_slice, out):
+        self.calls.append("sq_encode")
+        assert data.device == codebooks.device == out.device
+
+
+@pytest.mark.parametrize("table", ["cuda:0", "cuda:1"])
+def test_sq_codes_of_a_table_on_a_device_that_is_not_the_current_one(table, monkeypatch):
+    """Codes and codebooks are made on the current device, wherever the table lies."""
+    lib = _Devices()
+    monkeypatch.setattr(pipeline, "_capi", lambda: lib)
+    with FakeTensorMode():
+        x = torch.empty((1000, 40), device=table)
+        codes, books = pipeline.sq_compress(x, 4, 16, sample_index=torch.arange(500))
+        assert str(codes.device) == str(books.device) == "cuda:0"
+    assert lib.calls == ["sq_codebooks", "sq_encode"]
