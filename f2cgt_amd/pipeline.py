@@ -292,7 +292,8 @@ def _train_all_slices(features, n_clusters, column_slice, sample_index, max_iter
     if not (sample_index.dtype == torch.int64 and sample_index.dim() == 1 and 0 < m <= 1 << 24 and m * feat_dim <= 1 << 28 and
             capi.kmeans_slices_covers(slices, n_clusters, column_slice) and features.shape[0] > 0):
         return None
-    if features.is_cuda and features.dtype == torch.float32 and features.stride(1) == 1 and features.stride(0) >= feat_dim:
+    if (features.is_cuda and features.device.index == torch.cuda.current_device() and features.dtype == torch.float32 and
+            features.stride(1) == 1 and features.stride(0) >= feat_dim):
         table, rows = features, sample_index.to(features.device)
     else:
         table, rows = features[sample_index.to(features.device)].to(torch.float32).cuda(), None

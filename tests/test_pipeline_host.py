@@ -75,6 +75,26 @@ class _Devices:
         self.calls.append("sq_encode")
         assert data.device == codebooks.device == out.device
 
+    def kmeans_slices_covers(self, slices, n, k):
+        return True
+
+    def slice_rows(self, x, rows, column_slice):
+        assert rows is None or rows.device == x.device
+        m, slices = (x.shape[0] if rows is None else rows.numel()), -(-x.shape[1] // column_slice)
+        return (torch.empty((slices, m, column_slice), device=x.device), torch.empty((m, slices), device=x.device),
+                torch.empty((1,), device=x.device, dtype=torch.int32))
+
+    def abs_order_stats(self, x, rows, column_slice, ranks):
+        return torch.empty((x.shape[1], 6), device=x.device, dtype=torch.float64)
+
+    def keep_rows(self, norms, stats, weight, weight_last):
+        return torch.empty((norms.shape[1], -(-norms.shape[0] // 32)), device=norms.device, dtype=torch.int32)
+
+    def kmeans_slices_fit(self, data, keep, centers, *rest):
+        self.calls.append("kmeans_slices_fit")
+        assert data.device == keep.device == centers.device
+        raise StopIteration
+
 
 @pytest.mark.parametrize("table", ["cuda:0", "cuda:1"])
 def test_sq_codes_of_a_table_on_a_device_that_is_not_the_current_one(table, monkeypatch):
@@ -86,3 +106,15 @@ def test_sq_codes_of_a_table_on_a_device_that_is_not_the_current_one(table, monk
         codes, books = pipeline.sq_compress(x, 4, 16, sample_index=torch.arange(500))
         assert str(codes.device) == str(books.device) == "cuda:0"
     assert lib.calls == ["sq_codebooks", "sq_encode"]
+
+
+@pytest.mark.parametrize("table", ["cuda:0", "cuda:1"])
+def test_codebooks_of_a_table_on_a_device_that_is_not_the_current_one(table, monkeypatch):
+    lib = _Devices()
+    monkeypatch.setattr(pipeline, "_capi", lambda: lib)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    with FakeTensorMode():
+        x = torch.empty((1000, 40), device=table)
+        with pytest.raises(StopIteration):
+            pipeline._train_all_slices(x, 16, 8, torch.arange(500), 4)
+    assert lib.calls == ["kmeans_slices_fit"]
