@@ -131,8 +131,15 @@ torch::Tensor unpackbits(torch::Tensor pack, int64_t target_bits, int64_t unpack
   return unpack;
 }
 
-torch::Tensor sq_codebooks_checked(torch::Tensor codebooks) {
+// Codebooks on another device than the data would be read through a pointer of that device.
+torch::Tensor beside(torch::Tensor codebooks, const torch::Tensor& data) {
   codebooks = dev_contig(codebooks, "codebooks");
+  TORCH_CHECK(codebooks.device() == data.device(), "codebooks are on ", codebooks.device(), ", the data on ", data.device());
+  return codebooks;
+}
+
+torch::Tensor sq_codebooks_checked(torch::Tensor codebooks, const torch::Tensor& data) {
+  codebooks = beside(codebooks, data);
   TORCH_CHECK(codebooks.scalar_type() == torch::kFloat32, "codebooks must be float32");
   TORCH_CHECK(codebooks.dim() == 2 && codebooks.size(1) == 5 && codebooks.size(0) >= 1,
               "SQ codebooks must be [n_codebooks, 5] = fmin,fmax,emin,emax,mean");
@@ -143,7 +150,7 @@ torch::Tensor sq_compress(torch::Tensor src, torch::Tensor codebooks, int64_t ta
                           int64_t column_slice) {
   src = dev_contig(src, "src");
   TORCH_CHECK(src.dim() == 2 && src.scalar_type() == torch::kFloat32, "src must be float32 [rows, feat_dim]");
-  codebooks = sq_codebooks_checked(codebooks);
+  codebooks = sq_codebooks_checked(codebooks, src);
   c10::DeviceGuard guard(src.device());
   auto out = torch::empty_like(src);
   check_rc(f2cgt_sq_compress(src.data_ptr<float>(), out.data_ptr<float>(), codebooks.data_ptr<float>(),
@@ -161,7 +168,7 @@ torch::Tensor sq_encode(torch::Tensor src, torch::Tensor codebooks, int64_t targ
   TORCH_CHECK(src.dim() == 2 && src.scalar_type() == torch::kFloat32, "src must be float32 [rows, feat_dim]");
   TORCH_CHECK(target_bits == 1 || target_bits == 2 || target_bits == 4 || target_bits == 8 || target_bits == 16,
               "target_bits must be 1, 2, 4, 8 or 16");
-  codebooks = sq_codebooks_checked(codebooks);
+  codebooks = sq_codebooks_checked(codebooks, src);
   c10::DeviceGuard guard(src.device());
   const int64_t d = src.size(1);
   const int64_t words = target_bits < 8 ? (d * target_bits + 7) / 8 : d;
@@ -236,7 +243,7 @@ torch::Tensor sq_decompress(torch::Tensor compress_data, torch::Tensor codebooks
                             int64_t column_slice, int64_t feat_dim) {
   compress_data = dev_contig(compress_data, "compress_data");
   TORCH_CHECK(compress_data.dim() == 2, "compress_data must be 2-D");
-  codebooks = sq_codebooks_checked(codebooks);
+  codebooks = sq_codebooks_checked(codebooks, compress_data);
   c10::DeviceGuard guard(compress_data.device());
   auto out = empty_f32({compress_data.size(0), feat_dim}, compress_data);
   check_rc(f2cgt_sq_decompress(compress_data.data_ptr(), dtype_tag(compress_data, "compress_data"),
@@ -249,7 +256,7 @@ torch::Tensor sq_decompress(torch::Tensor compress_data, torch::Tensor codebooks
 
 torch::Tensor vq_decompress(torch::Tensor index_tensor, torch::Tensor codebooks, int64_t feat_dim) {
   index_tensor = dev_contig(index_tensor, "index_tensor");
-  codebooks = dev_contig(codebooks, "codebooks");
+  codebooks = beside(codebooks, index_tensor);
   TORCH_CHECK(index_tensor.dim() == 2, "index_tensor must be [rows, n_codebooks]");
   TORCH_CHECK(codebooks.dim() == 3, "VQ codebooks must be [n_codebooks, K, width]");
   TORCH_CHECK(index_tensor.size(1) == codebooks.size(0), "index_tensor has ", index_tensor.size(1),
@@ -280,7 +287,7 @@ torch::Tensor spmm_csr(torch::Tensor feat, torch::Tensor indptr, torch::Tensor i
 torch::Tensor vq_decompress_spmm_csr(torch::Tensor compress_feat, torch::Tensor codebooks,
                                      torch::Tensor indptr, torch::Tensor indices, int64_t feat_dim) {
   compress_feat = dev_contig(compress_feat, "compress_feat");
-  codebooks = dev_contig(codebooks, "codebooks");
+  codebooks = beside(codebooks, compress_feat);
   TORCH_CHECK(compress_feat.dim() == 2, "compress_feat must be [rows, n_codebooks]");
   TORCH_CHECK(codebooks.dim() == 3 && codebooks.scalar_type() == torch::kFloat32,
               "VQ codebooks must be float32 [n_codebooks, K, width]");
@@ -303,7 +310,7 @@ torch::Tensor sq_decompress_spmm_csr(torch::Tensor compress_feat, torch::Tensor 
                                      int64_t column_slice, int64_t feat_dim) {
   compress_feat = dev_contig(compress_feat, "compress_feat");
   TORCH_CHECK(compress_feat.dim() == 2, "compress_feat must be 2-D");
-  codebooks = sq_codebooks_checked(codebooks);
+  codebooks = sq_codebooks_checked(codebooks, compress_feat);
   Graph g = graph_of(indptr, indices);
   c10::DeviceGuard guard(compress_feat.device());
   auto out = empty_f32({g.rows, feat_dim}, compress_feat);
@@ -764,7 +771,7 @@ torch::Tensor vq_decompress_spmm_csr_linear(torch::Tensor compress_feat, torch::
                                             torch::Tensor weight, c10::optional<torch::Tensor> bias,
                                             int64_t block_rows, bool overlap) {
   compress_feat = dev_contig(compress_feat, "compress_feat");
-  codebooks = dev_contig(codebooks, "codebooks");
+  codebooks = beside(codebooks, compress_feat);
   TORCH_CHECK(compress_feat.dim() == 2, "compress_feat must be [rows, n_codebooks]");
   TORCH_CHECK(codebooks.dim() == 3 && codebooks.scalar_type() == torch::kFloat32,
               "VQ codebooks must be float32 [n_codebooks, K, width]");
@@ -790,7 +797,7 @@ torch::Tensor sq_decompress_spmm_csr_linear(torch::Tensor compress_feat, torch::
                                             c10::optional<torch::Tensor> bias, int64_t block_rows, bool overlap) {
   compress_feat = dev_contig(compress_feat, "compress_feat");
   TORCH_CHECK(compress_feat.dim() == 2, "compress_feat must be 2-D");
-  codebooks = sq_codebooks_checked(codebooks);
+  codebooks = sq_codebooks_checked(codebooks, compress_feat);
   Graph g = graph_of(indptr, indices);
   c10::DeviceGuard guard(compress_feat.device());
   const int tag = dtype_tag(compress_feat, "compress_feat");
@@ -885,7 +892,7 @@ torch::Tensor sq_decompress_rows(torch::Tensor table, torch::Tensor index, torch
                 "slot_map must be a contiguous int32 tensor on the device of table");
   if (plain) {
     index = index.contiguous();
-    auto books = sq_codebooks_checked(codebooks);
+    auto books = sq_codebooks_checked(codebooks, table);
     c10::DeviceGuard guard(table.device());
     auto out = empty_f32({index.numel(), feat_dim}, table);
     torch::Tensor bad;
