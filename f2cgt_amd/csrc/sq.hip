@@ -441,7 +441,7 @@ int decode_f4_launch(const uint8_t* codes, float* out, const float* table, int64
   if (feat_dim % 2 != 0 || feat_dim < 8 || feat_dim > 8192 || !aligned(out, 16)) return -1;
   const size_t lds = AFFINE ? (size_t)feat_dim * 8
                             : ((((size_t)n_cb << BITS) + 3) / 4 * 4 + (size_t)feat_dim) * 4;
-  if (lds > (size_t)kMaxLutBytes) return -1;
+  if (lds + (ids != nullptr ? kSpanRows * sizeof(int64_t) : 0) > (size_t)kMaxLutBytes) return -1;   // (s_rows)
   F4Args a{};
   if (ids != nullptr) a = *ids;
   a.codes = codes; a.out = out; a.table = table;

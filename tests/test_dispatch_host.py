@@ -236,3 +236,12 @@ def test_dealt_items_and_column_form_of_one_codebook():
         assert block(120000, 300, 1, bits=bits) == 256           # wider rows
         assert block(480000, 128, 1, bits=bits) == 256           # streamed output (246 MB)
     assert block(100000, 32, 1, bits=2) == 256                   # fewer values
+
+
+def test_decode_through_a_row_list_counts_its_row_table():
+    """The looked-up rows (8.2 KB) lie in LDS beside the decode table: past 64 KB together the shape is left to fetch and
+    decode, refused before a launch.  (The admitted side, one codebook less, runs in the GPU tests.)"""
+    lib = capi.lib()
+    for feat_dim, n_cb in ((540, 54), (610, 61), (620, 62)):
+        assert lib.f2cgt_sq_decompress_rows(A16, capi.DT_I8, A16, capi.DT_I64, None, 0, None, A16, A16, 4, 100, feat_dim, feat_dim,
+                                            n_cb, 8, 10, None) == -2

@@ -36,7 +36,8 @@ def test_vq_rows(n, dim, w, k, dtype):
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("bits", [1, 2, 4, 8])
 @pytest.mark.parametrize("n,dim,slice_", [(1, 8, 8), (7, 10, 16), (1025, 128, 128), (3, 602, 608), (4001, 100, 32), (900, 30, 8), (64, 7, 8),
-                                          (2049, 8, 8), (3001, 10, 16), (5001, 154, 160)])   # most rows to a workgroup; an odd count of them
+                                          (2049, 8, 8), (3001, 10, 16), (5001, 154, 160),    # most rows to a workgroup; an odd count of them
+                                          (501, 530, 10), (501, 540, 10), (501, 610, 10), (501, 620, 10)])   # 8 bits: both sides of the LDS budget
 def test_sq_rows(n, dim, slice_, bits, dtype):
     print("case sq_rows", n, dim, slice_, bits, dtype, flush=True)
     lib = f2cgt_amd.load()
