@@ -330,7 +330,12 @@ def vq_metadata(features, n_clusters, column_slice, hotness=None, sample_index=N
     if sample_index is None:
         sample_index = sampling(150_000, num_items, hotness)
     num_slice = (feat_dim + column_slice - 1) // column_slice
-    codebooks = _train_all_slices(features, n_clusters, column_slice, sample_index, max_iter)
+    draws = torch.get_rng_state()
+    try:
+        codebooks = _train_all_slices(features, n_clusters, column_slice, sample_index, max_iter)
+    except torch.OutOfMemoryError:        # no room for the sample's slices side by side: one at a time, with the same draws
+        codebooks = None
+        torch.set_rng_state(draws)
     if codebooks is None:
         codebooks = torch.zeros((num_slice, n_clusters, column_slice), device="cuda", dtype=torch.float32)
         per_slice = range(num_slice)

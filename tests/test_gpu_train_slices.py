@@ -176,3 +176,28 @@ def test_vq_metadata_refuses_ids_outside():
     x = torch.randn((500, 16), device="cuda")
     with pytest.raises(IndexError):
         pipeline.vq_metadata(x, 8, 8, sample_index=torch.tensor([1, 2, 500]))
+
+
+@pytest.mark.parametrize("where", ["device", "host"])
+def test_vq_metadata_without_room_for_the_sample(where):
+    """The sample of all slices does not fit: slice by slice, with the same draws."""
+    x = torch.randn((60_000, 512), generator=torch.Generator().manual_seed(1))
+    x = x.cuda() if where == "device" else x
+    rows = torch.arange(0, 60_000)
+
+    def train():
+        torch.manual_seed(3)
+        return pipeline.vq_metadata(x, 16, 16, sample_index=rows, max_iter=1)
+
+    want = train()
+    after = torch.rand(1)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.mem_get_info()[1]
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)    # the sample: 123 MB
+    try:
+        got = train()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(after, torch.rand(1))
+    assert torch.allclose(got, want, rtol=0, atol=2e-5)
