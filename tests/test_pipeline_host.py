@@ -20,6 +20,16 @@ def test_sq_metadata_is_the_reference_codebook_statement():
         assert np.isclose(got[4], want[4], rtol=1e-6)
 
 
+def test_log2_of_a_codebook_is_correctly_rounded():
+    """As the device makes it, so that sq_metadata and sq_compress agree on the same sample."""
+    values = np.exp(np.random.default_rng(1).uniform(np.log(1e-5), np.log(1e3), 20000)).astype(np.float32)
+    want = np.log2(values.astype(np.float64)).astype(np.float32)
+    got = [pipeline._sq_codebook(v, v, torch.tensor(1.0)) for v in values]
+    assert np.array_equal([np.float32(b[2]) for b in got], want)
+    top = np.log2(np.maximum(values, np.float32(2e-5)).astype(np.float64)).astype(np.float32) + np.float32(1e-5)
+    assert np.array_equal([np.float32(b[3]) for b in got], top)
+
+
 def test_normalize_rescales_rows_to_the_mean_norm():
     x = torch.tensor([[3.0, 4.0], [0.0, 1.0], [6.0, 8.0]])
     y = pipeline.normalize(x)
