@@ -584,14 +584,22 @@ int run(Dec dec, const void* indptr, const void* indices, int idx_dtype, typenam
 
 // Plain features: a group is as wide as a row needs (a row of 4 k columns takes D / 4 lanes).  Rows of four lanes and
 // fewer stay with the skeleton: eight rows in flight need ids for eight edges from one load of the group.  So do rows
-// beyond what the grid counts in.
+// beyond what the grid counts in, and graphs with up to 2.25 edges per row: there a row is a chain of offsets, ids and
+// source rows that handing the ids round only makes longer (skeleton -> groups that hand round, 30 000 rows of one edge:
+// 128 columns 6.5 -> 8.5 us, 602 columns 30.6 -> 41.6, 128 columns of fp16 13.9 -> 19.4; of two 7.5 -> 9.0, 42.3 -> 43.7,
+// 16.3 -> 20.4; of up to five, 2.5 on average, 10.4 -> 10.2, 57 -> 46, 20.9 -> 20.5; of three 11.5 -> 11.5, 55 -> 51,
+// 19.1 -> 21.7; power-law rows, 2.6 on average, 0.7 to 1.0 of the skeleton's time).  Where more than a third of the lanes
+// of four columns idle, up to three edges per row (154 columns, 39 of 64 lanes: of three 16.8 -> 20.8; of four 20.4 ->
+// 23.6, from 200 000 rows on level; of up to eight 0.9 of the time.  300 columns, 75 of 128 lanes: of three level).
 constexpr int64_t kPlainBlocks = 1 << 15;   // row blocks of the grid; more rows go round
 template <class Dec>
 int run_plain(Dec dec, const void* indptr, const void* indices, int idx_dtype, typename Dec::Out* out, int64_t R, int64_t E,
               int64_t N, int feat_dim, bool vec_ok, hipStream_t st, const char* what) {
   const Geometry g = plan(R, feat_dim, 1, Dec::NOUT, 0);
   const int64_t passes = ceil_div(feat_dim, (int64_t)g.G * Dec::NOUT);
-  if (g.G < kPlainUnroll || passes > 65535)
+  const int64_t idle = passes * g.G - ceil_div(feat_dim, Dec::NOUT);
+  const bool sparse = 4 * E <= 9 * R || (Dec::NOUT == 4 && E <= 3 * R && 3 * idle > passes * g.G);
+  if (g.G < kPlainUnroll || passes > 65535 || sparse)
     return run(dec, indptr, indices, idx_dtype, out, R, E, N, feat_dim, g, 0, vec_ok, st, what);
   const int64_t blocks = ceil_div(R, 256 / g.G);
   const dim3 grid((unsigned)passes, (unsigned)(blocks < kPlainBlocks ? blocks : kPlainBlocks));

@@ -245,3 +245,16 @@ def test_decode_through_a_row_list_counts_its_row_table():
     for feat_dim, n_cb in ((540, 54), (610, 61), (620, 62)):
         assert lib.f2cgt_sq_decompress_rows(A16, capi.DT_I8, A16, capi.DT_I64, None, 0, None, A16, A16, 4, 100, feat_dim, feat_dim,
                                             n_cb, 8, 10, None) == -2
+
+
+def test_plain_rows_of_few_edges_stay_with_the_skeleton():
+    def kernel(rows, edges, dim, dtype=capi.DT_F32):
+        rc, plan = capi.dry_run("f2cgt_spmm_csr", A16, dtype, A16, A16, A16, capi.DT_I64, rows, edges, 100_000, dim, None)
+        assert rc == 0
+        return plan.kernel.decode()
+    for dtype, dim in ((capi.DT_F32, 128), (capi.DT_F32, 602), (capi.DT_F32, 33), (capi.DT_F16, 64), (capi.DT_F64, 64)):
+        assert kernel(1000, 2250, dim, dtype) == "agg_kernel" and kernel(1000, 2251, dim, dtype) == "agg_plain_kernel"
+        assert kernel(1000, 0, dim, dtype) == "agg_kernel"
+    # 39 of 64 lanes of four columns: up to three
+    assert kernel(1000, 3000, 154) == "agg_kernel" and kernel(1000, 3001, 154) == "agg_plain_kernel"
+    assert kernel(1000, 9000, 24) == "agg_plain_kernel" and kernel(1000, 9000, 16) == "agg_kernel"

@@ -34,9 +34,23 @@ def test_more_rows_than_the_grid_has_groups():
     assert torch.equal(f2cgt_amd.load().spmm_csr(feat, indptr, indices), feat[indices])
 
 
+# the same three times over: rows of three edges, which the groups that hand the ids round take
+def test_more_rows_of_three_edges_than_the_grid_has_groups():
+    rows, dim = (1 << 15) * 8 + 37, 128
+    feat = 3.0 * torch.randint(-1000, 1000, (64, dim), device="cuda")          # exact sums and means
+    indptr = torch.arange(0, 3 * rows + 1, 3, device="cuda")
+    a = torch.randint(0, 64, (rows, 3), device="cuda")
+    got = f2cgt_amd.load().spmm_csr(feat, indptr, a.flatten())
+    assert torch.equal(got, (feat[a[:, 0]] + feat[a[:, 1]] + feat[a[:, 2]]) / 3)
+
+
 def test_infinities_and_nans_stay_in_their_rows():
     feat = torch.zeros((4, 100), device="cuda")
     feat[1, 3], feat[2, 4] = float("inf"), float("nan")
     got = f2cgt_amd.load().spmm_csr(feat, torch.tensor([0, 2, 2, 4], device="cuda"), torch.tensor([0, 1, 3, 2], device="cuda"))
+    assert torch.isinf(got[0, 3]) and torch.isnan(got[2, 4])
+    assert int((got != 0).sum()) == 2
+    got = f2cgt_amd.load().spmm_csr(feat, torch.tensor([0, 4, 4, 9], device="cuda"),
+                                    torch.tensor([0, 1, 0, 0, 3, 2, 0, 3, 0], device="cuda"))   # three edges per row and more
     assert torch.isinf(got[0, 3]) and torch.isnan(got[2, 4])
     assert int((got != 0).sum()) == 2
