@@ -1339,13 +1339,15 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
   // shape: 845 -> 405 us); from about 8 edges per row the detour through LDS costs more than it saves
   a.dense_store = avg_deg <= 8.0;
   // Above that (up to 16 edges per row, four-row mini-blocks) the form is chosen by what binds the launch:
-  //  * a code table beyond the 256 MB last-level cache, rows of one to four whole column lines (feat_dim a multiple of 32,
-  //    at most 512) and an output of 32 MB and more: through LDS.  A minibatch finds neither its ids nor its output's lines
-  //    in the caches, and then a store instruction that writes half lines waits longest (four graphs in turn, skewed /
-  //    uniform ids, plain -> LDS: 16 x 8 at 15 edges per row from 480 MB 130 -> 117 / 205 -> 193 us, at 12 21.1 -> 20.0 /
-  //    40.0 -> 38.0; 16 x 16 at 10 64 -> 52 / 103 -> 92; 32 x 16 at 10 from 640 MB 43.6 -> 31.6 / 58.0 -> 54.5, at 15 253 ->
-  //    223 / 312 -> 289; an output of 24 MB 14.0 -> 13.8).  One graph again and again 63 -> 52 (16 x 16), 43 -> 35 (32 x 16),
-  //    85 -> 93 (16 x 8 at 15, skewed; uniform 204 -> 191).  304 columns 45 -> 50: rows that end inside a line stay as they are;
+  //  * a code table beyond the 256 MB last-level cache and 128, 256 or 512 columns: through LDS where that is ahead whatever
+  //    the ids (Zipf(1.1) or uniform) and whether one graph and output come again or four in turn.  128 columns from 60 MB of
+  //    output on (tables of 280, 480 and 1600 MB; the time through LDS 0.75 to 1.0 of the plain one's, 1.03 to 1.08 in a few of
+  //    one to two hundred; 16 x 8 at 15 edges per row, 240 MB: one graph 84 -> 80 us / uniform 200 -> 187, in turn 122 -> 111 /
+  //    199 -> 187; outputs of 40 and 50 MB up to 1.07).  256 columns from 60 to 160 MB and up to 10 edges per row (16 x 16 at 10,
+  //    100 MB 0.74 to 0.92; at 200 to 420 MB up to 1.10, at 12 edges per row up to 1.14).  512 columns from 96 MB on and up
+  //    to 11 edges per row (16 x 32 at 10, 240 MB: one graph 96 -> 53 / 79 -> 73, in turn 95 -> 53 / 113 -> 106; uniform ids up to
+  //    1.06 at single sizes where the others gain 1.3 and more; 64 MB in turn 1.09, 14 edges per row up to 1.14).  Other widths lose up to 1.2 with ids that keep to a few rows, which the caches then hold,
+  //    at any size of output (160, 224, 320, 384, 448 columns), and stay as they are;
   //  * a code table of 192 to 256 MB, or rows of more than four column tiles: the results are stored as they are (24 x 32
   //    at 12 edges per row from 240 MB, graphs in turn: 193 us, 208 through LDS; from 120 MB 178 against 195).  From 5.8 GB
   //    at 10 per row one graph again and again takes 420 us, 442 through LDS, and graphs in turn 681 against 585:
@@ -1368,8 +1370,10 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
   const bool big_table = a.N * (int64_t)a.n_cb > (256ll << 20);
   if (!a.dense_store && a.feat_dim % 8 == 0 && rpm4) {
     const bool cached_table = a.N * (int64_t)a.n_cb <= (192ll << 20);
-    if (store_mode() == F2CGT_STORE_STREAM ||
-        (big_table && a.feat_dim >= 128 && a.feat_dim % 32 == 0 && a.n_tiles <= 4 && out_bytes >= (32ll << 20))) {
+    const bool lines = (a.feat_dim == 128 && out_bytes >= (60ll << 20)) ||
+                       (a.feat_dim == 256 && out_bytes >= (60ll << 20) && out_bytes <= (160ll << 20) && avg_deg <= 10.0) ||
+                       (a.feat_dim == 512 && out_bytes >= (96ll << 20) && avg_deg <= 11.0);
+    if (store_mode() == F2CGT_STORE_STREAM || (big_table && lines)) {
       a.dense_store = 1;
     } else if (cached_table && a.feat_dim >= 128 && a.n_tiles <= 4) {
       const bool big_out = out_bytes >= (200ll << 20);
@@ -1448,16 +1452,20 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
     // 7 x 32 180 / 96 against 192 / 103).
     // Above that, rows that are no whole 64-byte pieces (feat_dim an odd multiple of 8): the same, where the eight-column
     // form has no exchange (more than four column tiles, or a table beyond the last-level cache) from 100 MB of output on,
-    // else from the size of the last-level cache on; up to 12 edges per row, and up to 16 from a table beyond that cache.
-    // Graphs in turn, skewed / uniform ids, eight-column form -> this: 19 x 32 at 600 columns, 9 edges per row, 457 MB
-    // 223 -> 144 / 180 -> 145 us, 12 per row, 114 MB 52 -> 44 / 51 -> 45, 16 per row from 362 MB of codes 60 -> 58 / 91 -> 85;
-    // 712 columns 127 -> 96 / 126 -> 100; 25 x 8 at 200, 305 MB, 9 per row 127 -> 112 / 173 -> 151, 12 per row 119 -> 117 /
-    // 206 -> 192; 152 columns 183 -> 163 / 199 -> 182.  At 13 and more from a small table it is ahead with uniform ids only
-    // (200 columns 214 -> 172, skewed 123 -> 132), below those sizes level; one tile loses (104 columns 82 -> 96), and so do
-    // rows of whole 64-byte pieces (304 columns 97 -> 108, 144 columns 137 -> 149).
-    const bool split_rows = a.feat_dim % 16 == 8 && a.n_tiles > 1 && rpm4 && store_mode() != F2CGT_STORE_STREAM &&
-                            out_bytes >= (a.n_tiles > 4 || big_table ? 100000000ll : 256ll << 20) &&
-                            (avg_deg <= 12.0 || big_table);
+    // else from the size of the last-level cache on.  A last tile of few columns leaves most lanes of its workgroups idle,
+    // which counts for more the fewer tiles there are and the longer the rows (one graph again and again, Zipf(1.1) ids, this
+    // form's time over the other's: 136 columns at 9 to 14 edges per row 1.08 to 1.15, 152 at 9 to 12 up to 1.08, 264 up to
+    // 1.10; 168 columns at 12 up to 1.02, at 14 1.06 to 1.10; 200 at 14 up to 1.14; 520 and 648 at 14 1.06): up to 12 edges per
+    // row it is taken from 40 columns in the last tile on, or with more than three tiles, above that, up to 16 from a table
+    // beyond the last-level cache, from 80 on, 56 with more than three tiles.  Four graphs in turn, Zipf(1.1) / uniform ids,
+    // eight-column form -> this: 200 columns, 305 MB, at 10 126 -> 112 / 186 -> 172 us, at 12 118 -> 114 / 211 -> 199; from
+    // 480 MB of codes at 10 157 -> 136 / 223 -> 194; 600 columns, 457 MB, at 9 216 -> 149 / 181 -> 141, 114 MB at 12 51 -> 41 / 50 -> 42;
+    // 712 columns, 200 MB, at 10 90 -> 68 / 81 -> 65; 504 columns from 480 MB of codes at 14 0.70 of the time / 0.89.  One tile
+    // loses (104 columns 82 -> 96), and so do rows of whole 64-byte pieces (304 columns 97 -> 108, 144 columns 137 -> 149).
+    const int tail = a.feat_dim % 128;
+    const bool filled = avg_deg <= 12.0 ? tail >= 40 || a.n_tiles > 3 : big_table && tail >= (a.n_tiles > 3 ? 56 : 80);
+    const bool split_rows = a.feat_dim % 16 == 8 && a.n_tiles > 1 && rpm4 && filled && store_mode() != F2CGT_STORE_STREAM &&
+                            out_bytes >= (a.n_tiles > 4 || big_table ? 100000000ll : 256ll << 20);
     if ((avg_deg <= 8.0 && a.feat_dim % 32 != 0) || split_rows) {
       a.dense_store = 0;
       a.own_lg = 0;

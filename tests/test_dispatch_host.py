@@ -202,19 +202,28 @@ def test_fused_vq_forms_for_tables_beyond_the_last_level_cache_and_rows_of_split
                              rows * fanout, n_src, d, n_cb, 256, w, None)
         assert rc == 0 and p.kernel.decode() == "vq_wave_kernel"
         return p.aux[0], p.aux[2]          # float4 per lane and edge, store form
-    # a table of more than 256 MB: through LDS from 32 MB of output on, up to four column tiles of whole lines
-    assert plan(65_536, 15, 128, 16, 8, 16_777_217) == (2, 1)
-    assert plan(65_535, 15, 128, 16, 8, 16_777_217) == (2, 0)
-    assert plan(65_536, 15, 128, 16, 8, 16_777_216) == (2, 0)
-    assert plan(65_536, 15, 512, 32, 16, 10_000_000) == (2, 1)
-    assert plan(65_536, 15, 544, 34, 16, 10_000_000) == (2, 0)
-    assert plan(65_536, 15, 304, 19, 16, 20_000_000) == (2, 0)
-    assert plan(65_536, 17, 128, 16, 8, 16_777_217) == (2, 0)
+    # a table of more than 256 MB: through LDS where that is ahead with any ids, warm and in turn
+    assert plan(122_880, 15, 128, 16, 8, 16_777_217) == (2, 1)      # 60 MB
+    assert plan(122_879, 15, 128, 16, 8, 16_777_217) == (2, 0)
+    assert plan(122_880, 15, 128, 16, 8, 16_777_216) == (2, 0)
+    assert plan(122_880, 17, 128, 16, 8, 16_777_217) == (2, 0)
+    assert plan(61_440, 10, 256, 16, 16, 20_000_000) == plan(163_840, 10, 256, 32, 8, 20_000_000) == (2, 1)   # 60 to 160 MB
+    assert plan(61_439, 10, 256, 16, 16, 20_000_000) == plan(163_841, 10, 256, 16, 16, 20_000_000) == (2, 0)
+    assert plan(100_000, 11, 256, 16, 16, 20_000_000) == (2, 0)
+    assert plan(49_152, 11, 512, 16, 32, 20_000_000) == plan(400_000, 9, 512, 64, 8, 5_000_000) == (2, 1)
+    assert plan(49_151, 11, 512, 16, 32, 20_000_000) == plan(49_152, 12, 512, 16, 32, 20_000_000) == (2, 0)
+    for dim in (160, 192, 224, 304, 320, 384, 416, 448, 480, 544, 768):
+        assert plan(300_000, 10, dim, dim // 8, 8, 20_000_000) == (2, 0)
     # odd multiples of eight columns: one float4 per lane
     assert plan(41_667, 12, 600, 19, 32, 1_000_000) == (1, 0)
     assert plan(41_666, 12, 600, 19, 32, 1_000_000) == (2, 0)
     assert plan(41_667, 13, 600, 19, 32, 1_000_000) == (2, 0)
     assert plan(41_667, 16, 600, 19, 32, 15_000_000) == (1, 0)
+    # a last tile of few columns leaves the lanes of its workgroups idle
+    for dim, up_to in ((136, 8), (152, 8), (168, 12), (200, 12), (216, 16), (264, 8), (280, 8), (296, 12), (328, 12), (360, 16),
+                       (392, 12), (456, 16), (504, 16), (520, 12), (568, 16), (648, 12), (712, 16), (760, 16)):
+        forms = [plan(300_000, fanout, dim, -(-dim // 8), 8, 30_000_000)[0] for fanout in (8, 9, 12, 13, 16, 17)]
+        assert forms == [1 if fanout <= up_to else 2 for fanout in (8, 9, 12, 13, 16, 17)], dim
     assert plan(335_545, 12, 200, 25, 8, 1_000_000)[0] == 1 and plan(335_544, 12, 200, 25, 8, 1_000_000)[0] == 2
     assert plan(125_000, 12, 200, 25, 8, 12_000_000)[0] == 1
     assert plan(700_000, 9, 104, 13, 8, 1_000_000)[0] == 2          # one column tile

@@ -10,7 +10,9 @@ pytestmark = pytest.mark.gpu
 # rows of 600 and 680 columns and an output of 100 MB; 200 columns, an output beyond the last-level cache; a table beyond it
 @pytest.mark.parametrize("n_src,books,width,dim,rows,fanout", [(3000, 19, 32, 600, 41_667, 12), (3000, 85, 8, 680, 36_765, 9),
                                                                (3000, 25, 8, 200, 335_545, 10), (16_777_217, 16, 8, 128, 65_537, 15),
-                                                               (16_777_217, 25, 8, 200, 125_001, 13)])
+                                                               (16_777_217, 25, 8, 200, 125_001, 12), (16_777_217, 27, 8, 216, 115_741, 13),
+                                                               (16_777_217, 16, 8, 128, 122_881, 15), (16_777_217, 17, 16, 256, 61_441, 10),
+                                                               (8_388_609, 33, 16, 512, 49_153, 11), (16_777_217, 25, 8, 200, 125_001, 13)])
 @pytest.mark.parametrize("ragged", [False, True])
 def test_store_forms_agree_with_the_unfused_operators(n_src, books, width, dim, rows, fanout, ragged):
     capi = f2cgt_amd.load()
