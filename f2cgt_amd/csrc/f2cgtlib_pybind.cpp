@@ -859,7 +859,8 @@ torch::Tensor vq_decompress_rows(torch::Tensor table, torch::Tensor index, torch
                      codebooks.device() == table.device() && table.dim() == 2 && table.is_contiguous() && index.dim() == 1 &&
                      codebooks.dim() == 3 && table.scalar_type() == torch::kUInt8 && codebooks.scalar_type() == torch::kFloat32 &&
                      (index.scalar_type() == torch::kInt64 || index.scalar_type() == torch::kInt32) &&
-                     table.size(0) > 0 && table.size(1) == codebooks.size(0) && feat_dim >= 0;
+                     table.size(0) > 0 && table.size(1) == codebooks.size(0) &&
+                     index.numel() >= 1024 && feat_dim >= 64 && feat_dim % 2 == 0;   // (others would be refused after an allocation: 1 us)
   if (plain) {
     index = index.contiguous();
     codebooks = codebooks.contiguous();
@@ -884,7 +885,7 @@ torch::Tensor sq_decompress_rows(torch::Tensor table, torch::Tensor index, torch
   const bool plain = table.defined() && index.defined() && table.is_cuda() && index.device() == table.device() && table.dim() == 2 &&
                      table.is_contiguous() && index.dim() == 1 && table.size(0) > 0 &&
                      (table.scalar_type() == torch::kInt8 || table.scalar_type() == torch::kUInt8) &&
-                     (index.scalar_type() == torch::kInt64 || index.scalar_type() == torch::kInt32) && feat_dim >= 0;
+                     (index.scalar_type() == torch::kInt64 || index.scalar_type() == torch::kInt32) && feat_dim >= 8 && feat_dim % 2 == 0;
   const bool mapped = slot_map.has_value();
   if (mapped)
     TORCH_CHECK(slot_map->device() == table.device() && slot_map->dim() == 1 && slot_map->is_contiguous() &&
