@@ -924,8 +924,16 @@ torch::Tensor sq_decompress_rows(torch::Tensor table, torch::Tensor index, torch
     }
   }
   if (mapped) {
-    auto slots = slot_map->index({index.to(torch::kInt64)}).to(torch::kInt64);
-    if (check && slots.lt(0).any().item<bool>()) throw py::key_error("a requested id is not a seed row");
+    // ids are held to the map, as in the kernel: an index beyond it would end the process
+    auto ids = index.to(slot_map->device(), torch::kInt64);
+    ids = torch::where(ids.lt(0), ids.add(slot_map->numel()), ids);
+    auto held = ids.clamp(0, slot_map->numel() - 1);
+    auto slots = slot_map->index({held}).to(torch::kInt64);
+    if (check) {
+      auto seen = torch::stack({ids.ne(held).any(), slots.lt(0).any()}).cpu();
+      if (seen.data_ptr<bool>()[0]) throw py::index_error("an id lies outside the slot map");
+      if (seen.data_ptr<bool>()[1]) throw py::key_error("a requested id is not a seed row");
+    }
     index = slots;
   } else if (index.scalar_type() != torch::kInt64 && index.scalar_type() != torch::kInt32) {
     index = index.to(torch::kInt64);

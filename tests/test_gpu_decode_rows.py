@@ -80,11 +80,20 @@ def test_seed_lookup(dim, bits, dtype):
     assert torch.equal(got[6:], want[6:]) and torch.equal(got[5], manager._decompress(0, manager.seeds_data[pick[:1] * 0])[0])
 
 
-def test_ids_outside_the_seed_map():
+# 7 columns: looked up with torch, fetched and decoded
+@pytest.mark.parametrize("dim", [8, 7])
+def test_ids_outside_the_seed_map(dim):
     lib = f2cgt_amd.load()
-    table = torch.zeros((10, 8), dtype=torch.int8, device="cuda")
+    table = torch.arange(80, dtype=torch.int8, device="cuda").view(10, 8)[:, :dim].contiguous()
     slots = torch.arange(10, dtype=torch.int32, device="cuda")
+    slots[3] = -1
     cb = torch.tensor([[0.01, 3.0, -6.6, 1.6, 0.8]], device="cuda")
     for bad in (10, -11, 2 ** 40):
         with pytest.raises(IndexError):
-            lib.sq_decompress_rows(table, torch.tensor([1, bad, 2]).cuda(), cb, 8, 8, 8, slots, True)
+            lib.sq_decompress_rows(table, torch.tensor([1, bad, 2]).cuda(), cb, 8, 8, dim, slots, True)
+        got = lib.sq_decompress_rows(table, torch.tensor([1, bad, -8]).cuda(), cb, 8, 8, dim, slots, False)
+        assert torch.equal(got[::2], lib.sq_decompress(table[1:3], cb, 8, 8, dim)) and bool(torch.isfinite(got).all())
+    with pytest.raises(KeyError):
+        lib.sq_decompress_rows(table, torch.tensor([1, 3], dtype=torch.int32).cuda(), cb, 8, 8, dim, slots, True)
+    empty = torch.empty((0,), dtype=torch.int64, device="cuda")
+    assert lib.sq_decompress_rows(table, empty, cb, 8, 8, dim, slots, True).shape == (0, dim)
