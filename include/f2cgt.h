@@ -273,7 +273,9 @@ int f2cgt_pairwise_distance(const float* x, const float* y, float* dist, int64_t
  * the callers run on pairwise_distance (examples/my_kmeans.py:116-125).
  * x fp32 [m,k], centers fp32 [n,k], n <= 65536.  Writes the index of the nearest centre
  * (first minimum) to labels_i64 [m] and/or labels_u8 [m] (either may be NULL; labels_u8
- * needs n <= 256).  The distance matrix is never materialised. */
+ * needs n <= 256).  The distance matrix is never materialised.  Cosine: the nearest by direction; the 1e-8 below which
+ * f2cgt_pairwise_distance does not let |x||y| fall counts only between centres whose directions are equally near to
+ * rounding. */
 int f2cgt_kmeans_predict(const float* x, const float* centers, int64_t* labels_i64,
                          uint8_t* labels_u8, int64_t m, int64_t n, int64_t k, int metric,
                          void* stream);
@@ -335,7 +337,8 @@ int f2cgt_kmeans_update_static(const float* x, const int64_t* labels_i64, const 
  * f2cgt_kmeans_slices_step: one Lloyd iteration of every slice whose stop flag is zero, as f2cgt_kmeans_predict and
  * f2cgt_kmeans_update would make it from the rows kept: x fp32 [slices, m, k], keep as above or NULL (all), centers fp32
  * [slices, n, k] updated in place, stop int32 [slices] (device) with stop_rule and tol as in f2cgt_kmeans_update.  A label
- * is the true first minimum; the sums are fp32, a workgroup's rows added in LDS, the sets in a fixed order.
+ * is the true first minimum.  Sums: a workgroup's rows in fp64 (LDS), each workgroup's set rounded to fp32 once, the sets
+ * added in fp64 in a fixed order.
  * workspace: f2cgt_kmeans_slices_workspace_bytes, 16-byte aligned.  f2cgt_kmeans_slices_covers: 1 where the shape is
  * taken (operands and sums of a slice in LDS, up to 256 slices, 512 centres, 64 columns), else 0. */
 int f2cgt_slice_rows(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols, int64_t k,

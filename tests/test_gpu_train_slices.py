@@ -53,9 +53,10 @@ def test_keep_rows(m, width, last):
     assert not lib.keep_rows(norms, stats, places[0][2], places[1][2])[1].any()
 
 
-def step64(x, keep, centers, metric):
-    """One Lloyd step of a slice in float64."""
+def step64(x, keep, centers, metric, values=None):
+    """One Lloyd step of a slice in float64: the means of the rows, or of `values` in their places, by label."""
     x, c = x.astype(np.float64), centers.astype(np.float64)
+    values = x if values is None else values.astype(np.float64)
     if metric == "cosine":
         d = 1.0 - (x @ c.T) / np.maximum(np.linalg.norm(x, axis=1)[:, None] * np.linalg.norm(c, axis=1)[None], 1e-8)
     else:
@@ -65,7 +66,7 @@ def step64(x, keep, centers, metric):
     for j in range(c.shape[0]):
         mine = keep & (label == j)
         if mine.any():
-            new[j] = x[mine].mean(0)
+            new[j] = values[mine].mean(0)
     return new
 
 
@@ -93,8 +94,24 @@ def test_one_step(metric, slices, m, n, k, masked):
     assert flags.tolist() == [0] * slices
     for s in range(slices):
         want = step64(x[s], keep[s], c[s], metric)
-        # fp32 sums of r rows of unit variance: r^2 2^-24 |x| at the very most, over r rows
-        assert np.abs(got[s] - want).max() <= 6e-8 * 5.0 * max(2, m / n * 8)
+        # each set's fp64 sums are rounded once, which makes 2^-24 of the mean of |x| at most, their total and its
+        # quotient once more each
+        bound = 1.01 * 2.0 ** -24 * (step64(x[s], keep[s], c[s], metric, np.abs(x[s])) + 2 * np.abs(want))
+        assert (np.abs(got[s] - want) <= bound).all()
+
+
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+def test_sums_hold_more_than_fp32(metric):
+    """Rows of one value that an fp32 sum beyond 256 rounds down every time: 2^-24 100 of the mean and more, where each of a
+    workgroup's sums has some 600 rows."""
+    value = 1.0 + 0.4 * 2.0 ** -15
+    x = torch.full((1, 300_000, 5), value)
+    x[:, ::2] *= -1.0
+    centers = torch.tensor([[[1.0] * 5, [-1.0] * 5]]).cuda()
+    f2cgt_amd.load().kmeans_slices_fit(x.cuda(), None, centers, metric, 0, 0.0, 1.0, 1, 8)
+    want = float(np.float32(value))
+    got = centers.cpu().double()[0]
+    assert (got[0] - want).abs().max() <= 3.03 * 2.0 ** -24 * want and (got[1] + want).abs().max() <= 3.03 * 2.0 ** -24 * want
 
 
 @pytest.mark.parametrize("metric", ["cosine", "l2"])
