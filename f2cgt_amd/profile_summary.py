@@ -217,10 +217,10 @@ def main(argv):
             fh.write("\n")
     A = "python3 bench.py --all --steps 200 --warmup 20 --cpu-seconds 0"
     tall = os.path.join(O, "trace_all")
-    k = kstats(tall, "assign_kernel<2, 4, true>")
+    k = kstats(tall, "assign_kernel<2, 4, true, false>")
     if k:
         with open(os.path.join(P, "assign_kernel_c5_encode.md"), "w") as fh:
-            fh.write("# assign_kernel<2, 4, true> on the C5 encode step (1e6 x 32 fp32 vs 256 centres, squared L2 + arg-min)\n\n")
+            fh.write("# assign_kernel<2, 4, true, false> on the C5 encode step (1e6 x 32 fp32 vs 256 centres, squared L2 + arg-min)\n\n")
             fh.write("Commands (separate runs):\n\n")
             fh.write("    rocprofv3 --kernel-trace --stats --output-format csv -d out/trace_all -o t -- %s\n" % A)
             fh.write("    rocprofv3 --pmc SQ_INSTS_VALU_MFMA_MOPS_F16 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_INSTS_MFMA "
@@ -232,7 +232,7 @@ def main(argv):
                      "product block (two fp16 pieces per value), i.e. %.0f TFLOP/s of fp16 MFMA = %.3f of the 2500 TFLOP/s "
                      "peak.\n\n" % (fl, fl / (k[2] * 1e-6) / 1e12, 3 * fl / (k[2] * 1e-6) / 1e12,
                                          3 * fl / (k[2] * 1e-6) / 1e12 / 2500))
-            vals = counters(os.path.join(O, "mfma_all"), "assign_kernel<2, 4, true>")
+            vals = counters(os.path.join(O, "mfma_all"), "assign_kernel<2, 4, true, false>")
             if vals:
                 fh.write("| counter (mean per dispatch) | value |\n|---|---|\n")
                 for cn in sorted(vals):
@@ -241,26 +241,28 @@ def main(argv):
                     util = vals["SQ_VALU_MFMA_BUSY_CYCLES"][0] / N_SIMD / (vals["GRBM_GUI_ACTIVE"][0] / N_XCD)
                     fh.write("\nMFMA utilisation = SQ_VALU_MFMA_BUSY_CYCLES / %d SIMDs / (GRBM_GUI_ACTIVE / %d XCDs) = %.3f\n"
                              % (N_SIMD, N_XCD, util))
-        k = kstats(tall, "pairwise_split_kernel<2, 2>")
-        if k:
-            with open(os.path.join(P, "pairwise_split_kernel_c5_encode_shape.md"), "w") as fh:
-                fh.write("# pairwise_split_kernel<2, 2> (pairwise_distance) at the C5 encode shape: 1e6 x 32 against 256 rows, L2 and cosine\n\n")
-                fh.write("    rocprofv3 --kernel-trace --stats --output-format csv -d out/trace_all -o t -- %s\n\n" % A)
-                fh.write("| kernel | calls | avg us | min us | max us |\n|---|---|---|---|---|\n")
-                fh.write("| `%s` | %d | %.2f | %.2f | %.2f |\n\n" % (k[0][:60], k[1], k[2], k[3], k[4]))
-                nb = 1e6 * 256 * 4
-                fh.write("The [1e6, 256] fp32 matrix is %.0f MB: %.0f GB/s of matrix write = %.2f of the 8 TB/s peak (both "
-                         "metrics in one average).\n" % (nb / 1e6, nb / (k[2] * 1e-6) / 1e9, nb / (k[2] * 1e-6) / 8e12))
+    k = kstats(tall, "pairwise_split_kernel<2, 2>")
+    if k:
+        with open(os.path.join(P, "pairwise_split_kernel_c5_encode_shape.md"), "w") as fh:
+            fh.write("# pairwise_split_kernel<2, 2> (pairwise_distance) at the C5 encode shape: 1e6 x 32 against 256 rows, L2 and cosine\n\n")
+            fh.write("    rocprofv3 --kernel-trace --stats --output-format csv -d out/trace_all -o t -- %s\n\n" % A)
+            fh.write("| kernel | calls | avg us | min us | max us |\n|---|---|---|---|---|\n")
+            fh.write("| `%s` | %d | %.2f | %.2f | %.2f |\n\n" % (k[0][:60], k[1], k[2], k[3], k[4]))
+            nb = 1e6 * 256 * 4
+            fh.write("The [1e6, 256] fp32 matrix is %.0f MB: %.0f GB/s of matrix write = %.2f of the 8 TB/s peak (both "
+                     "metrics in one average).\n" % (nb / 1e6, nb / (k[2] * 1e-6) / 1e9, nb / (k[2] * 1e-6) / 8e12))
+    n, d = 2400000, 100
+    rows = [(kstats(tall, name), nbytes) for name, nbytes in (
+        ("::pack_flat_kernel", n * d * 1.5), ("::unpack_flat_kernel", n * d * 1.5),
+        ("sq_decode_f4_kernel<4, true, void>", n * d * 4.5), ("sq_decode_f4_kernel<4, false, void>", n * d * 4.5),
+        ("vq_decompress_tile_kernel<false, void>", n * (16 + 512)), ("sq_encode_f4_kernel<4, true", n * d * 4.5),
+        ("sq_encode_f4_kernel<4, false", n * d * 8.0))]
+    if any(k for k, _ in rows):
         with open(os.path.join(P, "streaming_ops_c2_table_shape.md"), "w") as fh:
             fh.write("# Streaming kernels at the C2 table shape (2.4e6 rows), from the `bench.py --all` kernel trace\n\n")
             fh.write("    rocprofv3 --kernel-trace --stats --output-format csv -d out/trace_all -o t -- %s\n\n" % A)
             fh.write("| kernel | calls | avg us | bytes moved (algorithmic) | GB/s |\n|---|---|---|---|---|\n")
-            n, d = 2400000, 100
-            for name, nbytes in (("::pack_flat_kernel", n * d * 1.5), ("::unpack_flat_kernel", n * d * 1.5),
-                                 ("sq_decode_f4_kernel<4, true>", n * d * 4.5), ("sq_decode_f4_kernel<4, false>", n * d * 4.5),
-                                 ("vq_decompress_tile_kernel", n * (16 + 512)), ("sq_encode_f4_kernel<4, true", n * d * 4.5),
-                                 ("sq_encode_f4_kernel<4, false", n * d * 8.0)):
-                k = kstats(tall, name)
+            for k, nbytes in rows:
                 if k:
                     fh.write("| `%s` | %d | %.2f | %.0f MB | %.0f |\n" % (k[0][:60], k[1], k[2], nbytes / 1e6,
                                                                           nbytes / (k[2] * 1e-6) / 1e9))
