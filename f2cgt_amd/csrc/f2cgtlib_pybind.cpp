@@ -132,9 +132,9 @@ torch::Tensor unpackbits(torch::Tensor pack, int64_t target_bits, int64_t unpack
 }
 
 // Codebooks on another device than the data would be read through a pointer of that device.
-torch::Tensor beside(torch::Tensor codebooks, const torch::Tensor& data) {
-  codebooks = dev_contig(codebooks, "codebooks");
-  TORCH_CHECK(codebooks.device() == data.device(), "codebooks are on ", codebooks.device(), ", the data on ", data.device());
+torch::Tensor beside(torch::Tensor codebooks, const torch::Tensor& data, const char* name = "codebooks") {
+  codebooks = dev_contig(codebooks, name);
+  TORCH_CHECK(codebooks.device() == data.device(), name, " are on ", codebooks.device(), ", the data on ", data.device());
   return codebooks;
 }
 
@@ -562,8 +562,8 @@ class KMeans {
 
 // ---- extensions (not in the reference; defined by the benchmark configurations) -------
 
-torch::Tensor affine_params_checked(torch::Tensor params, int64_t feat_dim) {
-  params = dev_contig(params, "params");
+torch::Tensor affine_params_checked(torch::Tensor params, int64_t feat_dim, const torch::Tensor& data) {
+  params = beside(params, data, "params");
   TORCH_CHECK(params.scalar_type() == torch::kFloat32 && params.dim() == 2 && params.size(0) == 2 &&
                   params.size(1) >= feat_dim,
               "affine params must be float32 [2, >= feat_dim] = (min, scale)");
@@ -576,7 +576,7 @@ torch::Tensor sq_affine_decompress(torch::Tensor compress_data, torch::Tensor pa
   TORCH_CHECK(compress_data.dim() == 2 && (compress_data.scalar_type() == torch::kUInt8 ||
                                            compress_data.scalar_type() == torch::kInt8),
               "compress_data must be uint8 [rows, src_dim]");
-  params = affine_params_checked(params, feat_dim);
+  params = affine_params_checked(params, feat_dim, compress_data);
   c10::DeviceGuard guard(compress_data.device());
   auto out = empty_f32({compress_data.size(0), feat_dim}, compress_data);
   check_rc(f2cgt_sq_affine_decompress(static_cast<const uint8_t*>(compress_data.data_ptr()),
@@ -594,7 +594,7 @@ torch::Tensor sq_affine_decompress_spmm_csr(torch::Tensor compress_feat, torch::
   TORCH_CHECK(compress_feat.dim() == 2 && (compress_feat.scalar_type() == torch::kUInt8 ||
                                            compress_feat.scalar_type() == torch::kInt8),
               "compress_feat must be uint8 [rows, src_dim]");
-  params = affine_params_checked(params, feat_dim);
+  params = affine_params_checked(params, feat_dim, compress_feat);
   Graph g = graph_of(indptr, indices);
   c10::DeviceGuard guard(compress_feat.device());
   auto out = empty_f32({g.rows, feat_dim}, compress_feat);
@@ -614,7 +614,7 @@ torch::Tensor hybrid_decompress_spmm_csr(torch::Tensor row_map, torch::Tensor sq
   row_map = dev_contig(row_map, "row_map");
   sq_codes = dev_contig(sq_codes, "sq_codes");
   vq_codes = dev_contig(vq_codes, "vq_codes");
-  vq_codebooks = dev_contig(vq_codebooks, "vq_codebooks");
+  vq_codebooks = beside(vq_codebooks, vq_codes, "vq_codebooks");
   TORCH_CHECK(row_map.dim() == 1 && row_map.scalar_type() == torch::kInt32, "row_map must be int32 [n]");
   TORCH_CHECK(sq_codes.dim() == 2 && sq_codes.scalar_type() == torch::kUInt8 && sq_codes.size(1) == feat_dim,
               "sq_codes must be uint8 [n_sq, feat_dim]");
@@ -622,7 +622,7 @@ torch::Tensor hybrid_decompress_spmm_csr(torch::Tensor row_map, torch::Tensor sq
   TORCH_CHECK(vq_codebooks.dim() == 3 && vq_codebooks.scalar_type() == torch::kFloat32 &&
                   vq_codebooks.size(0) == vq_codes.size(1),
               "vq_codebooks must be float32 [n_codebooks, K, width]");
-  sq_params = affine_params_checked(sq_params, feat_dim);
+  sq_params = affine_params_checked(sq_params, feat_dim, sq_codes);
   Graph g = graph_of(indptr, indices);
   c10::DeviceGuard guard(row_map.device());
   auto out = empty_f32({g.rows, feat_dim}, row_map);

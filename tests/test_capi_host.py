@@ -186,3 +186,31 @@ def test_bench_refuses_more_than_one_gpu_and_needs_a_gpu():
                              capture_output=True, text=True, timeout=300)
         assert one.returncode != 0          # no CPU stand-in for the measured path
         assert one.stdout.strip() == ""     # and no result line
+
+
+def test_extension_refuses_codebooks_on_another_device():
+    """A kernel would read them through a pointer of that device.  Refused before any data is touched, so that tensors
+    without data show it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    lib = f2cgt_amd.load()
+    with FakeTensorMode():
+        def t(*shape, dtype=torch.float32, device="cuda:0"):
+            return torch.empty(shape, dtype=dtype, device=device)
+        there = "cuda:1"
+        x, bytes_, words = t(10, 8), t(10, 8, dtype=torch.uint8), t(10, 8, dtype=torch.int8)
+        graph, w = (t(4, dtype=torch.int64), t(9, dtype=torch.int64)), t(3, 8)
+        sq, vq, params = t(1, 5, device=there), t(8, 4, 1, device=there), t(2, 8, device=there)
+        rows, row_map = t(4, dtype=torch.int64), t(20, dtype=torch.int32)
+        for call in (lambda: lib.sq_compress(x, sq, 4, 8), lambda: lib.sq_encode(x, sq, 4, 8), lambda: lib.sq_decompress(words, sq, 8, 8, 8),
+                     lambda: lib.vq_decompress(bytes_, vq, 8), lambda: lib.vq_decompress_spmm_csr(bytes_, vq, *graph, 8),
+                     lambda: lib.sq_decompress_spmm_csr(words, sq, *graph, 8, 8, 8),
+                     lambda: lib.sq_decompress_rows(words, rows, sq, 8, 8, 8),
+                     lambda: lib.vq_decompress_spmm_csr_linear(bytes_, vq, *graph, 8, w),
+                     lambda: lib.sq_decompress_spmm_csr_linear(words, sq, *graph, 8, 8, 8, w),
+                     lambda: lib.sq_affine_decompress(bytes_, params, 8, 8),
+                     lambda: lib.sq_affine_decompress_spmm_csr(bytes_, params, *graph, 8, 8),
+                     lambda: lib.hybrid_decompress_spmm_csr(row_map, bytes_, t(2, 8), bytes_, vq, *graph, 8),
+                     lambda: lib.hybrid_decompress_spmm_csr(row_map, bytes_, params, bytes_, t(8, 4, 1), *graph, 8)):
+            with pytest.raises(RuntimeError, match="are on cuda:1, the data on cuda:0"):
+                call()
