@@ -606,7 +606,21 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     for (int st = 0; st < S; ++st)
 #pragma unroll
       for (int e = 0; e < 8; ++e) sum = __fmaf_rn(q[st][e], q[st][e], sum);
-    const float xn = add_halves(sum);
+    float xn = add_halves(sum);
+    // Cosine: a row whose square vanishes is scored 2^100 times as long, which its direction does not see.  L2 has the
+    // centres' norm beside it, or products below kTinyGap.
+    if (cosine && __any(xn < FLT_MIN)) {
+      const float up = xn < FLT_MIN ? pow2(100) : 1.f;
+      sum = 0.f;
+#pragma unroll
+      for (int st = 0; st < S; ++st)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          q[st][e] *= up;
+          sum = __fmaf_rn(q[st][e], q[st][e], sum);
+        }
+      xn = add_halves(sum);
+    }
     const int x_shift = norm_shift(xn);
     const float x_scale = -pow2(x_shift);
     // what takes a scaled product to -x . c (cosine) or -2 x . c
@@ -734,8 +748,7 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     // fp64, one rounding for 1 / |c|, one for the product, one for - m: 3 units, doubled) does not
     const float scale = cosine ? sqrtf(xn) * (cdev + 3.5762787e-7f / unit) : xn + cmax;
     const float bound = unit * scale + kTinyGap + slack;
-    // Padding leads where no real score is a number.  A row whose square is below the smallest normal float has pieces of
-    // too few bits and no norm to bound that by; L2 has the centres' norm, or products below kTinyGap.
+    // Padding leads where no real score is a number; cosine: a row of zeros has no direction.
     const bool ask = besti >= n || !(scale < finite_below) || !((runner - bs) > bound) || (cosine && xn < FLT_MIN);
     // exact evaluation of the flagged rows (of a training step, of those that take part: the rows left out are the shortest
     // ones, and a row of zeros ties with every centre)

@@ -126,3 +126,24 @@ def test_rows_whose_squares_vanish(short, k):
     c = rng.standard_normal((140, k)) * 1e31
     near = check(x.astype(np.float32), c.astype(np.float32), "cosine")
     assert near.sum() < 40
+
+
+# the same against centres of ordinary length, where the clamp makes the float64 distances equal: the label is that of the
+# row's direction, which a power of two does not change
+@pytest.mark.parametrize("power", [50, 62, 63, 64, 66, 80, 100, 110])
+@pytest.mark.parametrize("k", [3, 16, 30, 64])
+def test_rows_whose_squares_vanish_keep_their_direction(power, k):
+    print("case assign short direction", power, k, flush=True)
+    rng = np.random.default_rng(k)
+    c = rng.standard_normal((140, k)).astype(np.float32)
+    to = rng.integers(0, 140, 700)
+    x = (c[to] * rng.uniform(0.5, 2, (700, 1)) + 0.01 * rng.standard_normal((700, k))).astype(np.float32)
+    want, _ = labels64(x, c, "cosine")
+    d = 1 - (x / np.linalg.norm(x, axis=1)[:, None]).astype(np.float64) @ (c / np.linalg.norm(c, axis=1)[:, None]).astype(np.float64).T
+    clear = np.partition(d, 1, axis=1)[:, :2] @ [-1, 1] > 1e-3
+    x[::3] *= np.float32(2.0 ** -power)             # beside rows of ordinary length
+    x[1::50] = 0
+    clear[1::50] = False
+    got = capi.kmeans_predict(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), "cosine").cpu().numpy()
+    assert np.array_equal(got[clear], want[clear]) and clear.sum() > 300
+    assert (got[1::50] == 0).all()                  # a row of zeros is as far from every centre
