@@ -441,7 +441,7 @@ bool kmeans_slices_covers(int64_t slices, int64_t n, int64_t k) { return f2cgt_k
 
 // Lloyd iterations of all slices on x [slices, m, k] from `centers` [slices, n, k] (updated in place), until every slice
 // has met `rule` or for max_iter steps; tol grows by `growth` each step.  The flags are read every check_every steps and
-// at the end.  -> int32 [slices] on the host: 0 not met, 1 met, 2 the shift became NaN.
+// at the end.  -> int32 [slices] on the host: 0 not met, 1 met, 2 the shift became NaN, 3 no rows.
 torch::Tensor kmeans_slices_fit(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, std::string metric,
                                 int64_t rule, double tol, double growth, int64_t max_iter, int64_t check_every) {
   x = dev_contig(x, "x");

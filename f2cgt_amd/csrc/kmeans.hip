@@ -310,7 +310,7 @@ __global__ __launch_bounds__(kKmMergeThreads) void km_merge_slices_kernel(KmArgs
   s_cnt[q][at] = cnt;
   __syncthreads();
   if (q == 0) {
-    float d2 = 0.f;
+    float d2 = -0.f;
 #pragma unroll
     for (int w = 1; w < kSide; ++w) { total += s_part[w][at]; cnt += s_cnt[w][at]; }
     if (on && cnt > 0u) {
@@ -323,8 +323,8 @@ __global__ __launch_bounds__(kKmMergeThreads) void km_merge_slices_kernel(KmArgs
   }
   __syncthreads();
   if (t < held && c0 + t < a.n) {
-    float d2 = 0.f;
-    for (int i = 0; i < a.k; ++i) d2 += s_d2[t * a.k + i];
+    float d2 = s_d2[t * a.k];               // (-0 from all columns where the centre has no member)
+    for (int i = 1; i < a.k; ++i) d2 += s_d2[t * a.k + i];
     // device-wide: the workgroup that reads the shifts may run behind another L2
     __hip_atomic_store(moves + c0 + t, d2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -333,11 +333,14 @@ __global__ __launch_bounds__(kKmMergeThreads) void km_merge_slices_kernel(KmArgs
   __syncthreads();
   if (!s_last || t >= kWave) return;
   float sum = 0.f, sq = 0.f;
+  bool members = false;
   for (int i = lane; i < a.n; i += kWave) {
     const float m2 = __hip_atomic_load(moves + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     sum += sqrtf(m2);
     sq += m2;
+    members = members || __float_as_uint(m2) != 0x80000000u;
   }
+  members = __any(members);
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) {
     sum += __shfl_xor(sum, off);
@@ -346,7 +349,8 @@ __global__ __launch_bounds__(kKmMergeThreads) void km_merge_slices_kernel(KmArgs
   if (lane == 0) {
     a.shift[0] = sum;
     a.shift[1] = sq;
-    km_decide(a, sum, sq);
+    if (!members && a.stop != nullptr) *a.stop = 3;
+    else km_decide(a, sum, sq);
   }
 }
 

@@ -314,7 +314,10 @@ def _train_all_slices(features, n_clusters, column_slice, sample_index, max_iter
     flags = capi.kmeans_slices_fit(data, keep, centers, "cosine", 2, 5e-2, 1.2, max_iter, 8)
     if rows is not None and int(bad_row.item()):
         raise IndexError("a sample id lies outside the table's %d rows" % features.shape[0])
-    if bool((flags == 2).any()):
+    worst = int(flags.max())
+    if worst == 3:       # their quantile is no number: a NaN among the lengths, or infinities
+        raise RuntimeError("a column slice has no rows to train on")
+    if worst == 2:
         import warnings
         warnings.warn("vq_metadata: the centre shift became NaN; no centres were produced")
         raise TypeError("a column slice has no centres")

@@ -336,7 +336,8 @@ int f2cgt_kmeans_update_static(const float* x, const int64_t* labels_i64, const 
  *
  * f2cgt_kmeans_slices_step: one Lloyd iteration of every slice whose stop flag is zero, as f2cgt_kmeans_predict and
  * f2cgt_kmeans_update would make it from the rows kept: x fp32 [slices, m, k], keep as above or NULL (all), centers fp32
- * [slices, n, k] updated in place, stop int32 [slices] (device) with stop_rule and tol as in f2cgt_kmeans_update.  A label
+ * [slices, n, k] updated in place, stop int32 [slices] (device) with stop_rule and tol as in f2cgt_kmeans_update,
+ * and 3 where no row takes part.  A label
  * is the true first minimum.  Sums: a workgroup's rows in fp64 (LDS), each workgroup's set rounded to fp32 once, the sets
  * added in fp64 in a fixed order.
  * workspace: f2cgt_kmeans_slices_workspace_bytes, 16-byte aligned.  f2cgt_kmeans_slices_covers: 1 where the shape is

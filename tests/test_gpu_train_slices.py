@@ -170,6 +170,22 @@ def test_slices_stop_one_by_one():
     assert lib.kmeans_slices_fit(x, None, start.clone(), "l2", 2, 1e-9, 1.0, 4, 8).tolist()[2] == 2
 
 
+@pytest.mark.parametrize("m,n,k,rule", [(500, 40, 12, 2), (20000, 256, 16, 2), (500, 5, 3, 1), (3000, 130, 8, 0)])
+def test_a_slice_without_rows_is_flagged(m, n, k, rule):
+    """Its centres stay as they are; a slice with a single row that does not move its centre is no such slice."""
+    g = torch.Generator().manual_seed(m)
+    x, centers = torch.randn((3, m, k), generator=g).cuda(), torch.randn((3, n, k), generator=g).cuda()
+    keep = torch.full((3, (m + 31) // 32), -1, dtype=torch.int32)
+    keep[1] = 0
+    keep[2] = 0
+    keep[2, 3] = 1 << 5
+    centers[2, n - 1] = x[2, 3 * 32 + 5]
+    start = centers.clone()
+    flags = f2cgt_amd.load().kmeans_slices_fit(x, keep.cuda(), centers, "l2", rule, 1e-9, 1.0, 1, 8)
+    assert flags.tolist() == [0, 3, 0 if rule == 0 else 1]
+    assert torch.equal(centers[1:], start[1:]) and not torch.equal(centers[0], start[0])
+
+
 @pytest.mark.parametrize("dim,k,n", [(40, 16, 64), (33, 8, 32), (21, 7, 20), (16, 16, 256), (5, 8, 8)])
 @pytest.mark.parametrize("where", ["device", "host", "double"])
 def test_vq_metadata_as_slice_by_slice(dim, k, n, where, monkeypatch):
@@ -193,6 +209,16 @@ def test_vq_metadata_refuses_ids_outside():
     x = torch.randn((500, 16), device="cuda")
     with pytest.raises(IndexError):
         pipeline.vq_metadata(x, 8, 8, sample_index=torch.tensor([1, 2, 500]))
+
+
+@pytest.mark.parametrize("where", ["device", "host"])
+@pytest.mark.parametrize("value,columns", [(float("nan"), 1), (float("inf"), 40), (1e30, 40)])
+def test_vq_metadata_refuses_lengths_without_a_quantile(value, columns, where):
+    """A NaN among a slice's lengths, or infinite lengths all over, keep no row: an error, not the random start."""
+    x = torch.randn((500, 40), generator=torch.Generator().manual_seed(2))
+    x[7 if columns == 1 else slice(None), -columns:] = value
+    with pytest.raises(RuntimeError):
+        pipeline.vq_metadata(x.cuda() if where == "device" else x, 8, 16, sample_index=torch.arange(400))
 
 
 @pytest.mark.parametrize("where", ["device", "host"])
