@@ -147,7 +147,7 @@ __device__ __forceinline__ void split2(float v, _Float16& hi, _Float16& lo) {
 //   of its centre, which moves d^2 by at most 2^-21 d |c| <= 2^-22 (d^2 + |c|^2) <= 3 * 2^-22 (|x'|^2 + |c'|^2), and the
 //   rounding of the centring by 2^-22 (|x'|^2 + |c'|^2): 4 * 2^-22 (9.6e-7) for each of two distances.
 //   Cosine: -x . d with |d| <= cdev; fp32 sum, roundings of the normalisation and of m ((k + 2) cdev + 3) 2^-24 |x|, the
-//   pieces 2^-22 |x| cdev, for each of two scores.
+//   pieces 2^-22 |x| cdev, for each of two scores; products below the smallest normal float lose 2^-150 each.
 //   Where fp32 has no number for a distance (a centre beyond the range of the pieces, which |c|^2 beyond the largest float
 //   admits; sums that overflow) it leaves nothing out: such a distance passes, and where it makes the limit no number, or
 //   a row's dot products may overflow (|x| >= 1e38), every centre does.
@@ -217,7 +217,7 @@ __device__ __forceinline__ int exact_row(const AssignArgs& a, const float* __res
     xn += __shfl_xor(xn, off);
   }
   // (cosine: |x| from the fp64 sum, its square may vanish in fp32)
-  float limit = cosine ? nearest + (1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) + 4.9e-7f * cdev) * (float)sqrt(xn) * 1.001f + 1e-30f
+  float limit = cosine ? nearest + (1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) + 4.9e-7f * cdev) * (float)sqrt(xn) * 1.001f + 1e-42f
                        : nearest * (1.f + 1.1920929e-7f * (float)(k + 4)) + 1e-37f + 2.1e-6f * (xnorm2 + cmax);
   if (cosine && !(xn < 1e76)) limit = INFINITY;
   double bestv = DBL_MAX;

@@ -130,20 +130,24 @@ def test_rows_whose_squares_vanish(short, k):
 
 # the same against centres of ordinary length, where the clamp makes the float64 distances equal: the label is that of the
 # row's direction, which a power of two does not change
-@pytest.mark.parametrize("power", [50, 62, 63, 64, 66, 80, 100, 110])
+@pytest.mark.parametrize("power", [50, 62, 63, 64, 66, 80, 100, 110, 120, 130])
 @pytest.mark.parametrize("k", [3, 16, 30, 64])
 def test_rows_whose_squares_vanish_keep_their_direction(power, k):
     print("case assign short direction", power, k, flush=True)
     rng = np.random.default_rng(k)
     c = rng.standard_normal((140, k)).astype(np.float32)
+    c[139], c[100], c[60] = c[7], 2 * c[20], c[61] * np.float32(1 + 1e-6)       # ties, decided in float64 among them alone
     to = rng.integers(0, 140, 700)
     x = (c[to] * rng.uniform(0.5, 2, (700, 1)) + 0.01 * rng.standard_normal((700, k))).astype(np.float32)
     want, _ = labels64(x, c, "cosine")
     d = 1 - (x / np.linalg.norm(x, axis=1)[:, None]).astype(np.float64) @ (c / np.linalg.norm(c, axis=1)[:, None]).astype(np.float64).T
     clear = np.partition(d, 1, axis=1)[:, :2] @ [-1, 1] > 1e-3
-    x[::3] *= np.float32(2.0 ** -power)             # beside rows of ordinary length
-    x[1::50] = 0
-    clear[1::50] = False
+    zero = np.zeros(700, bool)
+    zero[1::50] = True
+    x[::3] *= np.float32(2.0 ** -(power - 20)) * np.float32(2.0 ** -20)         # beside rows of ordinary length
+    x[zero] = 0
     got = capi.kmeans_predict(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), "cosine").cpu().numpy()
-    assert np.array_equal(got[clear], want[clear]) and clear.sum() > 300
-    assert (got[1::50] == 0).all()                  # a row of zeros is as far from every centre
+    assert np.array_equal(got[clear & ~zero], want[clear & ~zero]) and clear.sum() > 300
+    # (1e-4: what rows of 2^-130 have left of their values)
+    assert (d[np.arange(700), got] - d.min(1))[~zero].max() < 1e-4
+    assert (got[zero] == 0).all()                   # a row of zeros is as far from every centre
