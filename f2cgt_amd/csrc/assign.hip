@@ -147,7 +147,7 @@ __device__ __forceinline__ void split2(float v, _Float16& hi, _Float16& lo) {
 //   of its centre, which moves d^2 by at most 2^-21 d |c| <= 2^-22 (d^2 + |c|^2) <= 3 * 2^-22 (|x'|^2 + |c'|^2), and the
 //   rounding of the centring by 2^-22 (|x'|^2 + |c'|^2): 4 * 2^-22 (9.6e-7) for each of two distances.
 //   Cosine: -x . d with |d| <= cdev; fp32 sum, roundings of the normalisation and of m ((k + 2) cdev + 3) 2^-24 |x|, the
-//   pieces 2^-22 |x| cdev, for each of two scores; products below the smallest normal float lose 2^-150 each.
+//   pieces 2^-22 |x| cdev, for each of two scores; products below the smallest normal float lose 2^-150 each (64 twice: 9e-44).
 //   Where fp32 has no number for a distance (a centre beyond the range of the pieces, which |c|^2 beyond the largest float
 //   admits; sums that overflow) it leaves nothing out: such a distance passes, and where it makes the limit no number, or
 //   a row's dot products may overflow (|x| >= 1e38), every centre does.
@@ -217,7 +217,7 @@ __device__ __forceinline__ int exact_row(const AssignArgs& a, const float* __res
     xn += __shfl_xor(xn, off);
   }
   // (cosine: |x| from the fp64 sum, its square may vanish in fp32)
-  float limit = cosine ? nearest + (1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) + 4.9e-7f * cdev) * (float)sqrt(xn) * 1.001f + 1e-42f
+  float limit = cosine ? nearest + (1.1920929e-7f * ((float)(k + 4) * cdev + 3.f) + 4.9e-7f * cdev) * (float)sqrt(xn) * 1.001f + 1e-43f
                        : nearest * (1.f + 1.1920929e-7f * (float)(k + 4)) + 1e-37f + 2.1e-6f * (xnorm2 + cmax);
   if (cosine && !(xn < 1e76)) limit = INFINITY;
   double bestv = DBL_MAX;
@@ -606,21 +606,7 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     for (int st = 0; st < S; ++st)
 #pragma unroll
       for (int e = 0; e < 8; ++e) sum = __fmaf_rn(q[st][e], q[st][e], sum);
-    float xn = add_halves(sum);
-    // Cosine: a row whose square vanishes is scored 2^100 times as long, which its direction does not see.  L2 has the
-    // centres' norm beside it, or products below kTinyGap.
-    if (cosine && __any(xn < FLT_MIN)) {
-      const float up = xn < FLT_MIN ? pow2(100) : 1.f;
-      sum = 0.f;
-#pragma unroll
-      for (int st = 0; st < S; ++st)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          q[st][e] *= up;
-          sum = __fmaf_rn(q[st][e], q[st][e], sum);
-        }
-      xn = add_halves(sum);
-    }
+    const float xn = add_halves(sum);
     const int x_shift = norm_shift(xn);
     const float x_scale = -pow2(x_shift);
     // what takes a scaled product to -x . c (cosine) or -2 x . c
@@ -748,7 +734,9 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     // fp64, one rounding for 1 / |c|, one for the product, one for - m: 3 units, doubled) does not
     const float scale = cosine ? sqrtf(xn) * (cdev + 3.5762787e-7f / unit) : xn + cmax;
     const float bound = unit * scale + kTinyGap + slack;
-    // Padding leads where no real score is a number; cosine: a row of zeros has no direction.
+    // Padding leads where no real score is a number.  A row whose square is below the smallest normal float has pieces of
+    // too few bits and no norm to bound that by (scored 2^100 times as long it would not need float64, at 2 % of the time of
+    // every other row); L2 has the centres' norm, or products below kTinyGap.
     const bool ask = besti >= n || !(scale < finite_below) || !((runner - bs) > bound) || (cosine && xn < FLT_MIN);
     // exact evaluation of the flagged rows (of a training step, of those that take part: the rows left out are the shortest
     // ones, and a row of zeros ties with every centre)

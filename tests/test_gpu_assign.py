@@ -148,6 +148,6 @@ def test_rows_whose_squares_vanish_keep_their_direction(power, k):
     x[zero] = 0
     got = capi.kmeans_predict(torch.from_numpy(x).cuda(), torch.from_numpy(c).cuda(), "cosine").cpu().numpy()
     assert np.array_equal(got[clear & ~zero], want[clear & ~zero]) and clear.sum() > 300
-    # (1e-4: what rows of 2^-130 have left of their values)
-    assert (d[np.arange(700), got] - d.min(1))[~zero].max() < 1e-4
+    # (3e-4: what rows of 2^-130 have left of their values, and products of theirs)
+    assert (d[np.arange(700), got] - d.min(1))[~zero].max() < 3e-4
     assert (got[zero] == 0).all()                   # a row of zeros is as far from every centre
