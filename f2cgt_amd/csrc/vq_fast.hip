@@ -39,8 +39,7 @@ struct VqArgs {
   int n_cb, K, w, feat_dim;
   int n_tiles, n_stripes;
   int stripes_per_xcd;  // > 0: the column tiles of a stripe share one XCD (see the kernel)
-  int dense_store;      // sparse rows: results go through LDS so that every store instruction is dense
-  int own_lg;           // 2: the launch takes the form whose lanes own their columns in groups of four (pair_pos)
+  int probe_stores;     // experiments build only: 2 = the launch without its stores; the strip kernel's store form
   int store_late;       // experiments build only: 9 = the time-stamped form of the wave kernel
   unsigned long long* trace;   // experiments build only: per wave {start, first step, end} in 100 MHz ticks
 };
@@ -69,6 +68,23 @@ __device__ __forceinline__ float mean_scale(int n) {
   const float d = (float)n;
   const float r = __builtin_amdgcn_rcpf(d);
   return __fmaf_rn(__fmaf_rn(-d, r, 1.f), r, r);
+}
+
+// Non-temporal stores to `base` (the same for all lanes) + off; a lane with off = kNowhere writes nothing.  The
+// buffer's bound drops its 16 (8) bytes, so that a lane without columns of its own needs no branch and every path
+// through a step issues the same number of stores (see vq_wave_kernel).
+constexpr uint32_t kNowhere = 0x80000000u;
+constexpr int kStreamed = 2;   // cache policy bits of the buffer instruction: non-temporal
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t out_buffer(char* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, kNowhere, 0x00027000);
+}
+__device__ __forceinline__ void store_at4(char* base, uint32_t off, float a, float b, float c, float d) {
+  const u32x4 v = {__float_as_uint(a), __float_as_uint(b), __float_as_uint(c), __float_as_uint(d)};
+  __builtin_amdgcn_raw_buffer_store_b128(v, out_buffer(base), off, 0, kStreamed);
+}
+__device__ __forceinline__ void store_at2(char* base, uint32_t off, float a, float b) {
+  const u32x2 v = {__float_as_uint(a), __float_as_uint(b)};
+  __builtin_amdgcn_raw_buffer_store_b64(v, out_buffer(base), off, 0, kStreamed);
 }
 
 template <int BT, typename Idx>
@@ -311,11 +327,23 @@ __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlan
 // columns, 3e6 edges, 10 per row).  A tile of two columns in all (130 = 128 + 2) stores those alone.  The codebooks
 // hold the columns up to the next multiple of 4, since n_cb * w >= feat_dim is a multiple of 8, so the sums are
 // formed as for a full group.
-// QUAD (H == 2): the two 16-byte halves of a lane's result are exchanged inside lane quads before they are stored,
-// so that a store instruction writes whole 64-byte pieces (see the store at the end of a step).
-// OWN (H == 2): the binary logarithm of the number of lanes that own the columns of a code together (pair_pos).
-template <int BT, int H, int RPM, typename Idx, bool DENSE = false, bool TRACE = false, bool TAIL = false,
-          bool EVEN2 = false, bool QUAD = false, int OWN = 0>
+//
+// How H == 2 lanes write their eight columns.  Two plain 16-byte stores would each write 16 of every 32 bytes of a
+// row; the halves of a line then have to meet in the L2, and where the output's lines are not in the last-level cache
+// (a training loop never aggregates the same block twice) what leaves it are partial writes.
+//   RPM == 4: a row's sixteen lanes lie half in the lower and half in the upper 32 lanes of the wave: lane i of the lower
+//   ones has columns 8 i of the tile, its partner 32 lanes on columns 64 + 8 i (odd rows the other way round, so that the
+//   sixteen lanes that LDS serves together still read sixteen different 16-byte positions).  Four v_permlane32_swap
+//   hand the lower lanes' second halves up and the upper lanes' first halves down, after which each of the two store
+//   instructions writes 256 contiguous bytes of every row.  This took the place of four forms (as they are; turned
+//   round in LDS; halves exchanged inside quads, 64-byte pieces; columns owned by groups of four lanes, 64-byte
+//   pieces): graphs and outputs in turn, 24 x 32 from 5.8 GB of codes 637 / 584 / 642 / 643 -> 581 us, 16 x 8 from
+//   160 MB 123 / 111 / 124 -> 108, 16 x 16 at 10 edges per row 98 / 74 / 78 -> 67; one graph and output again and again
+//   447 / 463 / 490 / 475 -> 460, 79 / 76 / 78 -> 76 and 92 / 74 / 73 -> 68: only 24 x 32, whose output the last-level
+//   cache takes in part, is slower than with the plain halves, and only there.
+//   RPM < 4: the lane groups that share a row add their sums while they hand them on (v_permlane16_swap: a group ends up
+//   with the totals of one half), so that one store instruction writes the row's 512 bytes.
+template <int BT, int H, int RPM, typename Idx, bool TAIL = false, bool EVEN2 = false, bool TRACE = false>
 __global__ __launch_bounds__(kThreads) void vq_wave_kernel(VqArgs a, const Idx* __restrict__ indptr,
                                                            const Idx* __restrict__ indices,
                                                            float* __restrict__ out) {
@@ -382,19 +410,28 @@ __global__ __launch_bounds__(kThreads) void vq_wave_kernel(VqArgs a, const Idx* 
   // lanes per row: 32 lanes with one float4 each (H == 1) or 16 lanes with a whole 8-column code
   // each (H == 2); the wave then works on 2 or 4 rows at a time
   constexpr int kLanesPerRow = 32 / H, kRowsPerPass = 64 / kLanesPerRow;
-  // A lane beyond the columns of a partial tile takes the tile's last column group again (it
-  // computes and stores what that group's own lane does), so that no lane ever skips a store: the
-  // number of memory operations of a step is then the same on every path, and the waits in front
-  // of the next step's loads can leave this step's stores in flight (see the main loop).
+  constexpr bool SWAP = H == 2 && RPM == 4;    // a row's lanes lie half in the lower, half in the upper 32 (see above)
   const int groups = tile_cols / (4 * H);      // column groups of this tile (tile_cols % (4 H) == 0)
-  const int c4 = (lane & (kLanesPerRow - 1)) < groups ? (lane & (kLanesPerRow - 1)) : groups - 1;
-  const int half = lane / kLanesPerRow;
-  // first column of the lane inside the tile; with H == 2 its second float4 lies 4 << own_lg columns on (pair_pos)
-  constexpr int own_lg = H == 2 ? OWN : 0;
-  const int col0 = H == 2 ? ((c4 >> own_lg) << (3 + own_lg)) + 4 * (c4 & ((1 << own_lg) - 1)) : c4 * 4;
-  const int byte_idx = col0 / a.w;
-  const float* cbp = s_cb + c4 * 4;
+  const int half = SWAP ? (lane >> 3) & 3 : lane / kLanesPerRow;            // the lane's row of a pass
+  const int lane_col = SWAP ? (lane & 7) + 8 * ((lane >> 5) ^ (half & 1)) : lane & (kLanesPerRow - 1);
+  // A lane beyond the columns of a partial tile takes the last column group's code, reads the table at its own
+  // position (so that it meets no other lane's bank) and stores nowhere.
+  const int c4 = lane_col < groups ? lane_col : groups - 1;
+  const int byte_idx = c4 * 4 * H / a.w;
+  const float* cbp = s_cb + lane_col * 4;
   const int prev_group_lane = (lane & ~(kLanesPerRow - 1)) + (c4 > 0 ? c4 - 1 : 0);   // EVEN2
+  // byte offsets, inside the tile's columns of a row, of what the lane stores
+  uint32_t put_a = lane_col < groups ? 16u * H * (uint32_t)lane_col : kNowhere, put_b = 0;
+  if constexpr (SWAP) {
+    const int k = lane & 7;
+    const uint32_t at = 32u * (uint32_t)k + 16u * (uint32_t)(lane >> 5);
+    const uint32_t lo = k < groups ? at : kNowhere, hi = k + 8 < groups ? at + 256u : kNowhere;
+    put_a = (half & 1) ? hi : lo;
+    put_b = (half & 1) ? lo : hi;
+    if (groups <= 8) { put_a = lo; put_b = kNowhere; }
+  }
+  const bool half_group = EVEN2 && (tile_cols_out & 2) && lane_col == groups - 1;
+  if (EVEN2 && half_group && tile_cols_out >= 4) put_a -= 8u;
   const uint8_t* code_base = a.codes + tile * BT;
   const uint32_t n_last = (uint32_t)(a.N - 1);
   // the last source row whose BT bytes for this tile lie inside the table (TAIL only)
@@ -522,32 +559,25 @@ __global__ __launch_bounds__(kThreads) void vq_wave_kernel(VqArgs a, const Idx* 
       const Idx* src = on ? indices + e0 + eb1 + lane : indptr;
       Ireg = (int64_t)*src;                                // I(1)
     }
-    stage_codebook_store<kThreads, H == 2>(s_cb, cbv, a.K, own_lg);
+    stage_codebook_store<kThreads, H == 2>(s_cb, cbv, a.K);
     __syncthreads();
     if (!has_rows) return;
     g_first = 0;
   } else {
-    stage_codebook_tile<kThreads, H == 2>(s_cb, a.codebooks, a.K, a.w, tile, tile_cols, own_lg);
+    stage_codebook_tile<kThreads, H == 2>(s_cb, a.codebooks, a.K, a.w, tile, tile_cols);
     if (threadIdx.x == 0) *s_next = kWaves;
     __syncthreads();
     if (!has_rows) return;
     issue_P(base_cur);
     park_P(0);
   }
-  // The two 16-byte stores of a lane and step are issued where the results are ready, at the end of
-  // the step, back to back from one base register.  In the direct (not LDS-staged) form they are
-  // the two halves of the lane's 32 bytes, and they have to reach the L1 together: issued a few
-  // instructions apart (separate predicated blocks) the halves are written to memory separately
-  // and the kernel falls into a regime twice as slow (24 x 32 codebooks: 497 -> 870-960 us, L2 ->
-  // memory write-credit stalls up from 2e4 to 3.7e7 cycles per launch).
-  //
   // Loads and stores complete in order on one counter.  A step issues its loads (code bytes of the
   // next mini-block, source ids of the one after) in front of its sums and its stores behind them,
   // and the next step waits for those loads only: it may leave the younger stores in flight if the
   // compiler can count them, i.e. if every path through a step issues the same number of stores.
   // Hence no store below sits under a condition: a lane group without a row of its own (the last
   // mini-block of a range) takes the mini-block's last row again and stores the same values to the
-  // same place, as do the lane groups that shared a row's edges.  With conditional stores every
+  // same place, and lanes without columns store beyond the buffer's bound.  With conditional stores every
   // step began by waiting for the stores of the one before, a full trip to memory per step and wave.
   unsigned long long t_first = 0;
   if constexpr (TRACE) t_first = wall_clock64();
@@ -718,130 +748,62 @@ __global__ __launch_bounds__(kThreads) void vq_wave_kernel(VqArgs a, const Idx* 
         }
         return n;
       };
-      auto mean = [&](int n, float (&acc)[H][4]) {
-        if (n > 1) {
-          const float r = mean_scale(n);
+      // uniform base + 32-bit byte offset of the lane: no 64-bit address arithmetic per lane
+      char* obase = reinterpret_cast<char*>(out + row0 * (int64_t)a.feat_dim + tile * 128);
 #pragma unroll
-          for (int h = 0; h < H; ++h)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) acc[h][t] *= r;
-        }
-      };
-      if constexpr (DENSE) {
-        static_assert(H == 2 && SPR == 1 && kPasses == 1, "the LDS-turned stores are for 4-row steps of 16-lane rows");
-        // Four rows, sixteen lanes each.  A lane's result is 32 consecutive bytes, which as two
-        // stores would be 16 of every 32 bytes per instruction (half-written sectors on the way to
-        // memory).  The wave's 1 KB staging area, free once the edge loops are done, turns them
-        // around: the lanes of columns [64 p, 64 p + 64) write their two float4, every lane reads
-        // back the float4 of its own lane index, and each store instruction covers 256 contiguous
-        // bytes of every row.  (Lanes beyond a partial tile's columns hold a copy of its last
-        // column group and skip the write to the staging area; their stores repeat the last float4.)
-        const int lane_c = lane & (kLanesPerRow - 1);
-        const int row = half < nr ? half : nr - 1;
+      for (int pass = 0; pass < kPasses; ++pass) {
+        const int slot = pass * kRowsPerPass + half;
+        int row = slot / SPR;
+        const int sub = slot % SPR;
+        row = row < nr ? row : nr - 1;
         float acc[H][4];
-        const int n = row_sum(row, 0, acc);
-        mean(n, acc);
-        float4* stg = reinterpret_cast<float4*>(s_codes);
-        char* obase = reinterpret_cast<char*>(out + row0 * (int64_t)a.feat_dim + tile * 128);   // uniform
-        const uint32_t orow_b = (uint32_t)row * ((uint32_t)a.feat_dim * 4u);
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          __builtin_amdgcn_wave_barrier();
-          if ((lane_c >> 3) == p && lane_c < groups) {
-#pragma unroll
-            for (int h = 0; h < H; ++h)
-              stg[half * 16 + (lane_c & 7) * 2 + h] = make_float4(acc[h][0], acc[h][1], acc[h][2], acc[h][3]);
-          }
-          __builtin_amdgcn_wave_barrier();
-          // a lane beyond the tile's columns stores the tile's last float4 again; when that lies in
-          // the other half (tile_cols <= 64 p) nobody wrote to the staging area in this pass and it
-          // still holds that half
-          int col = 64 * p + 4 * lane_c;
-          const int last = tile_cols - 4;                  // first column of the tile's last float4
-          col = col < last ? col : last;
-          const float4 v = stg[half * 16 + ((col & 63) >> 2)];
-          store_nt4(reinterpret_cast<float*>(obase + (orow_b + 4u * (uint32_t)col)), v.x, v.y, v.z, v.w);
-        }
-      } else {
-        // uniform base + 32-bit byte offset of the lane: no 64-bit address arithmetic per lane
-        char* obase = reinterpret_cast<char*>(out + row0 * (int64_t)a.feat_dim + tile * 128);
-#pragma unroll
-        for (int pass = 0; pass < kPasses; ++pass) {
-          const int slot = pass * kRowsPerPass + half;
-          int row = slot / SPR;
-          const int sub = slot % SPR;
-          row = row < nr ? row : nr - 1;
-          float acc[H][4];
-          const int n = row_sum(row, sub, acc);
-          if (SPR > 1) {
-#pragma unroll
-            for (int h = 0; h < H; ++h)
-#pragma unroll
-              for (int t = 0; t < 4; ++t) {
-                acc[h][t] += __shfl_xor(acc[h][t], kLanesPerRow);
-                if (SPR > 2) acc[h][t] += __shfl_xor(acc[h][t], 2 * kLanesPerRow);
-              }
-          }
-          mean(n, acc);
+        const int n = row_sum(row, sub, acc);
+        const float r = n > 1 ? mean_scale(n) : 1.f;
+        const uint32_t row_b = (uint32_t)row * ((uint32_t)a.feat_dim * 4u);
 #ifdef F2CGT_EXPERIMENTS
-          if (a.dense_store == 2 && acc[0][0] != 12345.678f) continue;   // no stores: what the rest of the kernel costs
+        if (a.probe_stores == 2 && acc[0][0] != 12345.678f) continue;   // no stores: what the rest of the kernel costs
 #endif
-          // the lane's two 16-byte stores: one address, the second 16 bytes on as an immediate offset,
-          // so that they are issued back to back (see above)
-          const uint32_t off_b = (uint32_t)row * ((uint32_t)a.feat_dim * 4u) + 4u * (uint32_t)col0;
-          float* dst = reinterpret_cast<float*>(obase + off_b);
-          if constexpr (EVEN2) {
-            if (tile_cols_out < 4) {          // a tile of two columns: nothing to pair them with
-              store_nt2(dst, acc[0][0], acc[0][1]);
-            } else if (tile_cols_out & 2) {   // the tile ends with a group of two columns
-              const bool half_group = col0 + 2 >= tile_cols_out;
-              const float p2 = __shfl(acc[0][2], prev_group_lane), p3 = __shfl(acc[0][3], prev_group_lane);
-              store_nt4_align8(half_group ? dst - 2 : dst, half_group ? p2 : acc[0][0], half_group ? p3 : acc[0][1],
-                               half_group ? acc[0][0] : acc[0][2], half_group ? acc[0][1] : acc[0][3]);
-            } else {
-              store_nt4_align8(dst, acc[0][0], acc[0][1], acc[0][2], acc[0][3]);
-            }
-          } else if constexpr (QUAD) {
-            // A lane's eight columns are 32 contiguous bytes; stored as they are, each of the two store
-            // instructions writes 16 of every 32 bytes.  Here the four lanes of a quad exchange their halves
-            // (lane permutes inside the quad, no LDS), so that one instruction writes the first 64 contiguous
-            // bytes of the quad's 128 and the other the last 64: lane k stores half (k & 1) of lane (k >> 1),
-            // then of lane 2 + (k >> 1).
-            const int lr = lane & (kLanesPerRow - 1), k = lr & 3;
-            const bool odd = (k & 1) != 0;
-            float va[4], vb[4];
+        if constexpr (SWAP) {
+          float va[4], vb[4];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              const int lo_a = __builtin_amdgcn_update_dpp(0, __float_as_int(acc[0][t]), 0x50, 0xf, 0xf, false);
-              const int hi_a = __builtin_amdgcn_update_dpp(0, __float_as_int(acc[1][t]), 0x50, 0xf, 0xf, false);
-              const int lo_b = __builtin_amdgcn_update_dpp(0, __float_as_int(acc[0][t]), 0xfa, 0xf, 0xf, false);
-              const int hi_b = __builtin_amdgcn_update_dpp(0, __float_as_int(acc[1][t]), 0xfa, 0xf, 0xf, false);
-              va[t] = __int_as_float(odd ? hi_a : lo_a);
-              vb[t] = __int_as_float(odd ? hi_b : lo_b);
-            }
-            // Columns of this lane's two pieces inside the tile.  A first piece beyond the tile's columns belongs to
-            // a lane beyond them as well, which holds a copy of the last column group: it stores that group's second
-            // half, the tile's last 16 bytes.  A second piece beyond the columns repeats the lane's first store.
-            const int col_a = (lr >> 2) * 32 + 4 * k, col_b = col_a + 16;
-            const int last = tile_cols - 4;
-            const bool in_a = col_a <= last, in_b = col_b <= last;
+          for (int t = 0; t < 4; ++t) {
+            const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0][t] * r), __float_as_uint(acc[1][t] * r),
+                                                            false, false);
+            va[t] = __uint_as_float(v[0]);
+            vb[t] = __uint_as_float(v[1]);
+          }
+          if (groups <= 8) {   // one piece per row: all four rows' in the first store
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              va[t] = in_a ? va[t] : acc[1][t];
-              vb[t] = in_b ? vb[t] : va[t];
+            for (int t = 0; t < 4; ++t) va[t] = (half & 1) ? vb[t] : va[t];
+          }
+          store_at4(obase, row_b + put_a, va[0], va[1], va[2], va[3]);
+          store_at4(obase, row_b + put_b, vb[0], vb[1], vb[2], vb[3]);
+        } else if constexpr (SPR > 1) {
+          // the groups of a row: the even one ends with the totals of columns 0..3 of its lanes, the odd one with 4..7
+          float v[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const auto s2 = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[0][t]), __float_as_uint(acc[H - 1][t]),
+                                                             false, false);
+            v[t] = __uint_as_float(s2[0]) + __uint_as_float(s2[1]);
+            if constexpr (SPR > 2) {
+              const auto s4 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[t]), __float_as_uint(v[t]), false, false);
+              v[t] = __uint_as_float(s4[0]) + __uint_as_float(s4[1]);
             }
-            const int pa = in_a ? col_a : last, pb = in_b ? col_b : pa;
-            const uint32_t row_b = (uint32_t)row * ((uint32_t)a.feat_dim * 4u);
-            store_nt4(reinterpret_cast<float*>(obase + (row_b + 4u * (uint32_t)pa)), va[0], va[1], va[2], va[3]);
-            store_nt4(reinterpret_cast<float*>(obase + (row_b + 4u * (uint32_t)pb)), vb[0], vb[1], vb[2], vb[3]);
+            v[t] *= r;
+          }
+          store_at4(obase, row_b + (sub < 2 ? put_a : kNowhere) + 16u * (uint32_t)(sub & 1), v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) acc[0][t] *= r;
+          if (EVEN2 && tile_cols_out < 4) {          // a tile of two columns: nothing to pair them with
+            store_at2(obase, row_b + put_a, acc[0][0], acc[0][1]);
+          } else if (EVEN2 && (tile_cols_out & 2)) {   // the tile ends with a group of two columns
+            const float p2 = __shfl(acc[0][2], prev_group_lane), p3 = __shfl(acc[0][3], prev_group_lane);
+            store_at4(obase, row_b + put_a, half_group ? p2 : acc[0][0], half_group ? p3 : acc[0][1],
+                      half_group ? acc[0][0] : acc[0][2], half_group ? acc[0][1] : acc[0][3]);
           } else {
-            // H == 2: the second float4 lies 16 bytes on, or 64 with columns owned in groups of four lanes (pair_pos).
-            // The distance is a literal so that it folds into the second store: with it in a register the two are no
-            // longer issued back to back, the halves of a 32-byte piece reach the L2 apart and leave it as partial
-            // writes (24 x 32 from a 5.8 GB table: 433 -> 958 us).
-#pragma unroll
-            for (int h = 0; h < H; ++h)
-              store_nt4(dst + ((4 * h) << own_lg), acc[h][0], acc[h][1], acc[h][2], acc[h][3]);
+            store_at4(obase, row_b + put_a, acc[0][0], acc[0][1], acc[0][2], acc[0][3]);
           }
         }
       }
@@ -964,7 +926,7 @@ __global__ __launch_bounds__(kSThreads) void vq_strip_kernel(VqArgs a, const Idx
   // a lane's float4 of the staged rows: column (lane & 31) * 4 of staged row 2 i + (lane >> 5)
   const uint32_t out_lane = (uint32_t)((lane & 31) * 4) + (uint32_t)(lane >> 5) * (uint32_t)a.feat_dim;
   const bool col_ok = (lane & 31) * 4 < tile_cols;
-  const bool nt = a.dense_store == 1 || a.dense_store == 3;
+  const bool nt = a.probe_stores == 1 || a.probe_stores == 3;
 
   // pipeline registers: two generations of everything that is in flight for two steps
   Idx praw0[2] = {0, 0}, praw1[2] = {0, 0};          // P -> I
@@ -1119,7 +1081,7 @@ __global__ __launch_bounds__(kSThreads) void vq_strip_kernel(VqArgs a, const Idx
 #pragma unroll
       for (int k = 0; k < KE; ++k) {
         if (__ballot(k < deg) == 0) break;
-        if (a.dense_store == 3 && k >= 1) break;   // experiment: stores only
+        if (a.probe_stores == 3 && k >= 1) break;   // experiment: stores only
         if (k == 0) {
           if (0 < deg) {   // the first edge lands in the accumulators as it is
             f4v v[8];
@@ -1155,7 +1117,7 @@ __global__ __launch_bounds__(kSThreads) void vq_strip_kernel(VqArgs a, const Idx
 #pragma unroll
           for (int t = 0; t < 4; ++t) acc[j][t] = div_by(acc[j][t], d, r);
       }
-      if (a.dense_store != 2) {
+      if (a.probe_stores != 2) {
         if (IL) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) direct_store(i, acc, g);
@@ -1220,21 +1182,42 @@ unsigned long long* g_trace = nullptr;   // device buffer for the time stamps of
 template <int BT>
 int launch_wave_trace(const VqArgs& a, const void* indptr, const void* indices, float* out, hipStream_t st,
                       const char* what, unsigned grid, size_t wlds) {
-  const void* kern = reinterpret_cast<const void*>(vq_wave_kernel<BT, 2, 4, int64_t, false, true>);
+  const void* kern = reinterpret_cast<const void*>(vq_wave_kernel<BT, 2, 4, int64_t, false, false, true>);
   const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wlds);
   if (e != hipSuccess) return fail((int)e, "%s: cannot reserve %zu B of LDS", what, wlds);
-  vq_wave_kernel<BT, 2, 4, int64_t, false, true><<<grid, kThreads, wlds, st>>>(
+  vq_wave_kernel<BT, 2, 4, int64_t, false, false, true><<<grid, kThreads, wlds, st>>>(
       a, static_cast<const int64_t*>(indptr), static_cast<const int64_t*>(indices), out);
   return launch_status(what);
 }
 #endif
 
+// What the plan of a launch reports beside its geometry (form, owners): the class of the launch by what binds it, which
+// selected between four ways of writing the output; all of them are the lane swap of vq_wave_kernel now.  1: up to 8
+// edges per row, tables beyond the last-level cache at 128, 256 and 512 columns and large outputs next to tables of 64 to
+// 192 MB; 4: large outputs and up to 11 edges per row from smaller tables; 0: the others, owners 2 with codebooks of
+// 32 columns.
+void plan_store_class(const VqArgs& a, bool rpm4, double avg_deg, int& form, int& owners) {
+  const int64_t out_bytes = a.R * (int64_t)a.feat_dim * 4, table = a.N * (int64_t)a.n_cb;
+  const bool lines = (a.feat_dim == 128 && out_bytes >= (60ll << 20)) ||
+                     (a.feat_dim == 256 && out_bytes >= (60ll << 20) && out_bytes <= (160ll << 20) && avg_deg <= 10.0) ||
+                     (a.feat_dim == 512 && out_bytes >= (96ll << 20) && avg_deg <= 11.0);
+  form = avg_deg <= 8.0;
+  if (!form && a.feat_dim % 8 == 0 && rpm4) {
+    if (store_mode() == F2CGT_STORE_STREAM || (table > (256ll << 20) && lines)) {
+      form = 1;
+    } else if (table <= (192ll << 20) && a.feat_dim >= 128 && a.n_tiles <= 4) {
+      const bool big_out = out_bytes >= (200ll << 20);
+      form = big_out && table >= (64ll << 20) ? 1 : (big_out || avg_deg <= 11.0 ? 4 : 0);
+    }
+  }
+  owners = form == 0 && a.w == 32 && a.feat_dim % 32 == 0 && a.feat_dim >= 128 && rpm4 && table <= (192ll << 20) ? 2 : 0;
+}
+
 template <int BT, int H, int RPM>
 int launch_wave(const VqArgs& a, const void* indptr, const void* indices, int idx_dtype, float* out, hipStream_t st,
-                const char* what, unsigned grid, size_t wlds) {
+                const char* what, unsigned grid, size_t wlds, int form = 0, int owners = 0) {
   if (plan_only()) {
-    plan_record("vq_wave_kernel", grid, kThreads, (int64_t)wlds, 0, H, RPM, a.dense_store,
-                (H == 2 && RPM == 4 && BT == 4 && a.dense_store == 0) ? a.own_lg : 0);
+    plan_record("vq_wave_kernel", grid, kThreads, (int64_t)wlds, 0, H, RPM, form, owners);
     return 0;
   }
 #ifdef F2CGT_EXPERIMENTS
@@ -1242,67 +1225,20 @@ int launch_wave(const VqArgs& a, const void* indptr, const void* indices, int id
     if (a.store_late == 9 && a.trace) return launch_wave_trace<BT>(a, indptr, indices, out, st, what, grid, wlds);
   }
 #endif
-  // the sparse-row form (results turned round in LDS before they are stored) is its own instantiation
-  constexpr bool CAN_DENSE = H == 2 && RPM == 4;
   const bool tail = a.n_cb % BT != 0 || !aligned(a.codes, BT);
-  const bool dense = CAN_DENSE && a.dense_store == 1;
+  const bool i32 = idx_dtype == F2CGT_DT_I32;
+  constexpr bool CAN_EVEN2 = H == 1 && RPM == 4;   // even widths that are no multiple of 4
   const void* kern;
-  if constexpr (H == 1 && RPM == 4) {
-    if (a.feat_dim % 4 != 0) {   // even widths that are no multiple of 4
-      kern = tail ? (idx_dtype == F2CGT_DT_I32
-                         ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false, false, true, true>)
-                         : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, false, false, true, true>))
-                  : (idx_dtype == F2CGT_DT_I32
-                         ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false, false, false, true>)
-                         : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, false, false, false, true>));
-      const hipError_t e2 = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wlds);
-      if (e2 != hipSuccess) return fail((int)e2, "%s: cannot reserve %zu B of LDS", what, wlds);
-      void* params2[] = {const_cast<VqArgs*>(&a), &indptr, &indices, &out};
-      const hipError_t le2 = hipLaunchKernel(kern, dim3(grid), dim3(kThreads), params2, wlds, st);
-      if (le2 != hipSuccess) return fail((int)le2, "%s: launch failed: %s", what, hipGetErrorString(le2));
-      return launch_status(what);
-    }
-  }
-  constexpr bool CAN_QUAD = H == 2 && RPM == 4;
-  const bool quad = CAN_QUAD && a.dense_store == 4;
-  if constexpr (H == 2 && RPM == 4 && BT == 4) {   // codebooks of 32 columns
-    if (a.own_lg == 2 && a.dense_store == 0) {
-      kern = tail ? (idx_dtype == F2CGT_DT_I32
-                         ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false, false, true, false, false, 2>)
-                         : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, false, false, true, false, false, 2>))
-                  : (idx_dtype == F2CGT_DT_I32
-                         ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false, false, false, false, false, 2>)
-                         : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, false, false, false, false, false, 2>));
-      const hipError_t e3 = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wlds);
-      if (e3 != hipSuccess) return fail((int)e3, "%s: cannot reserve %zu B of LDS", what, wlds);
-      void* params3[] = {const_cast<VqArgs*>(&a), &indptr, &indices, &out};
-      const hipError_t le3 = hipLaunchKernel(kern, dim3(grid), dim3(kThreads), params3, wlds, st);
-      if (le3 != hipSuccess) return fail((int)le3, "%s: launch failed: %s", what, hipGetErrorString(le3));
-      return launch_status(what);
-    }
-  }
-  if (quad && tail)
-    kern = idx_dtype == F2CGT_DT_I32
-               ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false, false, true, false, CAN_QUAD>)
-               : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, false, false, true, false, CAN_QUAD>);
-  else if (quad)
-    kern = idx_dtype == F2CGT_DT_I32
-               ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false, false, false, false, CAN_QUAD>)
-               : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, false, false, false, false, CAN_QUAD>);
-  else if (tail && dense)
-    kern = idx_dtype == F2CGT_DT_I32
-               ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, CAN_DENSE, false, true>)
-               : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, CAN_DENSE, false, true>);
-  else if (tail)
-    kern = idx_dtype == F2CGT_DT_I32
-               ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false, false, true>)
-               : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, false, false, true>);
-  else if (idx_dtype == F2CGT_DT_I32)
-    kern = dense ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, CAN_DENSE>)
-                 : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false>);
+  if (CAN_EVEN2 && a.feat_dim % 4 != 0)
+    kern = tail ? (i32 ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, true, CAN_EVEN2>)
+                       : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, true, CAN_EVEN2>))
+                : (i32 ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false, CAN_EVEN2>)
+                       : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, false, CAN_EVEN2>));
   else
-    kern = dense ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, CAN_DENSE>)
-                 : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, false>);
+    kern = tail ? (i32 ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, true>)
+                       : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, true>))
+                : (i32 ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t>)
+                       : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t>));
   const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wlds);
   if (e != hipSuccess) return fail((int)e, "%s: cannot reserve %zu B of LDS", what, wlds);
   void* params[] = {const_cast<VqArgs*>(&a), &indptr, &indices, &out};
@@ -1335,63 +1271,21 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
   // 1-row ones beyond (larger mini-blocks for sparse rows were tried and were slower than 4-row ones).
   const size_t wlds = (size_t)a.K * 128 * 4 + (size_t)(kThreads / 64) * (kWEdges * BT > 1024 ? kWEdges * BT : 1024) +
                       (size_t)(kThreads / 64) * 2 * kWPtr * 4;
-  // with few edges per row the output dominates and its store pattern decides (fanout 2 at the C3
-  // shape: 845 -> 405 us); from about 8 edges per row the detour through LDS costs more than it saves
-  a.dense_store = avg_deg <= 8.0;
-  // Above that (up to 16 edges per row, four-row mini-blocks) the form is chosen by what binds the launch:
-  //  * a code table beyond the 256 MB last-level cache and 128, 256 or 512 columns: through LDS where that is ahead whatever
-  //    the ids (Zipf(1.1) or uniform) and whether one graph and output come again or four in turn.  128 columns from 60 MB of
-  //    output on (tables of 280, 480 and 1600 MB; the time through LDS 0.75 to 1.0 of the plain one's, 1.03 to 1.08 in a few of
-  //    one to two hundred; 16 x 8 at 15 edges per row, 240 MB: one graph 84 -> 80 us / uniform 200 -> 187, in turn 122 -> 111 /
-  //    199 -> 187; outputs of 40 and 50 MB up to 1.07).  256 columns from 60 to 160 MB and up to 10 edges per row (16 x 16 at 10,
-  //    100 MB 0.74 to 0.92; at 200 to 420 MB up to 1.10, at 12 edges per row up to 1.14).  512 columns from 96 MB on and up
-  //    to 11 edges per row (16 x 32 at 10, 240 MB: one graph 96 -> 53 / 79 -> 73, in turn 95 -> 53 / 113 -> 106; uniform ids up to
-  //    1.06 at single sizes where the others gain 1.3 and more; 64 MB in turn 1.09, 14 edges per row up to 1.14).  Other widths lose up to 1.2 with ids that keep to a few rows, which the caches then hold,
-  //    at any size of output (160, 224, 320, 384, 448 columns), and stay as they are;
-  //  * a code table of 192 to 256 MB, or rows of more than four column tiles: the results are stored as they are (24 x 32
-  //    at 12 edges per row from 240 MB, graphs in turn: 193 us, 208 through LDS; from 120 MB 178 against 195).  From 5.8 GB
-  //    at 10 per row one graph again and again takes 420 us, 442 through LDS, and graphs in turn 681 against 585:
-  //    F2CGT_STORE_STREAM is for the latter;
-  //  * an output of 200 MB and more from a table of 64 to 192 MB, which shares the last-level cache with it: through
-  //    LDS as for sparse rows, the form whose store instructions write whole lines.  Warm it is level with the exchange
-  //    (7.5e6 edges at 15 per row from a 160 MB table, 16 x 8: 79.1 against 79.4 us; plain 80.7), with graphs and
-  //    outputs in rotation, where the output's lines are not in the last-level cache when they are written, well
-  //    ahead (108.7 against 125.8 us, plain 120; 16 x 16 at 10 edges per row 73 / 99 against 79 / 102);
-  //  * from a smaller table, such an output or up to 11 edges per row (an output of 340 MB from 32 MB of codes,
-  //    32 x 16 at 12 edges per row: 130 / 131 us warm / in rotation against 135 / 136 through LDS): the halves of a
-  //    lane's eight columns are exchanged inside lane
-  //    quads so that every store instruction writes whole 64-byte pieces (dense_store 4; 1e6 source rows, 3e6 edges
-  //    at 10 per row, plain -> exchange: 16 x 16 121 -> 87 us, 32 x 16 166 -> 90, 8 x 32 126 -> 90, 64 x 8 150 -> 93,
-  //    16 x 8 49 -> 42; the plain form's time at these shapes varies by a factor of two between builds and boxes,
-  //    the exchange's does not).  64-column tiles (half the lanes of a row idle) measured 6-13 % slower with it.
-  // F2CGT_STORE_STREAM (the caller's outputs are written once and read later) takes the LDS form throughout.
   const bool rpm4 = avg_deg <= 16.0 * ((a.R > 0 && a.E % a.R == 0) ? 1.0 : 0.9);
   const int64_t out_bytes = a.R * (int64_t)a.feat_dim * 4;
   const bool big_table = a.N * (int64_t)a.n_cb > (256ll << 20);
-  if (!a.dense_store && a.feat_dim % 8 == 0 && rpm4) {
-    const bool cached_table = a.N * (int64_t)a.n_cb <= (192ll << 20);
-    const bool lines = (a.feat_dim == 128 && out_bytes >= (60ll << 20)) ||
-                       (a.feat_dim == 256 && out_bytes >= (60ll << 20) && out_bytes <= (160ll << 20) && avg_deg <= 10.0) ||
-                       (a.feat_dim == 512 && out_bytes >= (96ll << 20) && avg_deg <= 11.0);
-    if (store_mode() == F2CGT_STORE_STREAM || (big_table && lines)) {
-      a.dense_store = 1;
-    } else if (cached_table && a.feat_dim >= 128 && a.n_tiles <= 4) {
-      const bool big_out = out_bytes >= (200ll << 20);
-      if (big_out && a.N * (int64_t)a.n_cb >= (64ll << 20)) a.dense_store = 1;
-      else if (big_out || avg_deg <= 11.0) a.dense_store = 4;
-    }
-  }
+  int form = 0, owners = 0;
+  plan_store_class(a, rpm4, avg_deg, form, owners);
 #ifdef F2CGT_EXPERIMENTS
   {
     if (const char* d = getenv("F2CGT_VQ_DEFER")) a.store_late = atoi(d);
     a.trace = g_trace;
-    if (const char* d = getenv("F2CGT_VQ_DENSE")) a.dense_store = atoi(d) != 0;   // results through LDS at any degree
     const char* v = getenv("F2CGT_VQ_STRIP");
     const int mode = v ? atoi(v) : 0;     // 0 off; tens: 0 plain, 1 non-temporal, 2 no stores; units: 2 = KE by degree, 6 = KE 16
-    if (mode == 20) a.dense_store = 2;
+    if (mode == 20) a.probe_stores = 2;
     if (mode % 10 > 0 && avg_deg <= 24.0 && a.n_cb % BT == 0 && aligned(a.codes, BT) && a.feat_dim % 4 == 0) {
       VqArgs b = a;
-      b.dense_store = (mode / 10) % 10;
+      b.probe_stores = (mode / 10) % 10;
       if (mode >= 100) b.N = 1;   // experiment: every source id reads row 0
       const int ke = (mode % 10) == 6 ? 16 : (avg_deg <= 6.0 ? 8 : (avg_deg <= 10.0 ? 12 : 16));
       switch (a.w) {
@@ -1402,23 +1296,10 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
     }
   }
 #endif
-  // Codebooks of 32 columns: the four lanes that share a code can own its columns as a group, so that a store
-  // instruction writes 64 contiguous bytes per group at no cost in instructions (pair_pos; its own instantiation,
-  // OWN = 2).  Taken where the exchange inside quads is not and the code table stays cached.
-  a.own_lg = 0;
-  if (a.dense_store == 0 && a.w == 32 && a.feat_dim % 32 == 0 && a.feat_dim >= 128 &&
-      avg_deg <= 16.0 * ((a.R > 0 && a.E % a.R == 0) ? 1.0 : 0.9) && a.N * (int64_t)a.n_cb <= (192ll << 20))
-    a.own_lg = 2;
 #ifdef F2CGT_EXPERIMENTS
-  if (const char* v = getenv("F2CGT_VQ_STORE")) {   // the store form whatever the shape: plain | lds | quad | own | h1
-    const bool rpm4 = avg_deg <= 16.0 * ((a.R > 0 && a.E % a.R == 0) ? 1.0 : 0.9);
+  if (const char* v = getenv("F2CGT_VQ_STORE")) {   // lanes per row whatever the shape: h1 (32) | h2 (16)
     if (a.feat_dim % 8 == 0 && rpm4) {
-      if (!strcmp(v, "h1")) {
-        a.dense_store = 0; a.own_lg = 0;
-        return launch_wave<BT, 1, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
-      }
-      a.own_lg = (!strcmp(v, "own") && a.w == 32 && a.feat_dim % 32 == 0) ? 2 : 0;
-      a.dense_store = !strcmp(v, "lds") ? 1 : (!strcmp(v, "quad") ? 4 : 0);
+      if (!strcmp(v, "h1")) return launch_wave<BT, 1, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
       return launch_wave<BT, 2, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
     }
   }
@@ -1445,33 +1326,15 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
     // fixed fanout): those get the exact limits, ragged rows 0.9 of them (capped at 32 with 15.2 on average: 112 us
     // in fours, 91 in twos; capped at 64 with 30.1: 198 in twos, 171 one by one).
     const double fit = (a.R > 0 && a.E % a.R == 0) ? 1.0 : 0.9;
-    // Sparse rows that are no whole 128-byte lines (feat_dim no multiple of 32): one float4 per lane, 32 lanes per
-    // row, is ahead of the eight-column form whose results are turned round in LDS (3e6 edges at 3 / 6 per row:
-    // 25 x 8 326 / 165 -> 299 / 146 us, 21 x 8 299 / 150 -> 257 / 123, 15 x 8 186 / 102 -> 152 / 76, 19 x 32 at 600
-    // columns 603 / 313 -> 551 / 279; rows of whole lines the other way round: 24 x 8 172 / 101 against 191 / 100,
-    // 7 x 32 180 / 96 against 192 / 103).
-    // Above that, rows that are no whole 64-byte pieces (feat_dim an odd multiple of 8): the same, where the eight-column
-    // form has no exchange (more than four column tiles, or a table beyond the last-level cache) from 100 MB of output on,
-    // else from the size of the last-level cache on.  A last tile of few columns leaves most lanes of its workgroups idle,
-    // which counts for more the fewer tiles there are and the longer the rows (one graph again and again, Zipf(1.1) ids, this
-    // form's time over the other's: 136 columns at 9 to 14 edges per row 1.08 to 1.15, 152 at 9 to 12 up to 1.08, 264 up to
-    // 1.10; 168 columns at 12 up to 1.02, at 14 1.06 to 1.10; 200 at 14 up to 1.14; 520 and 648 at 14 1.06): up to 12 edges per
-    // row it is taken from 40 columns in the last tile on, or with more than three tiles, above that, up to 16 from a table
-    // beyond the last-level cache, from 80 on, 56 with more than three tiles.  Four graphs in turn, Zipf(1.1) / uniform ids,
-    // eight-column form -> this: 200 columns, 305 MB, at 10 126 -> 112 / 186 -> 172 us, at 12 118 -> 114 / 211 -> 199; from
-    // 480 MB of codes at 10 157 -> 136 / 223 -> 194; 600 columns, 457 MB, at 9 216 -> 149 / 181 -> 141, 114 MB at 12 51 -> 41 / 50 -> 42;
-    // 712 columns, 200 MB, at 10 90 -> 68 / 81 -> 65; 504 columns from 480 MB of codes at 14 0.70 of the time / 0.89.  One tile
-    // loses (104 columns 82 -> 96), and so do rows of whole 64-byte pieces (304 columns 97 -> 108, 144 columns 137 -> 149).
+    // Rows that are an odd multiple of 8 columns start at any 32 bytes: the 256-byte pieces of the eight-column form
+    // straddle lines, where one float4 per lane, 32 lanes per row, writes 512 bytes at a time.
     const int tail = a.feat_dim % 128;
     const bool filled = avg_deg <= 12.0 ? tail >= 40 || a.n_tiles > 3 : big_table && tail >= (a.n_tiles > 3 ? 56 : 80);
-    const bool split_rows = a.feat_dim % 16 == 8 && a.n_tiles > 1 && rpm4 && filled && store_mode() != F2CGT_STORE_STREAM &&
-                            out_bytes >= (a.n_tiles > 4 || big_table ? 100000000ll : 256ll << 20);
-    if ((avg_deg <= 8.0 && a.feat_dim % 32 != 0) || split_rows) {
-      a.dense_store = 0;
-      a.own_lg = 0;
-      return launch_wave<BT, 1, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
-    }
-    if (avg_deg <= 16.0 * fit) return launch_wave<BT, 2, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
+    const bool split_rows = a.feat_dim % 16 == 8 && a.n_tiles > 1 &&
+                            (avg_deg <= 8.0 || (rpm4 && filled && out_bytes >= (a.n_tiles > 4 || big_table ? 100000000ll : 256ll << 20)));
+    if (split_rows) return launch_wave<BT, 1, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
+    if (avg_deg <= 16.0 * fit)
+      return launch_wave<BT, 2, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds, form, owners);
     if (avg_deg <= 32.0 * fit) return launch_wave<BT, 2, 2>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
     return launch_wave<BT, 2, 1>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
   } else if (avg_deg <= 15.0 || a.n_cb % BT != 0 || !aligned(a.codes, BT) || a.feat_dim % 4 != 0) {
@@ -1508,7 +1371,7 @@ bool vq_pipe_eligible(const void* codes, const float* codebooks, const float* ou
   if (w != 8 && w != 16 && w != 32) return false;
   if (feat_dim < 16 || feat_dim % 2 != 0 || feat_dim > n_cb * w) return false;
   if (!aligned(out, 16) || !aligned(codebooks, 4)) return false;
-  if (N >= (1ll << 32)) return false;
+  if (N >= (1ll << 32) || feat_dim > (1 << 27)) return false;   // row offsets of a step inside the buffer's 2 GB
   if (R < 4 * kRows) return false;  // tiny problems: the per-row skeleton has less start-up cost
   return true;
 }

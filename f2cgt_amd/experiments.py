@@ -339,12 +339,10 @@ def vq_degrees(_):
 
 
 def vq_store_forms(how):
-    """The fused VQ kernel's ways of storing a lane's eight columns (F2CGT_VQ_STORE; experiments build): as they are
-    (two 16-byte stores that each write 16 of every 32 bytes), turned round in LDS (256 contiguous bytes per row and
-    instruction), halves exchanged inside lane quads (64 contiguous bytes), columns owned by groups of four lanes
-    (codebooks of 32 columns: 64 contiguous bytes at no cost in instructions), and one float4 per lane (32 lanes per
-    row).  `warm`: one graph and one output; `rotate`: five graphs and outputs in turn, so that neither the source ids
-    nor the output lines of a launch are cached when it starts."""
+    """The fused VQ kernel's two lane layouts (F2CGT_VQ_STORE; experiments build): 16 lanes of eight columns per row, whose
+    halves are exchanged between the halves of the wave before they are stored (256 contiguous bytes per row and
+    instruction), and 32 lanes of one float4 (512).  `warm`: one graph and one output; `rotate`: five graphs and outputs
+    in turn, so that neither the source ids nor the output lines of a launch are cached when it starts."""
     import torch
 
     sys.path.insert(0, ROOT)
@@ -368,9 +366,8 @@ def vq_store_forms(how):
         torch.cuda.synchronize()
         return t0.elapsed_time(t1) / steps * 1e3
 
-    forms = ("", "plain", "lds", "quad", "own", "h1")
-    print("us per launch (%s): shipped | plain | through LDS | quad exchange | groups of four lanes | one float4 per lane"
-          % how)
+    forms = ("", "h2", "h1")
+    print("us per launch (%s): shipped | eight columns per lane | one float4 per lane" % how)
     shapes = [(1_000_000, d, w, f, 3_000_000 if d <= 256 else 2_000_000)
               for w, d in ((8, 128), (8, 256), (8, 512), (8, 768), (16, 128), (16, 256), (16, 512), (32, 128), (32, 256),
                            (32, 768), (8, 64), (8, 200), (32, 600))
@@ -389,16 +386,13 @@ def vq_store_forms(how):
         res = []
         for form in forms:
             os.environ.pop("F2CGT_VQ_STORE", None)
-            if form == "own" and not (w == 32 and dim % 32 == 0):
-                res.append(float("nan"))
-                continue
             if form:
                 os.environ["F2CGT_VQ_STORE"] = form
             res.append(timed(fns))
         os.environ.pop("F2CGT_VQ_STORE", None)
         print("  %9d source rows, %3d columns as %2d x %-2d, %2d edges per row, %4d MB out: " % (
             n_src, dim, n_cb, w, fanout, rows * dim * 4 // 1_000_000)
-            + " | ".join("     -" if r != r else "%6.1f" % r for r in res), flush=True)
+            + " | ".join("%6.1f" % r for r in res), flush=True)
         del codes, ids, outs, fns
         torch.cuda.empty_cache()
 
