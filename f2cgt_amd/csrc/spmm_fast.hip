@@ -1018,19 +1018,19 @@ __device__ __forceinline__ float mean_of(float sum, float d, float r) {
   return __fmaf_rn(__fmaf_rn(-q, d, sum), r, q);
 }
 
-// Adds the first G 1-bit values of a code byte to s: +plus where the bit is set, -plus where it is not, the two values a
-// 1-bit log-domain codebook has.  The bits become the signs of halves (-1 or 1, two per instruction) and the sums
-// fma(+-1, -plus, s), which rounds as the addition does: two instructions per value and no table read.
-template <int G>
-__device__ __forceinline__ void add_signs(float (&s)[G], uint32_t byte, float minus_plus) {
-  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-  const uint32_t w = byte | (byte << (16 - G / 2));   // bit i at i, bit i + G / 2 at i + 16
+// Adds the eight 1-bit values of a code byte to s: +plus where the bit is set, -plus where it is not, the two values a
+// 1-bit log-domain codebook has.  A nibble's four signs come out of LDS as halves (1 or -1 each; sixteen entries that lie
+// in banks of their own, so that no two lanes ever wait for each other) and the sums are fma(+-1, -plus, s), which rounds
+// as the addition does: eleven instructions for eight values.  (Signs made from the bits, two per instruction: 16 to 20.)
+typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+constexpr int kSignTable = 256;   // bytes: sixteen entries, 16 bytes apart
+__device__ __forceinline__ void add_signs(float (&s)[8], uint32_t byte, const unsigned char* signs, float minus_plus) {
+  const half4v lo = *reinterpret_cast<const half4v*>(signs + ((byte << 4) & 0xf0u));
+  const half4v hi = *reinterpret_cast<const half4v*>(signs + (byte & 0xf0u));
 #pragma unroll
-  for (int i = 0; i < G / 2; ++i) {
-    const uint32_t pair = ((w << (15 - i)) & 0x80008000u) | 0x3c003c00u;
-    const half2v h = __builtin_bit_cast(half2v, pair);
-    s[i] = __builtin_fmaf((float)h[0], minus_plus, s[i]);
-    s[i + G / 2] = __builtin_fmaf((float)h[1], minus_plus, s[i + G / 2]);
+  for (int i = 0; i < 4; ++i) {
+    s[i] = __builtin_fmaf((float)lo[i], minus_plus, s[i]);
+    s[i + 4] = __builtin_fmaf((float)hi[i], minus_plus, s[i + 4]);
   }
 }
 
@@ -1040,6 +1040,9 @@ __device__ __forceinline__ void add_signs(float (&s)[G], uint32_t byte, float mi
 // (3e6 edges, 10 per row, 4 bit: 97.8 -> 93.7 us at 128 columns, 592 -> 489 us at 600); 1- and 2-bit rows measured
 // level to 2 % slower and keep the run-time test.
 // ITEM: 0 (a lane keeps a column group), or the columns of the items that are dealt to the lanes: 4, or 8 (1 bit).
+// The eight columns of a 1-bit item are stored after the two halves of the wave have exchanged theirs
+// (v_permlane32_swap): the lower lanes' items go out with one store instruction, 16 bytes per lane one after the other,
+// the upper lanes' with the next, where a lane's own two 16-byte stores would each write 16 of every 32 bytes.
 template <int BITS, bool AFFINE, typename Idx, int TB, int HALF = 0, int ITEM = 0>
 __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __restrict__ indptr,
                                                              const Idx* __restrict__ indices,
@@ -1049,7 +1052,8 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
   constexpr int NCODE = 1 << BITS;
   constexpr uint32_t MASK = NCODE - 1;
   extern __shared__ __align__(16) unsigned char smem[];
-  float* s_lut = reinterpret_cast<float*>(smem);
+  constexpr bool SIGNS = ITEM != 0 && BITS == 1;
+  float* s_lut = reinterpret_cast<float*>(smem + (SIGNS ? kSignTable : 0));
   const int lut_floats = AFFINE ? 0 : ((a.num_codebooks * NCODE + 3) & ~3);
   int* s_ptr = reinterpret_cast<int*>(s_lut + lut_floats);                       // [RB + 1] (+3 pad)
   int* s_cnt = s_ptr + a.rows_per_block + 4;                                     // [16] rows per degree class
@@ -1071,6 +1075,14 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
     s_ptr[i] = (int)(v - e0 > 0x7fffffff ? 0x7fffffff : v - e0);
   }
   if (t < 16) s_cnt[t] = 0;
+  if constexpr (SIGNS) {   // entry q: half i is -1 where bit i of q is set (the sums take -plus times it)
+    if (t < 16) {
+      half4v h;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) h[i] = (t >> i) & 1 ? (_Float16)-1.f : (_Float16)1.f;
+      *reinterpret_cast<half4v*>(smem + 16 * t) = h;
+    }
+  }
   if (!AFFINE) {
     for (int i = t; i < a.num_codebooks * NCODE; i += TB) {
       const float* cb = a.table + (int64_t)(i >> BITS) * 5;
@@ -1148,14 +1160,86 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
   __syncthreads();
 
   if constexpr (ITEM != 0) {
-    // decode + sum: (row, column group) items dealt to the lanes one after the other.  Bound by instruction issue: 60001
-    // rows of 602 columns, 10 edges per row, 1 bit, execute 30.9 million vector instructions (5.5 per wave of values, ids
-    // and addresses included), 50 us of the 58 at four clocks each; the vector ALUs are active in 99 % of the CUs' busy
-    // clocks.  The output goes out at 2.5 TB/s (staged rows with a column group per lane: 0.9 TB/s).
+    // decode + sum: (row, column group) items dealt to the lanes one after the other.  60001 rows of 602 columns, up to 20
+    // edges per row, 1 bit, streamed output: 58.1 us with signs made from the bits and items of four columns (30.9 million
+    // vector instructions, 50 us of issue), 46.7 with the sign table and eight columns exchanged for the store (21.6
+    // million, 35 us; the output alone takes 30).  Tried beside it: eight edges per trip (no faster, 4 to 20 % slower with
+    // two or three edges per row), row offsets instead of ids in LDS (the same), the code bits as scalar masks (one
+    // select and one addition per 64 values, but 70 us: the scalar cache takes a new line every dozen clocks).
     constexpr int G = ITEM;                              // columns of an item
-    constexpr int GB = G * BITS < 8 ? 1 : G * BITS / 8;  // code bytes that hold them
+    constexpr int GB = G * BITS / 8;                     // code bytes that hold them
     const int items = nrows * a.items_per_row;
-    const float minus_plus = -s_lut[1];
+    if constexpr (SIGNS) {
+      const float minus_plus = -s_lut[1];
+      const int lane = t & 63;
+      char* obase = reinterpret_cast<char*>(out + row0 * (int64_t)a.feat_dim);
+      for (int first = t - lane; first < items; first += TB) {     // the same for all lanes of a wave
+        const int item = first + lane < items ? first + lane : items - 1;
+        const int ri = (int)__umulhi((uint32_t)item, a.item_magic);
+        const int c = item - ri * a.items_per_row;
+        const int r = s_order[ri];
+        const int b = s_ptr[r], e = s_ptr[r + 1];
+        float s[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[i] = 0.f;
+        const uint8_t* column = a.codes + c;
+        auto code_at = [&](uint32_t id) -> uint32_t { return column[(uint64_t)id * (uint32_t)a.src_dim]; };
+        auto walk = [&](auto read) {
+          int k = b;
+          for (; k + 4 <= e; k += 4) {
+            const uint32_t w0 = read(k), w1 = read(k + 1), w2 = read(k + 2), w3 = read(k + 3);
+            add_signs(s, w0, smem, minus_plus);
+            add_signs(s, w1, smem, minus_plus);
+            add_signs(s, w2, smem, minus_plus);
+            add_signs(s, w3, smem, minus_plus);
+          }
+          if (k + 2 <= e) {
+            const uint32_t w0 = read(k), w1 = read(k + 1);
+            add_signs(s, w0, smem, minus_plus);
+            add_signs(s, w1, smem, minus_plus);
+            k += 2;
+          }
+          if (k < e) add_signs(s, read(k), smem, minus_plus);
+        };
+        if (have_ids) walk([&](int k) -> uint32_t { return code_at(s_ids[k]); });
+        else walk([&](int k) -> uint32_t { return code_at((uint32_t)clamp_idx(indices[e0 + k], a.N)); });
+        const int deg = e - b;
+        if (deg > 1) {
+          const float d = (float)deg;
+          float rc = __builtin_amdgcn_rcpf(d);
+          rc = __fmaf_rn(__fmaf_rn(-d, rc, 1.f), rc, rc);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) s[i] = mean_of(s[i], d, rc);
+        }
+        // Where the item's eight columns go, and how many of them the row has (two, four, six or eight); lanes without
+        // an item of their own have none.
+        const uint32_t at = ((uint32_t)r * (uint32_t)a.feat_dim + 8u * (uint32_t)c) * 4u;
+        const int left = first + lane < items ? (a.feat_dim - 8 * c < 8 ? a.feat_dim - 8 * c : 8) : 0;
+        const uint32_t where = at | (uint32_t)left >> 1;      // a multiple of 8 plus 0, 1, 2, 3 or 4
+        const auto own = __builtin_amdgcn_permlane32_swap(where, where, false, false);
+        float v[2][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(s[i]), __float_as_uint(s[4 + i]), false, false);
+          v[0][i] = __uint_as_float(x[0]);
+          v[1][i] = __uint_as_float(x[1]);
+        }
+        const int h = lane >> 5;                              // the half of an item that the lane stores
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {                         // the lower lanes' items, the upper lanes'
+          float* dst = reinterpret_cast<float*>(obase + ((own[p] & ~7u) + 16u * (uint32_t)h));
+          const int pairs = (int)(own[p] & 7u) - 2 * h;       // column pairs of this half
+          if (pairs >= 2) {
+            if constexpr (HALF == 2) store_nt4_align8(dst, v[p][0], v[p][1], v[p][2], v[p][3]);
+            else store4_align8(dst, v[p][0], v[p][1], v[p][2], v[p][3]);
+          } else if (pairs == 1) {
+            if constexpr (HALF == 2) store_nt2(dst, v[p][0], v[p][1]);
+            else *reinterpret_cast<float2*>(dst) = make_float2(v[p][0], v[p][1]);
+          }
+        }
+      }
+      return;
+    }
     for (int item = t; item < items; item += TB) {
       const int ri = (int)__umulhi((uint32_t)item, a.item_magic);
       const int c = item - ri * a.items_per_row;
@@ -1170,24 +1254,19 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
       // issued together (with a branch per load they were waited for one by one: 1000 rows of 300 edges, 128
       // columns, 4 bit 129 -> 64 us; 30000 rows of power-law degrees, 100 columns, 4 bit 105 -> 59, 8 bit 112 -> 59).
       const bool half = GB > 1 && HALF != 0 && left < G;
-      const int first = c * (G * BITS) / 8;              // first code byte; four 1-bit codes start at bit 0 or 4 of it
-      const uint32_t bit = G * BITS < 8 ? (uint32_t)(c * (G * BITS)) & 7u : 0u;
+      const int first = c * (G * BITS) / 8;              // first code byte
       const uint32_t at = (uint32_t)(first - (half ? GB / 2 : 0));
       const uint32_t sh = half ? 4 * GB : 0;
       auto code_at = [&](uint32_t id) -> uint32_t {
         const uint8_t* q = a.codes + ((uint64_t)id * (uint32_t)a.src_dim + at);
-        if constexpr (GB == 1) return (uint32_t)*q >> bit;
+        if constexpr (GB == 1) return (uint32_t)*q;
         uint32_t w = 0;
         __builtin_memcpy(&w, q, GB);
         return w >> sh;
       };
       auto add = [&](uint32_t w) {
-        if constexpr (BITS == 1) {
-          add_signs<G>(s, w, minus_plus);
-        } else {
 #pragma unroll
-          for (int i = 0; i < G; ++i) s[i] += s_lut[(w >> (BITS * i)) & MASK];
-        }
+        for (int i = 0; i < G; ++i) s[i] += s_lut[(w >> (BITS * i)) & MASK];
       };
       auto walk = [&](auto read) {
         int k = b;
@@ -1207,7 +1286,7 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
           const unsigned char* q = s_codes + k * a.pitch + first;
           if constexpr (GB == 4) return *reinterpret_cast<const uint32_t*>(q);
           else if constexpr (GB == 2) return *reinterpret_cast<const uint16_t*>(q);
-          else return (uint32_t)*q >> bit;
+          else return (uint32_t)*q;
         });
       } else if (have_ids) {
         walk([&](int k) -> uint32_t { return code_at(s_ids[k]); });
@@ -1365,12 +1444,7 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
                            a.R > 0 ? (double)a.E / (double)a.R : 0.0) ? 1 : 0;
   const size_t lut_bytes = AFFINE ? 0 : (size_t)(((a.num_codebooks << BITS) + 3) & ~3) * 4;
   const double avg_deg = a.R > 0 ? (double)a.E / (double)a.R : 1.0;
-  // 1-bit items of eight columns read a code byte once, but a lane's two 16-byte stores have every store instruction
-  // write 16 of every 32 bytes, which streamed stores take to memory as partial lines: streamed outputs take items of
-  // four columns, whose stores are contiguous (240000 rows of 256 columns: 115 us with eight, 46 with four at one edge
-  // per row, 81 and 71 at eight; 60001 x 602 at 10 edges per row: 65.6 and 57.8).  Cached outputs take eight columns
-  // (1000 rows of 300 columns, one edge per row: 4.0 against 4.4 us; 60000 rows of 128 columns, level).
-  const bool wide = DEAL && BITS == 1 && !a.nt_out;
+  const bool wide = DEAL && BITS == 1;   // items of eight columns: a code byte
   a.items_per_row = (int)ceil_div(a.feat_dim, wide ? 8 : 4);
   a.item_magic = (uint32_t)(((1ull << 32) + a.items_per_row - 1) / a.items_per_row);   // items < 64 * 1024: exact
   const double dg = avg_deg > 0.5 ? avg_deg : 0.5;
@@ -1425,7 +1499,7 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
     if (direct) a.id_cap = need < 2048 ? need : 2048;
     else a.id_cap = a.edge_cap = need < a.edge_cap ? need : a.edge_cap;
   }
-  const size_t lds = lut_bytes + (size_t)(rb + 4) * 4 + 64 + (size_t)rb * 4 + (size_t)a.id_cap * 4 +
+  const size_t lds = (wide ? kSignTable : 0) + lut_bytes + (size_t)(rb + 4) * 4 + 64 + (size_t)rb * 4 + (size_t)a.id_cap * 4 +
                      (size_t)a.edge_cap * a.pitch + 16;
   const int64_t grid = ceil_div(a.R, rb);
   if (grid > 0x7fffffffll) return fail(F2CGT_E_UNSUPPORTED, "%s: too many row blocks", what);
@@ -1445,7 +1519,7 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
       if (half == 0) F2CGT_ROWS_GO(I, 0, DEAL ? 4 : 0);                          \
     }                                                                            \
     if (half == 1) F2CGT_ROWS_GO(I, 1, DEAL ? (BITS == 1 ? 8 : 4) : 0);          \
-    else if (half == 2) F2CGT_ROWS_GO(I, 2, DEAL ? 4 : 0);                       \
+    else if (half == 2) F2CGT_ROWS_GO(I, 2, DEAL ? (BITS == 1 ? 8 : 4) : 0);     \
   } while (0)
   if (idx_dtype == F2CGT_DT_I32) F2CGT_ROWS_IDX(int32_t);
   else F2CGT_ROWS_IDX(int64_t);
