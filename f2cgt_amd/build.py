@@ -21,7 +21,7 @@ OBJ = os.path.join(PKG, "build")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 HIP_SOURCES = ["runtime.hip", "packbits.hip", "sq.hip", "vq.hip", "spmm.hip", "spmm_fast.hip",
-               "vq_fast.hip", "assign.hip", "encode.hip", "fetch.hip", "kmeans.hip", "stats.hip"]
+               "vq_fast.hip", "assign.hip", "encode.hip", "fetch.hip", "kmeans.hip", "stats.hip", "sage.hip"]
 EXPERIMENT_SOURCES = ["overlap_probe.hip", "lds_rate_probe.hip"]   # compiled into the --experiments build only
 HIP_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-ffp-contract=off",

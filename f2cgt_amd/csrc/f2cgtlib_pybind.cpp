@@ -19,6 +19,12 @@
 #include <string>
 #include <vector>
 
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/forward_grad.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+
 #include "../../include/f2cgt.h"
 
 namespace py = pybind11;
@@ -941,6 +947,92 @@ torch::Tensor sq_decompress_rows(torch::Tensor table, torch::Tensor index, torch
   return sq_decompress(fetch_rows(table, index, c10::nullopt, c10::nullopt), codebooks, target_bits, column_slice, feat_dim);
 }
 
+// ---- the dense part of a GraphSAGE layer in one kernel each way ---------------------------------------
+using torch::autograd::AutogradContext;
+using torch::autograd::Variable;
+using torch::autograd::variable_list;
+
+// act(x0 w0^T + x1 w1^T + bias); only w0, w1 and bias are differentiated.
+struct SageLinear : public torch::autograd::Function<SageLinear> {
+  static Variable forward(AutogradContext* ctx, const Variable& x0, const Variable& x1, const Variable& w0, const Variable& w1,
+                          const c10::optional<Variable>& bias, bool relu) {
+    c10::DeviceGuard guard(x0.device());
+    const int64_t m = x0.size(0), n = w0.size(0);
+    auto out = torch::empty({m, n}, x0.options());
+    check_rc(f2cgt_sage_linear(x0.data_ptr<float>(), w0.data_ptr<float>(), x1.data_ptr<float>(), w1.data_ptr<float>(),
+                               bias.has_value() ? bias->data_ptr<float>() : nullptr, out.data_ptr<float>(), m, n, x0.size(1),
+                               x1.size(1), relu ? 1 : 0, current_stream()),
+             "sage_linear");
+    ctx->saved_data["relu"] = relu;
+    ctx->saved_data["bias"] = bias.has_value();
+    if (relu) ctx->save_for_backward({x0, x1, out});
+    else ctx->save_for_backward({x0, x1});
+    return out;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const bool relu = ctx->saved_data["relu"].toBool();
+    const Variable& x0 = saved[0];
+    const Variable& x1 = saved[1];
+    const bool want0 = ctx->needs_input_grad(2), want1 = ctx->needs_input_grad(3), want_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(4);
+    variable_list result(6);
+    Variable g = grads[0];
+    if (!g.defined() || !(want0 || want1 || want_b)) return result;
+    if (c10::GradMode::is_enabled() || !g.is_cuda() || g.scalar_type() != torch::kFloat32 || g.layout() != torch::kStrided) {
+      // a gradient that is differentiated itself: the same sums from operators that are
+      if (relu) g = at::threshold_backward(g, saved[2], 0);
+      if (want0) result[2] = g.t().mm(x0);
+      if (want1) result[3] = g.t().mm(x1);
+      if (want_b) result[4] = g.sum(0);
+      return result;
+    }
+    g = g.contiguous();
+    c10::DeviceGuard guard(g.device());
+    const int64_t m = x0.size(0), n = g.size(1), k0 = x0.size(1), k1 = x1.size(1);
+    if (want0) result[2] = torch::empty({n, k0}, g.options());
+    if (want1) result[3] = torch::empty({n, k1}, g.options());
+    if (want_b) result[4] = torch::empty({n}, g.options());
+    auto ptr = [](const Variable& v) { return v.defined() ? v.data_ptr<float>() : nullptr; };
+    torch::Tensor ws;
+    const int64_t bytes = f2cgt_sage_linear_grad_workspace_bytes(m, n, k0, k1);
+    if (bytes > 0) ws = torch::empty({bytes}, g.options().dtype(torch::kUInt8));
+    check_rc(f2cgt_sage_linear_grad(g.data_ptr<float>(), relu ? saved[2].data_ptr<float>() : nullptr, x0.data_ptr<float>(),
+                                    x1.data_ptr<float>(), ptr(result[2]), ptr(result[3]), ptr(result[4]),
+                                    bytes > 0 ? ws.data_ptr() : nullptr, bytes, m, n, k0, k1, current_stream()),
+             "sage_linear_grad");
+    return result;
+  }
+};
+
+// -> the layer's output, or None for the calls that are left to the module's own operators: other types, layouts, devices
+// and sizes; inputs that are differentiated; and whenever an operator's call would not go straight to the device
+// (transforms, forward-mode gradients, autocast, dispatch and function modes, tracing).
+c10::optional<torch::Tensor> sage_linear(const torch::Tensor& x0, const torch::Tensor& x1, const torch::Tensor& w0,
+                                         const torch::Tensor& w1, const c10::optional<torch::Tensor>& bias, bool relu) {
+  using c10::DispatchKey;
+  static const c10::DispatchKeySet plain_keys = c10::DispatchKeySet({DispatchKey::CUDA, DispatchKey::AutogradCUDA,
+                                                                     DispatchKey::ADInplaceOrView, DispatchKey::AutocastCUDA});
+  static const c10::DispatchKeySet plain_tls = c10::DispatchKeySet({DispatchKey::BackendSelect, DispatchKey::ADInplaceOrView});
+  auto plain = [&](const torch::Tensor& t, int64_t dims) {
+    return t.defined() && (t.key_set() | plain_keys) == plain_keys && t.scalar_type() == torch::kFloat32 &&
+           t.layout() == torch::kStrided && t.dim() == dims && t.is_contiguous() && t.device() == x0.device() &&
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  const auto tls = c10::impl::tls_local_dispatch_key_set();
+  if (!((tls.included_ | plain_tls) == plain_tls) || at::autocast::is_autocast_enabled(at::kCUDA) || at::impl::PythonTorchFunctionTLS::stack_len() > 0 || torch::jit::tracer::isTracing() ||
+      torch::autograd::ForwardADLevel::try_get_by_idx(0) != nullptr)
+    return c10::nullopt;
+  if (!plain(x0, 2) || !plain(x1, 2) || !plain(w0, 2) || !plain(w1, 2) || (bias.has_value() && !plain(*bias, 1)))
+    return c10::nullopt;
+  const int64_t m = x0.size(0), n = w0.size(0), k0 = x0.size(1), k1 = x1.size(1);
+  if (x0.requires_grad() || x1.requires_grad() || m < 1 || n < 1 || k0 < 4 || k1 < 4 || k0 % 4 != 0 || k1 % 4 != 0 ||
+      x1.size(0) != m || w1.size(0) != n || w0.size(1) != k0 || w1.size(1) != k1 || (bias.has_value() && bias->size(0) != n) ||
+      !f2cgt_sage_linear_ahead(m, n, k0, k1))
+    return c10::nullopt;
+  return SageLinear::apply(x0, x1, w0, w1, bias, relu);
+}
+
 torch::Tensor vq_encode(torch::Tensor x, torch::Tensor centers, std::string metric) {
   return kmeans_predict_impl(x, centers, metric, true);
 }
@@ -1028,6 +1120,8 @@ PYBIND11_MODULE(F2CGTLib, m) {
       .def("sq_decompress_rows", &sq_decompress_rows, py::arg("table"), py::arg("index"), py::arg("codebooks"),
            py::arg("target_bits"), py::arg("column_slice"), py::arg("feat_dim"), py::arg("slot_map") = py::none(),
            py::arg("check") = false)
+      .def("sage_linear", &sage_linear, py::arg("h_self"), py::arg("h_neigh"), py::arg("w_self"), py::arg("w_neigh"),
+           py::arg("bias"), py::arg("relu"))
       .def("fetch_rows", &fetch_rows, py::arg("table"), py::arg("index"), py::arg("hot") = py::none(),
            py::arg("slot_map") = py::none())
       .def("kmeans_update", &kmeans_update, py::arg("data"), py::arg("labels"), py::arg("centers"),

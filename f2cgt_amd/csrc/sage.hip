@@ -1,0 +1,273 @@
+// The dense part of a GraphSAGE layer on a minibatch (examples/conv.py:68-76): fc_self(h_self) + fc_neigh(h_neigh), with
+// bias and ReLU, and the gradients of its parameters, each one launch on the fp32 matrix instructions.
+//
+// What bounds it: at a minibatch's sizes (a thousand destination rows, 128 + 128 columns, 256 outputs: 67 million
+// multiply-adds, half a microsecond of matrix time) launches and host time; two library products, an addition and an
+// activation forward and two products, a reduction and a mask backward cost the host 200 us a step.  Hence one kernel each
+// way, with tiles small enough that a launch of that size still covers the chip.
+#include "common.hpp"
+
+namespace f2cgt {
+namespace {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+constexpr int kTile = 32;            // rows and outputs of a tile: one 32 x 32 x 2 matrix instruction
+constexpr int kForwardWaves = 4;     // they share a tile's columns
+constexpr int kGradWaves = 16;       // they share a tile's rows
+
+struct SageArgs {
+  const float* x[2];                 // h_self, h_neigh: [m, k[s]]
+  const float* w[2];                 // [n, k[s]]
+  const float* bias;                 // [n] or null
+  float* out;                        // [m, n]
+  int64_t m;
+  int n, k[2], relu;
+};
+
+// out = x0 w0^T + x1 w1^T + bias, a 32 x 32 tile per workgroup; its waves take the columns 32 at a time in turn, so that
+// 1024 rows and 256 outputs make 256 workgroups, and add their tiles in LDS.
+// Lane l of the matrix instruction has row l % 32 of x and of w and one of its two columns; here columns 4 (l / 32) + t
+// of every eight are those of the instruction's step t, so that a lane reads 16 bytes of its row at a time.
+__global__ __launch_bounds__(kForwardWaves * kWave) void sage_linear_kernel(SageArgs a) {
+  __shared__ __align__(16) float s_tile[kForwardWaves][kTile][kTile + 4];
+  const int t = threadIdx.x, wave = t / kWave, lane = t & (kWave - 1), at = lane & 31, side = lane >> 5;
+  const int64_t m0 = (int64_t)blockIdx.x * kTile;
+  const int n0 = blockIdx.y * kTile;
+  const int64_t row = m0 + at < a.m ? m0 + at : a.m - 1;
+  const int col = n0 + at < a.n ? n0 + at : a.n - 1;
+  const int chunks0 = (a.k[0] + 31) / 32, chunks = chunks0 + (a.k[1] + 31) / 32;
+  float4 x[4], w[4];
+  auto load = [&](int c) {
+    const int s = c >= chunks0 ? 1 : 0;
+    const int k = a.k[s], k0 = (c - (s ? chunks0 : 0)) * 32 + 4 * side;
+    const float* xr = a.x[s] + row * k;
+    const float* wr = a.w[s] + (int64_t)col * k;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int kq = k0 + 8 * q;
+      const bool in = kq < k;                              // (a multiple of four columns: all four or none)
+      x[q] = *reinterpret_cast<const float4*>(xr + (in ? kq : 0));
+      w[q] = *reinterpret_cast<const float4*>(wr + (in ? kq : 0));
+      if (!in) x[q] = w[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  floatx16 acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+  if (wave < chunks) load(wave);
+  for (int c = wave; c < chunks; c += kForwardWaves) {
+    float4 xc[4], wc[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) { xc[q] = x[q]; wc[q] = w[q]; }
+    if (c + kForwardWaves < chunks) load(c + kForwardWaves);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xc[q].x, wc[q].x, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xc[q].y, wc[q].y, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xc[q].z, wc[q].z, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xc[q].w, wc[q].w, acc, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 16; ++v) s_tile[wave][8 * (v / 4) + 4 * side + v % 4][at] = acc[v];
+  __syncthreads();
+  const int r = t / 8, c4 = t % 8 * 4;
+  float v[4];
+  {
+    float4 sum = *reinterpret_cast<const float4*>(&s_tile[0][r][c4]);
+#pragma unroll
+    for (int i = 1; i < kForwardWaves; ++i) {
+      const float4 p = *reinterpret_cast<const float4*>(&s_tile[i][r][c4]);
+      sum.x += p.x; sum.y += p.y; sum.z += p.z; sum.w += p.w;
+    }
+    v[0] = sum.x; v[1] = sum.y; v[2] = sum.z; v[3] = sum.w;
+  }
+  if (m0 + r >= a.m) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = n0 + c4 + i;
+    if (a.bias != nullptr) v[i] += a.bias[c < a.n ? c : a.n - 1];
+    if (a.relu) v[i] = v[i] <= 0.f ? 0.f : v[i];           // (a NaN stays one)
+  }
+  float* dst = a.out + (m0 + r) * a.n + n0 + c4;
+  if ((a.n & 3) == 0) {
+    if (n0 + c4 < a.n) *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (n0 + c4 + i < a.n) dst[i] = v[i];
+  }
+}
+
+struct SageGradArgs {
+  const float* grad;                 // [m, n]
+  const float* out;                  // [m, n] for the ReLU's mask, or null
+  const float* x[2];
+  float* dw[2];                      // [n, k[s]]
+  float* db;                         // [n]
+  float* part;                       // [splits][n * (k0 + k1) + n], or null: straight into dw and db
+  int64_t m, rows_per_split;
+  int n, k[2];
+};
+
+// dw[s] = (grad masked)^T x[s], db = column sums of it: a 32 x 32 tile of a weight per workgroup, whose sixteen waves share
+// the rows and add their tiles in LDS in a fixed order; many rows are split over the grid too, the parts added afterwards.
+__global__ __launch_bounds__(kGradWaves * kWave) void sage_grad_kernel(SageGradArgs a) {
+  __shared__ float s_tile[kGradWaves / 2][kTile][kTile];
+  __shared__ float s_bias[kGradWaves][kTile];
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / kWave), lane = t & (kWave - 1), at = lane & 31, side = lane >> 5;
+  const int n0 = blockIdx.x * kTile;
+  const int tiles0 = (a.k[0] + kTile - 1) / kTile;
+  const int s = (int)blockIdx.y >= tiles0 ? 1 : 0;
+  const int k = a.k[s], k0 = ((int)blockIdx.y - (s ? tiles0 : 0)) * kTile;
+  const bool bias = blockIdx.y == 0;
+  const bool n_in = n0 + at < a.n, k_in = k0 + at < k;
+  const float* __restrict__ g = a.grad + (n_in ? n0 + at : a.n - 1);
+  const float* __restrict__ o = a.out != nullptr ? a.out + (n_in ? n0 + at : a.n - 1) : nullptr;
+  const float* __restrict__ x = a.x[s] + (k_in ? k0 + at : k - 1);
+  const int64_t first = (int64_t)blockIdx.z * a.rows_per_split;
+  const int64_t end = first + a.rows_per_split < a.m ? first + a.rows_per_split : a.m;
+  constexpr int U = 8;                                     // row pairs in flight
+  floatx16 acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+  float sum = 0.f;
+  for (int64_t r0 = first + wave * (2 * U); r0 < end; r0 += kGradWaves * 2 * U) {
+    float gv[U], ov[U], xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      int64_t r = r0 + 2 * u + side;
+      r = r < end ? r : end - 1;
+      gv[u] = g[r * a.n];
+      xv[u] = x[r * k];
+      if (o != nullptr) ov[u] = o[r * a.n];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = r0 + 2 * u + side < end;
+      float v = in && n_in ? gv[u] : 0.f;
+      if (o != nullptr) v = ov[u] <= 0.f ? 0.f : v;        // (as the ReLU's own gradient: a NaN passes it on)
+      sum += v;
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(v, in && k_in ? xv[u] : 0.f, acc, 0, 0, 0);
+    }
+  }
+  if (wave >= kGradWaves / 2) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s_tile[wave - kGradWaves / 2][8 * (v / 4) + 4 * side + v % 4][at] = acc[v];
+  }
+  sum += __shfl_xor(sum, 32);
+  if (side == 0) s_bias[wave][at] = sum;
+  __syncthreads();
+  if (wave < kGradWaves / 2) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s_tile[wave][8 * (v / 4) + 4 * side + v % 4][at] += acc[v];
+  }
+  __syncthreads();
+  const int64_t words = (int64_t)a.n * (a.k[0] + a.k[1]) + a.n;
+  float* dw = a.part != nullptr ? a.part + blockIdx.z * words + (s ? (int64_t)a.n * a.k[0] : 0) : a.dw[s];
+  float* db = a.part != nullptr ? a.part + blockIdx.z * words + (int64_t)a.n * (a.k[0] + a.k[1]) : a.db;
+  const int r = t / kTile, c = t % kTile;                  // a value per thread
+  if (n0 + r < a.n && k0 + c < k && dw != nullptr) {
+    float v = s_tile[0][r][c];
+#pragma unroll
+    for (int i = 1; i < kGradWaves / 2; ++i) v += s_tile[i][r][c];
+    dw[(int64_t)(n0 + r) * k + k0 + c] = v;
+  }
+  if (bias && t < kTile && n0 + t < a.n && db != nullptr) {
+    float v = s_bias[0][t];
+#pragma unroll
+    for (int i = 1; i < kGradWaves; ++i) v += s_bias[i][t];
+    db[n0 + t] = v;
+  }
+}
+
+__global__ __launch_bounds__(256) void sage_grad_add_kernel(SageGradArgs a, int splits) {
+  const int64_t words0 = (int64_t)a.n * a.k[0], words1 = (int64_t)a.n * a.k[1], words = words0 + words1 + a.n;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= words) return;
+  float v = 0.f;
+#pragma unroll 8
+  for (int p = 0; p < splits; ++p) v += a.part[p * words + i];
+  if (i < words0) { if (a.dw[0] != nullptr) a.dw[0][i] = v; }
+  else if (i < words0 + words1) { if (a.dw[1] != nullptr) a.dw[1][i - words0] = v; }
+  else if (a.db != nullptr) a.db[i - words0 - words1] = v;
+}
+
+int sage_check(const char* what, int64_t m, int64_t n, int64_t k0, int64_t k1) {
+  F2CGT_REQUIRE(m > 0 && n > 0 && k0 > 0 && k1 > 0, F2CGT_E_INVALID, "%s: sizes must be positive", what);
+  F2CGT_REQUIRE(m < (1ll << 31) && n < (1 << 20) && k0 < (1 << 20) && k1 < (1 << 20), F2CGT_E_UNSUPPORTED,
+                "%s: too many rows or columns", what);
+  return 0;
+}
+
+int64_t sage_splits(int64_t m, int64_t n, int64_t k0, int64_t k1) {
+  const int64_t tiles = ceil_div(n, kTile) * (ceil_div(k0, kTile) + ceil_div(k1, kTile));
+  const int64_t most = ceil_div(m, 1024), want = ceil_div(2 * (int64_t)num_cus(), tiles);
+  return most < want ? most : want;
+}
+
+}  // namespace
+}  // namespace f2cgt
+
+using namespace f2cgt;
+
+extern "C" int f2cgt_sage_linear(const float* x0, const float* w0, const float* x1, const float* w1, const float* bias, float* out,
+                                 int64_t m, int64_t n, int64_t k0, int64_t k1, int relu, void* stream) {
+  const char* what = "sage_linear";
+  if (int rc = sage_check(what, m, n, k0, k1)) return rc;
+  F2CGT_REQUIRE(x0 && w0 && x1 && w1 && out, F2CGT_E_INVALID, "%s: null buffer", what);
+  F2CGT_REQUIRE(k0 % 4 == 0 && k1 % 4 == 0 && aligned(x0, 16) && aligned(w0, 16) && aligned(x1, 16) && aligned(w1, 16) &&
+                    aligned(out, 16), F2CGT_E_UNSUPPORTED, "%s: rows of whole 16-byte pieces only", what);
+  SageArgs a{};
+  a.x[0] = x0; a.x[1] = x1; a.w[0] = w0; a.w[1] = w1; a.bias = bias; a.out = out;
+  a.m = m; a.n = (int)n; a.k[0] = (int)k0; a.k[1] = (int)k1; a.relu = relu;
+  const dim3 grid((unsigned)ceil_div(m, kTile), (unsigned)ceil_div(n, kTile));
+  sage_linear_kernel<<<grid, kForwardWaves * kWave, 0, as_stream(stream)>>>(a);
+  return launch_status(what);
+}
+
+// A tile of 32 outputs reads its rows and weights once per tile of the other side, which a library's larger tiles do half
+// as often: past 131 072 weights that is what the time goes into, in large launches.  Device time of a step forward and
+// backward, operators -> this, us (128 + 128 -> 256 means two inputs of 128 columns and 256 outputs):
+//   128 + 128 -> 256: 1024 rows 51 -> 25, 8192 158 -> 59, 60 000 497 -> 314, 120 000 1059 -> 610
+//   256 + 256 -> 256: 1024 rows 54 -> 27, 4096 109 -> 58, 32 000 375 -> 334;  100 + 100 -> 128: 500 rows 103 -> 19
+//   600 + 600 -> 16:  3000 rows 66 -> 35, 60 000 334 -> 241;  1000 + 1000 -> 64: 16 000 rows 311 -> 180
+//   384 + 384 -> 256: 2000 rows 77 -> 53, 8000 168 -> 160, 32 000 456 -> 572
+//   512 + 512 -> 512: 2000 rows 92 -> 97, 8000 226 -> 335;  768 + 768 -> 512: 1000 rows 75 -> 77
+// Up to 2^29 multiply-adds the host's 125 us less a step count for more than what the device loses there.
+extern "C" int f2cgt_sage_linear_ahead(int64_t m, int64_t n, int64_t k0, int64_t k1) {
+  if (m <= 0 || n <= 0 || k0 <= 0 || k1 <= 0 || m >= (1ll << 31) || n >= (1 << 20) || k0 >= (1 << 20) || k1 >= (1 << 20)) return 0;
+  const int64_t weights = n * (k0 + k1);
+  return weights <= 131072 || weights <= (1ll << 29) / m ? 1 : 0;
+}
+
+extern "C" int64_t f2cgt_sage_linear_grad_workspace_bytes(int64_t m, int64_t n, int64_t k0, int64_t k1) {
+  if (m <= 0 || n <= 0 || k0 <= 0 || k1 <= 0) return 0;
+  const int64_t splits = sage_splits(m, n, k0, k1);
+  return splits > 1 ? splits * (n * (k0 + k1) + n) * 4 : 0;
+}
+
+extern "C" int f2cgt_sage_linear_grad(const float* grad, const float* out, const float* x0, const float* x1, float* dw0, float* dw1,
+                                      float* db, void* workspace, int64_t workspace_bytes, int64_t m, int64_t n, int64_t k0,
+                                      int64_t k1, void* stream) {
+  const char* what = "sage_linear_grad";
+  if (int rc = sage_check(what, m, n, k0, k1)) return rc;
+  F2CGT_REQUIRE(grad && x0 && x1, F2CGT_E_INVALID, "%s: null buffer", what);
+  const int64_t splits = sage_splits(m, n, k0, k1);
+  F2CGT_REQUIRE(splits == 1 || (workspace && workspace_bytes >= f2cgt_sage_linear_grad_workspace_bytes(m, n, k0, k1)),
+                F2CGT_E_INVALID, "%s: workspace too small", what);
+  SageGradArgs a{};
+  a.grad = grad; a.out = out; a.x[0] = x0; a.x[1] = x1; a.dw[0] = dw0; a.dw[1] = dw1; a.db = db;
+  a.part = splits > 1 ? static_cast<float*>(workspace) : nullptr;
+  a.m = m; a.n = (int)n; a.k[0] = (int)k0; a.k[1] = (int)k1;
+  a.rows_per_split = ceil_div(m, splits);
+  const dim3 grid((unsigned)ceil_div(n, kTile), (unsigned)(ceil_div(k0, kTile) + ceil_div(k1, kTile)),
+                  (unsigned)ceil_div(m, a.rows_per_split));
+  F2CGT_REQUIRE(grid.y <= 65535 && grid.z <= 65535, F2CGT_E_UNSUPPORTED, "%s: too many tiles", what);
+  hipStream_t st = as_stream(stream);
+  sage_grad_kernel<<<grid, kGradWaves * kWave, 0, st>>>(a);
+  if (a.part != nullptr)
+    sage_grad_add_kernel<<<(unsigned)ceil_div(n * (k0 + k1) + n, (int64_t)256), 256, 0, st>>>(a, (int)grid.z);
+  return launch_status(what);
+}

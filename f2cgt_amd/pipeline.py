@@ -20,6 +20,7 @@ import math
 import numpy as np
 import torch
 from torch import nn
+from torch.nn.modules import module as _modules
 
 import f2cgt_amd
 
@@ -654,10 +655,26 @@ class CompressionManager:
         return part_feature
 
 
+_MODULE_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+
+
+def _plain_linear(layer):
+    """Whether calling `layer` is nn.Linear's own product and nothing else: no subclass or replaced forward, no
+    parametrization (which is a subclass), no hook on it or on all modules."""
+    return (type(layer) is nn.Linear and "forward" not in layer.__dict__ and
+            not any(getattr(layer, name) for name in _MODULE_HOOKS) and
+            not any(getattr(_modules, "_global" + name) for name in _MODULE_HOOKS))
+
+
 class MySAGEConv(nn.Module):
     """examples/conv.py:9-76.  `forward(csc, feat)`: `csc = (indptr, indices)` of the block
     (destination rows x source rows), `feat = (h_self, h_neigh)`; with a fusing manager `h_neigh`
-    is the compressed code rows of the source nodes and the aggregation decodes them on the fly."""
+    is the compressed code rows of the source nodes and the aggregation decodes them on the fly.
+
+    The two products, their sum, the bias and a ReLU are one launch forward and one or two backward (`sage_linear`) where
+    the two layers are plain `nn.Linear`s on dense fp32 device tensors, the inputs are not differentiated and the size is
+    one it is ahead at; the layers' own operators otherwise, also under transforms, modes, autocast and tracing.  A step
+    at 1024 x (128 + 128) -> 256 takes the host 62 us where the operators take 187, the device 25 where they take 51."""
 
     def __init__(self, in_feats, out_feats, aggregator_type, compression_manager, bias=True, norm=None,
                  activation=None):
@@ -694,8 +711,13 @@ class MySAGEConv(nn.Module):
             else:
                 h_neigh = capi.sq_decompress_spmm_csr(h_neigh, sm.codebooks[level], indptr, indices,
                                                       sm.configs[level][1], sm.configs[level][0], sm.feat_dim)
-        rst = self.fc_self(h_self) + self.fc_neigh(h_neigh)
-        if self.activation is not None:
+        relu = self.activation is torch.relu or self.activation is nn.functional.relu
+        rst = None
+        if _plain_linear(self.fc_self) and _plain_linear(self.fc_neigh) and self.fc_neigh.bias is None:
+            rst = capi.sage_linear(h_self, h_neigh, self.fc_self.weight, self.fc_neigh.weight, self.fc_self.bias, relu)
+        if rst is None:
+            rst, relu = self.fc_self(h_self) + self.fc_neigh(h_neigh), False
+        if self.activation is not None and not relu:
             rst = self.activation(rst)
         if self.norm is not None:
             rst = self.norm(rst)

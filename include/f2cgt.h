@@ -350,6 +350,24 @@ int f2cgt_kmeans_slices_step(const float* x, const uint32_t* keep, float* center
                              void* workspace, int64_t workspace_bytes, int64_t m, int64_t slices, int64_t n, int64_t k,
                              int metric, void* stream);
 
+/* The dense part of a GraphSAGE layer (examples/conv.py:68-76) at the sizes of a minibatch, fp32 throughout.
+ *
+ * f2cgt_sage_linear: out[m, n] = x0 w0^T + x1 w1^T + bias, through max(., 0) where relu is nonzero (a NaN stays one).
+ * x0 [m, k0], w0 [n, k0], x1 [m, k1], w1 [n, k1], bias [n] or NULL, all dense; k0 and k1 multiples of four and the buffers
+ * 16-byte aligned (others: F2CGT_E_UNSUPPORTED).
+ *
+ * f2cgt_sage_linear_grad: dw0 = g^T x0, dw1 = g^T x1, db = column sums of g, each left out where NULL, with g = grad, or
+ * (out given: the values f2cgt_sage_linear wrote with relu) grad where out is not <= 0 and 0 elsewhere.  The sums are made
+ * in a fixed order.  workspace: f2cgt_sage_linear_grad_workspace_bytes (0 up to 1024 rows), contents irrelevant. */
+int f2cgt_sage_linear(const float* x0, const float* w0, const float* x1, const float* w1, const float* bias, float* out,
+                      int64_t m, int64_t n, int64_t k0, int64_t k1, int relu, void* stream);
+int64_t f2cgt_sage_linear_grad_workspace_bytes(int64_t m, int64_t n, int64_t k0, int64_t k1);
+int f2cgt_sage_linear_grad(const float* grad, const float* out, const float* x0, const float* x1, float* dw0, float* dw1,
+                           float* db, void* workspace, int64_t workspace_bytes, int64_t m, int64_t n, int64_t k0, int64_t k1,
+                           void* stream);
+/* 1 where the two launches are no slower than a library's products, sum and activation one by one, 0 where they are. */
+int f2cgt_sage_linear_ahead(int64_t m, int64_t n, int64_t k0, int64_t k1);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,126 @@
+"""The dense part of the GraphSAGE layer as one kernel each way, against float64; and which calls keep the module's own
+operators."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+if torch.cuda.is_available():
+    import f2cgt_amd
+    from f2cgt_amd import pipeline
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(m, k0, k1, n, seed=0):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed + m + 7 * n)
+    x0, x1 = torch.randn((m, k0), generator=g, device="cuda"), torch.randn((m, k1), generator=g, device="cuda")
+    w0 = (torch.randn((n, k0), generator=g, device="cuda") / k0 ** 0.5).requires_grad_()
+    w1 = (torch.randn((n, k1), generator=g, device="cuda") / k1 ** 0.5).requires_grad_()
+    b = torch.randn((n,), generator=g, device="cuda").requires_grad_()
+    return x0, x1, w0, w1, b, torch.randn((m, n), generator=g, device="cuda")
+
+
+@pytest.mark.parametrize("m,k0,k1,n", [(1, 4, 4, 1), (31, 32, 36, 33), (32, 4, 100, 32), (33, 64, 28, 70), (1024, 128, 128, 256),
+                                       (1025, 100, 100, 5), (2500, 12, 200, 31), (5000, 260, 36, 64)])
+@pytest.mark.parametrize("relu", [True, False])
+def test_output_and_gradients_against_float64(m, k0, k1, n, relu):
+    lib = f2cgt_amd.load()
+    x0, x1, w0, w1, b, g = _inputs(m, k0, k1, n)
+    out = lib.sage_linear(x0, x1, w0, w1, b, relu)
+    out.backward(g)
+    X0, X1, W0, W1, B, G = (t.detach().double() for t in (x0, x1, w0, w1, b, g))
+    z = X0 @ W0.t() + X1 @ W1.t() + B
+    unit = 2.0 ** -24
+    # a sum of k products, each rounded, partial sums within the sum of the magnitudes; any order
+    size = X0.abs() @ W0.abs().t() + X1.abs() @ W1.abs().t() + B.abs()
+    assert bool(((out.double() - (z.clamp(min=0) if relu else z)).abs() <= (k0 + k1 + 4) * unit * size).all())
+    if relu:
+        G = torch.where(out.detach() <= 0, 0.0, G)
+    for got, want, size in ((w0.grad, G.t() @ X0, G.abs().t() @ X0.abs()), (w1.grad, G.t() @ X1, G.abs().t() @ X1.abs()),
+                            (b.grad, G.sum(0), G.abs().sum(0))):
+        assert bool(((got.double() - want).abs() <= (m + 4) * unit * size).all())
+
+
+def test_special_values_and_absent_parts():
+    lib = f2cgt_amd.load()
+    x0, x1, w0, w1, b, g = _inputs(40, 8, 12, 6)
+    x0[3, 2], x0[5, 0] = float("nan"), float("inf")
+    out = lib.sage_linear(x0, x1, w0, w1, b, True)
+    want = torch.relu(torch.nn.functional.linear(x0, w0, b) + torch.nn.functional.linear(x1, w1))
+    assert torch.equal(out.isnan(), want.isnan()) and bool(out[3].isnan().all())
+    assert torch.equal(out.isinf(), want.isinf())
+    w1.requires_grad_(False)
+    out = lib.sage_linear(x0[10:], x1[10:], w0, w1, None, False)     # no bias; a weight without a gradient
+    out.backward(g[10:])
+    assert w0.grad is not None and w1.grad is None and b.grad is None
+    torch.testing.assert_close(w0.grad, g[10:].t() @ x0[10:], rtol=1e-5, atol=1e-4)
+    with torch.no_grad():
+        assert not lib.sage_linear(x0, x1, w0, w1, b, True).requires_grad
+
+
+def test_gradient_of_the_gradient():
+    lib = f2cgt_amd.load()
+    x0, x1, w0, w1, b, g = _inputs(50, 8, 8, 7)
+    g.requires_grad_()
+    got = torch.autograd.grad(lib.sage_linear(x0, x1, w0, w1, b, True), (w0, b), g, create_graph=True)
+    want = torch.autograd.grad(torch.relu(torch.nn.functional.linear(x0, w0, b) + torch.nn.functional.linear(x1, w1)), (w0, b), g,
+                               create_graph=True)
+    for a, c in zip(got, want):
+        torch.testing.assert_close(a, c, rtol=1e-5, atol=1e-4)
+    (gg,) = torch.autograd.grad(got[0].square().sum(), g)
+    (ww,) = torch.autograd.grad(want[0].square().sum(), g)
+    torch.testing.assert_close(gg, ww, rtol=1e-4, atol=1e-2)
+
+
+def test_calls_left_to_the_modules_operators():
+    """Each is what the layer did without the kernel: the layer's result is that of its two Linears."""
+    lib = f2cgt_amd.load()
+    x0, x1, w0, w1, b, _ = _inputs(64, 16, 16, 8)
+    take = lambda *a: lib.sage_linear(*a) is not None
+    assert take(x0, x1, w0, w1, b, True)
+    assert not take(x0.double(), x1.double(), w0.double(), w1.double(), b.double(), True)
+    assert not take(x0.cpu(), x1.cpu(), w0.cpu(), w1.cpu(), b.cpu(), True)
+    assert not take(x0.clone().requires_grad_(), x1, w0, w1, b, True)         # the input is differentiated
+    assert not take(x0.t().contiguous().t(), x1, w0, w1, b, True)             # not dense rows
+    assert not take(x0[:0], x1[:0], w0, w1, b, True)
+    assert not take(x0[:, :15].contiguous(), x1, w0[:, :15].contiguous(), w1, b, True)
+    assert not take(x0.reshape(-1)[1:1 + 63 * 16].view(63, 16), x1[:63], w0, w1, b, True)   # 4 bytes off
+    assert not take(x0, x1[:63], w0, w1, b, True) and not take(x0, x1, w0[:7], w1, b, True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not take(x0, x1, w0, w1, b, True)
+    with torch.autograd.forward_ad.dual_level():
+        assert not take(x0, x1, w0, w1, b, True)
+    seen = []
+    torch.func.grad(lambda w: (seen.append(take(x0, x1, w, w1, b, True)), w.sum())[1])(w0.detach())
+    torch.func.vmap(lambda w: (seen.append(take(x0, x1, w, w1, b, True)), w)[1])(w0.detach()[None])
+    assert seen == [False, False]
+    from torch.utils.flop_counter import FlopCounterMode
+    with FlopCounterMode(display=False):
+        assert not take(x0, x1, w0, w1, b, True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: seen.append(t.shape) or t.cpu(), lambda t: t.cuda()):
+        out = lib.sage_linear(x0, x1, w0, w1, b, True)
+    out.sum().backward()                                                      # the saved tensors went through the hooks
+    assert len(seen) == 5 and torch.allclose(b.grad, (out > 0).sum(0).float())
+
+
+def test_layer_equals_its_linears_with_hooks_and_without():
+    torch.manual_seed(0)
+    conv = pipeline.MySAGEConv(16, 8, "mean", None, activation=torch.relu).cuda()
+    h = torch.randn((300, 16), device="cuda")
+    indptr = torch.arange(0, 301, 3, device="cuda")
+    indices = torch.randint(0, 300, (300,), device="cuda")
+    plain = conv((indptr, indices), (h[:100], h))
+    assert type(plain.grad_fn).__name__.startswith("CppNode") or "Sage" in plain.grad_fn.name()
+    calls = []
+    handle = conv.fc_neigh.register_forward_hook(lambda *a: calls.append(1))
+    hooked = conv((indptr, indices), (h[:100], h))
+    handle.remove()
+    assert calls == [1]
+    torch.testing.assert_close(plain, hooked, rtol=1e-5, atol=1e-5)
+    scaled = torch.nn.utils.parametrizations.weight_norm(conv.fc_self)
+    assert scaled is conv.fc_self
+    torch.testing.assert_close(conv((indptr, indices), (h[:100], h)), plain, rtol=1e-5, atol=1e-5)
+    conv.activation = torch.tanh
+    out = conv((indptr, indices), (h[:100], h))
+    assert float(out.detach().min()) < 0
