@@ -587,21 +587,27 @@ class CompressionManager:
                                        self.configs[level][0], self.feat_dim)
 
     def get_seeds_data(self, seeds_key):
-        """Decoded first-level rows of `seeds_key`, produced on `seeds_task_stream`; the result may be
-        used on another stream only after `seeds_task_event` (reorganize_seeds_data waits for it)."""
+        """Decoded first-level rows of `seeds_key`; the result may be used on another stream only after
+        `seeds_task_event` (reorganize_seeds_data waits for it).  Produced on `seeds_task_stream`, or, where the one kernel
+        that looks the rows up, checks, fetches and decodes them is followed by a wait for its check, on the current stream:
+        the call returns with the rows made either way, and handing the work to another stream and back took longer than
+        the kernel (57 -> 25 us of the host's time a minibatch)."""
         if not self.is_two_level:
             return None
+        seeds = self.seeds_data
+        in_one = (self.methods[0] == "sq" and seeds.data.is_cuda and not seeds.has_cache and
+                  seeds_key.dtype in (torch.int32, torch.int64))
+        if in_one and self.check_seed_keys:
+            seeds_feature = self._decode_seeds(seeds_key)
+            self.seeds_task_event.record()
+            return seeds_feature
         side = self.seeds_task_stream
         side.wait_stream(torch.cuda.current_stream())      # seeds_key may still be in the making
         with torch.cuda.stream(side):
             # the caller may drop seeds_key as soon as this returns: tie its memory to the side stream
             seeds_key.record_stream(side)
-            seeds = self.seeds_data
-            if self.methods[0] == "sq" and seeds.data.is_cuda and not seeds.has_cache and seeds_key.dtype in (torch.int32, torch.int64):
-                # lookup, check, fetch and decode in one kernel
-                seeds_feature = _capi().sq_decompress_rows(seeds.data, seeds_key, self.codebooks[0], self.configs[0][1],
-                                                           self.configs[0][0], self.feat_dim, self.seed_slot,
-                                                           self.check_seed_keys)
+            if in_one:
+                seeds_feature = self._decode_seeds(seeds_key)
                 self.seeds_task_event.record(side)
                 return seeds_feature
             slots = self.seed_slot[seeds_key.long()].long()
@@ -610,6 +616,10 @@ class CompressionManager:
             seeds_feature = self._decompress(0, self.seeds_data[slots])
             self.seeds_task_event.record(side)
         return seeds_feature
+
+    def _decode_seeds(self, seeds_key):
+        return _capi().sq_decompress_rows(self.seeds_data.data, seeds_key, self.codebooks[0], self.configs[0][1],
+                                          self.configs[0][0], self.feat_dim, self.seed_slot, self.check_seed_keys)
 
     def get_all_data(self, keys):
         if self.is_fusion:
