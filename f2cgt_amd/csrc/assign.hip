@@ -38,7 +38,6 @@ namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4_dword __attribute__((ext_vector_type(4), aligned(4)));   // loaded from any float's address
-typedef float floatx2_dword __attribute__((ext_vector_type(2), aligned(4)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 
@@ -264,7 +263,9 @@ __device__ __forceinline__ int exact_row(const AssignArgs& a, const float* __res
 
 // S: steps of 16 dimensions.  T: tiles of a chunk (a class has T centres).  PACKED: update_packed.  SUMS: the training
 // step, which adds the rows up by label in LDS (n * (16 S + 1) doubles) and leaves a set of sums per workgroup.
-template <int S, int T, bool PACKED, bool SUMS>
+// METRIC: the launch's, where it is fixed when the kernel is chosen, or kEither.
+constexpr int kEither = -1;
+template <int S, int T, bool PACKED, bool SUMS, int METRIC>
 __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kernel(AssignArgs a) {
   constexpr int kThreads = assign_threads(S), kWaves = kThreads / kWave;
   constexpr int U = T == 1 ? 1 : 2;                              // tiles a step
@@ -311,7 +312,7 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
   // (measured, addresses as here; 32-bit integers 6): a step of six slices of 150 000 x 16 rows took 110 us, now 56.
   double* sums = reinterpret_cast<double*>(psum + 2 * kThreads + kWaves * 32 * S);
   uint32_t* counts = reinterpret_cast<uint32_t*>(sums + n * kPitch);
-  const bool cosine = a.metric == F2CGT_METRIC_COSINE;
+  const bool cosine = METRIC == kEither ? a.metric == F2CGT_METRIC_COSINE : METRIC == F2CGT_METRIC_COSINE;
   const int lane = threadIdx.x & 63;
   const int j = lane & 31;
   const int g = lane >> 5;
@@ -361,44 +362,36 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
       hi4[at] = w;
     }
   }
-  const bool wide = kx >= 8;                // a row holds the eight values that an idle lane reads from it
-  const int rest = kx & 7;                  // values in the chunk that a row ends in
   const bool ragged = kx < kWidth;          // there are operand places without a dimension
   float q[S][8] = {};                       // this lane's share of a row: dimensions 16 st + 8 g + e
-  // Loads of a group's rows, issued always (lanes past the last row or dimension read others): whole chunks of 8 as
-  // 16-byte loads, which rows of any width and start take (4-byte alignment), and the chunk that a row ends in by fours,
-  // twos and ones.
+  // Loads of a group's rows, issued always: two 16-byte loads per step, which take any float's address, from one address
+  // for the group and an offset for the lane.  A row of fewer than 16 S values is read past its end, into the rows after
+  // it (the places without a dimension are cleared before they are used): the groups whose last row has enough of them
+  // behind it.  The others' values are read one by one, of dimensions that the row has.  Lanes past the last row read
+  // the group's first.
+  const int64_t behind = ragged ? (kWidth + ldx - 1) / ldx : 0;
+  const int64_t whole_groups = ldx >= (1 << 24) ? 0 : !ragged ? n_groups : m > behind ? (m - behind) / 32 : 0;
+  const uint32_t row_at = 4u * ((uint32_t)j * (uint32_t)ldx + 8u * (uint32_t)g);   // bytes (below 4 GB: ldx < 2^24)
   auto load_rows = [&](int64_t grp) {
     const int64_t left = m - grp * 32;
-    const float* __restrict__ xr = x + (grp * 32 + (j < left ? j : 0)) * ldx;
+    if (grp < whole_groups) {
+      const char* group = reinterpret_cast<const char*>(x + grp * 32 * ldx);
+      const uint32_t at = j < left ? row_at : 32u * (uint32_t)g;
 #pragma unroll
-    for (int st = 0; st < S; ++st) {
-      const int kk0 = 16 * st + 8 * g;
-      if (wide) {
-        const floatx4_dword* x4 = reinterpret_cast<const floatx4_dword*>(xr + (kk0 + 8 <= kx ? kk0 : 0));
-        const floatx4_dword u = x4[0], w = x4[1];
+      for (int st = 0; st < S; ++st) {
+        const floatx4_dword u = *reinterpret_cast<const floatx4_dword*>(group + (at + 64 * st));
+        const floatx4_dword w = *reinterpret_cast<const floatx4_dword*>(group + (at + 64 * st + 16));
 #pragma unroll
         for (int e = 0; e < 4; ++e) { q[st][e] = u[e]; q[st][4 + e] = w[e]; }
       }
-      if (rest != 0 && kk0 < kx && kk0 + 8 > kx) {
-        const float* xt = xr + kk0;
-        if (rest & 4) {
-          const floatx4_dword u = *reinterpret_cast<const floatx4_dword*>(xt);
+    } else {
+      int from = 8 * g;                     // (opaque: the places below are not worth registers over the loop)
+      asm volatile("" : "+v"(from));
+      const float* __restrict__ xr = x + (grp * 32 + (j < left ? j : 0)) * ldx;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) q[st][e] = u[e];
-        }
-        if (rest & 2) {
-          const floatx2_dword u = *reinterpret_cast<const floatx2_dword*>(xt + (rest & 4));
-          const bool behind = (rest & 4) != 0;
-          q[st][0] = behind ? q[st][0] : u[0]; q[st][1] = behind ? q[st][1] : u[1];
-          q[st][4] = behind ? u[0] : q[st][4]; q[st][5] = behind ? u[1] : q[st][5];
-        }
-        if (rest & 1) {
-          const float u = xt[rest - 1];
+      for (int st = 0; st < S; ++st)
 #pragma unroll
-          for (int e = 0; e < 8; e += 2) q[st][e] = rest == e + 1 ? u : q[st][e];
-        }
-      }
+        for (int e = 0; e < 8; ++e) q[st][e] = xr[from + 16 * st + e < kx ? from + 16 * st + e : 0];
     }
   };
   int64_t grp = wg_lo + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -556,11 +549,11 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
   // >= |c|^2: each of the S leading instructions cuts its 17 addends at 2^-22 of the largest
   // (<= P): 68 S; the small pairs (2^-11 P and below) together stay below 1; the pieces of x and c
   // stop at 2^-22 of the value (4 P each way in these units, on half of P) and the dropped pair is
-  // as large: 6; below the smallest normal half 1; the bias sum k + 1; its addition 2; the rounding
+  // twice as large: 8; below the smallest normal half 1; the bias sum k + 1; its addition 2; the rounding
   // of x - mu and c - mu 4 (L2: 2^-22 (|x|^2 + |c|^2)); 2 spare.  A class is decided by fp32 sums of
   // the same pieces (3 * 8 S roundings of partial sums <= P / 2: 24 S), which stays below.  Doubled
   // for the two scores of a gap.
-  const float unit = 5.9604645e-8f * (float)(2 * (68 * S + k + 17));
+  const float unit = 5.9604645e-8f * (float)(2 * (68 * S + k + 19));
   // Packed minima have to be finite.  An L2 score |c|^2 - 2 x . c is at most 2 (|x|^2 + |c|^2), which may exceed the
   // largest float (3.4e38) while the bound above is finite; cosine has |x . c^| <= |x|, below 2e19 wherever |x|^2 is finite.
   const float finite_below = cosine ? INFINITY : 1.6e38f;
@@ -587,10 +580,12 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
         for (int e = 0; e < 8; ++e) own[st][e] = q[st][e];
     }
     if (ragged) {
+      int has = kx - 8 * g;                 // compared here: as lane masks kept over the loop these were spilled scalars
+      asm volatile("" : "+v"(has));
 #pragma unroll
       for (int st = 0; st < S; ++st)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) q[st][e] = 16 * st + 8 * g + e < kx ? q[st][e] : 0.f;
+        for (int e = 0; e < 8; ++e) q[st][e] = 16 * st + e < has ? q[st][e] : 0.f;
     }
     if (use_mu) {                           // (zero from dimension k on)
 #pragma unroll
@@ -611,13 +606,18 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     const float x_scale = -pow2(x_shift);
     // what takes a scaled product to -x . c (cosine) or -2 x . c
     const float back = ldexpf(cosine ? 1.f : 2.f, -(x_shift + c_shift));
+    // The leading pieces are cut off, two with one conversion, not rounded: the second ones, which are, then end at 2^-22
+    // of the value (2^-23 behind rounded ones), and the dropped product is twice as large.
 #pragma unroll
     for (int st = 0; st < S; ++st)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        _Float16 a0, a1;
-        split2(q[st][e] * x_scale, a0, a1);
-        xp[st][0][e] = a0; xp[st][1][e] = a1;
+      for (int e = 0; e < 8; e += 2) {
+        const auto lead = __builtin_amdgcn_cvt_pkrtz(q[st][e] * x_scale, q[st][e + 1] * x_scale);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          xp[st][0][e + i] = (_Float16)lead[i];
+          xp[st][1][e + i] = (_Float16)__fmaf_rn(q[st][e + i], x_scale, -(float)lead[i]);   // (exact before the rounding)
+        }
       }
     // The next rows travel while these are scored, behind the last ones' labels: the wait for the rows is one for every
     // access before them too, and a store that has just been issued takes as long as the rows.
@@ -704,12 +704,10 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     const float slack = PACKED ? 1.92e-6f * fabsf(runner) : 0.f;
     // The class's centres one by one (a class of the last chunk may reach into the padding): each half of the wave takes
     // the dimensions that it has of the row.
-    float bs = INFINITY;
-    int bt = 0;
+    float dots[T];
     const half8* cand = ap + (cls >> 5) * S * 64 + g * 32 + (cls & 31);
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      if (t >= n_ct) break;
       float dot = 0.f;
 #pragma unroll
       for (int st = 0; st < S; ++st) {
@@ -724,15 +722,34 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
           dot = __builtin_amdgcn_fdot2(xh, ch, dot, false);
         }
       }
-      const float sc = __fmaf_rn(add_halves(dot), back, bias[cls + 32 * t]);
-      runner = min2(runner, max2(bs, sc));
-      bt = sc < bs ? t : bt;
-      bs = min2(bs, sc);
+      dots[t] = dot;
+    }
+    // The halves of a dot product meet: with one swap for two of them the lower half of the wave gets the even centre's
+    // sum and the upper half the odd one's, each takes the best of its own, and then of both.
+    float bs, other = INFINITY;
+    int bt = 0;
+    if constexpr (T == 1) {
+      bs = __fmaf_rn(add_halves(dots[0]), back, bias[cls]);
+    } else {
+      bs = INFINITY;
+#pragma unroll
+      for (int t = 0; t < T; t += 2) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(dots[t]), __float_as_uint(dots[t + 1]), false, false);
+        const float sc = __fmaf_rn(__uint_as_float(r[0]) + __uint_as_float(r[1]), back, bias[cls + 32 * (t + g)]);
+        other = t == 0 ? other : min2(other, max2(bs, sc));
+        bt = sc < bs ? t + g : bt;
+        bs = t == 0 ? sc : min2(bs, sc);
+      }
+      const Halves b2 = halves(__float_as_uint(bs)), o2 = halves(__float_as_uint(other)), t2 = halves((uint32_t)bt);
+      const float b0 = __uint_as_float(b2.lo), b1 = __uint_as_float(b2.hi);
+      bs = min2(b0, b1);
+      bt = (int)(b1 < b0 ? t2.hi : t2.lo);
+      runner = min3(runner, max2(b0, b1), min2(__uint_as_float(o2.lo), __uint_as_float(o2.hi)));
     }
     int besti = cls + 32 * bt;
     // cosine: the evaluation's share shrinks with the operands, the rounding of c / |c| (norm in
     // fp64, one rounding for 1 / |c|, one for the product, one for - m: 3 units, doubled) does not
-    const float scale = cosine ? sqrtf(xn) * (cdev + 3.5762787e-7f / unit) : xn + cmax;
+    const float scale = cosine ? __builtin_amdgcn_sqrtf(xn) * (cdev + 3.5762787e-7f / unit) : xn + cmax;
     const float bound = unit * scale + kTinyGap + slack;
     // Padding leads where no real score is a number.  A row whose square is below the smallest normal float has pieces of
     // too few bits and no norm to bound that by (scored 2^100 times as long it would not need float64, at 2 % of the time of
@@ -753,13 +770,14 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
       const int to = (int)halves((uint32_t)besti).lo;            // the exact evaluation's label is in the lower half
       const bool in = grp * 32 + j < m && (kept >> j & 1u);
       if (in) {
+        int has = kx - 8 * g;
+        asm volatile("" : "+v"(has));       // (as above)
+        double* centre = sums + to * kPitch + 8 * g;
 #pragma unroll
         for (int st = 0; st < S; ++st)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int d = 16 * st + 8 * g + e;
-            if (d < kx) unsafeAtomicAdd(sums + to * kPitch + d, (double)own[st][e]);
-          }
+          for (int e = 0; e < 8; ++e)
+            if (!ragged || 16 * st + e < has) unsafeAtomicAdd(centre + 16 * st + e, (double)own[st][e]);
         if (g == 0) atomicAdd(counts + to, 1u);
       }
     }
@@ -805,9 +823,9 @@ int64_t assign_shares(int64_t m, int64_t slices, int64_t resident, int waves) {
 }
 size_t assign_sums_lds(int64_t n, int64_t k) { return assign_lds(n, k) + (size_t)(n * (16 * ceil_div(k, 16) + 1) * 8 + n * 4); }
 
-template <int S, int T, bool PACKED, bool SUMS>
+template <int S, int T, bool PACKED, bool SUMS, int METRIC>
 int launch_assign(AssignArgs a, size_t lds, hipStream_t st) {
-  auto kern = assign_kernel<S, T, PACKED, SUMS>;
+  auto kern = assign_kernel<S, T, PACKED, SUMS, METRIC>;
   constexpr int threads = assign_threads(S);
   if (lds > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -834,15 +852,26 @@ int launch_assign(AssignArgs a, size_t lds, hipStream_t st) {
   return launch_status("kmeans_predict");
 }
 
+// Up to 32 columns and more than 64 centres, what the encoder is run with, have a kernel for each metric: the general one
+// asks for it in every tile of every group of rows.
+template <int S, int T, bool SUMS>
+int assign_metric(const AssignArgs& a, size_t lds, hipStream_t st) {
+  if constexpr (S <= 2 && T == 4)
+    return a.metric == F2CGT_METRIC_COSINE ? launch_assign<S, T, true, SUMS, F2CGT_METRIC_COSINE>(a, lds, st)
+                                           : launch_assign<S, T, true, SUMS, F2CGT_METRIC_L2>(a, lds, st);
+  else
+    return launch_assign<S, T, true, SUMS, kEither>(a, lds, st);
+}
+
 template <int S, int T>
 int assign_pick(const AssignArgs& a, size_t lds, hipStream_t st) {
-  if (a.sums != nullptr) return launch_assign<S, T, true, true>(a, lds, st);
+  if (a.sums != nullptr) return assign_metric<S, T, true>(a, lds, st);
   if constexpr (S == 1) {
     // In fewer than four dimensions so many centres are close to a row that the slots' share of the near-tie bound
     // sends more rows to the exact evaluation than the packed update saves.
-    if (a.k < 4) return launch_assign<1, T, false, false>(a, lds, st);
+    if (a.k < 4) return launch_assign<1, T, false, false, kEither>(a, lds, st);
   }
-  return launch_assign<S, T, true, false>(a, lds, st);
+  return assign_metric<S, T, false>(a, lds, st);
 }
 
 template <int S>
