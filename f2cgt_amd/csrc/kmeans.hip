@@ -271,9 +271,9 @@ __global__ __launch_bounds__(kKmThreads) void km_merge_kernel(KmArgs a, int part
 // The same for the sets of a step of several column slices (blockIdx.y: the slice, with sums, centres, shifts, counter and
 // flag of its own one behind the other).  A workgroup takes as many whole centres as VALUES values hold, over 1024 / VALUES
 // sets side by side: both the chain of loads per thread and the workgroups at the counter count, whose release has the L2
-// write back.  With a workgroup per centre six slices of 256 centres of 16 columns, 42 sets, took 35 us, with 256 values
-// per workgroup 10.8; one slice of 256 sets takes 32 that way and 12.8 with 64 values.  fp64 sums: a set is rounded once,
-// the sum of the sets once more.
+// write back.  With a workgroup per centre six slices of 256 centres of 16 columns, 40 sets, took 35 us, with 256 values
+// per workgroup 10.8, with all reads of a thread in one round 8.2; one slice of 200 sets takes 32 with 256 values, 10.7
+// with 64 and 7.3 in one round.  fp64 sums: a set is rounded once, the sum of the sets once more.
 template <int VALUES>
 __global__ __launch_bounds__(kKmMergeThreads) void km_merge_slices_kernel(KmArgs a, int parts, float* moves, uint32_t* arrived) {
   const int slice = blockIdx.y;
@@ -298,12 +298,27 @@ __global__ __launch_bounds__(kKmMergeThreads) void km_merge_slices_kernel(KmArgs
   double total = 0.0;
   uint32_t cnt = 0;
   if (on) {
+    // Sixteen sets in flight per thread: another CU of another die wrote them, and a second round of reads is 2 us.  A
+    // place beyond the last set reads the first one's and adds nothing; the members are counted by a centre's first lane.
+    constexpr int U = 16;
     const float* from = a.sums + (int64_t)c * a.k + col;
     const uint32_t* count = reinterpret_cast<const uint32_t*>(a.sums) + (int64_t)a.n * a.k + c;
-#pragma unroll 8
-    for (int p = q; p < parts; p += kSide) {
-      total += (double)from[(int64_t)p * words];
-      cnt += count[(int64_t)p * words];
+    for (int p0 = q; p0 < parts; p0 += kSide * U) {
+      float v[U];
+      uint32_t m[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int p = p0 + u * kSide;
+        v[u] = from[(int64_t)(p < parts ? p : q) * words];
+        m[u] = 0u;
+        if (col == 0) m[u] = count[(int64_t)(p < parts ? p : q) * words];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool in = p0 + u * kSide < parts;
+        total += in ? (double)v[u] : 0.0;
+        cnt += in ? m[u] : 0u;
+      }
     }
   }
   s_part[q][at] = total;
@@ -311,8 +326,11 @@ __global__ __launch_bounds__(kKmMergeThreads) void km_merge_slices_kernel(KmArgs
   __syncthreads();
   if (q == 0) {
     float d2 = -0.f;
+    cnt = 0u;
 #pragma unroll
-    for (int w = 1; w < kSide; ++w) { total += s_part[w][at]; cnt += s_cnt[w][at]; }
+    for (int w = 1; w < kSide; ++w) total += s_part[w][at];
+#pragma unroll
+    for (int w = 0; w < kSide; ++w) cnt += s_cnt[w][at - col];
     if (on && cnt > 0u) {
       float* centre = a.centers + (int64_t)c * a.k + col;
       const float now = (float)total / (float)cnt;
@@ -627,9 +645,10 @@ extern "C" int f2cgt_kmeans_slices_step(const float* x, const uint32_t* keep, fl
   KmArgs a{};
   a.centers = centers; a.shift = shift; a.stop = stop; a.sums = sums; a.m = m; a.n = (int)n; a.k = (int)k;
   a.rule = stop_rule; a.tol = tol;
-  const int values = parts <= 64 ? 256 : 64;
+  const int values = parts <= 64 ? 256 : parts <= 128 ? 128 : 64;
   const dim3 grid((unsigned)ceil_div(n, values / k), (unsigned)slices);
   if (parts <= 64) km_merge_slices_kernel<256><<<grid, kKmMergeThreads, 0, st>>>(a, parts, moves, arrived);
+  else if (parts <= 128) km_merge_slices_kernel<128><<<grid, kKmMergeThreads, 0, st>>>(a, parts, moves, arrived);
   else km_merge_slices_kernel<64><<<grid, kKmMergeThreads, 0, st>>>(a, parts, moves, arrived);
   return launch_status(what);
 }
