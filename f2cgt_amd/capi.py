@@ -54,6 +54,7 @@ SIGNATURES = {
     "f2cgt_kmeans_slices_step": ([P, P, P, P, I, ctypes.c_float, P, L, L, L, L, L, I, P], c_int),
     "f2cgt_kmeans_update_workspace_bytes": ([L, L], c_int64),
     "f2cgt_kmeans_update": ([P, P, P, P, P, P, I, ctypes.c_float, P, L, L, L, L, P], c_int),
+    "f2cgt_kmeans_rescale": ([P, P, L, L, L, P, P, P], c_int),
     "f2cgt_sage_linear": ([P, P, P, P, P, P, L, L, L, L, I, P], c_int),
     "f2cgt_sage_linear_ahead": ([L, L, L, L], c_int),
     "f2cgt_sage_linear_grad_workspace_bytes": ([L, L, L, L], c_int64),

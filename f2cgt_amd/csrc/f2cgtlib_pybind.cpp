@@ -448,8 +448,9 @@ bool kmeans_slices_covers(int64_t slices, int64_t n, int64_t k) { return f2cgt_k
 // Lloyd iterations of all slices on x [slices, m, k] from `centers` [slices, n, k] (updated in place), until every slice
 // has met `rule` or for max_iter steps; tol grows by `growth` each step.  The flags are read every check_every steps and
 // at the end.  -> int32 [slices] on the host: 0 not met, 1 met, 2 the shift became NaN, 3 no rows.
-torch::Tensor kmeans_slices_fit(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, std::string metric,
-                                int64_t rule, double tol, double growth, int64_t max_iter, int64_t check_every) {
+// The loop of kmeans_slices_fit on flags[0, slices), which it leaves on the device; true where a read-back found them all set.
+bool fit_slices(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, const std::string& metric, int64_t rule,
+                double tol, double growth, int64_t max_iter, int64_t check_every, torch::Tensor& flags) {
   x = dev_contig(x, "x");
   TORCH_CHECK(x.dim() == 3 && x.scalar_type() == torch::kFloat32, "x must be float32 [slices, m, k]");
   TORCH_CHECK(centers.is_cuda() && centers.is_contiguous() && centers.scalar_type() == torch::kFloat32 && centers.dim() == 3 &&
@@ -466,24 +467,55 @@ torch::Tensor kmeans_slices_fit(torch::Tensor x, c10::optional<torch::Tensor> ke
   TORCH_CHECK(check_every > 0, "check_every must be positive");
   const int tag = metric_tag(metric);
   c10::DeviceGuard guard(x.device());
-  auto stop = torch::zeros({slices}, torch::TensorOptions().dtype(torch::kInt32).device(x.device()));
+  flags = torch::zeros({slices + 2}, torch::TensorOptions().dtype(torch::kInt32).device(x.device()));
   auto ws = torch::empty({f2cgt_kmeans_slices_workspace_bytes(m, slices, n, k)},
                          torch::TensorOptions().dtype(torch::kUInt8).device(x.device()));
   py::gil_scoped_release unlocked;
   for (int64_t it = 0; it < max_iter; ++it) {
-    check_rc(f2cgt_kmeans_slices_step(x.data_ptr<float>(), bits, centers.data_ptr<float>(), stop.data_ptr<int32_t>(), (int)rule,
+    check_rc(f2cgt_kmeans_slices_step(x.data_ptr<float>(), bits, centers.data_ptr<float>(), flags.data_ptr<int32_t>(), (int)rule,
                                       (float)tol, ws.data_ptr(), ws.numel(), m, slices, n, k, tag, current_stream()),
              "kmeans_slices_fit");
     tol *= growth;
     if (it % check_every == check_every - 1 && it + 1 < max_iter) {
-      auto seen = stop.cpu();
+      auto seen = flags.cpu();
       const int32_t* f = seen.data_ptr<int32_t>();
       bool all = true;
       for (int64_t s = 0; s < slices; ++s) all = all && f[s] != 0;
-      if (all) return seen;
+      if (all) return true;
     }
   }
-  return stop.cpu();
+  return false;
+}
+
+torch::Tensor kmeans_slices_fit(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, std::string metric,
+                                int64_t rule, double tol, double growth, int64_t max_iter, int64_t check_every) {
+  torch::Tensor flags;
+  fit_slices(x, keep, centers, metric, rule, tol, growth, max_iter, check_every, flags);
+  py::gil_scoped_release unlocked;
+  return flags.narrow(0, 0, centers.size(0)).cpu();
+}
+
+// The same, and the centres rescaled to their slice's mean length.  -> (flags int32 [slices + 2] on the host: the stop flags,
+// bad_row's word, 1 where a value is no number; codebooks fp32 [slices, n, k]).
+std::tuple<torch::Tensor, torch::Tensor> kmeans_slices_codebooks(torch::Tensor x, c10::optional<torch::Tensor> keep,
+                                                                 torch::Tensor centers, std::string metric, int64_t rule,
+                                                                 double tol, double growth, int64_t max_iter,
+                                                                 int64_t check_every, c10::optional<torch::Tensor> bad_row) {
+  torch::Tensor flags;
+  const int32_t* bad = nullptr;
+  if (bad_row.has_value()) {
+    TORCH_CHECK(bad_row->device() == centers.device() && bad_row->scalar_type() == torch::kInt32 && bad_row->numel() == 1,
+                "bad_row must be one int32 word on the device of centers");
+    bad = bad_row->data_ptr<int32_t>();
+  }
+  fit_slices(x, keep, centers, metric, rule, tol, growth, max_iter, check_every, flags);
+  c10::DeviceGuard guard(centers.device());
+  auto books = torch::empty_like(centers);
+  check_rc(f2cgt_kmeans_rescale(centers.data_ptr<float>(), books.data_ptr<float>(), centers.size(1), centers.size(2),
+                                centers.size(0), bad, flags.data_ptr<int32_t>(), current_stream()),
+           "kmeans_slices_codebooks");
+  py::gil_scoped_release unlocked;
+  return {flags.cpu(), books};
 }
 
 // Counterpart of the reference's raft-backed KMeans (src/kmeans.h:13-31, src/kmeans.cu).
@@ -1131,6 +1163,8 @@ PYBIND11_MODULE(F2CGTLib, m) {
       .def("kmeans_slices_covers", &kmeans_slices_covers, py::arg("slices"), py::arg("n"), py::arg("k"))
       .def("kmeans_slices_fit", &kmeans_slices_fit, py::arg("x"), py::arg("keep"), py::arg("centers"), py::arg("metric"),
            py::arg("rule"), py::arg("tol"), py::arg("growth"), py::arg("max_iter"), py::arg("check_every"))
+      .def("kmeans_slices_codebooks", &kmeans_slices_codebooks, py::arg("x"), py::arg("keep"), py::arg("centers"), py::arg("metric"),
+           py::arg("rule"), py::arg("tol"), py::arg("growth"), py::arg("max_iter"), py::arg("check_every"), py::arg("bad_row"))
       .def("set_store_mode", &set_store_mode, py::arg("mode"));
   py::class_<KMeans>(m, "KMeans")
       .def(py::init<int64_t, int64_t, std::string, int, double, int, double, int, int, bool>(),

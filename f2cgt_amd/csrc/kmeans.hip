@@ -372,6 +372,46 @@ __global__ __launch_bounds__(kKmMergeThreads) void km_merge_slices_kernel(KmArgs
   }
 }
 
+// A slice's centres rescaled to their mean length (examples/process_compress.py:16-18), by one workgroup: divide, then
+// multiply, the lengths and their mean summed in fp64 and rounded.  flags[slices]: the rows' bad_row; flags[slices + 1]: set
+// where a rescaled value is no number.  Six small operators and two reads of flags by the host, 60 us behind a training
+// run, come down to this launch (7 us) and the read of the stop flags.
+__global__ __launch_bounds__(kKmMergeThreads) void km_rescale_kernel(const float* __restrict__ centers, float* __restrict__ out,
+                                                                     int n, int k, int slices, const int32_t* bad_row,
+                                                                     int32_t* flags) {
+  constexpr int kWaves = kKmMergeThreads / kWave;
+  extern __shared__ float s_len[];                          // [n]
+  __shared__ double s_sum[kWaves];
+  const int t = threadIdx.x, slice = blockIdx.x;
+  centers += (int64_t)slice * n * k;
+  out += (int64_t)slice * n * k;
+  double sum = 0.0;
+  for (int c = t; c < n; c += kKmMergeThreads) {
+    double sq = 0.0;
+#pragma unroll 8
+    for (int i = 0; i < k; ++i) sq += (double)centers[c * k + i] * (double)centers[c * k + i];
+    const float len = (float)sqrt(sq);
+    s_len[c] = len;
+    sum += (double)len;
+  }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  if ((t & (kWave - 1)) == 0) s_sum[t / kWave] = sum;
+  __syncthreads();
+  sum = 0.0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) sum += s_sum[w];
+  const float mean = (float)(sum / (double)n);
+  bool nan = false;
+  for (int i = t; i < n * k; i += kKmMergeThreads) {
+    const float v = __fdiv_rn(centers[i], s_len[i / k]) * mean;
+    nan = nan || v != v;
+    out[i] = v;
+  }
+  if (nan) atomicOr(flags + slices + 1, 1);
+  if (slice == 0 && t == 0 && bad_row != nullptr) flags[slices] = *bad_row;
+}
+
 // Rows of a sample, column slice by column slice: out[s][i] = columns [s k, s k + k) of row rows[i] (zeros after the
 // table's last column), norms[i][s] its length.  LANES lanes of four columns each per row and slice, the slices of a row
 // side by side, so that a row is read as one run.
@@ -650,5 +690,16 @@ extern "C" int f2cgt_kmeans_slices_step(const float* x, const uint32_t* keep, fl
   if (parts <= 64) km_merge_slices_kernel<256><<<grid, kKmMergeThreads, 0, st>>>(a, parts, moves, arrived);
   else if (parts <= 128) km_merge_slices_kernel<128><<<grid, kKmMergeThreads, 0, st>>>(a, parts, moves, arrived);
   else km_merge_slices_kernel<64><<<grid, kKmMergeThreads, 0, st>>>(a, parts, moves, arrived);
+  return launch_status(what);
+}
+
+extern "C" int f2cgt_kmeans_rescale(const float* centers, float* out, int64_t n, int64_t k, int64_t slices, const int32_t* bad_row,
+                                    int32_t* flags, void* stream) {
+  const char* what = "kmeans_rescale";
+  F2CGT_REQUIRE(n > 0 && k > 0 && slices > 0, F2CGT_E_INVALID, "%s: sizes must be positive", what);
+  F2CGT_REQUIRE(n <= 8192 && k <= 4096 && slices <= 65535, F2CGT_E_UNSUPPORTED, "%s: too many centres, columns or slices", what);
+  F2CGT_REQUIRE(centers && out && flags, F2CGT_E_INVALID, "%s: null buffer", what);
+  km_rescale_kernel<<<(unsigned)slices, kKmMergeThreads, (size_t)n * 4, as_stream(stream)>>>(centers, out, (int)n, (int)k, (int)slices,
+                                                                                             bad_row, flags);
   return launch_status(what);
 }

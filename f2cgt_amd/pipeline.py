@@ -312,18 +312,20 @@ def _train_all_slices(features, n_clusters, column_slice, sample_index, max_iter
     if whole < slices:
         start[whole, :, :last] = _circle_centers(n_clusters, last)
     centers = start.cuda()
-    flags = capi.kmeans_slices_fit(data, keep, centers, "cosine", 2, 5e-2, 1.2, max_iter, 8)
-    if rows is not None and int(bad_row.item()):
+    flags, codebooks = capi.kmeans_slices_codebooks(data, keep, centers, "cosine", 2, 5e-2, 1.2, max_iter, 8, bad_row)
+    *stop, bad, nan = flags.tolist()
+    if rows is not None and bad:
         raise IndexError("a sample id lies outside the table's %d rows" % features.shape[0])
-    worst = int(flags.max())
+    worst = max(stop)
     if worst == 3:       # their quantile is no number: a NaN among the lengths, or infinities
         raise RuntimeError("a column slice has no rows to train on")
     if worst == 2:
         import warnings
         warnings.warn("vq_metadata: the centre shift became NaN; no centres were produced")
         raise TypeError("a column slice has no centres")
-    norms = torch.linalg.vector_norm(centers, ord=2, dim=2, keepdim=True)
-    return (centers / norms) * norms.mean(dim=1, keepdim=True)
+    if nan:
+        raise ValueError("codebooks has nan")
+    return codebooks
 
 
 def vq_metadata(features, n_clusters, column_slice, hotness=None, sample_index=None, max_iter=1000):
@@ -356,7 +358,7 @@ def vq_metadata(features, n_clusters, column_slice, hotness=None, sample_index=N
         km.fit(data)
         centers = normalize(km.get_centers())
         codebooks[i, :, :hi - lo] = centers
-    if torch.isnan(codebooks).any():
+    if per_slice and torch.isnan(codebooks).any():
         raise ValueError("codebooks has nan")
     return codebooks
 

@@ -349,6 +349,11 @@ int64_t f2cgt_kmeans_slices_workspace_bytes(int64_t m, int64_t slices, int64_t n
 int f2cgt_kmeans_slices_step(const float* x, const uint32_t* keep, float* centers, int32_t* stop, int stop_rule, float tol,
                              void* workspace, int64_t workspace_bytes, int64_t m, int64_t slices, int64_t n, int64_t k,
                              int metric, void* stream);
+/* out [slices, n, k] = every centre divided by its length and multiplied by its slice's mean length
+ * (examples/process_compress.py:16-18).  flags int32 [slices + 2] (device): word `slices` becomes *bad_row (device; NULL: is
+ * left), word slices + 1 is set where a value of out is no number; the others are left alone. */
+int f2cgt_kmeans_rescale(const float* centers, float* out, int64_t n, int64_t k, int64_t slices, const int32_t* bad_row,
+                         int32_t* flags, void* stream);
 
 /* The dense part of a GraphSAGE layer (examples/conv.py:68-76) at the sizes of a minibatch, fp32 throughout.
  *
