@@ -43,6 +43,7 @@ SIGNATURES = {
     "f2cgt_abs_order_stats_workspace_bytes": ([L, L, L], c_int64),
     "f2cgt_abs_order_stats": ([P, L, P, L, L, L, L, P, P, L, P, P], c_int),
     "f2cgt_sq_codebooks": ([P, L, P, L, L, L, L, P, P, P, L, P, P, P], c_int),
+    "f2cgt_sq_codebooks_checked": ([P, L, P, L, L, L, L, P, P, P, L, P, P, P, P, P], c_int),
     "f2cgt_pairwise_distance": ([P, P, P, L, L, L, I, P], c_int),
     "f2cgt_kmeans_predict": ([P, P, P, P, L, L, L, I, P], c_int),
     "f2cgt_vq_encode_slices_covers": ([L, L], c_int),

@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -196,8 +197,38 @@ torch::Tensor sq_encode(torch::Tensor src, torch::Tensor codebooks, int64_t targ
 
 // Extension: order statistics, sum and flags (1: a NaN, 2: a row id outside the table) of |x| per column slice of the rows
 // `rows` (None: all of them), for the codebooks of sq_encode.  ranks: four ranks in a full slice, four in the last one.  -> float64 [n_slices, 6] on the GPU.
+// A flag in pinned memory that a kernel may still set, and the event behind that kernel.
+class PendingFlag {
+ public:
+  PendingFlag() : word_(torch::empty({1}, torch::TensorOptions().dtype(torch::kInt32).pinned_memory(true))) {
+    *word_.data_ptr<int32_t>() = 0;
+    const hipError_t e = hipEventCreateWithFlags(&event_, hipEventDisableTiming);
+    TORCH_CHECK(e == hipSuccess, "cannot create an event: ", hipGetErrorString(e));
+  }
+  PendingFlag(const PendingFlag&) = delete;
+  PendingFlag& operator=(const PendingFlag&) = delete;
+  ~PendingFlag() {                 // the word goes back to its pool only when the kernel is done with it
+    (void)hipEventSynchronize(event_);
+    (void)hipEventDestroy(event_);
+  }
+  // Waits for the kernel.  -> whether it set the flag
+  bool wait() {
+    py::gil_scoped_release unlocked;
+    const hipError_t e = hipEventSynchronize(event_);
+    TORCH_CHECK(e == hipSuccess, "waiting for a check failed: ", hipGetErrorString(e));
+    return *const_cast<volatile int32_t*>(word_.data_ptr<int32_t>()) != 0;
+  }
+  int32_t* word() { return word_.data_ptr<int32_t>(); }
+  void* event() { return static_cast<void*>(event_); }
+
+ private:
+  torch::Tensor word_;
+  hipEvent_t event_ = nullptr;
+};
+
 std::tuple<torch::Tensor, torch::Tensor> order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
-                                                     const std::vector<int64_t>& ranks, const std::vector<float>* weights) {
+                                                     const std::vector<int64_t>& ranks, const std::vector<float>* weights,
+                                                     std::shared_ptr<PendingFlag>* pending = nullptr) {
   TORCH_CHECK(x.defined() && x.device().is_cuda(), "x must be a GPU tensor");
   TORCH_CHECK(x.dim() == 2 && x.scalar_type() == torch::kFloat32, "x must be float32 [rows, feat_dim]");
   // columns apart, or rows that overlap (an expanded row): a copy.  The stride of a single row may be anything.
@@ -222,6 +253,14 @@ std::tuple<torch::Tensor, torch::Tensor> order_stats(torch::Tensor x, c10::optio
   torch::Tensor books;
   if (weights != nullptr) {
     books = torch::empty({slices, 5}, opts.dtype(torch::kFloat32));
+    if (pending != nullptr) {
+      *pending = std::make_shared<PendingFlag>();
+      check_rc(f2cgt_sq_codebooks_checked(x.data_ptr<float>(), ld, list, m, x.size(0), cols, column_slice, ranks.data(),
+                                          weights->data(), ws.data_ptr(), ws.numel(), out.data_ptr<double>(),
+                                          books.data_ptr<float>(), (*pending)->word(), (*pending)->event(), current_stream()),
+               "sq_codebooks_checked");
+      return {out, books};
+    }
     check_rc(f2cgt_sq_codebooks(x.data_ptr<float>(), ld, list, m, x.size(0), cols, column_slice, ranks.data(), weights->data(),
                                 ws.data_ptr(), ws.numel(), out.data_ptr<double>(), books.data_ptr<float>(), current_stream()),
              "sq_codebooks");
@@ -243,6 +282,16 @@ std::tuple<torch::Tensor, torch::Tensor> sq_codebooks(torch::Tensor x, c10::opti
                                                       const std::vector<int64_t>& ranks, const std::vector<float>& weights) {
   auto both = order_stats(x, rows, column_slice, ranks, &weights);
   return {std::get<1>(both), std::get<0>(both)};
+}
+
+// The same, with the check of the row ids on its way to the host.  -> (codebooks, PendingFlag: an id outside the table)
+std::tuple<torch::Tensor, std::shared_ptr<PendingFlag>> sq_codebooks_checked_ids(torch::Tensor x, torch::Tensor rows,
+                                                                                int64_t column_slice,
+                                                                                const std::vector<int64_t>& ranks,
+                                                                                const std::vector<float>& weights) {
+  std::shared_ptr<PendingFlag> pending;
+  auto both = order_stats(x, rows, column_slice, ranks, &weights, &pending);
+  return {std::get<1>(both), pending};
 }
 
 torch::Tensor sq_decompress(torch::Tensor compress_data, torch::Tensor codebooks, int64_t target_bits,
@@ -1144,6 +1193,8 @@ PYBIND11_MODULE(F2CGTLib, m) {
       .def("abs_order_stats", &abs_order_stats, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"))
       .def("sq_codebooks", &sq_codebooks, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"),
            py::arg("weights"))
+      .def("sq_codebooks_checked", &sq_codebooks_checked_ids, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"),
+           py::arg("weights"))
       .def("kmeans_predict", &kmeans_predict, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode", &vq_encode, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode_slices", &vq_encode_slices, py::arg("x"), py::arg("codebooks"), py::arg("out"), py::arg("metric"))
@@ -1166,6 +1217,7 @@ PYBIND11_MODULE(F2CGTLib, m) {
       .def("kmeans_slices_codebooks", &kmeans_slices_codebooks, py::arg("x"), py::arg("keep"), py::arg("centers"), py::arg("metric"),
            py::arg("rule"), py::arg("tol"), py::arg("growth"), py::arg("max_iter"), py::arg("check_every"), py::arg("bad_row"))
       .def("set_store_mode", &set_store_mode, py::arg("mode"));
+  py::class_<PendingFlag, std::shared_ptr<PendingFlag>>(m, "PendingFlag").def("wait", &PendingFlag::wait);
   py::class_<KMeans>(m, "KMeans")
       .def(py::init<int64_t, int64_t, std::string, int, double, int, double, int, int, bool>(),
            py::arg("n_cluster"), py::arg("feat_dim"), py::arg("metric"), py::arg("max_iter") = 300,

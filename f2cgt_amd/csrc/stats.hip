@@ -12,11 +12,11 @@
 //
 // What bounds it: two reads of the sample (17 us each at 120 000 x 100 values, 2.9 TB/s through the row list; the first is
 // as long on its LDS counters as on its loads), the sums between the passes (4 us each) and the third pass, which reads
-// what the second kept and takes 5 us (17 with the sample read again).  The seven launches take 56 us, with eight rows and
-// the next eight ids in flight per thread, where four rows without the ids of the next took 66 and the host took 195 ms
-// on a copy of the sample (np.percentile, two selections).  The codebook is made by the last of them, so that the encoder
-// can follow at once: the whole sq_compress call takes 90 us (130 with the codebook made on the host, 102 with three
-// reads), of which the encoder is 15 and the read-back of the flags at the end about 20.  100 000 x 602 values 598 -> 445;
+// what the second kept and takes 5 us (17 with the sample read again).  The codebook is made by the last workgroup of the
+// last sum, so that the encoder can follow at once, and the ids' check is on the host as soon as the first pass is done, so
+// that a caller does not wait for the rest: the six launches take 52 us (seven 56; four rows in flight without the ids of the
+// next 66; the host 195 ms on a copy of the sample, np.percentile), a sq_compress call among others 70 (90 with a wait for
+// its end, 130 with the codebook made on the host), of which the encoder is 15.  100 000 x 602 values 598 -> 445;
 // tables on which a workgroup has to read its rows again are no slower than before (all values equal 438 -> 412, 80 %
 // zeros 253 -> 219).
 #include "common.hpp"
@@ -56,6 +56,8 @@ struct StatArgs {
   uint32_t* kept;                    // [n_slices][blocks][kStatWaves][keep]: values that share the first digit of a wanted rank
   uint32_t* n_kept;                  // [n_slices][blocks][kStatWaves]: how many; more than `keep`: not all of them are there
   double* out;                       // [n_slices][6]
+  uint32_t* arrived;                 // [n_slices]: workgroups of the last sum that are done with a slice
+  int32_t* bad;                      // host memory: set by the first pass where a row id lies outside the table; or null
   float* books;                      // [n_slices][5], or null
   float weights[4];                  // lower and upper percentile of a slice, and of the last one: where between its ranks
 };
@@ -290,30 +292,13 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
     }
   }
   if (PASS == 0 && t == 0) {
+    if (blockIdx.x == 0) a.arrived[slice] = 0u;
+    if (a.bad != nullptr && (s_flags & kSawBadRow)) *a.bad = 1;
     double total = 0.0;
     for (int w = 0; w < kStatThreads / kWave; ++w) total += s_sum[w];
     a.sums[place] = total;
     a.flags[place] = s_flags;
   }
-}
-
-// hist[bin] = sum of the workgroups' counts: a wave reads 64 neighbouring bins of every sixteenth workgroup, all its
-// reads in flight at once (with four waves to 64 bins, four rounds of reads each, the kernel took 9 us instead of 4).
-__global__ __launch_bounds__(kStatThreads) void stat_reduce_kernel(StatArgs a) {
-  constexpr int WAVES = kStatThreads / kWave;
-  __shared__ uint32_t s_part[WAVES][kWave];
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int bin = blockIdx.x * kWave + lane, slice = blockIdx.y;
-  const uint32_t* src = a.partial + (int64_t)slice * a.blocks * kBins + bin;
-  uint32_t c = 0;
-#pragma unroll 16
-  for (int b = wave; b < a.blocks; b += WAVES) c += src[(int64_t)b * kBins];
-  s_part[wave][lane] = c;
-  __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int w = 1; w < WAVES; ++w) c += s_part[w][lane];
-  a.hist[(int64_t)slice * kBins + bin] = c;
 }
 
 // The quantiser's codebook of a slice (fmin, fmax, emin, emax, mean) from its statistics: percentiles interpolated in
@@ -341,12 +326,9 @@ __device__ void sq_codebook(const StatArgs& a, int slice, const float (&at)[4], 
   book[4] = level;
 }
 
-// Last digit, and the outputs of a slice: the values at the four ranks, the sum, the flags.
-__global__ __launch_bounds__(kStatThreads) void stat_finish_kernel(StatArgs a) {
-  __shared__ uint64_t s_scan[kStatThreads / kWave];
-  __shared__ uint32_t s_digit[4];
-  __shared__ uint64_t s_rest[4];
-  const int slice = blockIdx.x, t = threadIdx.x;
+// Last digit, and the outputs of a slice: the values at the four ranks, the sum, the flags; by one workgroup.
+__device__ void stat_finish(const StatArgs& a, int slice, uint64_t* s_scan, uint32_t* s_digit, uint64_t* s_rest) {
+  const int t = threadIdx.x;
   uint32_t prefix[4];
   uint64_t rank[4];
   known_digits<3>(a, slice, s_scan, s_digit, s_rest, prefix, rank);
@@ -375,6 +357,40 @@ __global__ __launch_bounds__(kStatThreads) void stat_finish_kernel(StatArgs a) {
   }
 }
 
+// hist[bin] = sum of the workgroups' counts: a wave reads 64 neighbouring bins of every sixteenth workgroup, all its
+// reads in flight at once (with four waves to 64 bins, four rounds of reads each, the kernel took 9 us instead of 4).
+// LAST: the workgroup that finishes a slice goes on to its last digit and outputs, a launch less (3.8 us of 55).
+template <bool LAST>
+__global__ __launch_bounds__(kStatThreads) void stat_reduce_kernel(StatArgs a) {
+  constexpr int WAVES = kStatThreads / kWave;
+  __shared__ uint32_t s_part[WAVES][kWave];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int bin = blockIdx.x * kWave + lane, slice = blockIdx.y;
+  const uint32_t* src = a.partial + (int64_t)slice * a.blocks * kBins + bin;
+  uint32_t c = 0;
+#pragma unroll 16
+  for (int b = wave; b < a.blocks; b += WAVES) c += src[(int64_t)b * kBins];
+  s_part[wave][lane] = c;
+  __syncthreads();
+  if (wave == 0) {
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) c += s_part[w][lane];
+    a.hist[(int64_t)slice * kBins + bin] = c;
+  }
+  if constexpr (LAST) {
+    __shared__ uint64_t s_scan[kStatThreads / kWave];
+    __shared__ uint32_t s_digit[4];
+    __shared__ uint64_t s_rest[4];
+    __shared__ int s_last;
+    __syncthreads();
+    // release: the other workgroups' sums before their count; acquire: this one's reads of them behind it
+    if (threadIdx.x == 0)
+      s_last = __hip_atomic_fetch_add(a.arrived + slice, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u;
+    __syncthreads();
+    if (s_last) stat_finish(a, slice, s_scan, s_digit, s_rest);
+  }
+}
+
 // Workgroups per slice: one per CU over all slices, each with at least 32 values per thread.
 int stat_blocks(int64_t m, int64_t cols, int64_t slice, int64_t n_slices) {
   const int64_t width = cols < slice ? cols : slice;
@@ -388,7 +404,7 @@ int64_t round256(int64_t v) { return (v + 255) / 256 * 256; }
 
 int stat_keep(int64_t blocks, int64_t n_slices) { return n_slices * blocks <= kKeepBlocks ? kKept : 0; }
 
-struct StatLayout { int64_t hist, state, sums, flags, kept, n_kept, total; };
+struct StatLayout { int64_t hist, state, sums, flags, kept, n_kept, arrived, total; };
 StatLayout stat_layout(int64_t blocks, int64_t n_slices) {
   StatLayout l;
   l.hist = round256(n_slices * blocks * kBins * 4);
@@ -397,21 +413,24 @@ StatLayout stat_layout(int64_t blocks, int64_t n_slices) {
   l.flags = l.sums + round256(n_slices * blocks * 8);
   l.kept = l.flags + round256(n_slices * blocks * 4);
   l.n_kept = l.kept + round256(n_slices * blocks * kStatWaves * stat_keep(blocks, n_slices) * 4);
-  l.total = l.n_kept + round256(n_slices * blocks * kStatWaves * 4);
+  l.arrived = l.n_kept + round256(n_slices * blocks * kStatWaves * 4);
+  l.total = l.arrived + round256(n_slices * 4);
   return l;
 }
 
+// checked: recorded behind the first pass, which has then reported the row ids outside the table; or null.
 template <int V>
-void stat_launch(const StatArgs& a, hipStream_t st) {
+hipError_t stat_launch(const StatArgs& a, hipEvent_t checked, hipStream_t st) {
   const dim3 grid((unsigned)a.blocks, (unsigned)a.n_slices), rgrid(kBins / kWave, (unsigned)a.n_slices);
   const dim3 rgrid_last(2048 / kWave, (unsigned)a.n_slices);
   stat_pass_kernel<0, V><<<grid, kStatThreads, 0, st>>>(a);
-  stat_reduce_kernel<<<rgrid, kStatThreads, 0, st>>>(a);
+  const hipError_t e = checked != nullptr ? hipEventRecord(checked, st) : hipSuccess;
+  stat_reduce_kernel<false><<<rgrid, kStatThreads, 0, st>>>(a);
   stat_pass_kernel<1, V><<<grid, kStatThreads, 0, st>>>(a);
-  stat_reduce_kernel<<<rgrid, kStatThreads, 0, st>>>(a);
+  stat_reduce_kernel<false><<<rgrid, kStatThreads, 0, st>>>(a);
   stat_pass_kernel<2, V><<<grid, kStatThreads, 0, st>>>(a);
-  stat_reduce_kernel<<<rgrid_last, kStatThreads, 0, st>>>(a);
-  stat_finish_kernel<<<(unsigned)a.n_slices, kStatThreads, 0, st>>>(a);
+  stat_reduce_kernel<true><<<rgrid_last, kStatThreads, 0, st>>>(a);
+  return e;
 }
 
 int stat_check(const char* what, int64_t m, int64_t cols, int64_t slice) {
@@ -434,7 +453,7 @@ extern "C" int64_t f2cgt_abs_order_stats_workspace_bytes(int64_t m, int64_t cols
 namespace {
 int order_stats(const char* what, const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols,
                 int64_t column_slice, const int64_t* ranks, const float* weights, void* workspace, int64_t workspace_bytes,
-                double* out, float* books, void* stream) {
+                double* out, float* books, int32_t* bad, void* checked, void* stream) {
   if (int rc = stat_check(what, m, cols, column_slice)) return rc;
   F2CGT_REQUIRE(ld >= cols && num_rows > 0 && (rows != nullptr || m <= num_rows), F2CGT_E_INVALID,
                 "%s: the sample does not fit the table", what);
@@ -464,6 +483,8 @@ int order_stats(const char* what, const float* x, int64_t ld, const int64_t* row
   a.keep = stat_keep(a.blocks, n_slices);
   a.kept = reinterpret_cast<uint32_t*>(ws + l.kept);
   a.n_kept = reinterpret_cast<uint32_t*>(ws + l.n_kept);
+  a.arrived = reinterpret_cast<uint32_t*>(ws + l.arrived);
+  a.bad = bad;
   a.out = out;
   a.books = books;
   if (books != nullptr)
@@ -474,9 +495,9 @@ int order_stats(const char* what, const float* x, int64_t ld, const int64_t* row
     return ld % v == 0 && (n_slices == 1 || column_slice % v == 0) && last_width % v == 0 && aligned(x, 4 * v);
   };
   hipStream_t st = as_stream(stream);
-  if (fits(4)) stat_launch<4>(a, st);
-  else if (fits(2)) stat_launch<2>(a, st);
-  else stat_launch<1>(a, st);
+  hipEvent_t ev = static_cast<hipEvent_t>(checked);
+  const hipError_t e = fits(4) ? stat_launch<4>(a, ev, st) : fits(2) ? stat_launch<2>(a, ev, st) : stat_launch<1>(a, ev, st);
+  if (e != hipSuccess) return fail((int)e, "%s: cannot record the event: %s", what, hipGetErrorString(e));
   return launch_status(what);
 }
 }  // namespace
@@ -485,7 +506,7 @@ extern "C" int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* 
                                      int64_t cols, int64_t column_slice, const int64_t* ranks, void* workspace,
                                      int64_t workspace_bytes, double* out, void* stream) {
   return order_stats("abs_order_stats", x, ld, rows, m, num_rows, cols, column_slice, ranks, nullptr, workspace,
-                     workspace_bytes, out, nullptr, stream);
+                     workspace_bytes, out, nullptr, nullptr, nullptr, stream);
 }
 
 extern "C" int f2cgt_sq_codebooks(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols,
@@ -493,5 +514,14 @@ extern "C" int f2cgt_sq_codebooks(const float* x, int64_t ld, const int64_t* row
                                   int64_t workspace_bytes, double* stats, float* codebooks, void* stream) {
   F2CGT_REQUIRE(weights && codebooks, F2CGT_E_INVALID, "sq_codebooks: null buffer");
   return order_stats("sq_codebooks", x, ld, rows, m, num_rows, cols, column_slice, ranks, weights, workspace,
-                     workspace_bytes, stats, codebooks, stream);
+                     workspace_bytes, stats, codebooks, nullptr, nullptr, stream);
+}
+
+extern "C" int f2cgt_sq_codebooks_checked(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols,
+                                          int64_t column_slice, const int64_t* ranks, const float* weights, void* workspace,
+                                          int64_t workspace_bytes, double* stats, float* codebooks, int32_t* bad_row, void* checked,
+                                          void* stream) {
+  F2CGT_REQUIRE(weights && codebooks && bad_row && checked, F2CGT_E_INVALID, "sq_codebooks_checked: null buffer or event");
+  return order_stats("sq_codebooks_checked", x, ld, rows, m, num_rows, cols, column_slice, ranks, weights, workspace,
+                     workspace_bytes, stats, codebooks, bad_row, checked, stream);
 }

@@ -163,15 +163,16 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
     if sample_index is None:
         sample_index = sampling(250_000, num_items, hotness)
     sample_index = sample_index.to(features.device)
-    stats = None
+    bad_id = None
     if (features.is_cuda and features.dtype == torch.float32 and features.stride(1) == 1 and features.stride(0) >= feat_dim and
             sample_index.dtype == torch.int64 and sample_index.dim() == 1 and not features.requires_grad and
             _device_takes(sample_index.numel(), feat_dim, column_slice)):
-        # the sample's rows are read in place, the codebooks made where they are used; a bad id is found at the end
+        # the sample's rows are read in place, the codebooks made where they are used; the ids' check comes to the host
+        # from the first of these kernels, so that only that one is waited for
         places = _percentile_places(sample_index.numel(), feat_dim, column_slice)[1]
-        codebooks, stats = capi.sq_codebooks(features, sample_index, column_slice,
-                                             [r for per_size in places for place in per_size for r in place[:2]],
-                                             [place[2] for per_size in places for place in per_size])
+        codebooks, bad_id = capi.sq_codebooks_checked(features, sample_index, column_slice,
+                                                      [r for per_size in places for place in per_size for r in place[:2]],
+                                                      [place[2] for per_size in places for place in per_size])
         codebooks = codebooks.cuda()      # (the codes are made on the current device, wherever the table lies)
     else:
         per_slice = [[float(v) for v in values] for values in _sampled_sq_codebooks(features, sample_index, column_slice)]
@@ -188,7 +189,7 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
         data = features[start:end].cuda().to(torch.float32)
         # one pass; the reference calls sq_compress, casts and packs (process_compress.py:128-139)
         capi.sq_encode(data, codebooks, target_bits, column_slice, out[start:end])
-    if stats is not None and stats.cpu().numpy()[:, 5].max() >= 2:
+    if bad_id is not None and bad_id.wait():
         raise IndexError("a sample id lies outside the table's %d rows" % num_items)
     return out, codebooks
 

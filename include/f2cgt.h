@@ -258,6 +258,13 @@ int f2cgt_abs_order_stats(const float* x, int64_t ld, const int64_t* rows, int64
 int f2cgt_sq_codebooks(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols,
                        int64_t column_slice, const int64_t* ranks, const float* weights, void* workspace,
                        int64_t workspace_bytes, double* stats, float* codebooks, void* stream);
+/* The same; the first kernel also sets *bad_row (host memory that the device can write, e.g. hipHostMalloc'ed, cleared by the
+ * caller) where an id of rows lies outside the table, and the event `checked` (a hipEvent_t) is recorded behind it, so that a
+ * caller can wait for the ids alone. */
+int f2cgt_sq_codebooks_checked(const float* x, int64_t ld, const int64_t* rows, int64_t m, int64_t num_rows, int64_t cols,
+                               int64_t column_slice, const int64_t* ranks, const float* weights, void* workspace,
+                               int64_t workspace_bytes, double* stats, float* codebooks, int32_t* bad_row, void* checked,
+                               void* stream);
 
 /* ---- VQ encode ---------------------------------------------------------------- */
 
