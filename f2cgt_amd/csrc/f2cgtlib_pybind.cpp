@@ -9,6 +9,7 @@
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
 #include <hip/hip_runtime_api.h>
@@ -277,21 +278,17 @@ torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows
   return std::get<0>(order_stats(x, rows, column_slice, ranks, nullptr));
 }
 
-// -> (codebooks fp32 [slices, 5], the statistics they were made from fp64 [slices, 6]), both on the device.
-std::tuple<torch::Tensor, torch::Tensor> sq_codebooks(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
-                                                      const std::vector<int64_t>& ranks, const std::vector<float>& weights) {
-  auto both = order_stats(x, rows, column_slice, ranks, &weights);
-  return {std::get<1>(both), std::get<0>(both)};
-}
-
-// The same, with the check of the row ids on its way to the host.  -> (codebooks, PendingFlag: an id outside the table)
-std::tuple<torch::Tensor, std::shared_ptr<PendingFlag>> sq_codebooks_checked_ids(torch::Tensor x, torch::Tensor rows,
-                                                                                int64_t column_slice,
-                                                                                const std::vector<int64_t>& ranks,
-                                                                                const std::vector<float>& weights) {
+// -> (codebooks fp32 [slices, 5], the statistics they were made from fp64 [slices, 6]), both on the device.  With a row list,
+// outside a graph's capture, the check of its ids is on its way to the host: the statistics carry it as `bad_rows`, a
+// PendingFlag.
+std::tuple<torch::Tensor, py::object> sq_codebooks(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
+                                                   const std::vector<int64_t>& ranks, const std::vector<float>& weights) {
   std::shared_ptr<PendingFlag> pending;
-  auto both = order_stats(x, rows, column_slice, ranks, &weights, &pending);
-  return {std::get<1>(both), pending};
+  const bool check = rows.has_value() && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+  auto both = order_stats(x, rows, column_slice, ranks, &weights, check ? &pending : nullptr);
+  py::object stats = py::cast(std::get<0>(both));
+  if (check) stats.attr("bad_rows") = py::cast(pending);
+  return {std::get<1>(both), stats};
 }
 
 torch::Tensor sq_decompress(torch::Tensor compress_data, torch::Tensor codebooks, int64_t target_bits,
@@ -536,21 +533,13 @@ bool fit_slices(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tenso
   return false;
 }
 
-torch::Tensor kmeans_slices_fit(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, std::string metric,
-                                int64_t rule, double tol, double growth, int64_t max_iter, int64_t check_every) {
-  torch::Tensor flags;
-  fit_slices(x, keep, centers, metric, rule, tol, growth, max_iter, check_every, flags);
-  py::gil_scoped_release unlocked;
-  return flags.narrow(0, 0, centers.size(0)).cpu();
-}
-
-// The same, and the centres rescaled to their slice's mean length.  -> (flags int32 [slices + 2] on the host: the stop flags,
-// bad_row's word, 1 where a value is no number; codebooks fp32 [slices, n, k]).
-std::tuple<torch::Tensor, torch::Tensor> kmeans_slices_codebooks(torch::Tensor x, c10::optional<torch::Tensor> keep,
-                                                                 torch::Tensor centers, std::string metric, int64_t rule,
-                                                                 double tol, double growth, int64_t max_iter,
-                                                                 int64_t check_every, c10::optional<torch::Tensor> bad_row) {
-  torch::Tensor flags;
+// -> the stop flags, int32 [slices] on the host.  rescale: the centres are also rescaled to their slice's mean length, and
+// the result is (flags int32 [slices + 2] on the host: the stop flags, bad_row's word, 1 where a value is no number;
+// codebooks fp32 [slices, n, k]), with one wait for all of it.
+py::object kmeans_slices_fit(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, std::string metric,
+                             int64_t rule, double tol, double growth, int64_t max_iter, int64_t check_every,
+                             c10::optional<torch::Tensor> bad_row, bool rescale) {
+  torch::Tensor flags, books;
   const int32_t* bad = nullptr;
   if (bad_row.has_value()) {
     TORCH_CHECK(bad_row->device() == centers.device() && bad_row->scalar_type() == torch::kInt32 && bad_row->numel() == 1,
@@ -558,13 +547,22 @@ std::tuple<torch::Tensor, torch::Tensor> kmeans_slices_codebooks(torch::Tensor x
     bad = bad_row->data_ptr<int32_t>();
   }
   fit_slices(x, keep, centers, metric, rule, tol, growth, max_iter, check_every, flags);
-  c10::DeviceGuard guard(centers.device());
-  auto books = torch::empty_like(centers);
-  check_rc(f2cgt_kmeans_rescale(centers.data_ptr<float>(), books.data_ptr<float>(), centers.size(1), centers.size(2),
-                                centers.size(0), bad, flags.data_ptr<int32_t>(), current_stream()),
-           "kmeans_slices_codebooks");
-  py::gil_scoped_release unlocked;
-  return {flags.cpu(), books};
+  const int64_t slices = centers.size(0);
+  if (rescale) {
+    c10::DeviceGuard guard(centers.device());
+    books = torch::empty_like(centers);
+    check_rc(f2cgt_kmeans_rescale(centers.data_ptr<float>(), books.data_ptr<float>(), centers.size(1), centers.size(2), slices, bad,
+                                  flags.data_ptr<int32_t>(), current_stream()),
+             "kmeans_slices_fit");
+  } else {
+    flags = flags.narrow(0, 0, slices);
+  }
+  {
+    py::gil_scoped_release unlocked;
+    flags = flags.cpu();
+  }
+  if (!rescale) return py::cast(flags);
+  return py::make_tuple(flags, books);
 }
 
 // Counterpart of the reference's raft-backed KMeans (src/kmeans.h:13-31, src/kmeans.cu).
@@ -1193,8 +1191,6 @@ PYBIND11_MODULE(F2CGTLib, m) {
       .def("abs_order_stats", &abs_order_stats, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"))
       .def("sq_codebooks", &sq_codebooks, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"),
            py::arg("weights"))
-      .def("sq_codebooks_checked", &sq_codebooks_checked_ids, py::arg("x"), py::arg("rows"), py::arg("column_slice"), py::arg("ranks"),
-           py::arg("weights"))
       .def("kmeans_predict", &kmeans_predict, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode", &vq_encode, py::arg("x"), py::arg("centers"), py::arg("metric"))
       .def("vq_encode_slices", &vq_encode_slices, py::arg("x"), py::arg("codebooks"), py::arg("out"), py::arg("metric"))
@@ -1213,9 +1209,8 @@ PYBIND11_MODULE(F2CGTLib, m) {
       .def("keep_rows", &keep_rows, py::arg("norms"), py::arg("stats"), py::arg("weight"), py::arg("weight_last"))
       .def("kmeans_slices_covers", &kmeans_slices_covers, py::arg("slices"), py::arg("n"), py::arg("k"))
       .def("kmeans_slices_fit", &kmeans_slices_fit, py::arg("x"), py::arg("keep"), py::arg("centers"), py::arg("metric"),
-           py::arg("rule"), py::arg("tol"), py::arg("growth"), py::arg("max_iter"), py::arg("check_every"))
-      .def("kmeans_slices_codebooks", &kmeans_slices_codebooks, py::arg("x"), py::arg("keep"), py::arg("centers"), py::arg("metric"),
-           py::arg("rule"), py::arg("tol"), py::arg("growth"), py::arg("max_iter"), py::arg("check_every"), py::arg("bad_row"))
+           py::arg("rule"), py::arg("tol"), py::arg("growth"), py::arg("max_iter"), py::arg("check_every"),
+           py::arg("bad_row") = py::none(), py::arg("rescale") = false)
       .def("set_store_mode", &set_store_mode, py::arg("mode"));
   py::class_<PendingFlag, std::shared_ptr<PendingFlag>>(m, "PendingFlag").def("wait", &PendingFlag::wait);
   py::class_<KMeans>(m, "KMeans")

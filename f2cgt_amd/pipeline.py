@@ -154,6 +154,12 @@ def _sampled_sq_codebooks(features, sample_index, column_slice):
     return per_slice
 
 
+def _bad_rows(stats):
+    """Whether an id of the sample that statistics were made of lies outside its table."""
+    pending = getattr(stats, "bad_rows", None)
+    return pending.wait() if pending is not None else stats.cpu().numpy()[:, 5].max() >= 2
+
+
 def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=None, batch_rows=1_000_000):
     """-> (storage, codebooks).  storage: int8 [N, ceil(D * bits / 8)] holding the packed bit
     patterns (bits <= 8) or int16 [N, D]; codebooks fp32 [ceil(D / column_slice), 5] on the GPU
@@ -163,16 +169,16 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
     if sample_index is None:
         sample_index = sampling(250_000, num_items, hotness)
     sample_index = sample_index.to(features.device)
-    bad_id = None
+    stats = None
     if (features.is_cuda and features.dtype == torch.float32 and features.stride(1) == 1 and features.stride(0) >= feat_dim and
             sample_index.dtype == torch.int64 and sample_index.dim() == 1 and not features.requires_grad and
             _device_takes(sample_index.numel(), feat_dim, column_slice)):
         # the sample's rows are read in place, the codebooks made where they are used; the ids' check comes to the host
         # from the first of these kernels, so that only that one is waited for
         places = _percentile_places(sample_index.numel(), feat_dim, column_slice)[1]
-        codebooks, bad_id = capi.sq_codebooks_checked(features, sample_index, column_slice,
-                                                      [r for per_size in places for place in per_size for r in place[:2]],
-                                                      [place[2] for per_size in places for place in per_size])
+        codebooks, stats = capi.sq_codebooks(features, sample_index, column_slice,
+                                             [r for per_size in places for place in per_size for r in place[:2]],
+                                             [place[2] for per_size in places for place in per_size])
         codebooks = codebooks.cuda()      # (the codes are made on the current device, wherever the table lies)
     else:
         per_slice = [[float(v) for v in values] for values in _sampled_sq_codebooks(features, sample_index, column_slice)]
@@ -189,7 +195,7 @@ def sq_compress(features, target_bits, column_slice, hotness=None, sample_index=
         data = features[start:end].cuda().to(torch.float32)
         # one pass; the reference calls sq_compress, casts and packs (process_compress.py:128-139)
         capi.sq_encode(data, codebooks, target_bits, column_slice, out[start:end])
-    if bad_id is not None and bad_id.wait():
+    if stats is not None and _bad_rows(stats):
         raise IndexError("a sample id lies outside the table's %d rows" % num_items)
     return out, codebooks
 
@@ -313,7 +319,7 @@ def _train_all_slices(features, n_clusters, column_slice, sample_index, max_iter
     if whole < slices:
         start[whole, :, :last] = _circle_centers(n_clusters, last)
     centers = start.cuda()
-    flags, codebooks = capi.kmeans_slices_codebooks(data, keep, centers, "cosine", 2, 5e-2, 1.2, max_iter, 8, bad_row)
+    flags, codebooks = capi.kmeans_slices_fit(data, keep, centers, "cosine", 2, 5e-2, 1.2, max_iter, 8, bad_row, True)
     *stop, bad, nan = flags.tolist()
     if rows is not None and bad:
         raise IndexError("a sample id lies outside the table's %d rows" % features.shape[0])

@@ -21,14 +21,14 @@ def test_codebooks_and_flag(rows, dim, slice_):
         places = pipeline._percentile_places(m, dim, slice_)[1]
         ranks = [r for per_size in places for place in per_size for r in place[:2]]
         weights = [place[2] for per_size in places for place in per_size]
-        want, stats = lib.sq_codebooks(x, ids, slice_, ranks, weights)
+        want, stats = lib.sq_codebooks(x[ids], None, slice_, ranks, weights)
+        assert not hasattr(stats, "bad_rows")
         for _ in range(3):                        # the workgroup that finishes last differs from run to run
-            books, flag = lib.sq_codebooks_checked(x, ids, slice_, ranks, weights)
-            assert not flag.wait() and torch.equal(books, want) and not flag.wait()
+            books, stats = lib.sq_codebooks(x, ids, slice_, ranks, weights)
+            assert not stats.bad_rows.wait() and torch.equal(books, want) and not stats.bad_rows.wait()
         assert int(stats[:, 5].max()) == 0
         ids[m // 2] = rows
-        flag = lib.sq_codebooks_checked(x, ids, slice_, ranks, weights)[1]
-        assert flag.wait()
+        assert lib.sq_codebooks(x, ids, slice_, ranks, weights)[1].bad_rows.wait()
 
 
 def test_errors_and_calls_one_after_the_other():
@@ -47,3 +47,29 @@ def test_errors_and_calls_one_after_the_other():
             assert torch.equal(books, want[1]) and torch.equal(codes, want[0])
     with pytest.raises(NotImplementedError):
         pipeline.sq_compress(x, 17, 64, sample_index=good)      # raised with the statistics still on their way
+
+
+def test_codebooks_in_a_captured_graph():
+    lib = f2cgt_amd.load()
+    x = torch.randn((20000, 32), device="cuda")
+    ids = torch.randint(0, 20000, (9000,), device="cuda")
+    places = pipeline._percentile_places(9000, 32, 32)[1]
+    ranks = [r for per_size in places for place in per_size for r in place[:2]]
+    weights = [place[2] for per_size in places for place in per_size]
+    make = lambda: lib.sq_codebooks(x, ids, 32, ranks, weights)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        make()[1].bad_rows.wait()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        books, stats = make()
+    assert not hasattr(stats, "bad_rows")             # nothing waits during a capture
+    for _ in range(4):
+        x.normal_()
+        ids.copy_(torch.randint(0, 20000, (9000,), device="cuda"))
+        torch.cuda.synchronize()
+        graph.replay()
+        got = books.clone()
+        assert torch.equal(got, make()[0])

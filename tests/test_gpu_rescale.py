@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 def _codebooks(centers, bad=None):
     """The loop with no step to make, so that the centres are the ones given."""
     x = torch.randn((centers.shape[0], 64, centers.shape[2]), device="cuda")
-    return f2cgt_amd.load().kmeans_slices_codebooks(x, None, centers, "cosine", 2, 5e-2, 1.2, 0, 8, bad)
+    return f2cgt_amd.load().kmeans_slices_fit(x, None, centers, "cosine", 2, 5e-2, 1.2, 0, 8, bad, True)
 
 
 @pytest.mark.parametrize("slices,n,k", [(1, 1, 1), (3, 16, 8), (6, 256, 16), (2, 257, 33), (1, 512, 64)])
