@@ -1009,7 +1009,7 @@ struct RowsArgs {
   uint32_t fin_magic;
   int nt_out;            // output larger than the last-level cache: non-temporal stores
   int items_per_row;     // ITEM: column groups of a row, and ceil(2^32 / that)
-  uint32_t item_magic;
+  uint32_t item_magic;   // of eight columns: ceil(2^31 / items_per_row), times twice the item
 };
 
 
@@ -1039,8 +1039,8 @@ __device__ __forceinline__ void add_signs(float (&s)[8], uint32_t byte, const un
 // with the store form fixed at compile time the row loop came out 3-5 % faster at 100-256 columns and 17-19 % at 600
 // (3e6 edges, 10 per row, 4 bit: 97.8 -> 93.7 us at 128 columns, 592 -> 489 us at 600); 1- and 2-bit rows measured
 // level to 2 % slower and keep the run-time test.
-// ITEM: 0 (a lane keeps a column group), or the columns of the items that are dealt to the lanes: 4, or 8 (1 bit).
-// The eight columns of a 1-bit item are stored after the two halves of the wave have exchanged theirs
+// ITEM: 0 (a lane keeps a column group), or the columns of the items that are dealt to the lanes: 4 (staged codes), or 8
+// (codes read where they are).  The eight columns of such an item are stored after the two halves of the wave have exchanged theirs
 // (v_permlane32_swap): the lower lanes' items go out with one store instruction, 16 bytes per lane one after the other,
 // the upper lanes' with the next, where a lane's own two 16-byte stores would each write 16 of every 32 bytes.
 template <int BITS, bool AFFINE, typename Idx, int TB, int HALF = 0, int ITEM = 0>
@@ -1169,40 +1169,56 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
     constexpr int G = ITEM;                              // columns of an item
     constexpr int GB = G * BITS / 8;                     // code bytes that hold them
     const int items = nrows * a.items_per_row;
-    if constexpr (SIGNS) {
-      const float minus_plus = -s_lut[1];
+    if constexpr (ITEM == 8) {
+      // codes read where they are, see launch_sq_rows_sized
+      const float minus_plus = SIGNS ? -s_lut[1] : 0.f;
+      using Word = std::conditional_t<BITS == 8, uint64_t, uint32_t>;
+      constexpr int WB = BITS;                               // bytes of eight codes
       const int lane = t & 63;
       char* obase = reinterpret_cast<char*>(out + row0 * (int64_t)a.feat_dim);
       for (int first = t - lane; first < items; first += TB) {     // the same for all lanes of a wave
         const int item = first + lane < items ? first + lane : items - 1;
-        const int ri = (int)__umulhi((uint32_t)item, a.item_magic);
+        const int ri = (int)__umulhi(2u * (uint32_t)item, a.item_magic);
         const int c = item - ri * a.items_per_row;
         const int r = s_order[ri];
         const int b = s_ptr[r], e = s_ptr[r + 1];
         float s[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) s[i] = 0.f;
-        const uint8_t* column = a.codes + c;
-        auto code_at = [&](uint32_t id) -> uint32_t { return column[(uint64_t)id * (uint32_t)a.src_dim]; };
+        // an item that a row ends in is read earlier, inside the row (rows have at least eight bytes), and shifted
+        const int first_byte = c * WB;
+        const int at_byte = BITS > 1 && first_byte > a.eff_bytes - WB ? a.eff_bytes - WB : first_byte;
+        const int shift = 8 * (first_byte - at_byte);
+        auto load = [&](const uint8_t* q) -> Word {
+          if constexpr (BITS == 1) return *q;
+          Word w = 0;
+          __builtin_memcpy(&w, q, WB);
+          return w >> shift;
+        };
+        auto code_at = [&](uint32_t id) -> Word { return load(a.codes + ((uint64_t)id * (uint32_t)a.src_dim + (uint32_t)at_byte)); };
+        auto add = [&](Word w) {
+          if constexpr (SIGNS) {
+            add_signs(s, (uint32_t)w, smem, minus_plus);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) s[i] += s_lut[(uint32_t)(w >> (BITS * i)) & MASK];
+          }
+        };
         auto walk = [&](auto read) {
           int k = b;
           for (; k + 4 <= e; k += 4) {
-            const uint32_t w0 = read(k), w1 = read(k + 1), w2 = read(k + 2), w3 = read(k + 3);
-            add_signs(s, w0, smem, minus_plus);
-            add_signs(s, w1, smem, minus_plus);
-            add_signs(s, w2, smem, minus_plus);
-            add_signs(s, w3, smem, minus_plus);
+            const Word w0 = read(k), w1 = read(k + 1), w2 = read(k + 2), w3 = read(k + 3);
+            add(w0); add(w1); add(w2); add(w3);
           }
           if (k + 2 <= e) {
-            const uint32_t w0 = read(k), w1 = read(k + 1);
-            add_signs(s, w0, smem, minus_plus);
-            add_signs(s, w1, smem, minus_plus);
+            const Word w0 = read(k), w1 = read(k + 1);
+            add(w0); add(w1);
             k += 2;
           }
-          if (k < e) add_signs(s, read(k), smem, minus_plus);
+          if (k < e) add(read(k));
         };
-        if (have_ids) walk([&](int k) -> uint32_t { return code_at(s_ids[k]); });
-        else walk([&](int k) -> uint32_t { return code_at((uint32_t)clamp_idx(indices[e0 + k], a.N)); });
+        if (have_ids) walk([&](int k) -> Word { return code_at(s_ids[k]); });
+        else walk([&](int k) -> Word { return code_at((uint32_t)clamp_idx(indices[e0 + k], a.N)); });
         const int deg = e - b;
         if (deg > 1) {
           const float d = (float)deg;
@@ -1284,8 +1300,7 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
       if (staged) {
         walk([&](int k) -> uint32_t {
           const unsigned char* q = s_codes + k * a.pitch + first;
-          if constexpr (GB == 4) return *reinterpret_cast<const uint32_t*>(q);
-          else if constexpr (GB == 2) return *reinterpret_cast<const uint16_t*>(q);
+          if constexpr (GB == 2) return *reinterpret_cast<const uint16_t*>(q);
           else return (uint32_t)*q;
         });
       } else if (have_ids) {
@@ -1444,9 +1459,6 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
                            a.R > 0 ? (double)a.E / (double)a.R : 0.0) ? 1 : 0;
   const size_t lut_bytes = AFFINE ? 0 : (size_t)(((a.num_codebooks << BITS) + 3) & ~3) * 4;
   const double avg_deg = a.R > 0 ? (double)a.E / (double)a.R : 1.0;
-  const bool wide = DEAL && BITS == 1;   // items of eight columns: a code byte
-  a.items_per_row = (int)ceil_div(a.feat_dim, wide ? 8 : 4);
-  a.item_magic = (uint32_t)(((1ull << 32) + a.items_per_row - 1) / a.items_per_row);   // items < 64 * 1024: exact
   const double dg = avg_deg > 0.5 ? avg_deg : 0.5;
   int cap = (int)((20 * 1024) / (a.pitch + 4));
   cap = cap > 2 * TB ? 2 * TB : cap;
@@ -1471,11 +1483,21 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
   // (250000 x 100, 2 bit 31 / 36, 4 bit 35 / 38), level to a tenth behind at 10 edges per row (250000 x 128, 2 bit 64 / 61,
   // 4 bit 71 / 68; 100000 x 256, 4 bit 53 / 47).
   const bool direct = DEAL && (BITS == 1 || BITS == 8 || a.pitch > 128 || (int)(8.0 * dg * 1.1) + 8 > a.edge_cap);
+  // Items of eight columns where the codes are read directly, of four where they are staged: half the loads and stores
+  // per value, each twice as wide, and half the row bookkeeping (four / eight, us: 8 bit, 3 edges per row, 312500 x 128
+  // 54 / 47, 10 per row with power-law degrees 312500 x 128 46 / 42, 3 edges per row 66666 x 602 76 / 68; 4 bit 67 / 59;
+  // 2 bit 62 / 55; short launches of 1000 columns 21 / 17; narrow rows level).  Staged rows have their loads behind them,
+  // and fewer items leave lanes idle there: 25 edges per row, 4 bit, 117000 x 128 72 / 81, 2 bit, 150000 x 100 65 / 68.
+  const bool wide = direct;
+  a.items_per_row = (int)ceil_div(a.feat_dim, wide ? 8 : 4);
+  // item / items_per_row as a high product, exact for items < 64 * 1024: rows of eight columns are one item of eight, and
+  // 2^32 / 1 has no room in the word, so the wide form takes 2^31 / items_per_row and doubles the item
+  a.item_magic = (uint32_t)(((wide ? 1ull << 31 : 1ull << 32) + a.items_per_row - 1) / a.items_per_row);
   if (direct) {
-    // about two rounds of items per thread for eight columns, four for four; at most 480 edges in a block of more
-    // than eight rows, so that long rows spread over the chip
+    // about two rounds of items per thread; at most 480 edges in a block of more than eight rows, so that long rows
+    // spread over the chip
     a.edge_cap = 0;
-    rb = ((wide ? 600 : 1024) / a.items_per_row + 4) / 8 * 8;
+    rb = (600 / a.items_per_row + 4) / 8 * 8;
     const int few = (int)(480.0 / dg) / 8 * 8;
     rb = rb > few ? few : rb;
   }
@@ -1499,7 +1521,7 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
     if (direct) a.id_cap = need < 2048 ? need : 2048;
     else a.id_cap = a.edge_cap = need < a.edge_cap ? need : a.edge_cap;
   }
-  const size_t lds = (wide ? kSignTable : 0) + lut_bytes + (size_t)(rb + 4) * 4 + 64 + (size_t)rb * 4 + (size_t)a.id_cap * 4 +
+  const size_t lds = (wide && BITS == 1 ? kSignTable : 0) + lut_bytes + (size_t)(rb + 4) * 4 + 64 + (size_t)rb * 4 + (size_t)a.id_cap * 4 +
                      (size_t)a.edge_cap * a.pitch + 16;
   const int64_t grid = ceil_div(a.R, rb);
   if (grid > 0x7fffffffll) return fail(F2CGT_E_UNSUPPORTED, "%s: too many row blocks", what);
@@ -1508,18 +1530,27 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
                 a.id_cap);
     return 0;
   }
-  constexpr bool STORE_FIXED = BITS >= 4 || (DEAL && BITS == 1);   // the store kind is always fixed when the kernel is chosen
-  const int half = (a.feat_dim % 4 == 0 && !STORE_FIXED) ? 0 : (a.nt_out ? 2 : 1);
+  // the store kind is fixed when the kernel is chosen, but for 1- and 2-bit rows of whole groups of four columns
+  const int half = (BITS <= 2 && !wide && a.feat_dim % 4 == 0) ? 0 : (a.nt_out ? 2 : 1);
 #define F2CGT_ROWS_GO(I, H, N)                                                   \
   sq_rows_kernel<BITS, AFFINE, I, TB, H, N><<<(unsigned)grid, TB, lds, st>>>(    \
       a, static_cast<const I*>(indptr), static_cast<const I*>(indices), out)
 #define F2CGT_ROWS_IDX(I)                                                        \
   do {                                                                           \
-    if constexpr (!STORE_FIXED) {                                                \
-      if (half == 0) F2CGT_ROWS_GO(I, 0, DEAL ? 4 : 0);                          \
+    if constexpr (DEAL) {                                                        \
+      if (wide) {                                                                \
+        if (half == 1) F2CGT_ROWS_GO(I, 1, 8);                                   \
+        else F2CGT_ROWS_GO(I, 2, 8);                                             \
+        break;                                                                   \
+      }                                                                          \
     }                                                                            \
-    if (half == 1) F2CGT_ROWS_GO(I, 1, DEAL ? (BITS == 1 ? 8 : 4) : 0);          \
-    else if (half == 2) F2CGT_ROWS_GO(I, 2, DEAL ? (BITS == 1 ? 8 : 4) : 0);     \
+    if constexpr (!DEAL || BITS == 2 || BITS == 4) {   /* 1 and 8 bits: always direct */ \
+      if constexpr (BITS <= 2) {                                                 \
+        if (half == 0) F2CGT_ROWS_GO(I, 0, DEAL ? 4 : 0);                        \
+      }                                                                          \
+      if (half == 1) F2CGT_ROWS_GO(I, 1, DEAL ? 4 : 0);                          \
+      else if (half == 2) F2CGT_ROWS_GO(I, 2, DEAL ? 4 : 0);                     \
+    }                                                                            \
   } while (0)
   if (idx_dtype == F2CGT_DT_I32) F2CGT_ROWS_IDX(int32_t);
   else F2CGT_ROWS_IDX(int64_t);
