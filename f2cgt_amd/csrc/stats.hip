@@ -10,15 +10,15 @@
 // and third pass), and no counter is shared between workgroups: the hot bins of a normal distribution lie in a dozen
 // cache lines, on which device-wide atomics of 256 workgroups would queue up.
 //
-// What bounds it: two reads of the sample (17 us each at 120 000 x 100 values, 2.9 TB/s through the row list; the first is
-// as long on its LDS counters as on its loads), the sums between the passes (4 us each) and the third pass, which reads
-// what the second kept and takes 5 us (17 with the sample read again).  The codebook is made by the last workgroup of the
-// last sum, so that the encoder can follow at once, and the ids' check is on the host as soon as the first pass is done, so
-// that a caller does not wait for the rest: the six launches take 52 us (seven 56; four rows in flight without the ids of the
-// next 66; the host 195 ms on a copy of the sample, np.percentile), a sq_compress call among others 70 (90 with a wait for
-// its end, 130 with the codebook made on the host), of which the encoder is 15.  100 000 x 602 values 598 -> 445;
-// tables on which a workgroup has to read its rows again are no slower than before (all values equal 438 -> 412, 80 %
-// zeros 253 -> 219).
+// What bounds it: one read of the sample (15 us at 120 000 x 100 values, 3.2 TB/s through the row list, as long on its LDS
+// counters and sums as on its loads; 22 with the values that it keeps for the second pass), the sums between the passes
+// (4 us each) and two passes over what was kept, 7 and 5 us (17 us each with the sample read again).  The codebook is made by
+// the last workgroup of the last sum, so that the encoder can follow at once, and the ids' check is on the host as soon as
+// the first pass is done, so that a caller does not wait for the rest: the six launches take 49 us (52 with two reads of the
+// sample; three 66; the host 195 ms on a copy of the sample, np.percentile).  100 000 x 602 values 151 -> 101 us, 60 000 x 1030
+// 203 -> 130, 1 000 000 x 128 238 -> 151 (with two reads -> with one).  Tables on which a workgroup has to read its rows again
+// are 0 to 6 % slower for it (120 000 x 100: all values equal 369 -> 377, 80 % zeros 180 -> 188, rows of very different lengths
+// 52 -> 55).
 #include "common.hpp"
 
 namespace f2cgt {
@@ -29,8 +29,11 @@ constexpr int kBins = 4096;          // counters of a pass: 4096, 4 x 1024 or 4 
 constexpr int kReplicas = 4;         // copies of the first pass's counters in LDS, by lane: its hot bins are few
 constexpr int kMaxBlocks = 256;      // workgroups per pass over all slices (one per CU)
 constexpr int kStatWaves = kStatThreads / kWave;
-constexpr int kKept = 512;           // values a wave of the second pass can hand to the third
-constexpr int kKeepBlocks = 1024;    // more workgroups than that in all hand over none (32 KB of workspace each)
+constexpr int kKept = 1024;          // values a wave of a pass can hand to the next one
+constexpr int kRoomBlocks = 256;     // more workgroups than that in all hand over half as many per wave,
+constexpr int kKeepBlocks = 1024;    // and more than that none (32 KB of workspace each)
+
+constexpr int kInFlight = 8;         // rows that a lane reads at a time
 
 constexpr uint32_t kSawNan = 1u, kSawBadRow = 2u;   // a NaN among the values; a row id outside the table
 
@@ -53,8 +56,12 @@ struct StatArgs {
   double* sums;                      // [n_slices][blocks]
   uint32_t* flags;                   // [n_slices][blocks]: kSawNan, kSawBadRow
   int keep;                          // kKept, or 0 where there is no room for them
-  uint32_t* kept;                    // [n_slices][blocks][kStatWaves][keep]: values that share the first digit of a wanted rank
+  int ahead;                         // the first pass keeps values for the second
+  // [n_slices][blocks][kStatWaves][keep]: the values of a workgroup's windows, then those that share the first digit of a
+  // wanted rank
+  uint32_t* kept;
   uint32_t* n_kept;                  // [n_slices][blocks][kStatWaves]: how many; more than `keep`: not all of them are there
+  uint32_t* windows;                 // [n_slices][blocks][2]: the digits between these two are not kept
   double* out;                       // [n_slices][6]
   uint32_t* arrived;                 // [n_slices]: workgroups of the last sum that are done with a slice
   int32_t* bad;                      // host memory: set by the first pass where a row id lies outside the table; or null
@@ -64,8 +71,9 @@ struct StatArgs {
 
 // Finds, in `groups` runs of kBins / groups counters, the counter that holds rank[t] (run t, or the only run), for all
 // four ranks, by the whole workgroup: digit[t] is the counter's place in its run and rank[t] becomes the rank inside it.
-template <int GROUPS, int USED>
-__device__ __forceinline__ void find_digits(const uint32_t* __restrict__ hist, const uint64_t (&rank)[4],
+// counter(i): the i-th one.
+template <int GROUPS, int USED, typename Counter>
+__device__ __forceinline__ void find_digits(Counter counter, const uint64_t (&rank)[4],
                                             uint64_t* s_scan, uint32_t* s_digit, uint64_t* s_rest) {
   constexpr int PER = USED / (kStatThreads / GROUPS);   // counters per thread
   static_assert(PER >= 1, "a thread owns at least one counter");
@@ -75,7 +83,7 @@ __device__ __forceinline__ void find_digits(const uint32_t* __restrict__ hist, c
   uint64_t own = 0;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    c[i] = hist[group * USED + at * PER + i];
+    c[i] = counter(group * USED + at * PER + i);
     own += c[i];
   }
   uint64_t run = own;                                   // inclusive sum over the wave
@@ -118,17 +126,18 @@ __device__ __forceinline__ void wanted_ranks(const StatArgs& a, int slice, uint6
 template <int PASS>
 __device__ __forceinline__ void known_digits(const StatArgs& a, int slice, uint64_t* s_scan, uint32_t* s_digit,
                                              uint64_t* s_rest, uint32_t (&prefix)[4], uint64_t (&rank)[4]) {
-  const uint32_t* hist = a.hist + (int64_t)slice * kBins;
+  const uint32_t* __restrict__ hist = a.hist + (int64_t)slice * kBins;
+  auto counter = [&](int i) { return hist[i]; };
   if (PASS == 1) {
     wanted_ranks(a, slice, rank);
-    find_digits<1, 4096>(hist, rank, s_scan, s_digit, s_rest);
+    find_digits<1, 4096>(counter, rank, s_scan, s_digit, s_rest);
 #pragma unroll
     for (int k = 0; k < 4; ++k) prefix[k] = s_digit[k];
   } else {
     const StatState& st = a.state[(PASS - 2) * a.n_slices + slice];
 #pragma unroll
     for (int k = 0; k < 4; ++k) rank[k] = st.rank[k];
-    find_digits<4, PASS == 2 ? 1024 : 512>(hist, rank, s_scan, s_digit, s_rest);
+    find_digits<4, PASS == 2 ? 1024 : 512>(counter, rank, s_scan, s_digit, s_rest);
 #pragma unroll
     for (int k = 0; k < 4; ++k) prefix[k] = (st.prefix[k] << (PASS == 2 ? 10 : 9)) | s_digit[k];
   }
@@ -139,9 +148,15 @@ __device__ __forceinline__ void known_digits(const StatArgs& a, int slice, uint6
 // One pass over the sample.  A thread keeps its place in the row (a V-wide column group) and walks rows; eight rows are in
 // flight at a time, and the ids of the eight after them.
 //
-// The second pass meets all the values that the third will count, those that share the first digit of a wanted rank: one in
-// a few hundred of a feature table.  Its waves keep them, and the third pass reads these instead of the sample.  A
-// workgroup with a wave that met more than `keep` of them (a table of few different values) reads its rows again.
+// A later pass needs only the values that share the digits found so far with a wanted rank, one in a few hundred of a
+// feature table, so the pass before keeps them, wave by wave, and the sample is read once.
+//   The second pass knows the first digits and keeps what the third will count.
+//   The first pass does not know them yet.  Its workgroups take the first rows that they count for a sample of the sample:
+//   a wanted rank lies, with six standard deviations to either side, between two of its ranks, and the values between these
+//   two (a window of first digits; one or two of a hundred values at the percentiles 0.5 and 99.5) are kept.  The second
+//   pass holds the true digits against the windows.
+// A workgroup whose windows missed a digit (rows in an order that its first ones say nothing about), or with a wave that
+// met more than `keep` of the values (a table of few different values), reads its rows again.
 template <int PASS, int V>
 __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   __shared__ __align__(16) uint32_t s_hist[PASS == 0 ? kBins * kReplicas : kBins];
@@ -150,7 +165,7 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   __shared__ uint64_t s_rest[4];
   __shared__ double s_sum[kStatThreads / kWave];
   __shared__ uint32_t s_flags;
-  __shared__ uint32_t s_kept[PASS == 1 ? kStatWaves * kKept : 1];
+  __shared__ uint32_t s_kept[PASS < 2 ? kStatWaves * kKept : 1];
   __shared__ uint32_t s_n_kept[kStatWaves];
   const int t = threadIdx.x, slice = blockIdx.y, wave = t / kWave;
   constexpr int LDS_BINS = PASS == 0 ? kBins * kReplicas : kBins;
@@ -207,22 +222,122 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   };
   const int64_t place = (int64_t)slice * a.blocks + blockIdx.x;
   bool read_rows = true;
-  if constexpr (PASS == 2) {
+  if (PASS == 2 || (PASS == 1 && a.ahead)) {
     uint32_t most = 0;
 #pragma unroll
     for (int w = 0; w < kStatWaves; ++w) {
       const uint32_t n = a.n_kept[place * kStatWaves + w];
       most = n > most ? n : most;
     }
-    if (most <= (uint32_t)a.keep) {
+    bool whole = most <= (uint32_t)a.keep;
+    if (PASS == 1) {
+      const uint32_t* between = a.windows + place * 2;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) whole &= prefix[k] <= between[0] || prefix[k] >= between[1];
+    }
+    if (whole) {
       read_rows = false;
       const uint32_t n = a.n_kept[place * kStatWaves + wave];
       const uint32_t* kept = a.kept + (place * kStatWaves + wave) * a.keep;
       for (uint32_t i = t & (kWave - 1); i < n; i += kWave) take(__uint_as_float(kept[i]));
     }
   }
+  constexpr int U = kInFlight;
+  if constexpr (PASS == 0) {
+    if (a.ahead) {
+      // All lanes walk together, as many rounds as the first row has; rows that a lane has not are its first, and not counted.
+      read_rows = false;
+      const int64_t base = (int64_t)blockIdx.x * rpp;
+      const int64_t first = base + r0 < a.m ? base + r0 : 0;
+      const int rounds = base < a.m ? (int)((a.m - base + step * U - 1) / (step * U)) : 0;
+      int mine = r0 < rpp && base + r0 < a.m ? (int)((a.m - base - r0 + step - 1) / step) : 0;   // rows of this lane left
+      int64_t id[U], row = base + r0;
+      auto row_ids = [&](int have) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t ru = u < have ? row + u * step : first;
+          id[u] = a.rows != nullptr ? a.rows[ru] : ru;
+        }
+      };
+      uint32_t from = 0u, span = 0x80000000u, kept = 0u;   // magnitudes that are not kept; what the wave has kept
+      auto keep = [&](float v, bool counts) {
+        const uint32_t mag = __float_as_uint(v) & 0x7fffffffu;
+        if (kept > (uint32_t)a.keep) return;                // (the same for the wave)
+        const bool in = counts && mag - from >= span;
+        const uint64_t all = __ballot(in);
+        if (all == 0) return;
+        const uint32_t at = kept + __builtin_amdgcn_mbcnt_hi((uint32_t)(all >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)all, 0u));
+        if (in && at < (uint32_t)a.keep) s_kept[wave * kKept + at] = mag;
+        kept += (uint32_t)__popcll(all);
+      };
+      row_ids(mine);
+      for (int round = 0; round < rounds; ++round) {
+        float v[U][V];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t want = id[u] < 0 ? id[u] + a.num_rows : id[u];
+          const int64_t at = clamp_idx(want, a.num_rows);
+          flags |= at != want ? kSawBadRow : 0u;
+          const float* p = a.x + at * a.ld + col0 + c0 * V;
+          if constexpr (V == 4) {
+            const float4 q = *reinterpret_cast<const float4*>(p);
+            v[u][0] = q.x; v[u][1] = q.y; v[u][2] = q.z; v[u][3] = q.w;
+          } else if constexpr (V == 2) {
+            const float2 q = *reinterpret_cast<const float2*>(p);
+            v[u][0] = q.x; v[u][1] = q.y;
+          } else {
+            v[u][0] = *p;
+          }
+        }
+        row += step * U;
+        if (round + 1 < rounds) row_ids(mine - U);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (u < mine)
+#pragma unroll
+            for (int i = 0; i < V; ++i) take(v[u][i]);
+        if (round == 0) {
+          int64_t rows = 0;
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int64_t left = a.m - (base + u * step);
+            rows += left < 0 ? 0 : left < rpp ? left : rpp;
+          }
+          const float n = (float)(rows * width), all = (float)a.m * (float)width;
+          uint64_t rank[4], edge[4] = {0u, 0u, (uint64_t)n - 1u, 0u};
+          wanted_ranks(a, slice, rank);
+          uint64_t low = rank[0] > rank[1] ? rank[0] : rank[1], high = rank[2] < rank[3] ? rank[2] : rank[3];
+          const float p = (float)low / all, q = (float)high / all;
+          const float below = n * p + 6.f * __builtin_amdgcn_sqrtf(n * p * (1.f - p)) + 4.f;
+          const float above = n * q - 6.f * __builtin_amdgcn_sqrtf(n * q * (1.f - q)) - 4.f;
+          edge[0] = below < n - 1.f ? (uint64_t)below : (uint64_t)n - 1u;
+          edge[1] = above > 0.f ? (uint64_t)above : 0u;
+          __syncthreads();
+          auto counter = [&](int i) {
+            const uint4 c = *reinterpret_cast<const uint4*>(s_hist + i * kReplicas);
+            return c.x + c.y + c.z + c.w;
+          };
+          find_digits<1, 4096>(counter, edge, s_scan, s_digit, s_rest);
+          // kept: digits up to the one that `below` of the sample's values reach, and from the one that `above` do
+          const uint32_t lo = __builtin_amdgcn_readfirstlane(s_digit[0]), hi = __builtin_amdgcn_readfirstlane(s_digit[1]);
+          from = (lo + 1) << 19;
+          span = hi > lo ? (hi - lo - 1) << 19 : 0u;
+          if (t == 0) {
+            a.windows[place * 2] = lo;
+            a.windows[place * 2 + 1] = hi;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int i = 0; i < V; ++i) keep(v[u][i], u < mine);
+        mine -= U;
+      }
+      if ((t & (kWave - 1)) == 0) s_n_kept[wave] = kept;
+      if (rounds == 0 && t < 2) a.windows[place * 2 + t] = t == 0 ? kBins : 0u;   // nothing that could be left out
+    }
+  }
   if (read_rows && r0 < rpp) {
-    constexpr int U = 8;
     int64_t id[U];
     // the rows r, r + step, ...: a place beyond the sample takes row r again, which the sample has
     auto row_ids = [&](int64_t r, int64_t (&id)[U]) {
@@ -274,7 +389,7 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
     if ((t & (kWave - 1)) == 0) s_sum[t / kWave] = sum;
   }
   __syncthreads();
-  if constexpr (PASS == 1) {
+  if (PASS == 1 || (PASS == 0 && a.ahead)) {
     const uint32_t n = s_n_kept[wave];
     if ((t & (kWave - 1)) == 0) a.n_kept[place * kStatWaves + wave] = n;
     uint32_t* kept = a.kept + (place * kStatWaves + wave) * a.keep;
@@ -402,9 +517,27 @@ int stat_blocks(int64_t m, int64_t cols, int64_t slice, int64_t n_slices) {
 
 int64_t round256(int64_t v) { return (v + 255) / 256 * 256; }
 
-int stat_keep(int64_t blocks, int64_t n_slices) { return n_slices * blocks <= kKeepBlocks ? kKept : 0; }
+int stat_keep(int64_t blocks, int64_t n_slices) {
+  return n_slices * blocks <= kRoomBlocks ? kKept : n_slices * blocks <= kKeepBlocks ? kKept / 2 : 0;
+}
 
-struct StatLayout { int64_t hist, state, sums, flags, kept, n_kept, arrived, total; };
+// Whether the first pass keeps values for the second: where they are expected to fit, with a lane's column group the same in
+// every row (the first rows are a sample of all columns then), and from three million values on.  Finding the window takes
+// the first pass 3 us, and a smaller sample is read as quickly again (10 000 x 128: 33 us, 35 with the window; 50 000 x 75
+// 56 and 48).
+bool stat_ahead(const StatArgs& a, int v) {
+  const int64_t width = a.slice, groups = width / v;
+  if (a.keep == 0 || groups > kStatThreads) return false;
+  const double all = (double)a.m * (double)width, own = all / a.blocks;              // values of a slice, of a workgroup
+  double n = (double)kInFlight * (double)(kStatThreads / groups) * (double)width;                  // of its first round
+  n = n < own ? n : own;
+  const double p = (double)(a.ranks[0] > a.ranks[1] ? a.ranks[0] : a.ranks[1]) / all;
+  const double q = (double)(a.ranks[2] < a.ranks[3] ? a.ranks[2] : a.ranks[3]) / all;
+  const double part = p + (6.0 * sqrt(n * p * (1.0 - p)) + 4.0) / n + 1.0 - q + (6.0 * sqrt(n * q * (1.0 - q)) + 4.0) / n + 0.005;
+  return a.m * a.cols >= 3000000 && 1.3 * part * own / kStatWaves <= (double)a.keep;
+}
+
+struct StatLayout { int64_t hist, state, sums, flags, kept, n_kept, arrived, windows, total; };
 StatLayout stat_layout(int64_t blocks, int64_t n_slices) {
   StatLayout l;
   l.hist = round256(n_slices * blocks * kBins * 4);
@@ -414,7 +547,8 @@ StatLayout stat_layout(int64_t blocks, int64_t n_slices) {
   l.kept = l.flags + round256(n_slices * blocks * 4);
   l.n_kept = l.kept + round256(n_slices * blocks * kStatWaves * stat_keep(blocks, n_slices) * 4);
   l.arrived = l.n_kept + round256(n_slices * blocks * kStatWaves * 4);
-  l.total = l.arrived + round256(n_slices * 4);
+  l.windows = l.arrived + round256(n_slices * 4);
+  l.total = l.windows + round256(n_slices * blocks * 2 * 4);
   return l;
 }
 
@@ -484,6 +618,7 @@ int order_stats(const char* what, const float* x, int64_t ld, const int64_t* row
   a.kept = reinterpret_cast<uint32_t*>(ws + l.kept);
   a.n_kept = reinterpret_cast<uint32_t*>(ws + l.n_kept);
   a.arrived = reinterpret_cast<uint32_t*>(ws + l.arrived);
+  a.windows = reinterpret_cast<uint32_t*>(ws + l.windows);
   a.bad = bad;
   a.out = out;
   a.books = books;
@@ -496,6 +631,7 @@ int order_stats(const char* what, const float* x, int64_t ld, const int64_t* row
   };
   hipStream_t st = as_stream(stream);
   hipEvent_t ev = static_cast<hipEvent_t>(checked);
+  a.ahead = stat_ahead(a, fits(4) ? 4 : fits(2) ? 2 : 1) ? 1 : 0;
   const hipError_t e = fits(4) ? stat_launch<4>(a, ev, st) : fits(2) ? stat_launch<2>(a, ev, st) : stat_launch<1>(a, ev, st);
   if (e != hipSuccess) return fail((int)e, "%s: cannot record the event: %s", what, hipGetErrorString(e));
   return launch_status(what);
