@@ -2,23 +2,24 @@
 // is made of (examples/process_compress.py:45-68: two percentiles and the mean of the absolute values of a slice).
 //
 // The statistics are exact: the requested ranks are found by a radix selection on the bit pattern of |x| (for
-// non-negative floats the order of the values is the order of the bit patterns), three digits of 12, 10 and 9 bits, each
-// one pass over the sample.  A pass counts the next digit of the values that share the digits found so far with a
-// wanted rank; the counts stay in LDS and are written once per workgroup, a small kernel adds the workgroups' counts, and
-// the next pass finds the digit from the sums in its prologue.  Nothing is sorted, nothing is copied (the rows are read
-// through the sample's row list each time; a sample that fits the 256 MB last-level cache comes from there in the second
-// and third pass), and no counter is shared between workgroups: the hot bins of a normal distribution lie in a dozen
-// cache lines, on which device-wide atomics of 256 workgroups would queue up.
+// non-negative floats the order of the values is the order of the bit patterns), three digits of 12, 10 and 9 bits.  A pass
+// counts the next digit of the values that share the digits found so far with a wanted rank, in LDS, and the next pass finds
+// the digit from the sums in its prologue.  Nothing is sorted and nothing is copied but the few values that a pass keeps for
+// the next one (see stat_pass_kernel); the rows are read through the sample's row list.
+//   The first pass shares no counter between workgroups: the hot bins of a normal distribution lie in a dozen cache lines, on
+// which device-wide atomics of 256 workgroups would queue up.  Each writes its counts and a small kernel adds them.  What the
+// second and the third pass count are a few hundred values a workgroup, which go to the sums by atomics as they are.
 //
 // What bounds it: one read of the sample (15 us at 120 000 x 100 values, 3.2 TB/s through the row list, as long on its LDS
-// counters and sums as on its loads; 22 with the values that it keeps for the second pass), the sums between the passes
-// (4 us each) and two passes over what was kept, 7 and 5 us (17 us each with the sample read again).  The codebook is made by
-// the last workgroup of the last sum, so that the encoder can follow at once, and the ids' check is on the host as soon as
-// the first pass is done, so that a caller does not wait for the rest: the six launches take 49 us (52 with two reads of the
-// sample; three 66; the host 195 ms on a copy of the sample, np.percentile).  100 000 x 602 values 151 -> 101 us, 60 000 x 1030
-// 203 -> 130, 1 000 000 x 128 238 -> 151 (with two reads -> with one).  Tables on which a workgroup has to read its rows again
-// are 0 to 6 % slower for it (120 000 x 100: all values equal 369 -> 377, 80 % zeros 180 -> 188, rows of very different lengths
-// 52 -> 55).
+// counters and sums as on its loads; 22 with the values that it keeps for the second pass), the sum behind it (4 us) and two
+// passes over what was kept, 9 and 10 us, the last with the outputs.  The codebook is made by the last workgroup of the last
+// pass, so that the encoder can follow at once, and the ids' check is on the host as soon as the first pass is done, so that a
+// caller does not wait for the rest.  The four launches take 44 us; six, with sums of all counters behind the second and third
+// pass too, 49, with a second read of the sample 52, a third 66 (the host 195 ms on a copy of the sample, np.percentile).
+// Likewise 100 000 x 602 values 151 -> 101 -> 96 us (second read saved, sums saved), 60 000 x 1030 203 -> 130 -> 125, 1 000 000 x 128
+// 238 -> 151 -> 146, 1000 x 64 31 -> 27.  Tables on which a workgroup has to read its rows again lose up to 6 % by what it kept in
+// vain and gain the sums (120 000 x 100: all values equal 369 us before and after, 80 % zeros 180, rows of very different
+// lengths 52 -> 48).
 #include "common.hpp"
 
 namespace f2cgt {
@@ -37,7 +38,7 @@ constexpr int kInFlight = 8;         // rows that a lane reads at a time
 
 constexpr uint32_t kSawNan = 1u, kSawBadRow = 2u;   // a NaN among the values; a row id outside the table
 
-struct StatState {                   // per slice, written by the first workgroup of a pass for the passes after it
+struct StatState {                   // per slice, written by the first workgroup of the second pass for the third
   uint32_t prefix[4];                // digits found so far of the value at each wanted rank
   uint32_t pad[4];
   uint64_t rank[4];                  // its rank among the values that share them
@@ -50,9 +51,9 @@ struct StatArgs {
   int cols, slice, n_slices;
   int blocks;                        // workgroups per slice
   uint64_t ranks[8];                 // wanted ranks of a full slice, and of the last one
-  uint32_t* partial;                 // [n_slices][blocks][kBins]
-  uint32_t* hist;                    // [n_slices][kBins]
-  StatState* state;                  // [2][n_slices]: after the first and the second digit
+  uint32_t* partial;                 // [n_slices][blocks][kBins]: of the first pass
+  uint32_t* hist;                    // [3][n_slices][kBins]: the passes' counters
+  StatState* state;                  // [n_slices]: after the first digit
   double* sums;                      // [n_slices][blocks]
   uint32_t* flags;                   // [n_slices][blocks]: kSawNan, kSawBadRow
   int keep;                          // kKept, or 0 where there is no room for them
@@ -63,7 +64,7 @@ struct StatArgs {
   uint32_t* n_kept;                  // [n_slices][blocks][kStatWaves]: how many; more than `keep`: not all of them are there
   uint32_t* windows;                 // [n_slices][blocks][2]: the digits between these two are not kept
   double* out;                       // [n_slices][6]
-  uint32_t* arrived;                 // [n_slices]: workgroups of the last sum that are done with a slice
+  uint32_t* arrived;                 // [n_slices]: workgroups of the last pass that are done with a slice
   int32_t* bad;                      // host memory: set by the first pass where a row id lies outside the table; or null
   float* books;                      // [n_slices][5], or null
   float weights[4];                  // lower and upper percentile of a slice, and of the last one: where between its ranks
@@ -126,7 +127,7 @@ __device__ __forceinline__ void wanted_ranks(const StatArgs& a, int slice, uint6
 template <int PASS>
 __device__ __forceinline__ void known_digits(const StatArgs& a, int slice, uint64_t* s_scan, uint32_t* s_digit,
                                              uint64_t* s_rest, uint32_t (&prefix)[4], uint64_t (&rank)[4]) {
-  const uint32_t* __restrict__ hist = a.hist + (int64_t)slice * kBins;
+  const uint32_t* __restrict__ hist = a.hist + ((int64_t)(PASS - 1) * a.n_slices + slice) * kBins;
   auto counter = [&](int i) { return hist[i]; };
   if (PASS == 1) {
     wanted_ranks(a, slice, rank);
@@ -134,15 +135,74 @@ __device__ __forceinline__ void known_digits(const StatArgs& a, int slice, uint6
 #pragma unroll
     for (int k = 0; k < 4; ++k) prefix[k] = s_digit[k];
   } else {
-    const StatState& st = a.state[(PASS - 2) * a.n_slices + slice];
+    const StatState& st = a.state[slice];
 #pragma unroll
     for (int k = 0; k < 4; ++k) rank[k] = st.rank[k];
-    find_digits<4, PASS == 2 ? 1024 : 512>(counter, rank, s_scan, s_digit, s_rest);
+    find_digits<4, 1024>(counter, rank, s_scan, s_digit, s_rest);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) prefix[k] = (st.prefix[k] << (PASS == 2 ? 10 : 9)) | s_digit[k];
+    for (int k = 0; k < 4; ++k) prefix[k] = (st.prefix[k] << 10) | s_digit[k];
   }
 #pragma unroll
   for (int k = 0; k < 4; ++k) rank[k] = s_rest[k];
+}
+
+// The quantiser's codebook of a slice (fmin, fmax, emin, emax, mean) from its statistics: percentiles interpolated in
+// float32 from the nearer rank, floored at 1e-5 and 2e-5, their log2 correctly rounded, and the mean, lifted by 0.1 where
+// it is below 0.1 (examples/process_compress.py:45-68).  A NaN stays one.
+__device__ void sq_codebook(const StatArgs& a, int slice, const float (&at)[4], double total, uint32_t flags) {
+  const bool last = slice == a.n_slices - 1;
+  auto between = [](float below, float above, float w) {
+    const float gap = above - below;
+    return w < 0.5f ? below + gap * w : above - gap * (1.f - w);
+  };
+  float lo = between(at[0], at[1], a.weights[last ? 2 : 0]), hi = between(at[2], at[3], a.weights[last ? 3 : 1]);
+  if (flags & kSawNan) lo = hi = __uint_as_float(0x7fc00000u);
+  const float floor = 1e-5f;
+  lo = floor > lo ? floor : lo;
+  hi = 2e-5f > hi ? 2e-5f : hi;
+  const int64_t width = last ? a.cols - (int64_t)slice * a.slice : a.slice;
+  float level = (float)(total / (double)(a.m * width));
+  level = level < 0.1f ? level + 0.1f : level;
+  float* book = a.books + slice * 5;
+  book[0] = lo;
+  book[1] = hi;
+  book[2] = log2_cr(lo);
+  book[3] = log2_cr(hi) + floor;
+  book[4] = level;
+}
+
+// Last digit, and the outputs of a slice: the values at the four ranks, the sum, the flags; by one workgroup.
+__device__ void stat_finish(const StatArgs& a, int slice, uint64_t* s_scan, uint32_t* s_digit, uint64_t* s_rest,
+                            uint32_t (&prefix)[4], const uint64_t (&rank)[4]) {
+  const int t = threadIdx.x;
+  uint32_t* hist = a.hist + ((int64_t)2 * a.n_slices + slice) * kBins;
+  find_digits<4, 512>([&](int i) { return __hip_atomic_load(hist + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }, rank,
+                      s_scan, s_digit, s_rest);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) prefix[k] = (prefix[k] << 9) | s_digit[k];
+  if (t < 4) a.out[slice * 6 + t] = (double)__uint_as_float(t == 0 ? prefix[0] : t == 1 ? prefix[1] : t == 2 ? prefix[2] : prefix[3]);
+  if (t >= kWave && t < 2 * kWave) {                    // the second wave
+    double total = 0.0;
+    uint32_t flags = 0;
+    for (int b = t - kWave; b < a.blocks; b += kWave) {
+      total += a.sums[(int64_t)slice * a.blocks + b];
+      flags |= a.flags[(int64_t)slice * a.blocks + b];
+    }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+      total += __shfl_xor(total, off);
+      flags |= __shfl_xor(flags, off);
+    }
+    if (t == kWave) {
+      a.out[slice * 6 + 4] = total;
+      a.out[slice * 6 + 5] = (double)flags;
+      if (a.books != nullptr) {
+        const float at[4] = {__uint_as_float(prefix[0]), __uint_as_float(prefix[1]), __uint_as_float(prefix[2]),
+                             __uint_as_float(prefix[3])};
+        sq_codebook(a, slice, at, total, flags);
+      }
+    }
+  }
 }
 
 // One pass over the sample.  A thread keeps its place in the row (a V-wide column group) and walks rows; eight rows are in
@@ -173,13 +233,13 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   if (t == 0) s_flags = 0u;
   if (t < kStatWaves) s_n_kept[t] = 0u;
   uint32_t prefix[4] = {0u, 0u, 0u, 0u};
+  uint64_t rank[4] = {0u, 0u, 0u, 0u};
   if constexpr (PASS > 0) {
-    uint64_t rank[4];
     known_digits<PASS>(a, slice, s_scan, s_digit, s_rest, prefix, rank);
 #pragma unroll
     for (int k = 0; k < 4; ++k) prefix[k] = __builtin_amdgcn_readfirstlane(prefix[k]);
-    if (blockIdx.x == 0 && t == 0) {
-      StatState& st = a.state[(PASS - 1) * a.n_slices + slice];
+    if (PASS == 1 && blockIdx.x == 0 && t == 0) {
+      StatState& st = a.state[slice];
 #pragma unroll
       for (int k = 0; k < 4; ++k) { st.prefix[k] = prefix[k]; st.rank[k] = rank[k]; }
     }
@@ -304,7 +364,7 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
             rows += left < 0 ? 0 : left < rpp ? left : rpp;
           }
           const float n = (float)(rows * width), all = (float)a.m * (float)width;
-          uint64_t rank[4], edge[4] = {0u, 0u, (uint64_t)n - 1u, 0u};
+          uint64_t edge[4] = {0u, 0u, (uint64_t)n - 1u, 0u};
           wanted_ranks(a, slice, rank);
           uint64_t low = rank[0] > rank[1] ? rank[0] : rank[1], high = rank[2] < rank[3] ? rank[2] : rank[3];
           const float p = (float)low / all, q = (float)high / all;
@@ -395,16 +455,35 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
     uint32_t* kept = a.kept + (place * kStatWaves + wave) * a.keep;
     for (uint32_t i = t & (kWave - 1); i < (n < (uint32_t)a.keep ? n : (uint32_t)a.keep); i += kWave) kept[i] = s_kept[wave * kKept + i];
   }
-  uint32_t* dst = a.partial + place * kBins;
-  for (int i = t; i < (PASS == 2 ? 2048 : kBins); i += kStatThreads) {
-    if constexpr (PASS == 0) {
+  if constexpr (PASS == 0) {
+    uint32_t* dst = a.partial + place * kBins;
+    for (int i = t; i < kBins; i += kStatThreads) {
       uint32_t c = 0;
 #pragma unroll
       for (int k = 0; k < kReplicas; ++k) c += s_hist[i * kReplicas + k];
       dst[i] = c;
-    } else {
-      dst[i] = s_hist[i];
     }
+    // the counters of the passes after this one
+    for (int i = blockIdx.x * kStatThreads + t; i < 2 * kBins; i += a.blocks * kStatThreads)
+      a.hist[((int64_t)(1 + i / kBins) * a.n_slices + slice) * kBins + i % kBins] = 0u;
+  } else {
+    // A few hundred values of a workgroup share the digits of a wanted rank: its counters go to the slice's one by one.
+    uint32_t* dst = a.hist + ((int64_t)PASS * a.n_slices + slice) * kBins;
+    for (int i = t; i < (PASS == 2 ? 2048 : kBins); i += kStatThreads) {
+      const uint32_t c = s_hist[i];
+      if (c != 0) __hip_atomic_fetch_add(dst + i, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if constexpr (PASS == 2) {
+    // The workgroup that finishes a slice goes on to its last digit and outputs, a launch less (3.8 us of 55).
+    __shared__ int s_last;
+    // Each wave's additions have reached the memory before the workgroup arrives, and nothing else that the last one reads
+    // was written in this launch: no cache has to be written back (as a fence of each wave, that took 65 us).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (t == 0) s_last = __hip_atomic_fetch_add(a.arrived + slice, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u;
+    __syncthreads();
+    if (s_last) stat_finish(a, slice, s_scan, s_digit, s_rest, prefix, rank);
   }
   if (PASS == 0 && t == 0) {
     if (blockIdx.x == 0) a.arrived[slice] = 0u;
@@ -416,66 +495,8 @@ __global__ __launch_bounds__(kStatThreads) void stat_pass_kernel(StatArgs a) {
   }
 }
 
-// The quantiser's codebook of a slice (fmin, fmax, emin, emax, mean) from its statistics: percentiles interpolated in
-// float32 from the nearer rank, floored at 1e-5 and 2e-5, their log2 correctly rounded, and the mean, lifted by 0.1 where
-// it is below 0.1 (examples/process_compress.py:45-68).  A NaN stays one.
-__device__ void sq_codebook(const StatArgs& a, int slice, const float (&at)[4], double total, uint32_t flags) {
-  const bool last = slice == a.n_slices - 1;
-  auto between = [](float below, float above, float w) {
-    const float gap = above - below;
-    return w < 0.5f ? below + gap * w : above - gap * (1.f - w);
-  };
-  float lo = between(at[0], at[1], a.weights[last ? 2 : 0]), hi = between(at[2], at[3], a.weights[last ? 3 : 1]);
-  if (flags & kSawNan) lo = hi = __uint_as_float(0x7fc00000u);
-  const float floor = 1e-5f;
-  lo = floor > lo ? floor : lo;
-  hi = 2e-5f > hi ? 2e-5f : hi;
-  const int64_t width = last ? a.cols - (int64_t)slice * a.slice : a.slice;
-  float level = (float)(total / (double)(a.m * width));
-  level = level < 0.1f ? level + 0.1f : level;
-  float* book = a.books + slice * 5;
-  book[0] = lo;
-  book[1] = hi;
-  book[2] = log2_cr(lo);
-  book[3] = log2_cr(hi) + floor;
-  book[4] = level;
-}
-
-// Last digit, and the outputs of a slice: the values at the four ranks, the sum, the flags; by one workgroup.
-__device__ void stat_finish(const StatArgs& a, int slice, uint64_t* s_scan, uint32_t* s_digit, uint64_t* s_rest) {
-  const int t = threadIdx.x;
-  uint32_t prefix[4];
-  uint64_t rank[4];
-  known_digits<3>(a, slice, s_scan, s_digit, s_rest, prefix, rank);
-  if (t < 4) a.out[slice * 6 + t] = (double)__uint_as_float(t == 0 ? prefix[0] : t == 1 ? prefix[1] : t == 2 ? prefix[2] : prefix[3]);
-  if (t >= kWave && t < 2 * kWave) {                    // the second wave
-    double total = 0.0;
-    uint32_t flags = 0;
-    for (int b = t - kWave; b < a.blocks; b += kWave) {
-      total += a.sums[(int64_t)slice * a.blocks + b];
-      flags |= a.flags[(int64_t)slice * a.blocks + b];
-    }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-      total += __shfl_xor(total, off);
-      flags |= __shfl_xor(flags, off);
-    }
-    if (t == kWave) {
-      a.out[slice * 6 + 4] = total;
-      a.out[slice * 6 + 5] = (double)flags;
-      if (a.books != nullptr) {
-        const float at[4] = {__uint_as_float(prefix[0]), __uint_as_float(prefix[1]), __uint_as_float(prefix[2]),
-                             __uint_as_float(prefix[3])};
-        sq_codebook(a, slice, at, total, flags);
-      }
-    }
-  }
-}
-
-// hist[bin] = sum of the workgroups' counts: a wave reads 64 neighbouring bins of every sixteenth workgroup, all its
+// The first pass's counts: hist[bin] = sum of the workgroups'.  A wave reads 64 neighbouring bins of every sixteenth workgroup, all its
 // reads in flight at once (with four waves to 64 bins, four rounds of reads each, the kernel took 9 us instead of 4).
-// LAST: the workgroup that finishes a slice goes on to its last digit and outputs, a launch less (3.8 us of 55).
-template <bool LAST>
 __global__ __launch_bounds__(kStatThreads) void stat_reduce_kernel(StatArgs a) {
   constexpr int WAVES = kStatThreads / kWave;
   __shared__ uint32_t s_part[WAVES][kWave];
@@ -491,18 +512,6 @@ __global__ __launch_bounds__(kStatThreads) void stat_reduce_kernel(StatArgs a) {
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) c += s_part[w][lane];
     a.hist[(int64_t)slice * kBins + bin] = c;
-  }
-  if constexpr (LAST) {
-    __shared__ uint64_t s_scan[kStatThreads / kWave];
-    __shared__ uint32_t s_digit[4];
-    __shared__ uint64_t s_rest[4];
-    __shared__ int s_last;
-    __syncthreads();
-    // release: the other workgroups' sums before their count; acquire: this one's reads of them behind it
-    if (threadIdx.x == 0)
-      s_last = __hip_atomic_fetch_add(a.arrived + slice, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1u;
-    __syncthreads();
-    if (s_last) stat_finish(a, slice, s_scan, s_digit, s_rest);
   }
 }
 
@@ -541,8 +550,8 @@ struct StatLayout { int64_t hist, state, sums, flags, kept, n_kept, arrived, win
 StatLayout stat_layout(int64_t blocks, int64_t n_slices) {
   StatLayout l;
   l.hist = round256(n_slices * blocks * kBins * 4);
-  l.state = l.hist + round256(n_slices * kBins * 4);
-  l.sums = l.state + round256(2 * n_slices * (int64_t)sizeof(StatState));
+  l.state = l.hist + round256(3 * n_slices * kBins * 4);
+  l.sums = l.state + round256(n_slices * (int64_t)sizeof(StatState));
   l.flags = l.sums + round256(n_slices * blocks * 8);
   l.kept = l.flags + round256(n_slices * blocks * 4);
   l.n_kept = l.kept + round256(n_slices * blocks * kStatWaves * stat_keep(blocks, n_slices) * 4);
@@ -556,14 +565,11 @@ StatLayout stat_layout(int64_t blocks, int64_t n_slices) {
 template <int V>
 hipError_t stat_launch(const StatArgs& a, hipEvent_t checked, hipStream_t st) {
   const dim3 grid((unsigned)a.blocks, (unsigned)a.n_slices), rgrid(kBins / kWave, (unsigned)a.n_slices);
-  const dim3 rgrid_last(2048 / kWave, (unsigned)a.n_slices);
   stat_pass_kernel<0, V><<<grid, kStatThreads, 0, st>>>(a);
   const hipError_t e = checked != nullptr ? hipEventRecord(checked, st) : hipSuccess;
-  stat_reduce_kernel<false><<<rgrid, kStatThreads, 0, st>>>(a);
+  stat_reduce_kernel<<<rgrid, kStatThreads, 0, st>>>(a);
   stat_pass_kernel<1, V><<<grid, kStatThreads, 0, st>>>(a);
-  stat_reduce_kernel<false><<<rgrid, kStatThreads, 0, st>>>(a);
   stat_pass_kernel<2, V><<<grid, kStatThreads, 0, st>>>(a);
-  stat_reduce_kernel<true><<<rgrid_last, kStatThreads, 0, st>>>(a);
   return e;
 }
 
