@@ -17,7 +17,7 @@
 // caller does not wait for the rest.  The four launches take 44 us; six, with sums of all counters behind the second and third
 // pass too, 49, with a second read of the sample 52, a third 66 (the host 195 ms on a copy of the sample, np.percentile).
 // Likewise 100 000 x 602 values 151 -> 101 -> 96 us (second read saved, sums saved), 60 000 x 1030 203 -> 130 -> 125, 1 000 000 x 128
-// 238 -> 151 -> 146, 1000 x 64 31 -> 27.  Tables on which a workgroup has to read its rows again lose up to 6 % by what it kept in
+// 238 -> 151 -> 146, 1000 x 64 31 -> 27 (25 with more workgroups).  Tables on which a workgroup has to read its rows again lose up to 6 % by what it kept in
 // vain and gain the sums (120 000 x 100: all values equal 369 us before and after, 80 % zeros 180, rows of very different
 // lengths 52 -> 48).
 #include "common.hpp"
@@ -515,10 +515,14 @@ __global__ __launch_bounds__(kStatThreads) void stat_reduce_kernel(StatArgs a) {
   }
 }
 
-// Workgroups per slice: one per CU over all slices, each with at least 32 values per thread.
+// Workgroups per slice: one per CU over all slices, each with at least four rows per lane of what a lane reads of a row at a
+// time.  A short sample is the length of its chains, the counters' additions in LDS most of all, not the sum of its workgroups
+// (32 values per lane / four rows: 150 000 x 6 in slices of one column 88 / 37 us, 5000 x 75 39 / 26, 3000 x 50 31 / 25, 1000 x 64 27 /
+// 25, 50 000 x 128 in slices of 32 level; two rows of four columns lose: 10 000 x 128 28 / 30).
 int stat_blocks(int64_t m, int64_t cols, int64_t slice, int64_t n_slices) {
   const int64_t width = cols < slice ? cols : slice;
-  int64_t b = ceil_div(m * width, (int64_t)kStatThreads * 32);
+  const int64_t least = width % 4 == 0 ? 16 : width % 2 == 0 ? 8 : 4;
+  int64_t b = ceil_div(m * width, (int64_t)kStatThreads * least);
   const int64_t cap = n_slices >= kMaxBlocks / 4 ? 4 : kMaxBlocks / n_slices;
   b = b > cap ? cap : b;
   return (int)(b < 1 ? 1 : b);
