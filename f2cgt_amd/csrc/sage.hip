@@ -11,9 +11,10 @@ namespace f2cgt {
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTile = 32;            // rows and outputs of a tile: one 32 x 32 x 2 matrix instruction
-constexpr int kForwardWaves = 4;     // they share a tile's columns
+constexpr int kForwardWaves = 4;     // a quarter of a tile each
 constexpr int kGradWaves = 16;       // they share a tile's rows
 
 struct SageArgs {
@@ -25,78 +26,70 @@ struct SageArgs {
   int n, k[2], relu;
 };
 
-// out = x0 w0^T + x1 w1^T + bias, a 32 x 32 tile per workgroup; its waves take the columns 32 at a time in turn, so that
-// 1024 rows and 256 outputs make 256 workgroups, and add their tiles in LDS.
-// Lane l of the matrix instruction has row l % 32 of x and of w and one of its two columns; here columns 4 (l / 32) + t
-// of every eight are those of the instruction's step t, so that a lane reads 16 bytes of its row at a time.
+// out = (x0 w0^T + bias) + x1 w1^T, a 32 x 32 tile per workgroup and 16 x 16 of it per wave, so that 1024 rows and 256 outputs
+// make 1024 waves, one per SIMD, of which a wave's chain of loads and matrix instructions is the time: 11 us at 128 + 128 columns (12 with
+// 128 columns in flight; 6.8 with the columns shared among four waves, which adds in another order).
+//
+// A product is one chain of 16 x 16 x 4 instructions over its columns, of every eight the even ones and then the odd ones, four
+// after four behind the last whole 16, and the two products meet behind it: the order in which the library that stands behind torch's operators adds at a
+// minibatch's sizes (taken from its results, which these equal bit for bit).  A ReLU's gradient is why that matters: a value
+// next to zero that another order puts on the other side of it, one in 10^7, passes its whole gradient or none of it.
 __global__ __launch_bounds__(kForwardWaves * kWave) void sage_linear_kernel(SageArgs a) {
-  __shared__ __align__(16) float s_tile[kForwardWaves][kTile][kTile + 4];
-  const int t = threadIdx.x, wave = t / kWave, lane = t & (kWave - 1), at = lane & 31, side = lane >> 5;
-  const int64_t m0 = (int64_t)blockIdx.x * kTile;
-  const int n0 = blockIdx.y * kTile;
+  constexpr int U = 8;                                  // blocks of eight columns in flight, and as many more on their way
+  const int t = threadIdx.x, wave = t / kWave, lane = t & (kWave - 1), at = lane & 15, part = lane >> 4;
+  const int64_t m0 = (int64_t)blockIdx.x * kTile + 16 * (wave & 1);
+  const int n0 = blockIdx.y * kTile + 16 * (wave >> 1);
+  if (m0 >= a.m || n0 >= a.n) return;
   const int64_t row = m0 + at < a.m ? m0 + at : a.m - 1;
   const int col = n0 + at < a.n ? n0 + at : a.n - 1;
-  const int chunks0 = (a.k[0] + 31) / 32, chunks = chunks0 + (a.k[1] + 31) / 32;
-  float4 x[4], w[4];
-  auto load = [&](int c) {
-    const int s = c >= chunks0 ? 1 : 0;
-    const int k = a.k[s], k0 = (c - (s ? chunks0 : 0)) * 32 + 4 * side;
+  const int batches0 = (a.k[0] + 8 * U - 1) / (8 * U), batches = batches0 + (a.k[1] + 8 * U - 1) / (8 * U);
+  float2 x[U], w[U];
+  // Lane part p has columns 2 p and 2 p + 1 of a block; behind the last whole 16 columns it has p and, of eight, 4 + p.
+  auto load = [&](int b) {
+    const int s = b >= batches0 ? 1 : 0;
+    const int k = a.k[s], from = (b - (s ? batches0 : 0)) * 8 * U;
     const float* xr = a.x[s] + row * k;
     const float* wr = a.w[s] + (int64_t)col * k;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int kq = k0 + 8 * q;
-      const bool in = kq < k;                              // (a multiple of four columns: all four or none)
-      x[q] = *reinterpret_cast<const float4*>(xr + (in ? kq : 0));
-      w[q] = *reinterpret_cast<const float4*>(wr + (in ? kq : 0));
-      if (!in) x[q] = w[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int u = 0; u < U; ++u) {
+      const int c = from + 8 * u;
+      if (c < (k & ~15)) {
+        x[u] = *reinterpret_cast<const float2*>(xr + c + 2 * part);
+        w[u] = *reinterpret_cast<const float2*>(wr + c + 2 * part);
+      } else if (c < k) {
+        const int second = c + 8 <= k ? c + 4 + part : c + part;
+        x[u] = make_float2(xr[c + part], xr[second]);
+        w[u] = make_float2(wr[c + part], wr[second]);
+      }
     }
   };
-  floatx16 acc;
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f}, self = acc;
+  load(0);
+  for (int b = 0; b < batches; ++b) {
+    float2 xc[U], wc[U];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-  if (wave < chunks) load(wave);
-  for (int c = wave; c < chunks; c += kForwardWaves) {
-    float4 xc[4], wc[4];
+    for (int u = 0; u < U; ++u) { xc[u] = x[u]; wc[u] = w[u]; }
+    if (b + 1 < batches) load(b + 1);
+    if (b == batches0) {
+      self = acc;
+      acc = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    const int left = b >= batches0 ? a.k[1] - (b - batches0) * 8 * U : a.k[0] - b * 8 * U;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) { xc[q] = x[q]; wc[q] = w[q]; }
-    if (c + kForwardWaves < chunks) load(c + kForwardWaves);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xc[q].x, wc[q].x, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xc[q].y, wc[q].y, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xc[q].z, wc[q].z, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xc[q].w, wc[q].w, acc, 0, 0, 0);
+    for (int u = 0; u < U; ++u) {
+      if (8 * u >= left) break;
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xc[u].x, wc[u].x, acc, 0, 0, 0);
+      if (8 * u + 4 < left) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xc[u].y, wc[u].y, acc, 0, 0, 0);
     }
   }
-#pragma unroll
-  for (int v = 0; v < 16; ++v) s_tile[wave][8 * (v / 4) + 4 * side + v % 4][at] = acc[v];
-  __syncthreads();
-  const int r = t / 8, c4 = t % 8 * 4;
-  float v[4];
-  {
-    float4 sum = *reinterpret_cast<const float4*>(&s_tile[0][r][c4]);
-#pragma unroll
-    for (int i = 1; i < kForwardWaves; ++i) {
-      const float4 p = *reinterpret_cast<const float4*>(&s_tile[i][r][c4]);
-      sum.x += p.x; sum.y += p.y; sum.z += p.z; sum.w += p.w;
-    }
-    v[0] = sum.x; v[1] = sum.y; v[2] = sum.z; v[3] = sum.w;
-  }
-  if (m0 + r >= a.m) return;
+  const float bias = a.bias != nullptr ? a.bias[col] : 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int c = n0 + c4 + i;
-    if (a.bias != nullptr) v[i] += a.bias[c < a.n ? c : a.n - 1];
-    if (a.relu) v[i] = v[i] <= 0.f ? 0.f : v[i];           // (a NaN stays one)
-  }
-  float* dst = a.out + (m0 + r) * a.n + n0 + c4;
-  if ((a.n & 3) == 0) {
-    if (n0 + c4 < a.n) *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (n0 + c4 + i < a.n) dst[i] = v[i];
+    const int64_t r = m0 + 4 * part + i;
+    float v = a.bias != nullptr ? self[i] + bias : self[i];
+    v += acc[i];
+    if (a.relu && v <= 0.f) v = 0.f;                    // (a NaN stays one)
+    if (r < a.m && n0 + at < a.n) a.out[r * a.n + n0 + at] = v;
   }
 }
 
@@ -229,7 +222,8 @@ extern "C" int f2cgt_sage_linear(const float* x0, const float* w0, const float* 
 
 // A tile of 32 outputs reads its rows and weights once per tile of the other side, which a library's larger tiles do half
 // as often: past 131 072 weights that is what the time goes into, in large launches.  Device time of a step forward and
-// backward, operators -> this, us (128 + 128 -> 256 means two inputs of 128 columns and 256 outputs):
+// backward, operators -> this, us (128 + 128 -> 256 means two inputs of 128 columns and 256 outputs; measured with a forward
+// kernel that shared the columns among four waves, 6.8 us of the first 25 where this one takes 11):
 //   128 + 128 -> 256: 1024 rows 51 -> 25, 8192 158 -> 59, 60 000 497 -> 314, 120 000 1059 -> 610
 //   256 + 256 -> 256: 1024 rows 54 -> 27, 4096 109 -> 58, 32 000 375 -> 334;  100 + 100 -> 128: 500 rows 103 -> 19
 //   600 + 600 -> 16:  3000 rows 66 -> 35, 60 000 334 -> 241;  1000 + 1000 -> 64: 16 000 rows 311 -> 180

@@ -59,6 +59,29 @@ def test_special_values_and_absent_parts():
         assert not lib.sage_linear(x0, x1, w0, w1, b, True).requires_grad
 
 
+# columns with and without a rest of sixteen, and past what the kernel takes; a minibatch's rows
+@pytest.mark.parametrize("k0,k1", [(128, 128), (96, 96), (100, 100), (64, 28), (36, 48), (260, 36), (256, 256)])
+@pytest.mark.parametrize("m,n", [(500, 128), (1024, 256), (3001, 128), (8192, 64)])
+@pytest.mark.parametrize("relu", [True, False])
+@pytest.mark.parametrize("with_bias", [True, False])
+def test_a_pass_that_is_differentiated_has_the_operators_values(m, k0, k1, n, relu, with_bias):
+    """Bit for bit: next to zero another last bit would be another mask of the gradient."""
+    x0, x1, w0, w1, b, _ = _inputs(m, k0, k1, n)
+    got = f2cgt_amd.load().sage_linear(x0, x1, w0, w1, b if with_bias else None, relu)
+    want = torch.nn.functional.linear(x0, w0, b if with_bias else None) + torch.nn.functional.linear(x1, w1)
+    assert torch.equal(got, torch.relu(want) if relu else want)
+
+
+def test_passes_of_many_rows_are_differentiated_by_the_operators():
+    x0, x1, w0, w1, b, _ = _inputs(8193, 8, 8, 4)
+    lib = f2cgt_amd.load()
+    assert lib.sage_linear(x0, x1, w0, w1, b, True) is None and lib.sage_linear(x0[1:], x1[1:], w0, w1, b, True) is not None
+    with torch.no_grad():
+        out = lib.sage_linear(x0, x1, w0, w1, b, True)
+    torch.testing.assert_close(out, torch.relu(torch.nn.functional.linear(x0, w0, b) + torch.nn.functional.linear(x1, w1)),
+                               rtol=1e-5, atol=1e-5)
+
+
 def test_gradient_of_the_gradient():
     lib = f2cgt_amd.load()
     x0, x1, w0, w1, b, g = _inputs(50, 8, 8, 7)
