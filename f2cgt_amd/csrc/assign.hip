@@ -16,10 +16,10 @@
 // cut, at twice the matrix instructions, 1.6 times the conversions and half as much LDS again.)
 //
 // What bounds it: the issue of vector and matrix instructions, which hardly run side by side on a SIMD (measured with two
-// waves on it: six of the matrix instructions 194 clocks, 96 v_fma 220, both 396), behind that the fixed part of a launch,
-// 15 us at 32 dimensions: centres from memory, their means, norms and pieces, then the loop with cold instruction caches.
-// Against three bf16 pieces with (best, second) kept per tile: 1e6 x 32, 256 centres, L2 121 -> 94 us; 1e6 x 16 cosine
-// 69 -> 47, 150 000 x 16 26 -> 17.5; 1e6 x 16 against 1024 centres 430 -> 154; 500 000 x 128 in slices of 16 229 -> 162.
+// waves on it: six of the matrix instructions 194 clocks, 96 v_fma 220, both 396), behind that the staging of a launch, 4 us
+// at 16 dimensions and 7 at 32 by time stamps: centres from memory, their means, norms and pieces.
+// Against three bf16 pieces with (best, second) kept per tile: 1e6 x 32, 256 centres, L2 121 -> 79 us; 1e6 x 16 cosine
+// 69 -> 47, 150 000 x 16 26 -> 17.5; 1e6 x 16 against 1024 centres 430 -> 154; 500 000 x 128 in slices of 16 229 -> 149.
 // A wave owns 32 rows of x at a time and walks the centres a 32 x 32 tile at a time, A = centre tile (LDS), B = x tile (registers),
 // so that a lane holds 16 scores of ONE row per tile.  It does not look for the best two of them: it keeps, over the T
 // tiles of a chunk, the minimum of every slot (a class of T centres), half an instruction per score, and only the 16

@@ -217,10 +217,10 @@ def main(argv):
             fh.write("\n")
     A = "python3 bench.py --all --steps 200 --warmup 20 --cpu-seconds 0"
     tall = os.path.join(O, "trace_all")
-    k = kstats(tall, "assign_kernel<2, 4, true, false>")
+    k = kstats(tall, "assign_kernel<2, 4, true, false, 0>")
     if k:
         with open(os.path.join(P, "assign_kernel_c5_encode.md"), "w") as fh:
-            fh.write("# assign_kernel<2, 4, true, false> on the C5 encode step (1e6 x 32 fp32 vs 256 centres, squared L2 + arg-min)\n\n")
+            fh.write("# assign_kernel<2, 4, true, false, 0> on the C5 encode step (1e6 x 32 fp32 vs 256 centres, squared L2 + arg-min)\n\n")
             fh.write("Commands (separate runs):\n\n")
             fh.write("    rocprofv3 --kernel-trace --stats --output-format csv -d out/trace_all -o t -- %s\n" % A)
             fh.write("    rocprofv3 --pmc SQ_INSTS_VALU_MFMA_MOPS_F16 SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_INSTS_MFMA "
@@ -232,7 +232,7 @@ def main(argv):
                      "product block (two fp16 pieces per value), i.e. %.0f TFLOP/s of fp16 MFMA = %.3f of the 2500 TFLOP/s "
                      "peak.\n\n" % (fl, fl / (k[2] * 1e-6) / 1e12, 3 * fl / (k[2] * 1e-6) / 1e12,
                                          3 * fl / (k[2] * 1e-6) / 1e12 / 2500))
-            vals = counters(os.path.join(O, "mfma_all"), "assign_kernel<2, 4, true, false>")
+            vals = counters(os.path.join(O, "mfma_all"), "assign_kernel<2, 4, true, false, 0>")
             if vals:
                 fh.write("| counter (mean per dispatch) | value |\n|---|---|\n")
                 for cn in sorted(vals):
