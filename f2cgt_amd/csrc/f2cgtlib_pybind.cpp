@@ -1121,9 +1121,9 @@ c10::optional<torch::Tensor> sage_linear(const torch::Tensor& x0, const torch::T
       !f2cgt_sage_linear_ahead(m, n, k0, k1))
     return c10::nullopt;
   if (c10::GradMode::is_enabled() && (w0.requires_grad() || w1.requires_grad() || (bias.has_value() && bias->requires_grad()))) {
-    // The library adds a gradient up over the rows in an order of its own: 4e-7 of the gradients away at 1024 rows, 1.5e-6 at
-    // 16 000, most of it the library's own error.  Up to 8192 rows that is below what callers compare such sums to.
-    if (m > 8192) return c10::nullopt;
+    // The library adds a gradient up over the rows in an order of its own: 4e-7 of the gradients away at 1024 rows, 8e-7 at
+    // 3400, 1.5e-6 at 16 000, most of it the library's own error.  Up to 4096 rows that is half of what callers compare such sums to.
+    if (m > 4096) return c10::nullopt;
     return SageLinear::apply(x0, x1, w0, w1, bias, relu);
   }
   c10::DeviceGuard guard(x0.device());
