@@ -1031,6 +1031,29 @@ using torch::autograd::AutogradContext;
 using torch::autograd::Variable;
 using torch::autograd::variable_list;
 
+// Whether an operator's call goes straight to the device now: no transform, forward-mode gradient, autocast, dispatch or
+// function mode and no tracing is active.
+bool plain_calls() {
+  using c10::DispatchKey;
+  static const c10::DispatchKeySet plain = c10::DispatchKeySet({DispatchKey::BackendSelect, DispatchKey::ADInplaceOrView});
+  return (c10::impl::tls_local_dispatch_key_set().included_ | plain) == plain && !at::autocast::is_autocast_enabled(at::kCUDA) &&
+         at::impl::PythonTorchFunctionTLS::stack_len() == 0 && !torch::jit::tracer::isTracing() &&
+         torch::autograd::ForwardADLevel::try_get_by_idx(0) == nullptr;
+}
+
+// Whether t is fp32 memory on `device` and nothing else: no wrapper (a batch, a subclass with its own dispatch), no lazily
+// negated or zero tensor.
+bool plain_tensor(const torch::Tensor& t, const c10::Device& device) {
+  using c10::DispatchKey;
+  static const c10::DispatchKeySet plain = c10::DispatchKeySet({DispatchKey::CUDA, DispatchKey::AutogradCUDA,
+                                                                DispatchKey::ADInplaceOrView, DispatchKey::AutocastCUDA});
+  return t.defined() && (t.key_set() | plain) == plain && t.scalar_type() == torch::kFloat32 && t.layout() == torch::kStrided &&
+         t.device() == device;
+}
+bool dense_rows(const torch::Tensor& t, const c10::Device& device, int64_t rows, int64_t cols) {
+  return plain_tensor(t, device) && t.dim() == 2 && t.is_contiguous() && t.size(0) == rows && t.size(1) == cols;
+}
+
 // act(x0 w0^T + x1 w1^T + bias); only w0, w1 and bias are differentiated.  The products have the values of the modules' own,
 // bit for bit: a value next to zero that two orders of summation put on either side of it, one in 10^7, passes its whole
 // gradient in one and none in the other (a gradient of 16 000 rows is 5e-4 away for it).  sage_linear_kernel adds as the
@@ -1069,17 +1092,22 @@ struct SageLinear : public torch::autograd::Function<SageLinear> {
     variable_list result(6);
     Variable g = grads[0];
     if (!g.defined() || !(want0 || want1 || want_b)) return result;
-    if (c10::GradMode::is_enabled() || !g.is_cuda() || g.scalar_type() != torch::kFloat32 || g.layout() != torch::kStrided) {
-      // a gradient that is differentiated itself: the same sums from operators that are
+    // The saved tensors went through the caller's hooks, the gradient through operators between: each is looked at again.
+    const c10::Device device = x0.device();
+    const bool own = !c10::GradMode::is_enabled() && plain_calls() && plain_tensor(g, device) && g.dim() == 2 &&
+                     x0.dim() == 2 && x1.dim() == 2 && dense_rows(x0, device, g.size(0), x0.size(1)) &&
+                     dense_rows(x1, device, g.size(0), x1.size(1)) && (!relu || dense_rows(saved[2], device, g.size(0), g.size(1)));
+    if (!own) {
+      // a gradient that is differentiated itself or is a batch of them, a mode: the same sums from operators
       if (relu) g = at::threshold_backward(g, saved[2], 0);
       if (want0) result[2] = g.t().mm(x0);
       if (want1) result[3] = g.t().mm(x1);
       if (want_b) result[4] = g.sum(0);
       return result;
     }
+    c10::DeviceGuard guard(device);
     g = g.contiguous();
-    c10::DeviceGuard guard(g.device());
-    const int64_t m = x0.size(0), n = g.size(1), k0 = x0.size(1), k1 = x1.size(1);
+    const int64_t m = g.size(0), n = g.size(1), k0 = x0.size(1), k1 = x1.size(1);
     if (want0) result[2] = torch::empty({n, k0}, g.options());
     if (want1) result[3] = torch::empty({n, k1}, g.options());
     if (want_b) result[4] = torch::empty({n}, g.options());
@@ -1100,19 +1128,11 @@ struct SageLinear : public torch::autograd::Function<SageLinear> {
 // (transforms, forward-mode gradients, autocast, dispatch and function modes, tracing).
 c10::optional<torch::Tensor> sage_linear(const torch::Tensor& x0, const torch::Tensor& x1, const torch::Tensor& w0,
                                          const torch::Tensor& w1, const c10::optional<torch::Tensor>& bias, bool relu) {
-  using c10::DispatchKey;
-  static const c10::DispatchKeySet plain_keys = c10::DispatchKeySet({DispatchKey::CUDA, DispatchKey::AutogradCUDA,
-                                                                     DispatchKey::ADInplaceOrView, DispatchKey::AutocastCUDA});
-  static const c10::DispatchKeySet plain_tls = c10::DispatchKeySet({DispatchKey::BackendSelect, DispatchKey::ADInplaceOrView});
+  if (!plain_calls()) return c10::nullopt;
+  if (!x0.defined()) return c10::nullopt;
   auto plain = [&](const torch::Tensor& t, int64_t dims) {
-    return t.defined() && (t.key_set() | plain_keys) == plain_keys && t.scalar_type() == torch::kFloat32 &&
-           t.layout() == torch::kStrided && t.dim() == dims && t.is_contiguous() && t.device() == x0.device() &&
-           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    return plain_tensor(t, x0.device()) && t.dim() == dims && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
-  const auto tls = c10::impl::tls_local_dispatch_key_set();
-  if (!((tls.included_ | plain_tls) == plain_tls) || at::autocast::is_autocast_enabled(at::kCUDA) || at::impl::PythonTorchFunctionTLS::stack_len() > 0 || torch::jit::tracer::isTracing() ||
-      torch::autograd::ForwardADLevel::try_get_by_idx(0) != nullptr)
-    return c10::nullopt;
   if (!plain(x0, 2) || !plain(x1, 2) || !plain(w0, 2) || !plain(w1, 2) || (bias.has_value() && !plain(*bias, 1)))
     return c10::nullopt;
   const int64_t m = x0.size(0), n = w0.size(0), k0 = x0.size(1), k1 = x1.size(1);

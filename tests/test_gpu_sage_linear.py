@@ -147,3 +147,55 @@ def test_layer_equals_its_linears_with_hooks_and_without():
     conv.activation = torch.tanh
     out = conv((indptr, indices), (h[:100], h))
     assert float(out.detach().min()) < 0
+
+
+def _against_the_operators(run, relu=True):
+    """`run(out, parameters)` on the kernel's output and on the two Linears': the same gradients."""
+    x0, x1, w0, w1, b, g = _inputs(300, 16, 24, 40)
+    got = run(f2cgt_amd.load().sage_linear(x0, x1, w0, w1, b, relu), (w0, w1, b), g)
+    z = torch.nn.functional.linear(x0, w0, b) + torch.nn.functional.linear(x1, w1)
+    want = run(torch.relu(z) if relu else z, (w0, w1, b), g)
+    for a, c in zip(got, want):
+        assert a.shape == c.shape
+        torch.testing.assert_close(a, c, rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("relu", [True, False])
+def test_batched_gradients(relu):
+    _against_the_operators(lambda out, p, g: torch.autograd.grad(out, p, torch.stack([g, 2 * g, g.flip(0)]), is_grads_batched=True), relu)
+
+
+def test_gradients_that_are_not_plain_memory():
+    """A view that negates, rows that are one row, columns apart: what an operator in between may hand on."""
+    for form in (torch._neg_view, lambda g: g[:1].expand_as(g), lambda g: g.t().contiguous().t()):
+        _against_the_operators(lambda out, p, g: torch.autograd.grad(out, p, form(g)))
+    zero = torch._efficientzerotensor((300, 40), device="cuda")
+    _against_the_operators(lambda out, p, g: torch.autograd.grad(out, p, zero))
+
+
+def test_a_mode_around_the_backward_pass_sees_its_operators():
+    from torch.utils._python_dispatch import TorchDispatchMode
+    seen = []
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    def run(out, p, g):
+        with Seen():
+            return torch.autograd.grad(out, p, g)
+    x0, x1, w0, w1, b, g = _inputs(300, 16, 24, 40)
+    run(f2cgt_amd.load().sage_linear(x0, x1, w0, w1, b, True), (w0, w1, b), g)
+    assert sum("mm" in name for name in seen) == 2 and any("threshold_backward" in name for name in seen)
+    _against_the_operators(run)
+
+
+def test_saved_tensors_that_come_back_in_another_layout():
+    x0, x1, w0, w1, b, g = _inputs(300, 16, 24, 40)
+    want = torch.autograd.grad(f2cgt_amd.load().sage_linear(x0, x1, w0, w1, b, True), (w0, w1, b), g)
+    for unpack in (lambda t: t.t().contiguous().t(), lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            out = f2cgt_amd.load().sage_linear(x0, x1, w0, w1, b, True)
+        for a, c in zip(torch.autograd.grad(out, (w0, w1, b), g), want):
+            torch.testing.assert_close(a, c, rtol=1e-5, atol=1e-4)
