@@ -1041,6 +1041,13 @@ bool plain_calls() {
          torch::autograd::ForwardADLevel::try_get_by_idx(0) == nullptr;
 }
 
+// Whether t is a torch.Tensor or a Parameter in Python: a subclass of them may have operators of its own
+// (__torch_function__), which its keys do not tell.  Holds the GIL.
+bool own_class(const torch::Tensor& t) {
+  const auto object = py::reinterpret_steal<py::object>(THPVariable_Wrap(t));
+  return THPVariable_CheckExact(object.ptr());
+}
+
 // Whether t is fp32 memory on `device` and nothing else: no wrapper (a batch, a subclass with its own dispatch), no lazily
 // negated or zero tensor.
 bool plain_tensor(const torch::Tensor& t, const c10::Device& device) {
@@ -1125,7 +1132,7 @@ struct SageLinear : public torch::autograd::Function<SageLinear> {
 
 // -> the layer's output, or None for the calls that are left to the module's own operators: other types, layouts, devices
 // and sizes; inputs that are differentiated; and whenever an operator's call would not go straight to the device
-// (transforms, forward-mode gradients, autocast, dispatch and function modes, tracing).
+// (subclasses of Tensor, transforms, forward-mode gradients, autocast, dispatch and function modes, tracing).
 c10::optional<torch::Tensor> sage_linear(const torch::Tensor& x0, const torch::Tensor& x1, const torch::Tensor& w0,
                                          const torch::Tensor& w1, const c10::optional<torch::Tensor>& bias, bool relu) {
   if (!plain_calls()) return c10::nullopt;
@@ -1134,6 +1141,8 @@ c10::optional<torch::Tensor> sage_linear(const torch::Tensor& x0, const torch::T
     return plain_tensor(t, x0.device()) && t.dim() == dims && t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   };
   if (!plain(x0, 2) || !plain(x1, 2) || !plain(w0, 2) || !plain(w1, 2) || (bias.has_value() && !plain(*bias, 1)))
+    return c10::nullopt;
+  if (!own_class(x0) || !own_class(x1) || !own_class(w0) || !own_class(w1) || (bias.has_value() && !own_class(*bias)))
     return c10::nullopt;
   const int64_t m = x0.size(0), n = w0.size(0), k0 = x0.size(1), k1 = x1.size(1);
   if (x0.requires_grad() || x1.requires_grad() || m < 1 || n < 1 || k0 < 4 || k1 < 4 || k0 % 4 != 0 || k1 % 4 != 0 ||

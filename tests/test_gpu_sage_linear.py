@@ -199,3 +199,33 @@ def test_saved_tensors_that_come_back_in_another_layout():
             out = f2cgt_amd.load().sage_linear(x0, x1, w0, w1, b, True)
         for a, c in zip(torch.autograd.grad(out, (w0, w1, b), g), want):
             torch.testing.assert_close(a, c, rtol=1e-5, atol=1e-4)
+
+
+def test_subclasses_with_operators_of_their_own_keep_them():
+    calls = []
+
+    class Tagged(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            calls.append(getattr(func, "__name__", str(func)))
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    class Bare(torch.Tensor):        # results of its operators are of its class
+        pass
+
+    lib = f2cgt_amd.load()
+    x0, x1, w0, w1, b, _ = _inputs(300, 16, 16, 40)
+    for kind in (Tagged, Bare):
+        for at in range(5):
+            args = [x0, x1, w0, w1, b]
+            args[at] = args[at].detach().as_subclass(kind)
+            assert lib.sage_linear(*args, True) is None, (kind, at)
+    conv = pipeline.MySAGEConv(16, 40, "mean", None, activation=torch.relu).cuda()
+    indptr, indices = torch.arange(0, 301, device="cuda"), torch.arange(0, 300, device="cuda")
+    plain = conv((indptr, indices), (x0, x1))
+    del calls[:]
+    got = conv((indptr, indices), (x0.as_subclass(Tagged), x1))
+    assert isinstance(got, Tagged) and "linear" in calls and type(plain) is torch.Tensor
+    torch.testing.assert_close(got.as_subclass(torch.Tensor), plain, rtol=1e-5, atol=1e-5)
+    parameter = torch.nn.Parameter(w0.detach())      # (a class of its own without operators)
+    assert lib.sage_linear(x0, x1, parameter, w1, b, True) is not None
