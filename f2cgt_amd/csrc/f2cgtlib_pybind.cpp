@@ -1061,28 +1061,33 @@ bool dense_rows(const torch::Tensor& t, const c10::Device& device, int64_t rows,
   return plain_tensor(t, device) && t.dim() == 2 && t.is_contiguous() && t.size(0) == rows && t.size(1) == cols;
 }
 
-// act(x0 w0^T + x1 w1^T + bias); only w0, w1 and bias are differentiated.  The products have the values of the modules' own,
-// bit for bit: a value next to zero that two orders of summation put on either side of it, one in 10^7, passes its whole
-// gradient in one and none in the other (a gradient of 16 000 rows is 5e-4 away for it).  sage_linear_kernel adds as the
-// library does up to 128 columns (tests name the sizes); beyond them it chooses among orders, and the products are its own.
+// act(x0 w0^T + x1 w1^T + bias) by the kernel or by the library's products.  The two have the same bits at the shapes that
+// the kernel is taken for: a value next to zero that two orders of summation put on either side of it, one in 10^7, passes
+// its whole gradient in one and none in the other (a gradient of 16 000 rows is 5e-4 away for it).
+torch::Tensor sage_forward(bool kernel, const torch::Tensor& x0, const torch::Tensor& x1, const torch::Tensor& w0,
+                           const torch::Tensor& w1, const c10::optional<torch::Tensor>& bias, bool relu) {
+  if (kernel) {
+    c10::DeviceGuard guard(x0.device());
+    const int64_t m = x0.size(0), n = w0.size(0);
+    auto out = torch::empty({m, n}, x0.options());
+    check_rc(f2cgt_sage_linear(x0.data_ptr<float>(), w0.data_ptr<float>(), x1.data_ptr<float>(), w1.data_ptr<float>(),
+                               bias.has_value() ? bias->data_ptr<float>() : nullptr, out.data_ptr<float>(), m, n, x0.size(1),
+                               x1.size(1), relu ? 1 : 0, current_stream()),
+             "sage_linear");
+    return out;
+  }
+  at::AutoDispatchBelowADInplaceOrView products;        // (nothing in here is differentiated by itself)
+  auto out = bias.has_value() ? at::addmm(*bias, x0, w0.t()) : at::mm(x0, w0.t());
+  out.add_(at::mm(x1, w1.t()));
+  if (relu) out.relu_();
+  return out;
+}
+
+// Only w0, w1 and bias are differentiated.
 struct SageLinear : public torch::autograd::Function<SageLinear> {
   static Variable forward(AutogradContext* ctx, const Variable& x0, const Variable& x1, const Variable& w0, const Variable& w1,
-                          const c10::optional<Variable>& bias, bool relu) {
-    c10::DeviceGuard guard(x0.device());
-    const int64_t m = x0.size(0), n = w0.size(0), k0 = x0.size(1), k1 = x1.size(1);
-    torch::Tensor out;
-    if (k0 <= 128 && k1 <= 128) {
-      out = torch::empty({m, n}, x0.options());
-      check_rc(f2cgt_sage_linear(x0.data_ptr<float>(), w0.data_ptr<float>(), x1.data_ptr<float>(), w1.data_ptr<float>(),
-                                 bias.has_value() ? bias->data_ptr<float>() : nullptr, out.data_ptr<float>(), m, n, k0, k1,
-                                 relu ? 1 : 0, current_stream()),
-               "sage_linear");
-    } else {
-      at::AutoDispatchBelowADInplaceOrView products;    // (nothing in here is differentiated by itself)
-      out = bias.has_value() ? at::addmm(*bias, x0, w0.t()) : at::mm(x0, w0.t());
-      out.add_(at::mm(x1, w1.t()));
-      if (relu) out.relu_();
-    }
+                          const c10::optional<Variable>& bias, bool relu, bool kernel) {
+    torch::Tensor out = sage_forward(kernel, x0, x1, w0, w1, bias, relu);
     ctx->saved_data["relu"] = relu;
     ctx->saved_data["bias"] = bias.has_value();
     if (relu) ctx->save_for_backward({x0, x1, out});
@@ -1096,7 +1101,7 @@ struct SageLinear : public torch::autograd::Function<SageLinear> {
     const Variable& x0 = saved[0];
     const Variable& x1 = saved[1];
     const bool want0 = ctx->needs_input_grad(2), want1 = ctx->needs_input_grad(3), want_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(4);
-    variable_list result(6);
+    variable_list result(7);
     Variable g = grads[0];
     if (!g.defined() || !(want0 || want1 || want_b)) return result;
     // The saved tensors went through the caller's hooks, the gradient through operators between: each is looked at again.
@@ -1146,22 +1151,14 @@ c10::optional<torch::Tensor> sage_linear(const torch::Tensor& x0, const torch::T
     return c10::nullopt;
   const int64_t m = x0.size(0), n = w0.size(0), k0 = x0.size(1), k1 = x1.size(1);
   if (x0.requires_grad() || x1.requires_grad() || m < 1 || n < 1 || k0 < 4 || k1 < 4 || k0 % 4 != 0 || k1 % 4 != 0 ||
-      x1.size(0) != m || w1.size(0) != n || w0.size(1) != k0 || w1.size(1) != k1 || (bias.has_value() && bias->size(0) != n) ||
-      !f2cgt_sage_linear_ahead(m, n, k0, k1))
+      x1.size(0) != m || w1.size(0) != n || w0.size(1) != k0 || w1.size(1) != k1 || (bias.has_value() && bias->size(0) != n))
     return c10::nullopt;
+  const int take = f2cgt_sage_linear_ahead(m, n, k0, k1);
   if (c10::GradMode::is_enabled() && (w0.requires_grad() || w1.requires_grad() || (bias.has_value() && bias->requires_grad()))) {
-    // The library adds a gradient up over the rows in an order of its own: 4e-7 of the gradients away at 1024 rows, 8e-7 at
-    // 3400, 1.5e-6 at 16 000, most of it the library's own error.  Up to 4096 rows that is half of what callers compare such sums to.
-    if (m > 4096) return c10::nullopt;
-    return SageLinear::apply(x0, x1, w0, w1, bias, relu);
+    if (!(take & F2CGT_SAGE_GRAD)) return c10::nullopt;
+    return SageLinear::apply(x0, x1, w0, w1, bias, relu, (take & F2CGT_SAGE_STEP) != 0);
   }
-  c10::DeviceGuard guard(x0.device());
-  auto out = torch::empty({m, n}, x0.options());
-  check_rc(f2cgt_sage_linear(x0.data_ptr<float>(), w0.data_ptr<float>(), x1.data_ptr<float>(), w1.data_ptr<float>(),
-                             bias.has_value() ? bias->data_ptr<float>() : nullptr, out.data_ptr<float>(), m, n, k0, k1,
-                             relu ? 1 : 0, current_stream()),
-           "sage_linear");
-  return out;
+  return sage_forward((take & F2CGT_SAGE_FORWARD) != 0, x0, x1, w0, w1, bias, relu);
 }
 
 torch::Tensor vq_encode(torch::Tensor x, torch::Tensor centers, std::string metric) {

@@ -31,9 +31,10 @@ struct SageArgs {
 // 128 columns in flight; 6.8 with the columns shared among four waves, which adds in another order).
 //
 // A product is one chain of 16 x 16 x 4 instructions over its columns, of every eight the even ones and then the odd ones, four
-// after four behind the last whole 16, and the two products meet behind it: the order in which the library that stands behind torch's operators adds at a
-// minibatch's sizes (taken from its results, which these equal bit for bit).  A ReLU's gradient is why that matters: a value
-// next to zero that another order puts on the other side of it, one in 10^7, passes its whole gradient or none of it.
+// after four behind the last whole 16, and the two products meet behind it: the order in which the library behind torch's
+// operators adds at the sizes that library_order below admits, as its results show.  A ReLU's gradient is why that matters: a
+// value next to zero that another order puts on the other side of it, one in 10^7, passes its whole gradient or none of it.
+// (A library that adds in another order leaves both as good as they were, but no longer equal: the tests compare the bits.)
 __global__ __launch_bounds__(kForwardWaves * kWave) void sage_linear_kernel(SageArgs a) {
   constexpr int U = 8;                                  // blocks of eight columns in flight, and as many more on their way
   const int t = threadIdx.x, wave = t / kWave, lane = t & (kWave - 1), at = lane & 15, part = lane >> 4;
@@ -220,6 +221,15 @@ extern "C" int f2cgt_sage_linear(const float* x0, const float* w0, const float* 
   return launch_status(what);
 }
 
+// Where the forward kernel has the library's bits: its order is that of the library's kernels for products of some size.
+// Few rows, few outputs and very large products go to others, which split the columns.  Compared over 1 to 4096 rows, 1 to
+// 600 outputs and every multiple of four up to 128 columns: the products differ at 16 outputs or fewer, at
+// 256 rows or fewer and from 684 000 outputs in all, there not at multiples of 32 up to 256 outputs per row.  Of 300 000
+// sizes drawn from the admitted ones none differs.
+bool library_order(int64_t m, int64_t n, int64_t k0, int64_t k1) {
+  return k0 <= 128 && k1 <= 128 && m > 256 && n > 16 && (m <= (1ll << 19) / n || (m <= 4096 && n <= 256 && n % 32 == 0));
+}
+
 // A tile of 32 outputs reads its rows and weights once per tile of the other side, which a library's larger tiles do half
 // as often: past 131 072 weights that is what the time goes into, in large launches.  Device time of a step forward and
 // backward, operators -> this, us (128 + 128 -> 256 means two inputs of 128 columns and 256 outputs; measured with a forward
@@ -233,7 +243,10 @@ extern "C" int f2cgt_sage_linear(const float* x0, const float* w0, const float* 
 extern "C" int f2cgt_sage_linear_ahead(int64_t m, int64_t n, int64_t k0, int64_t k1) {
   if (m <= 0 || n <= 0 || k0 <= 0 || k1 <= 0 || m >= (1ll << 31) || n >= (1 << 20) || k0 >= (1 << 20) || k1 >= (1 << 20)) return 0;
   const int64_t weights = n * (k0 + k1);
-  return weights <= 131072 || weights <= (1ll << 29) / m ? 1 : 0;
+  int take = 0;
+  if (library_order(m, n, k0, k1)) take |= F2CGT_SAGE_STEP | F2CGT_SAGE_FORWARD;
+  if (m <= 4096 && (weights <= 131072 || weights <= (1ll << 29) / m)) take |= F2CGT_SAGE_GRAD;
+  return take;
 }
 
 extern "C" int64_t f2cgt_sage_linear_grad_workspace_bytes(int64_t m, int64_t n, int64_t k0, int64_t k1) {

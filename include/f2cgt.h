@@ -377,7 +377,13 @@ int64_t f2cgt_sage_linear_grad_workspace_bytes(int64_t m, int64_t n, int64_t k0,
 int f2cgt_sage_linear_grad(const float* grad, const float* out, const float* x0, const float* x1, float* dw0, float* dw1,
                            float* db, void* workspace, int64_t workspace_bytes, int64_t m, int64_t n, int64_t k0, int64_t k1,
                            void* stream);
-/* 1 where the two launches are no slower than a library's products, sum and activation one by one, 0 where they are. */
+/* Which of the two a caller with a library's products beside them takes: bits of F2CGT_SAGE_FORWARD (f2cgt_sage_linear in a
+ * pass that is not differentiated), F2CGT_SAGE_STEP (f2cgt_sage_linear in a pass whose gradients f2cgt_sage_linear_grad makes)
+ * and F2CGT_SAGE_GRAD (f2cgt_sage_linear_grad).  The first two are set only where f2cgt_sage_linear adds in the order in
+ * which rocBLAS and hipBLASLt of ROCm 7.0 were seen to. */
+#define F2CGT_SAGE_FORWARD 1
+#define F2CGT_SAGE_STEP 2
+#define F2CGT_SAGE_GRAD 4
 int f2cgt_sage_linear_ahead(int64_t m, int64_t n, int64_t k0, int64_t k1);
 
 #ifdef __cplusplus

@@ -267,3 +267,20 @@ def test_plain_rows_of_few_edges_stay_with_the_skeleton():
     # 39 of 64 lanes of four columns: up to three
     assert kernel(1000, 3000, 154) == "agg_kernel" and kernel(1000, 3001, 154) == "agg_plain_kernel"
     assert kernel(1000, 9000, 24) == "agg_plain_kernel" and kernel(1000, 9000, 16) == "agg_kernel"
+
+
+def test_which_of_the_dense_layers_kernels_a_size_takes():
+    """Bits: 1 the forward kernel without gradients, 2 with them, 4 the backward kernel."""
+    take = lambda m, n, k0, k1=None: capi.lib().f2cgt_sage_linear_ahead(m, n, k0, k0 if k1 is None else k1)
+    assert take(1024, 256, 128) == take(257, 17, 4) == take(4096, 128, 128) == take(4096, 47, 100) == 7
+    # where the library splits the columns: few rows, few outputs, large products but for outputs in whole tiles
+    assert take(256, 256, 128) == take(1024, 16, 128) == take(4096, 129, 128) == take(1024, 600, 64) == 4
+    assert take(4096, 256, 128) == 7 and take(4096, 256, 64) == 7 and take(4096, 224, 128) == 7 and take(4096, 288, 64) == 4
+    # more columns than one order covers
+    assert take(1024, 256, 132, 4) == take(1024, 256, 4, 132) == 4
+    # many rows: no gradients
+    assert take(4097, 127, 128) == 3 and take(4097, 128, 128) == 0 and take(30840, 17, 128) == 3 and take(30841, 17, 128) == 0
+    assert take(60000, 256, 128) == take(60000, 256, 1000) == 0
+    # wide gradients
+    assert take(4096, 512, 128) == 4 and take(1024, 512, 512) == 4 and take(1025, 512, 512) == 0
+    assert take(0, 1, 4) == take(1, 0, 4) == take(1, 1 << 20, 4) == take(1 << 31, 1, 4) == 0

@@ -229,3 +229,35 @@ def test_subclasses_with_operators_of_their_own_keep_them():
     torch.testing.assert_close(got.as_subclass(torch.Tensor), plain, rtol=1e-5, atol=1e-5)
     parameter = torch.nn.Parameter(w0.detach())      # (a class of its own without operators)
     assert lib.sage_linear(x0, x1, parameter, w1, b, True) is not None
+
+
+# few rows, few outputs, class counts and outputs of no whole tile, more columns than the kernel takes, many rows
+_SHAPES = [(m, k0, k1, n) for m in (1, 2, 33, 100, 256, 257, 300, 1000, 2049, 4096)
+           for n in (1, 5, 16, 17, 40, 41, 47, 128, 172, 256, 349, 600)
+           for k0, k1 in ((128, 128), (116, 84), (100, 4), (52, 96), (36, 16), (8, 12), (132, 64))]
+_MANY = [(m, k, k, n) for m in (4097, 8192, 20000, 30840, 30841, 70000) for n in (8, 17, 47, 64, 128, 256) for k in (128, 100, 36, 600)]
+
+
+@pytest.mark.parametrize("relu", [True, False])
+def test_values_are_the_operators_at_any_size(relu):
+    """Bit for bit, with gradients (where the pass is taken) and without: a kernel that adds in another order than the
+    library's at some size, or a library that does, shows here."""
+    lib = f2cgt_amd.load()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    pool = [torch.randn(max(m * k for m, k, *_ in _MANY), generator=g, device="cuda") for _ in range(2)]
+    weights = [torch.randn(600 * 600, generator=g, device="cuda") / 10 for _ in range(2)]
+    bias = torch.randn(600, generator=g, device="cuda")
+    bad = []
+    for m, k0, k1, n in _SHAPES + _MANY:
+        x0, x1 = pool[0][:m * k0].view(m, k0), pool[1][:m * k1].view(m, k1)
+        w0, w1, b = weights[0][:n * k0].view(n, k0), weights[1][:n * k1].view(n, k1), bias[:n]
+        want = torch.nn.functional.linear(x0, w0, b) + torch.nn.functional.linear(x1, w1)
+        want = torch.relu(want) if relu else want
+        if not torch.equal(lib.sage_linear(x0, x1, w0, w1, b, relu), want):
+            bad.append((m, k0, k1, n))
+        if m <= 4096:
+            out = lib.sage_linear(x0, x1, w0.requires_grad_(), w1, b, relu)
+            if out is not None and not torch.equal(out.detach(), want):
+                bad.append((m, k0, k1, n, "differentiated"))
+    assert not bad
