@@ -230,21 +230,26 @@ bool library_order(int64_t m, int64_t n, int64_t k0, int64_t k1) {
   return k0 <= 128 && k1 <= 128 && m > 256 && n > 16 && (m <= (1ll << 19) / n || (m <= 4096 && n <= 256 && n % 32 == 0));
 }
 
-// A tile of 32 outputs reads its rows and weights once per tile of the other side, which a library's larger tiles do half
-// as often: past 131 072 weights that is what the time goes into, in large launches.  Device time of a step forward and
-// backward, operators -> this, us (128 + 128 -> 256 means two inputs of 128 columns and 256 outputs; measured with a forward
-// kernel that shared the columns among four waves, 6.8 us of the first 25 where this one takes 11):
-//   128 + 128 -> 256: 1024 rows 51 -> 25, 8192 158 -> 59, 60 000 497 -> 314, 120 000 1059 -> 610
-//   256 + 256 -> 256: 1024 rows 54 -> 27, 4096 109 -> 58, 32 000 375 -> 334;  100 + 100 -> 128: 500 rows 103 -> 19
-//   600 + 600 -> 16:  3000 rows 66 -> 35, 60 000 334 -> 241;  1000 + 1000 -> 64: 16 000 rows 311 -> 180
-//   384 + 384 -> 256: 2000 rows 77 -> 53, 8000 168 -> 160, 32 000 456 -> 572
-//   512 + 512 -> 512: 2000 rows 92 -> 97, 8000 226 -> 335;  768 + 768 -> 512: 1000 rows 75 -> 77
-// Up to 2^29 multiply-adds the host's 125 us less a step count for more than what the device loses there.
+// FORWARD, up to 2^27 multiply-adds: a tile of 32 outputs reads its rows and weights once per tile of the other side, which a
+// library's larger tiles do half as often.  Device time of the two products, their sum and the ReLU, operators -> this, us
+// (128 + 128 -> 256 means two inputs of 128 columns and 256 outputs), and what the host takes, 47 -> 5 us:
+//   128 + 128 -> 256: 1024 rows 13.9 -> 10.3, 2048 15.8 -> 17.1, 4096 23.1 -> 31.6, 8192 33 -> 60, 60 000 131 -> 423
+//   128 + 128 -> 128: 1024 rows 12.8 -> 10.0, 4096 17.8 -> 17.2, 8192 21 -> 32;  128 + 128 -> 47: 8192 15.4 -> 13.7
+//   100 + 100 -> 128: 1024 rows 13.0 -> 7.0, 4096 18.4 -> 11.3;  64 + 64 -> 256: 4096 rows 20.0 -> 17.6, 8192 29 -> 33
+// STEP, GRAD: forward and backward, 185 -> 65 us of the host's time with both kernels and 115 with the backward one alone.
+// Device time:
+//   128 + 128 -> 256: 300 rows 102 -> 16, 1024 44 -> 23, 2048 60 -> 33, 4096 93 -> 49;  100 + 100 -> 128: 4096 82 -> 29
+//   the backward kernel behind the library's products: 256 + 256 -> 256: 1024 rows 47 -> 30, 4096 99 -> 57;
+//   600 + 600 -> 16: 1024 38 -> 29, 4096 65 -> 35;  1000 + 1000 -> 64: 1024 56 -> 36, 4096 107 -> 58;
+//   512 + 512 -> 512: 300 rows 49 -> 28, 1024 57 -> 49 (the backward alone 33 -> 25);  384 + 384 -> 256: 2048 65 -> 49
+// Up to 4096 rows: the sums over the rows are closer to float64 than the library's at any size (relative error at
+// 128 + 128 -> 256, 1024 rows 4.4e-7 -> 1.3e-7, 4096 9.0e-7 -> 1.4e-7) and differ from them by the library's error, which grows with
+// the rows (2.1e-6 at 60 000).  Gradients of a layer that is given more rows than that stay bit for bit the operators'.
 extern "C" int f2cgt_sage_linear_ahead(int64_t m, int64_t n, int64_t k0, int64_t k1) {
   if (m <= 0 || n <= 0 || k0 <= 0 || k1 <= 0 || m >= (1ll << 31) || n >= (1 << 20) || k0 >= (1 << 20) || k1 >= (1 << 20)) return 0;
   const int64_t weights = n * (k0 + k1);
   int take = 0;
-  if (library_order(m, n, k0, k1)) take |= F2CGT_SAGE_STEP | F2CGT_SAGE_FORWARD;
+  if (library_order(m, n, k0, k1)) take |= F2CGT_SAGE_STEP | (weights <= (1ll << 27) / m ? F2CGT_SAGE_FORWARD : 0);
   if (m <= 4096 && (weights <= 131072 || weights <= (1ll << 29) / m)) take |= F2CGT_SAGE_GRAD;
   return take;
 }
