@@ -126,7 +126,9 @@ __global__ __launch_bounds__(kGradWaves * kWave) void sage_grad_kernel(SageGradA
   floatx16 acc;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-  float sum = 0.f;
+  // The columns' sums in four chains per lane and pairs of waves: in one chain each they were further from float64 than the
+  // operators' (relative error at 1024 rows 1.33e-7, theirs 1.04e-7, these 0.93e-7; no slower).
+  float sums[4] = {0.f, 0.f, 0.f, 0.f};
   for (int64_t r0 = first + wave * (2 * U); r0 < end; r0 += kGradWaves * 2 * U) {
     float gv[U], ov[U], xv[U];
 #pragma unroll
@@ -142,7 +144,7 @@ __global__ __launch_bounds__(kGradWaves * kWave) void sage_grad_kernel(SageGradA
       const bool in = r0 + 2 * u + side < end;
       float v = in && n_in ? gv[u] : 0.f;
       if (o != nullptr) v = ov[u] <= 0.f ? 0.f : v;        // (as the ReLU's own gradient: a NaN passes it on)
-      sum += v;
+      sums[u & 3] += v;
       acc = __builtin_amdgcn_mfma_f32_32x32x2f32(v, in && k_in ? xv[u] : 0.f, acc, 0, 0, 0);
     }
   }
@@ -150,6 +152,7 @@ __global__ __launch_bounds__(kGradWaves * kWave) void sage_grad_kernel(SageGradA
 #pragma unroll
     for (int v = 0; v < 16; ++v) s_tile[wave - kGradWaves / 2][8 * (v / 4) + 4 * side + v % 4][at] = acc[v];
   }
+  float sum = (sums[0] + sums[1]) + (sums[2] + sums[3]);
   sum += __shfl_xor(sum, 32);
   if (side == 0) s_bias[wave][at] = sum;
   __syncthreads();
@@ -169,10 +172,14 @@ __global__ __launch_bounds__(kGradWaves * kWave) void sage_grad_kernel(SageGradA
     dw[(int64_t)(n0 + r) * k + k0 + c] = v;
   }
   if (bias && t < kTile && n0 + t < a.n && db != nullptr) {
-    float v = s_bias[0][t];
+    float v[kGradWaves];
 #pragma unroll
-    for (int i = 1; i < kGradWaves; ++i) v += s_bias[i][t];
-    db[n0 + t] = v;
+    for (int i = 0; i < kGradWaves; ++i) v[i] = s_bias[i][t];
+#pragma unroll
+    for (int by = 1; by < kGradWaves; by *= 2)
+#pragma unroll
+      for (int i = 0; i < kGradWaves; i += 2 * by) v[i] += v[i + by];
+    db[n0 + t] = v[0];
   }
 }
 

@@ -261,3 +261,19 @@ def test_values_are_the_operators_at_any_size(relu):
             if out is not None and not torch.equal(out.detach(), want):
                 bad.append((m, k0, k1, n, "differentiated"))
     assert not bad
+
+
+@pytest.mark.parametrize("m", [100, 300, 1024, 2000, 4096])
+def test_gradients_are_as_close_to_float64_as_the_operators(m):
+    """Relative error (2-norm), the mean of forty inputs: of the bias's 256 sums and of the weights'."""
+    lib = f2cgt_amd.load()
+    err = torch.zeros((2, 2), dtype=torch.float64, device="cuda")
+    for seed in range(40):
+        x0, x1, w0, w1, b, g = _inputs(m, 8, 8, 256, seed)
+        exact = (g.double().t() @ x0.double(), g.double().sum(0))
+        for i, out in enumerate((lib.sage_linear(x0, x1, w0, w1, b, False),
+                                 torch.nn.functional.linear(x0, w0, b) + torch.nn.functional.linear(x1, w1))):
+            for j, (a, e) in enumerate(zip(torch.autograd.grad(out, (w0, b), g), exact)):
+                err[i, j] += (a.double() - e).norm() / e.norm()
+    # the mean of forty such errors is itself known to about 1 % (256 values each, of spread 1 about their size: 1 / sqrt(2 * 256 * 40))
+    assert bool((err[0] <= 1.01 * err[1]).all()), (err / 40).tolist()
