@@ -38,6 +38,7 @@ namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4_dword __attribute__((ext_vector_type(4), aligned(4)));   // loaded from any float's address
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 
@@ -549,11 +550,11 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
   // >= |c|^2: each of the S leading instructions cuts its 17 addends at 2^-22 of the largest
   // (<= P): 68 S; the small pairs (2^-11 P and below) together stay below 1; the pieces of x and c
   // stop at 2^-22 of the value (4 P each way in these units, on half of P) and the dropped pair is
-  // twice as large: 8; below the smallest normal half 1; the bias sum k + 1; its addition 2; the rounding
+  // as large: 6; below the smallest normal half 1; the bias sum k + 1; its addition 2; the rounding
   // of x - mu and c - mu 4 (L2: 2^-22 (|x|^2 + |c|^2)); 2 spare.  A class is decided by fp32 sums of
   // the same pieces (3 * 8 S roundings of partial sums <= P / 2: 24 S), which stays below.  Doubled
   // for the two scores of a gap.
-  const float unit = 5.9604645e-8f * (float)(2 * (68 * S + k + 19));
+  const float unit = 5.9604645e-8f * (float)(2 * (68 * S + k + 17));
   // Packed minima have to be finite.  An L2 score |c|^2 - 2 x . c is at most 2 (|x|^2 + |c|^2), which may exceed the
   // largest float (3.4e38) while the bound above is finite; cosine has |x . c^| <= |x|, below 2e19 wherever |x|^2 is finite.
   const float finite_below = cosine ? INFINITY : 1.6e38f;
@@ -606,16 +607,17 @@ __global__ __launch_bounds__(assign_threads(S), S <= 3 ? 3 : 2) void assign_kern
     const float x_scale = -pow2(x_shift);
     // what takes a scaled product to -x . c (cosine) or -2 x . c
     const float back = ldexpf(cosine ? 1.f : 2.f, -(x_shift + c_shift));
-    // The leading pieces are cut off, two with one conversion, not rounded: the second ones, which are, then end at 2^-22
-    // of the value (2^-23 behind rounded ones), and the dropped product is twice as large.
+    // The leading pieces, two with one conversion, rounded as one by one (cut off they would leave the second ones to end at
+    // 2^-22 of the value instead of 2^-23, at the same cost).
 #pragma unroll
     for (int st = 0; st < S; ++st)
 #pragma unroll
       for (int e = 0; e < 8; e += 2) {
-        const auto lead = __builtin_amdgcn_cvt_pkrtz(q[st][e] * x_scale, q[st][e + 1] * x_scale);
+        const floatx2 scaled = {q[st][e] * x_scale, q[st][e + 1] * x_scale};
+        const half2v lead = __builtin_convertvector(scaled, half2v);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          xp[st][0][e + i] = (_Float16)lead[i];
+          xp[st][0][e + i] = lead[i];
           xp[st][1][e + i] = (_Float16)__fmaf_rn(q[st][e + i], x_scale, -(float)lead[i]);   // (exact before the rounding)
         }
       }
