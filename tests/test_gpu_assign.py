@@ -151,3 +151,12 @@ def test_rows_whose_squares_vanish_keep_their_direction(power, k):
     # (3e-4: what rows of 2^-130 have left of their values, and products of theirs)
     assert (d[np.arange(700), got] - d.min(1))[~zero].max() < 3e-4
     assert (got[zero] == 0).all()                   # a row of zeros is as far from every centre
+
+
+@pytest.mark.parametrize("metric", ["cosine", "l2"])
+@pytest.mark.parametrize("m", [1, 31, 33, 70])
+def test_rows_at_the_end_of_a_table_at_every_width(metric, m):
+    """The last groups' rows, whose ends are read from inside the row: every length of the chunk of eight that a row ends in."""
+    rng = np.random.default_rng(m)
+    for k in range(1, 65):
+        check(rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((70, k)).astype(np.float32), metric)
