@@ -1191,33 +1191,14 @@ int launch_wave_trace(const VqArgs& a, const void* indptr, const void* indices, 
 }
 #endif
 
-// What the plan of a launch reports beside its geometry (form, owners): the class of the launch by what binds it, which
-// selected between four ways of writing the output; all of them are the lane swap of vq_wave_kernel now.  1: up to 8
-// edges per row, tables beyond the last-level cache at 128, 256 and 512 columns and large outputs next to tables of 64 to
-// 192 MB; 4: large outputs and up to 11 edges per row from smaller tables; 0: the others, owners 2 with codebooks of
-// 32 columns.
-void plan_store_class(const VqArgs& a, bool rpm4, double avg_deg, int& form, int& owners) {
-  const int64_t out_bytes = a.R * (int64_t)a.feat_dim * 4, table = a.N * (int64_t)a.n_cb;
-  const bool lines = (a.feat_dim == 128 && out_bytes >= (60ll << 20)) ||
-                     (a.feat_dim == 256 && out_bytes >= (60ll << 20) && out_bytes <= (160ll << 20) && avg_deg <= 10.0) ||
-                     (a.feat_dim == 512 && out_bytes >= (96ll << 20) && avg_deg <= 11.0);
-  form = avg_deg <= 8.0;
-  if (!form && a.feat_dim % 8 == 0 && rpm4) {
-    if (store_mode() == F2CGT_STORE_STREAM || (table > (256ll << 20) && lines)) {
-      form = 1;
-    } else if (table <= (192ll << 20) && a.feat_dim >= 128 && a.n_tiles <= 4) {
-      const bool big_out = out_bytes >= (200ll << 20);
-      form = big_out && table >= (64ll << 20) ? 1 : (big_out || avg_deg <= 11.0 ? 4 : 0);
-    }
-  }
-  owners = form == 0 && a.w == 32 && a.feat_dim % 32 == 0 && a.feat_dim >= 128 && rpm4 && table <= (192ll << 20) ? 2 : 0;
-}
-
 template <int BT, int H, int RPM>
 int launch_wave(const VqArgs& a, const void* indptr, const void* indices, int idx_dtype, float* out, hipStream_t st,
-                const char* what, unsigned grid, size_t wlds, int form = 0, int owners = 0) {
+                const char* what, unsigned grid, size_t wlds) {
+  const bool tail = a.n_cb % BT != 0 || !aligned(a.codes, BT);
+  constexpr bool CAN_EVEN2 = H == 1 && RPM == 4;   // even widths that are no multiple of 4
+  const bool even2 = CAN_EVEN2 && a.feat_dim % 4 != 0;
   if (plan_only()) {
-    plan_record("vq_wave_kernel", grid, kThreads, (int64_t)wlds, 0, H, RPM, form, owners);
+    plan_record("vq_wave_kernel", grid, kThreads, (int64_t)wlds, 0, H, RPM, even2, tail);
     return 0;
   }
 #ifdef F2CGT_EXPERIMENTS
@@ -1225,11 +1206,9 @@ int launch_wave(const VqArgs& a, const void* indptr, const void* indices, int id
     if (a.store_late == 9 && a.trace) return launch_wave_trace<BT>(a, indptr, indices, out, st, what, grid, wlds);
   }
 #endif
-  const bool tail = a.n_cb % BT != 0 || !aligned(a.codes, BT);
   const bool i32 = idx_dtype == F2CGT_DT_I32;
-  constexpr bool CAN_EVEN2 = H == 1 && RPM == 4;   // even widths that are no multiple of 4
   const void* kern;
-  if (CAN_EVEN2 && a.feat_dim % 4 != 0)
+  if (even2)
     kern = tail ? (i32 ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, true, CAN_EVEN2>)
                        : reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int64_t, true, CAN_EVEN2>))
                 : (i32 ? reinterpret_cast<const void*>(vq_wave_kernel<BT, H, RPM, int32_t, false, CAN_EVEN2>)
@@ -1274,8 +1253,6 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
   const bool rpm4 = avg_deg <= 16.0 * ((a.R > 0 && a.E % a.R == 0) ? 1.0 : 0.9);
   const int64_t out_bytes = a.R * (int64_t)a.feat_dim * 4;
   const bool big_table = a.N * (int64_t)a.n_cb > (256ll << 20);
-  int form = 0, owners = 0;
-  plan_store_class(a, rpm4, avg_deg, form, owners);
 #ifdef F2CGT_EXPERIMENTS
   {
     if (const char* d = getenv("F2CGT_VQ_DEFER")) a.store_late = atoi(d);
@@ -1334,7 +1311,7 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
                             (avg_deg <= 8.0 || (rpm4 && filled && out_bytes >= (a.n_tiles > 4 || big_table ? 100000000ll : 256ll << 20)));
     if (split_rows) return launch_wave<BT, 1, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
     if (avg_deg <= 16.0 * fit)
-      return launch_wave<BT, 2, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds, form, owners);
+      return launch_wave<BT, 2, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
     if (avg_deg <= 32.0 * fit) return launch_wave<BT, 2, 2>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
     return launch_wave<BT, 2, 1>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
   } else if (avg_deg <= 15.0 || a.n_cb % BT != 0 || !aligned(a.codes, BT) || a.feat_dim % 4 != 0) {

@@ -81,8 +81,9 @@ int f2cgt_set_store_mode(int mode);
  * the device or dereferencing any pointer (pointers only need the alignment of the real buffers;
  * the device is taken to have 256 compute units).  f2cgt_last_plan copies the last choice:
  * grid / block / lds_bytes of the launch, destination rows per workgroup (0 = not row-blocked),
- * and kernel-specific lane-group counts in aux[] (every one of them must be >= 1 for the kernel's
- * loops to advance).  f2cgt_set_plan_only returns the previous setting. */
+ * and kernel-specific numbers in aux[]: lane-group counts (every one of them must be >= 1 for the kernel's
+ * loops to advance); of vq_wave_kernel the float4 per lane and edge, the rows of a mini-block, 1 where the columns are no
+ * multiple of four and 1 where codes are read byte by byte.  f2cgt_set_plan_only returns the previous setting. */
 typedef struct {
   char kernel[48];
   int64_t grid;

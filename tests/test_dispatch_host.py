@@ -148,86 +148,68 @@ def test_rows_per_block_follow_the_launch_size():
     assert rc == 0 and plan.rows_per_block == 8
 
 
-def test_fused_vq_store_form_by_shape():
-    """aux[2] of a vq_wave_kernel plan is the store form: 1 = results turned round in LDS (up to 8 edges per row, and up
-    to 16 for an output of 200 MB and more from a code table of 64 to 192 MB, or throughout in the streaming store mode),
-    4 = halves exchanged inside lane quads (a cached table: up to 11 edges per row, or a large output), 0 = stored as they
-    are; aux[3] is the binary logarithm of the number of lanes that own the columns of a code together (2 for
-    codebooks of 32 columns from a cached table where neither of the other forms is taken)."""
-    def form(rows, fanout, d, n_cb, w, n_src):
-        rc, plan = capi.dry_run("f2cgt_vq_decompress_spmm_csr", A16, capi.DT_U8, A16, A16, A16, capi.DT_I64, A16, rows,
-                                rows * fanout, n_src, d, n_cb, 256, w, None)
-        assert rc == 0 and plan.kernel.decode() == "vq_wave_kernel"
-        return plan.aux[2], plan.aux[3]
-    assert form(300_000, 5, 128, 16, 8, 1_000_000) == (1, 0)
-    assert form(300_000, 5, 128, 4, 32, 1_000_000) == (1, 0)
-    assert form(300_000, 10, 128, 16, 8, 1_000_000) == (4, 0)
-    assert form(150_000, 10, 256, 16, 16, 1_000_000) == (4, 0)
-    assert form(300_000, 10, 256, 16, 16, 1_000_000) == (4, 0)      # 307 MB of output from 16 MB of codes
-    assert form(300_000, 14, 256, 16, 16, 1_000_000) == (4, 0)
-    assert form(300_000, 14, 256, 16, 16, 10_000_000) == (1, 0)     # from 160 MB of codes
-    assert form(100_000, 14, 256, 16, 16, 1_000_000) == (0, 0)
-    assert form(300_000, 10, 512, 16, 32, 1_000_000) == (4, 0)
-    assert form(100_000, 14, 512, 16, 32, 1_000_000) == (0, 2)
-    assert form(200_000, 10, 768, 24, 32, 1_000_000) == (0, 2)       # six column tiles
-    assert form(500_000, 15, 128, 16, 8, 10_000_000) == (1, 0)      # 256 MB of output from a 160 MB table
-    assert form(100_000, 15, 128, 16, 8, 10_000_000) == (0, 0)      # 51 MB of output: the halves meet in the cache
-    assert form(600_000, 10, 768, 24, 32, 240_000_000) == (0, 0)    # a 5.8 GB table: the gather dominates
-    assert form(200_000, 10, 768, 96, 8, 1_000_000) == (0, 0)       # six column tiles
-    assert form(300_000, 10, 64, 8, 8, 1_000_000) == (0, 0)         # half the lanes of a row beyond the columns
-    assert form(300_000, 20, 128, 16, 8, 1_000_000) == (0, 0)       # two-row mini-blocks
-    assert form(300_000, 20, 128, 4, 32, 1_000_000) == (0, 0)
-    assert form(300_000, 10, 600, 19, 32, 1_000_000) == (0, 0)      # 600 columns: the last tile ends inside a group of 32
-    assert form(300_000, 10, 100, 13, 8, 1_000_000)[1] == 0         # four columns per lane: dense as they are
-    was = capi.set_store_mode(capi.STORE_STREAM)
-    try:
-        assert form(600_000, 10, 768, 24, 32, 240_000_000) == (1, 0)
-        assert form(300_000, 10, 128, 16, 8, 1_000_000) == (1, 0)
-        assert form(300_000, 20, 128, 16, 8, 1_000_000) == (0, 0)
-    finally:
-        capi.set_store_mode(was)
-    # aux[0]: float4 per lane and edge (2 = a lane owns eight columns); sparse rows that are no whole 128-byte lines
-    # take one, code rows that are no multiple of a tile (24 x 8, 7 x 32) can take the turn through LDS
-    lanes = lambda rows, fanout, d, n_cb, w: capi.dry_run(
-        "f2cgt_vq_decompress_spmm_csr", A16, capi.DT_U8, A16, A16, A16, capi.DT_I64, A16, rows, rows * fanout,
-        1_000_000, d, n_cb, 256, w, None)[1].aux[0]
-    assert lanes(1_000_000, 3, 200, 25, 8) == 1 and lanes(300_000, 10, 200, 25, 8) == 2
-    assert lanes(1_000_000, 3, 192, 24, 8) == 2 and form(1_000_000, 3, 192, 24, 8, 1_000_000) == (1, 0)
-    assert lanes(1_000_000, 3, 224, 7, 32) == 2 and lanes(1_000_000, 3, 600, 19, 32) == 1
+def plan_vq(rows, fanout, d, n_cb, w, n_src, edges=None, codes=A16):
+    rc, plan = capi.dry_run("f2cgt_vq_decompress_spmm_csr", codes, capi.DT_U8, A16, A16, A16, capi.DT_I64, A16, rows,
+                            rows * fanout if edges is None else edges, n_src, d, n_cb, 256, w, None)
+    assert rc == 0
+    return plan
 
 
-def test_fused_vq_forms_for_tables_beyond_the_last_level_cache_and_rows_of_split_pieces():
-    def plan(rows, fanout, d, n_cb, w, n_src):
-        rc, p = capi.dry_run("f2cgt_vq_decompress_spmm_csr", A16, capi.DT_U8, A16, A16, A16, capi.DT_I64, A16, rows,
-                             rows * fanout, n_src, d, n_cb, 256, w, None)
-        assert rc == 0 and p.kernel.decode() == "vq_wave_kernel"
-        return p.aux[0], p.aux[2]          # float4 per lane and edge, store form
-    # a table of more than 256 MB: through LDS where that is ahead with any ids, warm and in turn
-    assert plan(122_880, 15, 128, 16, 8, 16_777_217) == (2, 1)      # 60 MB
-    assert plan(122_879, 15, 128, 16, 8, 16_777_217) == (2, 0)
-    assert plan(122_880, 15, 128, 16, 8, 16_777_216) == (2, 0)
-    assert plan(122_880, 17, 128, 16, 8, 16_777_217) == (2, 0)
-    assert plan(61_440, 10, 256, 16, 16, 20_000_000) == plan(163_840, 10, 256, 32, 8, 20_000_000) == (2, 1)   # 60 to 160 MB
-    assert plan(61_439, 10, 256, 16, 16, 20_000_000) == plan(163_841, 10, 256, 16, 16, 20_000_000) == (2, 0)
-    assert plan(100_000, 11, 256, 16, 16, 20_000_000) == (2, 0)
-    assert plan(49_152, 11, 512, 16, 32, 20_000_000) == plan(400_000, 9, 512, 64, 8, 5_000_000) == (2, 1)
-    assert plan(49_151, 11, 512, 16, 32, 20_000_000) == plan(49_152, 12, 512, 16, 32, 20_000_000) == (2, 0)
+def test_fused_vq_lane_layout_by_shape():
+    """aux of a vq_wave_kernel plan: float4 per lane and edge (2: a row has sixteen lanes of eight columns, 1: 32 of four),
+    rows of a mini-block, columns that are no multiple of four, codes read byte by byte.  The output is written in one way
+    per layout, whatever the table, the output's size and the store mode."""
+    def layout(*args, **kw):
+        plan = plan_vq(*args, **kw)
+        assert plan.kernel.decode() == "vq_wave_kernel"
+        return tuple(plan.aux)
+    eight = (2, 4, 0, 0)
+    shapes = [(300_000, 5, 128, 16, 8, 1_000_000), (300_000, 10, 128, 16, 8, 1_000_000), (300_000, 5, 128, 4, 32, 1_000_000),
+              (300_000, 14, 256, 16, 16, 10_000_000), (100_000, 14, 512, 16, 32, 1_000_000), (500_000, 15, 128, 16, 8, 10_000_000),
+              (600_000, 10, 768, 24, 32, 240_000_000), (122_880, 15, 128, 16, 8, 16_777_217), (49_152, 11, 512, 16, 32, 20_000_000)]
+    for mode in (capi.STORE_AUTO, capi.STORE_STREAM, capi.STORE_CACHED):
+        was = capi.set_store_mode(mode)
+        try:
+            for shape in shapes:
+                assert layout(*shape) == eight, shape
+        finally:
+            capi.set_store_mode(was)
+    # rows of a mini-block: rows of one length up to 16 / 32 edges, ragged ones up to 0.9 of that
+    assert [layout(100_000, f, 128, 16, 8, 1_000_000)[1] for f in (16, 17, 32, 33, 200)] == [4, 2, 2, 1, 1]
+    assert [layout(100_000, 0, 128, 16, 8, 1_000_000, edges=e)[1] for e in (1_439_999, 1_440_001, 2_879_999, 2_880_001)] == [4, 2, 2, 1]
+    # widths that are no multiple of eight: one float4 per lane; of two columns over; the block kernel for long rows of
+    # whole code words
+    assert layout(300_000, 10, 100, 25, 8, 1_000_000) == (1, 4, 0, 1) and layout(300_000, 10, 124, 16, 8, 1_000_000) == (1, 4, 0, 0)
+    assert layout(300_000, 10, 602, 19, 32, 1_000_000) == (1, 4, 1, 1) and layout(300_000, 40, 602, 19, 32, 1_000_000)[:2] == (1, 4)
+    assert plan_vq(300_000, 16, 124, 16, 8, 1_000_000).kernel.decode() == "vq_pipe_kernel"
+    # codes read byte by byte: rows of codes that are no whole words, or not aligned to them
+    assert layout(300_000, 10, 192, 24, 8, 1_000_000) == (2, 4, 0, 1)
+    assert layout(300_000, 10, 128, 16, 8, 1_000_000, codes=ctypes.c_void_p((1 << 20) + 8)) == (2, 4, 0, 1)
+    # odd multiples of eight columns in several tiles, few edges: one float4 per lane
+    lanes = lambda *args: layout(*args)[0]
+    assert lanes(1_000_000, 3, 200, 25, 8, 1_000_000) == 1 and lanes(300_000, 10, 200, 25, 8, 1_000_000) == 2
+    assert lanes(1_000_000, 3, 192, 24, 8, 1_000_000) == 2 and lanes(1_000_000, 3, 64, 8, 8, 1_000_000) == 2
+    assert lanes(1_000_000, 3, 224, 7, 32, 1_000_000) == 2 and lanes(1_000_000, 3, 600, 19, 32, 1_000_000) == 1
+
+
+def test_fused_vq_rows_of_split_pieces():
+    lanes = lambda *args: plan_vq(*args).aux[0]
     for dim in (160, 192, 224, 304, 320, 384, 416, 448, 480, 544, 768):
-        assert plan(300_000, 10, dim, dim // 8, 8, 20_000_000) == (2, 0)
+        assert lanes(300_000, 10, dim, dim // 8, 8, 20_000_000) == 2
     # odd multiples of eight columns: one float4 per lane
-    assert plan(41_667, 12, 600, 19, 32, 1_000_000) == (1, 0)
-    assert plan(41_666, 12, 600, 19, 32, 1_000_000) == (2, 0)
-    assert plan(41_667, 13, 600, 19, 32, 1_000_000) == (2, 0)
-    assert plan(41_667, 16, 600, 19, 32, 15_000_000) == (1, 0)
+    assert lanes(41_667, 12, 600, 19, 32, 1_000_000) == 1
+    assert lanes(41_666, 12, 600, 19, 32, 1_000_000) == 2
+    assert lanes(41_667, 13, 600, 19, 32, 1_000_000) == 2
+    assert lanes(41_667, 16, 600, 19, 32, 15_000_000) == 1
     # a last tile of few columns leaves the lanes of its workgroups idle
     for dim, up_to in ((136, 8), (152, 8), (168, 12), (200, 12), (216, 16), (264, 8), (280, 8), (296, 12), (328, 12), (360, 16),
                        (392, 12), (456, 16), (504, 16), (520, 12), (568, 16), (648, 12), (712, 16), (760, 16)):
-        forms = [plan(300_000, fanout, dim, -(-dim // 8), 8, 30_000_000)[0] for fanout in (8, 9, 12, 13, 16, 17)]
+        forms = [lanes(300_000, fanout, dim, -(-dim // 8), 8, 30_000_000) for fanout in (8, 9, 12, 13, 16, 17)]
         assert forms == [1 if fanout <= up_to else 2 for fanout in (8, 9, 12, 13, 16, 17)], dim
-    assert plan(335_545, 12, 200, 25, 8, 1_000_000)[0] == 1 and plan(335_544, 12, 200, 25, 8, 1_000_000)[0] == 2
-    assert plan(125_000, 12, 200, 25, 8, 12_000_000)[0] == 1
-    assert plan(700_000, 9, 104, 13, 8, 1_000_000)[0] == 2          # one column tile
-    assert plan(400_000, 12, 208, 26, 8, 1_000_000)[0] == 2         # whole 64-byte pieces
+    assert lanes(335_545, 12, 200, 25, 8, 1_000_000) == 1 and lanes(335_544, 12, 200, 25, 8, 1_000_000) == 2
+    assert lanes(125_000, 12, 200, 25, 8, 12_000_000) == 1
+    assert lanes(700_000, 9, 104, 13, 8, 1_000_000) == 2          # one column tile
+    assert lanes(400_000, 12, 208, 26, 8, 1_000_000) == 2         # whole 64-byte pieces
 
 
 def test_dealt_items_and_column_form_of_one_codebook():

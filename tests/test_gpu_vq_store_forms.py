@@ -1,4 +1,5 @@
-"""The fused VQ operator where the store form goes by the size of table and output, against decode + spmm_csr."""
+"""The fused VQ operator with tables and outputs around the size of the last-level cache, and rows of split pieces, against
+decode + spmm_csr."""
 import pytest
 import torch
 
