@@ -357,7 +357,7 @@ __global__ __launch_bounds__(kThreads) void vq_wave_kernel(VqArgs a, const Idx* 
   extern __shared__ __align__(16) unsigned char smem[];
   float* s_cb = reinterpret_cast<float*>(smem);
   const int wave = uni((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-  constexpr int kStage = kWEdges * BT > 1024 ? kWEdges * BT : 1024;     // code bytes of a mini-block, or 64 float4
+  constexpr int kStage = kWEdges * BT;          // code bytes of a mini-block
   unsigned char* s_codes = smem + (size_t)a.K * 128 * 4 + (size_t)wave * kStage;
   int* s_ptr = reinterpret_cast<int*>(smem + (size_t)a.K * 128 * 4 + (size_t)kWaves * kStage) + wave * 2 * kWPtr;
 
@@ -1248,7 +1248,7 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
   // The wave-granular kernel: 4-row mini-blocks up to 16 edges per row, and, with whole 8-column
   // groups in every tile (one lane per group, two float4 per edge), 2-row mini-blocks up to 32 and
   // 1-row ones beyond (larger mini-blocks for sparse rows were tried and were slower than 4-row ones).
-  const size_t wlds = (size_t)a.K * 128 * 4 + (size_t)(kThreads / 64) * (kWEdges * BT > 1024 ? kWEdges * BT : 1024) +
+  const size_t wlds = (size_t)a.K * 128 * 4 + (size_t)(kThreads / 64) * kWEdges * BT +
                       (size_t)(kThreads / 64) * 2 * kWPtr * 4;
   const bool rpm4 = avg_deg <= 16.0 * ((a.R > 0 && a.E % a.R == 0) ? 1.0 : 0.9);
   const int64_t out_bytes = a.R * (int64_t)a.feat_dim * 4;
