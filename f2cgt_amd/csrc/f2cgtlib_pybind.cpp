@@ -196,8 +196,6 @@ torch::Tensor sq_encode(torch::Tensor src, torch::Tensor codebooks, int64_t targ
   return out;
 }
 
-// Extension: order statistics, sum and flags (1: a NaN, 2: a row id outside the table) of |x| per column slice of the rows
-// `rows` (None: all of them), for the codebooks of sq_encode.  ranks: four ranks in a full slice, four in the last one.  -> float64 [n_slices, 6] on the GPU.
 // A flag in pinned memory that a kernel may still set, and the event behind that kernel.
 class PendingFlag {
  public:
@@ -227,6 +225,10 @@ class PendingFlag {
   hipEvent_t event_ = nullptr;
 };
 
+// Extension: order statistics, sum and flags (1: a NaN, 2: a row id outside the table) of |x| per column slice of the rows
+// `rows` (None: all of them), for the codebooks of sq_encode.  ranks: four ranks in a full slice, four in the last one.
+// -> (float64 [n_slices, 6], the codebooks fp32 [n_slices, 5] where weights are given), on the GPU; pending: the check of the
+// row ids, on its way to the host.
 std::tuple<torch::Tensor, torch::Tensor> order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
                                                      const std::vector<int64_t>& ranks, const std::vector<float>* weights,
                                                      std::shared_ptr<PendingFlag>* pending = nullptr) {
@@ -491,11 +493,8 @@ torch::Tensor keep_rows(torch::Tensor norms, torch::Tensor stats, double weight,
 
 bool kmeans_slices_covers(int64_t slices, int64_t n, int64_t k) { return f2cgt_kmeans_slices_covers(slices, n, k) != 0; }
 
-// Lloyd iterations of all slices on x [slices, m, k] from `centers` [slices, n, k] (updated in place), until every slice
-// has met `rule` or for max_iter steps; tol grows by `growth` each step.  The flags are read every check_every steps and
-// at the end.  -> int32 [slices] on the host: 0 not met, 1 met, 2 the shift became NaN, 3 no rows.
-// The loop of kmeans_slices_fit on flags[0, slices), which it leaves on the device; true where a read-back found them all set.
-bool fit_slices(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, const std::string& metric, int64_t rule,
+// The loop of kmeans_slices_fit, on flags[0, slices), which it leaves on the device.
+void fit_slices(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, const std::string& metric, int64_t rule,
                 double tol, double growth, int64_t max_iter, int64_t check_every, torch::Tensor& flags) {
   x = dev_contig(x, "x");
   TORCH_CHECK(x.dim() == 3 && x.scalar_type() == torch::kFloat32, "x must be float32 [slices, m, k]");
@@ -527,13 +526,15 @@ bool fit_slices(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tenso
       const int32_t* f = seen.data_ptr<int32_t>();
       bool all = true;
       for (int64_t s = 0; s < slices; ++s) all = all && f[s] != 0;
-      if (all) return true;
+      if (all) return;
     }
   }
-  return false;
 }
 
-// -> the stop flags, int32 [slices] on the host.  rescale: the centres are also rescaled to their slice's mean length, and
+// Lloyd iterations of all slices on x [slices, m, k] from `centers` [slices, n, k] (updated in place), until every slice
+// has met `rule` or for max_iter steps; tol grows by `growth` each step.  The flags are read every check_every steps and
+// at the end.  -> the stop flags, int32 [slices] on the host: 0 not met, 1 met, 2 the shift became NaN, 3 no rows.
+// rescale: the centres are also rescaled to their slice's mean length, and
 // the result is (flags int32 [slices + 2] on the host: the stop flags, bad_row's word, 1 where a value is no number;
 // codebooks fp32 [slices, n, k]), with one wait for all of it.
 py::object kmeans_slices_fit(torch::Tensor x, c10::optional<torch::Tensor> keep, torch::Tensor centers, std::string metric,
