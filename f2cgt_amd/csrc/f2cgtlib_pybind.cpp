@@ -285,6 +285,8 @@ torch::Tensor abs_order_stats(torch::Tensor x, c10::optional<torch::Tensor> rows
 // PendingFlag.
 std::tuple<torch::Tensor, py::object> sq_codebooks(torch::Tensor x, c10::optional<torch::Tensor> rows, int64_t column_slice,
                                                    const std::vector<int64_t>& ranks, const std::vector<float>& weights) {
+  TORCH_CHECK(x.defined() && x.device().is_cuda(), "x must be a GPU tensor");
+  c10::DeviceGuard guard(x.device());      // the stream that is asked below is the one that is worked on
   std::shared_ptr<PendingFlag> pending;
   const bool check = rows.has_value() && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
   auto both = order_stats(x, rows, column_slice, ranks, &weights, check ? &pending : nullptr);
