@@ -606,7 +606,7 @@ class CompressionManager:
         seeds = self.seeds_data
         in_one = (self.methods[0] == "sq" and seeds.data.is_cuda and not seeds.has_cache and
                   seeds_key.dtype in (torch.int32, torch.int64))
-        if in_one and self.check_seed_keys:
+        if in_one and self.check_seed_keys and seeds_key.is_cuda:     # (keys on the host are refused below)
             seeds_feature = self._decode_seeds(seeds_key)
             self.seeds_task_event.record()
             return seeds_feature

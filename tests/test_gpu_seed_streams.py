@@ -77,3 +77,13 @@ def test_rows_for_several_threads(manager):
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("check", [True, False])
+def test_keys_on_the_host_are_refused(manager, check):
+    manager.check_seed_keys = check
+    try:
+        with pytest.raises(RuntimeError):
+            manager.get_seeds_data(manager.keys[:10].cpu())
+    finally:
+        manager.check_seed_keys = True
