@@ -39,6 +39,8 @@ struct VqArgs {
   int n_cb, K, w, feat_dim;
   int n_tiles, n_stripes;
   int stripes_per_xcd;  // > 0: the column tiles of a stripe share one XCD (see the kernel)
+  int in_step;          // workgroups of a half column tile store twice, so that they do not run ahead of the full tiles'
+  int pause;            // a wave sleeps before it stores (see launch_vq)
   int probe_stores;     // experiments build only: 2 = the launch without its stores; the strip kernel's store form
   int store_late;       // experiments build only: 9 = the time-stamped form of the wave kernel
   unsigned long long* trace;   // experiments build only: per wave {start, first step, end} in 100 MHz ticks
@@ -428,7 +430,7 @@ __global__ __launch_bounds__(kThreads) void vq_wave_kernel(VqArgs a, const Idx* 
     const uint32_t lo = k < groups ? at : kNowhere, hi = k + 8 < groups ? at + 256u : kNowhere;
     put_a = (half & 1) ? hi : lo;
     put_b = (half & 1) ? lo : hi;
-    if (groups <= 8) { put_a = lo; put_b = kNowhere; }
+    if (groups <= 8) { put_a = lo; put_b = a.in_step ? lo : kNowhere; }
   }
   const bool half_group = EVEN2 && (tile_cols_out & 2) && lane_col == groups - 1;
   if (EVEN2 && half_group && tile_cols_out >= 4) put_a -= 8u;
@@ -774,8 +776,9 @@ __global__ __launch_bounds__(kThreads) void vq_wave_kernel(VqArgs a, const Idx* 
           }
           if (groups <= 8) {   // one piece per row: all four rows' in the first store
 #pragma unroll
-            for (int t = 0; t < 4; ++t) va[t] = (half & 1) ? vb[t] : va[t];
+            for (int t = 0; t < 4; ++t) va[t] = vb[t] = (half & 1) ? vb[t] : va[t];
           }
+          if (a.pause) __builtin_amdgcn_s_sleep(6);
           store_at4(obase, row_b + put_a, va[0], va[1], va[2], va[3]);
           store_at4(obase, row_b + put_b, vb[0], vb[1], vb[2], vb[3]);
         } else if constexpr (SPR > 1) {
@@ -1309,6 +1312,21 @@ int launch_vq(VqArgs a, const void* indptr, const void* indices, int idx_dtype, 
     const bool filled = avg_deg <= 12.0 ? tail >= 40 || a.n_tiles > 3 : big_table && tail >= (a.n_tiles > 3 ? 56 : 80);
     const bool split_rows = a.feat_dim % 16 == 8 && a.n_tiles > 1 &&
                             (avg_deg <= 8.0 || (rpm4 && filled && out_bytes >= (a.n_tiles > 4 || big_table ? 100000000ll : 256ll << 20)));
+    // Large outputs of several column tiles, rows of one length and few edges: the tiles of a stripe read the same code
+    // rows, and only while their workgroups stay within a few microseconds of each other does one of them fetch a line for
+    // all.  Bound by their stores they drift apart, which slower stores, turned round in LDS, kept them from before the lane
+    // swap.  Those / the swap alone / with one of two brakes, us, outputs of 640 MB, 2e6 source rows in codes of 16 columns,
+    // uniform ids (skewed ones):
+    //   a last tile of up to 64 columns stores its pieces twice, so that its workgroups do not run ahead: 192 columns, 4 edges
+    //   174 / 195 / 175 (166 / 157 / 160), 6 edges 199 / 239 / 199 (175 / 162 / 162); 288, 6 edges 189 / 203 / 174; 160,
+    //   5 edges 199 / 251 / 228 (185 / 172 / 175)
+    //   whole tiles sleep 384 clocks before the stores of a step: 640 columns, 2 edges 126 / 130 / 121 (123 / 132 / 117), 4
+    //   edges 135 / 130 / 132 (133 / 123 / 131); 384, 3 edges in another run 120 / 129 / 119 (118 / 133 / 117); 512, 3 edges
+    //   123 / 130 / 128 (123 / 136 / 130)
+    // Ragged rows, outputs of 150 MB and more than 8 edges are ahead as they are.
+    const bool drifts = a.n_tiles > 1 && a.E % a.R == 0 && out_bytes >= (256ll << 20);
+    a.in_step = drifts && tail > 0 && tail <= 64 && avg_deg >= (a.n_tiles == 2 ? 3.0 : 5.0) && avg_deg <= 8.0 ? 1 : 0;
+    a.pause = drifts && tail == 0 && avg_deg >= 2.0 && avg_deg <= 5.0 ? 1 : 0;
     if (split_rows) return launch_wave<BT, 1, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);
     if (avg_deg <= 16.0 * fit)
       return launch_wave<BT, 2, 4>(a, indptr, indices, idx_dtype, out, st, what, grid, wlds);

@@ -13,7 +13,11 @@ pytestmark = pytest.mark.gpu
                                                                (3000, 25, 8, 200, 335_545, 10), (16_777_217, 16, 8, 128, 65_537, 15),
                                                                (16_777_217, 25, 8, 200, 125_001, 12), (16_777_217, 27, 8, 216, 115_741, 13),
                                                                (16_777_217, 16, 8, 128, 122_881, 15), (16_777_217, 17, 16, 256, 61_441, 10),
-                                                               (8_388_609, 33, 16, 512, 49_153, 11), (16_777_217, 25, 8, 200, 125_001, 13)])
+                                                               (8_388_609, 33, 16, 512, 49_153, 11), (16_777_217, 25, 8, 200, 125_001, 13),
+                                                               # large outputs of few edges per row: half a last tile, whole tiles
+                                                               (3000, 12, 16, 192, 349_526, 3), (3000, 24, 8, 192, 349_527, 8),
+                                                               (3000, 14, 32, 448, 149_799, 5), (3000, 11, 16, 176, 381_303, 6),
+                                                               (3000, 24, 16, 384, 174_763, 3), (3000, 16, 16, 256, 262_145, 5)])
 @pytest.mark.parametrize("ragged", [False, True])
 def test_store_forms_agree_with_the_unfused_operators(n_src, books, width, dim, rows, fanout, ragged):
     capi = f2cgt_amd.load()
