@@ -1039,8 +1039,8 @@ __device__ __forceinline__ void add_signs(float (&s)[8], uint32_t byte, const un
 // with the store form fixed at compile time the row loop came out 3-5 % faster at 100-256 columns and 17-19 % at 600
 // (3e6 edges, 10 per row, 4 bit: 97.8 -> 93.7 us at 128 columns, 592 -> 489 us at 600); 1- and 2-bit rows measured
 // level to 2 % slower and keep the run-time test.
-// ITEM: 0 (a lane keeps a column group), or the columns of the items that are dealt to the lanes: 4 (staged codes), or 8
-// (codes read where they are).  The eight columns of such an item are stored after the two halves of the wave have exchanged theirs
+// ITEM: 0 (a lane keeps a column group), or the columns of the items that are dealt to the lanes: 4 (staged codes, and short
+// launches of 8-bit rows), or 8 (codes read where they are).  The eight columns of such an item are stored after the two halves of the wave have exchanged theirs
 // (v_permlane32_swap): the lower lanes' items go out with one store instruction, 16 bytes per lane one after the other,
 // the upper lanes' with the next, where a lane's own two 16-byte stores would each write 16 of every 32 bytes.
 template <int BITS, bool AFFINE, typename Idx, int TB, int HALF = 0, int ITEM = 0>
@@ -1277,7 +1277,7 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
         const uint8_t* q = a.codes + ((uint64_t)id * (uint32_t)a.src_dim + at);
         if constexpr (GB == 1) return (uint32_t)*q;
         uint32_t w = 0;
-        __builtin_memcpy(&w, q, GB);
+        __builtin_memcpy(&w, q, GB < 4 ? GB : 4);
         return w >> sh;
       };
       auto add = [&](uint32_t w) {
@@ -1300,7 +1300,8 @@ __global__ __launch_bounds__(TB) void sq_rows_kernel(RowsArgs a, const Idx* __re
       if (staged) {
         walk([&](int k) -> uint32_t {
           const unsigned char* q = s_codes + k * a.pitch + first;
-          if constexpr (GB == 2) return *reinterpret_cast<const uint16_t*>(q);
+          if constexpr (GB == 4) return *reinterpret_cast<const uint32_t*>(q);
+          else if constexpr (GB == 2) return *reinterpret_cast<const uint16_t*>(q);
           else return (uint32_t)*q;
         });
       } else if (have_ids) {
@@ -1488,7 +1489,10 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
   // 54 / 47, 10 per row with power-law degrees 312500 x 128 46 / 42, 3 edges per row 66666 x 602 76 / 68; 4 bit 67 / 59;
   // 2 bit 62 / 55; short launches of 1000 columns 21 / 17; narrow rows level).  Staged rows have their loads behind them,
   // and fewer items leave lanes idle there: 25 edges per row, 4 bit, 117000 x 128 72 / 81, 2 bit, 150000 x 100 65 / 68.
-  const bool wide = direct;
+  // Short launches of 8-bit rows too (blocks of eight rows, where a row's groups of four are one round of items): items of
+  // eight leave half the lanes of a block idle there (before / eight / four, us, 100 columns: 2500 rows, 8 edges 4.2 / 4.5 /
+  // 4.2, 24 edges 5.9 / 6.6 / 5.9; level at 30 000 rows; from 136 columns eight are ahead at any size).
+  const bool wide = direct && !(BITS == 8 && a.R <= 16384 && 8 * ceil_div(a.feat_dim, 4) <= TB);
   a.items_per_row = (int)ceil_div(a.feat_dim, wide ? 8 : 4);
   // item / items_per_row as a high product, exact for items < 64 * 1024: rows of eight columns are one item of eight, and
   // 2^32 / 1 has no room in the word, so the wide form takes 2^31 / items_per_row and doubles the item
@@ -1544,7 +1548,7 @@ int launch_sq_rows_sized(RowsArgs a, const void* indptr, const void* indices, in
         break;                                                                   \
       }                                                                          \
     }                                                                            \
-    if constexpr (!DEAL || BITS == 2 || BITS == 4) {   /* 1 and 8 bits: always direct */ \
+    if constexpr (!DEAL || BITS != 1) {   /* 1 bit: always items of eight */      \
       if constexpr (BITS <= 2) {                                                 \
         if (half == 0) F2CGT_ROWS_GO(I, 0, DEAL ? 4 : 0);                        \
       }                                                                          \

@@ -1,5 +1,5 @@
-"""Log-domain rows with one codebook whose codes are read where they are: items of eight columns.  The same values in the
-same order as decoding the rows and aggregating them, so bit for bit the same."""
+"""Log-domain rows with one codebook whose codes are read where they are: items of eight columns, or of four in short
+launches of 8-bit rows.  The same values in the same order as decoding the rows and aggregating them, so bit for bit the same."""
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -12,6 +12,12 @@ pytestmark = pytest.mark.gpu
 # widths about whole items and, for 2 and 4 bits, about the line between staged (four columns) and direct
 WIDTHS = [(8, d) for d in (8, 10, 12, 14, 16, 18, 130, 254, 602, 1030)] + \
          [(4, d) for d in (16, 254, 256, 258, 260, 262, 264, 602)] + [(2, d) for d in (32, 512, 514, 516, 518, 520, 1030)]
+
+
+def test_eight_bit_rows_on_both_sides_of_a_short_launch():
+    for dim in (8, 10, 12, 14, 20, 66, 126, 128, 130, 132):
+        for rows in (16384, 16385):
+            test_equal_to_decode_and_aggregate(8, dim, rows, 6)
 
 
 @pytest.mark.parametrize("bits,dim", WIDTHS)
