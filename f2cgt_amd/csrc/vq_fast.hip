@@ -342,7 +342,7 @@ __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlan
 //   pieces): graphs and outputs in turn, 24 x 32 from 5.8 GB of codes 637 / 584 / 642 / 643 -> 581 us, 16 x 8 from
 //   160 MB 123 / 111 / 124 -> 108, 16 x 16 at 10 edges per row 98 / 74 / 78 -> 67; one graph and output again and again
 //   447 / 463 / 490 / 475 -> 460, 79 / 76 / 78 -> 76 and 92 / 74 / 73 -> 68: only 24 x 32, whose output the last-level
-//   cache takes in part, is slower than with the plain halves, and only there.
+//   cache takes in part, is slower than with the plain halves.  (Few edges per row: see launch_vq.)
 //   RPM < 4: the lane groups that share a row add their sums while they hand them on (v_permlane16_swap: a group ends up
 //   with the totals of one half), so that one store instruction writes the row's 512 bytes.
 template <int BT, int H, int RPM, typename Idx, bool TAIL = false, bool EVEN2 = false, bool TRACE = false>

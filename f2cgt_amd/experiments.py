@@ -9,7 +9,7 @@
     python3 -m f2cgt_amd.experiments affine-geometry x   the affine kernel by edges per row: edge mapping, accumulator sizing, block rows, workgroup size
     python3 -m f2cgt_amd.experiments hybrid-geometry x   the two-table kernel by edges per row: workgroup size and edge batch
     python3 -m f2cgt_amd.experiments vq-degrees x        the fused VQ kernel on uniform and ragged rows: rows per mini-block
-    python3 -m f2cgt_amd.experiments vq-store-forms warm|rotate   the fused VQ kernel's store forms by shape
+    python3 -m f2cgt_amd.experiments vq-store-forms warm|rotate   the fused VQ kernel's two lane layouts by shape
     python3 -m f2cgt_amd.experiments store-form x        plain against non-temporal output stores by shape (any build)
     python3 -m f2cgt_amd.experiments lds-rate x          bytes per clock and CU that conflict-free LDS reads return
     python3 -m f2cgt_amd.experiments cold-parts c2|c3|c4|c5   launch time by what of the input is still cached (any build)
