@@ -1157,6 +1157,7 @@ c10::optional<torch::Tensor> sage_linear(const torch::Tensor& x0, const torch::T
       x1.size(0) != m || w1.size(0) != n || w0.size(1) != k0 || w1.size(1) != k1 || (bias.has_value() && bias->size(0) != n))
     return c10::nullopt;
   const int take = f2cgt_sage_linear_ahead(m, n, k0, k1);
+  py::gil_scoped_release unlocked;         // as the operators do: the library may look for a kernel, other threads go on
   if (c10::GradMode::is_enabled() && (w0.requires_grad() || w1.requires_grad() || (bias.has_value() && bias->requires_grad()))) {
     if (!(take & F2CGT_SAGE_GRAD)) return c10::nullopt;
     return SageLinear::apply(x0, x1, w0, w1, bias, relu, (take & F2CGT_SAGE_STEP) != 0);

@@ -277,3 +277,28 @@ def test_gradients_are_as_close_to_float64_as_the_operators(m):
                 err[i, j] += (a.double() - e).norm() / e.norm()
     # the mean of forty such errors is itself known to about 1 % (256 values each, of spread 1 about their size: 1 / sqrt(2 * 256 * 40))
     assert bool((err[0] <= 1.01 * err[1]).all()), (err / 40).tolist()
+
+
+def test_several_threads_with_hooks():
+    """The call runs without the interpreter's lock; hooks on saved tensors take it for themselves."""
+    import threading
+    lib = f2cgt_amd.load()
+    x0, x1, w0, w1, b, g = _inputs(300, 16, 24, 40)
+    want = torch.autograd.grad(lib.sage_linear(x0, x1, w0, w1, b, True), (w0, w1, b), g)
+    torch.cuda.synchronize()
+    same = []
+
+    def work():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            mine = [p.detach().clone().requires_grad_() for p in (w0, w1, b)]
+            for _ in range(20):
+                with torch.autograd.graph.saved_tensors_hooks(lambda t: [t], lambda kept: kept[0]):
+                    out = lib.sage_linear(x0, x1, *mine, True)
+                same.append(all(torch.equal(p, q) for p, q in zip(torch.autograd.grad(out, mine, g), want)))
+            torch.cuda.current_stream().synchronize()
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert same == [True] * 80
